@@ -3,17 +3,23 @@
 The directory name carries a hyphen, so the package is loaded by path under the
 module name `tensorrt_incubator_amd` (see `__graft_entry__.load_package`).
 
-torch is used only to own device memory and streams: every wrapper below passes
+torch is used only to own device memory and streams: every call below passes
 raw device pointers, extents and the current stream handle to the C ABI declared
-in include/mtrt_hip.h.  There is no fallback: if the shared library is missing or
-no gfx950 device is usable, the calls raise.
+in include/mtrt_hip.h.  The calls that a program makes on each step do so from the
+extension module built from csrc/frontend/frontend.cpp (the function here carries the
+signature, the checks and the launch are native); set-up calls go through ctypes.
+There is no fallback: if a shared library is missing or no gfx950 device is usable,
+the calls raise.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_DIR = os.path.join(_HERE, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libmtrt_hip.so")
+FRONTEND_PATH = os.path.join(LIB_DIR, "mtrt_frontend.so")
 KERNEL_MODULE_PATH = os.path.join(LIB_DIR, "mtrt_kernels.hsaco")
 FIXTURE_MODULE_PATH = os.path.join(LIB_DIR, "mtrt_test_fixtures.hsaco")
 
@@ -140,6 +146,26 @@ def lib():
     return _lib
 
 
+_frontend = None
+
+
+def frontend():
+    """The extension module with the native side of the calls below; raises if it is not built."""
+    global _frontend
+    if _frontend is None:
+        lib()
+        _torch()                                       # its libraries are loaded before the extension that needs them
+        if not os.path.exists(FRONTEND_PATH):
+            raise RuntimeError(
+                "%s is missing: run `python tensorrt-incubator_amd/build.py` (there is no fallback path)" % FRONTEND_PATH)
+        loader = importlib.machinery.ExtensionFileLoader("mtrt_frontend", FRONTEND_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("mtrt_frontend", loader))
+        loader.exec_module(module)
+        module.set_error_type(MtrtHipError)
+        _frontend = module
+    return _frontend
+
+
 def check(status):
     if status != 0:
         raise MtrtHipError(status, lib().mtrt_hip_last_error().decode())
@@ -167,10 +193,6 @@ def _stream():
     return _torch().cuda.current_stream().cuda_stream
 
 
-def _ptr(t):
-    return None if t is None else t.data_ptr()
-
-
 def code_tensor(q_dtype, numel, device):
     """Uninitialised storage for `numel` quantized codes (uint8/int8 bytes)."""
     torch = _torch()
@@ -183,82 +205,36 @@ def code_tensor(q_dtype, numel, device):
 
 def amax(x, qmax):
     """Returns (amax, scale) as two 0-d f32 device tensors; scale = amax / qmax."""
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous()
-    out = torch.empty(2, dtype=torch.float32, device=x.device)
-    check(lib().mtrt_hip_amax(_stream(), x.data_ptr(), float_dtype_of(x), x.numel(), float(qmax),
-                              out.data_ptr(), out.data_ptr() + 4))
-    return out[0], out[1]
+    return (_frontend or frontend()).amax(x, qmax)
 
 
 def amax_scales(x, qmax, kind, d0=None, d1=None, nb=1):
     """(amax, scale) f32 device tensors with one element per scale element of the addressing (kind, nb) over the
     [d0, d1] view of x: nb elements for SCALE_ROW, (d0 / nb) * d1 for SCALE_COL, one for SCALE_UNIFORM."""
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous()
-    d0, d1 = _view2d(x, d0, d1)
-    count = 1 if kind == SCALE_UNIFORM else (nb if kind == SCALE_ROW else (d0 // nb) * d1)
-    out = torch.empty((2, max(count, 0)), dtype=torch.float32, device=x.device)
-    check(lib().mtrt_hip_amax_scales(_stream(), x.data_ptr(), float_dtype_of(x), kind, d0, d1, nb, float(qmax),
-                                     out[0].data_ptr(), out[1].data_ptr()))
-    return out[0], out[1]
+    return (_frontend or frontend()).amax_scales(x, qmax, kind, d0, d1, nb)
 
 
 def quantize(x, scale, q_dtype, kind=SCALE_UNIFORM, d0=None, d1=None, nb=1, flags=0, out=None):
-    assert x.is_cuda and x.is_contiguous() and scale.is_cuda and scale.dtype == _torch().float32
-    d0, d1 = _view2d(x, d0, d1)
-    q = code_tensor(q_dtype, d0 * d1, x.device) if out is None else out
-    check(lib().mtrt_hip_quantize(_stream(), x.data_ptr(), float_dtype_of(x), q.data_ptr(), q_dtype,
-                                  scale.data_ptr(), kind, d0, d1, nb, flags))
-    return q
+    return (_frontend or frontend()).quantize(x, scale, q_dtype, kind, d0, d1, nb, flags, out)
 
 
 def dequantize(q, scale, q_dtype, out_torch_dtype, shape, kind=SCALE_UNIFORM, d0=None, d1=None, nb=1, out=None):
-    torch = _torch()
-    assert q.is_cuda and q.is_contiguous() and scale.dtype == torch.float32
-    y = torch.empty(shape, dtype=out_torch_dtype, device=q.device) if out is None else out
-    d0, d1 = _view2d(y, d0, d1)
-    check(lib().mtrt_hip_dequantize(_stream(), q.data_ptr(), q_dtype, y.data_ptr(), float_dtype_of(y),
-                                    scale.data_ptr(), kind, d0, d1, nb))
-    return y
+    return (_frontend or frontend()).dequantize(q, scale, q_dtype, out_torch_dtype, shape, kind, d0, d1, nb, out)
 
 
 def quantize_dequantize(x, scale, q_dtype, kind=SCALE_UNIFORM, d0=None, d1=None, nb=1, flags=0, q_out=None, y_out=None):
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous() and scale.dtype == torch.float32
-    d0, d1 = _view2d(x, d0, d1)
-    q = code_tensor(q_dtype, d0 * d1, x.device) if q_out is None else q_out
-    y = torch.empty_like(x) if y_out is None else y_out
-    check(lib().mtrt_hip_quantize_dequantize(_stream(), x.data_ptr(), float_dtype_of(x), q.data_ptr(), q_dtype,
-                                             y.data_ptr(), scale.data_ptr(), kind, d0, d1, nb, flags))
-    return q, y
+    return (_frontend or frontend()).quantize_dequantize(x, scale, q_dtype, kind, d0, d1, nb, flags, q_out, y_out)
 
 
 def dynamic_quantize_dequantize(x, q_dtype, qmax, flags=0, dequantize=True):
     """amax -> scale -> quantize (-> dequantize) of the whole tensor in one call; returns (q, y or None, amax, scale)."""
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous()
-    out = torch.empty(2, dtype=torch.float32, device=x.device)
-    q = code_tensor(q_dtype, x.numel(), x.device)
-    y = torch.empty_like(x) if dequantize else None
-    check(lib().mtrt_hip_dynamic_quantize_dequantize(_stream(), x.data_ptr(), float_dtype_of(x), q.data_ptr(), q_dtype,
-                                                     _ptr(y), x.numel(), float(qmax), out.data_ptr(), out.data_ptr() + 4,
-                                                     flags))
-    return q, y, out[0], out[1]
+    return (_frontend or frontend()).dynamic_quantize_dequantize(x, q_dtype, qmax, flags, dequantize)
 
 
 def dynamic_quantize_rows(x, q_dtype, qmax, flags=0, want_amax=True):
     """Per-row amax -> scale -> quantize of a [rows, d] tensor (leading axes folded into rows) in one call; returns
     (q [rows * d] codes, amax [rows] or None, scale [rows])."""
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous() and x.dim() >= 1
-    d = x.shape[-1]
-    rows = x.numel() // d if d else 0
-    out = torch.empty((2, rows), dtype=torch.float32, device=x.device)
-    q = code_tensor(q_dtype, x.numel(), x.device)
-    check(lib().mtrt_hip_dynamic_quantize_rows(_stream(), x.data_ptr(), float_dtype_of(x), q.data_ptr(), q_dtype, rows, d,
-                                               float(qmax), out[0].data_ptr() if want_amax else None, out[1].data_ptr(), flags))
-    return q, (out[0] if want_amax else None), out[1]
+    return (_frontend or frontend()).dynamic_quantize_rows(x, q_dtype, qmax, flags, want_amax)
 
 
 class View2d(ctypes.Structure):
@@ -296,51 +272,19 @@ def nvfp4_quantize(x, tensor_amax, axis=-1):
     """NVFP4 codes (uint8, two per byte) and block scales (uint8 f8e4m3fn bytes, the shape of `x` with the blocked
     extent divided by 16) of `x`, blocks of 16 along `axis` (-1 or -2); `tensor_amax` is a 0-d f32 device
     tensor (what amax() returns)."""
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous() and tensor_amax.is_cuda and tensor_amax.dtype == torch.float32
-    assert axis in (-1, -2, x.dim() - 1, x.dim() - 2)
-    last = axis in (-1, x.dim() - 1)
-    d1 = x.shape[-1]
-    d0 = x.numel() // d1 if d1 else 0
-    q = torch.empty(x.numel() // 2, dtype=torch.uint8, device=x.device)
-    sshape = x.shape[:-1] + (d1 // 16,) if last else x.shape[:-2] + (x.shape[-2] // 16, d1)
-    s = torch.empty(sshape, dtype=torch.uint8, device=x.device)
-    check(lib().mtrt_hip_nvfp4_quantize(_stream(), x.data_ptr(), float_dtype_of(x), q.data_ptr(), s.data_ptr(),
-                                        tensor_amax.data_ptr(), d0, d1, 1 if last else 0))
-    return q, s
+    return (_frontend or frontend()).nvfp4_quantize(x, tensor_amax, axis)
 
 
 def nvfp4_dequantize(q, scales, tensor_amax, out_torch_dtype, shape, axis=-1):
-    torch = _torch()
-    assert q.is_cuda and q.dtype == torch.uint8 and scales.dtype == torch.uint8 and tensor_amax.dtype == torch.float32
-    y = torch.empty(shape, dtype=out_torch_dtype, device=q.device)
-    last = axis in (-1, y.dim() - 1)
-    d1 = y.shape[-1]
-    d0 = y.numel() // d1 if d1 else 0
-    check(lib().mtrt_hip_nvfp4_dequantize(_stream(), q.data_ptr(), scales.data_ptr(), tensor_amax.data_ptr(),
-                                          y.data_ptr(), float_dtype_of(y), d0, d1, 1 if last else 0))
-    return y
+    return (_frontend or frontend()).nvfp4_dequantize(q, scales, tensor_amax, out_torch_dtype, shape, axis)
 
 
 def layernorm(x, gamma, beta, eps, out=None):
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous() and gamma.dtype == x.dtype and beta.dtype == x.dtype
-    d = x.shape[-1]
-    rows = x.numel() // d if d else 0
-    y = torch.empty_like(x) if out is None else out
-    check(lib().mtrt_hip_layernorm(_stream(), x.data_ptr(), gamma.data_ptr(), beta.data_ptr(), y.data_ptr(),
-                                   float_dtype_of(x), rows, d, float(eps)))
-    return y
+    return (_frontend or frontend()).layernorm(x, gamma, beta, eps, out)
 
 
 def softmax(x, out=None):
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous()
-    d = x.shape[-1]
-    rows = x.numel() // d if d else 0
-    y = torch.empty_like(x) if out is None else out
-    check(lib().mtrt_hip_softmax(_stream(), x.data_ptr(), y.data_ptr(), float_dtype_of(x), rows, d))
-    return y
+    return (_frontend or frontend()).softmax(x, out)
 
 
 def gemm_w8a8_prepack(w_kn):
@@ -354,16 +298,7 @@ def gemm_w8a8_prepack(w_kn):
 
 
 def gemm_w8a8(a, w_nk, a_scale, w_scale, out=None):
-    torch = _torch()
-    assert a.is_cuda and a.is_contiguous() and a.dtype == torch.int8 and w_nk.is_contiguous() and w_nk.dtype == torch.int8
-    assert a_scale.dtype == torch.float32 and w_scale.dtype == torch.float32
-    M, K = a.shape
-    N = w_nk.shape[0]
-    assert w_nk.shape[1] == K and a_scale.numel() == M and w_scale.numel() == N
-    y = torch.empty((M, N), dtype=torch.float16, device=a.device) if out is None else out
-    check(lib().mtrt_hip_gemm_w8a8(_stream(), a.data_ptr(), w_nk.data_ptr(), a_scale.data_ptr(), w_scale.data_ptr(),
-                                   y.data_ptr(), M, K, N))
-    return y
+    return (_frontend or frontend()).gemm_w8a8(a, w_nk, a_scale, w_scale, out)
 
 
 def gemm_w8a8_prepack_fragments(w, is_nk=False):
@@ -379,16 +314,7 @@ def gemm_w8a8_prepack_fragments(w, is_nk=False):
 
 
 def gemm_w8a8_fragments(a, w_frag, a_scale, w_scale, N, out=None):
-    torch = _torch()
-    assert a.is_cuda and a.is_contiguous() and a.dtype == torch.int8 and w_frag.dtype == torch.int8
-    assert a_scale.dtype == torch.float32 and w_scale.dtype == torch.float32
-    M, K = a.shape
-    assert a_scale.numel() == M and w_scale.numel() == N
-    assert w_frag.numel() == lib().mtrt_hip_gemm_w8a8_fragments_bytes(K, N)
-    y = torch.empty((M, N), dtype=torch.float16, device=a.device) if out is None else out
-    check(lib().mtrt_hip_gemm_w8a8_fragments(_stream(), a.data_ptr(), w_frag.data_ptr(), a_scale.data_ptr(),
-                                             w_scale.data_ptr(), y.data_ptr(), M, K, N))
-    return y
+    return (_frontend or frontend()).gemm_w8a8_fragments(a, w_frag, a_scale, w_scale, N, out)
 
 
 def gemm_w4a16_prepack(w_kn_packed, K, N):
@@ -403,32 +329,9 @@ def gemm_w4a16_prepack(w_kn_packed, K, N):
 
 
 def gemm_w4a16(a, scale, K, N, block, w_kn_packed=None, w_prepacked=None, out=None):
-    torch = _torch()
-    assert a.is_cuda and a.is_contiguous() and a.dtype == torch.float16 and scale.dtype == torch.float16
-    M = a.shape[0]
-    y = torch.empty((M, N), dtype=torch.float16, device=a.device) if out is None else out
-    check(lib().mtrt_hip_gemm_w4a16(_stream(), a.data_ptr(), _ptr(w_kn_packed), _ptr(w_prepacked), scale.data_ptr(),
-                                    y.data_ptr(), M, K, N, block))
-    return y
+    return (_frontend or frontend()).gemm_w4a16(a, scale, K, N, block, w_kn_packed, w_prepacked, out)
 
 
 def linear_dense(x, w_nk, bias=None, out=None):
     """y = x @ w_nk^T (+ bias) in the operands' float type, f32 accumulation; x [M,K], w_nk [N,K]."""
-    torch = _torch()
-    assert x.is_cuda and x.is_contiguous() and w_nk.is_contiguous() and w_nk.dtype == x.dtype and x.dim() == 2
-    M, K = x.shape
-    N = w_nk.shape[0]
-    assert w_nk.shape[1] == K and (bias is None or (bias.dtype == x.dtype and bias.numel() == N and bias.is_contiguous()))
-    y = torch.empty((M, N), dtype=x.dtype, device=x.device) if out is None else out
-    check(lib().mtrt_hip_linear_dense(_stream(), x.data_ptr(), w_nk.data_ptr(), _ptr(bias), y.data_ptr(),
-                                      float_dtype_of(x), M, K, N))
-    return y
-
-
-def _view2d(t, d0, d1):
-    if d0 is None or d1 is None:
-        if t.dim() == 0:
-            return 1, 1
-        d1 = t.shape[-1]
-        d0 = t.numel() // d1 if d1 else 0
-    return int(d0), int(d1)
+    return (_frontend or frontend()).linear_dense(x, w_nk, bias, out)

@@ -4,6 +4,7 @@
   lib/mtrt_test_fixtures.hsaco  the two launch-ABI test kernels, as a separate module
   lib/libmtrt_hip.so            C ABI (launch layer + cluster layer) with the kernel
                                 module embedded as read-only data
+  lib/mtrt_frontend.so          CPython extension: the Python front end's calls on torch tensors, over the C ABI
   lib/mtrt_standalone_selftest  host program in the style of EmitC-generated C++ that calls the
                                 `namespace mtrt` flavour of the launch layer (run by the tests)
 
@@ -77,6 +78,19 @@ def build_runtime():
           "-o", os.path.join(LIB, "libmtrt_hip.so")])
 
 
+def build_frontend():
+    """The extension sees torch's tensors, so it is compiled against the installed torch's headers; torch is imported
+    (its libraries loaded) before the extension is, so no path to them is recorded."""
+    import sysconfig
+    from torch.utils.cpp_extension import COMMON_HIP_FLAGS, include_paths, library_paths
+    flags = ["-I" + p for p in include_paths() + [sysconfig.get_paths()["include"], os.path.join(ROCM, "include"), os.path.join(ROOT, "include")]]
+    flags += [f for f in COMMON_HIP_FLAGS if f.startswith("-D")] + ["-L" + p for p in library_paths()]
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-unused-function", "-w",
+          os.path.join(CSRC, "frontend", "frontend.cpp")] + flags +
+         ["-L" + LIB, "-lmtrt_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN",
+          "-o", os.path.join(LIB, "mtrt_frontend.so")])
+
+
 def build_selftest():
     src = os.path.join(CSRC, "selftest", "standalone_selftest.cpp")
     # include/standalone holds the reference's header NAMES (MTRTRuntimeCuda.h ...), as generated code includes them
@@ -93,6 +107,7 @@ def build_oracle():
 def build_all():
     build_kernels()
     build_runtime()
+    build_frontend()
     build_selftest()
     build_oracle()
 

@@ -139,6 +139,21 @@ def _produced(t, d):
     return Tensor(t, _produced=True, _tp_dtype=d)
 
 
+_bound = None
+
+
+def _native():
+    """The extension's functions for steady-state calls (operands in device memory, constant scales uploaded): they answer
+    NotImplemented for anything else, and the general path below each call runs."""
+    global _bound
+    if _bound is None:
+        from . import frontend
+        module = frontend()
+        module.bind_tp(Tensor, float32, float16, bfloat16, int8, int4, float8)
+        _bound = module
+    return _bound
+
+
 def ones(shape, dtype=float32):
     """An operation result, hence not a constant (tripy/tests/frontend/ops/test_quantize.py:76-84 relies on it).
     Values are made on the host and uploaded on first use by a kernel."""
@@ -259,6 +274,9 @@ def _stream():
 
 def quantize(input, scale, dtype, dim=None):
     """tp.quantize: clamp(round_half_even(input / scale)) in `dtype` (int8, int4 or float8)."""
+    done = (_bound or _native()).tp_quantize(input, scale, dtype, dim)
+    if done is not NotImplemented:
+        return done
     if not isinstance(input, Tensor):
         input = Tensor(input)
     scale = _convert_scale(scale, input.dtype)
@@ -279,6 +297,9 @@ def quantize(input, scale, dtype, dim=None):
 
 def dequantize(input, scale, dtype, dim=None):
     """tp.dequantize: input * scale in `dtype` (float32, float16 or bfloat16)."""
+    done = (_bound or _native()).tp_dequantize(input, scale, dtype, dim)
+    if done is not NotImplemented:
+        return done
     if not isinstance(input, Tensor):
         input = Tensor(input)
     scale = _convert_scale(scale, dtype)
@@ -466,6 +487,9 @@ def layernorm(input, weight, bias, eps):
     """tripy/nvtripy/frontend/module/layernorm.py:36-77: normalises over the last D = weight.rank
     dimensions, y = (x - mean) * rsqrt(var + eps) * weight + bias, in the input's dtype.  One launch of the
     LayerNorm cluster over [prod(leading dims), prod(normalized_shape)]."""
+    done = (_bound or _native()).tp_layernorm(input, weight, bias, eps)
+    if done is not NotImplemented:
+        return done
     from . import layernorm as _layernorm_rows
     for t in (input, weight, bias):
         if not isinstance(t, Tensor):
@@ -546,6 +570,9 @@ class LayerNorm:
 def softmax(input, dim=None):
     """tripy/nvtripy/frontend/ops/softmax.py:30-82: over `dim`, or over the flattened input when dim is None.
     The cluster works on rows; another dimension is brought last for the launch and put back."""
+    done = (_bound or _native()).tp_softmax(input, dim)
+    if done is not NotImplemented:
+        return done
     from . import softmax as _softmax_rows
     if not isinstance(input, Tensor):
         input = Tensor(input)

@@ -1,0 +1,80 @@
+"""The native side of the Python calls (csrc/frontend/frontend.cpp): the steady-state path of each `tp` function gives what
+its general path gives on the same values, for every scale addressing, type and rank it takes on; what it does not
+take on (values still in host memory, other axes, views that are not dense) goes to the general path; preconditions
+are reported as the package's functions always did."""
+import importlib
+
+import numpy as np
+import pytest
+
+from helpers import rng
+
+
+@pytest.fixture(scope="module")
+def tp(pkg):
+    return importlib.import_module(pkg.__name__ + ".tp")
+
+
+def test_preconditions_are_assertions(pkg):
+    import torch
+    x = torch.zeros((2, 16))
+    for call in (lambda: pkg.amax(x, 127.0), lambda: pkg.softmax(x), lambda: pkg.quantize(x, x, pkg.I8),
+                 lambda: pkg.layernorm(x, x[0], x[0], 1e-5), lambda: pkg.linear_dense(x, x), lambda: pkg.nvfp4_quantize(x, x[0, 0]),
+                 lambda: pkg.dynamic_quantize_rows(x, pkg.I8, 127.0), lambda: pkg.gemm_w4a16(x, x, 16, 2, 16)):
+        with pytest.raises(AssertionError):
+            call()
+    with pytest.raises(TypeError):
+        pkg.softmax([1.0, 2.0])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dname", ["float32", "float16", "bfloat16"])
+@pytest.mark.parametrize("shape,dim,qname", [((3, 5, 7), 1, "int8"), ((3, 5, 7), -1, "float8"), ((6, 33), 0, "int8"), ((17,), None, "int8"),
+                                             ((256, 48), "block", "int4"), ((), None, "float8"), ((1, 1, 1), 2, "int4"), ((2, 3, 4, 5), 0, "int4")])
+def test_steady_state_calls_equal_the_general_path(tp, dname, shape, dim, qname):
+    import torch
+    td, d, qd = getattr(torch, dname), getattr(tp, dname), getattr(tp, qname)
+    r = rng(31 + len(shape))
+    host = torch.from_numpy(np.asarray(r.standard_normal(shape) * 3, dtype=np.float32)).to(td)
+    sshape = () if dim is None else (shape[0] // 64, shape[1]) if dim == "block" else (shape[dim],)
+    scale = tp.Tensor(torch.from_numpy(np.asarray(r.uniform(0.02, 0.2, sshape), dtype=np.float32)).to(td))
+    dim = None if dim == "block" else dim
+    native = tp._native()
+    general = tp.quantize(tp.Tensor(host), scale, qd, dim)           # values in host memory: the general path uploads them
+    x = tp.Tensor(host.cuda())
+    q = native.tp_quantize(x, scale, qd, dim)
+    assert q is not NotImplemented and type(q) is tp.Tensor and q.dtype is qd and q.shape == tuple(shape) and not q.is_cpu_constant
+    assert torch.equal(q.torch(), general.torch())
+    y = native.tp_dequantize(q, scale, d, dim)
+    assert y is not NotImplemented and y.dtype is d and y.shape == tuple(shape)
+    scale2 = tp.Tensor(scale.torch())                                # not uploaded yet: the general path
+    assert native.tp_dequantize(q, scale2, d, dim) is NotImplemented
+    assert torch.equal(tp.dequantize(q, scale2, d, dim).torch(), y.torch())
+
+
+@pytest.mark.gpu
+def test_what_is_left_to_the_general_path(tp):
+    import torch
+    native = tp._native()
+    x = torch.randn(4, 6, device="cuda")
+    one = tp.Tensor(np.float32(1.0))
+    tp.quantize(tp.Tensor(x), one, tp.int8)
+    t = tp.Tensor(x.t())                                             # not dense
+    assert native.tp_quantize(t, one, tp.int8, None) is NotImplemented
+    assert torch.equal(tp.quantize(t, one, tp.int8).torch(), tp.quantize(tp.Tensor(x), one, tp.int8).torch().t())
+    for args in ((tp.Tensor(x), 1.0, tp.int8, None), (tp.Tensor(x), one, tp.float16, None), (tp.Tensor(x), one, tp.int8, 0),
+                 (tp.Tensor(x.half()), one, tp.int8, None), (x, one, tp.int8, None), (tp.Tensor(x[:0]), one, tp.int8, None)):
+        assert native.tp_quantize(*args) is NotImplemented
+    assert native.tp_softmax(tp.Tensor(x), 0) is NotImplemented and native.tp_softmax(tp.Tensor(x), None) is NotImplemented
+    w = tp.Tensor(torch.ones(6, device="cuda"))
+    b = tp.Tensor(torch.zeros(6, device="cuda"))
+    assert native.tp_layernorm(tp.Tensor(x), w, tp.Tensor(torch.zeros(5, device="cuda")), 1e-5) is NotImplemented
+    assert native.tp_layernorm(tp.Tensor(x[0].contiguous()), w, b, 1e-5) is NotImplemented
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):                                       # enqueued on the current stream, whichever it is
+        torch.cuda._sleep(1000000)
+        late = tp.Tensor(x * 2)
+        y = native.tp_softmax(late, -1)
+    s.synchronize()
+    assert torch.allclose(y.torch(), torch.softmax(x * 2, -1), atol=1e-6)
+    assert torch.allclose(native.tp_layernorm(tp.Tensor(x), w, b, 1e-5).torch(), torch.nn.functional.layer_norm(x, (6,)), atol=1e-5)
