@@ -394,8 +394,8 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w8a8(mtrt_stream_t stream, const void *
  * in that form only).  `w` is the program's [K,N] constant (w_is_nk = 0) or an [N,K] array (w_is_nk = 1);
  * w_frag holds mtrt_hip_gemm_w8a8_fragments_bytes(K, N) bytes (0 = shape not supported: K % 128 != 0)
  * and must be 16-byte aligned.  Same results, bit for bit.  Up to 32 rows (decode) take a kernel of their own
- * that is bound by reading the weights once, not by a tile's K loop, and so do 33 to 128 rows while that is
- * shorter than a tile launch. */
+ * that is bound by reading the weights once, not by a tile's K loop, and so do 33 to 64 rows while that is
+ * shorter than a tile launch; the tile (32 x 128 to 256 x 384) follows from the shape. */
 MTRT_CAPI_EXPORTED int64_t mtrt_hip_gemm_w8a8_fragments_bytes(int64_t K, int64_t N);
 MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w8a8_prepack_fragments(mtrt_stream_t stream, const void *w,
                                                                 int32_t w_is_nk, void *w_frag, int64_t K,
@@ -404,6 +404,15 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w8a8_fragments(mtrt_stream_t stream, co
                                                         const void *w_frag, const float *a_scale,
                                                         const float *w_scale, void *y, int64_t M, int64_t K,
                                                         int64_t N);
+/* The same call with scratch memory of the caller's (16-byte aligned device memory that stays the call's own until its work
+ * on `stream` is done, mtrt_hip_gemm_w8a8_fragments_workspace(M, K, N) bytes): few-tile shapes with a long K then
+ * share each output tile's K range among several workgroups (M = 200, K = 12288, N = 512: 52.7 -> 10.6 us).  Less or no
+ * scratch: the unsplit form.  Same bits either way. */
+MTRT_CAPI_EXPORTED int64_t mtrt_hip_gemm_w8a8_fragments_workspace(int64_t M, int64_t K, int64_t N);
+MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w8a8_fragments_ws(mtrt_stream_t stream, const void *a,
+                                                           const void *w_frag, const float *a_scale,
+                                                           const float *w_scale, void *y, int64_t M, int64_t K,
+                                                           int64_t N, void *workspace, int64_t workspace_bytes);
 
 /* W4A16 block-wise GEMM:
  *   wd[k,n] = f16(f16(w[k,n]) * scale[k / block, n])   ;   y[m,n] = f16(sum_k f32(a[m,k]) * f32(wd[k,n]))
@@ -524,7 +533,8 @@ struct mtrt_lua_builtin {
 MTRT_CAPI_EXPORTED const struct mtrt_lua_builtin *mtrt_lua_cuda_builtins(size_t *count);
 
 /* Name of the kernel that the most recent successful part-2 call on this thread
- * launched last (for profiles and tests). */
+ * launched last (for profiles and tests).  Where one GEMM exists in several tiles the name is that of the class of
+ * shapes the call belongs to; the symbol of the tile adds a suffix to it or replaces it. */
 MTRT_CAPI_EXPORTED const char *mtrt_hip_last_kernel(void);
 
 #ifdef __cplusplus

@@ -114,6 +114,8 @@ PROTOTYPES = {
     "mtrt_hip_gemm_w8a8_fragments_bytes": (_i64, [_i64, _i64]),
     "mtrt_hip_gemm_w8a8_prepack_fragments": (_i32, [_vp, _vp, _i32, _vp, _i64, _i64]),
     "mtrt_hip_gemm_w8a8_fragments": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64]),
+    "mtrt_hip_gemm_w8a8_fragments_workspace": (_i64, [_i64, _i64, _i64]),
+    "mtrt_hip_gemm_w8a8_fragments_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64]),
     "mtrt_hip_linear_dense": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64]),
     "mtrt_hip_gemm_w4a16_prepacked_bytes": (_i64, [_i64, _i64]),
     "mtrt_hip_gemm_w4a16_prepack": (_i32, [_vp, _vp, _vp, _i64, _i64]),

@@ -88,6 +88,10 @@ at::Tensor empty_like_device(at::IntArrayRef shape, at::ScalarType type, const a
   return at::Tensor(at::detail::empty_cuda(shape, type, where.device(), std::nullopt));
 }
 
+// Scratch memory of a call: back with torch's allocator when the call returns, which hands it only to work that follows on
+// the same stream.
+at::Tensor bytes_on(const at::Tensor &where, int64_t n) { return empty_like_device({n}, at::ScalarType::Byte, where); }
+
 // storage for n codes: int8 for MTRT_I8, else bytes; two to a byte for the packed types
 at::Tensor code_storage(int32_t q_dtype, int64_t n, const at::Tensor &where) {
   const bool packed = q_dtype == MTRT_I4_PACKED || q_dtype == MTRT_F4_PACKED;
@@ -543,8 +547,11 @@ PyObject *w8a8(PyObject *const *a, const at::Tensor &x, const at::Tensor &w, con
   const at::Tensor y = out ? *out : empty_like_device({M, N}, at::ScalarType::Half, x);
   const mtrt_stream_t s = current_stream();
   const float *asp = static_cast<const float *>(as.data_ptr()), *wsp = static_cast<const float *>(ws.data_ptr());
+  const int64_t scratch_bytes = fragments ? mtrt_hip_gemm_w8a8_fragments_workspace(M, K, N) : 0;
+  const at::Tensor scratch = scratch_bytes ? bytes_on(x, scratch_bytes) : at::Tensor();
   if (!launch([&] {
-        return fragments ? mtrt_hip_gemm_w8a8_fragments(s, x.data_ptr(), w.data_ptr(), asp, wsp, y.data_ptr(), M, K, N)
+        return fragments ? mtrt_hip_gemm_w8a8_fragments_ws(s, x.data_ptr(), w.data_ptr(), asp, wsp, y.data_ptr(), M, K, N,
+                                                           scratch_bytes ? scratch.data_ptr() : nullptr, scratch_bytes)
                          : mtrt_hip_gemm_w8a8(s, x.data_ptr(), w.data_ptr(), asp, wsp, y.data_ptr(), M, K, N);
       }))
     return nullptr;

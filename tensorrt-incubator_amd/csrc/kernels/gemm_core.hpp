@@ -49,6 +49,8 @@ namespace gemm_core {
 using namespace mtrt_dev;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_halves __attribute__((aligned(2)));
+typedef f32x4 f32x4_words __attribute__((aligned(4)));
 
 constexpr int BM = 256, BN = 256, BKB = 128;           // tile; K slice in bytes
 constexpr int THREADS = 256;
@@ -127,17 +129,19 @@ struct Frags {
 template <int JT, int NWN, int SLOTS, int IT, class Acc, class Epilogue>
 __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, uint16_t* __restrict__ y, int64_t M, int64_t N,
                                            int64_t m0, int64_t n0, int8_t* lds, int slot, bool active) {
-  static_assert(IT % 4 == 0, "waves cover whole groups of 128 rows");
+  static_assert(IT < 4 || IT % 4 == 0, "waves cover whole groups of 128 rows, or fewer rows than that");
+  constexpr int RT = IT < 4 ? IT : 4, ROWS = 32 * RT;  // row tiles and rows of one pass
+  constexpr int kOut = ROWS * kOutRow;                 // a wave's staging
   constexpr int WCOLS = 32 * JT;
   constexpr int HC = JT >= 2 ? 2 : 1;                  // column tiles staged at a time: 64 or 32 columns
   const int lane = threadIdx.x & 63;
   const int wm = slot / NWN, wn = slot % NWN;
   const int frow = lane & 31, fhalf = lane >> 5;
   __syncthreads();                                     // every wave is done with the operand stages
-  epi.setup(lds + SLOTS * kOutWave, m0, M, n0, N);
+  epi.setup(lds + SLOTS * kOut, m0, M, n0, N);
   __syncthreads();
   if (!active) return;
-  int8_t* out = lds + slot * kOutWave;
+  int8_t* out = lds + slot * kOut;
   const bool vec_ok = (N % 8 == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
   // all rows of the workgroup's tile lie inside y (the rows of all SLOTS / NWN wave rows)
   const bool rows_inside = vec_ok && m0 + (SLOTS / NWN) * (32 * IT) <= M;
@@ -145,14 +149,14 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
   auto pass = [&](auto hcp, int ib, int jt0) {
     constexpr int HCP = decltype(hcp)::value;
     constexpr int CHUNKS = HCP * 4;                    // 16-byte chunks per staged row
-    const int wrow = wm * (32 * IT) + ib * 128;         // first row of this pass inside the workgroup's tile
+    const int wrow = wm * (32 * IT) + ib * ROWS;        // first row of this pass inside the workgroup's tile
     const int64_t pcol = n0 + wn * WCOLS + jt0 * 32;    // first column of this pass
     if (pcol >= N) return;                             // a tile that hangs over the last column: nothing to store
     const bool inside = rows_inside && pcol + 32 * HCP <= N;
     // what the epilogue needs per column (the same for every row of the pass) is fetched once, before the rows
     epi.template columns<HCP>(wn * WCOLS + jt0 * 32 + fhalf * 4);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < RT; ++i) {
       const int lrow = i * 32 + frow;
       epi.row(wrow + lrow);
 #pragma unroll
@@ -161,7 +165,7 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
         for (int q = 0; q < 4; ++q) {
           const int lcol = jj * 32 + q * 8 + fhalf * 4;  // columns lcol .. lcol+3 of this group <-> r = 4q .. 4q+3
           uint32_t words[2];                             // four 16-bit outputs, the first in the low half of words[0]
-          epi.convert4(acc[ib * 4 + i][jt0 + jj], q, jj, words);
+          epi.convert4(acc[ib * RT + i][jt0 + jj], q, jj, words);
           u32x2 packed;
           packed[0] = words[0];
           packed[1] = words[1];
@@ -176,22 +180,28 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
       uint16_t* dst = y + (m0 + wrow + r0) * N + (n0 + wn * WCOLS + jt0 * 32 + ch * 8);
       const int64_t step = int64_t(64 / CHUNKS) * N;
 #pragma unroll
-      for (int it = 0; it < 128 * CHUNKS / 64; ++it) {
+      for (int it = 0; it < ROWS * CHUNKS / 64; ++it) {
         const u32x4 v = *reinterpret_cast<const u32x4*>(out + (it * (64 / CHUNKS) + r0) * kOutRow + ch * 16);
         __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(dst));
         dst += step;
       }
       return;
     }
+    // The last row or column tile, or rows that do not start on 16 bytes (N % 8 != 0).  Whole chunks go out as 16-byte stores at
+    // element alignment, ordinary ones, so that the pieces of a cache line meet in L2; one element at a time the launch was
+    // bound by these stores (int8 M = 2792, K = 2816, N = 6020: 79 us, 42 for N = 6016).
+    const int ch = lane % CHUNKS;
+    const int64_t col = pcol + ch * 8;
+    if (col >= N) return;
+    const bool whole = col + 8 <= N;
 #pragma unroll
-    for (int it = 0; it < 128 * CHUNKS / 64; ++it) {
-      const int lrow = it * (64 / CHUNKS) + lane / CHUNKS, ch = lane % CHUNKS;
+    for (int it = 0; it < ROWS * CHUNKS / 64; ++it) {
+      const int lrow = it * (64 / CHUNKS) + lane / CHUNKS;
       const int64_t row = m0 + wrow + lrow;
-      const int64_t col = n0 + wn * WCOLS + jt0 * 32 + ch * 8;
       const u32x4 v = *reinterpret_cast<const u32x4*>(out + lrow * kOutRow + ch * 16);
       if (row < M) {
-        if (vec_ok) {
-          if (col < N) __builtin_nontemporal_store(v, reinterpret_cast<u32x4*>(y + row * N + col));
+        if (whole) {
+          *reinterpret_cast<u32x4_halves*>(y + row * N + col) = v;
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
@@ -201,7 +211,7 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
     }
   };
 #pragma unroll
-  for (int ib = 0; ib < IT / 4; ++ib) {
+  for (int ib = 0; ib < IT / RT; ++ib) {
 #pragma unroll
     for (int half = 0; half < JT / HC; ++half) pass(IntC<HC>{}, ib, half * HC);
     if constexpr (JT % HC != 0) pass(IntC<1>{}, ib, JT - 1);   // an odd tile left over: 32 columns
@@ -235,6 +245,8 @@ __device__ __forceinline__ void write_tile_f32(Acc (&acc)[4][JT], Epilogue& epi,
         if (vec_ok && col + 3 < N) {
           const f32x4 t = {v[0], v[1], v[2], v[3]};
           __builtin_nontemporal_store(t, reinterpret_cast<f32x4*>(y + row * N + col));
+        } else if (col + 3 < N) {                      // rows that do not start on 16 bytes
+          *reinterpret_cast<f32x4_words*>(y + row * N + col) = (f32x4){v[0], v[1], v[2], v[3]};
         } else {
 #pragma unroll
           for (int e = 0; e < 4; ++e)
@@ -375,13 +387,8 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 // (Tile counts fit 32 bits: the index arithmetic is 32-bit on purpose.  As 64-bit divisions, which the hardware does
 // not have, it was some 500 scalar instructions, over a microsecond, in front of the first load of every workgroup.)
 __device__ __host__ __forceinline__ int64_t even_blocks(int64_t tiles) { return 8 * ((tiles + 7) / 8); }
-__device__ __forceinline__ bool tile_of_even(uint32_t id, uint32_t nblocks, int64_t tiles_m64, int64_t panels64, int64_t group64,
-                                             int64_t& tile_m, int64_t& panel) {
-  const uint32_t tiles_m = uint32_t(tiles_m64), panels = uint32_t(panels64);
-  const uint32_t group = uint32_t(group64) < tiles_m ? uint32_t(group64) : tiles_m;
-  const uint32_t per = nblocks >> 3;
-  const uint32_t at = (id & 7) * per + (id >> 3);
-  if (at >= tiles_m * panels) return false;
+__device__ __forceinline__ void tile_at(uint32_t at, uint32_t tiles_m, uint32_t panels, uint32_t group, int64_t& tile_m, int64_t& panel) {
+  group = group < tiles_m ? group : tiles_m;
   const uint32_t per_group = panels * group;
   const uint32_t full = tiles_m / group;                 // whole groups; a last group holds the remainder
   uint32_t g = at / per_group, r, size;
@@ -396,6 +403,13 @@ __device__ __forceinline__ bool tile_of_even(uint32_t id, uint32_t nblocks, int6
   const uint32_t q = r / size;
   panel = q;
   tile_m = g * group + (r - q * size);
+}
+__device__ __forceinline__ bool tile_of_even(uint32_t id, uint32_t nblocks, int64_t tiles_m64, int64_t panels64, int64_t group64,
+                                             int64_t& tile_m, int64_t& panel) {
+  const uint32_t tiles_m = uint32_t(tiles_m64), panels = uint32_t(panels64);
+  const uint32_t at = (id & 7) * (nblocks >> 3) + (id >> 3);
+  if (at >= tiles_m * panels) return false;
+  tile_at(at, tiles_m, panels, uint32_t(group64), tile_m, panel);
   return true;
 }
 
@@ -416,8 +430,6 @@ namespace edge {
 constexpr int kTile = 128, kStep = 128, kPitch = 144;
 constexpr int kLdsBytes = 2 * kTile * kPitch;
 typedef u32x4 u32x4_bytes __attribute__((aligned(1)));
-typedef u32x4 u32x4_halves __attribute__((aligned(2)));
-typedef f32x4 f32x4_words __attribute__((aligned(4)));
 
 // A 16-byte chunk that lies wholly inside its row; zeros otherwise (rows past the last one, the chunk that straddles
 // the end of a row: see finish_chunk).  No loop in here: the callers' loads stay in flight together.

@@ -12,7 +12,7 @@
 // instead (mtrt_gemm_dense_mfma_*): both operands are K-contiguous per row, which is the form the shared tile
 // loop of gemm_core.hpp takes (both panels through LDS, 256 x 256 tiles, v_mfma_f32_32x32x16_{f16,bf16}; a
 // product of two 16-bit floats is exact in f32), with the bias added to the f32 sum before the one narrowing.
-#include "gemm_core.hpp"
+#include "gemm_frag.hpp"
 
 using namespace mtrt_dev;
 
@@ -88,6 +88,9 @@ template <> struct HalfTraits<F16> {
     ua.i = a; ub.i = b;
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(ua.h, ub.h, c, 0, 0, 0);
   }
+  // accumulators in ordinary vector registers (gemm_frag::run_wide)
+  static __device__ __forceinline__ void mfma_vgpr(v4i a, v4i b, Acc& c) { __asm__ volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
+  static __device__ __forceinline__ void clear_vgpr(v4i a, v4i b, Acc& c) { __asm__ volatile("v_mfma_f32_32x32x16_f16 %0, %1, %2, 0" : "=v"(c) : "v"(a), "v"(b)); }
 };
 template <> struct HalfTraits<BF16> {
   using Acc = v16f;
@@ -98,6 +101,8 @@ template <> struct HalfTraits<BF16> {
     ua.i = a; ub.i = b;
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(ua.h, ub.h, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ void mfma_vgpr(v4i a, v4i b, Acc& c) { __asm__ volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b)); }
+  static __device__ __forceinline__ void clear_vgpr(v4i a, v4i b, Acc& c) { __asm__ volatile("v_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=v"(c) : "v"(a), "v"(b)); }
 };
 
 // f32 operands: a 16-byte fragment holds four k values per lane, and v_mfma_f32_32x32x2_f32 takes one per lane (the two

@@ -35,19 +35,13 @@ namespace tuning {
 // K loop.  int8: M = 16, K = 4096, N = 11008 32.7 us; M = 1, K = N = 4096 27.6 us; M = 32, K = N = 8192 57.1 us
 // (8 + 0.006 * 4096 = 32.6, 8 + 0.006 * 8192 = 57.2).
 constexpr double kTileFixedUs = 8.0, kTileUsPerRowByte = 0.006;
-// Tile loop on fragment-order int8 weights (weights straight into registers), per round: M = 64 at (K, N) =
-// (4096, 4096) 21.0 us, (4096, 11008) 23.2 us, (8192, 8192) 38.4 us; never below streaming the weights at 4.5 TB/s
-// ((11008, 4096) 34.1 us for 45 MB + the fixed part).
-constexpr double kFragTileFixedUs = 5.0, kFragTileUsPerK = 0.004, kFragTileBytesPerUs = 4.5e6;
 // Wave-private kernels that read the weights once (gemm_core::rows32), up to 64 rows: a fixed part plus the weight
 // bytes at the rate the kernel streams them.  [N,K] int8 weights 3.4 TB/s (M = 16, K = 4096, N = 11008 13.0 us;
-// M = 32, K = N = 8192 18.2 us); f16 / bf16 / f32 [N,K] weights and fragment-order int8 weights 4.0 TB/s
-// (dense f16 M = 16, K = 4096, N = 11008 23.4 us; fragment order M = 64 (4096, 4096) 9.3 us, (11008, 4096) 17.1 us).
-constexpr double kRowsFixedUs = 3.0, kRowsBytesPerUs = 3.4e6, kRowsWideBytesPerUs = 4.0e6, kFragRowsFixedUs = 5.0;
+// M = 32, K = N = 8192 18.2 us); f16 / bf16 / f32 [N,K] weights 4.0 TB/s (dense f16 M = 16, K = 4096, N = 11008 23.4 us).
+constexpr double kRowsFixedUs = 3.0, kRowsBytesPerUs = 3.4e6, kRowsWideBytesPerUs = 4.0e6;
 // The same kernels with four row tiles (65 to 128 rows): one workgroup per compute unit at a time, so rounds of 32-column
-// tiles, each the length of its K loop.  [N,K] operands 3.7 ns per row byte (int8 M = 128, K = N = 4096 18.4 us,
-// K = N = 8192 30.7 us); fragment-order weights 3.2 ns per k (16.1 us / 28.1 us at the same shapes).
-constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037, kFragRows128UsPerK = 0.0032;
+// tiles, each the length of its K loop: 3.7 ns per row byte (int8 M = 128, K = N = 4096 18.4 us, K = N = 8192 30.7 us).
+constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
 // W4A16 tile choice: a full round of 256 x 256 tiles takes 3.25 times a full round of 128 x 128 tiles (for four times
 // the work), and a last round filled to a fraction f of the units takes 0.56 + 0.44 f^2 of a full one (fewer units
 // share the power budget).  Fitted over M = 48 ... 4096 at (K, N) = (4096, 4096), (4096, 11008), (11008, 4096),
@@ -62,12 +56,69 @@ constexpr double kW4WideRoundPerBigRound = 1.5 * 0.95;
 // start and end; at 15 shapes with M = 300 ... 2048, (K, N) = (4096, 11008), (4096, 4096), (11008, 4096), (8192, 8192),
 // (5120, 13824) the estimate takes the fastest of the four tiles at every one).
 constexpr double kW4Mid256RoundPerSmallRound = 1.9;
-// W8A8 on fragment-order weights: a round of 256 x 384 tiles, in rounds of 256 x 256 tiles.  One and a half times the
-// MFMAs at 0.9 of the time per MFMA (K = 4096, N = 11008, the benchmark's data, both kernels in one process: M = 2048,
-// one round against one and a half, 77.9 against 83.5 us; M = 4096, two against three, 158 / 165; M = 8192, four
-// against five and a half, 321 / 338; M = 3072, two against two and a half, 137 / 135).
-constexpr double kW8WideRoundPerRound = 1.5 * 0.9;
+// Tiles on fragment-order weights (gemm_frag.hpp).  A launch of `tiles * splits` workgroups, L = ceil of that over the
+// compute units, each running s = slices / splits slices of 128 bytes of K, is estimated as
+//   max(first + first_slice * s, L * (next + next_slice * s)) + (splits > 1 ? meet + meet_each * splits : 0)   us.
+// Fitted to 8500 launches (int8 and f16, 220 log-uniform shapes each: M 17 ... 4096, K 256 ... 14336, N 64 ... 16384, every
+// tile, 1 to 8 splits); the tile and split the estimate takes are within 1.1 % of the fastest ones in the geometric mean
+// and within 22 % at worst.  int8 and the 16-bit types move the same bytes per slice and share the constants.
+struct FragTile {
+  const char *suffix;                                  // of the kernel's name
+  int rows, columns;
+  bool splits;                                         // whether its K may be split
+  double first, first_slice, next, next_slice, meet, meet_each;
+};
+constexpr FragTile kFragTiles[] = {
+    {"t32x128", 32, 128, true, 3.16, 0.144, 1.86, 0.206, 1.65, 0.456},
+    {"t64x128", 64, 128, true, 3.99, 0.128, 2.82, 0.243, 2.48, 0.70},
+    {"t128x128", 128, 128, true, 4.54, 0.20, 3.61, 0.359, 3.8, 1.03},
+    {"t128x256", 128, 256, true, 6.9, 0.127, 6.13, 0.51, 5.14, 1.55},
+    {"t128x384", 128, 384, true, 2.82, 0.78, 8.22, 0.724, 6.9, 2.2},
+    {"t256x256", 256, 256, false, 11.0, 0.25, 8.63, 0.912, 0.0, 0.0},
+    {"t256x384", 256, 384, false, 12.3, 0.764, 9.99, 1.346, 0.0, 0.0},
+};
+// The wave-private kernels up to 32 and 64 rows on the same weights (gemm_core::rows32): L = ceil of their 32-column tiles
+// over the compute units; int8 M = 16, K = N = 4096 5.7 us, (32, 3968, 11328) 13.2; M = 64, K = N = 4096 8.5, (54, 12032, 8682) 32.6.
+constexpr double kFragRows32Us = 2.0, kFragRows32TileUs = 1.2, kFragRows32SliceUs = 0.08, kFragRows32LaterSliceUs = 0.13;
+constexpr double kFragRows64Us = 1.6, kFragRows64TileUs = 1.9, kFragRows64SliceUs = 0.165;
 } // namespace tuning
+
+// The tile and the K split of a GEMM on fragment-order weights (see tuning::kFragTiles).
+struct FragPlan {
+  const tuning::FragTile *tile = nullptr;
+  int64_t tiles = 0;
+  uint32_t splits = 1;
+  double us = 0.0;
+  uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(splits) + 7) / 8)); }
+  int64_t workspace() const { return splits > 1 ? tiles * int64_t(splits) * tile->rows * tile->columns * 4 : 0; }
+};
+FragPlan frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may_split) {
+  static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
+  FragPlan best;
+  for (const tuning::FragTile &t : tuning::kFragTiles) {
+    const int64_t tiles = ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns);
+    if (tiles > int64_t(kMaxGrid) * 1024 - 8)
+      continue;
+    for (int splits : kSplits) {
+      // a part of at least two slices, a ticket for every split tile, and no more workgroups than two rounds hold
+      if (splits > 1 && (!may_split || !t.splits || slices < 2 * splits || tiles > int64_t(kTickets) || tiles * splits > 2 * units))
+        break;
+      const double s = double((slices + splits - 1) / splits), rounds = double((tiles * splits + units - 1) / units);
+      const double us = std::max(t.first + t.first_slice * s, rounds * (t.next + t.next_slice * s)) +
+                        (splits > 1 ? t.meet + t.meet_each * splits : 0.0);
+      if (!best.tile || us < best.us)
+        best = {&t, tiles, uint32_t(splits), us};
+    }
+  }
+  return best;
+}
+double frag_rows_us(int64_t M, int64_t N, int64_t slices, int64_t units) {
+  using namespace tuning;
+  const double rounds = double(((N + 31) / 32 + units - 1) / units), s = double(slices);
+  if (M <= 32)
+    return kFragRows32Us + rounds * (kFragRows32TileUs + s * (rounds > 1.0 ? kFragRows32LaterSliceUs : kFragRows32SliceUs));
+  return kFragRows64Us + rounds * (kFragRows64TileUs + s * kFragRows64SliceUs);
+}
 
 const char *float_name(int32_t dt) {
   switch (dt) {
@@ -890,8 +941,11 @@ int32_t mtrt_hip_gemm_w8a8(mtrt_stream_t stream, const void *a, const void *w_nk
     // Any other K or alignment still goes to the matrix cores: 128 x 128 tiles with byte-aligned loads and a
     // zero-padded last k-step (M=4096 K=4100 N=11008: 1.2 s on the one-element-per-lane kernel below).
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
+    uint32_t a_step = 1;
+    const void *bias = nullptr;
+    void *edge_args[] = {&a, &w_nk, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
     return launch(st, KernelName("mtrt_gemm_w8a8_nk_edge"), uint32_t(std::min<int64_t>(tiles, int64_t(kMaxGrid) * 1024)), kBlock,
-                  as_hip(stream), args);
+                  as_hip(stream), edge_args);
   }
   return launch(st, KernelName("mtrt_gemm_w8a8_nk_any"), blocks_for(M * N, kBlock), kBlock, as_hip(stream), args);
 }
@@ -920,9 +974,28 @@ int32_t mtrt_hip_gemm_w8a8_prepack_fragments(mtrt_stream_t stream, const void *w
   return launch(st, KernelName("mtrt_w8_prepack_frag"), blocks_for(chunks, kBlock), kBlock, as_hip(stream), args);
 }
 
-int32_t mtrt_hip_gemm_w8a8_fragments(mtrt_stream_t stream, const void *a, const void *w_frag, const float *a_scale,
-                                     const float *w_scale, void *y, int64_t M, int64_t K, int64_t N) {
-  clear_error();
+namespace {
+// Which kernel a W8A8 call on fragment-order weights takes.  Up to 32 rows: the kernels bound by reading the weights once
+// (17 to 32 rows, and fewer when at most half of the compute units would get a 32-column tile, the wave-private kernel with
+// eight waves splitting K: M = 32 at (K, N) = (11008, 4096) 18.6 -> 12.9 us, M = 16 there 15.1 -> 11.7; with more tiles and
+// up to 16 rows the four-wave kernel with its hand-counted waits: M = 1 at (4096, 11008) 10.7 against 12.5 us).
+// 33 to 64 rows: the wave-private kernel or a tile, by estimate.  Above: the tile and K split frag_plan estimates fastest.
+struct W8Plan {
+  enum { kSmall16, kRows, kTile } kind;
+  FragPlan tile;
+};
+W8Plan w8_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
+  if (M <= 32)
+    return {M > 16 || 2 * ((N + 31) / 32) <= units ? W8Plan::kRows : W8Plan::kSmall16, {}};
+  const FragPlan tile = frag_plan(M, N, K / 128, units, may_split);
+  if (M <= 64 && frag_rows_us(M, N, K / 128, units) < tile.us)
+    return {W8Plan::kRows, {}};
+  return {W8Plan::kTile, tile};
+}
+
+// a_step: 1 for a scale per row, 0 for one scale; bias: f16 [N] or null; workspace: for K-split tiles, may be null.
+int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, const float *a_scale, uint32_t a_step, const float *w_scale,
+                       const void *bias, void *y, int64_t M, int64_t K, int64_t N, void *workspace, int64_t workspace_bytes) {
   if (M < 0 || K <= 0 || N < 0 || K % 128 != 0)
     return set_error(MTRT_INVALID_ARGUMENT, "fragment-order GEMM needs K %% 128 == 0 and non-negative extents, got M=%lld K=%lld N=%lld",
                      (long long)M, (long long)K, (long long)N);
@@ -933,78 +1006,78 @@ int32_t mtrt_hip_gemm_w8a8_fragments(mtrt_stream_t stream, const void *a, const 
     return MTRT_OK;
   if (!a || !w_frag || !a_scale || !w_scale || !y)
     return set_error(MTRT_INVALID_ARGUMENT, "null operand");
-  if (!aligned(y, 2) || !aligned(a, 16) || !aligned(w_frag, 16))
-    return set_error(MTRT_INVALID_ARGUMENT, "a and w_frag must be 16-byte aligned, y 2-byte aligned");
+  if (!aligned(y, 2) || !aligned(a, 16) || !aligned(w_frag, 16) || !aligned(bias, 2))
+    return set_error(MTRT_INVALID_ARGUMENT, "a and w_frag must be 16-byte aligned, y and bias 2-byte aligned");
   if (M * K >= (int64_t(1) << 32))
     return set_error(MTRT_INVALID_ARGUMENT, "activations of %lld bytes exceed the kernel's 32-bit offsets", (long long)(M * K));
   DeviceState *st = device_state();
   if (!st)
     return MTRT_RUNTIME_ERROR;
-  if (M > 32 && M <= 128) {
-    // 33 to 128 rows: a tile launch lasts one 256-row tile's whole K loop per round (about 5 us + 4 ns per k, and no less
-    // than reading the weights at 4.5 TB/s) and is mostly padding.  The wave-private kernels of gemm_core::rows32 with the
-    // weight fragments straight into registers read the weights once with two (up to 64 rows) or four row tiles per
-    // fragment: 64 rows about 5 us + 1 us per 4 MB of weights (K = N = 4096: 17.1 -> 10.2 us, K = 11008, N = 4096
-    // 34.1 -> 17.5, K = N = 8192 29.3 -> 19.0), 128 rows one workgroup per compute unit at a time, rounds of about
-    // 3.2 ns per k (K = N = 4096: 21.6 -> 16.0 us, K = N = 8192 38.0 -> 27.1; N = 11008 needs two rounds, 30.5 us, and
-    // stays on the tiles at 23.9).
-    const int64_t tiles32 = (N + 31) / 32, units = num_compute_units(st);
-    const double weights = double(N) * double(K);
-    const double tile_us = std::max(tuning::kFragTileFixedUs + tuning::kFragTileUsPerK * double(K), weights / tuning::kFragTileBytesPerUs) *
-                           double(((N + 255) / 256 + units - 1) / units);
-    const double rows_us = M <= 64 ? tuning::kFragRowsFixedUs + weights / tuning::kRowsWideBytesPerUs
-                                   : tuning::kRows128FixedUs + tuning::kFragRows128UsPerK * double(K) * double((tiles32 + units - 1) / units);
-    if (rows_us < tile_us) {
-      void *rargs[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N};
-      return launch(st, KernelName(M <= 64 ? "mtrt_gemm_w8a8_frag_rows64" : "mtrt_gemm_w8a8_frag_rows128"),
-                    uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), M <= 64 ? 512 : 256, as_hip(stream), rargs);
-    }
-  }
-  if (M <= 32 && (M > 16 || 2 * ((N + 31) / 32) <= int64_t(num_compute_units(st)))) {
-    // 17 to 32 rows, and fewer rows when at most half of the compute units would get a 32-column tile: the wave-private
-    // kernel, eight waves splitting K (M = 32 at (K, N) = (11008, 4096) 18.6 -> 12.9 us, (4096, 11008) 14.3 -> 13.5,
-    // (8192, 8192) 15.8 -> 14.9; M = 16 at (11008, 4096) 15.1 -> 11.7).  With more tiles and up to 16 rows the
-    // four-wave kernel below with its hand-counted waits stays ahead (M = 1 at (4096, 11008): 10.7 against 12.5 us).
-    const int64_t tiles32 = (N + 31) / 32;
-    void *rargs[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N};
-    return launch(st, KernelName("mtrt_gemm_w8a8_frag_rows32"), uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), 512,
-                  as_hip(stream), rargs);
-  }
-  if (M <= 16) {
+  const int64_t units = num_compute_units(st), tiles32 = (N + 31) / 32;
+  W8Plan plan = w8_plan(M, K, N, units, true);
+  if (plan.kind == W8Plan::kTile && plan.tile.workspace() > (workspace && aligned(workspace, 16) ? workspace_bytes : 0))
+    plan = w8_plan(M, K, N, units, false);
+  if (plan.kind == W8Plan::kSmall16) {
     // one workgroup per 32-column tile, its four waves splitting K; between one and two tiles per compute unit one
     // workgroup per unit instead, the first ones taking a second tile (as for the int4 weights)
-    const int64_t tiles32 = (N + 31) / 32, cus = num_compute_units(st);
-    const uint32_t grid = uint32_t(M > 8 && tiles32 > cus && tiles32 <= 2 * cus ? cus : tiles32);
-    void *sargs[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N};
-    return launch(st, KernelName("mtrt_gemm_w8a8_small16"), grid, kBlock, as_hip(stream), sargs);
+    const uint32_t grid = uint32_t(M > 8 && tiles32 > units && tiles32 <= 2 * units ? units : tiles32);
+    void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
+    return launch(st, KernelName("mtrt_gemm_w8a8_small16"), grid, kBlock, stream, args);
   }
-  // Tiles and rounds as in mtrt_hip_gemm_w8a8: 256 x 256, one workgroup per compute unit at a time;
-  // a last round that would use at most half of the units is cut into 128-wide half tiles.
-  const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256, units = num_compute_units(st);
-  const int64_t tiles = panels * tiles_m, rest = tiles % units;
-  {
-    // ... or 256 x 384 tiles (fewer bytes moved per MFMA, every weight fragment loaded once per workgroup) where their
-    // rounds come out shorter
-    const double rounds = tiles * 2 <= units ? 0.5 : double(tiles / units) + (rest == 0 ? 0.0 : rest * 2 <= units ? 0.5 : 1.0);
-    const int64_t wide_tiles = ((N + 383) / 384) * tiles_m;
-    const double wide_rounds = tuning::kW8WideRoundPerRound * double((wide_tiles + units - 1) / units);
-    const int64_t wide_grid = 8 * ((wide_tiles + 7) / 8);
-    if (wide_rounds < rounds && wide_grid <= int64_t(kMaxGrid) * 1024) {
-      void *wargs[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N};
-      return launch(st, KernelName("mtrt_gemm_w8a8_frag_t256x384"), uint32_t(wide_grid), 256, as_hip(stream), wargs);
-    }
+  if (plan.kind == W8Plan::kRows) {
+    void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
+    return launch(st, KernelName(M <= 32 ? "mtrt_gemm_w8a8_frag_rows32" : "mtrt_gemm_w8a8_frag_rows64"),
+                  uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), 512, stream, args);
   }
-  int64_t full_panels = panels;
-  if (tiles * 2 <= units)
-    full_panels = 0;
-  else if (rest > 0 && rest * 2 <= units)
-    full_panels = panels - (rest + tiles_m - 1) / tiles_m;
-  const int64_t half_panels = (N - full_panels * 256 + 127) / 128;
-  const int64_t grid = 8 * ((full_panels * tiles_m + 7) / 8) + 8 * ((half_panels * tiles_m + 7) / 8);   // each kind dealt evenly to the XCDs
-  if (grid > int64_t(kMaxGrid) * 1024)
+  const FragPlan &p = plan.tile;
+  if (!p.tile)
     return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
-  void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &full_panels};
-  return launch(st, KernelName("mtrt_gemm_w8a8_frag"), uint32_t(grid), 256, as_hip(stream), args);
+  if (p.tile->rows == 256 && p.tile->columns == 384) {
+    void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
+    const bool plain = a_step == 1 && !bias;
+    return launch(st, KernelName(plain ? "mtrt_gemm_w8a8_frag_t256x384" : "mtrt_gemm_w8a8_frag_t256x384_linear").as("mtrt_gemm_w8a8_frag_t256x384"),
+                  p.grid(), 256, stream, args);
+  }
+  uint32_t splits = p.splits;
+  uint32_t *tickets = nullptr;
+  if (splits > 1) {
+    tickets = reduction_slot(st, stream);
+    if (!tickets)
+      return MTRT_RUNTIME_ERROR;
+    tickets += kTicketOffset;
+  }
+  KernelName name("mtrt_gemm_w8a8_frag");
+  if (p.tile->rows == 32)
+    name + "_rows128";
+  else if (p.tile->rows != 64)
+    name + "_" + p.tile->suffix;
+  void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &splits, &workspace, &tickets, &a_step, &bias};
+  return launch(st, name.as(p.tile->rows == 32 && M > 64 && M <= 128 ? "mtrt_gemm_w8a8_frag_rows128" : "mtrt_gemm_w8a8_frag"), p.grid(), 256,
+                stream, args);
+}
+} // namespace
+
+int32_t mtrt_hip_gemm_w8a8_fragments(mtrt_stream_t stream, const void *a, const void *w_frag, const float *a_scale,
+                                     const float *w_scale, void *y, int64_t M, int64_t K, int64_t N) {
+  clear_error();
+  return w8a8_fragments(as_hip(stream), a, w_frag, a_scale, 1, w_scale, nullptr, y, M, K, N, nullptr, 0);
+}
+
+int64_t mtrt_hip_gemm_w8a8_fragments_workspace(int64_t M, int64_t K, int64_t N) {
+  if (M <= 32 || K <= 0 || N <= 0 || M > kMaxMatrixExtent || K > kMaxMatrixExtent || N > kMaxMatrixExtent)
+    return 0;
+  DeviceState *st = device_state();
+  if (!st)
+    return 0;
+  const W8Plan plan = w8_plan(M, K, N, num_compute_units(st), true);
+  return plan.kind == W8Plan::kTile && plan.tile.tile ? plan.tile.workspace() : 0;
+}
+
+int32_t mtrt_hip_gemm_w8a8_fragments_ws(mtrt_stream_t stream, const void *a, const void *w_frag, const float *a_scale,
+                                        const float *w_scale, void *y, int64_t M, int64_t K, int64_t N, void *workspace,
+                                        int64_t workspace_bytes) {
+  clear_error();
+  return w8a8_fragments(as_hip(stream), a, w_frag, a_scale, 1, w_scale, nullptr, y, M, K, N, workspace, workspace_bytes);
 }
 
 int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w_nk, const void *bias, void *y,

@@ -79,9 +79,10 @@ struct DeviceState {
   std::unordered_map<std::string, hipFunction_t> funcs;
   // One block per stream for single-launch grid reductions, zero when a stream first uses it: 33 lines of
   // 128 bytes for the arrival tree (root + 32 first-level groups, see amax.hip), which the kernels return to
-  // zero, and 18 for the tagged slots and counters of dynq.hip, which never need clearing; rounded up to 64.
+  // zero, and 18 for the tagged slots and counters of dynq.hip, which never need clearing; rounded up to 64; behind
+  // them the tickets of the K-split GEMM tiles (gemm_frag.hpp), which the kernels return to zero.
   static constexpr int kSlots = 256;
-  static constexpr int kSlotWords = 64 * 32;
+  static constexpr int kSlotWords = kTicketOffset + kTickets;
   uint32_t *slots = nullptr;
   // The stream -> block mapping has a mutex of its own (slot_mu), which reduction_slot holds across the launch of
   // a fresh block's clear; that launch may take `mu` to resolve the fill kernel.  Order: slot_mu, then mu.
@@ -314,10 +315,10 @@ int32_t launch(DeviceState *st, const KernelName &kernel, uint32_t grid, uint32_
     return set_error(MTRT_DRIVER_ERROR, "launching '%s' grid %u block %u: %s", kernel.text, grid, block,
                      hipGetErrorString(e));
   }
-  if (hit) {
+  if (hit && !kernel.shown[0]) {
     tl_kernel_ptr = hit->name;
   } else {
-    std::snprintf(tl_kernel, sizeof(tl_kernel), "%s", kernel.text);
+    std::snprintf(tl_kernel, sizeof(tl_kernel), "%s", kernel.shown[0] ? kernel.shown : kernel.text);
     tl_kernel_ptr = tl_kernel;
   }
   return MTRT_OK;

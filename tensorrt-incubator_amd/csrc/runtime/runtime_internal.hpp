@@ -37,6 +37,8 @@ hipModule_t builtin_module(DeviceState *);
 int num_compute_units(DeviceState *);
 hipFunction_t find_kernel(DeviceState *, const std::string &name);   // nullptr + set_error
 uint32_t *reduction_slot(DeviceState *, hipStream_t stream);         // nullptr + set_error
+// The tickets of K-split GEMM tiles inside a stream's reduction block: one zero word per tile, returned to zero by the launch.
+constexpr uint32_t kTicketOffset = 64 * 32, kTickets = 512;          // in 32-bit words
 int32_t reset_reduction_slot(DeviceState *, hipStream_t stream);     // stream-ordered clear of the stream's block
 void forget_stream(hipStream_t stream);                              // before a stream is destroyed
 
@@ -47,8 +49,14 @@ int32_t no_alloc_setup(DeviceState *, int device);
 // A kernel name put together on the stack (no heap, no locale): KernelName("mtrt_q_") + kind + "_" + x.
 struct KernelName {
   char text[72];
+  char shown[72];                                      // what mtrt_hip_last_kernel reports, when not `text`
   uint32_t len = 0;
-  KernelName(const char *s) { text[0] = '\0'; *this + s; }
+  KernelName(const char *s) { text[0] = shown[0] = '\0'; *this + s; }
+  // Reported under another name: the tiles of one GEMM go by the name of the class of shapes they serve.
+  KernelName &as(const KernelName &name) {
+    __builtin_memcpy(shown, name.text, sizeof(shown));
+    return *this;
+  }
   KernelName &operator+(const char *s) {
     while (*s && len + 1 < sizeof(text))
       text[len++] = *s++;

@@ -1,0 +1,102 @@
+"""GEMMs whose output tiles are shared by several workgroups along K (gemm_frag.hpp), and the tiles and epilogues around
+them, at the sizes where they can go wrong: one slice per part and uneven parts, ragged rows and columns, row lengths of
+the output that are no whole vectors, a launch repeated on the same tickets, two streams at once, graph replays."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _inputs(seed, M, K, N):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+
+    def q8(shape):
+        return torch.clamp(torch.round(torch.randn(shape, generator=g, device="cuda") * 40), -128, 127).to(torch.int8)
+    return q8((M, K)), q8((K, N)), torch.rand(M, generator=g, device="cuda") * 0.01 + 0.005, torch.rand(N, generator=g, device="cuda") * 3e-4 + 1e-4
+
+
+def _expect(a, w, a_s, w_s):
+    acc = a.double() @ w.double()                      # |sums| < 2^31: exact
+    return ((acc.float() * a_s[:, None]) * w_s[None, :]).half()
+
+
+# (M, K, N): the host's estimate splits K in most of these (few tiles, many slices)
+@pytest.mark.parametrize("shape", [(200, 12288, 512), (33, 2048, 40), (100, 4096, 300), (129, 11520, 257), (398, 11520, 1856), (65, 1152, 129),
+                                   (700, 6528, 200), (1000, 8064, 1000), (256, 8192, 8), (40, 14336, 2051)])
+def test_w8a8_split_tiles_are_exact(pkg, shape):
+    """Integer sums: bit-exact whatever the number of parts, and the same without scratch memory (unsplit)."""
+    import torch
+    M, K, N = shape
+    a, w, a_s, w_s = _inputs(M + K + N, M, K, N)
+    wf = pkg.gemm_w8a8_prepack_fragments(w)
+    expect = _expect(a, w, a_s, w_s)
+    for _ in range(3):                                 # the tickets are back at zero after each launch
+        assert torch.equal(pkg.gemm_w8a8_fragments(a, wf, a_s, w_s, N), expect)
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    L = pkg.lib()
+    stream = torch.cuda.current_stream().cuda_stream
+    pkg.check(L.mtrt_hip_gemm_w8a8_fragments(stream, a.data_ptr(), wf.data_ptr(), a_s.data_ptr(), w_s.data_ptr(), y.data_ptr(), M, K, N))
+    assert torch.equal(y, expect)
+    need = L.mtrt_hip_gemm_w8a8_fragments_workspace(M, K, N)
+    if need:                                           # one byte too few: the unsplit form again
+        scratch = torch.empty(need, dtype=torch.uint8, device="cuda")
+        y.fill_(float("nan"))
+        pkg.check(L.mtrt_hip_gemm_w8a8_fragments_ws(stream, a.data_ptr(), wf.data_ptr(), a_s.data_ptr(), w_s.data_ptr(), y.data_ptr(), M, K, N,
+                                                    scratch.data_ptr(), need - 1))
+        assert torch.equal(y, expect)
+
+
+def test_some_shape_is_split(pkg):
+    L = pkg.lib()
+    assert L.mtrt_hip_gemm_w8a8_fragments_workspace(200, 12288, 512) > 0
+    assert L.mtrt_hip_gemm_w8a8_fragments_workspace(16, 12288, 512) == 0 and L.mtrt_hip_gemm_w8a8_fragments_workspace(200, 128, 512) == 0
+
+
+@pytest.mark.parametrize("N", [8, 12, 129, 1001, 2048 + 6])
+@pytest.mark.parametrize("M", [65, 300, 1100, 2100])
+def test_w8a8_outputs_inside_a_larger_buffer(pkg, M, N):
+    """Row lengths that are no whole 16-byte vectors and outputs off 16-byte alignment, for tiles of every height: the
+    results are exact and nothing around them is written."""
+    import torch
+    K = 256
+    a, w, a_s, w_s = _inputs(M * N, M, K, N)
+    wf = pkg.gemm_w8a8_prepack_fragments(w)
+    buf = torch.full((M * N + 9,), 7.0, dtype=torch.float16, device="cuda")
+    y = buf[1:1 + M * N].view(M, N)
+    pkg.gemm_w8a8_fragments(a, wf, a_s, w_s, N, out=y)
+    assert torch.equal(y, _expect(a, w, a_s, w_s))
+    assert float(buf[0]) == 7.0 and bool((buf[1 + M * N:] == 7.0).all())
+
+
+def test_w8a8_split_launches_on_two_streams_and_in_a_graph(pkg):
+    """Tickets belong to a stream: launches on two streams do not meet; a captured launch gives the eager result on every
+    replay, with eager work between the replays."""
+    import torch
+    cases = [_inputs(k, 200, 12288, 512) for k in range(2)]
+    frag = [pkg.gemm_w8a8_prepack_fragments(w) for _, w, _, _ in cases]
+    expect = [_expect(*c) for c in cases]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    out = [[], []]
+    for _ in range(8):
+        for k, s in enumerate(streams):
+            with torch.cuda.stream(s):
+                a, _, a_s, w_s = cases[k]
+                out[k].append(pkg.gemm_w8a8_fragments(a, frag[k], a_s, w_s, 512))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, expect[k]) for k in range(2) for y in out[k])
+    a, _, a_s, w_s = cases[0]
+    static = a.clone()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        pkg.gemm_w8a8_fragments(static, frag[0], a_s, w_s, 512)      # the stream's block is bound before the capture
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        y = pkg.gemm_w8a8_fragments(static, frag[0], a_s, w_s, 512)
+    for k in range(4):
+        static.copy_(torch.roll(a, k, 0))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, pkg.gemm_w8a8_fragments(static, frag[0], a_s, w_s, 512)), k
