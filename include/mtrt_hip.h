@@ -447,6 +447,36 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const voi
                                                  const void *bias, void *y, int32_t dtype, int64_t M,
                                                  int64_t K, int64_t N);
 
+/* A Linear module in one call: y = Linear(x), x [M,K] and y [M,N] in `dtype`, the activations quantized on the way where the
+ * module says so.  The parameters are re-laid once (w_frag) and described by a plan that the caller keeps; a call is two
+ * launches at most (the activation pass, the GEMM with both scales and the bias in its epilogue), one where x needs no pass.
+ *   MTRT_LINEAR_W8A8  (dtype F16): q = quantize(x, x_scale) to int8; y = f16(f16((f32(q . w) * x_scale) * w_scale[n]) + bias[n]);
+ *                     w: int8 [N,K], w_scale: f32 [N], w_frag: mtrt_hip_linear_prepack_fragments of w
+ *   MTRT_LINEAR_W4A16 (dtype F16): y = f16(f16(x . dequantized w) + bias[n]); w_frag: mtrt_hip_gemm_w4a16_prepack's buffer,
+ *                     w_scale: f16 [1,N] (one block of all of K, K % 64 == 0); w unused
+ *   MTRT_LINEAR_DENSE: x' = q_dtype < 0 ? x : dequantize(quantize(x, x_scale, q_dtype), x_scale); y = narrow(x' . w + bias[n]);
+ *                     w: [N,K] in dtype, w_frag (F16 and BF16): mtrt_hip_linear_prepack_fragments of w, K rounded up to 64
+ * w may be NULL when w_frag is given and K is a multiple of 128 (int8) or 64 (16-bit), w_frag when the shape or type has none.
+ * The results are those of the single calls (quantize, dequantize, the GEMM entry point, an addition in dtype).
+ * `workspace`: mtrt_hip_linear_workspace(plan, M) bytes of device memory, 16-byte aligned, the call's own until its work
+ * on `stream` is done; less is MTRT_INVALID_ARGUMENT. */
+enum mtrt_hip_linear_route { MTRT_LINEAR_W8A8 = 0, MTRT_LINEAR_W4A16 = 1, MTRT_LINEAR_DENSE = 2 };
+typedef struct mtrt_hip_linear_plan {
+  int32_t route, dtype, q_dtype, reserved;
+  int64_t K, N;
+  const void *w, *w_frag, *w_scale;
+  const float *x_scale;
+  const void *bias;
+} mtrt_hip_linear_plan;
+/* Bytes of the fragment order of [N,K] weights of int8 (MTRT_I8), f16 or bf16, K rounded up to whole 128-byte slices with
+ * zeros; 0 for other types. */
+MTRT_CAPI_EXPORTED int64_t mtrt_hip_linear_fragments_bytes(int32_t dtype, int64_t K, int64_t N);
+MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_prepack_fragments(mtrt_stream_t stream, const void *w_nk, int32_t dtype,
+                                                             void *w_frag, int64_t K, int64_t N);
+MTRT_CAPI_EXPORTED int64_t mtrt_hip_linear_workspace(const mtrt_hip_linear_plan *plan, int64_t M);
+MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, const void *x, void *y,
+                                           int64_t M, void *workspace, int64_t workspace_bytes);
+
 /* ------------------------------------------------------------------------- */
 /* Part 3 — the interpreter's builtin set, status-returning                    */
 /* (mlir-tensorrt/executor/lib/Runtime/Backend/Lua/Modules/CUDA/CUDAModule.cpp) */

@@ -117,6 +117,10 @@ PROTOTYPES = {
     "mtrt_hip_gemm_w8a8_fragments_workspace": (_i64, [_i64, _i64, _i64]),
     "mtrt_hip_gemm_w8a8_fragments_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _vp, _i64]),
     "mtrt_hip_linear_dense": (_i32, [_vp, _vp, _vp, _vp, _vp, _i32, _i64, _i64, _i64]),
+    "mtrt_hip_linear_fragments_bytes": (_i64, [_i32, _i64, _i64]),
+    "mtrt_hip_linear_prepack_fragments": (_i32, [_vp, _vp, _i32, _vp, _i64, _i64]),
+    "mtrt_hip_linear_workspace": (_i64, [_vp, _i64]),
+    "mtrt_hip_linear": (_i32, [_vp, _vp, _vp, _vp, _i64, _vp, _i64]),
     "mtrt_hip_gemm_w4a16_prepacked_bytes": (_i64, [_i64, _i64]),
     "mtrt_hip_gemm_w4a16_prepack": (_i32, [_vp, _vp, _vp, _i64, _i64]),
     "mtrt_hip_gemm_w4a16": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64]),

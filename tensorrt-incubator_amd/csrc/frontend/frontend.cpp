@@ -22,6 +22,8 @@
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <memory>
+
 #include "mtrt_hip.h"
 
 namespace {
@@ -838,6 +840,147 @@ PyObject *f_tp_softmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
   FRONTEND_CATCH
 }
 
+// The prepared weight side of a tp.Linear: the operands of mtrt_hip_linear, and the parameter objects and versions they were
+// made from.
+struct LinearPlan {
+  mtrt_hip_linear_plan plan{};
+  at::Tensor w, w_frag, w_scale, x_scale;
+  at::ScalarType type;
+  const TpDtype *dtype;
+  PyObject *owners[3];                                 // weight, weight_scale, input_scale (what the module held)
+  int64_t versions[3];
+  PyObject *options[2];                                // quant_dtype, weight_quant_dim
+};
+constexpr const char *kPlanName = "mtrt_frontend.LinearPlan";
+PyObject *s_weight, *s_weight_scale, *s_input_scale, *s_quant_dtype, *s_quant_dim, *s_native_plan, *s_bias;
+
+int64_t version_of(PyObject *o) {
+  TpTensor t;
+  return t.read(o) ? int64_t(t.t->_version()) : -1;
+}
+
+// linear_plan(module, route, q_dtype or None, K, N, w, w_frag, w_scale, x_scale) -> what tp_linear reads from the module's
+// _native_plan; the tensors are None or lie contiguous on the GPU
+PyObject *f_linear_plan(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  FRONTEND_TRY
+  if (!arity(n, 9, "linear_plan"))
+    return nullptr;
+  auto made = std::make_unique<LinearPlan>();
+  const at::Tensor *t[4];
+  for (int i = 0; i < 4; ++i) {
+    if (!optional_tensor(a[5 + i], &t[i]))
+      return nullptr;
+    if (t[i] && !dense_on_gpu(*t[i]))
+      return fail("a plan's operands must be contiguous and on the GPU"), nullptr;
+  }
+  mtrt_hip_linear_plan &p = made->plan;
+  PyObject *d = PyObject_GetAttr(a[0], s_dtype);
+  made->dtype = d ? tp_dtype(d) : nullptr;
+  Py_XDECREF(d);
+  const TpDtype *q = a[2] == Py_None ? nullptr : tp_dtype(a[2]);
+  if (!integer32(a[1], &p.route) || !integer(a[3], &p.K) || !integer(a[4], &p.N))
+    return nullptr;
+  if (!is_float(made->dtype) || (a[2] != Py_None && !is_code(q)))
+    return fail("a plan needs a float dtype and a quantized one or None"), nullptr;
+  p.dtype = made->dtype->code;
+  p.q_dtype = q ? q->code : -1;
+  made->type = made->dtype->storage;
+  at::Tensor *held[4] = {&made->w, &made->w_frag, &made->w_scale, &made->x_scale};
+  for (int i = 0; i < 4; ++i)
+    if (t[i])
+      *held[i] = *t[i];
+  p.w = t[0] ? t[0]->data_ptr() : nullptr;
+  p.w_frag = t[1] ? t[1]->data_ptr() : nullptr;
+  p.w_scale = t[2] ? t[2]->data_ptr() : nullptr;
+  p.x_scale = t[3] ? static_cast<const float *>(t[3]->data_ptr()) : nullptr;
+  PyObject *const names[5] = {s_weight, s_weight_scale, s_input_scale, s_quant_dtype, s_quant_dim};
+  PyObject *found[5];
+  for (int i = 0; i < 5; ++i)
+    if (!(found[i] = PyObject_GetAttr(a[0], names[i]))) {
+      while (i-- > 0)
+        Py_DECREF(found[i]);
+      return nullptr;
+    }
+  for (int i = 0; i < 3; ++i) {
+    made->owners[i] = found[i];
+    made->versions[i] = version_of(found[i]);
+  }
+  made->options[0] = found[3];
+  made->options[1] = found[4];
+  PyObject *capsule = PyCapsule_New(made.get(), kPlanName, [](PyObject *c) {
+    auto *gone = static_cast<LinearPlan *>(PyCapsule_GetPointer(c, kPlanName));
+    for (PyObject *o : gone->owners)
+      Py_DECREF(o);
+    for (PyObject *o : gone->options)
+      Py_DECREF(o);
+    delete gone;
+  });
+  if (!capsule) {
+    for (PyObject *o : found)
+      Py_DECREF(o);
+    return nullptr;
+  }
+  made.release();
+  return capsule;
+  FRONTEND_CATCH
+}
+
+// tp_linear(module, x): the forward pass when the plan is current, x and the bias lie on the GPU in the module's dtype
+PyObject *f_tp_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
+  FRONTEND_TRY
+  if (!arity(n, 2, "tp_linear"))
+    return nullptr;
+  struct Attr {
+    PyObject *o;
+    Attr(PyObject *of, PyObject *name) : o(PyObject_GetAttr(of, name)) {}
+    ~Attr() { Py_XDECREF(o); }
+  };
+  const Attr capsule(a[0], s_native_plan);
+  const LinearPlan *lp = capsule.o && PyCapsule_IsValid(capsule.o, kPlanName)
+                             ? static_cast<const LinearPlan *>(PyCapsule_GetPointer(capsule.o, kPlanName))
+                             : nullptr;
+  TpTensor x;
+  if (!lp || !x.read(a[1])) {
+    PyErr_Clear();
+    return not_here();
+  }
+  PyObject *const names[5] = {s_weight, s_weight_scale, s_input_scale, s_quant_dtype, s_quant_dim};
+  for (int i = 0; i < 5; ++i) {
+    const Attr now(a[0], names[i]);
+    // options are compared by identity: an equal object that is not the same one takes the general path, which compares values
+    if (now.o != (i < 3 ? lp->owners[i] : lp->options[i - 3]) || (i < 3 && version_of(now.o) != lp->versions[i])) {
+      PyErr_Clear();
+      return not_here();
+    }
+  }
+  const Attr dtype(a[0], s_dtype), bias_object(a[0], s_bias);
+  if (!dtype.o || !bias_object.o) {
+    PyErr_Clear();
+    return not_here();
+  }
+  TpTensor bias;
+  const bool has_bias = bias_object.o != Py_None;
+  mtrt_hip_linear_plan p = lp->plan;
+  if (dtype.o != lp->dtype->object || x.dtype != lp->dtype || !dense_on_gpu(*x.t) || x.t->dim() < 1 || x.t->size(-1) != p.K ||
+      (has_bias && (!bias.read(bias_object.o) || bias.dtype != lp->dtype || !dense_on_gpu(*bias.t) || bias.t->dim() != 1 ||
+                    bias.t->size(0) != p.N)) ||
+      (p.route == MTRT_LINEAR_W4A16 && has_bias) || (p.q_dtype < 0 && reinterpret_cast<uintptr_t>(x.t->data_ptr()) % 16 != 0))
+    return not_here();
+  p.bias = has_bias ? bias.t->data_ptr() : nullptr;
+  c10::SmallVector<int64_t, 6> shape(x.t->sizes().begin(), x.t->sizes().end());
+  shape.back() = p.N;
+  const int64_t M = x.t->numel() / p.K, scratch_bytes = mtrt_hip_linear_workspace(&p, M);
+  const at::Tensor y = empty_like_device(shape, lp->type, *x.t);
+  const at::Tensor scratch = scratch_bytes ? bytes_on(*x.t, scratch_bytes) : at::Tensor();
+  const mtrt_stream_t s = current_stream();
+  if (!launch([&] {
+        return mtrt_hip_linear(s, &p, x.t->data_ptr(), y.data_ptr(), M, scratch_bytes ? scratch.data_ptr() : nullptr, scratch_bytes);
+      }))
+    return nullptr;
+  return produced(y, lp->dtype);
+  FRONTEND_CATCH
+}
+
 // ---- set-up --------------------------------------------------------------------------------------
 PyObject *f_set_error_type(PyObject *, PyObject *type) {
   Py_INCREF(type);
@@ -886,6 +1029,8 @@ PyMethodDef g_methods[] = {
     FAST("tp_dequantize", f_tp_qdq<false>),
     FAST("tp_layernorm", f_tp_layernorm),
     FAST("tp_softmax", f_tp_softmax),
+    FAST("linear_plan", f_linear_plan),
+    FAST("tp_linear", f_tp_linear),
     {"set_error_type", f_set_error_type, METH_O, nullptr},
     FAST("bind_tp", f_bind_tp),
     {nullptr, nullptr, 0, nullptr},
@@ -900,7 +1045,15 @@ PyMODINIT_FUNC PyInit_mtrt_frontend(void) {
   s_constant = PyUnicode_InternFromString("is_cpu_constant");
   s_f32_dev = PyUnicode_InternFromString("_f32_dev");
   g_no_args = PyTuple_New(0);
-  if (!s_t || !s_dtype || !s_constant || !s_f32_dev || !g_no_args)
+  s_weight = PyUnicode_InternFromString("weight");
+  s_weight_scale = PyUnicode_InternFromString("weight_scale");
+  s_input_scale = PyUnicode_InternFromString("input_scale");
+  s_quant_dtype = PyUnicode_InternFromString("quant_dtype");
+  s_quant_dim = PyUnicode_InternFromString("weight_quant_dim");
+  s_native_plan = PyUnicode_InternFromString("_native_plan");
+  s_bias = PyUnicode_InternFromString("bias");
+  if (!s_t || !s_dtype || !s_constant || !s_f32_dev || !g_no_args || !s_weight || !s_weight_scale || !s_input_scale || !s_quant_dtype ||
+      !s_quant_dim || !s_native_plan || !s_bias)
     return nullptr;
   return PyModule_Create(&g_module);
 }

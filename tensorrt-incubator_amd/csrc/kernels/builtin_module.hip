@@ -3,6 +3,7 @@
 #include "amax.hip"
 #include "amax_scales.hip"
 #include "qdq.hip"
+#include "activations.hip"
 #include "dynq.hip"
 #include "dynq_rows.hip"
 #include "nvfp4.hip"

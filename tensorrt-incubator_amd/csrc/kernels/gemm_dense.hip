@@ -135,16 +135,16 @@ template <typename X> __device__ __forceinline__ uint32_t narrow16x2(float lo, f
 template <> __device__ __forceinline__ uint32_t narrow16x2<F16>(float lo, float hi) { return f32x2_to_f16x2_bits(lo, hi); }
 template <> __device__ __forceinline__ uint32_t narrow16x2<BF16>(float lo, float hi) { return f32x2_to_bf16x2_bits(lo, hi); }
 
-// y = narrow(acc + f32(bias[n])) (no addition without a bias, as in the kernel above)
-template <typename X>
+// y = narrow(acc + f32(bias[n])); without a bias zeros are added, which changes no sum (an accumulator that starts at +0
+// is never -0).  BN: columns of the tile (scratch floats)
+template <typename X, int BN = 256>
 struct BiasEpilogue {
   const typename X::storage* bias;
-  const float* sb;                                   // bias of this tile's 256 columns as f32, in LDS
+  const float* sb;                                   // bias of this tile's columns as f32, in LDS
   f32x4 br[2][4];
   __device__ __forceinline__ void setup(int8_t* scratch, int64_t, int64_t, int64_t n0, int64_t N) {
     float* dst = reinterpret_cast<float*>(scratch);
-    const int64_t col = n0 + threadIdx.x;             // 256 threads: 256 columns
-    if (threadIdx.x < 256) dst[threadIdx.x] = (bias && col < N) ? Tile<X>::load1(bias + col) : 0.0f;
+    for (int c = threadIdx.x; c < BN; c += blockDim.x) dst[c] = (bias && n0 + c < N) ? Tile<X>::load1(bias + n0 + c) : 0.0f;
     sb = dst;
   }
   __device__ __forceinline__ void row(int) {}
@@ -157,14 +157,7 @@ struct BiasEpilogue {
   }
   __device__ __forceinline__ void convert4(const v16f& acc, int q, int jj, uint32_t (&words)[2]) const {
 #pragma unroll
-    for (int e = 0; e < 4; e += 2) {
-      float v0 = acc[4 * q + e], v1 = acc[4 * q + e + 1];
-      if (bias) {
-        v0 = v0 + br[jj][q][e];
-        v1 = v1 + br[jj][q][e + 1];
-      }
-      words[e >> 1] = narrow16x2<X>(v0, v1);
-    }
+    for (int e = 0; e < 4; e += 2) words[e >> 1] = narrow16x2<X>(acc[4 * q + e] + br[jj][q][e], acc[4 * q + e + 1] + br[jj][q][e + 1]);
   }
 };
 
@@ -323,6 +316,83 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_rows128_f32(
   }
 MTRT_DENSE_ROWS128_KERNEL(f16, F16)
 MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
+
+// ---- weights in fragment order (gemm_frag.hpp) ---------------------------------------------------------
+// What a module's Linear runs on: its weights are re-laid once per parameter set.  Against the loops above, which bring both
+// operands through LDS in 256-row tiles (f16, us): (M, K, N) = (999, 4096, 11008) 113 -> 83, (2048, 4096, 11008) 197 -> 147,
+// (256, 4096, 4096) 58 -> 16, (398, 11520, 1856) 165 -> 30, (1024, 2048, 2048) 32 -> 12.5, (200, 12288, 512) 164 -> 12.7.
+// mtrt_gemm_dense_frag_<type>_t<rows>x<columns> (x [M,K], w_frag, bias [N] or null, y [M,N], M, K, N, splits, partial, tickets) ;
+// K % 64 == 0, x and w_frag 16-byte aligned, x below 4 GiB; the rest as mtrt_gemm_w8a8_frag.
+#define MTRT_DENSE_FRAG_KERNEL(XN, XT, IT, JT, D, WG, TILE)                                                               \
+  extern "C" __global__ void __launch_bounds__(256, WG) mtrt_gemm_dense_frag_##XN##_##TILE(                               \
+      const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t splits, f32x4* partial, uint32_t* tickets) {    \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<IT, D>(128 * JT)];                            \
+    gemm_frag::Part part;                                                                                                 \
+    if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, K / 64, splits, partial, tickets, part)) return; \
+    dense_cluster::BiasEpilogue<XT, 128 * JT> epi{bias, nullptr, {}};                                                     \
+    gemm_frag::run<dense_cluster::HalfTraits<XT>, IT, JT, D>(x, 2 * K, w_frag, epi, y, M, N, part, lds);                  \
+  }
+// ... 256 x 384 tiles: (x, w_frag, bias, y, M, K, N) ; grid = 8 * ceil(ceil(M/256) * ceil(N/384) / 8), block = 256.
+// ... up to 32 and 64 rows, a wave for itself (gemm_core::rows32): the same arguments; grid: any, block = 512.
+#define MTRT_DENSE_FRAG_KERNELS(XN, XT)                                                                                   \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 1, 1, 4, 2, t32x128)                                                                     \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 2, 1, 4, 2, t64x128)                                                                     \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 1, 2, 2, t128x128)                                                                    \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 2, 2, 1, t128x256)                                                                    \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 3, 2, 1, t128x384)                                                                    \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 8, 2, 2, 1, t256x256)                                                                    \
+  extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_dense_frag_##XN##_t256x384(                              \
+      const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                        \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<8, 2>(gemm_frag::kWideBN)];                   \
+    const int64_t tiles_m = (M + 255) / 256, panels = (N + gemm_frag::kWideBN - 1) / gemm_frag::kWideBN;                  \
+    int64_t tile_m, panel;                                                                                                \
+    if (!gemm_core::tile_of_even(blockIdx.x, gridDim.x, tiles_m, panels, tiles_m, tile_m, panel)) return;                 \
+    dense_cluster::BiasEpilogue<XT, gemm_frag::kWideBN> epi{bias, nullptr, {}};                                           \
+    gemm_frag::run_wide<dense_cluster::HalfTraits<XT>>(x, 2 * K, w_frag, (N + 31) / 32, epi, y, M, N, K / 64, tile_m * 256, \
+                                                       panel * gemm_frag::kWideBN, lds);                                  \
+  }                                                                                                                       \
+  extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##XN##_rows32(                                   \
+      const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                        \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8, 1, true>()];                       \
+    dense_cluster::RowsBiasEpilogue<XT> epi{bias};                                                                        \
+    gemm_core::rows32::run<dense_cluster::HalfTraits<XT>, 8, 1, true>(x, w_frag, 2 * K, epi, y, M, N, lds);               \
+  }                                                                                                                       \
+  extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##XN##_rows64(                                   \
+      const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                        \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8, 2, true>()];                       \
+    dense_cluster::RowsBiasEpilogue<XT> epi{bias};                                                                        \
+    gemm_core::rows32::run<dense_cluster::HalfTraits<XT>, 8, 2, true>(x, w_frag, 2 * K, epi, y, M, N, lds);               \
+  }
+MTRT_DENSE_FRAG_KERNELS(f16, F16)
+MTRT_DENSE_FRAG_KERNELS(bf16, BF16)
+
+// Re-layout of 16-bit weights [N,K] into fragment order, one 16-byte chunk per thread: (w, w_frag, K, N) ; w_frag holds
+// 32 * ceil(N/32) * 128 * ceil(K/64) bytes, zeros where w has no element.
+extern "C" __global__ void __launch_bounds__(256) mtrt_w16_prepack_frag(const uint16_t* __restrict__ w, u32x4* __restrict__ w_frag,
+                                                                      int64_t K, int64_t N) {
+  const int64_t slices = (K + 63) / 64, ntiles = (N + 31) / 32;
+  const int64_t total = ntiles * slices * 256;
+  for (int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; id < total; id += int64_t(gridDim.x) * blockDim.x) {
+    const int lane = int(id & 63), p = int((id >> 6) & 3);
+    const int64_t slice = (id >> 8) % slices, tile = (id >> 8) / slices;
+    const int64_t n = tile * 32 + (lane & 31), k0 = slice * 64 + 16 * p + 8 * (lane >> 5);
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (n < N) {
+      if (k0 + 8 <= K) {
+        v = *reinterpret_cast<const gemm_core::u32x4_halves*>(w + n * K + k0);
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (k0 + e < K) v[e >> 1] |= uint32_t(w[n * K + k0 + e]) << (16 * (e & 1));
+      }
+    }
+    w_frag[id] = v;
+  }
+}
 
 // Any K and any alignment on the matrix cores: (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N) ; grid: any
 // (128 x 128 tiles dealt round-robin), block = 256.

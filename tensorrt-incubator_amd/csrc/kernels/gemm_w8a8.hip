@@ -176,10 +176,10 @@ extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w8a8_frag_t256x38
   wide_kernel(a, w_frag, epi, y, M, K, N, lds);
 }
 // Weight re-layout into fragment order, from [K,N] (nk = 0) or [N,K] (nk = 1).  One 16-byte chunk per
-// thread.  (w, w_frag, K, N, nk) ; K % 128 == 0 ; w_frag holds 32 * ceil(N/32) * K bytes.
+// thread.  (w, w_frag, K, N, nk) ; w_frag holds 32 * ceil(N/32) * 128 * ceil(K/128) bytes, zeros where w has none.
 extern "C" __global__ void __launch_bounds__(256) mtrt_w8_prepack_frag(const int8_t* __restrict__ w, v4i* __restrict__ w_frag,
                                                                      int64_t K, int64_t N, int32_t nk) {
-  const int64_t slices = K / 128, ntiles = (N + 31) / 32;
+  const int64_t slices = (K + 127) / 128, ntiles = (N + 31) / 32;
   const int64_t total = ntiles * slices * 256;
   for (int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; id < total; id += int64_t(gridDim.x) * blockDim.x) {
     const int lane = int(id & 63), p = int((id >> 6) & 3);
@@ -187,7 +187,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w8_prepack_frag(const int
     const int64_t n = tile * 32 + (lane & 31), k0 = slice * 128 + 32 * p + 16 * (lane >> 5);
     union { v4i v; int8_t b[16]; } c;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) c.b[i] = n < N ? (nk ? w[n * K + k0 + i] : w[(k0 + i) * N + n]) : int8_t(0);
+    for (int i = 0; i < 16; ++i) c.b[i] = n < N && k0 + i < K ? (nk ? w[n * K + k0 + i] : w[(k0 + i) * N + n]) : int8_t(0);
     w_frag[id] = c.v;
   }
 }

@@ -1288,4 +1288,232 @@ int32_t mtrt_hip_gemm_w4a16(mtrt_stream_t stream, const void *a, const void *w_k
   return launch(st, KernelName("mtrt_gemm_w4a16_any"), blocks_for(M * N, kBlock), kBlock, as_hip(stream), args);
 }
 
+namespace {
+// Dense GEMM on fragment-order 16-bit weights: x [M,K] (K % 64 == 0, 16-byte aligned).  Up to 64 rows by estimate either the
+// wave-private kernel that reads the weights once or a tile; above, the tile and K split of frag_plan.
+struct DensePlan {
+  bool rows = false;
+  FragPlan tile;
+};
+DensePlan dense_frag_plan(int64_t M, int64_t K, int64_t N, int64_t units) {
+  DensePlan p;
+  p.tile = frag_plan(M, N, K / 64, units, true);
+  p.rows = M <= 64 && (!p.tile.tile || frag_rows_us(M, N, K / 64, units) < p.tile.us);
+  return p;
+}
+int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, const void *w_frag, const void *bias, void *y, int32_t dtype,
+                        int64_t M, int64_t K, int64_t N, void *partial) {
+  const DensePlan plan = dense_frag_plan(M, K, N, num_compute_units(st));
+  const char *xn = float_name(dtype);
+  // reported by the class of shapes, as the [N,K] kernels are named
+  const KernelName shown = KernelName(M <= 32 ? "mtrt_gemm_dense_rows32_" : M <= 64 ? "mtrt_gemm_dense_rows64_" : M <= 128 ? "mtrt_gemm_dense_rows128_"
+                                                                                                          : "mtrt_gemm_dense_mfma_") + xn;
+  KernelName name("mtrt_gemm_dense_frag_");
+  name + xn + "_" + (plan.rows ? (M <= 32 ? "rows32" : "rows64") : plan.tile.tile ? plan.tile.tile->suffix : "");
+  name.as(shown);
+  if (plan.rows || (plan.tile.tile && plan.tile.tile->columns == 384 && plan.tile.tile->rows == 256)) {
+    void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N};
+    return launch(st, name, plan.rows ? uint32_t(std::min<int64_t>((N + 31) / 32, int64_t(kMaxGrid) * 1024)) : plan.tile.grid(),
+                  plan.rows ? 512 : 256, stream, args);
+  }
+  if (!plan.tile.tile)
+    return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
+  uint32_t splits = plan.tile.splits;
+  uint32_t *tickets = nullptr;
+  if (splits > 1) {
+    tickets = reduction_slot(st, stream);
+    if (!tickets)
+      return MTRT_RUNTIME_ERROR;
+    tickets += kTicketOffset;
+  }
+  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &splits, &partial, &tickets};
+  return launch(st, name, plan.tile.grid(), 256, stream, args);
+}
+
+int64_t round_up(int64_t v, int64_t step) { return (v + step - 1) / step * step; }
+
+// How a plan's call runs: the row length its GEMM sees, whether x goes through the activation pass, and the two parts of the
+// workspace (the pass's result, then the partial tiles).
+struct LinearShape {
+  bool fragments = false, pass = false;
+  int64_t Kp = 0, act_bytes = 0, partial_bytes = 0;
+};
+LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units) {
+  LinearShape s;
+  const bool quantized = p.q_dtype >= 0;
+  const int eb = float_bytes(p.dtype);
+  s.Kp = p.K;
+  if (p.route == MTRT_LINEAR_W8A8) {
+    s.pass = true;
+    s.fragments = p.w_frag != nullptr;
+    s.Kp = s.fragments ? round_up(p.K, 128) : p.K;
+    s.act_bytes = round_up(M * s.Kp, 256);
+    if (s.fragments && M > 32) {
+      const W8Plan w = w8_plan(M, s.Kp, p.N, units, true);
+      s.partial_bytes = w.kind == W8Plan::kTile && w.tile.tile ? w.tile.workspace() : 0;
+    }
+  } else if (p.route == MTRT_LINEAR_DENSE) {
+    // A K that is no whole number of slices costs an unquantized x a pass of its own (2.3 us and up), so small products
+    // stay on the kernel that takes any K (about 15 us at a gigaflop).
+    s.fragments = p.w_frag && eb == 2 && (p.K % 64 == 0 || !p.w || quantized || 2.0 * double(M) * double(p.K) * double(p.N) >= 1e9);
+    s.Kp = s.fragments ? round_up(p.K, 64) : p.K;
+    s.pass = quantized || s.Kp != p.K;
+    s.act_bytes = s.pass ? round_up(M * s.Kp * eb, 256) : 0;
+    if (s.fragments) {
+      const DensePlan d = dense_frag_plan(M, s.Kp, p.N, units);
+      s.partial_bytes = !d.rows && d.tile.tile ? d.tile.workspace() : 0;
+    }
+  }
+  return s;
+}
+
+// Rows of one launch: the fragment kernels address the activations by 32-bit offsets, so more than 4 GiB of them go in parts.
+int64_t linear_rows(const mtrt_hip_linear_plan &p, int64_t M) {
+  const int64_t row = round_up(p.K, 128) * float_bytes(p.dtype);
+  return M * row < (int64_t(1) << 32) ? M : std::max<int64_t>(1, ((int64_t(1) << 32) - 1) / row / 256 * 256);
+}
+
+// x [M,K] -> out [M,Kp]: codes (codes != 0), dequantized codes, or (q_dtype < 0) the values, padded with zeros
+int32_t activation_pass(DeviceState *st, hipStream_t stream, bool codes, const void *x, int32_t dtype, int32_t q_dtype, const float *scale,
+                        void *out, int64_t M, int64_t K, int64_t Kp) {
+  if (Kp == K) {
+    // no padding between the rows: one row of all elements, so that a short row does not leave most of a wave idle and a row
+    // that is no whole number of groups needs none; the last group's padding lies in the workspace's own rounding
+    K *= M;
+    M = 1;
+    Kp = round_up(K, 16);
+  }
+  const int group = dtype == MTRT_F32 ? 4 : 8;
+  const int64_t chunks = (Kp / group + 127) / 128;
+  KernelName name(q_dtype < 0 ? "mtrt_act_pad_b16" : codes ? "mtrt_act_codes_" : "mtrt_act_fake_");
+  if (q_dtype >= 0)
+    name + float_name(dtype) + "_" + code_name(q_dtype);
+  void *args[] = {&x, &out, &scale, &M, &K, &Kp};
+  return launch(st, name, blocks_for(M * chunks, kBlock / 64), kBlock, stream, args);
+}
+
+// What of a plan is wrong, or nullptr.
+const char *linear_fault(const mtrt_hip_linear_plan *p, int64_t M) {
+  if (!p)
+    return "null plan";
+  if (p->route < MTRT_LINEAR_W8A8 || p->route > MTRT_LINEAR_DENSE || !float_name(p->dtype))
+    return "unknown route or dtype";
+  if (M < 0 || p->K <= 0 || p->N <= 0 || M > kMaxMatrixExtent || p->K > kMaxMatrixExtent || p->N > kMaxMatrixExtent)
+    return "extents must be positive and below 2^31";
+  if (p->route != MTRT_LINEAR_DENSE && p->dtype != MTRT_F16)
+    return "this route computes in f16";
+  if (p->q_dtype >= 0 && p->q_dtype != MTRT_I8 && p->q_dtype != MTRT_F8E4M3FN && p->q_dtype != MTRT_I4)
+    return "activations go through i8, f8E4M3FN or i4 codes";
+  if (p->route == MTRT_LINEAR_W8A8 && (p->q_dtype != MTRT_I8 || !p->x_scale || !p->w_scale || (!p->w && !p->w_frag)))
+    return "W8A8 needs int8 activations, both scales and weights";
+  if (p->route == MTRT_LINEAR_W4A16 && (p->q_dtype >= 0 || p->bias || !p->w_frag || !p->w_scale || p->K % 64 != 0))
+    return "W4A16 needs plain activations, re-laid weights, their scales and K % 64 == 0";
+  if (p->route == MTRT_LINEAR_DENSE && ((p->q_dtype >= 0 && !p->x_scale) || (!p->w && !(p->w_frag && float_bytes(p->dtype) == 2))))
+    return "the dense route needs weights, and a scale where it quantizes";
+  return nullptr;
+}
+} // namespace
+
+int64_t mtrt_hip_linear_fragments_bytes(int32_t dtype, int64_t K, int64_t N) {
+  const int eb = dtype == MTRT_I8 ? 1 : dtype == MTRT_F16 || dtype == MTRT_BF16 ? 2 : 0;
+  if (!eb || K <= 0 || N <= 0 || K > kMaxMatrixExtent || N > kMaxMatrixExtent)
+    return 0;
+  return ((N + 31) / 32) * 32 * round_up(K * eb, 128);
+}
+
+int32_t mtrt_hip_linear_prepack_fragments(mtrt_stream_t stream, const void *w_nk, int32_t dtype, void *w_frag, int64_t K, int64_t N) {
+  clear_error();
+  const int64_t bytes = mtrt_hip_linear_fragments_bytes(dtype, K, N);
+  if (bytes == 0)
+    return set_error(MTRT_INVALID_ARGUMENT, "fragment order holds i8, f16 or bf16 weights of positive extents, got dtype %d [%lld, %lld]", dtype,
+                     (long long)N, (long long)K);
+  if (!w_nk || !w_frag)
+    return set_error(MTRT_INVALID_ARGUMENT, "null operand");
+  if (!aligned(w_frag, 16) || (dtype != MTRT_I8 && !aligned(w_nk, 2)))
+    return set_error(MTRT_INVALID_ARGUMENT, "the fragment buffer must be 16-byte aligned, the weights aligned to their elements");
+  DeviceState *st = device_state();
+  if (!st)
+    return MTRT_RUNTIME_ERROR;
+  int32_t is_nk = 1;
+  void *args8[] = {&w_nk, &w_frag, &K, &N, &is_nk}, *args16[] = {&w_nk, &w_frag, &K, &N};
+  return launch(st, KernelName(dtype == MTRT_I8 ? "mtrt_w8_prepack_frag" : "mtrt_w16_prepack_frag"), blocks_for(bytes / 16, kBlock), kBlock,
+                as_hip(stream), dtype == MTRT_I8 ? args8 : args16);
+}
+
+int64_t mtrt_hip_linear_workspace(const mtrt_hip_linear_plan *plan, int64_t M) {
+  if (M <= 0 || linear_fault(plan, M))
+    return 0;
+  DeviceState *st = device_state();
+  if (!st)
+    return 0;
+  int64_t need = 0;
+  const int64_t most = linear_rows(*plan, M), last = M % most;
+  for (int64_t rows : {most, last}) {
+    if (rows > 0) {
+      const LinearShape s = linear_shape(*plan, rows, num_compute_units(st));
+      need = std::max(need, s.act_bytes + s.partial_bytes);
+    }
+  }
+  return need;
+}
+
+int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, const void *x, void *y, int64_t M, void *workspace,
+                        int64_t workspace_bytes) {
+  clear_error();
+  if (const char *fault = linear_fault(plan, M))
+    return set_error(MTRT_INVALID_ARGUMENT, "linear plan: %s", fault);
+  if (M == 0)
+    return MTRT_OK;
+  const mtrt_hip_linear_plan &p = *plan;
+  const int eb = float_bytes(p.dtype);
+  if (!x || !y)
+    return set_error(MTRT_INVALID_ARGUMENT, "null operand");
+  if (!aligned(x, eb) || !aligned(y, eb) || !aligned(p.bias, eb) || !aligned(p.w_frag, 16))
+    return set_error(MTRT_INVALID_ARGUMENT, "x, y and bias must be aligned to their elements, w_frag to 16 bytes");
+  DeviceState *st = device_state();
+  if (!st)
+    return MTRT_RUNTIME_ERROR;
+  if (p.route == MTRT_LINEAR_W4A16)
+    return mtrt_hip_gemm_w4a16(stream, x, nullptr, p.w_frag, p.w_scale, y, M, p.K, p.N, p.K);
+  const int64_t most = linear_rows(p, M);
+  if (most < M) {
+    for (int64_t m0 = 0; m0 < M; m0 += most) {
+      const int32_t rc = mtrt_hip_linear(stream, plan, static_cast<const char *>(x) + m0 * p.K * eb, static_cast<char *>(y) + m0 * p.N * eb,
+                                         std::min(most, M - m0), workspace, workspace_bytes);
+      if (rc != MTRT_OK)
+        return rc;
+    }
+    return MTRT_OK;
+  }
+  const LinearShape s = linear_shape(p, M, num_compute_units(st));
+  if (s.fragments && !s.pass && !aligned(x, 16))
+    return set_error(MTRT_INVALID_ARGUMENT, "x must be 16-byte aligned for these weights");
+  const int64_t need = s.act_bytes + s.partial_bytes;
+  if (need > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < need))
+    return set_error(MTRT_INVALID_ARGUMENT, "workspace of %lld bytes, 16-byte aligned, needed", (long long)need);
+  char *ws = static_cast<char *>(workspace);
+  const void *act = x;
+  if (s.pass) {
+    act = ws;
+    const int32_t rc = activation_pass(st, as_hip(stream), p.route == MTRT_LINEAR_W8A8, x, p.dtype, p.q_dtype, p.x_scale, ws, M, p.K, s.Kp);
+    if (rc != MTRT_OK)
+      return rc;
+  }
+  void *partial = s.partial_bytes ? ws + s.act_bytes : nullptr;
+  if (p.route == MTRT_LINEAR_W8A8) {
+    const float *w_scale = static_cast<const float *>(p.w_scale), *x_scale = p.x_scale;
+    if (s.fragments)
+      return w8a8_fragments(as_hip(stream), act, p.w_frag, x_scale, 0, w_scale, p.bias, y, M, s.Kp, p.N, partial, s.partial_bytes);
+    uint32_t a_step = 0;
+    const void *w = p.w, *bias = p.bias;
+    int64_t K = p.K, N = p.N;
+    void *args[] = {&act, &w, &x_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
+    return launch(st, KernelName("mtrt_gemm_w8a8_nk_edge"), uint32_t(std::min<int64_t>(((M + 127) / 128) * ((N + 127) / 128), int64_t(kMaxGrid) * 1024)),
+                  kBlock, as_hip(stream), args);
+  }
+  if (s.fragments)
+    return dense_fragments(st, as_hip(stream), act, p.w_frag, p.bias, y, p.dtype, M, s.Kp, p.N, partial);
+  return mtrt_hip_linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N);
+}
+
 } // extern "C"

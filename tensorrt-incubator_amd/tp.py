@@ -376,12 +376,13 @@ class Linear:
         self._plan_key = None
         self._plan_owners = None
         self._plan = None
+        self._native_plan = None
 
     def invalidate(self):
         """Forget the prepared weight side.  Call after changing a parameter's device memory in a way torch does not
         see (a kernel of this library writing into it, a raw pointer): assignments of new Tensors and torch's own
         in-place updates are noticed without it."""
-        self._plan_key = self._plan_owners = self._plan = None
+        self._plan_key = self._plan_owners = self._plan = self._native_plan = None
 
     def __call__(self, x):
         return self.forward(x)
@@ -409,9 +410,10 @@ class Linear:
         if (self._plan is not None and self._plan_key == key and
                 all(a is b for a, b in zip(self._plan_owners, owners))):
             return self._plan
-        from . import gemm_w4a16_prepack, gemm_w8a8_prepack_fragments
+        from . import gemm_w4a16_prepack
         N, K = self.weight.shape
         plan = {"route": "dense"}
+        has_x_scale = False
         if self.quant_dtype is None:
             plan["weight"] = self.weight.device_data().contiguous()
         else:
@@ -427,8 +429,9 @@ class Linear:
                 plan["route"] = "w8a8"
                 codes = q_weight.device_data().contiguous()          # [N, K], K contiguous
                 plan["s_w"] = _scale_on_device(w_scale).reshape(-1).expand(N).contiguous()
-                if K % 128 == 0:
-                    plan["w_frag"] = gemm_w8a8_prepack_fragments(codes, is_nk=True)
+                # below one 128-byte slice of K the padding of the fragment order would be most of the product
+                if K >= 128:
+                    plan["w_frag"] = self._fragments(codes)
                 else:
                     plan["w_nk"] = codes
             elif (self.quant_dtype == int4 and not has_x_scale and per_out and self.dtype == float16 and K % 64 == 0):
@@ -441,15 +444,76 @@ class Linear:
             else:
                 plan["weight"] = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
         self._plan_key, self._plan_owners, self._plan = key, owners, plan
+        self._native_plan = self._make_native_plan(plan, has_x_scale, K, N)
         return plan
+
+    @staticmethod
+    def _fragments(w_nk):
+        """[N, K] weights (int8, float16, bfloat16) in the fragment order of the matrix-core kernels."""
+        torch = _torch()
+        N, K = w_nk.shape
+        code = {torch.int8: I8, torch.float16: F16, torch.bfloat16: BF16}[w_nk.dtype]
+        frag = torch.empty(lib().mtrt_hip_linear_fragments_bytes(code, K, N), dtype=torch.int8, device=w_nk.device)
+        check(lib().mtrt_hip_linear_prepack_fragments(_stream(), w_nk.data_ptr(), code, frag.data_ptr(), K, N))
+        return frag
+
+    def _make_native_plan(self, plan, has_x_scale, K, N):
+        """What the one-call forward pass needs, or None where only the general path applies (empty or oddly typed
+        parameters; a combination whose checks must raise)."""
+        torch = _torch()
+        if not (K and N) or self.dtype not in QUANTIZABLE_DTYPES:
+            return None
+        q_dtype, x_scale = None, None
+        if has_x_scale:
+            s = self.input_scale
+            if s.rank != 0 or s.dtype != self.dtype or not s.is_cpu_constant:
+                return None
+            q_dtype, x_scale = self.quant_dtype, _scale_on_device(s)
+        native = _bound or _native()
+        if plan["route"] == "w8a8":
+            return native.linear_plan(self, 0, q_dtype, K, N, plan.get("w_nk"), plan.get("w_frag"), plan["s_w"], x_scale)
+        if plan["route"] == "w4a16":
+            return native.linear_plan(self, 1, None, K, N, None, plan["w_prepacked"], plan["scale_kn"], None)
+        w = plan["weight"]
+        if w.dtype != _torch_dtype(self.dtype):
+            return None
+        frag = None
+        if w.dtype != torch.float32 and K >= 64:
+            frag = self._fragments(w)
+            if K % 64 == 0:                            # every call reads the fragments: [N, K] is the owner's own copy or goes
+                del plan["weight"]
+                w = None
+        return native.linear_plan(self, 2, q_dtype, K, N, w, frag, None, x_scale)
+
+    def _dense_weight(self, plan):
+        """The [N, K] matrix of the dense route, made again where the plan keeps only its fragments."""
+        if "weight" in plan:
+            return plan["weight"]
+        if self.quant_dtype is None:
+            return self.weight.device_data().contiguous()
+        q_weight = quantize(self.weight, self.weight_scale, self.quant_dtype, self.weight_quant_dim)
+        return dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
 
     # -- forward ---------------------------------------------------------------------------------------
     def forward(self, x):
-        from . import gemm_w4a16, gemm_w8a8, gemm_w8a8_fragments, linear_dense
-        torch = _torch()
+        native = _bound or _native()
+        done = native.tp_linear(self, x)
+        if done is not NotImplemented:
+            return done
+        # first call, parameters that changed, operands on the host or strided: bring everything into place and call again
         if not isinstance(x, Tensor):
             x = Tensor(x)
         plan = self._prepared()
+        a = x.device_data().contiguous()
+        if self.bias is not None:
+            self.bias.device_data()
+        x = _produced(a if a.data_ptr() % 16 == 0 else a.clone(), x.dtype)
+        done = native.tp_linear(self, x)
+        if done is not NotImplemented:
+            return done
+        # mixed types and what the checks below refuse
+        from . import gemm_w4a16, gemm_w8a8, gemm_w8a8_fragments, linear_dense
+        torch = _torch()
         N, K = self.weight.shape
         lead = x.shape[:-1]
         bias = None if self.bias is None else self.bias.device_data().contiguous()
@@ -458,6 +522,8 @@ class Linear:
             M = q_x.shape[0]
             s_x = _scale_on_device(_convert_scale(self.input_scale, self.dtype)).reshape(-1).expand(M).contiguous()
             if "w_frag" in plan:
+                pad = -K % 128
+                q_x = torch.nn.functional.pad(q_x, (0, pad)) if pad else q_x
                 y = gemm_w8a8_fragments(q_x, plan["w_frag"], s_x, plan["s_w"], N)
             else:
                 y = gemm_w8a8(q_x, plan["w_nk"], s_x, plan["s_w"])
@@ -473,7 +539,7 @@ class Linear:
             if self.quant_dtype is not None and isinstance(self.input_scale, Tensor):
                 x = dequantize(quantize(x, self.input_scale, self.quant_dtype), self.input_scale, self.dtype)
             a = x.device_data().reshape(-1, K).contiguous()
-            out = linear_dense(a, plan["weight"], bias)
+            out = linear_dense(a, self._dense_weight(plan), bias)
         return _produced(out.reshape(lead + (N,)), self.dtype)
 
 
