@@ -435,6 +435,14 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w4a16(mtrt_stream_t stream, const void 
                                                const void *scale, void *y, int64_t M, int64_t K,
                                                int64_t N, int64_t block);
 
+/* The same with scratch memory, which lets several workgroups share the K range of a tile where a launch would otherwise
+ * leave compute units idle (never up to 32 rows): `workspace`, at least mtrt_hip_gemm_w4a16_workspace(M, K, N, block) bytes,
+ * 16-byte aligned, the call's own until its work on `stream` is done.  With less (or NULL) the call runs unsplit. */
+MTRT_CAPI_EXPORTED int64_t mtrt_hip_gemm_w4a16_workspace(int64_t M, int64_t K, int64_t N, int64_t block);
+MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w4a16_ws(mtrt_stream_t stream, const void *a, const void *w_kn_packed, const void *w_prepacked,
+                                                  const void *scale, void *y, int64_t M, int64_t K, int64_t N, int64_t block,
+                                                  void *workspace, int64_t workspace_bytes);
+
 /* Dense Linear in one float type: y[m,n] = narrow(sum_k f32(x[m,k]) * f32(w_nk[n,k]) + f32(bias[n])), f32
  * accumulation; bias may be NULL.  The float matmul of the fake-quant Linear (linear.py:112-151:
  * out = x' @ W'^T + b on dequantized operands) for the parameter combinations the two matrix-core clusters

@@ -124,6 +124,8 @@ PROTOTYPES = {
     "mtrt_hip_gemm_w4a16_prepacked_bytes": (_i64, [_i64, _i64]),
     "mtrt_hip_gemm_w4a16_prepack": (_i32, [_vp, _vp, _vp, _i64, _i64]),
     "mtrt_hip_gemm_w4a16": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64]),
+    "mtrt_hip_gemm_w4a16_workspace": (_i64, [_i64, _i64, _i64, _i64]),
+    "mtrt_hip_gemm_w4a16_ws": (_i32, [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _vp, _i64]),
 }
 
 _lib = None

@@ -598,9 +598,12 @@ PyObject *f_gemm_w4a16(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const int64_t M = x->size(0);
   const at::Tensor y = out ? *out : empty_like_device({M, N}, at::ScalarType::Half, *x);
   const mtrt_stream_t s = current_stream();
+  const int64_t scratch_bytes = prepacked ? mtrt_hip_gemm_w4a16_workspace(M, K, N, block) : 0;
+  const at::Tensor scratch = scratch_bytes ? bytes_on(*x, scratch_bytes) : at::Tensor();
   if (!launch([&] {
-        return mtrt_hip_gemm_w4a16(s, x->data_ptr(), packed ? packed->data_ptr() : nullptr, prepacked ? prepacked->data_ptr() : nullptr,
-                                   scale->data_ptr(), y.data_ptr(), M, K, N, block);
+        return mtrt_hip_gemm_w4a16_ws(s, x->data_ptr(), packed ? packed->data_ptr() : nullptr, prepacked ? prepacked->data_ptr() : nullptr,
+                                      scale->data_ptr(), y.data_ptr(), M, K, N, block, scratch_bytes ? scratch.data_ptr() : nullptr,
+                                      scratch_bytes);
       }))
     return nullptr;
   return none_or_new(a[7], y);
@@ -964,7 +967,7 @@ PyObject *f_tp_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (dtype.o != lp->dtype->object || x.dtype != lp->dtype || !dense_on_gpu(*x.t) || x.t->dim() < 1 || x.t->size(-1) != p.K ||
       (has_bias && (!bias.read(bias_object.o) || bias.dtype != lp->dtype || !dense_on_gpu(*bias.t) || bias.t->dim() != 1 ||
                     bias.t->size(0) != p.N)) ||
-      (p.route == MTRT_LINEAR_W4A16 && has_bias) || (p.q_dtype < 0 && reinterpret_cast<uintptr_t>(x.t->data_ptr()) % 16 != 0))
+      (p.q_dtype < 0 && reinterpret_cast<uintptr_t>(x.t->data_ptr()) % 16 != 0))
     return not_here();
   p.bias = has_bias ? bias.t->data_ptr() : nullptr;
   c10::SmallVector<int64_t, 6> shape(x.t->sizes().begin(), x.t->sizes().end());

@@ -388,7 +388,13 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 // not have, it was some 500 scalar instructions, over a microsecond, in front of the first load of every workgroup.)
 __device__ __host__ __forceinline__ int64_t even_blocks(int64_t tiles) { return 8 * ((tiles + 7) / 8); }
 __device__ __forceinline__ void tile_at(uint32_t at, uint32_t tiles_m, uint32_t panels, uint32_t group, int64_t& tile_m, int64_t& panel) {
-  group = group < tiles_m ? group : tiles_m;
+  // (a division is some eighty cycles of a chain in front of the launch's first load)
+  if (group >= tiles_m) {
+    const uint32_t q = at / tiles_m;
+    panel = q;
+    tile_m = at - q * tiles_m;
+    return;
+  }
   const uint32_t per_group = panels * group;
   const uint32_t full = tiles_m / group;                 // whole groups; a last group holds the remainder
   uint32_t g = at / per_group, r, size;

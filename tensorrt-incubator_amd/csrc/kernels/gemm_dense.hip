@@ -321,15 +321,15 @@ MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
 // What a module's Linear runs on: its weights are re-laid once per parameter set.  Against the loops above, which bring both
 // operands through LDS in 256-row tiles (f16, us): (M, K, N) = (999, 4096, 11008) 113 -> 83, (2048, 4096, 11008) 197 -> 147,
 // (256, 4096, 4096) 58 -> 16, (398, 11520, 1856) 165 -> 30, (1024, 2048, 2048) 32 -> 12.5, (200, 12288, 512) 164 -> 12.7.
-// mtrt_gemm_dense_frag_<type>_t<rows>x<columns> (x [M,K], w_frag, bias [N] or null, y [M,N], M, K, N, splits, partial, tickets) ;
+// mtrt_gemm_dense_frag_<type>_t<rows>x<columns> (x [M,K], w_frag, bias [N] or null, y [M,N], M, K, N, Split) ;
 // K % 64 == 0, x and w_frag 16-byte aligned, x below 4 GiB; the rest as mtrt_gemm_w8a8_frag.
 #define MTRT_DENSE_FRAG_KERNEL(XN, XT, IT, JT, D, WG, TILE)                                                               \
   extern "C" __global__ void __launch_bounds__(256, WG) mtrt_gemm_dense_frag_##XN##_##TILE(                               \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t splits, f32x4* partial, uint32_t* tickets) {    \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, gemm_frag::Split sp) {    \
     __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<IT, D>(128 * JT)];                            \
     gemm_frag::Part part;                                                                                                 \
-    if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, K / 64, splits, partial, tickets, part)) return; \
+    if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / 64, sp, part)) return; \
     dense_cluster::BiasEpilogue<XT, 128 * JT> epi{bias, nullptr, {}};                                                     \
     gemm_frag::run<dense_cluster::HalfTraits<XT>, IT, JT, D>(x, 2 * K, w_frag, epi, y, M, N, part, lds);                  \
   }

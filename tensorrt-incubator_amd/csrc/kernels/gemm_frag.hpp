@@ -102,23 +102,26 @@ __device__ __forceinline__ void load_through(f32x4& dst, const f32x4* src) {
   __asm__ volatile("global_load_dwordx4 %0, %1, off offset:%2 sc1" : "=v"(dst) : "v"(src), "n"(Q * 1024) : "memory");
 }
 
-// Adds up the partial tiles of a split tile; true for the workgroup that is to run the epilogue.
-template <class Scalar, int IT, int JT, class Acc>
-__device__ __forceinline__ bool meet(Acc (&acc)[IT][JT], const Part& part, int8_t* lds) {
+// Adds up the partial tiles of a split tile; true for the workgroup that is to run the epilogue.  Four waves hold the tile;
+// further waves of the workgroup (active = false) only take part in the barriers.
+template <class Scalar, int G, int IT, int JT, class Acc>
+__device__ __forceinline__ bool meet(Acc (&acc)[IT][JT], const Part& part, int8_t* lds, int wave, bool active = true) {
   constexpr int kTiles = IT * JT, kPer = 4 * kTiles;   // 32 x 32 tiles of the wave; 16-byte pieces per lane
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63;
   f32x4* mine = part.partial + (uint64_t(part.split) * 4 + wave) * (kPer * 64) + lane;
+  if (active) {
 #pragma unroll
-  for (int i = 0; i < IT; ++i)
+    for (int i = 0; i < IT; ++i)
 #pragma unroll
-    for (int j = 0; j < JT; ++j)
+      for (int j = 0; j < JT; ++j)
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        f32x4 v;
+        for (int q = 0; q < 4; ++q) {
+          f32x4 v;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = __builtin_bit_cast(float, Scalar(acc[i][j][4 * q + e]));
-        store_through(mine + ((i * JT + j) * 4 + q) * 64, v);
-      }
+          for (int e = 0; e < 4; ++e) v[e] = __builtin_bit_cast(float, Scalar(acc[i][j][4 * q + e]));
+          store_through(mine + ((i * JT + j) * 4 + q) * 64, v);
+        }
+  }
   __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // written through: visible to the whole device
   __syncthreads();
   uint32_t* seen = reinterpret_cast<uint32_t*>(lds);
@@ -126,8 +129,9 @@ __device__ __forceinline__ bool meet(Acc (&acc)[IT][JT], const Part& part, int8_
   __syncthreads();
   if (*seen != part.splits - 1) return false;
   if (threadIdx.x == 0) __hip_atomic_store(part.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!active) return true;
   // A round trip to memory for each group of G tiles, KB splits at a time (what the registers beside the accumulators hold).
-  constexpr int G = kTiles < 2 || kTiles >= 12 ? 1 : 2, KB = 4;
+  constexpr int KB = 4;
   const f32x4* all = part.partial + uint64_t(wave) * (kPer * 64) + lane;
 #pragma unroll
   for (int g = 0; g < kTiles; g += G) {
@@ -303,7 +307,7 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
   __syncthreads();
   // (a tile whose accumulators fill half of the register file is never split: the partial sums would not fit beside them)
   if constexpr (IT * JT < 16) {
-    if (part.splits > 1 && !meet<typename Traits::Scalar>(acc, part, lds)) return;
+    if (part.splits > 1 && !meet<typename Traits::Scalar, (IT * JT < 2 || IT * JT >= 12 ? 1 : 2)>(acc, part, lds, slot)) return;
   }
   write_tile<JT, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, true);
 }
@@ -449,27 +453,40 @@ __device__ __forceinline__ void run_wide(const int8_t* __restrict__ a, int64_t a
 }
 
 
+// The K split of a launch, by value among the kernel's arguments (clusters.cpp: FragSplit).
+struct Split {
+  uint32_t splits, per;                                // parts, and slices in each but the last, which has the rest (at least one)
+  f32x4* partial;                                      // splits > 1: BM * BN / 4 pieces per part, the parts of a tile together
+  uint32_t* tickets;                                   // splits > 1: a zeroed word per tile
+};
+
 // Which part of the problem workgroup `id` of `nblocks` takes: (split, tile) items dealt evenly to the eight XCDs in
 // split-major order, so that an XCD works on as few K ranges as possible (with eight splits on one: every operand byte is
-// then fetched into one L2 only).  partial_words: 16-byte pieces of one partial tile.
+// then fetched into one L2 only).  group: row tiles that keep a panel together (tile_at).
+// (M, N and K are below 2^31: 32 bits throughout.  This code is in front of the launch's first load; with 64-bit divisions
+// it was half a microsecond.)
 template <int BM, int BN>
-__device__ __forceinline__ bool part_of(uint32_t id, uint32_t nblocks, int64_t M, int64_t N, int64_t slices, uint32_t splits, f32x4* partial,
-                                        uint32_t* tickets, Part& part) {
-  const uint32_t tiles_m = uint32_t((M + BM - 1) / BM), panels = uint32_t((N + BN - 1) / BN), tiles = tiles_m * panels;
-  const uint32_t at = (id & 7) * (nblocks >> 3) + (id >> 3);
-  if (at >= tiles * splits) return false;
-  const uint32_t split = at / tiles, t = at - split * tiles;
+__device__ __forceinline__ bool part_of(uint32_t id, uint32_t nblocks, int64_t M, int64_t N, uint32_t slices, const Split& sp, Part& part,
+                                        uint32_t group = ~0u) {
+  const uint32_t tiles_m = (uint32_t(M) + (BM - 1)) / BM, panels = (uint32_t(N) + (BN - 1)) / BN, tiles = tiles_m * panels;
+  uint32_t t = (id & 7) * (nblocks >> 3) + (id >> 3);
+  if (t >= tiles * sp.splits) return false;
+  part.slice0 = 0;
+  part.nslices = slices;
+  part.splits = sp.splits;
+  part.split = 0;
+  if (sp.splits > 1) {
+    part.split = t / tiles;
+    t -= part.split * tiles;
+    part.slice0 = part.split * sp.per;
+    part.nslices = part.split + 1 < sp.splits ? sp.per : slices - part.slice0;
+    part.ticket = sp.tickets + t;
+    part.partial = sp.partial + uint64_t(t) * sp.splits * (BM * BN / 4);
+  }
   int64_t tile_m, panel;
-  tile_at(t, tiles_m, panels, tiles_m, tile_m, panel);
+  tile_at(t, tiles_m, panels, group, tile_m, panel);
   part.m0 = tile_m * BM;
   part.n0 = panel * BN;
-  const uint32_t begin = uint32_t(uint64_t(slices) * split / splits);
-  part.slice0 = begin;
-  part.nslices = uint32_t(uint64_t(slices) * (split + 1) / splits) - begin;
-  part.splits = splits;
-  part.split = split;
-  part.ticket = tickets + t;
-  part.partial = partial + uint64_t(t) * splits * (BM * BN / 4);
   return true;
 }
 

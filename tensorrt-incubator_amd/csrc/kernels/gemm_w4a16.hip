@@ -23,11 +23,12 @@
 //
 // All kernels take the weight fragments straight from global memory into registers and
 // dequantise them there; only the activations go through LDS (direct-to-LDS loads).
-// Large M: 256 x 256 tiles, 4 waves of 256 x 64.  Medium M: 128 x 64 / 128 x 128 tiles so that the grid still fills
-// the chip, 4 waves in two sets that split each K slice.
+// Large M: 256 x 256 and 256 x 384 tiles, 4 waves of 256 rows.  Below: 32- to 128-row tiles and K split over workgroups
+// (gemm_frag.hpp), so that the grid still fills the chip.
 // Small M (<= 32): the GEMM is bound by reading the weights once.  One workgroup per
 // 32 columns, its four waves split K, partial tiles are added through LDS at the end.
 #include "gemm_core.hpp"
+#include "gemm_frag.hpp"
 
 using namespace mtrt_dev;
 
@@ -86,6 +87,7 @@ __device__ __forceinline__ h2 load_scale2(const uint16_t* __restrict__ scale, in
 
 struct F16Traits {
   using Acc = v16f;
+  using Scalar = float;
   static __device__ __forceinline__ Acc zero() {
     Acc z;
 #pragma unroll
@@ -110,7 +112,9 @@ struct F16Traits {
   static __device__ __forceinline__ void settle_vgpr() { __asm__ volatile("s_nop 15\n\ts_nop 15" ::: "memory"); }
 };
 
+template <int BN>
 struct PlainEpilogue {
+  const uint16_t* none = nullptr;
   __device__ __forceinline__ void setup(int8_t*, int64_t, int64_t, int64_t, int64_t) {}
   __device__ __forceinline__ void row(int) {}
   template <int HC>
@@ -120,6 +124,41 @@ struct PlainEpilogue {
     for (int e = 0; e < 4; e += 2) words[e >> 1] = f32x2_to_f16x2_bits(acc[4 * q + e], acc[4 * q + e + 1]);
   }
 };
+// y = f16(f16(acc) + bias[n])
+template <int BN>
+struct BiasEpilogue {
+  const uint16_t* bias;
+  const uint16_t* sb = nullptr;                        // bias of this tile's columns, in LDS
+  u32x2 br[2][4] = {};
+  __device__ __forceinline__ void setup(int8_t* scratch, int64_t, int64_t, int64_t n0, int64_t N) {
+    uint16_t* dst = reinterpret_cast<uint16_t*>(scratch);
+    for (int c = threadIdx.x; c < BN; c += blockDim.x) dst[c] = n0 + c < N ? bias[n0 + c] : uint16_t(0);
+    sb = dst;
+  }
+  __device__ __forceinline__ void row(int) {}
+  template <int HC>
+  __device__ __forceinline__ void columns(int first_col_in_tile) {
+#pragma unroll
+    for (int jj = 0; jj < HC; ++jj)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) br[jj][q] = *reinterpret_cast<const u32x2*>(sb + first_col_in_tile + jj * 32 + q * 8);
+  }
+  __device__ __forceinline__ void convert4(const v16f& acc, int q, int jj, uint32_t (&words)[2]) const {
+#pragma unroll
+    for (int e = 0; e < 4; e += 2) {
+      H2Bits v, b;
+      v.u = f32x2_to_f16x2_bits(acc[4 * q + e], acc[4 * q + e + 1]);
+      b.u = br[jj][q][e >> 1];
+      v.h = v.h + b.h;
+      words[e >> 1] = v.u;
+    }
+  }
+};
+// the same for one output
+__device__ __forceinline__ uint16_t narrow_with_bias(float sum, const uint16_t* __restrict__ bias, int64_t c) {
+  const uint32_t h = f32_to_f16_bits(sum);
+  return uint16_t(bias ? f32_to_f16_bits(f16_bits_to_f32(h) + f16_bits_to_f32(bias[c])) : h);
+}
 
 // ---- large M, weights straight into registers -------------------------------------------
 // The prepacked stream is already in fragment order, so a wave can load the raw nibbles of
@@ -137,7 +176,7 @@ struct PlainEpilogue {
 // D register sets = slices fetched ahead; KEEP: the waves use only part of each vector (see half)
 template <int JT, int D, bool KEEP>
 struct WeightRegs {
-  const int8_t* wbase[JT];                           // slice 0 of each of this wave's 32-column tiles (uniform)
+  const int8_t* wbase[JT];                           // the first slice of each of this wave's 32-column tiles (uniform)
   const int8_t* scale;                               // as bytes (uniform)
   uint32_t wlane, scol[JT];                          // this lane's byte offsets inside a slice / inside a row of scales
   int64_t N;
@@ -145,7 +184,7 @@ struct WeightRegs {
   uint32_t sc_bits[D][JT];
   uint32_t mask = nibble_pair_mask(), mask_hi = nibble_pair_mask() << 4;
   // tile0: first 32-column tile of this wave
-  __device__ __forceinline__ void init(const uint32_t* wp, const uint16_t* sc, int64_t kblocks, int64_t n, int64_t tile0) {
+  __device__ __forceinline__ void init(const uint32_t* wp, const uint16_t* sc, int64_t kblocks, uint32_t slice0, int64_t n, int64_t tile0) {
     const int lane = threadIdx.x & 63;
     const int64_t last_tile = (n + 31) / 32 - 1;
     N = n;
@@ -157,7 +196,7 @@ struct WeightRegs {
       tile = tile < last_tile ? tile : last_tile;      // columns past N: some valid data, never stored
       int64_t col = tile * 32 + (lane & 31);
       col = col < n ? col : n - 1;
-      wbase[j] = reinterpret_cast<const int8_t*>(wp) + tile * kblocks * 1024;
+      wbase[j] = reinterpret_cast<const int8_t*>(wp) + (tile * kblocks + slice0) * 1024;
       scol[j] = uint32_t(col) * 2;
     }
   }
@@ -205,7 +244,7 @@ struct Shape {
   static constexpr int kBM = 32 * IT * MW, kBN = 32 * JT * NWN;
   static constexpr int kStageBytes = kBM * 128;        // one slice of the activation panel
   static constexpr int kRingBytes = STAGES * kStageBytes;
-  static constexpr int kOutBytes = kSlots * gemm_core::kOutWave + 2048;
+  static constexpr int kOutBytes = kSlots * 32 * (IT < 4 ? IT : 4) * gemm_core::kOutRow + 2048;
   static constexpr int kSumBytes = KW == 2 ? kSlots * (32 * IT) * 32 * JT * 4 : 0;
   static constexpr int kLds = kRingBytes > kOutBytes ? (kRingBytes > kSumBytes ? kRingBytes : kSumBytes)
                                                      : (kOutBytes > kSumBytes ? kOutBytes : kSumBytes);
@@ -222,8 +261,8 @@ __device__ __forceinline__ void static_for(F&& f) {
 template <class S, int KH, class Epilogue>
 __device__ __forceinline__ void run_weight_regs(const int8_t* __restrict__ a, int64_t a_row_bytes,
                                                 WeightRegs<S::kJT, S::kDepth, (S::kKW > 1)>& wr, uint32_t slices_per_block,
-                                                Epilogue& epi, uint16_t* __restrict__ y, int64_t M, int64_t N, int64_t slices,
-                                                int64_t m0, int64_t n0, int8_t* lds, int slot) {
+                                                Epilogue& epi, uint16_t* __restrict__ y, int64_t M, int64_t N,
+                                                const gemm_frag::Part& part, int8_t* lds, int slot) {
   using namespace gemm_core;
   constexpr int JT = S::kJT, NWN = S::kNWN, KW = S::kKW, IT = S::kIT, G = (4 * IT * S::kMW) / S::kWaves, NK = 4 / KW;
   constexpr int D = S::kDepth, NS = S::kStages;
@@ -241,15 +280,17 @@ __device__ __forceinline__ void run_weight_regs(const int8_t* __restrict__ a, in
   // ordinary vector registers (F16Traits::mfma_vgpr)
   constexpr int JA = IT * JT * 16 > 256 ? 256 / (IT * 16) : JT;
 
-  const uint32_t nslices = uint32_t(slices), last = nslices - 1;
+  // this workgroup's slices: counted from its first one, from which the operands' bases start
+  const uint32_t nslices = __builtin_amdgcn_readfirstlane(part.nslices), slice0 = __builtin_amdgcn_readfirstlane(part.slice0), last = nslices - 1;
   DmaLoaderT<G> al;
-  al.init(a, M, a_row_bytes, m0);
+  al.init(a + uint64_t(slice0) * 128, M, a_row_bytes, part.m0);
   // The slice fetched next, its row of scales and its position inside the block; moves on by one per slice until
   // it reaches the last slice (which is then fetched again into stages and registers that nobody reads).
   // (plain integer arithmetic instead of selects: it stays on the scalar unit)
-  uint32_t fslice = 0, frem = 0;
-  const int8_t* fsrow = wr.scale;
+  const uint32_t block0 = slice0 ? slice0 / slices_per_block : 0;
+  uint32_t fslice = 0, frem = slice0 - block0 * slices_per_block;
   const uint32_t scale_row_bytes = uint32_t(N) * 2;
+  const int8_t* fsrow = wr.scale + uint64_t(block0) * scale_row_bytes;
   auto advance = [&]() {
     const uint32_t go = uint32_t(fslice - last) >> 31;                     // fslice < last
     fslice += go;
@@ -424,28 +465,219 @@ __device__ __forceinline__ void run_weight_regs(const int8_t* __restrict__ a, in
           }
     }
   }
-  write_tile<JT, NWN, S::kSlots>(acc, epi, y, M, N, m0, n0, lds, slot, KH == 0);
+  if constexpr (IT * JT < 16) {                        // (larger tiles are never split: see gemm_frag::run)
+    if (part.splits > 1) {
+      __syncthreads();
+      if (!gemm_frag::meet<float, 1>(acc, part, lds, slot, KH == 0)) return;
+    }
+  }
+  write_tile<JT, NWN, S::kSlots>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, KH == 0);
 }
 
-// Common body of the weight-in-register kernels: which tile, which wave does what.
-template <class S>
+// ---- smaller tiles, K split over workgroups ---------------------------------------------------------------
+// The loop of gemm_frag::run (its header describes the structure: four waves of IT * 32 rows x JT * 32 columns each, fragment
+// reads four ahead, memory instructions in a fixed order and waited for by count) with 4-bit weights: one 16-byte
+// load per lane, slice and column tile brings the nibbles of four k-steps, a 2-byte load beside it the scales; register
+// sets for D slices; the fragments of a k-step are dequantised during the one before.
+//
+// What bounds it: in long loops the matrix cores and, added to them, the dequantisation (52 cycles of vector instructions
+// per fragment, against 32 for each of the IT MFMAs that use it: with the dequantisation taken out a 128 x 128 tile ran
+// 64.5 us instead of 81 at M = 240, K = 12928, N = 9728, a 64 x 128 tile 29 instead of 40 at M = 64, K = N = 8192; the
+// activations from L1 alone or half of the fragment reads changed nothing); in short launches their number: a launch
+// whose tiles leave compute units idle is cut along K as well.
+template <int IT, int JT, int D>
+struct Order4 {
+  using O = gemm_frag::Order<IT, JT, D>;
+  static constexpr int kSlice = IT + 2 * JT;           // memory instructions of a slice: activations, then nibbles and scales
+  static constexpr int dma_before(int t) { return t == 0 ? 0 : O::dma(t - 1) + dma_before(t - 1); }
+  // issued after the nibbles and scales of slice s + 1 and before k-step 3 of slice s
+  static constexpr int weights_in_flight() { return (D - 2) * kSlice + dma_before(3); }
+  // issued after the activations of slice s + 1 and before k-step `at` of slice s
+  static constexpr int activations_in_flight(int at) { return 2 * JT + (D - 2) * kSlice + dma_before(at); }
+};
+
+template <int IT, int JT, int D, class Epilogue>
+__device__ __forceinline__ void run_tiles(const int8_t* __restrict__ a, int64_t row_bytes, const uint32_t* __restrict__ wp,
+                                          const uint16_t* __restrict__ scale, uint32_t slices_per_block, Epilogue& epi,
+                                          uint16_t* __restrict__ y, int64_t M, int64_t N, const gemm_frag::Part& part, int8_t* lds) {
+  using namespace gemm_core;
+  using O = gemm_frag::Order<IT, JT, D>;
+  using O4 = Order4<IT, JT, D>;
+  constexpr int NS = gemm_frag::stages<IT, D>(), AN = 4, kStageBytes = IT * 32 * 128;
+  constexpr int TB = (4 * IT - AN) / IT;               // the first k-step that reads a fragment of the next slice
+  static_assert(D % 2 == 0 && O4::activations_in_flight(TB) < 64 && (D - 1) * O4::kSlice < 64, "wait counter range");
+  const int lane = threadIdx.x & 63;
+  const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int frow = lane & 31, fhalf = lane >> 5;
+  const int64_t total_slices = row_bytes / 128, ntiles = (N + 31) / 32;
+  const uint32_t nslices = __builtin_amdgcn_readfirstlane(part.nslices), slice0 = __builtin_amdgcn_readfirstlane(part.slice0);
+
+  v16f acc[IT][JT];
+  DmaLoaderT<IT> al;
+  al.init(a + uint64_t(slice0) * 128, M, row_bytes, part.m0);
+  v4i fa[2][AN];
+  u4 fb[2][JT], raw[D][JT];
+  uint32_t sc[D][JT];
+  const uint32_t mask = nibble_pair_mask(), mask_hi = mask << 4;
+  const int8_t* wsrc[JT];                              // the first slice of each column tile (uniform)
+  const uint32_t wlane = uint32_t(lane) * 16;
+  uint32_t scol[JT];
+#pragma unroll
+  for (int j = 0; j < JT; ++j) {
+    int64_t tile = int64_t(__builtin_amdgcn_readfirstlane(uint32_t(part.n0 / 32))) + slot * JT + j;
+    tile = tile < ntiles ? tile : ntiles - 1;          // tiles past N: some valid data, never stored
+    wsrc[j] = reinterpret_cast<const int8_t*>(wp) + (tile * total_slices + slice0) * 1024;
+    int64_t col = tile * 32 + frow;
+    scol[j] = uint32_t(col < N ? col : N - 1) * 2;
+  }
+  auto keep = [&](uint32_t slice) { return uint32_t(int32_t(slice - nslices) >> 31); };   // all ones up to the last slice
+  const uint32_t lds_base = uint32_t(uintptr_t((lds_void_t*)lds));
+  uint32_t a_lane[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) a_lane[p] = lds_base + uint32_t(lds_off(frow, 2 * p + fhalf));
+  auto read_a = [&](v4i& dst, uint32_t addr, auto tile) {
+    constexpr int I = decltype(tile)::value;
+    __asm__ volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(I * 4096) : "memory");
+  };
+  auto stage_off = [&](uint32_t slice) { return (slice & uint32_t(NS - 1)) * uint32_t(kStageBytes); };
+  auto issue_dma = [&](auto step, uint32_t slice) {
+    constexpr int T = decltype(step)::value;
+    if constexpr (O::dma(T) > 0) {
+      const uint32_t k = keep(slice);
+      const int8_t* src = al.base + uint64_t(slice & k) * 128;
+      int8_t* st = lds + stage_off(slice);
+#pragma unroll
+      for (int g = 0; g < O::dma(T); ++g) {
+        uint32_t off = al.off[O::first(T) + g] & k;
+        __asm__ volatile("" : "+v"(off));
+        __builtin_amdgcn_global_load_lds((global_void_t*)(src + off), (lds_void_t*)(st + (al.wave_u * IT + O::first(T) + g) * 1024), 16, 0, 0);
+      }
+    }
+  };
+  // the row of scales of the slice fetched next; moves on by one slice per call until the last one
+  const uint32_t scale_row_bytes = uint32_t(N) * 2, block0 = slice0 ? slice0 / slices_per_block : 0;
+  uint32_t frem = slice0 - block0 * slices_per_block;
+  const int8_t* srow = reinterpret_cast<const int8_t*>(scale) + uint64_t(block0) * scale_row_bytes;
+  auto issue_w = [&](auto set, uint32_t slice) {
+    constexpr int SET = decltype(set)::value;
+    const uint32_t k = keep(slice), at = __builtin_amdgcn_readfirstlane(slice & k);
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      const int8_t* from = wsrc[j] + uint64_t(at) * 1024;
+      __asm__ volatile("global_load_dwordx4 %0, %1, %2" : "=v"(raw[SET][j]) : "v"(wlane & k), "s"(from) : "memory");
+      __asm__ volatile("global_load_ushort %0, %1, %2" : "=v"(sc[SET][j]) : "v"(scol[j]), "s"(srow) : "memory");
+    }
+    const uint32_t go = (slice + 1 - nslices) >> 31;    // slice + 1 < nslices
+    frem += go;
+    const uint32_t wrap = 1u - ((frem - slices_per_block) >> 31);
+    frem &= wrap - 1u;
+    srow += wrap * scale_row_bytes;
+  };
+  auto dequant_half = [&](auto set, auto step, int j, int part_, u4& frag) {
+    H2Bits t;
+    t.u = sc[decltype(set)::value][j];
+    const h2 s2 = {t.h[0], t.h[0]};
+    dequant4(raw[decltype(set)::value][j][decltype(step)::value], s2, part_, mask, mask_hi, frag);
+  };
+
+  static_for<0, D>([&](auto v) {
+    constexpr int SD = decltype(v)::value;
+    static_for<0, 4>([&](auto t) { issue_dma(t, SD); });
+    issue_w(v, SD);
+  });
+  __builtin_amdgcn_sched_barrier(0);
+  {                                                    // accumulators cleared by the matrix cores under those loads
+    v4i none = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+#pragma unroll
+      for (int j = 0; j < JT; ++j) {
+        __asm__ volatile("" : "+v"(none));
+        acc[i][j] = F16Traits::mfma(none, none, F16Traits::zero());
+      }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+#pragma unroll
+  for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(raw[0][j]), "+v"(sc[0][j]) : "n"((D - 1) * O4::kSlice) : "memory");
+  __asm__ volatile("s_barrier" ::: "memory");
+  static_for<0, AN>([&](auto n) {
+    constexpr int X = decltype(n)::value;
+    read_a(fa[0][X], a_lane[X / IT] + stage_off(0), IntC<X % IT>{});
+  });
+#pragma unroll
+  for (int j = 0; j < JT; ++j) {
+    dequant_half(IntC<0>{}, IntC<0>{}, j, 0, fb[0][j]);
+    dequant_half(IntC<0>{}, IntC<0>{}, j, 1, fb[0][j]);
+  }
+
+  // k-step T of the slice at position U of the unrolled loop (slice s)
+  auto kstep = [&](auto pos, auto step, uint32_t s) {
+    constexpr int U = decltype(pos)::value, T = decltype(step)::value, Q = U * 4 + T;
+    constexpr int NSET = T == 3 ? (U + 1) % D : U;     // where the next k-step's weights come from
+    if constexpr (T == TB) {
+      __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(O4::activations_in_flight(TB)) : "memory");
+      __asm__ volatile("s_barrier" ::: "memory");
+    }
+    if constexpr (T == 3) {
+#pragma unroll
+      for (int j = 0; j < JT; ++j)
+        __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(raw[NSET][j]), "+v"(sc[NSET][j]) : "n"(O4::weights_in_flight()) : "memory");
+    }
+    const uint32_t here = stage_off(s), next = stage_off(s + 1);
+    static_for<0, IT>([&](auto cc) {
+      constexpr int c = decltype(cc)::value, X = Q * IT + c, SET = (X / AN) % 2, AI = X % AN;
+      constexpr int X2 = T * IT + c + AN, T2 = X2 / IT;  // the fragment read now, AN further on in the stream
+      __asm__ volatile("s_waitcnt lgkmcnt(%1)" : "+v"(fa[SET][AI]) : "n"(AN - 1) : "memory");
+#pragma unroll
+      for (int j = 0; j < JT; ++j) acc[c][j] = F16Traits::mfma(__builtin_bit_cast(v4i, fb[Q % 2][j]), fa[SET][AI], acc[c][j]);
+      read_a(fa[1 - SET][AI], a_lane[T2 % 4] + (T2 >= 4 ? next : here), IntC<X2 % IT>{});
+      if constexpr (c == 0) issue_dma(step, s + D);
+#pragma unroll
+      for (int u = 0; u < 2 * JT; ++u)
+        if ((u * IT) / (2 * JT) == c) dequant_half(IntC<NSET>{}, IntC<(T + 1) % 4>{}, u >> 1, u & 1, fb[1 - Q % 2][u >> 1]);
+      if constexpr (T == 3 && c == IT - 1) issue_w(pos, s + D);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  uint32_t s = 0;
+  for (; s + D - 1 < nslices; s += D)
+    static_for<0, 4 * D>([&](auto q) { kstep(IntC<decltype(q)::value / 4>{}, IntC<decltype(q)::value % 4>{}, s + decltype(q)::value / 4); });
+  static_for<0, D - 1>([&](auto p) {
+    constexpr int P = decltype(p)::value;
+    if (s + P < nslices) static_for<0, 4>([&](auto t) { kstep(p, t, s + P); });
+  });
+  __builtin_amdgcn_s_waitcnt(0x0070);                  // the surplus loads and fragment reads have landed: their
+#pragma unroll                                         // registers stay allocated up to here
+  for (int i = 0; i < AN; ++i) __asm__ volatile("s_waitcnt lgkmcnt(0)" ::"v"(fa[0][i]), "v"(fa[1][i]) : "memory");
+#pragma unroll
+  for (int q = 0; q < D; ++q)
+#pragma unroll
+    for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(0)" ::"v"(raw[q][j]), "v"(sc[q][j]) : "memory");
+  __syncthreads();
+  if constexpr (IT * JT < 16) {
+    if (part.splits > 1 && !gemm_frag::meet<float, (IT * JT < 2 || IT * JT >= 12 ? 1 : 2)>(acc, part, lds, slot)) return;
+  }
+  write_tile<JT, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, true);
+}
+
+// Common body of the weight-in-register kernels: which tile and which slices, which wave does what.
+template <class S, class Epilogue>
 __device__ __forceinline__ void weight_regs_kernel(const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp,
-                                                   const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
-                                                   int64_t K, int64_t N, int64_t block, int8_t* lds) {
-  int64_t tile_m, panel;
+                                                   const uint16_t* __restrict__ scale, Epilogue& epi, uint16_t* __restrict__ y, int64_t M,
+                                                   int64_t K, int64_t N, int64_t block, const gemm_frag::Split& sp, int8_t* lds) {
   // A slice of a 4-bit weight panel is a quarter of the bytes of an activation panel slice of the same
   // width: groups of four M tiles, eight panels at a time per XCD; every XCD the same number of tiles
-  if (!gemm_core::tile_of_even(blockIdx.x, gridDim.x, (M + S::kBM - 1) / S::kBM, (N + S::kBN - 1) / S::kBN, 4, tile_m, panel)) return;
-  const int64_t m0 = tile_m * S::kBM, n0 = panel * S::kBN;
+  gemm_frag::Part part;
+  if (!gemm_frag::part_of<S::kBM, S::kBN>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / BKH, sp, part, 4)) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int slot = wave % S::kSlots;
   WeightRegs<S::kJT, S::kDepth, (S::kKW > 1)> wr;
-  wr.init(wp, scale, K / BKH, N, n0 / 32 + (slot % S::kNWN) * S::kJT);
-  PlainEpilogue epi;
+  wr.init(wp, scale, K / BKH, __builtin_amdgcn_readfirstlane(part.slice0), N,
+          int64_t(__builtin_amdgcn_readfirstlane(uint32_t(part.n0 / 32))) + (slot % S::kNWN) * S::kJT);
   const int8_t* ab = reinterpret_cast<const int8_t*>(a);
   const uint32_t spb = uint32_t(block / BKH);
-  if (S::kKW == 1 || wave < S::kSlots) run_weight_regs<S, 0>(ab, 2 * K, wr, spb, epi, y, M, N, K / BKH, m0, n0, lds, slot);
-  else run_weight_regs<S, S::kKW - 1>(ab, 2 * K, wr, spb, epi, y, M, N, K / BKH, m0, n0, lds, slot);
+  if (S::kKW == 1 || wave < S::kSlots) run_weight_regs<S, 0>(ab, 2 * K, wr, spb, epi, y, M, N, part, lds, slot);
+  else run_weight_regs<S, S::kKW - 1>(ab, 2 * K, wr, spb, epi, y, M, N, part, lds, slot);
 }
 
 // (a [M,K] f16, w_prepacked, scale [K/block, N] f16, y [M,N] f16, M, K, N, block) ; K % 64 == 0, block % 64 == 0,
@@ -459,7 +691,8 @@ extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x256(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
     uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
   __shared__ __attribute__((aligned(16))) int8_t lds[BigShape::kLds];
-  weight_regs_kernel<BigShape>(a, wp, scale, y, M, K, N, block, lds);
+  PlainEpilogue<256> epi;
+  weight_regs_kernel<BigShape>(a, wp, scale, epi, y, M, K, N, block, {1, 0, nullptr, nullptr}, lds);
 }
 // 256 x 384 tiles: four waves of 256 x 96, 384 accumulator registers per lane, a third of them in ordinary vector
 // registers (F16Traits::mfma_vgpr), activation fragments read half a k-step ahead.  A workgroup moves 44 KiB per
@@ -473,42 +706,65 @@ extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x384(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
     uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
   __shared__ __attribute__((aligned(16))) int8_t lds[WideShape::kLds];
-  weight_regs_kernel<WideShape>(a, wp, scale, y, M, K, N, block, lds);
+  PlainEpilogue<384> epi;
+  weight_regs_kernel<WideShape>(a, wp, scale, epi, y, M, K, N, block, {1, 0, nullptr, nullptr}, lds);
 }
-// Medium M: 128 x 64 tiles so that the grid still fills the chip, two wave sets splitting each slice.
-// Same argument list.  grid = 8 * ceil(ceil(N/64) * ceil(M/128) / 8), block = 256.
-using MidShape = Shape<1, 2, 1, 2, 4, 5>;              // 128 x 64, 4 waves, four slices ahead (two workgroups share a CU's LDS)
-extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_t128x64(
+// 256-row tiles with a bias: the argument lists above, then bias [N] f16.
+extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x256_bias(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[MidShape::kLds];
-  weight_regs_kernel<MidShape>(a, wp, scale, y, M, K, N, block, lds);
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[BigShape::kLds];
+  BiasEpilogue<256> epi{bias};
+  weight_regs_kernel<BigShape>(a, wp, scale, epi, y, M, K, N, block, {1, 0, nullptr, nullptr}, lds);
+}
+extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x384_bias(
+    const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[WideShape::kLds];
+  BiasEpilogue<384> epi{bias};
+  weight_regs_kernel<WideShape>(a, wp, scale, epi, y, M, K, N, block, {1, 0, nullptr, nullptr}, lds);
 }
 
-// Medium M, wider: 128 x 128 tiles.  What a workgroup moves through its CU's L1 is dominated by the
-// activation panel (16 KiB per slice against 2 KiB of weights per 64 columns), and the L1 is what bounds
-// these launches, so the widest tile that still gives every compute unit a workgroup of its own is the
-// fastest.
-using MidWideShape = Shape<1, 4, 1, 2, 4, 8>;          // 128 x 128, 8 waves (two sets of four), four slices ahead, ring of eight stages (the stage of a slice is a mask away)
-extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_w4a16_t128x128(
-    const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[MidWideShape::kLds];
-  weight_regs_kernel<MidWideShape>(a, wp, scale, y, M, K, N, block, lds);
-}
-
-// Medium M, twice as wide: 128 x 256 tiles, the same eight waves with two column tiles each.  An activation fragment
-// read from LDS serves two MFMAs and the activation panel is fetched for half as many workgroups; a slice takes 0.48 us
-// against 0.37 us for twice the MFMAs, so a full round of these tiles costs 1.9 rounds of the 128 x 128 ones: ahead where
-// it saves a round (K = 4096, N = 11008: M = 512 56.9 -> 51.3 us, M = 300 53.8 -> 47.5; K = N = 8192, M = 1024 124.9 -> 115.9),
-// behind where the narrower tile fits one round anyway (M = 256: 43.6 against 27.3 us).
-using MidWide2Shape = Shape<1, 4, 2, 2, 4, 8>;         // 128 x 256, 8 waves (two sets of four), four slices ahead
-extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_w4a16_t128x256(
-    const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[MidWide2Shape::kLds];
-  weight_regs_kernel<MidWide2Shape>(a, wp, scale, y, M, K, N, block, lds);
-}
+// Tiles up to 128 rows: mtrt_gemm_w4a16_t<rows>x<columns> (a, w_prepacked, scale, y, M, K, N, block, bias [N] f16 (the _bias kernels),
+// Split) ; the first eight as above; grid = 8 * ceil(ceil(M/rows) * ceil(N/columns) * splits / 8).
+// Which one runs is the host's estimate (w4_plan); 621 launches over M = 33 ... 4096, K = 256 ... 14336, N = 64 ... 16384
+// took 1.44 times as long on average with the 128- and 256-row tiles alone and K unsplit, none less than 0.95 times:
+// (M, K, N) = (48, 4096, 4096) 13.0 -> 11.3 us, (128, 4096, 4096) 22.3 -> 14.2, (64, 8192, 8192) 25.7 -> 18.1,
+// (228, 4864, 160) 25.3 -> 9.7, (1020, 2176, 144) 13.9 -> 9.1, (1800, 640, 8576) 27.2 -> 24.7.
+#define MTRT_W4_ARGS                                                                                                    \
+  const uint16_t *__restrict__ a, const uint32_t *__restrict__ wp, const uint16_t *__restrict__ scale, uint16_t *__restrict__ y, \
+      int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t *__restrict__ bias, gemm_frag::Split sp
+#define MTRT_W4_TILE_KERNEL(TILE, EPI, IT, JT, D, WG)                                                                   \
+  extern "C" __global__ void __launch_bounds__(256, WG) mtrt_gemm_w4a16_##TILE(MTRT_W4_ARGS) {                          \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<IT, D>(128 * JT)];                          \
+    gemm_frag::Part part;                                                                                               \
+    if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / BKH, sp, part, 4)) return; \
+    EPI<128 * JT> epi{bias};                                                                                            \
+    run_tiles<IT, JT, D>(reinterpret_cast<const int8_t*>(a), 2 * K, wp, scale, uint32_t(block / BKH), epi, y, M, N, part, lds); \
+  }
+#define MTRT_W4_SETS_KERNEL(TILE, EPI, THREADS, WAVES, ...)                                                             \
+  extern "C" __global__ void __launch_bounds__(THREADS, WAVES) mtrt_gemm_w4a16_##TILE(MTRT_W4_ARGS) {                   \
+    using S = Shape<__VA_ARGS__>;                                                                                       \
+    __shared__ __attribute__((aligned(16))) int8_t lds[S::kLds];                                                        \
+    EPI<S::kBN> epi{bias};                                                                                              \
+    weight_regs_kernel<S>(a, wp, scale, epi, y, M, K, N, block, sp, lds);                         \
+  }
+// t128x256: an activation fragment read from LDS serves two MFMAs and the panel is fetched for half as many workgroups as
+// with 128 columns; two slices ahead (a ring of four stages), ahead of eight waves and four slices by 8 % on average.
+// t64x128, t128x128: eight waves in two sets that split each slice, four slices ahead: ahead of four waves (up to 15 %,
+// M = 200, K = 8832, N = 11520 68 -> 54 us) where the launch is not short.  What a workgroup moves through its CU's L1 is
+// dominated by the activation panel (16 KiB per slice of 128 rows against 4 KiB of weights).
+// t128x64: matrices at most 64 columns wide.
+// (With and without a bias: its addition costs the epilogue of a 128 x 128 tile 0.25 us.)
+#define MTRT_W4_TILE_KERNELS(SUFFIX, EPI)                          \
+  MTRT_W4_TILE_KERNEL(t32x128##SUFFIX, EPI, 1, 1, 4, 2)            \
+  MTRT_W4_TILE_KERNEL(t64x256##SUFFIX, EPI, 2, 2, 4, 2)            \
+  MTRT_W4_TILE_KERNEL(t128x256##SUFFIX, EPI, 4, 2, 2, 1)           \
+  MTRT_W4_SETS_KERNEL(t64x128##SUFFIX, EPI, 512, 2, 1, 4, 1, 2, 4, 8, 2) \
+  MTRT_W4_SETS_KERNEL(t128x128##SUFFIX, EPI, 512, 2, 1, 4, 1, 2, 4, 8)   \
+  MTRT_W4_SETS_KERNEL(t128x64##SUFFIX, EPI, 256, 1, 1, 2, 1, 2, 4, 5)
+MTRT_W4_TILE_KERNELS(, PlainEpilogue)
+MTRT_W4_TILE_KERNELS(_bias, BiasEpilogue)
 
 // Small M (<= 32): one workgroup per 32 columns, four waves split K.
 // G: groups of 8 activation rows kept per stage (M <= 8 * G); WAVES: waves that split K;
@@ -516,7 +772,7 @@ extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_w4a16_t128x256(
 template <int G, int WAVES, int JT>
 __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp,
                                        const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M, int64_t K,
-                                       int64_t N, int64_t block, int8_t* lds) {
+                                       int64_t N, int64_t block, const uint16_t* __restrict__ bias, int8_t* lds) {
   // Per wave a ring of four stages (8 * G rows x 64 k of activations each), filled by
   // direct-to-LDS loads three slices ahead: a fragment read straight from global memory would
   // touch 64 different cache lines per instruction (32 rows 8 KiB apart), the ring is filled
@@ -657,7 +913,7 @@ __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uin
       for (int w = 1; w < WAVES; ++w) v = v + partial[w][r][l];
       const int64_t row = (r >> 2) * 8 + (l >> 5) * 4 + (r & 3);
       const int64_t c = tile[j] * 32 + (l & 31);
-      if (row < M && c < N) y[row * N + c] = uint16_t(f32_to_f16_bits(v));
+      if (row < M && c < N) y[row * N + c] = narrow_with_bias(v, bias, c);
     }
   }
 }
@@ -669,27 +925,27 @@ __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uin
 template <int G>
 __device__ __forceinline__ void skinny_tiles(const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp,
                                              const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
-                                             int64_t K, int64_t N, int64_t block, int8_t* lds) {
+                                             int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias, int8_t* lds) {
   const int64_t tiles = (N + 31) / 32;
   if (int64_t(blockIdx.x) + gridDim.x < tiles)
-    skinny<G, 4, 2>(a, wp, scale, y, M, K, N, block, lds);
+    skinny<G, 4, 2>(a, wp, scale, y, M, K, N, block, bias, lds);
   else
-    skinny<G, 4, 1>(a, wp, scale, y, M, K, N, block, lds);
+    skinny<G, 4, 1>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 
 // M <= 16: half the activation rows per stage (8 waves splitting K were no faster than 4).
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny16(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
   __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 2 * 1024];
-  skinny_tiles<2>(a, wp, scale, y, M, K, N, block, lds);
+  skinny_tiles<2>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 // M <= 32: 4 waves split K.
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
   __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 4 * 1024];
-  skinny_tiles<4>(a, wp, scale, y, M, K, N, block, lds);
+  skinny_tiles<4>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 
 // ---- M <= 16: one strip of columns per compute unit --------------------------------------------------
@@ -711,7 +967,7 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 template <int WAVES, int JT>
 __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws,
                                              const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
-                                             int64_t K, int64_t N, int64_t block, int64_t tile0, int8_t* lds) {
+                                             int64_t K, int64_t N, int64_t block, int64_t tile0, const uint16_t* __restrict__ bias, int8_t* lds) {
   constexpr int kStages = 4, kStageBytes = 16 * 256;   // 16 rows x 128 k of f16
   constexpr int kLoads = 4 + 2 * JT;                   // memory instructions per slice and wave
   static_assert(3 * kLoads < 64, "wait counter range");
@@ -839,7 +1095,7 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
     for (int w = 1; w < WAVES; ++w) v = v + partial[((w * JT + j) * 4 + r) * 64 + l];
     const int64_t row = 4 * (l >> 4) + r;
     const int64_t c = (tile0 + j) * 16 + (l & 15);
-    if (row < M && c < N) y[row * N + c] = uint16_t(f32_to_f16_bits(v));
+    if (row < M && c < N) y[row * N + c] = narrow_with_bias(v, bias, c);
   }
   __syncthreads();                                     // the next chunk of this workgroup reuses the LDS
 }
@@ -856,7 +1112,7 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
 constexpr int kStripWaves = 4;
 extern "C" __global__ void __launch_bounds__(64 * kStripWaves) mtrt_gemm_w4a16_strips16(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
   __shared__ __attribute__((aligned(16))) int8_t lds[kStripWaves * 4 * 4096];
   // tiles / grid tiles each, the first tiles % grid workgroups one more (32-bit arithmetic: as 64-bit divisions this was
   // a microsecond of scalar instructions in front of the first load)
@@ -865,9 +1121,9 @@ extern "C" __global__ void __launch_bounds__(64 * kStripWaves) mtrt_gemm_w4a16_s
   const int64_t t0 = int64_t(b * per + (b < rem ? b : rem)), t1 = t0 + per + (b < rem ? 1 : 0);
   for (int64_t t = t0; t < t1; t += 3) {
     const int64_t left = t1 - t;
-    if (left >= 3) strips_chunk<kStripWaves, 3>(a, ws, scale, y, M, K, N, block, t, lds);
-    else if (left == 2) strips_chunk<kStripWaves, 2>(a, ws, scale, y, M, K, N, block, t, lds);
-    else strips_chunk<kStripWaves, 1>(a, ws, scale, y, M, K, N, block, t, lds);
+    if (left >= 3) strips_chunk<kStripWaves, 3>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else if (left == 2) strips_chunk<kStripWaves, 2>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else strips_chunk<kStripWaves, 1>(a, ws, scale, y, M, K, N, block, t, bias, lds);
   }
 }
 

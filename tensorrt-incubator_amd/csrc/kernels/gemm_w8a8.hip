@@ -120,24 +120,23 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
 }
 
 // ---- weights in fragment order (gemm_frag.hpp) ---------------------------------------------------------
-// mtrt_gemm_w8a8_frag[_rows128 | _t<rows>x<columns>] (a [M,K] i8, w_frag, a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, splits,
-// partial, tickets, a_step, bias) ; K % 128 == 0, a and w_frag 16-byte aligned, a below 4 GiB; a_step 1, or 0 for a
-// single a_scale; bias f16 [N] or null; splits workgroups per tile, each a range of K (1 .. K / 128; partial: splits x
-// tiles x rows x columns x 4 bytes, tickets: a zeroed word per tile; both unused with one).
+// mtrt_gemm_w8a8_frag[_rows128 | _t<rows>x<columns>] (a [M,K] i8, w_frag, a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, Split,
+// a_step, bias) ; K % 128 == 0, a and w_frag 16-byte aligned, a below 4 GiB; a_step 1, or 0 for a
+// single a_scale; bias f16 [N] or null.
 // grid = 8 * ceil(tiles * splits / 8), block = 256.  Tiles of 64 x 128 (no suffix), 32 x 128 (_rows128), 128 x 128 (two
 // workgroups per compute unit), 128 x 256, 128 x 384 and 256 x 256 (one; the last never split).  Which tile and how many splits: the host's
-// estimate of the launch (frag_tiles in clusters.cpp).  Measured, the one 256-row tile loop that these replaced -> now,
+// estimate of the launch (frag_plan in clusters.cpp).  Measured, the one 256-row tile loop that these replaced -> now,
 // us: (M, K, N) = (256, 4096, 4096) 21.8 -> 10.4, (398, 11520, 1856) 51.8 -> 19.3, (1024, 2048, 2048) 14.7 -> 8.8,
 // (200, 12288, 512) 52.7 -> 10.6, (999, 4096, 11008) 46.5 -> 44.
 #define MTRT_W8_FRAG_KERNEL(NAME, IT, JT, D, WG)                                                                          \
   extern "C" __global__ void __launch_bounds__(256, WG) NAME(                                                             \
       const int8_t* __restrict__ a, const int8_t* __restrict__ w_frag, const float* __restrict__ a_scale,                 \
-      const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t splits,      \
-      f32x4* partial, uint32_t* tickets, uint32_t a_step, const uint16_t* __restrict__ bias) {                            \
+      const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N,                       \
+      gemm_frag::Split sp, uint32_t a_step, const uint16_t* __restrict__ bias) {                                          \
     using Epilogue = ScaleEpilogueT<128 * JT, true>;                                                                      \
     __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<IT, D>(Epilogue::kScratch)];                  \
     gemm_frag::Part part;                                                                                                 \
-    if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, K / 128, splits, partial, tickets, part)) return; \
+    if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / 128, sp, part)) return; \
     Epilogue epi{a_scale, w_scale, a_step, bias};                                                                         \
     gemm_frag::run<I8Traits, IT, JT, D>(a, K, w_frag, epi, y, M, N, part, lds);                                           \
   }

@@ -52,10 +52,32 @@ constexpr double kW4BigRoundPerSmallRound = 3.25, kW4PartialRoundBase = 0.56, kW
 // data, old and new in one process: M = 4096, 3 rounds against 2, 298.4 -> 286.8 us; M = 8192 600 -> 571; M = 2048, two
 // rounds against one, 181 -> 145).
 constexpr double kW4WideRoundPerBigRound = 1.5 * 0.95;
-// ... and a round of 128 x 256 tiles 1.9 rounds of 128 x 128 tiles (0.48 against 0.37 us per 64-k slice and a longer
-// start and end; at 15 shapes with M = 300 ... 2048, (K, N) = (4096, 11008), (4096, 4096), (11008, 4096), (8192, 8192),
-// (5120, 13824) the estimate takes the fastest of the four tiles at every one).
+// ... and a round of 128 x 256 tiles 1.9 rounds of 128 x 128 tiles.
 constexpr double kW4Mid256RoundPerSmallRound = 1.9;
+// W4A16 tiles in time: n = tiles * splits workgroups of s = slices / splits slices of 64 k each, in L = ceil(n / units)
+// rounds the last of which is filled to f:
+//   fixed + (e + c s) (L - 1 + p + (1 - p) f^2) + (splits > 1 ? meet + meet_each * splits : 0)   us
+// (a launch that leaves units idle is shorter, more so for the large tiles: the clock is power's).  Fitted to 17000
+// launches of 621 log-uniform shapes, M 33 ... 4096, K 256 ... 14336, N 64 ... 16384, 1 to 12 splits.
+struct W4Tile {
+  const char *suffix;                                  // of the kernel's name
+  int rows, columns, threads;
+  bool splits;                                         // whether its K may be split
+  double fixed, e, c, p, meet, meet_each;
+};
+constexpr W4Tile kW4Tiles[] = {
+    {"t32x128", 32, 128, 256, true, 2.64, 0.89, 0.197, 1.0, 1.59, 0.334},
+    {"t64x128", 64, 128, 512, true, 0.99, 3.35, 0.252, 0.83, 2.59, 0.46},
+    {"t64x256", 64, 256, 256, true, 0.0, 4.38, 0.497, 0.79, 4.02, 0.645},
+    {"t128x128", 128, 128, 512, true, 0.0, 5.76, 0.523, 0.474, 3.54, 0.725},
+    {"t128x256", 128, 256, 256, true, 0.0, 5.98, 1.046, 0.467, 5.8, 1.19},
+    {"t256x256", 256, 256, 256, false, 0.0, 7.3, 1.589, 0.615, 0.0, 0.0},
+    {"t256x384", 256, 384, 256, false, 0.0, 8.46, 2.637, 0.525, 0.0, 0.0},
+};
+// The tile by rounds (above) is the better founded choice where the estimates are close: another tile or a split has to
+// promise a tenth.  Over the same launches, the chosen one against the fastest in each: 1.8 % longer on average; against
+// the choice by rounds alone 1.44 times as fast, 0.95 at worst.
+constexpr double kW4Promise = 0.9;
 // Tiles on fragment-order weights (gemm_frag.hpp).  A launch of `tiles * splits` workgroups, L = ceil of that over the
 // compute units, each running s = slices / splits slices of 128 bytes of K, is estimated as
 //   max(first + first_slice * s, L * (next + next_slice * s)) + (splits > 1 ? meet + meet_each * splits : 0)   us.
@@ -83,14 +105,26 @@ constexpr double kFragRows32Us = 2.0, kFragRows32TileUs = 1.2, kFragRows32SliceU
 constexpr double kFragRows64Us = 1.6, kFragRows64TileUs = 1.9, kFragRows64SliceUs = 0.165;
 } // namespace tuning
 
+// gemm_frag::Split, the kernels' argument of this layout.
+struct FragSplit {
+  uint32_t splits = 1, per = 0;
+  void *partial = nullptr;
+  uint32_t *tickets = nullptr;
+};
+// `splits` parts of equal length; fewer where the last ones would have nothing left.
+FragSplit split_of(int64_t slices, int splits) {
+  const int64_t per = (slices + splits - 1) / splits;
+  return {uint32_t((slices + per - 1) / per), uint32_t(per), nullptr, nullptr};
+}
+
 // The tile and the K split of a GEMM on fragment-order weights (see tuning::kFragTiles).
 struct FragPlan {
   const tuning::FragTile *tile = nullptr;
   int64_t tiles = 0;
-  uint32_t splits = 1;
+  FragSplit split;
   double us = 0.0;
-  uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(splits) + 7) / 8)); }
-  int64_t workspace() const { return splits > 1 ? tiles * int64_t(splits) * tile->rows * tile->columns * 4 : 0; }
+  uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(split.splits) + 7) / 8)); }
+  int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * tile->rows * tile->columns * 4 : 0; }
 };
 FragPlan frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may_split) {
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
@@ -103,11 +137,12 @@ FragPlan frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may
       // a part of at least two slices, a ticket for every split tile, and no more workgroups than two rounds hold
       if (splits > 1 && (!may_split || !t.splits || slices < 2 * splits || tiles > int64_t(kTickets) || tiles * splits > 2 * units))
         break;
-      const double s = double((slices + splits - 1) / splits), rounds = double((tiles * splits + units - 1) / units);
+      const FragSplit split = split_of(slices, splits);
+      const double s = double(split.per), rounds = double((tiles * int64_t(split.splits) + units - 1) / units);
       const double us = std::max(t.first + t.first_slice * s, rounds * (t.next + t.next_slice * s)) +
-                        (splits > 1 ? t.meet + t.meet_each * splits : 0.0);
+                        (split.splits > 1 ? t.meet + t.meet_each * split.splits : 0.0);
       if (!best.tile || us < best.us)
-        best = {&t, tiles, uint32_t(splits), us};
+        best = {&t, tiles, split, us};
     }
   }
   return best;
@@ -118,6 +153,70 @@ double frag_rows_us(int64_t M, int64_t N, int64_t slices, int64_t units) {
   if (M <= 32)
     return kFragRows32Us + rounds * (kFragRows32TileUs + s * (rounds > 1.0 ? kFragRows32LaterSliceUs : kFragRows32SliceUs));
   return kFragRows64Us + rounds * (kFragRows64TileUs + s * kFragRows64SliceUs);
+}
+
+
+// Tile and K split of a W4A16 launch of more than 32 rows.
+struct W4Plan {
+  const tuning::W4Tile *tile = nullptr;
+  int64_t tiles = 0;
+  FragSplit split;
+  double us = 0.0;
+  bool narrow = false;                                 // 128 x 64 tiles: matrices of at most 64 columns, where 128 x 128 would run
+  const char *by_rounds = nullptr;                     // the tile the choice by rounds names: how the launch is reported
+  uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(split.splits) + 7) / 8)); }
+  int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * tile->rows * tile->columns * 4 : 0; }
+};
+W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
+  using namespace tuning;
+  static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
+  const int64_t slices = K / 64;
+  auto tiles_of = [&](const W4Tile &t) { return ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns); };
+  auto plan_of = [&](const W4Tile &t, int splits) {
+    W4Plan p;
+    p.tile = &t;
+    p.tiles = tiles_of(t);
+    p.split = split_of(slices, splits);
+    const int64_t n = p.tiles * p.split.splits, full = (n - 1) / units;
+    const double s = double(p.split.per), f = double(n - full * units) / double(units);
+    p.us = t.fixed + (t.e + t.c * s) * (double(full) + t.p + (1.0 - t.p) * f * f) +
+           (p.split.splits > 1 ? t.meet + t.meet_each * p.split.splits : 0.0);
+    return p;
+  };
+  auto fits = [](int64_t tiles) { return tiles <= int64_t(kMaxGrid) * 1024 - 8; };
+  // 128- and 256-row tiles by rounds
+  auto rounds = [units](int64_t tiles) {
+    const double f = double(tiles % units) / double(units);
+    return double(tiles / units) + (tiles % units ? kW4PartialRoundBase + kW4PartialRoundSlope * f * f : 0.0);
+  };
+  const W4Tile &t128 = kW4Tiles[3], &t256w = kW4Tiles[4], &big = kW4Tiles[5], &wide = kW4Tiles[6];
+  const double cost128 = rounds(tiles_of(t128)), cost256w = N > 64 ? kW4Mid256RoundPerSmallRound * rounds(tiles_of(t256w)) : cost128;
+  const double cost_big = kW4BigRoundPerSmallRound * rounds(tiles_of(big));
+  const double cost_wide = kW4BigRoundPerSmallRound * kW4WideRoundPerBigRound * rounds(tiles_of(wide));
+  const double smaller = std::min(cost128, cost256w);
+  const W4Tile *by_rounds = cost_wide < cost_big && cost_wide < smaller ? &wide : cost_big < smaller ? &big : cost256w < cost128 ? &t256w : &t128;
+  if (!fits(tiles_of(*by_rounds)))
+    by_rounds = &wide;
+  W4Plan best;
+  if (M > 64 && fits(tiles_of(*by_rounds))) {
+    best = plan_of(*by_rounds, 1);
+    best.narrow = by_rounds == &t128 && N <= 64;
+    best.us *= kW4Promise;
+  }
+  for (const W4Tile &t : kW4Tiles) {
+    if (!fits(tiles_of(t)))
+      continue;
+    for (int splits : kSplits) {
+      // as for frag_plan: a part of at least two slices, a ticket for every split tile, at most two rounds of workgroups
+      if (splits > 1 && (!may_split || !t.splits || slices < 2 * splits || tiles_of(t) > int64_t(kTickets) || tiles_of(t) * splits > 2 * units))
+        break;
+      const W4Plan p = plan_of(t, splits);
+      if (!best.tile || p.us < best.us)
+        best = p;
+    }
+  }
+  best.by_rounds = by_rounds == &t128 && N <= 64 ? "t128x64" : by_rounds->suffix;
+  return best;
 }
 
 const char *float_name(int32_t dt) {
@@ -993,6 +1092,18 @@ W8Plan w8_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   return {W8Plan::kTile, tile};
 }
 
+// The memory of a split launch: the caller's workspace and the stream's tickets.
+bool bind_split(DeviceState *st, hipStream_t stream, FragSplit &split, void *workspace) {
+  if (split.splits <= 1)
+    return true;
+  uint32_t *slot = reduction_slot(st, stream);
+  if (!slot)
+    return false;
+  split.partial = workspace;
+  split.tickets = slot + kTicketOffset;
+  return true;
+}
+
 // a_step: 1 for a scale per row, 0 for one scale; bias: f16 [N] or null; workspace: for K-split tiles, may be null.
 int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, const float *a_scale, uint32_t a_step, const float *w_scale,
                        const void *bias, void *y, int64_t M, int64_t K, int64_t N, void *workspace, int64_t workspace_bytes) {
@@ -1038,20 +1149,15 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     return launch(st, KernelName(plain ? "mtrt_gemm_w8a8_frag_t256x384" : "mtrt_gemm_w8a8_frag_t256x384_linear").as("mtrt_gemm_w8a8_frag_t256x384"),
                   p.grid(), 256, stream, args);
   }
-  uint32_t splits = p.splits;
-  uint32_t *tickets = nullptr;
-  if (splits > 1) {
-    tickets = reduction_slot(st, stream);
-    if (!tickets)
-      return MTRT_RUNTIME_ERROR;
-    tickets += kTicketOffset;
-  }
+  FragSplit split = p.split;
+  if (!bind_split(st, stream, split, workspace))
+    return MTRT_RUNTIME_ERROR;
   KernelName name("mtrt_gemm_w8a8_frag");
   if (p.tile->rows == 32)
     name + "_rows128";
   else if (p.tile->rows != 64)
     name + "_" + p.tile->suffix;
-  void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &splits, &workspace, &tickets, &a_step, &bias};
+  void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &split, &a_step, &bias};
   return launch(st, name.as(p.tile->rows == 32 && M > 64 && M <= 128 ? "mtrt_gemm_w8a8_frag_rows128" : "mtrt_gemm_w8a8_frag"), p.grid(), 256,
                 stream, args);
 }
@@ -1189,9 +1295,14 @@ int32_t mtrt_hip_gemm_w4a16_prepack(mtrt_stream_t stream, const void *w_kn_packe
   return launch(st, KernelName("mtrt_w4_prepack_strips"), blocks_for(w4_strip_bytes(K, N) / 4, kBlock), kBlock, as_hip(stream), args2);
 }
 
-int32_t mtrt_hip_gemm_w4a16(mtrt_stream_t stream, const void *a, const void *w_kn_packed, const void *w_prepacked,
-                            const void *scale, void *y, int64_t M, int64_t K, int64_t N, int64_t block) {
-  clear_error();
+namespace {
+bool w4_fast(const void *a, const void *w_prepacked, int64_t K, int64_t block) {
+  return w_prepacked && K > 0 && K % 64 == 0 && block % 64 == 0 && aligned(a, 16) && aligned(w_prepacked, 16);
+}
+
+// bias: f16 [N], added to the rounded product, or null (only with re-laid weights)
+int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const void *w_prepacked, const void *scale, const void *bias, void *y,
+              int64_t M, int64_t K, int64_t N, int64_t block, void *workspace, int64_t workspace_bytes) {
   if (M < 0 || K < 0 || N < 0)
     return set_error(MTRT_INVALID_ARGUMENT, "negative extent M=%lld K=%lld N=%lld", (long long)M, (long long)K,
                      (long long)N);
@@ -1204,77 +1315,51 @@ int32_t mtrt_hip_gemm_w4a16(mtrt_stream_t stream, const void *a, const void *w_k
     return set_error(MTRT_INVALID_ARGUMENT, "block size %lld does not divide K=%lld", (long long)block, (long long)K);
   if (!y || (K > 0 && (!a || !scale)) || (!w_kn_packed && !w_prepacked && K > 0))
     return set_error(MTRT_INVALID_ARGUMENT, "null operand");
-  if (!aligned(a, 2) || !aligned(y, 2) || !aligned(scale, 2))
+  if (!aligned(a, 2) || !aligned(y, 2) || !aligned(scale, 2) || !aligned(bias, 2))
     return set_error(MTRT_INVALID_ARGUMENT, "operand is not aligned to its element size");
   DeviceState *st = device_state();
   if (!st)
     return MTRT_RUNTIME_ERROR;
-  const bool fast = w_prepacked && K > 0 && K % 64 == 0 && block % 64 == 0 && aligned(a, 16) && aligned(w_prepacked, 16);
-  if (fast && M > 32 && M <= 64) {
-    // Between 33 and 64 rows a 128-row tile is at least half padding and the launch lasts as long as one tile's K
-    // loop; two launches of the small-M kernels (rows 0..31, then the rest; the second finds the weights in cache)
-    // are shorter: M = 48 at (K, N) = (4096, 4096) 22.2 us as one tile launch, (11008, 4096) 52.0, (4096, 11008) 23.1.
-    const int32_t rc = mtrt_hip_gemm_w4a16(stream, a, w_kn_packed, w_prepacked, scale, y, 32, K, N, block);
-    if (rc != MTRT_OK)
-      return rc;
-    return mtrt_hip_gemm_w4a16(stream, static_cast<const char *>(a) + 32 * K * 2, w_kn_packed, w_prepacked, scale,
-                               static_cast<char *>(y) + 32 * N * 2, M - 32, K, N, block);
-  }
-  if (fast) {
-    void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block};
-    if (M <= 16 && K % 128 == 0 && block % 128 == 0) {
+  if (w4_fast(a, w_prepacked, K, block)) {
+    const bool strips = K % 128 == 0 && block % 128 == 0;
+    const int64_t cus = num_compute_units(st);
+    void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias};
+    if (M <= 16 && strips) {
       // one workgroup per compute unit, each a strip of 16-column tiles over all of K (weights in strip order)
-      const void *strips = static_cast<const char *>(w_prepacked) + w4_fragment_bytes(K, N);
-      void *sargs[] = {&a, &strips, &scale, &y, &M, &K, &N, &block};
+      const void *in_strips = static_cast<const char *>(w_prepacked) + w4_fragment_bytes(K, N);
+      void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias};
       const int64_t tiles = (N + 15) / 16;
-      return launch(st, KernelName("mtrt_gemm_w4a16_strips16"), uint32_t(std::min<int64_t>(tiles, num_compute_units(st))), kBlock,
-                    as_hip(stream), sargs);
+      return launch(st, KernelName("mtrt_gemm_w4a16_strips16"), uint32_t(std::min<int64_t>(tiles, cus)), kBlock, stream, sargs);
     }
     if (M <= 32) {
       // one workgroup per 32-column tile; between one and two tiles per compute unit, one workgroup per
       // compute unit instead (the kernel then gives workgroup g the tiles g and g + grid, which share the
       // activations; measured: 6 % faster at M = 16, 21 % at M = 32, 3 % slower at M = 5)
-      const int64_t tiles = (N + 31) / 32, cus = num_compute_units(st);
+      const int64_t tiles = (N + 31) / 32;
       const uint32_t grid = uint32_t(M > 8 && tiles > cus && tiles <= 2 * cus ? cus : tiles);
-      return launch(st, KernelName(M <= 16 ? "mtrt_gemm_w4a16_skinny16" : "mtrt_gemm_w4a16_skinny"), grid, kBlock, as_hip(stream), args);
+      return launch(st, KernelName(M <= 16 ? "mtrt_gemm_w4a16_skinny16" : "mtrt_gemm_w4a16_skinny"), grid, kBlock, stream, args);
     }
-    // 256 x 384 or 256 x 256 tiles (four waves) or 128 x 256 / 128 x 128 tiles (eight waves), one workgroup per compute unit at a time.  A
-    // launch runs in rounds of one tile per unit; a full round of the large tile takes 3.25 times a full round of
-    // the small one for four times the work, and a partly filled last round is shorter than a full one (fewer
-    // units share the power budget): 0.56 + 0.44 f^2 of it at fill f (measured over M = 48 ... 4096 at (K, N) =
-    // (4096, 4096), (4096, 11008), (11008, 4096), (8192, 8192), (5120, 13824), (4096, 14336), (8192, 28672),
-    // (4096, 2048): the estimate picks the faster kernel in all but near-ties; 128 x 64 tiles were never ahead
-    // by more than 1 % there and only serve matrices at most 64 columns wide).
     if (M * K * 2 < (int64_t(1) << 32)) {
-      const int64_t units = num_compute_units(st);
-      const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256, big_tiles = panels * tiles_m;
-      const int64_t wide_panels = (N + 127) / 128, wide_m = (M + 127) / 128, wide_tiles = wide_panels * wide_m;
-      auto rounds = [units](int64_t tiles) {
-        const double f = double(tiles % units) / double(units);
-        return double(tiles / units) + (tiles % units ? tuning::kW4PartialRoundBase + tuning::kW4PartialRoundSlope * f * f : 0.0);
-      };
-      // (grids: the tiles dealt evenly to the eight XCDs, gemm_core::tile_of_even)
-      const int64_t big = 8 * ((big_tiles + 7) / 8), wide = 8 * ((wide_tiles + 7) / 8);
-      const int64_t narrow = 8 * ((((N + 63) / 64) * wide_m + 7) / 8);
-      const int64_t huge_tiles = ((N + 383) / 384) * tiles_m, huge = 8 * ((huge_tiles + 7) / 8);
-      const int64_t mid_tiles = panels * wide_m, mid = 8 * ((mid_tiles + 7) / 8);   // 128 x 256
-      const double big_cost = tuning::kW4BigRoundPerSmallRound * rounds(big_tiles);
-      const double huge_cost = tuning::kW4BigRoundPerSmallRound * tuning::kW4WideRoundPerBigRound * rounds(huge_tiles);
-      const double mid_cost = tuning::kW4Mid256RoundPerSmallRound * rounds(mid_tiles);
-      const double small_cost = std::min(rounds(wide_tiles), mid_cost);
-      if (huge_cost < big_cost && huge_cost < small_cost && huge <= int64_t(kMaxGrid) * 1024)
-        return launch(st, KernelName("mtrt_gemm_w4a16_t256x384"), uint32_t(huge), 256, as_hip(stream), args);
-      if (big_cost < small_cost && big <= int64_t(kMaxGrid) * 1024)
-        return launch(st, KernelName("mtrt_gemm_w4a16_t256x256"), uint32_t(big), 256, as_hip(stream), args);
-      if (mid_cost < rounds(wide_tiles) && N > 64 && mid <= int64_t(kMaxGrid) * 1024)
-        return launch(st, KernelName("mtrt_gemm_w4a16_t128x256"), uint32_t(mid), 512, as_hip(stream), args);
-      if (N <= 64 && narrow <= int64_t(kMaxGrid) * 1024)
-        return launch(st, KernelName("mtrt_gemm_w4a16_t128x64"), uint32_t(narrow), kBlock, as_hip(stream), args);
-      if (wide <= int64_t(kMaxGrid) * 1024)
-        return launch(st, KernelName("mtrt_gemm_w4a16_t128x128"), uint32_t(wide), 512, as_hip(stream), args);
+      W4Plan p = w4_plan(M, K, N, cus, true);
+      if (p.workspace() > (workspace && aligned(workspace, 16) ? workspace_bytes : 0))
+        p = w4_plan(M, K, N, cus, false);
+      if (p.tile) {
+        // reported by the class of shapes: up to 64 rows as the small-M kernel of the rows past 32, else as the tile by rounds
+        const char *shown = M > 64 ? p.by_rounds : M > 48 ? "skinny" : strips ? "strips16" : "skinny16";
+        KernelName name("mtrt_gemm_w4a16_");
+        name + (p.narrow ? "t128x64" : p.tile->suffix) + (bias ? "_bias" : "");
+        name.as(KernelName("mtrt_gemm_w4a16_") + shown);
+        if (p.tile->rows == 256)
+          return launch(st, name, p.grid(), p.tile->threads, stream, args);
+        FragSplit split = p.split;
+        if (!bind_split(st, stream, split, workspace))
+          return MTRT_RUNTIME_ERROR;
+        void *targs[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias, &split};
+        return launch(st, name, p.grid(), p.narrow ? 256 : p.tile->threads, stream, targs);
+      }
     }
   }
-  if (!w_kn_packed)
+  if (!w_kn_packed || bias)
     return set_error(MTRT_INVALID_ARGUMENT, "this shape needs the original packed weights (K=%lld block=%lld)",
                      (long long)K, (long long)block);
   void *args[] = {&a, &w_kn_packed, &scale, &y, &M, &K, &N, &block};
@@ -1283,9 +1368,33 @@ int32_t mtrt_hip_gemm_w4a16(mtrt_stream_t stream, const void *a, const void *w_k
     // weight stage is dequantised in the kernel (M = 256, K = N = 4096, block 32: 3660 us on the kernel below)
     const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
     return launch(st, KernelName("mtrt_gemm_w4a16_edge"), uint32_t(std::min<int64_t>(tiles, int64_t(kMaxGrid) * 1024)), kBlock,
-                  as_hip(stream), args);
+                  stream, args);
   }
-  return launch(st, KernelName("mtrt_gemm_w4a16_any"), blocks_for(M * N, kBlock), kBlock, as_hip(stream), args);
+  return launch(st, KernelName("mtrt_gemm_w4a16_any"), blocks_for(M * N, kBlock), kBlock, stream, args);
+}
+} // namespace
+
+int32_t mtrt_hip_gemm_w4a16(mtrt_stream_t stream, const void *a, const void *w_kn_packed, const void *w_prepacked,
+                            const void *scale, void *y, int64_t M, int64_t K, int64_t N, int64_t block) {
+  clear_error();
+  return w4a16(as_hip(stream), a, w_kn_packed, w_prepacked, scale, nullptr, y, M, K, N, block, nullptr, 0);
+}
+
+int64_t mtrt_hip_gemm_w4a16_workspace(int64_t M, int64_t K, int64_t N, int64_t block) {
+  if (M <= 32 || K <= 0 || N <= 0 || block <= 0 || K % 64 != 0 || block % 64 != 0 || M > kMaxMatrixExtent || K > kMaxMatrixExtent ||
+      N > kMaxMatrixExtent || M * K * 2 >= (int64_t(1) << 32))
+    return 0;
+  DeviceState *st = device_state();
+  if (!st)
+    return 0;
+  const W4Plan p = w4_plan(M, K, N, num_compute_units(st), true);
+  return p.tile ? p.workspace() : 0;
+}
+
+int32_t mtrt_hip_gemm_w4a16_ws(mtrt_stream_t stream, const void *a, const void *w_kn_packed, const void *w_prepacked, const void *scale,
+                               void *y, int64_t M, int64_t K, int64_t N, int64_t block, void *workspace, int64_t workspace_bytes) {
+  clear_error();
+  return w4a16(as_hip(stream), a, w_kn_packed, w_prepacked, scale, nullptr, y, M, K, N, block, workspace, workspace_bytes);
 }
 
 namespace {
@@ -1318,15 +1427,10 @@ int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, cons
   }
   if (!plan.tile.tile)
     return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
-  uint32_t splits = plan.tile.splits;
-  uint32_t *tickets = nullptr;
-  if (splits > 1) {
-    tickets = reduction_slot(st, stream);
-    if (!tickets)
-      return MTRT_RUNTIME_ERROR;
-    tickets += kTicketOffset;
-  }
-  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &splits, &partial, &tickets};
+  FragSplit split = plan.tile.split;
+  if (!bind_split(st, stream, split, partial))
+    return MTRT_RUNTIME_ERROR;
+  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &split};
   return launch(st, name, plan.tile.grid(), 256, stream, args);
 }
 
@@ -1406,7 +1510,7 @@ const char *linear_fault(const mtrt_hip_linear_plan *p, int64_t M) {
     return "activations go through i8, f8E4M3FN or i4 codes";
   if (p->route == MTRT_LINEAR_W8A8 && (p->q_dtype != MTRT_I8 || !p->x_scale || !p->w_scale || (!p->w && !p->w_frag)))
     return "W8A8 needs int8 activations, both scales and weights";
-  if (p->route == MTRT_LINEAR_W4A16 && (p->q_dtype >= 0 || p->bias || !p->w_frag || !p->w_scale || p->K % 64 != 0))
+  if (p->route == MTRT_LINEAR_W4A16 && (p->q_dtype >= 0 || !p->w_frag || !p->w_scale || p->K % 64 != 0))
     return "W4A16 needs plain activations, re-laid weights, their scales and K % 64 == 0";
   if (p->route == MTRT_LINEAR_DENSE && ((p->q_dtype >= 0 && !p->x_scale) || (!p->w && !(p->w_frag && float_bytes(p->dtype) == 2))))
     return "the dense route needs weights, and a scale where it quantizes";
@@ -1450,6 +1554,10 @@ int64_t mtrt_hip_linear_workspace(const mtrt_hip_linear_plan *plan, int64_t M) {
   const int64_t most = linear_rows(*plan, M), last = M % most;
   for (int64_t rows : {most, last}) {
     if (rows > 0) {
+      if (plan->route == MTRT_LINEAR_W4A16) {
+        need = std::max(need, mtrt_hip_gemm_w4a16_workspace(rows, plan->K, plan->N, plan->K));
+        continue;
+      }
       const LinearShape s = linear_shape(*plan, rows, num_compute_units(st));
       need = std::max(need, s.act_bytes + s.partial_bytes);
     }
@@ -1473,8 +1581,6 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   DeviceState *st = device_state();
   if (!st)
     return MTRT_RUNTIME_ERROR;
-  if (p.route == MTRT_LINEAR_W4A16)
-    return mtrt_hip_gemm_w4a16(stream, x, nullptr, p.w_frag, p.w_scale, y, M, p.K, p.N, p.K);
   const int64_t most = linear_rows(p, M);
   if (most < M) {
     for (int64_t m0 = 0; m0 < M; m0 += most) {
@@ -1485,6 +1591,8 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
     }
     return MTRT_OK;
   }
+  if (p.route == MTRT_LINEAR_W4A16)
+    return w4a16(as_hip(stream), x, nullptr, p.w_frag, p.w_scale, p.bias, y, M, p.K, p.N, p.K, workspace, workspace_bytes);
   const LinearShape s = linear_shape(p, M, num_compute_units(st));
   if (s.fragments && !s.pass && !aligned(x, 16))
     return set_error(MTRT_INVALID_ARGUMENT, "x must be 16-byte aligned for these weights");

@@ -100,3 +100,52 @@ def test_w8a8_split_launches_on_two_streams_and_in_a_graph(pkg):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y, pkg.gemm_w8a8_fragments(static, frag[0], a_s, w_s, 512)), k
+
+
+def _w4_inputs(seed, M, K, N, B):
+    import torch
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    a = torch.randn((M, K), generator=g, device="cuda").half()
+    q = torch.randint(-8, 8, (K, N), generator=g, device="cuda")
+    s = (torch.rand((K // B, N), generator=g, device="cuda") * 0.02 + 0.005).half()
+    nibbles = (q & 15).to(torch.uint8).reshape(-1)
+    if nibbles.numel() % 2:
+        nibbles = torch.cat([nibbles, nibbles.new_zeros(1)])
+    return a, (nibbles[0::2] | (nibbles[1::2] << 4)).contiguous(), s, (q.half() * s.repeat_interleave(B, 0)).double()
+
+
+# (M, K, N, block): every tile up to 128 rows, split and not, ragged rows and columns, blocks of one slice and of all of K
+@pytest.mark.parametrize("case", [(33, 4096, 200, 128), (48, 2048, 1000, 64), (64, 8192, 96, 8192), (65, 1152, 129, 192), (100, 12288, 300, 128),
+                                  (130, 4096, 4096, 128), (200, 384, 8, 64), (256, 8192, 2051, 256), (300, 4096, 3000, 128), (600, 256, 40, 64),
+                                  (700, 4864, 60, 128), (1000, 640, 2000, 128), (1800, 640, 1160, 128), (517, 64, 472, 64), (2000, 2048, 769, 128)])
+def test_w4a16_tiles_and_splits(pkg, case):
+    """Against float64 on the dequantised weights: products exact, f32 sums in any order, one rounding to f16; nothing
+    around the output is written; the same bits on every launch."""
+    import torch
+    M, K, N, B = case
+    a, packed, s, wd = _w4_inputs(M + K + N, M, K, N, B)
+    pre = pkg.gemm_w4a16_prepack(packed, K, N)
+    ref, mass = a.double() @ wd, a.double().abs() @ wd.abs()
+    tol = 2.0 ** -11 * ref.abs() + (1 + 2.0 ** -11) * (K + 1) * 2.0 ** -24 * mass + 2.0 ** -25
+
+    buf = torch.full((M * N + 9,), 7.0, dtype=torch.float16, device="cuda")
+    y = buf[1:1 + M * N].view(M, N)
+    pkg.gemm_w4a16(a, s, K, N, B, w_prepacked=pre, out=y)
+    assert bool(((y.double() - ref).abs() <= tol).all()) and float(buf[0]) == 7.0 and bool((buf[1 + M * N:] == 7.0).all())
+    for _ in range(3):
+        assert torch.equal(pkg.gemm_w4a16(a, s, K, N, B, w_prepacked=pre), y)
+    L = pkg.lib()
+    need = L.mtrt_hip_gemm_w4a16_workspace(M, K, N, B)
+    z = torch.empty((M, N), dtype=torch.float16, device="cuda")
+    scratch = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    stream = torch.cuda.current_stream().cuda_stream
+    pkg.check(L.mtrt_hip_gemm_w4a16_ws(stream, a.data_ptr(), None, pre.data_ptr(), s.data_ptr(), z.data_ptr(), M, K, N, B, scratch.data_ptr(),
+                                       need - 1 if need else 0))                     # too little: unsplit
+    assert bool(((z.double() - ref).abs() <= tol).all())
+
+
+def test_some_w4a16_shape_is_split(pkg):
+    L = pkg.lib()
+    assert L.mtrt_hip_gemm_w4a16_workspace(64, 8192, 96, 128) > 0
+    assert L.mtrt_hip_gemm_w4a16_workspace(32, 8192, 96, 128) == 0 and L.mtrt_hip_gemm_w4a16_workspace(64, 8192, 96, 96) == 0

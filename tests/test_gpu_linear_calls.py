@@ -46,7 +46,7 @@ SHAPES = [(1, 64, 32), (16, 4096, 100), (32, 10496, 384), (33, 2048, 40), (64, 1
           (3, 65, 33), (17, 71, 640), (40, 1031, 260), (300, 2049, 1000), (900, 1023, 1030)]
 
 
-@pytest.mark.parametrize("qname,x_scale", [(None, False), ("float8", True), ("int8", True), ("int4", True), ("int8", False)])
+@pytest.mark.parametrize("qname,x_scale", [(None, False), ("float8", True), ("int8", True), ("int4", True), ("int8", False), ("int4", False)])
 @pytest.mark.parametrize("dname", ["float16", "bfloat16", "float32"])
 def test_linear_against_float64(tp, dname, qname, x_scale):
     import torch
@@ -64,10 +64,14 @@ def test_linear_against_float64(tp, dname, qname, x_scale):
             xd, wd = _operands(tp, lin, x)
         b = lin.bias.device_data().double() if lin.bias is not None else 0.0
         ref, mass = xd @ wd.T + b, xd.abs() @ wd.abs().T + (b.abs() if lin.bias is not None else 0.0)
+        assert qname != "int4" or x_scale or dname != "float16" or K % 64 or lin.route() == "w4a16"
         if lin.route() == "w8a8":
             # exact integer sums; two f32 products, a rounding to f16, the sum with the bias rounded once more
             core = ref - b
             tol = (3 * 2.0 ** -24 + u) * core.abs() + u * (ref.abs() + u * core.abs()) + 2.0 ** -24
+        elif lin.route() == "w4a16":                   # f32 sums rounded to f16, the sum with the bias rounded once more
+            core = ref - b
+            tol = u * core.abs() + (1 + u) * (K + 2) * 2.0 ** -24 * mass + u * ref.abs() * (1 + u) + 2.0 ** -24
         else:
             # f32 accumulation in any order (K additions, the products exact for 16-bit operands), one rounding
             tol = u * ref.abs() + (1 + u) * (K + 2) * 2.0 ** -24 * mass + 2.0 ** -24
