@@ -79,20 +79,26 @@ template <> struct FloatGroup<F16> {
 };
 
 // ---- quantized codes ---------------------------------------------------------------
-// enc(v): code of an already divided / rounded / clamped value.  dec(code): f32 value.
+// enc(v): code of an already divided, clamped and (for the float targets, where asked for) rounded value; the integer
+// targets round here.  dec(code): f32 value.
 // A group of G codes travels as G/4 (bytes) or G/8 (nibbles) 32-bit words; the
 // 4-nibble group of an f32 operand is a single 16-bit access.
 template <typename Q> struct Codes;
 
+// 1.5 x 2^23 + v for |v| < 2^22: the addition rounds v to a whole number, half to even as v_rndne does, and leaves it in
+// two's complement in the low bits.  One instruction instead of a rounding and a conversion; the low bytes of several
+// results are then gathered by v_perm.
+__device__ __forceinline__ uint32_t rounded_bits(float v) { return f32_to_bits(v + 12582912.0f); }
+
 template <> struct Codes<I8> {
   static constexpr float kLo = -128.0f, kHi = 127.0f;
-  static constexpr bool kAlwaysRound = true;
-  static __device__ __forceinline__ uint32_t enc(float v, int) { return uint32_t(int(v)) & 0xFFu; }
+  static constexpr bool kInteger = true;
+  static __device__ __forceinline__ uint32_t enc(float v, int) { return rounded_bits(v) & 0xFFu; }
   static __device__ __forceinline__ float dec(uint32_t c) { return float(int(c << 24) >> 24); }
 };
 template <> struct Codes<F8> {
   static constexpr float kLo = -448.0f, kHi = 448.0f;
-  static constexpr bool kAlwaysRound = false;
+  static constexpr bool kInteger = false;
   static __device__ __forceinline__ uint32_t enc(float v, int flags) {
     if (flags & kFlagF8RefHost) return f32_to_f8_refhost(v);
     if (flags & kFlagF8ViaF16) v = f16_bits_to_f32(f32_to_f16_bits(v));
@@ -104,16 +110,16 @@ template <> struct Codes<F8> {
 // DataTypes.cpp:494-519 keeps `bits_ & 0xF`).
 template <> struct Codes<I4> {
   static constexpr float kLo = -8.0f, kHi = 7.0f;
-  static constexpr bool kAlwaysRound = true;
-  static __device__ __forceinline__ uint32_t enc(float v, int) { return uint32_t(int(v)) & 0xFu; }
+  static constexpr bool kInteger = true;
+  static __device__ __forceinline__ uint32_t enc(float v, int) { return rounded_bits(v) & 0xFu; }
   static __device__ __forceinline__ float dec(uint32_t c) { return float(int(c << 28) >> 28); }
 };
 // int4 packed two per byte over the flattened array, element 2i in the low nibble
 // (mlir-tensorrt/tensorrt/lib/Target/TensorRTEncodingOpInterface/NetworkEncoder.cpp:552-595).
 template <> struct Codes<I4P> {
   static constexpr float kLo = -8.0f, kHi = 7.0f;
-  static constexpr bool kAlwaysRound = true;
-  static __device__ __forceinline__ uint32_t enc(float v, int) { return uint32_t(int(v)) & 0xFu; }
+  static constexpr bool kInteger = true;
+  static __device__ __forceinline__ uint32_t enc(float v, int) { return rounded_bits(v) & 0xFu; }
   static __device__ __forceinline__ float dec(uint32_t c) { return float(int(c << 28) >> 28); }
 };
 
@@ -130,7 +136,7 @@ __device__ __forceinline__ uint32_t f32x2_to_f4x2(float a, float b) {
 }
 template <> struct Codes<F4P> {
   static constexpr float kLo = -6.0f, kHi = 6.0f;
-  static constexpr bool kAlwaysRound = false;
+  static constexpr bool kInteger = false;
   static __device__ __forceinline__ uint32_t enc(float v, int) { return f32x2_to_f4x2(v, 0.0f) & 0xFu; }
   static __device__ __forceinline__ float dec(uint32_t c) { return __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(c & 0xFu, 1.0f, 0)[0]; }
 };
@@ -142,6 +148,15 @@ __device__ __forceinline__ uint32_t pack4(const float* v, int flags) {
   return Codes<Q>::enc(v[0], flags) | (Codes<Q>::enc(v[1], flags) << 8) | (Codes<Q>::enc(v[2], flags) << 16) |
          (Codes<Q>::enc(v[3], flags) << 24);
 }
+__device__ __forceinline__ uint32_t pack4_rounded(const float* v) {
+  const uint32_t lo = __builtin_amdgcn_perm(rounded_bits(v[1]), rounded_bits(v[0]), 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(rounded_bits(v[3]), rounded_bits(v[2]), 0x04000c0cu);
+  return lo | hi;
+}
+template <>
+__device__ __forceinline__ uint32_t pack4<I8>(const float* v, int) { return pack4_rounded(v); }
+template <>
+__device__ __forceinline__ uint32_t pack4<I4>(const float* v, int) { return pack4_rounded(v) & 0x0F0F0F0Fu; }
 template <>
 __device__ __forceinline__ uint32_t pack4<F8>(const float* v, int flags) {
   if (flags & kFlagF8RefHost) {
@@ -222,9 +237,9 @@ template <int G> struct CodeGroup<I4P, G> {
     uint32_t w = 0;
 #pragma unroll
     for (int k = 0; k < G; ++k) {
-      const int c = int(v[k]);
-      v[k] = float(c);
-      w |= (uint32_t(c) & 0xFu) << (4 * k);
+      const uint32_t c = rounded_bits(v[k]) & 0xFu;
+      v[k] = Codes<I4P>::dec(c);
+      w |= c << (4 * k);
     }
     if (G == 4) __builtin_nontemporal_store(uint16_t(w), reinterpret_cast<uint16_t*>(base + (e >> 1)));
     else __builtin_nontemporal_store(w, reinterpret_cast<uint32_t*>(base + (e >> 1)));
@@ -267,10 +282,11 @@ template <int G> struct CodeGroup<F4P, G> {
   }
 };
 
-// round (where the target asks for it) and clamp an exact quotient
+// clamp an exact quotient, rounding it first where a float target asks for that (integer targets round in enc; a clamp to
+// whole numbers before or after the rounding gives the same)
 template <typename Q>
 __device__ __forceinline__ float finish_quotient(float v, int flags) {
-  if (Codes<Q>::kAlwaysRound || (flags & kFlagRoundToInt))
+  if (!Codes<Q>::kInteger && (flags & kFlagRoundToInt))
     v = __builtin_rintf(v);                          // v_rndne_f32: exact round-half-even
   return fmaxf(fminf(v, Codes<Q>::kHi), Codes<Q>::kLo);
 }
@@ -317,15 +333,23 @@ struct ExactDivisor {
   // callers that have checked `fast` for the whole wave.  Same values as finish_quotient(divide(x)); the sign of
   // zero is put back after the clamp (a clamp keeps it), so that the clamp's operands are results of arithmetic
   // and need no quieting first.
+  // Integer targets: x is clamped to [kLo s, kHi s] instead (either order: s may be negative), which bounds the quotient
+  // to the codes' range, give or take an ulp at its ends, where it rounds to the end's code; a zero needs no sign.  All
+  // on -x and -q, because the clamp is one v_med3, which gives the least operand for a NaN: that of -x is the greatest
+  // of x, as above.  With the rounding in enc this is 8 instructions an element to a code and one to gather it, where
+  // minimum, maximum, rounding, clamp, sign, conversion, mask and shift made it 18: a tensor of 45 M bf16 took 18 us of
+  // the vector units.
   template <typename Q, bool ROUND>
   __device__ __forceinline__ float quantize_fast1(float x) const {
-    const float xc = fmaxf(fminf(x, bound), -bound);
-    const float q0 = xc * r;
-    float q = __builtin_fmaf(__builtin_fmaf(-q0, s, xc), r, q0);
-    q = __builtin_fmaf(__builtin_fmaf(-q, s, xc), r, q);
-    if (ROUND) q = __builtin_rintf(q);
-    q = fmaxf(fminf(q, Codes<Q>::kHi), Codes<Q>::kLo);
-    return __builtin_copysignf(q, q0);
+    const float nx = Codes<Q>::kInteger ? __builtin_amdgcn_fmed3f(-x, -Codes<Q>::kLo * s, -Codes<Q>::kHi * s)
+                                        : __builtin_amdgcn_fmed3f(-x, bound, -bound);
+    const float n0 = nx * r;
+    float n = __builtin_fmaf(__builtin_fmaf(-n0, s, nx), r, n0);
+    n = __builtin_fmaf(__builtin_fmaf(-n, s, nx), r, n);
+    if (Codes<Q>::kInteger) return -n;
+    if (ROUND) n = __builtin_rintf(n);
+    n = __builtin_amdgcn_fmed3f(n, -Codes<Q>::kHi, -Codes<Q>::kLo);
+    return -__builtin_copysignf(n, n0);
   }
   template <typename Q, bool ROUND, int G>
   __device__ __forceinline__ void quantize_fast(float (&v)[G]) const {
@@ -339,7 +363,7 @@ struct ExactDivisor {
 // loops over the group, not selects per element.
 template <typename Q, int G>
 __device__ __forceinline__ void quantize_group(const ExactDivisor& dv, float (&v)[G], int flags) {
-  const bool round = Codes<Q>::kAlwaysRound || (flags & kFlagRoundToInt);
+  const bool round = !Codes<Q>::kInteger && (flags & kFlagRoundToInt);
   if (__builtin_amdgcn_ballot_w64(!dv.fast) == 0) {
     if (round) dv.template quantize_fast<Q, true>(v);
     else dv.template quantize_fast<Q, false>(v);
@@ -358,33 +382,49 @@ enum ScaleKind { kUniform = 0, kRow = 1, kCol = 2 };
 // and chunk; every row of the chunk is one contiguous KiB of the float operand per wave, as before.
 // Host guarantees as for qdq_groups<kCol>: d1 % G == 0, n / G < 2^32, operands aligned for group accesses,
 // the scales 16-byte aligned.
-constexpr int kColChunkRows = 32;
+constexpr int kColChunkRows = 16;
 
+// Bound by memory once enough of it is in flight: 8 rows of a strip at a time, asked for before the scales, whose
+// reciprocals are formed while the rows are on their way, and chunks of 16 rows.  With 4 rows at a time and chunks of 32
+// a quantize of bf16 [4096, 11008] had 11 waves and 44 KiB per compute unit outstanding (a dequantize, 22 KiB). With the
+// shorter arithmetic of ExactDivisor bf16 [4096, 11008] to int4 in blocks of 128 rows and back went from 67.7 to 55.6 us
+// (270 MB: 4.0 to 4.9 TB/s).
 template <typename X, typename Q, int MODE>
 __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                                typename X::storage* __restrict__ y, const float* __restrict__ scale,
                                                int64_t n, int64_t d1, int64_t nb, int flags) {
   using FG = FloatGroup<X>;
   constexpr int G = FG::G;
-  constexpr int U = 4;                               // rows in flight per lane
+  constexpr int U = MODE == 2 ? 4 : 8;               // rows in flight per lane
   using CG = CodeGroup<Q, G>;
   const uint32_t groups_per_row = uint32_t(d1 / G), strips = (groups_per_row + kWave - 1) / kWave;
   const int64_t d0 = n / d1, nblocks = d0 / nb;
-  const uint32_t chunks = uint32_t((nb + kColChunkRows - 1) / kColChunkRows);
+  const int64_t chunks = (nb + kColChunkRows - 1) / kColChunkRows;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   const int64_t nwaves = int64_t(gridDim.x) * blockDim.x / kWave;
   const int64_t items = nblocks * chunks * strips;
-  const bool round = Codes<Q>::kAlwaysRound || (flags & kFlagRoundToInt);
+  const bool round = !Codes<Q>::kInteger && (flags & kFlagRoundToInt);
 
   for (int64_t item = wave; item < items; item += nwaves) {
-    const uint32_t strip = uint32_t(item % strips);
     const int64_t rest = item / strips;
-    const uint32_t chunk = uint32_t(rest % chunks);
-    const int64_t b = rest / chunks;
+    const uint32_t strip = uint32_t(item - rest * strips);
+    const int64_t b = rest / chunks, chunk = rest - b * chunks;
     const uint32_t cg = strip * kWave + lane;
     const bool live = cg < groups_per_row;
     const int64_t c0 = int64_t(live ? cg : groups_per_row - 1) * G;     // idle lanes repeat the last group, store nothing
+    const int64_t r0 = b * nb + chunk * kColChunkRows;
+    const int64_t r1 = r0 + kColChunkRows < (b + 1) * nb ? r0 + kColChunkRows : (b + 1) * nb;
+    u32x4 xin[U];
+    uint32_t qin[U][2];
+    const auto fetch = [&](int64_t r) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t e = (r + u < r1 ? r + u : r1 - 1) * d1 + c0;
+        if (MODE == 1) CG::load_raw(q, e, qin[u]);
+        else xin[u] = FG::load(x + e);
+      }
+    };
     float sc[G];
     const f32x4* sp = reinterpret_cast<const f32x4*>(scale + b * d1 + c0);
 #pragma unroll
@@ -392,8 +432,7 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
       const f32x4 t = sp[k];
       sc[4 * k] = t.x; sc[4 * k + 1] = t.y; sc[4 * k + 2] = t.z; sc[4 * k + 3] = t.w;
     }
-    const int64_t r0 = b * nb + int64_t(chunk) * kColChunkRows;
-    const int64_t r1 = r0 + kColChunkRows < (b + 1) * nb ? r0 + kColChunkRows : (b + 1) * nb;
+    fetch(r0);
     ExactDivisor dv[G];
     bool fast = true;
 #pragma unroll
@@ -404,14 +443,7 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
     const bool all_fast = MODE == 1 || __builtin_amdgcn_ballot_w64(!fast) == 0;
 
     for (int64_t r = r0; r < r1; r += U) {
-      u32x4 xin[U];
-      uint32_t qin[U][2];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t e = (r + u < r1 ? r + u : r1 - 1) * d1 + c0;
-        if (MODE == 1) CG::load_raw(q, e, qin[u]);
-        else xin[u] = FG::load(x + e);
-      }
+      if (r != r0) fetch(r);
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t e = (r + u) * d1 + c0;
@@ -464,8 +496,18 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
   const int64_t nwaves = int64_t(gridDim.x) * blockDim.x / kWave;
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
+  const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;
 
   for (int64_t base = wave * (kWave * J); base < ngroups; base += nwaves * (kWave * J)) {
+    // Row scales: the row of the trip's first group by two divisions for the whole wave, the others from there - a lane's
+    // own division and remainder, some 50 instructions, came with every 16 bytes of the tensor.
+    uint32_t row0 = 0, col0 = 0, srow0 = 0;
+    if (KIND == kRow) {
+      const uint32_t first = __builtin_amdgcn_readfirstlane(uint32_t(base));
+      row0 = first / groups_per_row;
+      col0 = first - row0 * groups_per_row;
+      srow0 = row0 % wrap;
+    }
     float v[J][G];
     float s[J][SN];
     bool live[J];
@@ -483,10 +525,16 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
         s[j][0] = s_uniform;
       } else {
         // group, row and scale indices are below 2^32 for anything that fits in HBM
-        const uint32_t row = uint32_t(g) / groups_per_row;
         if (KIND == kRow) {
-          s[j][0] = scale[row % uint32_t(nb)];
+          uint32_t col = col0 + uint32_t(j * kWave + lane), srow = srow0;
+          if (groups_per_row >= uint32_t(kWave * J)) {   // the trip holds the end of one row at most
+            if (col >= groups_per_row) srow = srow + 1 == wrap ? 0u : srow + 1;
+          } else {
+            srow = (srow + col / groups_per_row) % wrap;
+          }
+          s[j][0] = scale[srow];
         } else {
+          const uint32_t row = uint32_t(g) / groups_per_row;
           const int64_t c0 = int64_t(uint32_t(g) - row * groups_per_row) * G;
           const f32x4* sp = reinterpret_cast<const f32x4*>(scale + int64_t(row / uint32_t(nb)) * d1 + c0);
 #pragma unroll
