@@ -425,6 +425,123 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_nk_rows128(
   }
 MTRT_W8_FRAG_ROWS_KERNEL(mtrt_gemm_w8a8_frag_rows32, 1)
 MTRT_W8_FRAG_ROWS_KERNEL(mtrt_gemm_w8a8_frag_rows64, 2)
+
+// ---- a decode step's Linear in ONE launch: f16 activations, quantized where they are used ------------------
+// With one scale for all activations nothing has to be known before a row can be quantized, and at a decode step the pass
+// in front of the GEMM is all launch: M = 1, K = N = 4096 was 2.9 us of quantization and 6.3 us of GEMM.  Here every
+// workgroup quantizes the whole of x (at most 16 Ki elements, from L2) into LDS while its first weights are on their
+// way.  It owns 16 columns, half a tile of the fragment order (v_mfma_i32_16x16x64_i8 takes a k-step pair's halves in four
+// groups of lanes), so that 4096 columns fill the chip's 256 compute units; its 8 waves share K in slices of 128, four
+// slices in flight each (8 KiB a wave).  The sums are exact integers: the result is that of the two launches, bit for bit.
+// Bound by the weights' way from memory and, towards 16 Ki elements, by the quantization.  Kernel times in us against the
+// two launches (whose gap comes on top), (M, K, N): (1, 4096, 4096) 4.9 against 2.9 + 6.6, (1, 14336, 4096) 12.5 against
+// 3.7 + 12.0, (4, 4096, 4096) 5.9 against 3.4 + 6.6, (16, 1024, 16384) 10.8 against 3.9 + 8.9.  The LDS and the registers
+// for x end it at 16 Ki elements, where it is still the shorter by a sixth and more.
+namespace decode {
+
+constexpr int kWaves = 8, kMaxRows = 16, kMaxElements = 16384, kAhead = 4;
+constexpr int kXGroups = kMaxElements / 8 / (64 * kWaves);        // groups of 8 elements of x per lane at most
+constexpr int kRowPad = 16;                                       // LDS bytes between the rows of codes: their banks differ
+
+__device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag,
+                                    const RowsScaleEpilogue& epi, uint16_t* __restrict__ y, int M, int K, int Kp, int64_t N, int8_t* codes,
+                                    int (*partial)[64][4]) {
+  using qdq_cluster::ExactDivisor;
+  using qdq_cluster::FloatGroup;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, kgroup = lane >> 4;
+  const int slices = Kp / 128, kb0 = slices * wave / kWaves, kb1 = slices * (wave + 1) / kWaves;
+  const int64_t n0 = int64_t(blockIdx.x) * 16;
+
+  // x first: what is asked for first arrives first
+  const int row_groups = Kp / 8, groups = M * row_groups;
+  u32x4 xin[kXGroups];
+  int xrow[kXGroups], xk[kXGroups];
+#pragma unroll
+  for (int i = 0; i < kXGroups; ++i) {
+    const int g = int(threadIdx.x) + i * 64 * kWaves;
+    xrow[i] = g / row_groups;
+    xk[i] = (g - xrow[i] * row_groups) * 8;
+    xin[i] = (u32x4){0u, 0u, 0u, 0u};
+    if (g < groups && xk[i] + 8 <= K) xin[i] = *reinterpret_cast<const qdq_cluster::u32x4_unaligned*>(x + int64_t(xrow[i]) * K + xk[i]);
+  }
+  const ExactDivisor dv(x_scale[0]);
+
+  // lane (col, kgroup) of k-step pair p: bytes 64 p + 16 kgroup ... + 15 of its column
+  const int8_t* wp = w_frag + (n0 / 32) * slices * 4096 + (kgroup >> 1) * 1024 + ((kgroup & 1) * 32 + int(n0 & 16) + col) * 16;
+  const int last = kb1 > kb0 ? kb1 - 1 : 0;                        // a slice past the wave's last one is that one again
+  v4i w[kAhead][2];
+  const auto fetch = [&](int kb, v4i (&into)[2]) {
+    const int8_t* from = wp + int64_t(kb < kb1 ? kb : last) * 4096;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) into[p] = __builtin_nontemporal_load(reinterpret_cast<const v4i*>(from + p * 2048));
+  };
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s) fetch(kb0 + s, w[s]);
+
+  const int pitch = Kp + kRowPad;
+#pragma unroll
+  for (int i = 0; i < kXGroups; ++i) {
+    if (int(threadIdx.x) + i * 64 * kWaves >= groups) continue;
+    const int left = K - xk[i];                                    // the group that holds a row's end, and the padding behind it
+    if (left > 0 && left < 8) {
+      for (int e = 0; e < left; ++e) {
+        const uint32_t bits = uint32_t(x[int64_t(xrow[i]) * K + xk[i] + e]) << (16 * (e & 1));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xin[i][k] |= (e >> 1) == k ? bits : 0u;
+      }
+    }
+    float v[8];
+    FloatGroup<F16>::unpack(xin[i], v);
+    qdq_cluster::quantize_group<I8>(dv, v, 0);
+    const u32x2 c = {qdq_cluster::pack4<I8>(&v[0], 0), qdq_cluster::pack4<I8>(&v[4], 0)};
+    *reinterpret_cast<u32x2*>(codes + xrow[i] * pitch + xk[i]) = c;
+  }
+  __syncthreads();
+
+  v4i acc = {0, 0, 0, 0};
+  const int8_t* arow = codes + (col < M ? col : M - 1) * pitch + kgroup * 16;   // as the first operand the lane's row; rows past M repeat the last
+  for (int kb = kb0; kb < kb1; kb += kAhead) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      v4i held[2] = {w[s][0], w[s][1]};
+      if (kb + kAhead < kb1) fetch(kb + kAhead + s, w[s]);
+      if (kb + s < kb1) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const v4i a = *reinterpret_cast<const v4i*>(arow + (kb + s) * 128 + p * 64);
+          acc = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, held[p], acc, 0, 0, 0);
+        }
+      }
+    }
+  }
+  // lane (col, h = lane / 16) holds rows 4 h + r of its column in register r
+#pragma unroll
+  for (int r = 0; r < 4; ++r) partial[wave][lane][r] = acc[r];
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    const int l = threadIdx.x & 63, r = threadIdx.x >> 6;
+    int v = partial[0][l][r];
+#pragma unroll
+    for (int k = 1; k < kWaves; ++k) v = v + partial[k][l][r];
+    const int row = (l >> 4) * 4 + r;
+    const int64_t c = n0 + (l & 15);
+    if (row < M && c < N) y[int64_t(row) * N + c] = uint16_t(epi.finish(v, row, c));
+  }
+}
+
+}  // namespace decode
+
+// (x [M,K] f16, x_scale: one f32, w_frag (K padded to Kp), w_scale, y [M,N] f16, M <= 16, K, Kp, N, bias f16 or null) ;
+// Kp = K rounded up to 128, M * Kp <= 16384, w_frag 16-byte aligned, x aligned to its elements; grid = ceil(N / 16), block = 512.
+extern "C" __global__ void __launch_bounds__(512) mtrt_linear_w8a8_decode(
+    const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag, const float* __restrict__ w_scale,
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t Kp, int64_t N, const uint16_t* __restrict__ bias) {
+  __shared__ __attribute__((aligned(16))) int8_t codes[decode::kMaxElements + decode::kMaxRows * decode::kRowPad];
+  __shared__ __attribute__((aligned(16))) int partial[decode::kWaves][64][4];
+  decode::run(x, x_scale, w_frag, RowsScaleEpilogue{x_scale, w_scale, 0, bias}, y, int(M), int(K), int(Kp), N, codes, partial);
+}
+
 // Any K and any operand alignment on the matrix cores, for the shapes the kernels above do not take (K not a
 // multiple of 128, operands off 16-byte alignment, operands of 4 GiB and more): the 128 x 128 tile loop of
 // gemm_core::edge.  (a [M,K] i8, w_nk [N,K] i8, a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, a_step, bias)

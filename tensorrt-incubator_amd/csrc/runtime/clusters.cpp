@@ -1438,8 +1438,10 @@ int64_t round_up(int64_t v, int64_t step) { return (v + step - 1) / step * step;
 
 // How a plan's call runs: the row length its GEMM sees, whether x goes through the activation pass, and the two parts of the
 // workspace (the pass's result, then the partial tiles).
+// A decode step's W8A8 Linear quantizes its activations inside the GEMM (mtrt_linear_w8a8_decode) up to this many of them.
+constexpr int64_t kDecodeElements = 16384;
 struct LinearShape {
-  bool fragments = false, pass = false;
+  bool fragments = false, pass = false, one_launch = false;
   int64_t Kp = 0, act_bytes = 0, partial_bytes = 0;
 };
 LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units) {
@@ -1448,10 +1450,11 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
   const int eb = float_bytes(p.dtype);
   s.Kp = p.K;
   if (p.route == MTRT_LINEAR_W8A8) {
-    s.pass = true;
     s.fragments = p.w_frag != nullptr;
     s.Kp = s.fragments ? round_up(p.K, 128) : p.K;
-    s.act_bytes = round_up(M * s.Kp, 256);
+    s.one_launch = s.fragments && M <= 16 && M * s.Kp <= kDecodeElements;
+    s.pass = !s.one_launch;
+    s.act_bytes = s.pass ? round_up(M * s.Kp, 256) : 0;
     if (s.fragments && M > 32) {
       const W8Plan w = w8_plan(M, s.Kp, p.N, units, true);
       s.partial_bytes = w.kind == W8Plan::kTile && w.tile.tile ? w.tile.workspace() : 0;
@@ -1594,11 +1597,18 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   if (p.route == MTRT_LINEAR_W4A16)
     return w4a16(as_hip(stream), x, nullptr, p.w_frag, p.w_scale, p.bias, y, M, p.K, p.N, p.K, workspace, workspace_bytes);
   const LinearShape s = linear_shape(p, M, num_compute_units(st));
-  if (s.fragments && !s.pass && !aligned(x, 16))
+  if (s.fragments && !s.pass && !s.one_launch && !aligned(x, 16))
     return set_error(MTRT_INVALID_ARGUMENT, "x must be 16-byte aligned for these weights");
   const int64_t need = s.act_bytes + s.partial_bytes;
   if (need > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < need))
     return set_error(MTRT_INVALID_ARGUMENT, "workspace of %lld bytes, 16-byte aligned, needed", (long long)need);
+  if (s.one_launch) {
+    const float *w_scale = static_cast<const float *>(p.w_scale), *x_scale = p.x_scale;
+    const void *w_frag = p.w_frag, *bias = p.bias;
+    int64_t K = p.K, Kp = s.Kp, N = p.N;
+    void *args[] = {&x, &x_scale, &w_frag, &w_scale, &y, &M, &K, &Kp, &N, &bias};
+    return launch(st, KernelName("mtrt_linear_w8a8_decode"), uint32_t((N + 15) / 16), 512, as_hip(stream), args);
+  }
   char *ws = static_cast<char *>(workspace);
   const void *act = x;
   if (s.pass) {
