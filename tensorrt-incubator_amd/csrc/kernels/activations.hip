@@ -24,9 +24,9 @@ __device__ __forceinline__ void act_rows(const typename X::storage* __restrict__
   const uint32_t groups = uint32_t(Kp / G);            // Kp is a whole number of groups
   const uint32_t chunks = (groups + kWave * kActGroups - 1) / (kWave * kActGroups);
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t items = M * chunks, nwaves = int64_t(gridDim.x) * blockDim.x / kWave;
+  const int64_t items = M * chunks, nwaves = waves_in_launch();
   const ExactDivisor dv(MODE == 0 ? 1.0f : scale[0]);
-  for (int64_t item = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave; item < items; item += nwaves) {
+  for (int64_t item = wave_in_launch(); item < items; item += nwaves) {
     const int64_t row = item / chunks;
     const uint32_t g0 = uint32_t(item - row * chunks) * (kWave * kActGroups) + lane;
     u32x4 in[kActGroups];
@@ -74,11 +74,8 @@ __device__ __forceinline__ void act_rows(const typename X::storage* __restrict__
 #pragma unroll
             for (int k = 0; k < 4; ++k) t[k] = f32_to_bits(v[k]);
           } else {
-            typename X::storage h[8];
 #pragma unroll
-            for (int k = 0; k < 8; ++k) Tile<X>::store1(&h[k], v[k % G]);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) t[k] = uint32_t(uint16_t(h[2 * k])) | (uint32_t(uint16_t(h[2 * k + 1])) << 16);
+            for (int k = 0; k < 4; ++k) t[k] = narrow2<X>(v[(2 * k) % G], v[(2 * k + 1) % G]);
           }
           *reinterpret_cast<u32x4*>(dst) = t;
         }

@@ -60,7 +60,7 @@ __device__ __forceinline__ void rows_body(const typename X::storage* __restrict_
                                           float qmax, float* __restrict__ amax_out, float* __restrict__ scale_out) {
   using A = AbsBits<X>;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t s = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
+  const int64_t s = (int64_t(blockIdx.x) * block_threads() + threadIdx.x) / kWave;
   if (s >= nb) return;                               // whole waves leave together
   uint32_t m = 0;
   for (int64_t row = s; row < d0; row += nb) {
@@ -258,7 +258,7 @@ __device__ __forceinline__ void rows_split_body(const typename X::storage* __res
 // stage word (maximum bit pattern) -> amax and scale; `stage` may be amax_out or scale_out itself
 template <typename X>
 __device__ __forceinline__ void finish_body(const uint32_t* stage, int64_t count, float qmax, float* amax_out, float* scale_out) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const int64_t i = int64_t(blockIdx.x) * block_threads() + threadIdx.x;
   if (i >= count) return;
   emit(AbsBits<X>::finish(stage[i]), qmax, amax_out, scale_out, i);
 }
@@ -269,7 +269,7 @@ __device__ __forceinline__ void cols_any_body(const typename X::storage* __restr
                                               float qmax, float* __restrict__ amax_out, float* __restrict__ scale_out) {
   using A = AbsBits<X>;
   const int64_t total = (d0 / nb) * d1;
-  for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < total; e += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t e = int64_t(blockIdx.x) * block_threads() + threadIdx.x; e < total; e += int64_t(gridDim.x) * block_threads()) {
     const int64_t b = e / d1, c = e - b * d1;
     uint32_t m = 0;
     for (int64_t r = 0; r < nb; ++r) { const uint32_t a = A::one(x + (b * nb + r) * d1 + c); m = m > a ? m : a; }

@@ -65,9 +65,25 @@ __device__ __forceinline__ uint32_t f32x2_to_f16x2_bits(float lo, float hi) {
   c.h = __builtin_convertvector((f32x2_t){lo, hi}, f16x2_t);
   return c.u;
 }
+// v_cvt_pk_bf16_f32 on both halves; as two single conversions the compiler issues it twice and merges the words.
 __device__ __forceinline__ uint32_t f32x2_to_bf16x2_bits(float lo, float hi) {
-  return f32_to_bf16_bits(lo) | (f32_to_bf16_bits(hi) << 16);
+  typedef float f32x2_t __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+  union { bf16x2_t h; uint32_t u; } c;
+  c.h = __builtin_convertvector((f32x2_t){lo, hi}, bf16x2_t);
+  return c.u;
 }
+// blockDim.x, by a scalar load: hidden_group_size_x of the code object's implicit kernel arguments.  The builtin also allows
+// for a last workgroup of another size, which HIP does not launch, through a vector load with its own wait, about 0.7 us
+// in front of a kernel's first access.
+__device__ __forceinline__ uint32_t block_threads() {
+  return ((const uint32_t*)__builtin_amdgcn_implicitarg_ptr())[3] & 0xFFFFu;
+}
+// This wave's number in the launch, in scalar registers: rows, chunks and addresses derived from it are scalar too.
+__device__ __forceinline__ uint32_t wave_in_launch() {
+  return blockIdx.x * (block_threads() / kWave) + __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+}
+__device__ __forceinline__ uint32_t waves_in_launch() { return gridDim.x * (block_threads() / kWave); }
 
 // f8E4M3FN (OCP) pair conversion in hardware: RNE.  Inputs are pre-clamped to
 // [-448, 448] by every caller, so the saturation rule of the instruction is

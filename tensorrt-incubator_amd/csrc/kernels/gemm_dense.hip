@@ -144,7 +144,7 @@ struct BiasEpilogue {
   f32x4 br[2][4];
   __device__ __forceinline__ void setup(int8_t* scratch, int64_t, int64_t, int64_t n0, int64_t N) {
     float* dst = reinterpret_cast<float*>(scratch);
-    for (int c = threadIdx.x; c < BN; c += blockDim.x) dst[c] = (bias && n0 + c < N) ? Tile<X>::load1(bias + n0 + c) : 0.0f;
+    for (int c = threadIdx.x; c < BN; c += block_threads()) dst[c] = (bias && n0 + c < N) ? Tile<X>::load1(bias + n0 + c) : 0.0f;
     sb = dst;
   }
   __device__ __forceinline__ void row(int) {}
@@ -376,7 +376,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w16_prepack_frag(const ui
                                                                       int64_t K, int64_t N) {
   const int64_t slices = (K + 63) / 64, ntiles = (N + 31) / 32;
   const int64_t total = ntiles * slices * 256;
-  for (int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; id < total; id += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t id = int64_t(blockIdx.x) * block_threads() + threadIdx.x; id < total; id += int64_t(gridDim.x) * block_threads()) {
     const int lane = int(id & 63), p = int((id >> 6) & 3);
     const int64_t slice = (id >> 8) % slices, tile = (id >> 8) / slices;
     const int64_t n = tile * 32 + (lane & 31), k0 = slice * 64 + 16 * p + 8 * (lane >> 5);

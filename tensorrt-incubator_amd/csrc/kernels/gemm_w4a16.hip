@@ -132,7 +132,7 @@ struct BiasEpilogue {
   u32x2 br[2][4] = {};
   __device__ __forceinline__ void setup(int8_t* scratch, int64_t, int64_t, int64_t n0, int64_t N) {
     uint16_t* dst = reinterpret_cast<uint16_t*>(scratch);
-    for (int c = threadIdx.x; c < BN; c += blockDim.x) dst[c] = n0 + c < N ? bias[n0 + c] : uint16_t(0);
+    for (int c = threadIdx.x; c < BN; c += block_threads()) dst[c] = n0 + c < N ? bias[n0 + c] : uint16_t(0);
     sb = dst;
   }
   __device__ __forceinline__ void row(int) {}
@@ -1134,7 +1134,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w4_prepack_strips(const u
   const int64_t kblocks = K / 128;
   const int64_t ntiles = (N + 15) / 16;
   const int64_t total = ntiles * kblocks * 256;
-  for (int64_t d = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; d < total; d += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t d = int64_t(blockIdx.x) * block_threads() + threadIdx.x; d < total; d += int64_t(gridDim.x) * block_threads()) {
     const int j = int(d & 3), lane = int((d >> 2) & 63);
     const int64_t kb = (d >> 8) % kblocks, tile = (d >> 8) / kblocks;
     const int64_t n = tile * 16 + (lane & 15);
@@ -1308,7 +1308,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_any(
     const uint16_t* __restrict__ a, const uint8_t* __restrict__ w_kn_packed, const uint16_t* __restrict__ scale,
     uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block) {
   const int64_t total = M * N;
-  for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < total; e += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t e = int64_t(blockIdx.x) * block_threads() + threadIdx.x; e < total; e += int64_t(gridDim.x) * block_threads()) {
     const int64_t m = e / N, n = e - m * N;
     float acc = 0.0f;
     for (int64_t k = 0; k < K; ++k) {
@@ -1330,7 +1330,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w4_prepack(const uint8_t*
   const int64_t kblocks = K / BKH;
   const int64_t ntiles = (N + 31) / 32;
   const int64_t total = ntiles * kblocks * 256;
-  for (int64_t d = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; d < total; d += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t d = int64_t(blockIdx.x) * block_threads() + threadIdx.x; d < total; d += int64_t(gridDim.x) * block_threads()) {
     const int j = int(d & 3), lane = int((d >> 2) & 63);
     const int64_t kb = (d >> 8) % kblocks, tile = (d >> 8) / kblocks;
     const int h = lane >> 5;

@@ -58,9 +58,9 @@ struct ScaleEpilogueT {
     float* dst = reinterpret_cast<float*>(scratch);
     const int64_t row = m0 + threadIdx.x;              // the first 256 threads: 256 rows
     if (threadIdx.x < 256) dst[threadIdx.x] = row < M ? a_scale[row * a_step] : 0.0f;
-    for (int c = threadIdx.x; c < BN; c += blockDim.x) dst[256 + c] = n0 + c < N ? w_scale[n0 + c] : 0.0f;
+    for (int c = threadIdx.x; c < BN; c += block_threads()) dst[256 + c] = n0 + c < N ? w_scale[n0 + c] : 0.0f;
     if (BIAS && bias)
-      for (int c = threadIdx.x; c < BN; c += blockDim.x) dst[256 + BN + c] = n0 + c < N ? f16_bits_to_f32(bias[n0 + c]) : 0.0f;
+      for (int c = threadIdx.x; c < BN; c += block_threads()) dst[256 + BN + c] = n0 + c < N ? f16_bits_to_f32(bias[n0 + c]) : 0.0f;
     sa = dst;
     sw = dst + 256;
   }
@@ -180,7 +180,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w8_prepack_frag(const int
                                                                      int64_t K, int64_t N, int32_t nk) {
   const int64_t slices = (K + 127) / 128, ntiles = (N + 31) / 32;
   const int64_t total = ntiles * slices * 256;
-  for (int64_t id = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; id < total; id += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t id = int64_t(blockIdx.x) * block_threads() + threadIdx.x; id < total; id += int64_t(gridDim.x) * block_threads()) {
     const int lane = int(id & 63), p = int((id >> 6) & 3);
     const int64_t slice = (id >> 8) % slices, tile = (id >> 8) / slices;
     const int64_t n = tile * 32 + (lane & 31), k0 = slice * 128 + 32 * p + 16 * (lane >> 5);
@@ -377,7 +377,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_nk_any(
     const int8_t* __restrict__ a, const int8_t* __restrict__ w, const float* __restrict__ a_scale,
     const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {
   const int64_t total = M * N;
-  for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < total; e += int64_t(gridDim.x) * blockDim.x) {
+  for (int64_t e = int64_t(blockIdx.x) * block_threads() + threadIdx.x; e < total; e += int64_t(gridDim.x) * block_threads()) {
     const int64_t m = e / N, n = e - m * N;
     int acc = 0;
     for (int64_t k = 0; k < K; ++k) acc += int(a[m * K + k]) * int(w[n * K + k]);

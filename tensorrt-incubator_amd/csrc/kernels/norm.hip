@@ -54,7 +54,7 @@ template <> struct Vec<BF16> {
   static __device__ __forceinline__ u32x4 pack(const float* v) {
     u32x4 t;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) t[j] = f32_to_bf16_bits(v[2 * j]) | (f32_to_bf16_bits(v[2 * j + 1]) << 16);
+    for (int j = 0; j < 4; ++j) t[j] = f32x2_to_bf16x2_bits(v[2 * j], v[2 * j + 1]);
     return t;
   }
 };
@@ -67,7 +67,7 @@ template <> struct Vec<F16> {
   static __device__ __forceinline__ u32x4 pack(const float* v) {
     u32x4 t;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) t[j] = f32_to_f16_bits(v[2 * j]) | (f32_to_f16_bits(v[2 * j + 1]) << 16);
+    for (int j = 0; j < 4; ++j) t[j] = f32x2_to_f16x2_bits(v[2 * j], v[2 * j + 1]);
     return t;
   }
 };

@@ -101,7 +101,7 @@ __device__ __forceinline__ float divide_by_six(float x) {
 // S_enc / f32(s8) for every scale byte, one IEEE divide per lane of the workgroup (256 lanes): a block's second
 // divide becomes a look-up.  Every lane of the workgroup must get here (there is a barrier inside).
 __device__ __forceinline__ void fill_inverse_scales(float* table, float s_enc) {
-  for (uint32_t b = threadIdx.x; b < 256u; b += blockDim.x) table[b] = s_enc / f8_to_f32<0>(b);
+  for (uint32_t b = threadIdx.x; b < 256u; b += block_threads()) table[b] = s_enc / f8_to_f32<0>(b);
   __syncthreads();
 }
 

@@ -59,7 +59,7 @@ template <> struct FloatGroup<BF16> {
   static __device__ __forceinline__ void store(uint16_t* p, const float (&v)[8]) {
     u32x4 t;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) t[k] = f32_to_bf16_bits(v[2 * k]) | (f32_to_bf16_bits(v[2 * k + 1]) << 16);
+    for (int k = 0; k < 4; ++k) t[k] = f32x2_to_bf16x2_bits(v[2 * k], v[2 * k + 1]);
     __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
   }
 };
@@ -73,10 +73,14 @@ template <> struct FloatGroup<F16> {
   static __device__ __forceinline__ void store(uint16_t* p, const float (&v)[8]) {
     u32x4 t;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) t[k] = f32_to_f16_bits(v[2 * k]) | (f32_to_f16_bits(v[2 * k + 1]) << 16);
+    for (int k = 0; k < 4; ++k) t[k] = f32x2_to_f16x2_bits(v[2 * k], v[2 * k + 1]);
     __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
   }
 };
+
+// two values to one word of a 16-bit operand
+template <typename X> __device__ __forceinline__ uint32_t narrow2(float lo, float hi) { return f32x2_to_f16x2_bits(lo, hi); }
+template <> __device__ __forceinline__ uint32_t narrow2<BF16>(float lo, float hi) { return f32x2_to_bf16x2_bits(lo, hi); }
 
 // ---- quantized codes ---------------------------------------------------------------
 // enc(v): code of an already divided, clamped and (for the float targets, where asked for) rounded value; the integer
@@ -131,7 +135,7 @@ typedef _Float16 qdq_h2 __attribute__((ext_vector_type(2)));
 typedef float qdq_f2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t f32x2_to_f4x2(float a, float b) {
   union { uint32_t u; qdq_h2 h; } c;
-  c.u = f32_to_f16_bits(a) | (f32_to_f16_bits(b) << 16);
+  c.u = f32x2_to_f16x2_bits(a, b);
   return __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(0u, c.h, 1.0f, 0) & 0xFFu;
 }
 template <> struct Codes<F4P> {
@@ -202,28 +206,38 @@ __device__ __forceinline__ void unpack4<F8>(uint32_t w, float* v) {
   v[0] = f8_to_f32<0>(w); v[1] = f8_to_f32<1>(w); v[2] = f8_to_f32<2>(w); v[3] = f8_to_f32<3>(w);
 }
 
+// Codes are written and read with ordinary accesses, unlike the float operands: a wave's instruction writes half the
+// bytes of one of the float operand's, and written past the caches these pieces cost more than their share.  bf16 -> f8 -> bf16
+// of 128 Mi elements in one pass 109.5 -> 96.6 us, f32 -> i8 -> f32 of 43 Mi 69.7 -> 65.0; int8 codes of 43 Mi
+// bf16, then dequantized, 49.5 -> 46.5.  KEEP = false, where nothing but codes is written with one scale: such a pass alone is
+// 1 to 5 % the slower for it (43 Mi bf16 25.1 against 26.4 us).
+template <bool KEEP, typename T> __device__ __forceinline__ void store_codes(T v, T* p) {
+  if (KEEP) *p = v;
+  else __builtin_nontemporal_store(v, p);
+}
+
 // G codes of one group, at element offset `e` (a multiple of G) of the code array.
 // store() leaves f32(code) in v[]: the value a following dequantize multiplies by
 // the scale (this also turns the -0.0 a rounding can produce into the +0.0 that
 // reading the integer code back gives).
-template <typename Q, int G> struct CodeGroup {
+template <typename Q, int G, bool KEEP = true> struct CodeGroup {
   static constexpr int kWords = G / 4;
   static __device__ __forceinline__ void store(typename Q::storage* base, int64_t e, float (&v)[G], int flags) {
     uint32_t w[kWords];
 #pragma unroll
     for (int i = 0; i < kWords; ++i) { w[i] = pack4<Q>(&v[4 * i], flags); unpack4<Q>(w[i], &v[4 * i]); }
     if (kWords == 1) {
-      __builtin_nontemporal_store(w[0], reinterpret_cast<uint32_t*>(base + e));
+      store_codes<KEEP>(w[0], reinterpret_cast<uint32_t*>(base + e));
     } else {
       u32x2 t = {w[0], w[kWords - 1]};
-      __builtin_nontemporal_store(t, reinterpret_cast<u32x2*>(base + e));
+      store_codes<KEEP>(t, reinterpret_cast<u32x2*>(base + e));
     }
   }
   static __device__ __forceinline__ void load_raw(const typename Q::storage* base, int64_t e, uint32_t (&w)[2]) {
     if (kWords == 1) {
-      w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + e));
+      w[0] = *reinterpret_cast<const uint32_t*>(base + e);
     } else {
-      const u32x2 t = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(base + e));
+      const u32x2 t = *reinterpret_cast<const u32x2*>(base + e);
       w[0] = t.x; w[1] = t.y;
     }
   }
@@ -232,7 +246,7 @@ template <typename Q, int G> struct CodeGroup {
     for (int i = 0; i < kWords; ++i) unpack4<Q>(w[i], &v[4 * i]);
   }
 };
-template <int G> struct CodeGroup<I4P, G> {
+template <int G, bool KEEP> struct CodeGroup<I4P, G, KEEP> {
   static __device__ __forceinline__ void store(uint8_t* base, int64_t e, float (&v)[G], int) {
     uint32_t w = 0;
 #pragma unroll
@@ -241,12 +255,12 @@ template <int G> struct CodeGroup<I4P, G> {
       v[k] = Codes<I4P>::dec(c);
       w |= c << (4 * k);
     }
-    if (G == 4) __builtin_nontemporal_store(uint16_t(w), reinterpret_cast<uint16_t*>(base + (e >> 1)));
-    else __builtin_nontemporal_store(w, reinterpret_cast<uint32_t*>(base + (e >> 1)));
+    if (G == 4) store_codes<KEEP>(uint16_t(w), reinterpret_cast<uint16_t*>(base + (e >> 1)));
+    else store_codes<KEEP>(w, reinterpret_cast<uint32_t*>(base + (e >> 1)));
   }
   static __device__ __forceinline__ void load_raw(const uint8_t* base, int64_t e, uint32_t (&w)[2]) {
-    if (G == 4) w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(base + (e >> 1)));
-    else w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + (e >> 1)));
+    if (G == 4) w[0] = *reinterpret_cast<const uint16_t*>(base + (e >> 1));
+    else w[0] = *reinterpret_cast<const uint32_t*>(base + (e >> 1));
   }
   static __device__ __forceinline__ void decode(const uint32_t (&w)[2], float (&v)[G]) {
 #pragma unroll
@@ -254,19 +268,19 @@ template <int G> struct CodeGroup<I4P, G> {
   }
 };
 
-template <int G> struct CodeGroup<F4P, G> {
+template <int G, bool KEEP> struct CodeGroup<F4P, G, KEEP> {
   static __device__ __forceinline__ void store(uint8_t* base, int64_t e, float (&v)[G], int) {
     uint32_t w = 0;
 #pragma unroll
     for (int k = 0; k < G; k += 2) w |= f32x2_to_f4x2(v[k], v[k + 1]) << (4 * k);
     const uint32_t keep[2] = {w, 0};
     decode(keep, v);
-    if (G == 4) __builtin_nontemporal_store(uint16_t(w), reinterpret_cast<uint16_t*>(base + (e >> 1)));
-    else __builtin_nontemporal_store(w, reinterpret_cast<uint32_t*>(base + (e >> 1)));
+    if (G == 4) store_codes<KEEP>(uint16_t(w), reinterpret_cast<uint16_t*>(base + (e >> 1)));
+    else store_codes<KEEP>(w, reinterpret_cast<uint32_t*>(base + (e >> 1)));
   }
   static __device__ __forceinline__ void load_raw(const uint8_t* base, int64_t e, uint32_t (&w)[2]) {
-    if (G == 4) w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint16_t*>(base + (e >> 1)));
-    else w[0] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(base + (e >> 1)));
+    if (G == 4) w[0] = *reinterpret_cast<const uint16_t*>(base + (e >> 1));
+    else w[0] = *reinterpret_cast<const uint32_t*>(base + (e >> 1));
   }
   static __device__ __forceinline__ void decode(const uint32_t (&w)[2], float (&v)[G]) {
     qdq_f2 p = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(w[0], 1.0f, 0);
@@ -382,27 +396,26 @@ enum ScaleKind { kUniform = 0, kRow = 1, kCol = 2 };
 // and chunk; every row of the chunk is one contiguous KiB of the float operand per wave, as before.
 // Host guarantees as for qdq_groups<kCol>: d1 % G == 0, n / G < 2^32, operands aligned for group accesses,
 // the scales 16-byte aligned.
-constexpr int kColChunkRows = 16;
+constexpr int kColChunkRows = 8;
 
-// Bound by memory once enough of it is in flight: 8 rows of a strip at a time, asked for before the scales, whose
-// reciprocals are formed while the rows are on their way, and chunks of 16 rows.  With 4 rows at a time and chunks of 32
-// a quantize of bf16 [4096, 11008] had 11 waves and 44 KiB per compute unit outstanding (a dequantize, 22 KiB). With the
-// shorter arithmetic of ExactDivisor bf16 [4096, 11008] to int4 in blocks of 128 rows and back went from 67.7 to 55.6 us
-// (270 MB: 4.0 to 4.9 TB/s).
+// Bound by memory once enough of it is in flight and little else stands in the way: a chunk is what a lane has in flight,
+// asked for before the reciprocals are formed, and everything about a row but the lane's columns is in scalar registers.
+// bf16 [4096, 11008] to int4 in blocks of 128 rows and back (270 MB), us: 67.7 with 4 rows in flight, chunks of 32 and
+// 18 instructions an element; 55.6 with 8 rows, chunks of 16 and the short arithmetic of ExactDivisor; 51.7 with chunks
+// of 8 rows (chunks of 4: 60.6, of 32: 57.2) and the codes left in the caches (see CodeGroup); through the front end 49.4.
 template <typename X, typename Q, int MODE>
 __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                                typename X::storage* __restrict__ y, const float* __restrict__ scale,
                                                int64_t n, int64_t d1, int64_t nb, int flags) {
   using FG = FloatGroup<X>;
   constexpr int G = FG::G;
-  constexpr int U = MODE == 2 ? 4 : 8;               // rows in flight per lane
+  constexpr int U = kColChunkRows;
   using CG = CodeGroup<Q, G>;
   const uint32_t groups_per_row = uint32_t(d1 / G), strips = (groups_per_row + kWave - 1) / kWave;
   const int64_t d0 = n / d1, nblocks = d0 / nb;
   const int64_t chunks = (nb + kColChunkRows - 1) / kColChunkRows;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-  const int64_t nwaves = int64_t(gridDim.x) * blockDim.x / kWave;
+  const int64_t wave = wave_in_launch(), nwaves = waves_in_launch();
   const int64_t items = nblocks * chunks * strips;
   const bool round = !Codes<Q>::kInteger && (flags & kFlagRoundToInt);
 
@@ -417,14 +430,6 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
     const int64_t r1 = r0 + kColChunkRows < (b + 1) * nb ? r0 + kColChunkRows : (b + 1) * nb;
     u32x4 xin[U];
     uint32_t qin[U][2];
-    const auto fetch = [&](int64_t r) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t e = (r + u < r1 ? r + u : r1 - 1) * d1 + c0;
-        if (MODE == 1) CG::load_raw(q, e, qin[u]);
-        else xin[u] = FG::load(x + e);
-      }
-    };
     float sc[G];
     const f32x4* sp = reinterpret_cast<const f32x4*>(scale + b * d1 + c0);
 #pragma unroll
@@ -432,7 +437,12 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
       const f32x4 t = sp[k];
       sc[4 * k] = t.x; sc[4 * k + 1] = t.y; sc[4 * k + 2] = t.z; sc[4 * k + 3] = t.w;
     }
-    fetch(r0);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int64_t e = (r0 + u < r1 ? r0 + u : r1 - 1) * d1 + c0;
+      if (MODE == 1) CG::load_raw(q, e, qin[u]);
+      else xin[u] = FG::load(x + e);
+    }
     ExactDivisor dv[G];
     bool fast = true;
 #pragma unroll
@@ -442,36 +452,33 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
     }
     const bool all_fast = MODE == 1 || __builtin_amdgcn_ballot_w64(!fast) == 0;
 
-    for (int64_t r = r0; r < r1; r += U) {
-      if (r != r0) fetch(r);
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int64_t e = (r + u) * d1 + c0;
-        const bool store = live && r + u < r1;
-        float v[G];
-        if (MODE == 1) {
-          CG::decode(qin[u], v);
-        } else {
-          FG::unpack(xin[u], v);
-          if (all_fast) {
-            if (round) {
+    for (int u = 0; u < U; ++u) {
+      const int64_t e = (r0 + u) * d1 + c0;
+      const bool store = live && r0 + u < r1;
+      float v[G];
+      if (MODE == 1) {
+        CG::decode(qin[u], v);
+      } else {
+        FG::unpack(xin[u], v);
+        if (all_fast) {
+          if (round) {
 #pragma unroll
-              for (int k = 0; k < G; ++k) v[k] = dv[k].template quantize_fast1<Q, true>(v[k]);
-            } else {
-#pragma unroll
-              for (int k = 0; k < G; ++k) v[k] = dv[k].template quantize_fast1<Q, false>(v[k]);
-            }
+            for (int k = 0; k < G; ++k) v[k] = dv[k].template quantize_fast1<Q, true>(v[k]);
           } else {
 #pragma unroll
-            for (int k = 0; k < G; ++k) v[k] = quant_value<Q>(v[k], sc[k], flags);
+            for (int k = 0; k < G; ++k) v[k] = dv[k].template quantize_fast1<Q, false>(v[k]);
           }
-          if (store) CG::store(q, e, v, flags);       // leaves f32(code) in v
-        }
-        if (MODE != 0 && store) {
+        } else {
 #pragma unroll
-          for (int k = 0; k < G; ++k) v[k] = v[k] * sc[k];
-          FG::store(y + e, v);
+          for (int k = 0; k < G; ++k) v[k] = quant_value<Q>(v[k], sc[k], flags);
         }
+        if (store) CG::store(q, e, v, flags);         // leaves f32(code) in v
+      }
+      if (MODE != 0 && store) {
+#pragma unroll
+        for (int k = 0; k < G; ++k) v[k] = v[k] * sc[k];
+        FG::store(y + e, v);
       }
     }
   }
@@ -489,12 +496,11 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   constexpr int G = FG::G;
   constexpr int J = kTile / G;                       // groups per lane per trip
   constexpr int SN = KIND == kCol ? G : 1;           // scale values a lane needs per group
-  using CG = CodeGroup<Q, G>;
+  using CG = CodeGroup<Q, G, MODE != 0 || KIND != kUniform>;
   const int64_t ngroups = n / G;
   const uint32_t groups_per_row = KIND == kUniform ? 1u : uint32_t(d1 / G);
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-  const int64_t nwaves = int64_t(gridDim.x) * blockDim.x / kWave;
+  const int64_t wave = wave_in_launch(), nwaves = waves_in_launch();
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
   const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;
 
@@ -503,7 +509,7 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
     // own division and remainder, some 50 instructions, came with every 16 bytes of the tensor.
     uint32_t row0 = 0, col0 = 0, srow0 = 0;
     if (KIND == kRow) {
-      const uint32_t first = __builtin_amdgcn_readfirstlane(uint32_t(base));
+      const uint32_t first = uint32_t(base);
       row0 = first / groups_per_row;
       col0 = first - row0 * groups_per_row;
       srow0 = row0 % wrap;
@@ -635,8 +641,7 @@ __device__ __forceinline__ void qdq_rows_ragged(const typename X::storage* __res
   const int tail = int(d1 - nvec * G);
   const int64_t chunks = nvec > 0 ? (nvec + kWave - 1) / kWave : 1;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave;
-  const int64_t nwaves = int64_t(gridDim.x) * blockDim.x / kWave;
+  const int64_t wave = wave_in_launch(), nwaves = waves_in_launch();
   const int64_t items = d0 * chunks;
   for (int64_t item = wave; item < items; item += nwaves) {
     const int64_t row = item / chunks, c = item - row * chunks;
@@ -688,12 +693,8 @@ __device__ __forceinline__ void qdq_rows_ragged(const typename X::storage* __res
           t = (u32x4){f32_to_bits(f[0]), f32_to_bits(f[1]), f32_to_bits(f[2]), f32_to_bits(f[3])};
           *reinterpret_cast<u32x4_unaligned*>(y + fe0) = t;
         } else {
-          // 16-bit outputs: narrowed one by one through the element form, then stored as one vector
-          typename X::storage h[8];
 #pragma unroll
-          for (int k = 0; k < 8; ++k) Tile<X>::store1(&h[k % G], f[k % G]);
-#pragma unroll
-          for (int k = 0; k < 4; ++k) t[k] = uint32_t(uint16_t(h[(2 * k) % G])) | (uint32_t(uint16_t(h[(2 * k + 1) % G])) << 16);
+          for (int k = 0; k < 4; ++k) t[k] = narrow2<X>(f[(2 * k) % G], f[(2 * k + 1) % G]);
           *reinterpret_cast<u32x4_unaligned*>(y + fe0) = t;
         }
       }
@@ -723,8 +724,8 @@ __device__ __forceinline__ void qdq_any(const typename X::storage* __restrict__ 
                                         int64_t n, int64_t d1, int64_t nb, int kind, int flags) {
   constexpr int kPer = (Q::kBits == 4) ? 2 : 1;
   const int64_t units = (n + kPer - 1) / kPer;
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t u = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; u < units; u += stride) {
+  const int64_t stride = int64_t(gridDim.x) * block_threads();
+  for (int64_t u = int64_t(blockIdx.x) * block_threads() + threadIdx.x; u < units; u += stride) {
     uint32_t byte = (Q::kBits == 4 && MODE == 1) ? uint32_t(uint8_t(q[u])) : 0u;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
@@ -842,8 +843,8 @@ __device__ __forceinline__ void qdq_view(typename X::storage* __restrict__ xb, i
                                          typename Q::storage* __restrict__ qb, int64_t qo, int64_t qs0, int64_t qs1,
                                          const float* __restrict__ scale, int64_t d0, int64_t d1, int64_t nb, int kind, int flags) {
   const int64_t n = d0 * d1;
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; e < n; e += stride) {
+  const int64_t stride = int64_t(gridDim.x) * block_threads();
+  for (int64_t e = int64_t(blockIdx.x) * block_threads() + threadIdx.x; e < n; e += stride) {
     const int64_t r = e / d1, c = e - r * d1;
     const float s = kind == kUniform ? scale[0] : (kind == kRow ? scale[r % nb] : scale[(r / nb) * d1 + c]);
     typename X::storage* xp = xb + xo + r * xs0 + c * xs1;

@@ -7,8 +7,8 @@ using namespace mtrt_dev;
 // than a memset node: it can be recorded into a captured graph like any other launch.
 // (p, count, fill, width) ; count elements of `width` bytes, p aligned to `width`.
 extern "C" __global__ void __launch_bounds__(256) mtrt_fill(uint8_t* __restrict__ p, int64_t count, uint32_t fill, int32_t width) {
-  const int64_t stride = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < count; i += stride) {
+  const int64_t stride = int64_t(gridDim.x) * block_threads();
+  for (int64_t i = int64_t(blockIdx.x) * block_threads() + threadIdx.x; i < count; i += stride) {
     if (width == 4)
       reinterpret_cast<uint32_t*>(p)[i] = fill;
     else if (width == 2)
@@ -31,8 +31,8 @@ struct StridedCopyShape {
 template <typename U>
 __device__ __forceinline__ void copy_strided(const uint8_t* __restrict__ src, uint8_t* __restrict__ dst, int64_t total,
                                              int32_t rank, const StridedCopyShape& sh) {
-  const int64_t step = int64_t(gridDim.x) * blockDim.x;
-  for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < total; i += step) {
+  const int64_t step = int64_t(gridDim.x) * block_threads();
+  for (int64_t i = int64_t(blockIdx.x) * block_threads() + threadIdx.x; i < total; i += step) {
     int64_t rest = i, so = 0, dof = 0;
     for (int d = rank - 1; d > 0; --d) {
       const int64_t q = rest / sh.extent[d], r = rest - q * sh.extent[d];

@@ -348,8 +348,8 @@ int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtyp
   if (mode != 1) args[na++] = &flags_arg;
 
   if (tiles && kind == MTRT_SCALE_COL) {
-    // one wave per (scale block, chunk of 16 rows of it, strip of 64 groups of columns): see qdq_col_strips
-    const int64_t items = (d0 / nb) * ((nb + 15) / 16) * ((d1 / group + 63) / 64);
+    // one wave per (scale block, chunk of 8 rows of it, strip of 64 groups of columns): see qdq_col_strips
+    const int64_t items = (d0 / nb) * ((nb + 7) / 8) * ((d1 / group + 63) / 64);
     return launch(st, name, blocks_for(items, kBlock / 64), kBlock, stream, args);
   }
   if (ragged) {

@@ -1,6 +1,6 @@
 """Where a scale is looked up and a code is formed, at the sizes where either can go wrong: row scales whose trips of 64
 groups hold the ends of no, one or many rows and whose rows go through the scales more than once; column scales whose
-blocks end inside a chunk of 16 rows, a trip of 8, or are one row; integer codes at ties, the ends of their range, beyond it
+blocks end inside a chunk of 8 rows or are one row; integer codes at ties, the ends of their range, beyond it
 and at special values, with scales of either sign.  Bit-exact against the oracle."""
 import numpy as np
 import pytest
