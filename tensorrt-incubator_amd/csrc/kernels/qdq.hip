@@ -401,8 +401,8 @@ constexpr int kColChunkRows = 8;
 // Bound by memory once enough of it is in flight and little else stands in the way: a chunk is what a lane has in flight,
 // asked for before the reciprocals are formed, and everything about a row but the lane's columns is in scalar registers.
 // bf16 [4096, 11008] to int4 in blocks of 128 rows and back (270 MB), us: 67.7 with 4 rows in flight, chunks of 32 and
-// 18 instructions an element; 55.6 with 8 rows, chunks of 16 and the short arithmetic of ExactDivisor; 51.7 with chunks
-// of 8 rows (chunks of 4: 60.6, of 32: 57.2) and the codes left in the caches (see CodeGroup); through the front end 49.4.
+// 18 instructions an element; 55.6 with 8 rows, chunks of 16 and the short arithmetic of ExactDivisor; 53.0 with chunks
+// of 8 rows (of 4: 60.6); 49.4 with the codes left in the caches (see CodeGroup).
 template <typename X, typename Q, int MODE>
 __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                                typename X::storage* __restrict__ y, const float* __restrict__ scale,
