@@ -206,11 +206,16 @@ __device__ __forceinline__ void unpack4<F8>(uint32_t w, float* v) {
   v[0] = f8_to_f32<0>(w); v[1] = f8_to_f32<1>(w); v[2] = f8_to_f32<2>(w); v[3] = f8_to_f32<3>(w);
 }
 
-// Codes are written and read with ordinary accesses, unlike the float operands: a wave's instruction writes half the
-// bytes of one of the float operand's, and written past the caches these pieces cost more than their share.  bf16 -> f8 -> bf16
-// of 128 Mi elements in one pass 109.5 -> 96.6 us, f32 -> i8 -> f32 of 43 Mi 69.7 -> 65.0; int8 codes of 43 Mi
-// bf16, then dequantized, 49.5 -> 46.5.  KEEP = false, where nothing but codes is written with one scale: such a pass alone is
-// 1 to 5 % the slower for it (43 Mi bf16 25.1 against 26.4 us).
+// Codes are read with ordinary accesses, and written so (KEEP) where they are read again soon or are many; the float operands
+// go past the caches.  us, codes past the caches against kept:
+//   row and column scales, a quantize and its dequantize: kept at every size (bf16 -> f8 of 8, 24 and 64 Mi elements 12.3 and 12.4,
+//   32.4 and 30.2, 73.8 and 70.9 by rows; f32 -> i8 of 4 and 64 Mi 12.2 and 11.4, 120 and 109)
+//   quantize and dequantize in one pass (keep_fused): kept above 32 Mi codes, what the eight L2s hold.  Below, the codes
+//   are still dirty there when the launch ends and are written back then.  With the amax in front, bf16 -> f8: 4 Mi 10.2 and
+//   11.3, 16 Mi 25.0 and 25.6, 32 Mi 43.3 and 43.7, 64 Mi 80.6 and 76.8, 128 Mi 156 and 142; f32 -> i8: 8 Mi 22.2 and 22.5, 24 Mi 59.5
+//   and 58.8, 64 Mi 146 and 138
+//   a quantize with one scale: never (43 Mi bf16 alone 25.1 and 26.4, with the amax in front 43.2 and 44.3)
+__device__ __forceinline__ bool keep_fused(int64_t n) { return n > (int64_t(32) << 20); }
 template <bool KEEP, typename T> __device__ __forceinline__ void store_codes(T v, T* p) {
   if (KEEP) *p = v;
   else __builtin_nontemporal_store(v, p);
@@ -418,6 +423,7 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
   const int64_t wave = wave_in_launch(), nwaves = waves_in_launch();
   const int64_t items = nblocks * chunks * strips;
   const bool round = !Codes<Q>::kInteger && (flags & kFlagRoundToInt);
+  const bool keep = MODE != 2 || keep_fused(n);
 
   for (int64_t item = wave; item < items; item += nwaves) {
     const int64_t rest = item / strips;
@@ -473,7 +479,10 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
 #pragma unroll
           for (int k = 0; k < G; ++k) v[k] = quant_value<Q>(v[k], sc[k], flags);
         }
-        if (store) CG::store(q, e, v, flags);         // leaves f32(code) in v
+        if (store) {                                  // leaves f32(code) in v
+          if (keep) CG::store(q, e, v, flags);
+          else CodeGroup<Q, G, false>::store(q, e, v, flags);
+        }
       }
       if (MODE != 0 && store) {
 #pragma unroll
@@ -496,20 +505,24 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   constexpr int G = FG::G;
   constexpr int J = kTile / G;                       // groups per lane per trip
   constexpr int SN = KIND == kCol ? G : 1;           // scale values a lane needs per group
-  using CG = CodeGroup<Q, G, MODE != 0 || KIND != kUniform>;
+  using CG = CodeGroup<Q, G>;
   const int64_t ngroups = n / G;
   const uint32_t groups_per_row = KIND == kUniform ? 1u : uint32_t(d1 / G);
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = wave_in_launch(), nwaves = waves_in_launch();
+  // The fused pass keeps the wave's number per lane: with scalar numbers it was the slower (f16 -> f8 of 14 Mi elements with the amax
+  // in front 23.2 -> 24.3 us, bf16 of 128 Mi 155 -> 158), where a quantize and a dequantize of 4 and 128 Mi gained (7.4 -> 7.3, 133 -> 131).
+  const int64_t wave = MODE == 2 ? (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave : int64_t(wave_in_launch());
+  const int64_t nwaves = MODE == 2 ? int64_t(gridDim.x) * blockDim.x / kWave : int64_t(waves_in_launch());
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
   const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;
+  const bool keep = MODE == 2 ? keep_fused(n) : KIND != kUniform;
 
   for (int64_t base = wave * (kWave * J); base < ngroups; base += nwaves * (kWave * J)) {
     // Row scales: the row of the trip's first group by two divisions for the whole wave, the others from there - a lane's
     // own division and remainder, some 50 instructions, came with every 16 bytes of the tensor.
     uint32_t row0 = 0, col0 = 0, srow0 = 0;
     if (KIND == kRow) {
-      const uint32_t first = uint32_t(base);
+      const uint32_t first = __builtin_amdgcn_readfirstlane(uint32_t(base));
       row0 = first / groups_per_row;
       col0 = first - row0 * groups_per_row;
       srow0 = row0 % wrap;
@@ -568,7 +581,8 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
           const ExactDivisor dv(s[j][0]);
           quantize_group<Q>(dv, v[j], flags);
         }
-        CG::store(q, e, v[j], flags);
+        if (keep) CG::store(q, e, v[j], flags);
+        else CodeGroup<Q, G, false>::store(q, e, v[j], flags);
       }
       if (MODE != 0) {
 #pragma unroll
