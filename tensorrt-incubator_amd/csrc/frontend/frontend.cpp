@@ -857,9 +857,15 @@ struct LinearPlan {
 constexpr const char *kPlanName = "mtrt_frontend.LinearPlan";
 PyObject *s_weight, *s_weight_scale, *s_input_scale, *s_quant_dtype, *s_quant_dim, *s_native_plan, *s_bias;
 
+// The version of a parameter's storage, as tp.Linear._prepared takes it: of every tp.Tensor, instances of subclasses and of
+// other types than their storage's among them (TpTensor::read wants the exact class and would answer "none" then and now).
 int64_t version_of(PyObject *o) {
-  TpTensor t;
-  return t.read(o) ? int64_t(t.t->_version()) : -1;
+  if (!o || !g_tensor || !PyObject_TypeCheck(o, g_tensor))
+    return -1;
+  const std::unique_ptr<PyObject, void (*)(PyObject *)> t(PyObject_GetAttr(o, s_t), [](PyObject *held) { Py_XDECREF(held); });
+  if (!t)
+    PyErr_Clear();
+  return t && THPVariable_Check(t.get()) ? int64_t(THPVariable_Unpack(t.get())._version()) : -1;
 }
 
 // linear_plan(module, route, q_dtype or None, K, N, w, w_frag, w_scale, x_scale) -> what tp_linear reads from the module's

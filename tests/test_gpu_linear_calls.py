@@ -106,6 +106,24 @@ def test_the_general_path_gives_the_same(tp, dname, qname):
     assert torch.allclose(lin(tp.Tensor(host.cuda())).torch().float(), -zero.float(), atol=0.06 if qname == "int4" else 0.03)
 
 
+@pytest.mark.parametrize("dname,qname", [("float16", "int8"), ("float16", None), ("bfloat16", "float8"), ("float16", "int4")])
+def test_in_place_updates_of_a_subclass_parameter_are_noticed(tp, dname, qname):
+    """The prepared weights follow torch's own in-place updates of the weight, of whichever Tensor class it is."""
+    import torch
+
+    class Parameter(tp.Tensor):
+        pass
+    K, N = 192, 72
+    lin, g = _module(tp, 4, K, N, dname, qname, False, qname not in (None, "int4"))
+    lin.weight = Parameter(lin.weight.torch().cuda())
+    x = tp.Tensor(torch.randn((5, K), generator=g).to(getattr(torch, dname)).cuda())
+    y = lin(x).torch()
+    assert tp._native().tp_linear(lin, x) is not NotImplemented      # the plan is current
+    lin.weight.torch().zero_()
+    assert tp._native().tp_linear(lin, x) is NotImplemented
+    assert bool((lin(x).torch() == 0).all()) and bool((y != 0).any())
+
+
 def test_arguments_of_the_c_call(pkg):
     import ctypes
     L = pkg.lib()
