@@ -172,12 +172,16 @@ bool arity(Py_ssize_t n, Py_ssize_t want, const char *name) {
   return false;
 }
 
-// torch calls may throw (out of memory, a bad shape): their exceptions become Python's
+// torch calls may throw (out of memory, an axis that is not there, a bad shape): their exceptions become Python's
 #define FRONTEND_TRY try {
 #define FRONTEND_CATCH                                                   \
   }                                                                      \
   catch (const c10::OutOfMemoryError &e) {                               \
     PyErr_SetString(THPException_OutOfMemory(), e.what_without_backtrace()); \
+    return nullptr;                                                      \
+  }                                                                      \
+  catch (const c10::IndexError &e) {                                     \
+    PyErr_SetString(PyExc_IndexError, e.what_without_backtrace());       \
     return nullptr;                                                      \
   }                                                                      \
   catch (const std::exception &e) {                                      \
@@ -429,7 +433,8 @@ PyObject *f_dynamic_quantize_rows(PyObject *, PyObject *const *a, Py_ssize_t n) 
   FRONTEND_CATCH
 }
 
-// whether blocks run along the last axis (-1 or rank - 1); any axis but the last two fails
+// whether blocks run along the last axis (-1 or rank - 1); any axis but the last two fails, and so does one that a tensor of
+// this rank does not have
 bool last_axis(PyObject *o, int64_t rank, bool *last) {
   int64_t axis;
   if (!integer(o, &axis))
@@ -437,6 +442,10 @@ bool last_axis(PyObject *o, int64_t rank, bool *last) {
   if (axis != -1 && axis != -2 && axis != rank - 1 && axis != rank - 2)
     return fail("axis must be one of the last two");
   *last = axis == -1 || axis == rank - 1;
+  if (rank < (*last ? 1 : 2)) {
+    PyErr_Format(PyExc_IndexError, "axis %lld of a tensor of rank %lld", (long long)axis, (long long)rank);
+    return false;
+  }
   return true;
 }
 

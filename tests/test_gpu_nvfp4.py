@@ -197,3 +197,23 @@ def test_argument_checks(pkg):
     assert L.mtrt_hip_nvfp4_quantize(None, p + 4, pkg.F32, p, p, p, 2, 16, 1) == 1
     assert L.mtrt_hip_nvfp4_quantize(None, p, pkg.F32, p, p, None, 2, 16, 1) == 1
     assert L.mtrt_hip_nvfp4_dequantize(None, p, p, p, p, pkg.F32, 0, 16, 1) == 0
+
+
+def test_axes_a_tensor_does_not_have(pkg):
+    """The second last axis of a vector and any axis of a scalar are index errors; a vector's own axis goes by both names."""
+    import torch
+    amax = torch.tensor(3.0, device="cuda")
+    x = torch.linspace(-3.0, 3.0, 64, device="cuda")
+    with pytest.raises(IndexError):
+        pkg.nvfp4_quantize(x, amax, axis=-2)
+    for axis in (-1, -2):
+        with pytest.raises(IndexError):
+            pkg.nvfp4_quantize(x[0], amax, axis=axis)
+    for call in (lambda: pkg.softmax(x[0]), lambda: pkg.layernorm(x[0], x[0], x[0], 1e-5)):
+        with pytest.raises(IndexError):
+            call()
+    with pytest.raises(AssertionError):
+        pkg.nvfp4_quantize(x, amax, axis=1)
+    q, s = pkg.nvfp4_quantize(x, amax, axis=-1)
+    q2, s2 = pkg.nvfp4_quantize(x, amax, axis=0)
+    assert s.shape == (4,) and torch.equal(q, q2) and torch.equal(s, s2)
