@@ -703,9 +703,9 @@ PyObject *produced(const at::Tensor &t, const TpDtype *dtype) {
   return o;
 }
 
-// A constant scale: its f32 copy on the device (kept on the scale by tp._scale_on_device) and the addressing that its rank
-// and `dim` give over `shape`, by the rules of tp.check_qdq_args and tp._scale_addressing; false when anything is not
-// as those want it.
+// A constant scale: its f32 copy on the device (kept on the scale by tp._scale_on_device, with the version of the constant that
+// it was made from) and the addressing that its rank and `dim` give over `shape`, by the rules of tp.check_qdq_args and
+// tp._scale_addressing; false when anything is not as those want it.
 struct Scale {
   PyObject *hold = nullptr;
   const at::Tensor *dev = nullptr;
@@ -724,9 +724,16 @@ struct Scale {
       PyErr_Clear();
       return false;
     }
-    if (!THPVariable_Check(hold))
+    if (!PyTuple_Check(hold) || PyTuple_GET_SIZE(hold) != 2 || !THPVariable_Check(PyTuple_GET_ITEM(hold, 1)))
       return false;
-    dev = &THPVariable_Unpack(hold);
+    int64_t version;
+    if (!integer(PyTuple_GET_ITEM(hold, 0), &version)) {
+      PyErr_Clear();
+      return false;
+    }
+    if (version != (s.t->is_inference() ? -1 : int64_t(s.t->_version())))
+      return false;
+    dev = &THPVariable_Unpack(PyTuple_GET_ITEM(hold, 1));
     const int64_t rank = int64_t(shape.size()), srank = s.t->dim();
     int64_t numel = 1;
     for (int64_t e : shape)

@@ -260,12 +260,14 @@ def _scale_addressing(shape, scale, dim, op_str):
 
 
 def _scale_on_device(scale):
-    """The device ABI takes f32 scales; f16 / bf16 constants widen exactly."""
+    """The device ABI takes f32 scales; f16 / bf16 constants widen exactly.  Uploaded once per version of the constant: torch's
+    own in-place updates of it are noticed."""
+    version = -1 if scale._t.is_inference() else scale._t._version
     cached = getattr(scale, "_f32_dev", None)
-    if cached is None:
-        cached = scale.torch().to(_torch().float32).contiguous().cuda().reshape(-1)
+    if cached is None or cached[0] != version:
+        cached = (version, scale.torch().to(_torch().float32).contiguous().cuda().reshape(-1))
         scale._f32_dev = cached
-    return cached
+    return cached[1]
 
 
 def _stream():

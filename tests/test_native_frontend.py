@@ -78,3 +78,28 @@ def test_what_is_left_to_the_general_path(tp):
     s.synchronize()
     assert torch.allclose(y.torch(), torch.softmax(x * 2, -1), atol=1e-6)
     assert torch.allclose(native.tp_layernorm(tp.Tensor(x), w, b, 1e-5).torch(), torch.nn.functional.layer_norm(x, (6,)), atol=1e-5)
+
+
+@pytest.mark.gpu
+def test_in_place_updates_of_a_scale_are_noticed(tp):
+    """The device copy of a constant scale belongs to the values it was made from, in both paths and in a Linear."""
+    import torch
+    x = tp.Tensor(torch.full((4, 64), 8.0, device="cuda"))
+    scale = tp.Tensor(np.float32(1.0))
+    q = tp.quantize(x, scale, tp.int8)
+    assert tp._native().tp_quantize(x, scale, tp.int8, None) is not NotImplemented
+    scale.torch().mul_(2)
+    assert tp._native().tp_quantize(x, scale, tp.int8, None) is NotImplemented
+    assert bool((q.torch() == 8).all()) and bool((tp.quantize(x, scale, tp.int8).torch() == 4).all())
+    assert bool((tp.dequantize(q, scale, tp.float32).torch() == 16).all())
+    with torch.inference_mode():                                     # a constant without a version counter
+        fixed = tp.Tensor(torch.tensor(4.0))
+        assert bool((tp.quantize(x, fixed, tp.int8).torch() == 2).all())
+        assert bool((tp._native().tp_quantize(x, fixed, tp.int8, None).torch() == 2).all())
+    lin = tp.Linear(64, 8, bias=False, quant_dtype=tp.float8)
+    lin.load_state_dict({"weight": tp.Tensor(torch.ones(8, 64)), "weight_scale": tp.Tensor(np.float32(0.5)), "input_scale": tp.Tensor(np.float32(0.5))})
+    assert bool((lin(x).torch() == 512).all())
+    lin.input_scale.torch().fill_(2.0 ** -6)                         # 8 / 2^-6 is past the largest code: 448 * 2^-6 = 7
+    assert bool((lin(x).torch() == 448).all())
+    lin.weight_scale.torch().fill_(2.0 ** -9)                        # 448 * 2^-9 = 0.875
+    assert bool((lin(x).torch() == 392).all())
