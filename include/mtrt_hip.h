@@ -243,10 +243,12 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_amax_scales(mtrt_stream_t stream, const void
                                                 int32_t scale_kind, int64_t d0, int64_t d1, int64_t nb,
                                                 float qmax, float *amax_out, float *scale_out);
 
-/* Grid reductions (mtrt_hip_amax and the kernels that fold an amax into another pass) meet in a small
+/* Grid reductions (mtrt_hip_amax and the kernels that fold an amax into another pass) and the GEMMs that share a
+ * tile's K range among workgroups meet in a small
  * block of device memory that the library keeps per stream and that every launch leaves zeroed.  A launch
  * that did not run to completion (a device fault, a killed process sharing the context) can leave it
- * non-zero; this call clears the block of `stream` in stream order.  Blocks are also cleared when first
+ * non-zero; this call clears the block of `stream`, and the words that launches recorded on it into graphs
+ * were given, in stream order (none of those may be running).  Blocks are also cleared when first
  * bound to a stream and return to the pool when the stream is destroyed through any of the stream-destroy
  * entry points of this library. */
 MTRT_CAPI_EXPORTED int32_t mtrt_hip_reset_reductions(mtrt_stream_t stream);

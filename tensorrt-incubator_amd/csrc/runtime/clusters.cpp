@@ -252,6 +252,19 @@ uint32_t blocks_for(int64_t units, uint32_t per_block) {
   return uint32_t(std::max<int64_t>(1, std::min<int64_t>(b, kMaxGrid)));
 }
 
+// The memory of a split launch: the caller's workspace and a ticket per tile.  False where either is missing: the caller then
+// takes the plan without a split.
+template <class Plan>
+bool bind_split(DeviceState *st, hipStream_t stream, Plan &plan, void *workspace, int64_t workspace_bytes) {
+  if (!plan.tile || plan.split.splits <= 1)
+    return true;
+  if (!workspace || !aligned(workspace, 16) || workspace_bytes < plan.workspace())
+    return false;
+  plan.split.partial = workspace;
+  plan.split.tickets = split_tickets(st, stream, uint32_t(plan.tiles));
+  return plan.split.tickets != nullptr;
+}
+
 // mode: 0 quantize, 1 dequantize, 2 fused
 int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtype, void *q,
                      int32_t q_dtype, void *y, const float *scale, int32_t kind, int64_t d0,
@@ -1092,18 +1105,6 @@ W8Plan w8_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   return {W8Plan::kTile, tile};
 }
 
-// The memory of a split launch: the caller's workspace and the stream's tickets.
-bool bind_split(DeviceState *st, hipStream_t stream, FragSplit &split, void *workspace) {
-  if (split.splits <= 1)
-    return true;
-  uint32_t *slot = reduction_slot(st, stream);
-  if (!slot)
-    return false;
-  split.partial = workspace;
-  split.tickets = slot + kTicketOffset;
-  return true;
-}
-
 // a_step: 1 for a scale per row, 0 for one scale; bias: f16 [N] or null; workspace: for K-split tiles, may be null.
 int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, const float *a_scale, uint32_t a_step, const float *w_scale,
                        const void *bias, void *y, int64_t M, int64_t K, int64_t N, void *workspace, int64_t workspace_bytes) {
@@ -1126,7 +1127,7 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     return MTRT_RUNTIME_ERROR;
   const int64_t units = num_compute_units(st), tiles32 = (N + 31) / 32;
   W8Plan plan = w8_plan(M, K, N, units, true);
-  if (plan.kind == W8Plan::kTile && plan.tile.workspace() > (workspace && aligned(workspace, 16) ? workspace_bytes : 0))
+  if (plan.kind == W8Plan::kTile && !bind_split(st, stream, plan.tile, workspace, workspace_bytes))
     plan = w8_plan(M, K, N, units, false);
   if (plan.kind == W8Plan::kSmall16) {
     // one workgroup per 32-column tile, its four waves splitting K; between one and two tiles per compute unit one
@@ -1140,7 +1141,7 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     return launch(st, KernelName(M <= 32 ? "mtrt_gemm_w8a8_frag_rows32" : "mtrt_gemm_w8a8_frag_rows64"),
                   uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), 512, stream, args);
   }
-  const FragPlan &p = plan.tile;
+  FragPlan &p = plan.tile;
   if (!p.tile)
     return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
   if (p.tile->rows == 256 && p.tile->columns == 384) {
@@ -1149,15 +1150,12 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     return launch(st, KernelName(plain ? "mtrt_gemm_w8a8_frag_t256x384" : "mtrt_gemm_w8a8_frag_t256x384_linear").as("mtrt_gemm_w8a8_frag_t256x384"),
                   p.grid(), 256, stream, args);
   }
-  FragSplit split = p.split;
-  if (!bind_split(st, stream, split, workspace))
-    return MTRT_RUNTIME_ERROR;
   KernelName name("mtrt_gemm_w8a8_frag");
   if (p.tile->rows == 32)
     name + "_rows128";
   else if (p.tile->rows != 64)
     name + "_" + p.tile->suffix;
-  void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &split, &a_step, &bias};
+  void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &p.split, &a_step, &bias};
   return launch(st, name.as(p.tile->rows == 32 && M > 64 && M <= 128 ? "mtrt_gemm_w8a8_frag_rows128" : "mtrt_gemm_w8a8_frag"), p.grid(), 256,
                 stream, args);
 }
@@ -1341,7 +1339,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
     }
     if (M * K * 2 < (int64_t(1) << 32)) {
       W4Plan p = w4_plan(M, K, N, cus, true);
-      if (p.workspace() > (workspace && aligned(workspace, 16) ? workspace_bytes : 0))
+      if (!bind_split(st, stream, p, workspace, workspace_bytes))
         p = w4_plan(M, K, N, cus, false);
       if (p.tile) {
         // reported by the class of shapes: up to 64 rows as the small-M kernel of the rows past 32, else as the tile by rounds
@@ -1351,10 +1349,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
         name.as(KernelName("mtrt_gemm_w4a16_") + shown);
         if (p.tile->rows == 256)
           return launch(st, name, p.grid(), p.tile->threads, stream, args);
-        FragSplit split = p.split;
-        if (!bind_split(st, stream, split, workspace))
-          return MTRT_RUNTIME_ERROR;
-        void *targs[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias, &split};
+        void *targs[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias, &p.split};
         return launch(st, name, p.grid(), p.narrow ? 256 : p.tile->threads, stream, targs);
       }
     }
@@ -1404,15 +1399,17 @@ struct DensePlan {
   bool rows = false;
   FragPlan tile;
 };
-DensePlan dense_frag_plan(int64_t M, int64_t K, int64_t N, int64_t units) {
+DensePlan dense_frag_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   DensePlan p;
-  p.tile = frag_plan(M, N, K / 64, units, true);
+  p.tile = frag_plan(M, N, K / 64, units, may_split);
   p.rows = M <= 64 && (!p.tile.tile || frag_rows_us(M, N, K / 64, units) < p.tile.us);
   return p;
 }
 int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, const void *w_frag, const void *bias, void *y, int32_t dtype,
-                        int64_t M, int64_t K, int64_t N, void *partial) {
-  const DensePlan plan = dense_frag_plan(M, K, N, num_compute_units(st));
+                        int64_t M, int64_t K, int64_t N, void *partial, int64_t partial_bytes) {
+  DensePlan plan = dense_frag_plan(M, K, N, num_compute_units(st), true);
+  if (!plan.rows && !bind_split(st, stream, plan.tile, partial, partial_bytes))
+    plan = dense_frag_plan(M, K, N, num_compute_units(st), false);
   const char *xn = float_name(dtype);
   // reported by the class of shapes, as the [N,K] kernels are named
   const KernelName shown = KernelName(M <= 32 ? "mtrt_gemm_dense_rows32_" : M <= 64 ? "mtrt_gemm_dense_rows64_" : M <= 128 ? "mtrt_gemm_dense_rows128_"
@@ -1427,10 +1424,7 @@ int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, cons
   }
   if (!plan.tile.tile)
     return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
-  FragSplit split = plan.tile.split;
-  if (!bind_split(st, stream, split, partial))
-    return MTRT_RUNTIME_ERROR;
-  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &split};
+  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &plan.tile.split};
   return launch(st, name, plan.tile.grid(), 256, stream, args);
 }
 
@@ -1467,7 +1461,7 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
     s.pass = quantized || s.Kp != p.K;
     s.act_bytes = s.pass ? round_up(M * s.Kp * eb, 256) : 0;
     if (s.fragments) {
-      const DensePlan d = dense_frag_plan(M, s.Kp, p.N, units);
+      const DensePlan d = dense_frag_plan(M, s.Kp, p.N, units, true);
       s.partial_bytes = !d.rows && d.tile.tile ? d.tile.workspace() : 0;
     }
   }
@@ -1630,7 +1624,7 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
                   kBlock, as_hip(stream), args);
   }
   if (s.fragments)
-    return dense_fragments(st, as_hip(stream), act, p.w_frag, p.bias, y, p.dtype, M, s.Kp, p.N, partial);
+    return dense_fragments(st, as_hip(stream), act, p.w_frag, p.bias, y, p.dtype, M, s.Kp, p.N, partial, s.partial_bytes);
   return mtrt_hip_linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N);
 }
 

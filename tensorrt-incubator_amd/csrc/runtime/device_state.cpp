@@ -91,6 +91,16 @@ struct DeviceState {
   std::vector<int> free_slots;   // slots of destroyed streams, handed out again before new ones
   std::vector<bool> pinned = std::vector<bool>(kSlots, false);   // handed out under stream capture: never recycled
   int next_slot = 0;
+  // Words of recorded launches (slot_mu).  A launch recorded into a graph keeps its addresses for as long as the graph lives and
+  // runs wherever the graph is replayed, so it meets neither the eager launches of its capture stream nor those of another
+  // graph that was recorded there: its words are its own and never handed out again.  Zero at first, and the kernels return
+  // them to zero.  16 MiB of tickets: 32 thousand recorded launches of 128 tiles each.
+  static constexpr size_t kRecordedTickets = size_t(4) << 20;
+  struct Words {
+    uint32_t *base = nullptr;
+    size_t total = 0, used = 0;
+  } recorded_tickets;
+  std::map<hipStream_t, std::vector<std::pair<uint32_t *, size_t>>> recorded_on;   // by capture stream, for reset_reduction_slot
 };
 
 namespace {
@@ -131,10 +141,14 @@ DeviceState *device_state() {
     delete st;
     return nullptr;
   }
-  const size_t bytes = size_t(DeviceState::kSlots) * DeviceState::kSlotWords * sizeof(uint32_t);
+  const size_t slot_words = size_t(DeviceState::kSlots) * DeviceState::kSlotWords;
+  const size_t bytes = (slot_words + DeviceState::kRecordedTickets) * sizeof(uint32_t);
   e = hipMalloc(reinterpret_cast<void **>(&st->slots), bytes);
   if (e == hipSuccess)
     e = hipMemset(st->slots, 0, bytes);
+  if (e == hipSuccess)
+    e = hipStreamSynchronize(nullptr);   // the zeros of recorded launches' words are not made again on the launches' streams
+  st->recorded_tickets = {st->slots + slot_words, DeviceState::kRecordedTickets, 0};
   if (e != hipSuccess) {
     set_error(MTRT_RUNTIME_ERROR, "allocating reduction slots: %s", hipGetErrorString(e));
     (void)hipModuleUnload(st->module);
@@ -171,14 +185,36 @@ hipFunction_t find_kernel(DeviceState *st, const std::string &name) {
 }
 
 namespace {
-// Stream-ordered clear of one reduction block (a fill kernel, so that it may sit inside a captured graph).
-int32_t clear_slot(DeviceState *st, uint32_t *block, hipStream_t stream) {
+// Stream-ordered clear of one reduction block or of words of recorded launches (a fill kernel, so that it may sit inside a
+// captured graph).
+int32_t clear_words(DeviceState *st, uint32_t *block, int64_t count, hipStream_t stream) {
   uint8_t *p = reinterpret_cast<uint8_t *>(block);
-  int64_t count = DeviceState::kSlotWords;
   uint32_t fill = 0;
   int32_t width = 4;
   void *args[] = {&p, &count, &fill, &width};
-  return launch(st, KernelName("mtrt_fill"), 1, 256, stream, args);
+  return launch(st, KernelName("mtrt_fill"), uint32_t((count + 16383) / 16384), 256, stream, args);
+}
+int32_t clear_slot(DeviceState *st, uint32_t *block, hipStream_t stream) { return clear_words(st, block, DeviceState::kSlotWords, stream); }
+
+bool is_capturing(hipStream_t stream) {
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
+}
+
+// `words` words, in whole lines, for a launch that is being recorded on `stream`; nullptr when there are none left.
+uint32_t *take_recorded(DeviceState *st, DeviceState::Words &from, hipStream_t stream, size_t words) {
+  words = (words + 31) / 32 * 32;
+  std::lock_guard<std::mutex> lock(st->slot_mu);
+  if (from.total - from.used < words)
+    return nullptr;
+  uint32_t *p = from.base + from.used;
+  from.used += words;
+  auto &spans = st->recorded_on[stream];
+  if (!spans.empty() && spans.back().first + spans.back().second == p)
+    spans.back().second += words;
+  else
+    spans.emplace_back(p, words);
+  return p;
 }
 } // namespace
 
@@ -186,8 +222,7 @@ uint32_t *reduction_slot(DeviceState *st, hipStream_t stream) {
   // A kernel recorded into a graph keeps the block's address in its arguments for as long as the graph is replayed,
   // which can be long after the capture stream is gone: a block handed out while its stream is capturing stays out
   // of the free list for good (256 blocks per device; a capture stream is normally bound once).
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  const bool capturing = hipStreamIsCapturing(stream, &capture) == hipSuccess && capture != hipStreamCaptureStatusNone;
+  const bool capturing = is_capturing(stream);
   std::lock_guard<std::mutex> lock(st->slot_mu);
   auto it = st->slot_of.find(stream);
   if (it != st->slot_of.end()) {
@@ -220,13 +255,36 @@ uint32_t *reduction_slot(DeviceState *st, hipStream_t stream) {
   return block;
 }
 
+uint32_t *split_tickets(DeviceState *st, hipStream_t stream, uint32_t tiles) {
+  // hipStreamPerThread names another stream in every thread, so its block would not be one stream's
+  if (stream == hipStreamPerThread)
+    return nullptr;
+  if (is_capturing(stream))
+    return take_recorded(st, st->recorded_tickets, stream, tiles);
+  uint32_t *slot = reduction_slot(st, stream);
+  if (!slot) {
+    clear_error();                                     // no failure of the call: it runs unsplit
+    return nullptr;
+  }
+  return slot + kTicketOffset;
+}
+
 int32_t reset_reduction_slot(DeviceState *st, hipStream_t stream) {
   int slot = -1;
+  std::vector<std::pair<uint32_t *, size_t>> recorded;
   {
     std::lock_guard<std::mutex> lock(st->slot_mu);
     auto it = st->slot_of.find(stream);
     if (it != st->slot_of.end())
       slot = it->second;
+    auto rec = st->recorded_on.find(stream);
+    if (rec != st->recorded_on.end())
+      recorded = rec->second;
+  }
+  for (const auto &span : recorded) {
+    const int32_t rc = clear_words(st, span.first, int64_t(span.second), stream);
+    if (rc != MTRT_OK)
+      return rc;
   }
   if (slot < 0)
     return MTRT_OK;   // nothing bound: the next reduction on this stream clears its block itself
@@ -249,6 +307,7 @@ void forget_stream(hipStream_t stream) {
     {
       std::lock_guard<std::mutex> lock(st->slot_mu);
       bound = st->slot_of.count(stream) != 0;
+      st->recorded_on.erase(stream);                   // the words stay with their graphs
     }
     if (!bound)
       continue;

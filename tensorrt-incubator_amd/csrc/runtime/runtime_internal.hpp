@@ -39,7 +39,11 @@ hipFunction_t find_kernel(DeviceState *, const std::string &name);   // nullptr 
 uint32_t *reduction_slot(DeviceState *, hipStream_t stream);         // nullptr + set_error
 // The tickets of K-split GEMM tiles inside a stream's reduction block: one zero word per tile, returned to zero by the launch.
 constexpr uint32_t kTicketOffset = 64 * 32, kTickets = 512;          // in 32-bit words
-int32_t reset_reduction_slot(DeviceState *, hipStream_t stream);     // stream-ordered clear of the stream's block
+// The tickets of a K-split launch of `tiles` <= kTickets tiles on `stream`: the stream's, or, while the stream is being captured,
+// words of the launch's own.  nullptr (and no error set) when there are none: the launch then runs unsplit.
+uint32_t *split_tickets(DeviceState *, hipStream_t stream, uint32_t tiles);
+// Stream-ordered clear of the stream's block and of the words of what was recorded on it.
+int32_t reset_reduction_slot(DeviceState *, hipStream_t stream);
 void forget_stream(hipStream_t stream);                              // before a stream is destroyed
 
 // Set-up half of the allocation-free entry point (no_alloc.hip): looks up, with `device` current, the

@@ -1,0 +1,104 @@
+"""What the GEMM entry points launch, seen on the CPU (dispatch.py): the tickets of K-split launches belong to a stream, or to the one
+launch where it is recorded into a graph, and a call that gets none, for whatever reason, runs unsplit."""
+import pytest
+
+import dispatch
+
+TICKETS = 512 * 4                                                    # bytes a stream keeps
+
+
+@pytest.fixture(scope="module")
+def library(tmp_path_factory):
+    folder = tmp_path_factory.mktemp("dispatch")
+    return folder, dispatch.build(str(folder))
+
+
+@pytest.fixture
+def gpu(pkg, library, request):
+    folder, path = library
+    return dispatch.Dispatch(pkg, path, str(folder / (request.node.name.replace("/", "_") + ".so")))
+
+
+def _calls(gpu, pkg):
+    """One call of each family that splits its K."""
+    return [lambda s: gpu.w8a8(s, 200, 12288, 512), lambda s: gpu.w4a16(s, 64, 8192, 96), lambda s: gpu.linear(s, 100, 11520, 320, pkg.F16),
+            lambda s: gpu.linear(s, 100, 11520, 320, pkg.F16, route=0, q_dtype=pkg.I8)]
+
+
+def test_tickets_belong_to_a_stream_or_to_a_recorded_launch(gpu, pkg):
+    calls = _calls(gpu, pkg)
+    eager = {}
+    for stream in (8, 16):
+        words = {call(stream)[2][3] for call in calls for _ in range(2)}
+        assert len(words) == 1                                       # launches of one stream follow one another
+        eager[stream] = words.pop()
+    assert abs(eager[8] - eager[16]) >= TICKETS
+    taken = []                                                       # [first, past the last) of what was recorded
+    for stream in (8, 16, 24, 8):
+        gpu.capturing(stream, True)
+        for call in calls:
+            name, on, split = call(stream)
+            assert on == stream and split[0] > 1, name
+            taken.append((split[3], split[3] + 4))
+        gpu.capturing(stream, False)
+    # a launch's words end where the next one's begin at the latest, and none are a stream's
+    taken.sort()
+    assert all(a[1] <= b[0] and a[0] % 128 == 0 for a, b in zip(taken, taken[1:]))
+    assert all(t[0] >= e + TICKETS or t[1] <= e for t in taken for e in eager.values())
+    assert [call(8)[2][3] for call in calls] == [eager[8]] * len(calls)
+
+
+@pytest.mark.parametrize("tiles_n,tiles", [(512, 8), (4096, 32), (96, 1)])
+def test_a_recorded_launch_has_a_word_for_every_tile(gpu, tiles_n, tiles):
+    gpu.capturing(8, True)
+    first = gpu.w8a8(8, 200, 12288, tiles_n)
+    second = gpu.w8a8(8, 200, 12288, tiles_n)
+    assert first[2][0] > 1 and second[2][3] - first[2][3] >= 4 * tiles
+
+
+def test_a_call_without_tickets_runs_unsplit(gpu, pkg):
+    calls = _calls(gpu, pkg)
+    split = [call(8)[2][0] for call in calls]
+    assert min(split) > 1
+    # the stream handle that names another stream in every thread
+    assert all(call(2)[2] is None or call(2)[2][0] == 1 for call in calls)
+    # more streams than the library keeps blocks for; one given back serves the next
+    for stream in range(1, 256):
+        assert calls[1](4096 + 8 * stream)[2][0] > 1
+    for call in calls:
+        name, _, s = call(64)
+        assert s is None or s[0] == 1, name
+    assert not gpu.lib.mtrt_hip_last_error()
+    gpu.lib.fake_destroy_stream(4096 + 8)
+    assert [call(64)[2][0] for call in calls] == split
+
+
+def test_recorded_words_run_out_without_a_failure(gpu):
+    """Nothing that was recorded is handed out again, also not after its stream is gone; what comes after them runs unsplit."""
+    gpu.capturing(8, True)
+    seen = set()
+    while True:
+        _, _, split = gpu.w8a8(8, 200, 14336, 8192)
+        if split is None or split[0] == 1:
+            break
+        assert split[3] not in seen
+        seen.add(split[3])
+        assert len(seen) <= 1 << 17
+    assert len(seen) == (4 << 20) // 128 and not gpu.lib.mtrt_hip_last_error()       # 128 tiles each
+    gpu.capturing(8, False)
+    gpu.lib.fake_destroy_stream(8)
+    gpu.capturing(8, True)
+    _, _, split = gpu.w8a8(8, 200, 14336, 8192)
+    assert split is None or split[0] == 1
+    assert gpu.w8a8(16, 200, 14336, 8192)[2][0] > 1           # eager work is not concerned
+
+
+def test_a_reset_clears_what_was_recorded_on_the_stream(gpu):
+    gpu.capturing(8, True)
+    recorded = [gpu.w8a8(8, 200, 12288, 512)[2][3] for _ in range(3)]
+    gpu.capturing(8, False)
+    eager = gpu.w8a8(8, 200, 12288, 512)[2][3]
+    del gpu.fills[:]
+    assert gpu.lib.mtrt_hip_reset_reductions(8) == 0
+    for words in recorded + [eager]:
+        assert any(p <= words and words + 32 <= p + 4 * n for p, n, _ in gpu.fills), gpu.fills

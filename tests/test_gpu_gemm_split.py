@@ -102,6 +102,47 @@ def test_w8a8_split_launches_on_two_streams_and_in_a_graph(pkg):
         assert torch.equal(y, pkg.gemm_w8a8_fragments(static, frag[0], a_s, w_s, 512)), k
 
 
+def test_graphs_recorded_on_one_stream_replay_at_once(pkg):
+    """Two graphs recorded on the same stream, replayed together on two others, with eager launches on the recording stream beside
+    them: every launch has tickets of its own, so each result is the eager one."""
+    import importlib
+
+    import torch
+    tp = importlib.import_module(pkg.__name__ + ".tp")
+    a8, w8, a_s, w_s = _inputs(5, 200, 12288, 512)
+    f8 = pkg.gemm_w8a8_prepack_fragments(w8)
+    a4, packed, s4, _ = _w4_inputs(6, 64, 8192, 96, 128)
+    p4 = pkg.gemm_w4a16_prepack(packed, 8192, 96)
+    lin = tp.Linear(11520, 320, dtype=tp.float16)
+    lin.weight = tp.Tensor((torch.randn(320, 11520) * 0.05).half())
+    x = torch.randn(100, 11520).half().cuda()
+
+    def calls(shift):
+        return [pkg.gemm_w8a8_fragments(a8.roll(shift, 0), f8, a_s, w_s, 512),
+                pkg.gemm_w4a16(a4.roll(shift, 0), s4, 8192, 96, 128, w_prepacked=p4), lin(tp.Tensor(x.roll(shift, 0))).torch()]
+    want = [calls(k) for k in range(3)]
+    torch.cuda.synchronize()
+    record, streams = torch.cuda.Stream(), [torch.cuda.Stream(), torch.cuda.Stream()]
+    graphs, results = [torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()], [[], []]
+    for k in range(2):
+        with torch.cuda.graph(graphs[k], stream=record):             # a memory pool each
+            for _ in range(10):
+                results[k] += calls(k)
+    for replay in range(4):
+        for y in results[0] + results[1]:
+            y.zero_()
+        torch.cuda.synchronize()
+        for k in range(2):
+            with torch.cuda.stream(streams[k]):
+                graphs[k].replay()
+        with torch.cuda.stream(record):
+            eager = [y for _ in range(5) for y in calls(2)]
+        torch.cuda.synchronize()
+        for ys, expect, who in ((results[0], want[0], "first graph"), (results[1], want[1], "second graph"), (eager, want[2], "eager")):
+            for i, y in enumerate(ys):
+                assert torch.equal(y, expect[i % 3]), (replay, who, i)
+
+
 def _w4_inputs(seed, M, K, N, B):
     import torch
     g = torch.Generator(device="cuda")
