@@ -94,12 +94,13 @@ struct DeviceState {
   // Words of recorded launches (slot_mu).  A launch recorded into a graph keeps its addresses for as long as the graph lives and
   // runs wherever the graph is replayed, so it meets neither the eager launches of its capture stream nor those of another
   // graph that was recorded there: its words are its own and never handed out again.  Zero at first, and the kernels return
-  // them to zero.  16 MiB of tickets: 32 thousand recorded launches of 128 tiles each.
-  static constexpr size_t kRecordedTickets = size_t(4) << 20;
+  // them to zero (or, dynq.hip, to what the next run of the same launch takes for empty).  16 MiB of tickets: 32 thousand
+  // recorded launches of 128 tiles each; 16 MiB of reduction blocks: 2048 recorded reductions.
+  static constexpr size_t kRecordedTickets = size_t(4) << 20, kRecordedBlocks = size_t(4) << 20;
   struct Words {
     uint32_t *base = nullptr;
     size_t total = 0, used = 0;
-  } recorded_tickets;
+  } recorded_tickets, recorded_blocks;
   std::map<hipStream_t, std::vector<std::pair<uint32_t *, size_t>>> recorded_on;   // by capture stream, for reset_reduction_slot
 };
 
@@ -142,13 +143,14 @@ DeviceState *device_state() {
     return nullptr;
   }
   const size_t slot_words = size_t(DeviceState::kSlots) * DeviceState::kSlotWords;
-  const size_t bytes = (slot_words + DeviceState::kRecordedTickets) * sizeof(uint32_t);
+  const size_t bytes = (slot_words + DeviceState::kRecordedTickets + DeviceState::kRecordedBlocks) * sizeof(uint32_t);
   e = hipMalloc(reinterpret_cast<void **>(&st->slots), bytes);
   if (e == hipSuccess)
     e = hipMemset(st->slots, 0, bytes);
   if (e == hipSuccess)
     e = hipStreamSynchronize(nullptr);   // the zeros of recorded launches' words are not made again on the launches' streams
   st->recorded_tickets = {st->slots + slot_words, DeviceState::kRecordedTickets, 0};
+  st->recorded_blocks = {st->recorded_tickets.base + DeviceState::kRecordedTickets, DeviceState::kRecordedBlocks, 0};
   if (e != hipSuccess) {
     set_error(MTRT_RUNTIME_ERROR, "allocating reduction slots: %s", hipGetErrorString(e));
     (void)hipModuleUnload(st->module);
@@ -219,10 +221,14 @@ uint32_t *take_recorded(DeviceState *st, DeviceState::Words &from, hipStream_t s
 } // namespace
 
 uint32_t *reduction_slot(DeviceState *st, hipStream_t stream) {
-  // A kernel recorded into a graph keeps the block's address in its arguments for as long as the graph is replayed,
-  // which can be long after the capture stream is gone: a block handed out while its stream is capturing stays out
-  // of the free list for good (256 blocks per device; a capture stream is normally bound once).
+  // A launch that is being recorded gets a block of its own.  When there are none left it gets its stream's, whose address
+  // the graph then keeps for as long as it is replayed, which can be long after the capture stream is gone: such a block
+  // stays out of the free list for good.
   const bool capturing = is_capturing(stream);
+  if (capturing) {
+    if (uint32_t *own = take_recorded(st, st->recorded_blocks, stream, kTicketOffset))
+      return own;
+  }
   std::lock_guard<std::mutex> lock(st->slot_mu);
   auto it = st->slot_of.find(stream);
   if (it != st->slot_of.end()) {

@@ -38,7 +38,8 @@ def build(folder):
 
 class Dispatch:
     """The library with a state of its own (a copy of the file: a loaded library's state is the process's).  `launches`
-    collects (kernel, stream, (splits, per, partial, tickets) or None), `fills` the clears (address, words, stream)."""
+    collects (kernel, stream, its (splits, per, partial, tickets) or the address of its reduction block or None), `fills` the
+    clears (address, words, stream)."""
 
     def __init__(self, pkg, path, copy):
         shutil.copy(path, copy)
@@ -75,7 +76,9 @@ class Dispatch:
             return
         at = self._split_argument(name)
         split = None
-        if at is not None:
+        if name.startswith(("mtrt_amax_", "mtrt_dynqdq_")):
+            split = ctypes.cast(args[5 if name.startswith("mtrt_amax_") else 7], ctypes.POINTER(_vp))[0]
+        elif at is not None:
             s = ctypes.cast(args[at], ctypes.POINTER(Split))[0]
             split = (s.splits, s.per, s.partial, s.tickets)
         self.launches.append((name, stream, split))
@@ -99,4 +102,12 @@ class Dispatch:
                        x_scale=256 if q_dtype >= 0 else None)
         need = self.lib.mtrt_hip_linear_workspace(ctypes.byref(p), M)
         assert self.lib.mtrt_hip_linear(stream, ctypes.byref(p), 256, 256, M, 4096 if need else None, need) == 0
+        return self.launches[-1]
+
+    def amax(self, stream, dtype):
+        assert self.lib.mtrt_hip_amax(stream, 256, dtype, 4096, 127.0, 256, 256) == 0
+        return self.launches[-1]
+
+    def dynamic(self, stream, dtype, code):
+        assert self.lib.mtrt_hip_dynamic_quantize_dequantize(stream, 256, dtype, 256, code, 256, 1 << 20, 127.0, 256, 256, 0) == 0
         return self.launches[-1]

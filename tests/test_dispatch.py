@@ -1,5 +1,6 @@
-"""What the GEMM entry points launch, seen on the CPU (dispatch.py): the tickets of K-split launches belong to a stream, or to the one
-launch where it is recorded into a graph, and a call that gets none, for whatever reason, runs unsplit."""
+"""What the entry points launch, seen on the CPU (dispatch.py): the words in which workgroups meet (tickets of K-split GEMMs, blocks of
+grid-wide reductions) belong to a stream, or to the one launch where it is recorded into a graph; a GEMM that gets none, for
+whatever reason, runs unsplit, a reduction recorded when there are no more takes its stream's."""
 import pytest
 
 import dispatch
@@ -102,3 +103,34 @@ def test_a_reset_clears_what_was_recorded_on_the_stream(gpu):
     assert gpu.lib.mtrt_hip_reset_reductions(8) == 0
     for words in recorded + [eager]:
         assert any(p <= words and words + 32 <= p + 4 * n for p, n, _ in gpu.fills), gpu.fills
+
+
+def test_recorded_reductions_have_blocks_of_their_own(gpu, pkg):
+    calls = [lambda s: gpu.amax(s, pkg.BF16), lambda s: gpu.dynamic(s, pkg.F32, pkg.I8)]
+    eager = {stream: {call(stream)[2] for call in calls} for stream in (8, 16)}
+    assert all(len(blocks) == 1 for blocks in eager.values())
+    taken = []
+    for stream in (8, 24, 16):
+        gpu.capturing(stream, True)
+        taken += [call(stream)[2] for call in calls]
+        gpu.capturing(stream, False)
+    every = sorted(taken + [b for blocks in eager.values() for b in blocks])
+    assert all(a + 4 * 32 * 50 <= b for a, b in zip(every, every[1:]))   # 33 lines of amax.hip, 17 of dynq.hip
+    assert not gpu.fills or all(stream in (8, 16) for _, _, stream in gpu.fills)
+    assert {call(8)[2] for call in calls} == eager[8]
+    del gpu.fills[:]
+    assert gpu.lib.mtrt_hip_reset_reductions(8) == 0
+    for block in taken[:2] + list(eager[8]):
+        assert any(p <= block and block + 4 * 2048 <= p + 4 * n for p, n, _ in gpu.fills), gpu.fills
+
+
+def test_reductions_recorded_when_the_blocks_are_gone_take_their_streams(gpu, pkg):
+    gpu.capturing(8, True)
+    own = [gpu.amax(8, pkg.F32)[2] for _ in range(2048)]
+    assert len(set(own)) == 2048
+    shared = gpu.amax(8, pkg.F32)[2]
+    assert shared not in own and gpu.amax(8, pkg.F32)[2] == shared
+    gpu.capturing(8, False)
+    assert gpu.amax(8, pkg.F32)[2] == shared
+    gpu.lib.fake_destroy_stream(8)                                   # a graph names the block: it goes to nobody else
+    assert shared not in {gpu.amax(8 + 8 * k, pkg.F32)[2] for k in range(255)}

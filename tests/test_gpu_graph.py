@@ -1,7 +1,7 @@
 """The cluster entry points under HIP graph capture: a captured dynamic-fp8 pipeline (amax -> scale on
 device -> fused quantize + dequantize -> LayerNorm) replays with the results of the eager run, several times,
 with eager work and synchronisations between the replays.  Nothing in these entry points allocates, memsets
-or synchronises, so they can be recorded; the amax reduction cleans its own scratch at the end of each launch."""
+or synchronises, so they can be recorded; a recorded reduction has scratch of its own, which it cleans at the end of each launch."""
 import ctypes
 
 import numpy as np
@@ -108,3 +108,36 @@ def test_captured_one_launch_dynamic_quantization_replays_like_eager(pkg):
         x2 = torch.randn(300, 1024, device="cuda")
         q2, y2, a2, s2 = pkg.dynamic_quantize_dequantize(x2, pkg.I8, 127.0)
         assert float(a2) == float(x2.abs().max())
+
+
+def test_graphs_with_reductions_recorded_on_one_stream_replay_at_once(pkg):
+    """Two graphs of amax and one-launch dynamic quantizations recorded on the same stream, replayed together on two others, with
+    eager calls on the recording stream beside them: no launch meets another one's maxima."""
+    import torch
+    torch.manual_seed(13)
+    xs = [torch.randn(300, 4096, device="cuda") * 2.0 ** k for k in range(3)]
+
+    def calls(x):
+        q, y, amax, scale = pkg.dynamic_quantize_dequantize(x, pkg.I8, 127.0)
+        return [q, y, amax, scale, *pkg.amax(x, 448.0)]
+    want = [calls(x) for x in xs]
+    torch.cuda.synchronize()
+    record, streams = torch.cuda.Stream(), [torch.cuda.Stream(), torch.cuda.Stream()]
+    graphs, results = [torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()], [[], []]
+    for k in range(2):
+        with torch.cuda.graph(graphs[k], stream=record):             # a memory pool each
+            for _ in range(10):
+                results[k] += calls(xs[k])
+    for replay in range(4):
+        for t in results[0] + results[1]:
+            t.zero_()
+        torch.cuda.synchronize()
+        for k in range(2):
+            with torch.cuda.stream(streams[k]):
+                graphs[k].replay()
+        with torch.cuda.stream(record):
+            eager = [t for _ in range(5) for t in calls(xs[2])]
+        torch.cuda.synchronize()
+        for ts, expect, who in ((results[0], want[0], "first graph"), (results[1], want[1], "second graph"), (eager, want[2], "eager")):
+            for i, t in enumerate(ts):
+                assert torch.equal(t, expect[i % len(expect)]), (replay, who, i)
