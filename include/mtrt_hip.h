@@ -573,8 +573,7 @@ struct mtrt_lua_builtin {
 MTRT_CAPI_EXPORTED const struct mtrt_lua_builtin *mtrt_lua_cuda_builtins(size_t *count);
 
 /* Name of the kernel that the most recent successful part-2 call on this thread
- * launched last (for profiles and tests).  Where one GEMM exists in several tiles the name is that of the class of
- * shapes the call belongs to; the symbol of the tile adds a suffix to it or replaces it. */
+ * launched last (for profiles and tests): its symbol in the built-in module. */
 MTRT_CAPI_EXPORTED const char *mtrt_hip_last_kernel(void);
 
 #ifdef __cplusplus

@@ -322,7 +322,7 @@ MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
 // operands through LDS in 256-row tiles (f16, us): (M, K, N) = (999, 4096, 11008) 113 -> 83, (2048, 4096, 11008) 197 -> 147,
 // (256, 4096, 4096) 58 -> 16, (398, 11520, 1856) 165 -> 30, (1024, 2048, 2048) 32 -> 12.5, (200, 12288, 512) 164 -> 12.7.
 // mtrt_gemm_dense_frag_<type>_t<rows>x<columns> (x [M,K], w_frag, bias [N] or null, y [M,N], M, K, N, Split) ;
-// K % 64 == 0, x and w_frag 16-byte aligned, x below 4 GiB; the rest as mtrt_gemm_w8a8_frag.
+// K % 64 == 0, x and w_frag 16-byte aligned, x below 4 GiB; the rest as mtrt_gemm_w8a8_frag_t<rows>x<columns>.
 #define MTRT_DENSE_FRAG_KERNEL(XN, XT, IT, JT, D, WG, TILE)                                                               \
   extern "C" __global__ void __launch_bounds__(256, WG) mtrt_gemm_dense_frag_##XN##_##TILE(                               \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \

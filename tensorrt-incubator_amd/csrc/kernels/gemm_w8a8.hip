@@ -120,10 +120,10 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
 }
 
 // ---- weights in fragment order (gemm_frag.hpp) ---------------------------------------------------------
-// mtrt_gemm_w8a8_frag[_rows128 | _t<rows>x<columns>] (a [M,K] i8, w_frag, a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, Split,
+// mtrt_gemm_w8a8_frag_t<rows>x<columns> (a [M,K] i8, w_frag, a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, Split,
 // a_step, bias) ; K % 128 == 0, a and w_frag 16-byte aligned, a below 4 GiB; a_step 1, or 0 for a
 // single a_scale; bias f16 [N] or null.
-// grid = 8 * ceil(tiles * splits / 8), block = 256.  Tiles of 64 x 128 (no suffix), 32 x 128 (_rows128), 128 x 128 (two
+// grid = 8 * ceil(tiles * splits / 8), block = 256.  Tiles of 32 x 128, 64 x 128 and 128 x 128 (two
 // workgroups per compute unit), 128 x 256, 128 x 384 and 256 x 256 (one; the last never split).  Which tile and how many splits: the host's
 // estimate of the launch (frag_plan in clusters.cpp).  Measured, the one 256-row tile loop that these replaced -> now,
 // us: (M, K, N) = (256, 4096, 4096) 21.8 -> 10.4, (398, 11520, 1856) 51.8 -> 19.3, (1024, 2048, 2048) 14.7 -> 8.8,
@@ -140,8 +140,8 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
     Epilogue epi{a_scale, w_scale, a_step, bias};                                                                         \
     gemm_frag::run<I8Traits, IT, JT, D>(a, K, w_frag, epi, y, M, N, part, lds);                                           \
   }
-MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_rows128, 1, 1, 4, 2)
-MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag, 2, 1, 4, 2)
+MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t32x128, 1, 1, 4, 2)
+MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t64x128, 2, 1, 4, 2)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x128, 4, 1, 2, 2)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x256, 4, 2, 2, 1)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x384, 4, 3, 2, 1)
@@ -413,7 +413,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_nk_rows128(
 
 // Up to 32 and 64 rows on fragment-order weights: the same kernels with the weight fragments straight from
 // memory into registers.  (a [M,K] i8, w_frag, a_scale, w_scale, y, M, K, N, a_step, bias) ; K % 128 == 0, a and w_frag
-// 16-byte aligned; a_step and bias as for mtrt_gemm_w8a8_frag; grid: any, block = 512.
+// 16-byte aligned; a_step and bias as for the tiles; grid: any, block = 512.
 #define MTRT_W8_FRAG_ROWS_KERNEL(NAME, MT)                                                                                \
   extern "C" __global__ void __launch_bounds__(512) NAME(                                                                 \
       const int8_t* __restrict__ a, const int8_t* __restrict__ w_frag, const float* __restrict__ a_scale,                 \

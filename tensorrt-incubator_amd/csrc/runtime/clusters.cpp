@@ -163,7 +163,6 @@ struct W4Plan {
   FragSplit split;
   double us = 0.0;
   bool narrow = false;                                 // 128 x 64 tiles: matrices of at most 64 columns, where 128 x 128 would run
-  const char *by_rounds = nullptr;                     // the tile the choice by rounds names: how the launch is reported
   uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(split.splits) + 7) / 8)); }
   int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * tile->rows * tile->columns * 4 : 0; }
 };
@@ -215,7 +214,6 @@ W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
         best = p;
     }
   }
-  best.by_rounds = by_rounds == &t128 && N <= 64 ? "t128x64" : by_rounds->suffix;
   return best;
 }
 
@@ -1147,17 +1145,10 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
   if (p.tile->rows == 256 && p.tile->columns == 384) {
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
     const bool plain = a_step == 1 && !bias;
-    return launch(st, KernelName(plain ? "mtrt_gemm_w8a8_frag_t256x384" : "mtrt_gemm_w8a8_frag_t256x384_linear").as("mtrt_gemm_w8a8_frag_t256x384"),
-                  p.grid(), 256, stream, args);
+    return launch(st, KernelName(plain ? "mtrt_gemm_w8a8_frag_t256x384" : "mtrt_gemm_w8a8_frag_t256x384_linear"), p.grid(), 256, stream, args);
   }
-  KernelName name("mtrt_gemm_w8a8_frag");
-  if (p.tile->rows == 32)
-    name + "_rows128";
-  else if (p.tile->rows != 64)
-    name + "_" + p.tile->suffix;
   void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &p.split, &a_step, &bias};
-  return launch(st, name.as(p.tile->rows == 32 && M > 64 && M <= 128 ? "mtrt_gemm_w8a8_frag_rows128" : "mtrt_gemm_w8a8_frag"), p.grid(), 256,
-                stream, args);
+  return launch(st, KernelName("mtrt_gemm_w8a8_frag_") + p.tile->suffix, p.grid(), 256, stream, args);
 }
 } // namespace
 
@@ -1342,11 +1333,8 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
       if (!bind_split(st, stream, p, workspace, workspace_bytes))
         p = w4_plan(M, K, N, cus, false);
       if (p.tile) {
-        // reported by the class of shapes: up to 64 rows as the small-M kernel of the rows past 32, else as the tile by rounds
-        const char *shown = M > 64 ? p.by_rounds : M > 48 ? "skinny" : strips ? "strips16" : "skinny16";
         KernelName name("mtrt_gemm_w4a16_");
         name + (p.narrow ? "t128x64" : p.tile->suffix) + (bias ? "_bias" : "");
-        name.as(KernelName("mtrt_gemm_w4a16_") + shown);
         if (p.tile->rows == 256)
           return launch(st, name, p.grid(), p.tile->threads, stream, args);
         void *targs[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias, &p.split};
@@ -1411,12 +1399,8 @@ int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, cons
   if (!plan.rows && !bind_split(st, stream, plan.tile, partial, partial_bytes))
     plan = dense_frag_plan(M, K, N, num_compute_units(st), false);
   const char *xn = float_name(dtype);
-  // reported by the class of shapes, as the [N,K] kernels are named
-  const KernelName shown = KernelName(M <= 32 ? "mtrt_gemm_dense_rows32_" : M <= 64 ? "mtrt_gemm_dense_rows64_" : M <= 128 ? "mtrt_gemm_dense_rows128_"
-                                                                                                          : "mtrt_gemm_dense_mfma_") + xn;
   KernelName name("mtrt_gemm_dense_frag_");
   name + xn + "_" + (plan.rows ? (M <= 32 ? "rows32" : "rows64") : plan.tile.tile ? plan.tile.tile->suffix : "");
-  name.as(shown);
   if (plan.rows || (plan.tile.tile && plan.tile.tile->columns == 384 && plan.tile.tile->rows == 256)) {
     void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N};
     return launch(st, name, plan.rows ? uint32_t(std::min<int64_t>((N + 31) / 32, int64_t(kMaxGrid) * 1024)) : plan.tile.grid(),

@@ -380,10 +380,10 @@ int32_t launch(DeviceState *st, const KernelName &kernel, uint32_t grid, uint32_
     return set_error(MTRT_DRIVER_ERROR, "launching '%s' grid %u block %u: %s", kernel.text, grid, block,
                      hipGetErrorString(e));
   }
-  if (hit && !kernel.shown[0]) {
+  if (hit) {
     tl_kernel_ptr = hit->name;
   } else {
-    std::snprintf(tl_kernel, sizeof(tl_kernel), "%s", kernel.shown[0] ? kernel.shown : kernel.text);
+    std::snprintf(tl_kernel, sizeof(tl_kernel), "%s", kernel.text);
     tl_kernel_ptr = tl_kernel;
   }
   return MTRT_OK;

@@ -53,14 +53,8 @@ int32_t no_alloc_setup(DeviceState *, int device);
 // A kernel name put together on the stack (no heap, no locale): KernelName("mtrt_q_") + kind + "_" + x.
 struct KernelName {
   char text[72];
-  char shown[72];                                      // what mtrt_hip_last_kernel reports, when not `text`
   uint32_t len = 0;
-  KernelName(const char *s) { text[0] = shown[0] = '\0'; *this + s; }
-  // Reported under another name: the tiles of one GEMM go by the name of the class of shapes they serve.
-  KernelName &as(const KernelName &name) {
-    __builtin_memcpy(shown, name.text, sizeof(shown));
-    return *this;
-  }
+  KernelName(const char *s) { text[0] = '\0'; *this + s; }
   KernelName &operator+(const char *s) {
     while (*s && len + 1 < sizeof(text))
       text[len++] = *s++;

@@ -61,7 +61,7 @@ class Dispatch:
     @staticmethod
     def _split_argument(name):
         """Which argument of a kernel is its Split, or None."""
-        if name.startswith("mtrt_gemm_w8a8_frag") and "rows32" not in name and "rows64" not in name and "t256x384" not in name:
+        if name.startswith("mtrt_gemm_w8a8_frag_t") and "t256x384" not in name:
             return 8
         if name.startswith("mtrt_gemm_w4a16_t") and "_t256" not in name:
             return 9

@@ -134,3 +134,36 @@ def test_reductions_recorded_when_the_blocks_are_gone_take_their_streams(gpu, pk
     assert gpu.amax(8, pkg.F32)[2] == shared
     gpu.lib.fake_destroy_stream(8)                                   # a graph names the block: it goes to nobody else
     assert shared not in {gpu.amax(8 + 8 * k, pkg.F32)[2] for k in range(255)}
+
+
+def test_last_kernel_is_the_symbol_that_was_launched(gpu, pkg):
+    """Over every family and route, at sizes that take each kernel of it at some point."""
+    import random
+    r = random.Random(3)
+    seen = set()
+    for _ in range(1500):
+        M, K, N = int(2 ** r.uniform(0, 12)), 128 * int(2 ** r.uniform(0, 6.5)), int(2 ** r.uniform(3, 14))
+        for call in (lambda: gpu.w8a8(8, M, K, N), lambda: gpu.w8a8(8, M, K, N, scratch=False), lambda: gpu.w4a16(8, M, K, N, r.choice([64, 128])),
+                     lambda: gpu.linear(8, M, K, N, pkg.F16), lambda: gpu.linear(8, M, K, N, pkg.BF16, q_dtype=pkg.F8E4M3FN),
+                     lambda: gpu.linear(8, M, K, N, pkg.F16, route=0, q_dtype=pkg.I8), lambda: gpu.linear(8, M, K, N, pkg.F16, route=1)):
+            name, _, split = call()
+            assert gpu.lib.mtrt_hip_last_kernel().decode() == name
+            seen.add((name, split is not None and split[0] > 1))
+    with open(pkg.KERNEL_MODULE_PATH, "rb") as f:
+        image = f.read()
+    for name, _ in seen:
+        assert name.encode() + b"\0" in image, name
+    for family in ("w8a8_frag", "dense_frag_f16"):
+        tiles = ["mtrt_gemm_%s_t%s" % (family, t) for t in ("32x128", "64x128", "128x128", "128x256", "128x384", "256x256", "256x384")]
+        assert {(t, False) for t in tiles} | {(t, True) for t in tiles[:4]} <= seen
+
+
+@pytest.mark.parametrize("family,shape,kernel", [
+    ("w8a8", (256, 128, 128), "t32x128"), ("w8a8", (700, 256, 8200), "t128x256"), ("w8a8", (2000, 128, 16416), "t256x384"),
+    ("w8a8", (100, 256, 8209), "t64x128"), ("w8a8", (128, 4096, 1030), "t32x128"), ("w8a8", (2048, 4096, 11008), "t256x384"),
+    ("w4a16", (33, 256, 64), "t128x128"), ("w4a16", (128, 512, 64), "t128x64"), ("w4a16", (256, 4096, 11008), "t128x128"),
+    ("w4a16", (4096, 4096, 11008), "t256x384"), ("w4a16", (600, 256, 8480), "t128x256"), ("w4a16", (2000, 256, 8000), "t256x256"),
+    ("dense", (65, 2048, 33), "t32x128"), ("dense", (700, 1024, 8200), "t128x256"), ("dense", (999, 4096, 11008), "t128x384")])
+def test_the_tile_a_shape_takes(gpu, pkg, family, shape, kernel):
+    name = {"w8a8": lambda: gpu.w8a8(8, *shape), "w4a16": lambda: gpu.w4a16(8, *shape), "dense": lambda: gpu.linear(8, *shape, pkg.F16)}[family]()[0]
+    assert name == {"w8a8": "mtrt_gemm_w8a8_frag_", "w4a16": "mtrt_gemm_w4a16_", "dense": "mtrt_gemm_dense_frag_f16_"}[family] + kernel

@@ -91,9 +91,8 @@ def _frag_small_ok(kernel, M):
     return kernel in _FRAG_SMALL and (M <= 16 or kernel == "mtrt_gemm_w8a8_frag_rows32")
 
 
-# the tile kernels on fragment-order weights (one launch in rounds of tiles, or one workgroup per compute unit walking
-# its share of the columns)
-_FRAG_TILE = {"mtrt_gemm_w8a8_frag", "mtrt_gemm_w8a8_frag_t256x384"}
+# the tile kernels on fragment-order weights; which one a shape takes is the host's estimate (tests/test_dispatch.py)
+_FRAG_TILE = {"mtrt_gemm_w8a8_frag_t" + t for t in ("32x128", "64x128", "128x128", "128x256", "128x384", "256x256", "256x384")}
 
 
 def _run_w8a8_frag(pkg, a, w, a_s, w_s, from_nk=False):
@@ -107,13 +106,12 @@ def _run_w8a8_frag(pkg, a, w, a_s, w_s, from_nk=False):
 @pytest.mark.parametrize("shape", [(256, 128, 128), (512, 512, 256), (300, 256, 200), (1, 128, 1), (37, 384, 129),
                                    (257, 1024, 130), (700, 256, 8200), (2000, 128, 16416)])
 def test_w8a8_weights_in_registers_kernel(pkg, orc, shape):
-    """Full tiles, half-width tiles of a partial last round, ragged M and N, one slice and many."""
+    """Small and large tiles, full and ragged, one slice and many; up to 32 rows the kernels that read the weights once."""
     M, K, N = shape
     a, w, a_s, w_s = _w8a8_inputs(rng(M + K + N), M, K, N)
     print("case: w8a8 fragments", shape, flush=True)
     y, kernel = _run_w8a8_frag(pkg, a, w, a_s, w_s, from_nk=(M % 2 == 1))
-    assert (_frag_small_ok(kernel, M) if M <= 32 else kernel in ("mtrt_gemm_w8a8_frag_rows64", "mtrt_gemm_w8a8_frag") if M <= 64
-            else kernel in _FRAG_TILE), kernel
+    assert (_frag_small_ok(kernel, M) if M <= 32 else kernel in _FRAG_TILE or (M <= 64 and kernel == "mtrt_gemm_w8a8_frag_rows64")), kernel
     orc.set_threads(16)
     ref = orc.gemm_w8a8(a, w, a_s, w_s)
     orc.set_threads(1)
@@ -141,14 +139,14 @@ def test_w8a8_small_m_kernel(pkg, orc, shape):
                                    (128, 512, 4096), (65, 1024, 520), (100, 256, 8209), (128, 4096, 1030), (97, 128, 31), (96, 4096, 11008),
                                    (40, 128, 150000)])
 def test_w8a8_33_to_128_rows_on_fragment_order_weights(pkg, orc, shape):
-    """Two (up to 64 rows) or four activation row tiles against weight fragments that go from memory straight into
-    registers: every row of every tile, ragged M and N (the re-layout holds zeros past N), waves with and without
-    slices; shapes whose estimate favours the tile launch stay there.  Integer sums: bit-exact."""
+    """Tiles of 32 and 64 rows (or, up to 64 rows, the kernel with two activation row tiles per weight fragment) on weight
+    fragments that go from memory straight into registers: every row of every tile, ragged M and N (the re-layout
+    holds zeros past N), waves with and without slices.  Integer sums: bit-exact."""
     M, K, N = shape
     a, w, a_s, w_s = _w8a8_inputs(rng(M + K + N), M, K, N)
     print("case: w8a8 fragments, 33..128 rows", shape, flush=True)
     y, kernel = _run_w8a8_frag(pkg, a, w, a_s, w_s, from_nk=(M % 2 == 1))
-    assert kernel in (("mtrt_gemm_w8a8_frag_rows64" if M <= 64 else "mtrt_gemm_w8a8_frag_rows128"),) + tuple(_FRAG_TILE), kernel
+    assert kernel in _FRAG_TILE or (M <= 64 and kernel == "mtrt_gemm_w8a8_frag_rows64"), kernel
     orc.set_threads(16)
     ref = orc.gemm_w8a8(a, w, a_s, w_s)
     orc.set_threads(1)
@@ -392,10 +390,8 @@ def test_w4a16_small_shapes(pkg, orc, shape):
     B = 128
     a, w, wp, s = _w4a16_inputs(orc, rng(M + K + N), M, K, N, B)
     y, kernel = _run_w4a16(pkg, a, wp, s, K, N, B)
-    # 33..64 rows run as two launches of the small-M kernels; the last one is that of the rows beyond 32
-    last = M - 32 if 32 < M <= 64 else M
-    assert kernel == ("mtrt_gemm_w4a16_strips16" if last <= 16 else "mtrt_gemm_w4a16_skinny" if last <= 32 else
-                      "mtrt_gemm_w4a16_t128x64" if N <= 64 else "mtrt_gemm_w4a16_t128x128")
+    assert kernel == ("mtrt_gemm_w4a16_strips16" if M <= 16 else "mtrt_gemm_w4a16_skinny" if M <= 32 else
+                      "mtrt_gemm_w4a16_t128x64" if M > 64 and N <= 64 else "mtrt_gemm_w4a16_t128x128")
     _check_w4a16(orc, y, a, w, s, K, N, B, orc.gemm_w4a16(a, wp, s, K, N, B))
 
 
@@ -655,12 +651,11 @@ def test_w4a16_big_tile_kernel_ragged_edges(pkg, orc, N, want):
     _check_w4a16(orc, y[rows].contiguous(), a[rows], w, s, K, N, B, ref)
 
 
-@pytest.mark.parametrize("shape,kernel", [((1536, 4096), "t128x256"), ((600, 8480), "t128x256"), ((2048, 4096), "t128x256"), ((1024, 4096), "t128x128"),
+@pytest.mark.parametrize("shape,kernel", [((1536, 4096), "t128x256"), ((600, 8480), "t128x256"), ((2048, 4096), "t128x256"), ((1024, 4096), "t128x256"), ((512, 4096), "t128x128"),
                                           ((768, 11008), "t256x256"), ((1536, 11008), "t256x384"), ((3072, 4096), "t256x256")])
 def test_w4a16_tile_choice_and_results_at_mid_m(pkg, orc, shape, kernel):
-    """The tile is chosen by the estimated number of rounds of one tile per compute unit: 128 x 128 tiles where the
-    larger ones would fill half of the units or spill a few tiles into another round, 128 x 256 and 256 x 384 where
-    they save a round.  Sampled rows against the oracle for each choice (the expected choice is that of 256 compute units)."""
+    """The tile is chosen by the launch's estimated time: 128 x 128 tiles where the larger ones would leave units idle or
+    spill a few tiles into another round, 128 x 256 and 256 x 384 where they save a round.  Sampled rows against the oracle for each choice (the expected choice is that of 256 compute units)."""
     M, N = shape
     K, B = 256, 128
     a, w, wp, s = _w4a16_inputs(orc, rng(M + N), M, K, N, B)

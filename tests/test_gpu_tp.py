@@ -212,7 +212,7 @@ def test_quant_linear_int8_runs_on_the_w8a8_cluster(tp, orc, pkg):
     matrix cores (fragment-order weights prepared once): against a float64 product of the oracle's dequantized
     operands, 1e-3 relative (f16 result)."""
     r = rng(77)
-    for M, K, N, kernels in ((96, 256, 160, ("mtrt_gemm_w8a8_frag_rows128", "mtrt_gemm_w8a8_frag")), (5, 72, 33, ("mtrt_gemm_w8a8_nk_edge",))):
+    for M, K, N, kernels in ((96, 256, 160, ("mtrt_gemm_w8a8_frag_t32x128", "mtrt_gemm_w8a8_frag_t64x128")), (5, 72, 33, ("mtrt_gemm_w8a8_nk_edge",))):
         x = r.standard_normal((M, K)).astype(np.float16)
         w = (r.standard_normal((N, K)) * 0.05).astype(np.float16)
         b = r.standard_normal(N).astype(np.float16)
@@ -338,13 +338,16 @@ def test_dense_linear_against_float64(tp, pkg, dname):
         lin = tp.Linear(K, N, dtype=d)
         lin.weight, lin.bias = tp.Tensor(w, dtype=d), tp.Tensor(b, dtype=d)
         out = lin(tp.Tensor(x, dtype=d)).torch()
-        # operands whose rows are whole 128-byte slices of K run the 256 x 256 tile loop, everything else 128 x 128 tiles
-        # with element-aligned loads; both on the matrix cores
+        # 16-bit weights in fragment order; float32 ones [N, K]: up to 128 rows the kernels that read the weights once, above
+        # the 256 x 256 tile loop.  Rows that are no whole 128-byte slices of K: 128 x 128 tiles with element-aligned loads
         mfma = K % (32 if dname == "float32" else 64) == 0
-        rows = int(np.prod(lead))                          # up to 128 rows read the weights once
-        assert pkg.last_kernel() == ("mtrt_gemm_dense_rows32_" if mfma and rows <= 32 else "mtrt_gemm_dense_rows64_" if mfma and rows <= 64 else
-                                     "mtrt_gemm_dense_rows128_" if mfma and rows <= 128 else
-                                     "mtrt_gemm_dense_mfma_" if mfma else "mtrt_gemm_dense_edge_") + {"float32": "f32", "float16": "f16", "bfloat16": "bf16"}[dname]
+        rows = int(np.prod(lead))
+        kernel, short = pkg.last_kernel(), {"float32": "f32", "float16": "f16", "bfloat16": "bf16"}[dname]
+        if mfma and dname != "float32":
+            assert kernel.startswith("mtrt_gemm_dense_frag_%s_" % short), kernel
+        else:
+            assert kernel == ("mtrt_gemm_dense_rows32_" if mfma and rows <= 32 else "mtrt_gemm_dense_rows64_" if mfma and rows <= 64 else
+                              "mtrt_gemm_dense_rows128_" if mfma and rows <= 128 else "mtrt_gemm_dense_mfma_" if mfma else "mtrt_gemm_dense_edge_") + short
         assert tuple(out.shape) == lead + (N,)
         ref = x.double() @ w.double().T + b.double()
         mag = x.double().abs() @ w.double().abs().T + b.double().abs()
