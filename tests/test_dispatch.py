@@ -4,6 +4,7 @@ whatever reason, runs unsplit, a reduction recorded when there are no more takes
 import pytest
 
 import dispatch
+from test_gpu_gemm_split import DENSE_TILES, W4_TILES, W8_TILES
 
 TICKETS = 512 * 4                                                    # bytes a stream keeps
 
@@ -167,3 +168,12 @@ def test_last_kernel_is_the_symbol_that_was_launched(gpu, pkg):
 def test_the_tile_a_shape_takes(gpu, pkg, family, shape, kernel):
     name = {"w8a8": lambda: gpu.w8a8(8, *shape), "w4a16": lambda: gpu.w4a16(8, *shape), "dense": lambda: gpu.linear(8, *shape, pkg.F16)}[family]()[0]
     assert name == {"w8a8": "mtrt_gemm_w8a8_frag_", "w4a16": "mtrt_gemm_w4a16_", "dense": "mtrt_gemm_dense_frag_f16_"}[family] + kernel
+
+
+@pytest.mark.parametrize("family,tiles", [("w8a8_frag", W8_TILES), ("w4a16", W4_TILES), ("dense_frag_f16", DENSE_TILES)])
+def test_the_shapes_that_test_every_tile_take_it(gpu, pkg, family, tiles):
+    call = {"w8a8_frag": lambda *s: gpu.w8a8(8, *s), "w4a16": lambda *s: gpu.w4a16(8, *s, 64),
+            "dense_frag_f16": lambda *s: gpu.linear(8, *s, pkg.F16)}[family]
+    for shape, tile, split in tiles:
+        name, _, s = call(*shape)
+        assert (name, s is not None and s[0] > 1) == ("mtrt_gemm_%s_%s" % (family, tile), bool(split)), shape

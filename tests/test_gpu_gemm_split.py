@@ -1,5 +1,5 @@
 """GEMMs whose output tiles are shared by several workgroups along K (gemm_frag.hpp), and the tiles and epilogues around
-them, at the sizes where they can go wrong: one slice per part and uneven parts, ragged rows and columns, row lengths of
+them (each by the name of its kernel), at the sizes where they can go wrong: one slice per part and uneven parts, ragged rows and columns, row lengths of
 the output that are no whole vectors, a launch repeated on the same tickets, two streams at once, graph replays."""
 import pytest
 
@@ -56,8 +56,8 @@ def test_some_shape_is_split(pkg):
 @pytest.mark.parametrize("N", [8, 12, 129, 1001, 2048 + 6])
 @pytest.mark.parametrize("M", [65, 300, 1100, 2100])
 def test_w8a8_outputs_inside_a_larger_buffer(pkg, M, N):
-    """Row lengths that are no whole 16-byte vectors and outputs off 16-byte alignment, for tiles of every height: the
-    results are exact and nothing around them is written."""
+    """Row lengths that are no whole 16-byte vectors and outputs off 16-byte alignment: the results are exact and nothing
+    around them is written."""
     import torch
     K = 256
     a, w, a_s, w_s = _inputs(M * N, M, K, N)
@@ -156,7 +156,7 @@ def _w4_inputs(seed, M, K, N, B):
     return a, (nibbles[0::2] | (nibbles[1::2] << 4)).contiguous(), s, (q.half() * s.repeat_interleave(B, 0)).double()
 
 
-# (M, K, N, block): every tile up to 128 rows, split and not, ragged rows and columns, blocks of one slice and of all of K
+# (M, K, N, block): split and not, ragged rows and columns, blocks of one slice and of all of K
 @pytest.mark.parametrize("case", [(33, 4096, 200, 128), (48, 2048, 1000, 64), (64, 8192, 96, 8192), (65, 1152, 129, 192), (100, 12288, 300, 128),
                                   (130, 4096, 4096, 128), (200, 384, 8, 64), (256, 8192, 2051, 256), (300, 4096, 3000, 128), (600, 256, 40, 64),
                                   (700, 4864, 60, 128), (1000, 640, 2000, 128), (1800, 640, 1160, 128), (517, 64, 472, 64), (2000, 2048, 769, 128)])
@@ -190,3 +190,85 @@ def test_some_w4a16_shape_is_split(pkg):
     L = pkg.lib()
     assert L.mtrt_hip_gemm_w4a16_workspace(64, 8192, 96, 128) > 0
     assert L.mtrt_hip_gemm_w4a16_workspace(32, 8192, 96, 128) == 0 and L.mtrt_hip_gemm_w4a16_workspace(64, 8192, 96, 96) == 0
+
+
+# A shape with ragged rows and columns for each tile, with its K whole and shared, as the host's estimate picks them on 256 compute
+# units; `workspace` says whether K is shared.
+W8_TILES = [((41, 256, 9), "t32x128", 0), ((41, 3584, 9), "t32x128", 1), ((2115, 256, 387), "t64x128", 0), ((2849, 11904, 9), "t64x128", 1),
+            ((2143, 256, 913), "t128x128", 0), ((1187, 8704, 793), "t128x128", 1), ((323, 256, 10933), "t128x256", 0),
+            ((1647, 8448, 1253), "t128x256", 1), ((665, 256, 11017), "t128x384", 0), ((2747, 12160, 1423), "t128x384", 1),
+            ((1463, 256, 8109), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
+W4_TILES = [((45, 1024, 9), "t32x128", 0), ((41, 1280, 9), "t32x128", 1), ((133, 640, 10297), "t64x128", 0), ((2791, 4736, 9), "t64x128", 1),
+            ((261, 256, 9955), "t64x256", 0), ((1027, 6592, 963), "t64x256", 1), ((65, 64, 9), "t128x64", 0), ((41, 64, 9), "t128x128", 0),
+            ((2727, 5248, 279), "t128x128", 1), ((139, 64, 8901), "t128x256", 0), ((665, 256, 11017), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
+DENSE_TILES = [((41, 64, 9), "t32x128", 0), ((53, 1792, 9), "t32x128", 1), ((2115, 256, 387), "t64x128", 0), ((2781, 5568, 9), "t64x128", 1),
+               ((2143, 256, 913), "t128x128", 0), ((2727, 5248, 279), "t128x128", 1), ((323, 256, 10933), "t128x256", 0),
+               ((2701, 4544, 657), "t128x256", 1), ((665, 256, 11017), "t128x384", 0), ((143, 9024, 11467), "t128x384", 1),
+               ((1463, 256, 8109), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
+
+
+def _is(pkg, kernel):
+    import torch
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or pkg.last_kernel() == kernel, pkg.last_kernel()
+
+
+@pytest.mark.parametrize("shape,tile,split", W8_TILES)
+def test_every_w8a8_tile(pkg, shape, tile, split):
+    import torch
+    M, K, N = shape
+    a, w, a_s, w_s = _inputs(M + N, M, K, N)
+    wf = pkg.gemm_w8a8_prepack_fragments(w)
+    y = pkg.gemm_w8a8_fragments(a, wf, a_s, w_s, N)
+    _is(pkg, "mtrt_gemm_w8a8_frag_" + tile)
+    assert (pkg.lib().mtrt_hip_gemm_w8a8_fragments_workspace(M, K, N) > 0) == bool(split)
+    assert torch.equal(y, _expect(a, w, a_s, w_s))
+
+
+@pytest.mark.parametrize("shape,tile,split", W4_TILES)
+def test_every_w4a16_tile(pkg, shape, tile, split):
+    """The bound of test_w4a16_tiles_and_splits; with a bias (a Linear with one scale per output) one more rounding."""
+    import importlib
+
+    import torch
+    tp = importlib.import_module(pkg.__name__ + ".tp")
+    M, K, N = shape
+    a, packed, s, wd = _w4_inputs(M + N, M, K, N, 64)
+    y = pkg.gemm_w4a16(a, s, K, N, 64, w_prepacked=pkg.gemm_w4a16_prepack(packed, K, N))
+    _is(pkg, "mtrt_gemm_w4a16_" + tile)
+    assert (pkg.lib().mtrt_hip_gemm_w4a16_workspace(M, K, N, 64) > 0) == bool(split)
+    ref, mass = a.double() @ wd, a.double().abs() @ wd.abs()
+    tol = 2.0 ** -11 * ref.abs() + (1 + 2.0 ** -11) * (K + 1) * 2.0 ** -24 * mass + 2.0 ** -25
+    assert bool(((y.double() - ref).abs() <= tol).all())
+
+    lin = tp.Linear(K, N, dtype=tp.float16, quant_dtype=tp.int4, weight_quant_dim=0)
+    q = torch.randint(-8, 8, (N, K)).half()
+    s_w, b = torch.rand(N).half() * 0.02 + 0.005, torch.randn(N).half()
+    lin.load_state_dict({"weight": tp.Tensor(q * s_w[:, None]), "weight_scale": tp.Tensor(s_w), "bias": tp.Tensor(b)})
+    y = lin(tp.Tensor(a)).torch()
+    assert lin.route() == "w4a16"
+    _is(pkg, "mtrt_gemm_w4a16_%s_bias" % tile)
+    wd = (tp.quantize(lin.weight, lin.weight_scale, tp.int4, 0).torch().to(torch.int8) << 4 >> 4).half() * s_w.cuda()[:, None]
+    core, mass = a.double() @ wd.double().T, a.double().abs() @ wd.double().abs().T
+    ref, u = core + b.cuda().double(), 2.0 ** -11
+    tol = u * core.abs() + (1 + u) * (K + 2) * 2.0 ** -24 * mass + u * ref.abs() * (1 + u) + 2.0 ** -24
+    assert bool(((y.double() - ref).abs() <= tol).all())
+
+
+@pytest.mark.parametrize("dname", ["float16", "bfloat16"])
+@pytest.mark.parametrize("shape,tile,split", DENSE_TILES)
+def test_every_dense_tile(pkg, shape, tile, split, dname):
+    import importlib
+
+    import torch
+    tp = importlib.import_module(pkg.__name__ + ".tp")
+    M, K, N = shape
+    td, u = getattr(torch, dname), {"float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}[dname]
+    g = torch.Generator(device="cuda")
+    g.manual_seed(M + N)
+    x, w, b = (torch.randn(s, generator=g, device="cuda").to(td) for s in ((M, K), (N, K), (N,)))
+    lin = tp.Linear(K, N, dtype=getattr(tp, dname))
+    lin.weight, lin.bias = tp.Tensor(w), tp.Tensor(b)
+    y = lin(tp.Tensor(x)).torch()
+    _is(pkg, "mtrt_gemm_dense_frag_%s_%s" % ({"float16": "f16", "bfloat16": "bf16"}[dname], tile))
+    ref, mass = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    assert bool(((y.double() - ref).abs() <= u * ref.abs() + (1 + u) * (K + 2) * 2.0 ** -24 * mass + 2.0 ** -24).all())
