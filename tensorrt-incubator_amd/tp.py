@@ -480,7 +480,8 @@ class Linear:
         if w.dtype != _torch_dtype(self.dtype):
             return None
         frag = None
-        if w.dtype != torch.float32 and K >= 64:
+        # (a re-layout that is only recorded into a graph has no values before the graph is replayed)
+        if w.dtype != torch.float32 and K >= 64 and not torch.cuda.is_current_stream_capturing():
             frag = self._fragments(w)
             if K % 64 == 0:                            # every call reads the fragments: [N, K] is the owner's own copy or goes
                 del plan["weight"]

@@ -124,6 +124,28 @@ def test_in_place_updates_of_a_subclass_parameter_are_noticed(tp, dname, qname):
     assert bool((lin(x).torch() == 0).all()) and bool((y != 0).any())
 
 
+def test_a_first_call_that_is_recorded(tp):
+    """A plain Linear whose first call is recorded into a graph: eager calls before and after a replay give its result."""
+    import torch
+    lin, g = _module(tp, 10, 256, 200, "float16", None, True, False)
+    lin.weight, lin.bias = tp.Tensor(lin.weight.torch().cuda()), tp.Tensor(lin.bias.torch().cuda())
+    x = tp.Tensor(torch.randn((5, 256), generator=g).half().cuda())
+    xd, wd = _operands(tp, lin, x)
+    ref = xd @ wd.T + lin.bias.torch().double()
+    tol = UNIT["float16"] * ref.abs() + 260 * 2.0 ** -24 * (xd.abs() @ wd.abs().T + 8) + 2.0 ** -24
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = lin(x).torch()
+    assert bool(((lin(x).torch().double() - ref).abs() <= tol).all())
+    for _ in range(3):
+        y.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert bool(((y.double() - ref).abs() <= tol).all())
+        assert torch.equal(lin(x).torch(), y)
+
+
 def test_arguments_of_the_c_call(pkg):
     import ctypes
     L = pkg.lib()
