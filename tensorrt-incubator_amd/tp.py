@@ -489,13 +489,20 @@ class Linear:
         return native.linear_plan(self, 2, q_dtype, K, N, w, frag, None, x_scale)
 
     def _dense_weight(self, plan):
-        """The [N, K] matrix of the dense route, made again where the plan keeps only its fragments."""
+        """The [N, K] matrix of the dense route, for a plan that keeps only its fragments made on the first call that needs it
+        (a bias that is not contiguous does) and kept: not one recorded into a graph, whose values are the replay's."""
         if "weight" in plan:
             return plan["weight"]
         if self.quant_dtype is None:
-            return self.weight.device_data().contiguous()
-        q_weight = quantize(self.weight, self.weight_scale, self.quant_dtype, self.weight_quant_dim)
-        return dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
+            w = self.weight.device_data().contiguous()
+        else:
+            q_weight = quantize(self.weight, self.weight_scale, self.quant_dtype, self.weight_quant_dim)
+            w = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
+        cuda = _torch().cuda
+        if not cuda.is_current_stream_capturing():
+            cuda.current_stream().synchronize()        # the next call may come on another stream
+            plan["weight"] = w
+        return w
 
     # -- forward ---------------------------------------------------------------------------------------
     def forward(self, x):

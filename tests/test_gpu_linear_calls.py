@@ -124,6 +124,35 @@ def test_in_place_updates_of_a_subclass_parameter_are_noticed(tp, dname, qname):
     assert bool((lin(x).torch() == 0).all()) and bool((y != 0).any())
 
 
+@pytest.mark.parametrize("dname,qname,x_scale", [("float16", "int8", False), ("bfloat16", "float8", True), ("float16", None, False)])
+def test_a_strided_bias_prepares_the_weights_once(tp, monkeypatch, dname, qname, x_scale):
+    """A bias that is not contiguous takes the general path, which quantizes the weights on its first call only; the
+    results are those of the same bias laid out densely."""
+    import torch
+    K, N = 192, 72
+    lin, g = _module(tp, 8, K, N, dname, qname, True, x_scale)
+    x = tp.Tensor(torch.randn((5, K), generator=g).to(getattr(torch, dname)).cuda())
+    dense = lin(x).torch()
+    wide = torch.zeros((N, 2), dtype=dense.dtype, device="cuda")
+    wide[:, 0] = lin.bias.device_data()
+    lin.bias = tp.Tensor(wide[:, 0])
+    assert tp._native().tp_linear(lin, x) is NotImplemented
+    first = lin(x).torch()
+    quantize, of_weights = tp.quantize, []
+
+    def counted(t, *rest):
+        if t is lin.weight:
+            of_weights.append(t)
+        return quantize(t, *rest)
+    monkeypatch.setattr(tp, "quantize", counted)
+    assert torch.equal(lin(x).torch(), first) and not of_weights
+    assert torch.allclose(first.float(), dense.float(), rtol=4 * UNIT[dname], atol=1e-4)
+    lin.weight.device_data().zero_()                                 # a kept matrix goes with the plan
+    assert torch.equal(lin(x).torch(), lin.bias.torch().expand(5, N)) and bool(of_weights) == (qname is not None)
+    del of_weights[:]
+    assert torch.equal(lin(x).torch(), lin.bias.torch().expand(5, N)) and not of_weights
+
+
 def test_a_first_call_that_is_recorded(tp):
     """A plain Linear whose first call is recorded into a graph: eager calls before and after a replay give its result."""
     import torch
