@@ -482,11 +482,27 @@ class Linear:
         frag = None
         # (a re-layout that is only recorded into a graph has no values before the graph is replayed)
         if w.dtype != torch.float32 and K >= 64 and not torch.cuda.is_current_stream_capturing():
-            frag = self._fragments(w)
-            if K % 64 == 0:                            # every call reads the fragments: [N, K] is the owner's own copy or goes
+            # Every call reads the fragments where K is whole slices or the activations are quantized; [N, K] is then the
+            # parameter itself or goes.  Elsewhere small products read [N, K].
+            only_fragments = K % 64 == 0 or q_dtype is not None
+            if (only_fragments and self.quant_dtype is not None) or self._room_for(w):
+                try:
+                    frag = self._fragments(w)
+                except torch.OutOfMemoryError:         # the [N, K] kernels serve every shape
+                    pass
+            if frag is not None and only_fragments:
                 del plan["weight"]
                 w = None
         return native.linear_plan(self, 2, q_dtype, K, N, w, frag, None, x_scale)
+
+    @staticmethod
+    def _room_for(w):
+        """Whether a second copy of the weights `w` leaves a quarter of the device's memory free: 16-bit weights that stay
+        beside their fragments take twice the memory, and a model that fills the device must still run."""
+        cuda = _torch().cuda
+        free, total = cuda.mem_get_info(w.device)
+        free += cuda.memory_reserved(w.device) - cuda.memory_allocated(w.device)
+        return free - w.numel() * w.element_size() > total // 4
 
     def _dense_weight(self, plan):
         """The [N, K] matrix of the dense route, for a plan that keeps only its fragments made on the first call that needs it

@@ -153,6 +153,30 @@ def test_a_strided_bias_prepares_the_weights_once(tp, monkeypatch, dname, qname,
     assert torch.equal(lin(x).torch(), lin.bias.torch().expand(5, N)) and not of_weights
 
 
+@pytest.mark.parametrize("why", ["little memory", "none"])
+def test_weights_that_do_not_fit_twice(tp, pkg, monkeypatch, why):
+    """Without room for the fragments a plain 16-bit Linear runs on its parameter as it is, with the same result up to the
+    order of its sums."""
+    import torch
+    lin, g = _module(tp, 9, 4096, 200, "float16", None, True, False)
+    x = tp.Tensor(torch.randn((5, 4096), generator=g).half().cuda())
+    y = lin(x).torch()
+    assert pkg.last_kernel().startswith("mtrt_gemm_dense_frag_f16_")
+    total = torch.cuda.mem_get_info()[1]
+    if why == "none":
+        def full(w):
+            raise torch.OutOfMemoryError("no room")
+        monkeypatch.setattr(tp.Linear, "_fragments", staticmethod(full))
+    else:
+        monkeypatch.setattr(torch.cuda, "mem_get_info", lambda *a: (total // 8, total))
+    lin.invalidate()
+    again = lin(x).torch()
+    assert pkg.last_kernel() == "mtrt_gemm_dense_rows32_f16"
+    xd, wd = _operands(tp, lin, x)
+    tol = 2 * (UNIT["float16"] * y.double().abs() + 4100 * 2.0 ** -24 * (xd.abs() @ wd.abs().T) + 2.0 ** -24)
+    assert bool(((again.double() - y.double()).abs() <= tol).all())
+
+
 def test_a_first_call_that_is_recorded(tp):
     """A plain Linear whose first call is recorded into a graph: eager calls before and after a replay give its result."""
     import torch
