@@ -83,9 +83,11 @@ def build_frontend():
     (its libraries loaded) before the extension is, so no path to them is recorded."""
     import sysconfig
     from torch.utils.cpp_extension import COMMON_HIP_FLAGS, include_paths, library_paths
-    flags = ["-I" + p for p in include_paths() + [sysconfig.get_paths()["include"], os.path.join(ROCM, "include"), os.path.join(ROOT, "include")]]
+    flags = ["-I" + os.path.join(ROOT, "include")]
+    for p in include_paths() + [sysconfig.get_paths()["include"], os.path.join(ROCM, "include")]:
+        flags += ["-isystem", p]                       # their warnings are theirs
     flags += [f for f in COMMON_HIP_FLAGS if f.startswith("-D")] + ["-L" + p for p in library_paths()]
-    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wno-unused-function", "-w",
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden", "-Wall", "-Wextra",
           os.path.join(CSRC, "frontend", "frontend.cpp")] + flags +
          ["-L" + LIB, "-lmtrt_hip", "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python", "-Wl,-rpath,$ORIGIN",
           "-o", os.path.join(LIB, "mtrt_frontend.so")])

@@ -547,8 +547,8 @@ PyObject *f_softmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
 }
 
 // gemm_w8a8(a, w_nk, a_scale, w_scale, out) and gemm_w8a8_fragments(a, w_frag, a_scale, w_scale, N, out) -> y
-PyObject *w8a8(PyObject *const *a, const at::Tensor &x, const at::Tensor &w, const at::Tensor &as, const at::Tensor &ws, int64_t N,
-               PyObject *given, bool fragments) {
+PyObject *w8a8(const at::Tensor &x, const at::Tensor &w, const at::Tensor &as, const at::Tensor &ws, int64_t N, PyObject *given,
+               bool fragments) {
   const at::Tensor *out;
   if (!optional_tensor(given, &out))
     return nullptr;
@@ -577,7 +577,7 @@ PyObject *f_gemm_w8a8(PyObject *, PyObject *const *a, Py_ssize_t n) {
       w->scalar_type() != at::ScalarType::Char || w->dim() != 2 || as->scalar_type() != at::ScalarType::Float ||
       ws->scalar_type() != at::ScalarType::Float)
     return fail("a and w_nk must be contiguous int8 matrices on the GPU, the scales float32"), nullptr;
-  return w8a8(a, *x, *w, *as, *ws, w->size(0), a[4], false);
+  return w8a8(*x, *w, *as, *ws, w->size(0), a[4], false);
   FRONTEND_CATCH
 }
 PyObject *f_gemm_w8a8_fragments(PyObject *, PyObject *const *a, Py_ssize_t n) {
@@ -590,7 +590,7 @@ PyObject *f_gemm_w8a8_fragments(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!dense_on_gpu(*x) || x->scalar_type() != at::ScalarType::Char || x->dim() != 2 || w->scalar_type() != at::ScalarType::Char ||
       as->scalar_type() != at::ScalarType::Float || ws->scalar_type() != at::ScalarType::Float)
     return fail("a must be a contiguous int8 matrix on the GPU, w_frag int8, the scales float32"), nullptr;
-  return w8a8(a, *x, *w, *as, *ws, N, a[5], true);
+  return w8a8(*x, *w, *as, *ws, N, a[5], true);
   FRONTEND_CATCH
 }
 
