@@ -1,7 +1,9 @@
 // The activation side of a Linear, in one pass in front of its GEMM: rows of x [M, K] into rows of Kp elements, Kp = K rounded
-// up to the GEMM's K slices, the padding zero (so that a K that is no whole number of slices runs on the same kernels: the
-// padded products are exact zeros), and, where the module quantizes its input, the codes (mtrt_act_codes_*) or the
-// dequantized codes (mtrt_act_fake_*) instead of the values.  Same arithmetic, bit for bit, as mtrt_hip_quantize followed
+// up to the GEMM's K slices, and, where the module quantizes its input, the codes (mtrt_act_codes_*) or the dequantized
+// codes (mtrt_act_fake_*) instead of the values.  The padding is zero before it is quantized, so that a K that is no whole
+// number of slices runs on the same kernels: its products are exact zeros, for the padded weights are zero and the padding
+// is finite wherever x's own zeros are (with a scale of zero it has the largest code, as 0 / 0 is clamped to it, and that times
+// the scale is zero again).  Same arithmetic, bit for bit, as mtrt_hip_quantize followed
 // by mtrt_hip_dequantize with a per-tensor scale, in one launch that reads x once and writes the result once (as two they
 // move 3 bytes per element more for 16-bit types; bf16 [999, 4096] to f8 and back 10.6 us as two launches).
 //
@@ -61,7 +63,7 @@ __device__ __forceinline__ void act_rows(const typename X::storage* __restrict__
 #pragma unroll
         for (int i = 0; i < G / 4; ++i) {
           w[i] = pack4<Q>(&v[4 * i], 0);
-          if (MODE == 2) unpack4<Q>(w[i], &v[4 * i]);  // (the code of a padding zero is zero for every target)
+          if (MODE == 2) unpack4<Q>(w[i], &v[4 * i]);
         }
         if (MODE == 1) {
 #pragma unroll

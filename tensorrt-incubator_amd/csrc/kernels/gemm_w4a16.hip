@@ -1103,12 +1103,12 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
 // (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M <= 16, K % 128 == 0, N, block % 128 == 0)
 // grid = min(compute units, ceil(N / 16)), block = 256: workgroup g owns tiles / grid consecutive 16-column tiles (the first
 // tiles % grid workgroups one more), three at a time.
-// Four waves, one per SIMD.  Measured on M = 16, N = 11008, K = 4096 (rocprofv3 kernel durations): 2 / 4 / 8 waves take
-// 12.7 / 9.6 / 10.7 us; more than one workgroup per compute unit (grids of 344, 512, 688) 11.5-12.6 us.  In-kernel
-// timestamps of the four-wave form: 1.3 us until the loads are issued, first slice landed at 3.9 us, K loop done at
-// 10.4 us (1600 cycles per slice against some 800 of issue for 175 dequantisation instructions and 12 MFMAs), so what
-// is left is the dequantisation on one wave per SIMD and the 4 us before the first data; with eight waves the loop
-// shortens to 4.9 us but the first data arrives later by as much.
+// Four waves, one per SIMD, each with eight of the 32 blocks of 128 k at K = 4096.  Measured on M = 16, N = 11008, K = 4096
+// (rocprofv3 kernel durations, an earlier form of the loop): 2 / 4 / 8 waves take 12.7 / 9.6 / 10.7 us; more than one
+// workgroup per compute unit (grids of 344, 512, 688) 11.5-12.6 us.  In-kernel timestamps of this form, median wave, us from
+// the launch's first wave: entered 0.3, first slice asked for 1.3, landed 2.7, K loop done 7.4 (0.69 per slice against some
+// 0.35 of issue for 175 dequantisation instructions and 12 MFMAs), results stored 8.0; the slowest wave 0.9 later.
+// So what is left is the microsecond of set-up (addresses and divisions) and the loop; M = 1 is 0.5 us shorter.
 constexpr int kStripWaves = 4;
 extern "C" __global__ void __launch_bounds__(64 * kStripWaves) mtrt_gemm_w4a16_strips16(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
