@@ -501,8 +501,9 @@ class Linear:
         beside their fragments take twice the memory, and a model that fills the device must still run."""
         cuda = _torch().cuda
         free, total = cuda.mem_get_info(w.device)
-        free += cuda.memory_reserved(w.device) - cuda.memory_allocated(w.device)
-        return free - w.numel() * w.element_size() > total // 4
+        least = total // 4 + w.numel() * w.element_size()
+        # (what torch's allocator holds unused is free as well; asking it costs more than asking the device)
+        return free > least or free + cuda.memory_reserved(w.device) - cuda.memory_allocated(w.device) > least
 
     def _dense_weight(self, plan):
         """The [N, K] matrix of the dense route, for a plan that keeps only its fragments made on the first call that needs it
