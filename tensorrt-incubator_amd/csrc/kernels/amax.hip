@@ -33,6 +33,18 @@ constexpr int kAmaxUnroll = 4;     // 128-bit loads in flight per lane per step
 constexpr uint32_t kAmaxFanIn = 32;     // first-level groups of the cross-workgroup arrival tree
 constexpr uint32_t kAmaxLineWords = 32; // one 128-byte line per (ticket, max) pair
 
+// The pass that quantizes by this maximum reads the tensor again, beginning at its end (last_first_piece in common.hpp), so the
+// last 32 MiB, what the eight L2s hold, are read by ordinary loads, which leaves them there; what lies in front goes past
+// the caches.  amax and the fused pass behind it, bf16 -> f8, us, with contiguous chunks per workgroup and the fused pass
+// forwards; in pieces and from the end with nothing left in the L2s; with 16, 24, 32 and 96 MiB left:
+//   33 MB   24.8   25.0   22.8   21.8   20.3   20.7
+//   67 MB   41.5   40.2   38.7   38.4   38.6   37.3
+//   134 MB  73.8   73.9   71.6   70.7   70.8   72.6
+// (amax, NVFP4 and back of 67 MB: 43.5, 41.4, 40.2, 39.1, 38.0, 37.7; f32 -> i8 of 67 MB 41.5, 39.7, 38.9, 36.4, 36.0, 33.0).
+// It turns where both passes together fill the Infinity Cache: 200 MiB 109.4 and (32 left) 108.0, 224 MiB 121.3 and 122.9,
+// 256 MiB 136.6 and 144.9.  Hence kReadTwiceBelow, above which all loads go past the caches and the next pass runs forwards.
+constexpr int64_t kAmaxKept = (int64_t(32) << 20) / 16;   // in vectors
+
 template <typename X> struct AbsBits;
 template <> struct AbsBits<F32> {  // returns max over the 4 floats, as f32 bit pattern
   static __device__ __forceinline__ uint32_t of(u32x4 t) {
@@ -101,31 +113,47 @@ __device__ __forceinline__ void amax_body(const typename X::storage* __restrict_
   using A = AbsBits<X>;
   // Elements before the first 16-byte boundary ("head") and after the last full
   // vector ("tail") are taken one per lane by workgroup 0; everything between is
-  // streamed as 128-bit vectors, each workgroup owning one contiguous chunk.
+  // streamed as 128-bit vectors, in pieces of 32 KiB that the workgroups take in turn.
   constexpr int kElemBytes = 16 / A::kPerVec;
-  constexpr int64_t kStep = int64_t(kAmaxThreads) * kAmaxUnroll;
+  constexpr int64_t kStep = int64_t(kAmaxThreads) * kAmaxUnroll, kPiece = 2 * kStep;
   int64_t head = int64_t((16u - uint32_t(reinterpret_cast<uintptr_t>(x) & 15u)) & 15u) / kElemBytes;
   head = head < n ? head : n;
   const int64_t nvec = (n - head) / A::kPerVec;
   const u32x4* __restrict__ xv = reinterpret_cast<const u32x4*>(x + head);
-  // vectors per workgroup, rounded up; tensors below 2^32 vectors (64 GiB) take the 32-bit division (the 64-bit one is
-  // a hundred scalar instructions in front of the first load)
-  const uint64_t spread = uint64_t(nvec) + gridDim.x - 1;
-  const int64_t share = (spread >> 32) == 0 ? int64_t(uint32_t(spread) / gridDim.x) : int64_t(spread / gridDim.x);
-  const int64_t per = (share + kStep - 1) / kStep * kStep;                                  // chunk, whole steps
-  const int64_t c0 = int64_t(blockIdx.x) * per;
-  const int64_t c1 = c0 + per < nvec ? c0 + per : nvec;
+  const int64_t next = int64_t(gridDim.x) * kPiece;
+  const int64_t past = nvec * 16 >= kReadTwiceBelow ? nvec : nvec - kAmaxKept;   // up to here past the caches
   uint32_t m = 0;
-  int64_t i = c0 + threadIdx.x;
-  // kAmaxUnroll independent 128-bit loads per lane per trip
-  for (; i + (kAmaxUnroll - 1) * kAmaxThreads < c1; i += kStep) {
-    u32x4 t[kAmaxUnroll];
-#pragma unroll
-    for (int u = 0; u < kAmaxUnroll; ++u) t[u] = __builtin_nontemporal_load(xv + i + u * kAmaxThreads);
+  int64_t p = int64_t(blockIdx.x) * kPiece;
+  u32x4 t[kAmaxUnroll];
+  const auto fold = [&] {
 #pragma unroll
     for (int u = 0; u < kAmaxUnroll; ++u) { const uint32_t a = A::of(t[u]); m = m > a ? m : a; }
+  };
+  // (two loops: in the branches of one, the loads would be merged into ordinary ones)
+  for (; p < past && p + kPiece <= nvec; p += next) {
+#pragma unroll 1
+    for (int64_t h = 0; h < kPiece; h += kStep) {
+#pragma unroll
+      for (int u = 0; u < kAmaxUnroll; ++u) t[u] = __builtin_nontemporal_load(xv + p + h + u * kAmaxThreads + threadIdx.x);
+      fold();
+    }
   }
-  for (; i < c1; i += kAmaxThreads) { const uint32_t a = A::of(__builtin_nontemporal_load(xv + i)); m = m > a ? m : a; }
+  for (; p + kPiece <= nvec; p += next) {
+#pragma unroll 1
+    for (int64_t h = 0; h < kPiece; h += kStep) {
+#pragma unroll
+      for (int u = 0; u < kAmaxUnroll; ++u) t[u] = xv[p + h + u * kAmaxThreads + threadIdx.x];
+      fold();
+    }
+  }
+  for (int64_t h = p; h < nvec && h < p + kPiece; h += kStep) {   // the last piece: lanes past its end repeat its last vector
+#pragma unroll
+    for (int u = 0; u < kAmaxUnroll; ++u) {
+      const int64_t v = h + u * kAmaxThreads + threadIdx.x;
+      t[u] = xv[v < nvec ? v : nvec - 1];
+    }
+    fold();
+  }
   if (blockIdx.x == 0 && threadIdx.x < 2 * A::kPerVec) {
     const int64_t tail0 = head + nvec * A::kPerVec;
     const int64_t e = threadIdx.x < A::kPerVec ? int64_t(threadIdx.x) : tail0 + (threadIdx.x - A::kPerVec);

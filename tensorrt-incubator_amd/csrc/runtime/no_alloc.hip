@@ -113,10 +113,10 @@ extern "C" int32_t mtrt_hip_amax_no_alloc(mtrt_stream_t stream, const void *x, i
       return set_error(MTRT_DRIVER_ERROR, "launching the clear kernel: %s", hipGetErrorString(e));
   }
 
-  // launch shape of mtrt_hip_amax: at most two workgroups per compute unit, 4 x 128-bit loads per lane and trip
+  // launch shape of mtrt_hip_amax: at most two workgroups per compute unit, 8 x 128-bit loads per lane and trip
   const int per_vec = dtype == MTRT_F32 ? 4 : 8;
   const int64_t nvec = n / per_vec;
-  int64_t grid = (nvec + 256 * 4 - 1) / (256 * 4);
+  int64_t grid = (nvec + 256 * 8 - 1) / (256 * 8);
   if (grid > int64_t(d.num_cus) * 2) grid = int64_t(d.num_cus) * 2;
   if (grid < 1) grid = 1;
   const void *x_arg = x;
