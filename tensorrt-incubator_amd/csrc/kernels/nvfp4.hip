@@ -29,7 +29,9 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float f2 __attribute__((ext_vector_type(2)));
 
 constexpr int kThreads = 256;
-constexpr int kTrips = 8;
+// vectors per lane.  Codes and scales are a fifth of what a dequantize moves, so it needs little in flight: 2, 4 and 8 vectors take
+// bf16 of 134 MB 25.0, 25.4 and 25.7 us, f32 of 268 MB 42.9, 43.8 and 46.6
+constexpr int kTrips = 8, kDqTrips = 2;
 
 // the reference's table on one f16 bit pattern (exact, slow): used for blocks that contain NaN
 __device__ __forceinline__ uint32_t f16_bits_to_f4_exact(uint32_t h) {
@@ -203,19 +205,19 @@ __device__ __forceinline__ void dequantize_body(const uint8_t* __restrict__ q, c
   constexpr int G = FloatGroup<Y>::G;
   constexpr int LPB = 16 / G;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t span = (int64_t(blockIdx.x) * (kThreads / 64) + wave) * (kTrips * 64);
+  const int64_t span = (int64_t(blockIdx.x) * (kThreads / 64) + wave) * (kDqTrips * 64);
   if (span >= nvec) return;
   const float s_dec = *tensor_amax / 2688.0f;
-  uint32_t codes[kTrips], s8[kTrips];
+  uint32_t codes[kDqTrips], s8[kDqTrips];
 #pragma unroll
-  for (int j = 0; j < kTrips; ++j) {
+  for (int j = 0; j < kDqTrips; ++j) {
     int64_t v = span + j * 64 + lane;
     v = v < nvec ? v : nvec - 1;
     codes[j] = G == 4 ? uint32_t(*reinterpret_cast<const uint16_t*>(q + v * 2)) : *reinterpret_cast<const uint32_t*>(q + v * 4);
     s8[j] = scales[v / LPB];
   }
 #pragma unroll
-  for (int j = 0; j < kTrips; ++j) {
+  for (int j = 0; j < kDqTrips; ++j) {
     const int64_t v = span + j * 64 + lane;
     const float u = f8_to_f32<0>(s8[j]) * s_dec;
     float out[G];
@@ -234,58 +236,74 @@ __device__ __forceinline__ void dequantize_body(const uint8_t* __restrict__ q, c
 }
 
 // ---- blocks of 16 along the SECOND-TO-LAST axis ([d0, d1] view, d0 % 16 == 0) ----------------------
-// A lane owns G neighbouring columns of one block row: 16 vectors, one per row, a row's 64 vectors
-// of a wave being 1 KiB of contiguous memory.  The block amax is a maximum down the lane's own
-// registers, one chain per column.  Per row a wave stores 64 x G/2 bytes of codes and per block row
-// 64 x G scale bytes, each contiguous.
-// (x, q_packed, scales, tensor_amax, d0, d1) ; d1 % G == 0 ; one lane per (block row, column group)
+// A unit is G neighbouring columns of one block row.  The lanes l, l + 16, l + 32 and l + 48 of a wave share it, four of its
+// sixteen rows each: the block amax is a maximum down the lane's own registers and two exchanges, and every lane computes the
+// scales of a quarter of the columns.  Per row a wave reads 256 bytes and its workgroup 1 KiB of contiguous memory.
+// Bound by memory where enough waves are in flight, by the length of a lane's work where few are.  With all sixteen rows in
+// one lane (158 registers, three waves per SIMD), eight in each of two, and four in each of four (54 registers), us:
+//   bf16 [4096, 8192] 29.8, 20.4, 16.5   [16384, 4096] 42.5, 32.4, 28.9   [7136, 528] 14.5, 8.4, 5.7   [16384, 64] 9.3, 5.8, 4.1
+//   f32  [4096, 8192] 30.8, 26.9, 27.3   [16384, 4096] 55.0, 51.2, 52.3   [7136, 528] 9.6, 6.6, 5.4    [16384, 64] 6.5, 4.4, 3.4
+// (x, q_packed, scales, tensor_amax, d0, d1) ; d1 % G == 0 ; four lanes per unit
 template <typename X>
 __device__ __forceinline__ void quantize_cols_body(const typename X::storage* __restrict__ x, uint8_t* __restrict__ q,
                                                    uint8_t* __restrict__ scales, const float* __restrict__ tensor_amax,
                                                    int64_t d0, int64_t d1) {
   constexpr int G = FloatGroup<X>::G;
+  constexpr int R = 4;                                 // rows per lane
   __shared__ float inverse_scale[256];
-  const int64_t groups = d1 / G, units = (d0 / 16) * groups;
-  const int64_t u = int64_t(blockIdx.x) * kThreads + threadIdx.x;
+  const uint32_t groups = uint32_t(d1 / G), units = uint32_t((d0 / 16) * groups);   // below 2^32 for anything that fits in memory
+  const uint32_t part = (threadIdx.x >> 4) & 3;
+  uint32_t u = blockIdx.x * (kThreads / 4) + (threadIdx.x >> 6) * 16 + (threadIdx.x & 15);
+  u = u < units ? u : units - 1;                       // past the end: the last unit once more, which stores the same bytes
+  const uint32_t rb = u / groups;
+  const int64_t c0 = int64_t(u - rb * groups) * G, row0 = int64_t(rb) * 16 + part * R;
+  const typename X::storage* xp = x + row0 * d1 + c0;
+  u32x4 t[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) t[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xp + r * d1));
   const float s_enc = 2688.0f / *tensor_amax;
   fill_inverse_scales(inverse_scale, s_enc);
-  if (u >= units) return;
-  const int64_t rb = u / groups, c0 = (u - rb * groups) * G;
-  const typename X::storage* xp = x + rb * 16 * d1 + c0;
-  u32x4 t[16];
-#pragma unroll
-  for (int r = 0; r < 16; ++r) t[r] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(xp + r * d1));
   float amax[G];
 #pragma unroll
   for (int k = 0; k < G; ++k) amax[k] = 0.0f;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r = 0; r < R; ++r) {
     float v[G];
     FloatGroup<X>::unpack(t[r], v);
 #pragma unroll
     for (int k = 0; k < G; ++k) amax[k] = fmaxf(amax[k], fabsf(v[k]));
   }
+  // Two swaps of lane groups leave each lane with the block maxima of a quarter of the columns (16-lane group j: columns
+  // j G/4 ...); it computes their scales, and the same swaps hand those to all four lanes.
+  uint32_t m[G / 2], s8[G / 4];
   float s_enc_x[G];
-  uint32_t s8[G];
 #pragma unroll
-  for (int k = 0; k < G; ++k) {
-    const float s_dec_x = divide_by_six(amax[k]);
+  for (int k = 0; k < G / 2; ++k) {
+    const auto t2 = __builtin_amdgcn_permlane32_swap(f32_to_bits(amax[k]), f32_to_bits(amax[k + G / 2]), false, false);
+    m[k] = f32_to_bits(fmaxf(bits_to_f32(t2[0]), bits_to_f32(t2[1])));
+  }
+#pragma unroll
+  for (int k = 0; k < G / 4; ++k) {
+    const auto t2 = __builtin_amdgcn_permlane16_swap(m[k], m[k + G / 4], false, false);
+    const float s_dec_x = divide_by_six(fmaxf(bits_to_f32(t2[0]), bits_to_f32(t2[1])));
     uint32_t b = f32x2_to_f8_ieee(s_dec_x * s_enc, 0.0f) & 0xFFu;
     b = (b & 0x7Fu) == 0x7Fu ? 0x7Fu : b;
     s8[k] = b;
-    s_enc_x[k] = inverse_scale[b];                     // = s_enc / f32(b), the same IEEE quotient
-  }
-  uint8_t* sp = scales + rb * d1 + c0;
-  if (G == 4) {
-    *reinterpret_cast<uint32_t*>(sp) = s8[0] | (s8[1] << 8) | (s8[2] << 16) | (s8[3] << 24);
-  } else {
-    u32x2 w = {s8[0] | (s8[1] << 8) | (s8[2] << 16) | (s8[3] << 24),
-               s8[4 % G] | (s8[5 % G] << 8) | (s8[6 % G] << 16) | (s8[7 % G] << 24)};
-    *reinterpret_cast<u32x2*>(sp) = w;
-  }
-  uint8_t* qp = q + (rb * 16 * d1 + c0) / 2;
+    const uint32_t inverse = f32_to_bits(inverse_scale[b]);   // = s_enc / f32(b), the same IEEE quotient
+    const auto pair = __builtin_amdgcn_permlane16_swap(inverse, inverse, false, false);
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+    for (int p = 0; p < 2; ++p) {
+      const auto halves = __builtin_amdgcn_permlane32_swap(pair[p], pair[p], false, false);
+      s_enc_x[k + p * (G / 4)] = bits_to_f32(halves[0]);
+      s_enc_x[k + p * (G / 4) + G / 2] = bits_to_f32(halves[1]);
+    }
+  }
+  uint8_t* sp = scales + rb * d1 + c0 + part * (G / 4);
+  if (G == 4) *sp = uint8_t(s8[0]);
+  else *reinterpret_cast<uint16_t*>(sp) = uint16_t(s8[0] | (s8[1 % (G / 4)] << 8));
+  uint8_t* qp = q + (row0 * d1 + c0) / 2;
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
     float v[G], w[G];
     FloatGroup<X>::unpack(t[r], v);
 #pragma unroll
@@ -311,11 +329,11 @@ __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__
                                                      const float* __restrict__ tensor_amax,
                                                      typename Y::storage* __restrict__ y, int64_t d0, int64_t d1) {
   constexpr int G = FloatGroup<Y>::G;
-  const int64_t groups = d1 / G, nvec = d0 * groups;
+  const int64_t groups = d1 / G, nvec = d0 * groups;   // groups and nvec are below 2^32 for anything that fits in memory
   const float s_dec = *tensor_amax / 2688.0f;
   const int64_t stride = int64_t(gridDim.x) * kThreads;
   for (int64_t v = int64_t(blockIdx.x) * kThreads + threadIdx.x; v < nvec; v += stride) {
-    const int64_t r = v / groups, c0 = (v - r * groups) * G;
+    const int64_t r = uint32_t(v) / uint32_t(groups), c0 = (v - r * groups) * G;
     const uint32_t codes = G == 4 ? uint32_t(*reinterpret_cast<const uint16_t*>(q + v * 2)) : *reinterpret_cast<const uint32_t*>(q + v * 4);
     const uint8_t* sp = scales + (r / 16) * d1 + c0;
     uint32_t sw[2];
@@ -342,7 +360,7 @@ __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__
 }  // namespace nvfp4_cluster
 
 // mtrt_nvfp4_q_<t>(x, q_packed, scales, tensor_amax, nvec) ; mtrt_nvfp4_dq_<t>(q_packed, scales, tensor_amax, y, nvec)
-// grid = ceil(nvec / (4 waves * 8 trips * 64)), block = 256; x / y and q_packed 16-byte aligned.
+// grid = ceil(nvec / (4 waves * 64 * 8 vectors)) and, to dequantize, of 2 vectors; block = 256; x / y and q_packed 16-byte aligned.
 #define MTRT_NVFP4_KERNELS(XN, XT)                                                                                      \
   extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_q_##XN(                               \
       const XT::storage* x, uint8_t* q, uint8_t* scales, const float* tensor_amax, int64_t nvec) {                      \
@@ -353,7 +371,7 @@ __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__
     nvfp4_cluster::dequantize_body<XT>(q, scales, tensor_amax, y, nvec);                                                \
   }
 // Blocks along the second-to-last axis: mtrt_nvfp4_qc_<t>(x, q_packed, scales, tensor_amax, d0, d1) with
-// grid = ceil((d0 / 16) * (d1 / G) / 256); mtrt_nvfp4_dqc_<t>(q_packed, scales, tensor_amax, y, d0, d1).
+// grid = ceil((d0 / 16) * (d1 / G) / 64); mtrt_nvfp4_dqc_<t>(q_packed, scales, tensor_amax, y, d0, d1).
 // d1 % G == 0 (G = 4 for f32, 8 for f16 / bf16), x / y rows 16-byte aligned, scales 4- (G = 4) or 8-byte aligned.
 #define MTRT_NVFP4_COL_KERNELS(XN, XT)                                                                                  \
   extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_qc_##XN(                              \

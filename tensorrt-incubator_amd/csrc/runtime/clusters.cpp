@@ -822,7 +822,7 @@ int32_t nvfp4_dispatch(bool quantize, hipStream_t stream, const void *xy, int32_
     if (d1 % group != 0)
       return set_error(MTRT_INVALID_ARGUMENT, "blocks along the second-to-last axis need the last extent %% %d == 0, got %lld",
                        group, (long long)d1);
-    const int64_t units = quantize ? (d0 / 16) * (d1 / group) : d0 * (d1 / group);
+    const int64_t units = quantize ? 4 * (d0 / 16) * (d1 / group) : d0 * (d1 / group);   // lanes
     if ((units + kBlock - 1) / kBlock > int64_t(kMaxGrid) * 1024)
       return set_error(MTRT_INVALID_ARGUMENT, "tensor of %lld elements is too large", (long long)n);
     if (quantize) {
@@ -834,7 +834,8 @@ int32_t nvfp4_dispatch(bool quantize, hipStream_t stream, const void *xy, int32_
     return launch(st, KernelName("mtrt_nvfp4_dqc_") + xn, uint32_t(blocks), kBlock, stream, args);
   }
   int64_t nvec = n / group;
-  const int64_t blocks = (nvec + 4 * 8 * 64 - 1) / (4 * 8 * 64);   // 4 waves x 8 trips x 64 lanes per workgroup
+  const int64_t per_block = 4 * 64 * (quantize ? 8 : 2);   // 4 waves x 64 lanes x kTrips or kDqTrips vectors
+  const int64_t blocks = (nvec + per_block - 1) / per_block;
   if (blocks > int64_t(kMaxGrid) * 1024)
     return set_error(MTRT_INVALID_ARGUMENT, "tensor of %lld elements is too large", (long long)n);
   if (quantize) {
