@@ -113,40 +113,42 @@ __device__ __forceinline__ void amax_body(const typename X::storage* __restrict_
   using A = AbsBits<X>;
   // Elements before the first 16-byte boundary ("head") and after the last full
   // vector ("tail") are taken one per lane by workgroup 0; everything between is
-  // streamed as 128-bit vectors, in pieces of 32 KiB that the workgroups take in turn.
+  // streamed as 128-bit vectors, in pieces of 32 KiB that the workgroups take in turn (16 KiB beyond kReadTwiceBelow:
+  // f32 of 256 MiB 41.8 and 41.1 us, 320 MiB 51.5 and 50.4).
   constexpr int kElemBytes = 16 / A::kPerVec;
-  constexpr int64_t kStep = int64_t(kAmaxThreads) * kAmaxUnroll, kPiece = 2 * kStep;
+  constexpr int64_t kStep = int64_t(kAmaxThreads) * kAmaxUnroll;
   int64_t head = int64_t((16u - uint32_t(reinterpret_cast<uintptr_t>(x) & 15u)) & 15u) / kElemBytes;
   head = head < n ? head : n;
   const int64_t nvec = (n - head) / A::kPerVec;
   const u32x4* __restrict__ xv = reinterpret_cast<const u32x4*>(x + head);
-  const int64_t next = int64_t(gridDim.x) * kPiece;
-  const int64_t past = nvec * 16 >= kReadTwiceBelow ? nvec : nvec - kAmaxKept;   // up to here past the caches
+  const bool large = nvec * 16 >= kReadTwiceBelow;
+  const int64_t piece = large ? kStep : 2 * kStep, next = int64_t(gridDim.x) * piece;
+  const int64_t past = large ? nvec : nvec - kAmaxKept;   // up to here past the caches
   uint32_t m = 0;
-  int64_t p = int64_t(blockIdx.x) * kPiece;
+  int64_t p = int64_t(blockIdx.x) * piece;
   u32x4 t[kAmaxUnroll];
   const auto fold = [&] {
 #pragma unroll
     for (int u = 0; u < kAmaxUnroll; ++u) { const uint32_t a = A::of(t[u]); m = m > a ? m : a; }
   };
   // (two loops: in the branches of one, the loads would be merged into ordinary ones)
-  for (; p < past && p + kPiece <= nvec; p += next) {
+  for (; p < past && p + piece <= nvec; p += next) {
 #pragma unroll 1
-    for (int64_t h = 0; h < kPiece; h += kStep) {
+    for (int64_t h = 0; h < piece; h += kStep) {
 #pragma unroll
       for (int u = 0; u < kAmaxUnroll; ++u) t[u] = __builtin_nontemporal_load(xv + p + h + u * kAmaxThreads + threadIdx.x);
       fold();
     }
   }
-  for (; p + kPiece <= nvec; p += next) {
+  for (; p + piece <= nvec; p += next) {
 #pragma unroll 1
-    for (int64_t h = 0; h < kPiece; h += kStep) {
+    for (int64_t h = 0; h < piece; h += kStep) {
 #pragma unroll
       for (int u = 0; u < kAmaxUnroll; ++u) t[u] = xv[p + h + u * kAmaxThreads + threadIdx.x];
       fold();
     }
   }
-  for (int64_t h = p; h < nvec && h < p + kPiece; h += kStep) {   // the last piece: lanes past its end repeat its last vector
+  for (int64_t h = p; h < nvec && h < p + piece; h += kStep) {   // the last piece: lanes past its end repeat its last vector
 #pragma unroll
     for (int u = 0; u < kAmaxUnroll; ++u) {
       const int64_t v = h + u * kAmaxThreads + threadIdx.x;

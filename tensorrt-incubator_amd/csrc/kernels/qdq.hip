@@ -210,12 +210,15 @@ __device__ __forceinline__ void unpack4<F8>(uint32_t w, float* v) {
 // go past the caches.  us, codes past the caches against kept:
 //   row and column scales, a quantize and its dequantize: kept at every size (bf16 -> f8 of 8, 24 and 64 Mi elements 12.3 and 12.4,
 //   32.4 and 30.2, 73.8 and 70.9 by rows; f32 -> i8 of 4 and 64 Mi 12.2 and 11.4, 120 and 109)
-//   quantize and dequantize in one pass (keep_fused): kept above 32 Mi codes, what the eight L2s hold.  Below, the codes
-//   are still dirty there when the launch ends and are written back then.  With the amax in front, bf16 -> f8: 4 Mi 10.2 and
-//   11.3, 16 Mi 25.0 and 25.6, 32 Mi 43.3 and 43.7, 64 Mi 80.6 and 76.8, 128 Mi 156 and 142; f32 -> i8: 8 Mi 22.2 and 22.5, 24 Mi 59.5
-//   and 58.8, 64 Mi 146 and 138
-//   a quantize with one scale: never (43 Mi bf16 alone 25.1 and 26.4, with the amax in front 43.2 and 44.3)
-__device__ __forceinline__ bool keep_fused(int64_t n) { return n > (int64_t(32) << 20); }
+//   quantize and dequantize in one pass (keep_fused): kept above 24 Mi codes.  Below, the codes are still dirty in the L2s when
+//   the launch ends and are written back then.  With the amax in front, bf16 -> f8: 4 Mi 9.2 and 10.0, 9 Mi 13.7 and 14.4, 16 Mi
+//   20.6 and 21.0, 24 Mi 30.8 and 30.8, 48 Mi 56.6 and 54.6, 64 Mi 74.5 and 70.8, 128 Mi 149 and 138; f32 -> i8: 9 Mi and 32 Mi
+//   22.1 and 22.1, 67.0 and 66.6
+//   a quantize with one scale: kept, a dequantize reads them next (both, bf16 -> i4 of 22, 43 and 128 Mi 28.2 and 25.5, 49.4 and 46.6,
+//   131 and 123; f32 -> i8 of 22 and 64 Mi 42.8 and 39.6, 113 and 106; the quantize alone 43 Mi 25.1 and 26.4)
+//   ... behind its amax, with no dequantize asked for (kFlagCodesPast): not kept (bf16 -> f8 of 9, 16, 32 and 64 Mi 12.5 and 13.3,
+//   16.6 and 18.5, 29.7 and 31.2, 54.2 and 57.2): dirty lines take the place of the end of x in the L2s
+__device__ __forceinline__ bool keep_fused(int64_t n) { return n > (int64_t(24) << 20); }
 template <bool KEEP, typename T> __device__ __forceinline__ void store_codes(T v, T* p) {
   if (KEEP) *p = v;
   else __builtin_nontemporal_store(v, p);
@@ -300,6 +303,19 @@ template <int G, bool KEEP> struct CodeGroup<F4P, G, KEEP> {
     }
   }
 };
+
+// The choice made by the launch (uniform).  The comments in the assembly keep the two stores apart, which would otherwise become
+// one ordinary store.
+template <typename Q, int G>
+__device__ __forceinline__ void store_either(bool keep, typename Q::storage* q, int64_t e, float (&v)[G], int flags) {
+  if (keep) {
+    CodeGroup<Q, G, true>::store(q, e, v, flags);
+  } else {
+    __asm__ volatile("; codes past the caches");
+    CodeGroup<Q, G, false>::store(q, e, v, flags);
+    __asm__ volatile("; codes stored");
+  }
+}
 
 // clamp an exact quotient, rounding it first where a float target asks for that (integer targets round in enc; a clamp to
 // whole numbers before or after the rounding gives the same)
@@ -479,10 +495,7 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
 #pragma unroll
           for (int k = 0; k < G; ++k) v[k] = quant_value<Q>(v[k], sc[k], flags);
         }
-        if (store) {                                  // leaves f32(code) in v
-          if (keep) CG::store(q, e, v, flags);
-          else CodeGroup<Q, G, false>::store(q, e, v, flags);
-        }
+        if (store) store_either<Q, G>(keep, q, e, v, flags);   // leaves f32(code) in v
       }
       if (MODE != 0 && store) {
 #pragma unroll
@@ -518,7 +531,7 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   const int64_t nwaves = MODE == 2 ? int64_t(gridDim.x) * blockDim.x / kWave : int64_t(waves_in_launch());
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
   const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;
-  const bool keep = MODE == 2 ? keep_fused(n) : KIND != kUniform;
+  const bool keep = MODE == 2 ? keep_fused(n) : KIND != kUniform || !(flags & kFlagCodesPast);
 
   for (int64_t base = wave * (kWave * J); base < ngroups; base += nwaves * (kWave * J)) {
     // Row scales: the row of the trip's first group by two divisions for the whole wave, the others from there - a lane's
@@ -584,8 +597,7 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
           const ExactDivisor dv(s[j][0]);
           quantize_group<Q>(dv, v[j], flags);
         }
-        if (keep) CG::store(q, e, v[j], flags);
-        else CodeGroup<Q, G, false>::store(q, e, v[j], flags);
+        store_either<Q, G>(keep, q, e, v[j], flags);
       }
       if (MODE != 0) {
 #pragma unroll

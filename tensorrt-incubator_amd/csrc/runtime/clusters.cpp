@@ -263,10 +263,12 @@ bool bind_split(DeviceState *st, hipStream_t stream, Plan &plan, void *workspace
   return plan.split.tickets != nullptr;
 }
 
-// mode: 0 quantize, 1 dequantize, 2 fused
+constexpr int32_t kCodesPast = 1 << 8;  // kFlagCodesPast of the kernels (common.hpp)
+
+// mode: 0 quantize, 1 dequantize, 2 fused.  codes_past: nobody is known to read the codes next (see CodeGroup in qdq.hip)
 int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtype, void *q,
                      int32_t q_dtype, void *y, const float *scale, int32_t kind, int64_t d0,
-                     int64_t d1, int64_t nb, int32_t flags) {
+                     int64_t d1, int64_t nb, int32_t flags, bool codes_past = false) {
   clear_error();
   const char *xn = float_name(x_dtype);
   const char *qn = code_name(q_dtype);
@@ -338,7 +340,7 @@ int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtyp
   name + kModeName[mode] + "_" + (tiles ? kKindName[kind] : (ragged ? kRaggedName[kind] : "any")) + "_" + xn + "_" + qn;
 
   int64_t n_arg = n, d1_arg = d1, nb_arg = nb;
-  int32_t kind_arg = kind, flags_arg = flags;
+  int32_t kind_arg = kind, flags_arg = flags | (codes_past ? kCodesPast : 0);
   const void *x_arg = x;
   void *q_arg = q, *y_arg = y;
   const float *s_arg = scale;
@@ -726,7 +728,7 @@ int32_t mtrt_hip_dynamic_quantize_dequantize(mtrt_stream_t stream, const void *x
     return st1;
   if (y)
     return qdq_dispatch(2, as_hip(stream), x, x_dtype, q, q_dtype, y, scale_out, MTRT_SCALE_UNIFORM, 1, n, 1, flags);
-  return qdq_dispatch(0, as_hip(stream), x, x_dtype, q, q_dtype, nullptr, scale_out, MTRT_SCALE_UNIFORM, 1, n, 1, flags);
+  return qdq_dispatch(0, as_hip(stream), x, x_dtype, q, q_dtype, nullptr, scale_out, MTRT_SCALE_UNIFORM, 1, n, 1, flags, true);
 }
 
 int32_t mtrt_hip_dynamic_quantize_rows(mtrt_stream_t stream, const void *x, int32_t x_dtype, void *q, int32_t q_dtype,
