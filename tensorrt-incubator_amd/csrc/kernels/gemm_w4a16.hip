@@ -828,16 +828,12 @@ __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uin
       __asm__ volatile("global_load_ushort %0, %1, off" : "=v"(dst.sc[j]) : "v"(ssrc) : "memory");
     }
   };
-  // ties the registers of a slice to the wait, so that no use can be scheduled in front of it:
-  // four slices issued, the loads of three may fly -> those of the oldest slice have landed
-  auto landed = [&](Slice& sl) {
+  // ties the registers of a slice to the wait, so that no use can be scheduled in front of it: all loads but those of
+  // `in_flight` younger slices have landed
+  auto landed = [&](auto in_flight, Slice& sl) {
 #pragma unroll
     for (int j = 0; j < JT; ++j)
-      __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(sl.w[j]), "+v"(sl.sc[j]) : "n"(3 * kLoads) : "memory");
-  };
-  auto landed_all = [&](Slice& sl) {
-#pragma unroll
-    for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(0)" : "+v"(sl.w[j]), "+v"(sl.sc[j])::"memory");
+      __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(sl.w[j]), "+v"(sl.sc[j]) : "n"(decltype(in_flight)::value * kLoads) : "memory");
   };
 
   v16f acc[JT];
@@ -864,39 +860,36 @@ __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uin
   };
 
   // Main part: groups of four slices with four register sets, so that nothing is copied (a copy
-  // would have to wait for the load) and the loop has no branch; three slices stay in flight.
-  const int64_t kmain = kb0 + ((kb1 - kb0) & ~int64_t(3));
-  if (kb0 < kmain) {
-    const int64_t clamp = kmain - 1;                   // past the end: the last slice again, into a stage nobody reads
+  // would have to wait for the load) and the loop has no branch; three slices stay in flight.  The last slices, at most
+  // three, are on their way when it ends.
+  if (kb0 < kb1) {
+    using gemm_core::IntC;
+    const int64_t kmain = kb0 + ((kb1 - kb0) & ~int64_t(3)), clamp = kb1 - 1;   // past the end: the last slice again, into the stage that holds it
     Slice s0, s1, s2, s3;
     fetch(kb0, clamp, s0);
     fetch(kb0 + 1, clamp, s1);
     fetch(kb0 + 2, clamp, s2);
     for (int64_t kb = kb0; kb < kmain; kb += 4) {
       fetch(kb + 3, clamp, s3);
-      landed(s0);
+      landed(IntC<3>{}, s0);
       multiply(kb, s0);
       fetch(kb + 4, clamp, s0);
-      landed(s1);
+      landed(IntC<3>{}, s1);
       multiply(kb + 1, s1);
       fetch(kb + 5, clamp, s1);
-      landed(s2);
+      landed(IntC<3>{}, s2);
       multiply(kb + 2, s2);
       fetch(kb + 6, clamp, s2);
-      landed(s3);
+      landed(IntC<3>{}, s3);
       multiply(kb + 3, s3);
     }
-    // the surplus loads of the last group still target these registers: keep them until they land
-    landed_all(s0);
-    landed_all(s1);
-    landed_all(s2);
-  }
-  for (int64_t kb = kmain; kb < kb1; ++kb) {           // at most three slices, one at a time
-    Slice sl;
-    __builtin_amdgcn_s_waitcnt(0x0070);
-    fetch(kb, kb, sl);
-    landed_all(sl);
-    multiply(kb, sl);
+    // (surplus loads still target these registers: they stay allocated until those land)
+    landed(IntC<2>{}, s0);
+    if (kmain < kb1) multiply(kmain, s0);
+    landed(IntC<1>{}, s1);
+    if (kmain + 1 < kb1) multiply(kmain + 1, s1);
+    landed(IntC<0>{}, s2);
+    if (kmain + 2 < kb1) multiply(kmain + 2, s2);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);                  // surplus loads have landed before the ring is reused
   float (*partial)[16][64] = reinterpret_cast<float (*)[16][64]>(lds);
@@ -949,135 +942,157 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny(
 }
 
 // ---- M <= 16: one strip of columns per compute unit --------------------------------------------------
-// At this size the launch is bound by what each compute unit's L1 takes in: its share of the weights plus ALL of
-// the activations (16 rows x K).  One workgroup per 32-column tile leaves 344 workgroups on 256 compute units at
-// N = 11008, and the 88 units that hold two set the time.  Here the grid is one workgroup per compute unit, each
-// owning a contiguous strip of 16-column tiles (688 tiles -> 2 or 3 per workgroup, at most 48 of the ideal 43
-// columns) over ALL of K: no second round, no partial sums across workgroups.
+// At this size a compute unit has its share of the weights to dequantise plus ALL of the activations to take in (16 rows x
+// K).  One workgroup per 32-column tile leaves 344 workgroups on 256 compute units at N = 11008, and the 88 units that
+// hold two set the time.  Here the grid is one or two workgroups per compute unit, each owning a contiguous strip of
+// 16-column tiles (688 tiles -> 2 or 3 per workgroup, at most 48 of the ideal 43 columns) over ALL of K: no second
+// round, no partial sums across workgroups.
 // 16-column tiles need v_mfma_f32_16x16x32_f16 (lane l: column l % 16, k group l / 16, 8 consecutive k), so this
 // kernel reads the weights from a second re-layout made by mtrt_w4_prepack_strips:
 //   for each tile of 16 columns and each block of 128 k, 64 lanes x 4 dwords; dword j of lane l holds the 8 weights
 //   k = 128*kb + 32*j + 8*(l / 16) + [0..7] of column 16*tile + l % 16, nibbles ordered as in the 32-column layout.
-// The four waves of a workgroup split K; each keeps its own four-stage ring of activation slices (16 rows x 128 k,
+// The four waves of a workgroup split K; each keeps its own four-stage ring of activation slices (4 G rows x 128 k,
 // whole 256-byte row segments by direct-to-LDS loads, 16-byte chunks XOR-swizzled by the row so that the fragment
 // reads are conflict-free) and never touches another wave's ring: no barriers until the partial tiles are added
 // through LDS at the end.
+// G: groups of four activation rows (M <= 4 G); SC: scale rows per slice of 128 k (2: blocks of 64).
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-template <int WAVES, int JT>
+template <int WAVES, int JT, int G, int SC>
 __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws,
                                              const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
-                                             int64_t K, int64_t N, int64_t block, int64_t tile0, const uint16_t* __restrict__ bias, int8_t* lds) {
-  constexpr int kStages = 4, kStageBytes = 16 * 256;   // 16 rows x 128 k of f16
-  constexpr int kLoads = 4 + 2 * JT;                   // memory instructions per slice and wave
+                                             int64_t K, int64_t N, int64_t block, uint32_t tile0, const uint16_t* __restrict__ bias, int8_t* lds) {
+  constexpr int kStageBytes = G * 1024;                // 4 G rows x 128 k of f16
+  constexpr int kLoads = G + (1 + SC) * JT;            // memory instructions per slice and wave
   static_assert(3 * kLoads < 64, "wait counter range");
   const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int fcol = lane & 15, fgrp = lane >> 4;
-  const int64_t kblocks = K / 128;
-  const int64_t kb0 = kblocks * wave / WAVES, kb1 = kblocks * (wave + 1) / WAVES;
-  const uint32_t blocks_per_scale = uint32_t(block / 128);
-  int64_t col[JT];
-  const u4* bp[JT];
-#pragma unroll
-  for (int j = 0; j < JT; ++j) {
-    col[j] = (tile0 + j) * 16 + fcol;
-    col[j] = col[j] < N ? col[j] : N - 1;              // columns past N: the last column's scales, never stored
-    bp[j] = reinterpret_cast<const u4*>(ws) + ((tile0 + j) * kblocks) * 64 + lane;
-  }
-  int8_t* ring = lds + wave * (kStages * kStageBytes);
-
-  // direct-to-LDS load g (of 4) of a slice: rows 4g .. 4g+3; lane l <-> (row 4g + l / 16, LDS chunk position l % 16),
-  // which holds chunk (l % 16) ^ row of that row's 256 bytes
-  uint32_t aoff[4];
-#pragma unroll
-  for (int g = 0; g < 4; ++g) {
-    const int lrow = 4 * g + (lane >> 4);
-    const int64_t row = lrow < M ? lrow : M - 1;       // rows past M repeat the last row; never stored
-    aoff[g] = uint32_t(row * K * 2 + (((lane & 15) ^ lrow) << 4));
-  }
-  const int8_t* abase = reinterpret_cast<const int8_t*>(a);
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const uint32_t fcol = lane & 15, fgrp = lane >> 4;
+  const uint32_t kblocks = uint32_t(K) / 128;          // (K and N are below 2^31)
+  const uint32_t kb0 = kblocks * wave / WAVES, kb1 = kblocks * (wave + 1) / WAVES;
+  int8_t* ring = lds + wave * (4 * kStageBytes);
   struct Slice {
     u4 w[JT];
-    uint32_t sc[JT];
+    uint32_t sc[JT][SC];
   };
-  auto fetch = [&](int64_t kb, int64_t clamp, Slice& dst) {
-    kb = kb < clamp ? kb : clamp;
-    int8_t* st = ring + int(kb & (kStages - 1)) * kStageBytes;
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      __builtin_amdgcn_global_load_lds((gemm_core::global_void_t*)(abase + kb * 256 + aoff[g]),
-                                       (gemm_core::lds_void_t*)(st + g * 1024), 16, 0, 0);
-    // opaque register loads, waits placed by hand (see `skinny`)
-#pragma unroll
-    for (int j = 0; j < JT; ++j) {
-      const u4* wsrc = bp[j] + kb * 64;
-      const uint16_t* ssrc = scale + int64_t(uint32_t(kb) / blocks_per_scale) * N + col[j];
-      __asm__ volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(dst.w[j]) : "v"(wsrc) : "memory");
-      __asm__ volatile("global_load_ushort %0, %1, off" : "=v"(dst.sc[j]) : "v"(ssrc) : "memory");
-    }
-  };
-  auto landed = [&](Slice& sl) {
-#pragma unroll
-    for (int j = 0; j < JT; ++j)
-      __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(sl.w[j]), "+v"(sl.sc[j]) : "n"(3 * kLoads) : "memory");
-  };
-  auto landed_all = [&](Slice& sl) {
-#pragma unroll
-    for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(0)" : "+v"(sl.w[j]), "+v"(sl.sc[j])::"memory");
-  };
-
   v4f acc[JT];
 #pragma unroll
   for (int j = 0; j < JT; ++j) acc[j] = (v4f){0.0f, 0.0f, 0.0f, 0.0f};
-  const uint32_t mask = nibble_pair_mask(), mask_hi = mask << 4;
-  auto multiply = [&](int64_t kb, const Slice& sl) {
-    const int8_t* st = ring + int(kb & (kStages - 1)) * kStageBytes;
+
+  if (kb0 < kb1) {
+    // A wave alone on its SIMD issues one instruction in four cycles, whatever it is: addresses are scalar bases and 32-bit lane
+    // offsets that move on with the slices, and the stages of the ring are constants of the unrolled loop.
+    const uint32_t per_scale = uint32_t(block) / 128;
+    uint32_t at = kb0, row = kb0, left = 1;            // the slice that is fetched next, its row of scales, slices left of that row
+    if (SC == 2) {
+      row = 2 * kb0;
+    } else if (per_scale > 1) {
+      row = kb0 / per_scale;
+      left = per_scale - (kb0 - row * per_scale);
+    }
+    const uint64_t row_bytes = uint64_t(N) * 2;
+    const int8_t* wsrc[JT];
+    uint32_t soff[JT], woff = uint32_t(lane) * 16;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-      const v8h fa = *reinterpret_cast<const v8h*>(st + fcol * 256 + (((4 * ks + fgrp) ^ fcol) << 4));
+    for (int j = 0; j < JT; ++j) {
+      wsrc[j] = reinterpret_cast<const int8_t*>(ws) + (uint64_t(tile0 + j) * kblocks + kb0) * 1024;
+      const uint32_t col = (tile0 + j) * 16 + fcol;
+      soff[j] = (col < uint32_t(N) ? col : uint32_t(N) - 1) * 2;   // columns past N: the last column's scales, never stored
+    }
+    const int8_t* ssrc = reinterpret_cast<const int8_t*>(scale) + row * row_bytes;
+    const int8_t* asrc = reinterpret_cast<const int8_t*>(a) + uint64_t(kb0) * 256;
+    // direct-to-LDS load g (of G) of a slice: rows 4g .. 4g+3; lane l <-> (row 4g + l / 16, LDS chunk position l % 16),
+    // which holds chunk (l % 16) ^ row of that row's 256 bytes
+    uint32_t aoff[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const uint32_t lrow = 4 * g + fgrp;
+      const uint32_t arow = lrow < uint32_t(M) ? lrow : uint32_t(M) - 1;   // rows past M repeat the last row; never stored
+      aoff[g] = arow * (uint32_t(K) * 2) + ((fcol ^ lrow) << 4);
+    }
+    // the next slice into stage P, or past the end the last one again
+    auto fetch = [&](auto stage, Slice& dst) {
+      // opaque register loads, waits placed by hand (see `skinny`); what comes from memory is asked for first
+#pragma unroll
+      for (int j = 0; j < JT; ++j) __asm__ volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
+#pragma unroll
+      for (int j = 0; j < JT; ++j)
+#pragma unroll
+        for (int h = 0; h < SC; ++h)
+          __asm__ volatile("global_load_ushort %0, %1, %2" : "=v"(dst.sc[j][h]) : "v"(soff[j]), "s"(ssrc + h * row_bytes) : "memory");
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        __builtin_amdgcn_global_load_lds((gemm_core::global_void_t*)(asrc + aoff[g]),
+                                         (gemm_core::lds_void_t*)(ring + decltype(stage)::value * kStageBytes + g * 1024), 16, 0, 0);
+      const uint32_t go = at + 1 < kb1 ? 1 : 0;
+      at += go;
+      woff += go << 10;
+      asrc += go << 8;
+      if (SC == 2) {
+        ssrc += go ? 2 * row_bytes : 0;
+      } else {
+        left -= go;
+        if (left == 0) {
+          left = per_scale;
+          ssrc += row_bytes;
+        }
+      }
+    };
+    auto landed = [&](auto in_flight, Slice& sl) {     // all but the loads of `in_flight` younger slices
 #pragma unroll
       for (int j = 0; j < JT; ++j) {
-        H2Bits sp;
-        sp.u = sl.sc[j] * 0x00010001u;
-        union { u4 u; v8h h; } fb;
-        fb.u = dequant8_in_place(sl.w[j][ks], sp.h, mask, mask_hi);
-        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb.h, acc[j], 0, 0, 0);
+        __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(sl.w[j]) : "n"(decltype(in_flight)::value * kLoads) : "memory");
+#pragma unroll
+        for (int h = 0; h < SC; ++h)
+          __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(sl.sc[j][h]) : "n"(decltype(in_flight)::value * kLoads) : "memory");
       }
-    }
-  };
-
-  const int64_t kmain = kb0 + ((kb1 - kb0) & ~int64_t(3));
-  if (kb0 < kmain) {
-    const int64_t clamp = kmain - 1;                   // past the end: the last slice again, into a stage nobody reads
+    };
+    const uint32_t mask = nibble_pair_mask(), mask_hi = mask << 4;
+    const uint32_t frow = fcol & (4 * G - 1);          // rows past the ring: any valid data, never stored
+    auto multiply = [&](auto stage, const Slice& sl) {
+      const int8_t* st = ring + decltype(stage)::value * kStageBytes;
+      H2Bits sp[JT][SC];
+#pragma unroll
+      for (int j = 0; j < JT; ++j)
+#pragma unroll
+        for (int h = 0; h < SC; ++h) sp[j][h].u = sl.sc[j][h] * 0x00010001u;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const v8h fa = *reinterpret_cast<const v8h*>(st + frow * 256 + (((4 * ks + fgrp) ^ frow) << 4));
+        union { u4 u; v8h h; } fb[JT];
+#pragma unroll
+        for (int j = 0; j < JT; ++j) fb[j].u = dequant8_in_place(sl.w[j][ks], sp[j][SC == 2 ? ks / 2 : 0].h, mask, mask_hi);
+#pragma unroll
+        for (int j = 0; j < JT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fa, fb[j].h, acc[j], 0, 0, 0);
+      }
+    };
+    using gemm_core::IntC;
     Slice s0, s1, s2, s3;
-    fetch(kb0, clamp, s0);
-    fetch(kb0 + 1, clamp, s1);
-    fetch(kb0 + 2, clamp, s2);
-    for (int64_t kb = kb0; kb < kmain; kb += 4) {
-      fetch(kb + 3, clamp, s3);
-      landed(s0);
-      multiply(kb, s0);
-      fetch(kb + 4, clamp, s0);
-      landed(s1);
-      multiply(kb + 1, s1);
-      fetch(kb + 5, clamp, s1);
-      landed(s2);
-      multiply(kb + 2, s2);
-      fetch(kb + 6, clamp, s2);
-      landed(s3);
-      multiply(kb + 3, s3);
+    fetch(IntC<0>{}, s0);
+    fetch(IntC<1>{}, s1);
+    fetch(IntC<2>{}, s2);
+    uint32_t n = kb1 - kb0;                            // slices left
+    for (; n >= 4; n -= 4) {
+      fetch(IntC<3>{}, s3);
+      landed(IntC<3>{}, s0);
+      multiply(IntC<0>{}, s0);
+      fetch(IntC<0>{}, s0);
+      landed(IntC<3>{}, s1);
+      multiply(IntC<1>{}, s1);
+      fetch(IntC<1>{}, s1);
+      landed(IntC<3>{}, s2);
+      multiply(IntC<2>{}, s2);
+      fetch(IntC<2>{}, s2);
+      landed(IntC<3>{}, s3);
+      multiply(IntC<3>{}, s3);
     }
-    landed_all(s0);
-    landed_all(s1);
-    landed_all(s2);
-  }
-  for (int64_t kb = kmain; kb < kb1; ++kb) {           // at most three slices, one at a time
-    Slice sl;
-    __builtin_amdgcn_s_waitcnt(0x0070);
-    fetch(kb, kb, sl);
-    landed_all(sl);
-    multiply(kb, sl);
+    // at most three more slices, all on their way (past the end: surplus loads, whose registers stay allocated until they land)
+    landed(IntC<2>{}, s0);
+    if (n > 0) multiply(IntC<0>{}, s0);
+    landed(IntC<1>{}, s1);
+    if (n > 1) multiply(IntC<1>{}, s1);
+    landed(IntC<0>{}, s2);
+    if (n > 2) multiply(IntC<2>{}, s2);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);                  // surplus loads have landed before the ring is reused
   // partial tiles of the waves meet in LDS: [wave][tile][register][lane]
@@ -1094,38 +1109,52 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
 #pragma unroll
     for (int w = 1; w < WAVES; ++w) v = v + partial[((w * JT + j) * 4 + r) * 64 + l];
     const int64_t row = 4 * (l >> 4) + r;
-    const int64_t c = (tile0 + j) * 16 + (l & 15);
+    const int64_t c = int64_t(tile0 + j) * 16 + (l & 15);
     if (row < M && c < N) y[row * N + c] = narrow_with_bias(v, bias, c);
   }
   __syncthreads();                                     // the next chunk of this workgroup reuses the LDS
 }
 
-// (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M <= 16, K % 128 == 0, N, block % 128 == 0)
-// grid = min(compute units, ceil(N / 16)), block = 256: workgroup g owns tiles / grid consecutive 16-column tiles (the first
-// tiles % grid workgroups one more), three at a time.
-// Four waves, one per SIMD, each with eight of the 32 blocks of 128 k at K = 4096.  Measured on M = 16, N = 11008, K = 4096
-// (rocprofv3 kernel durations, an earlier form of the loop): 2 / 4 / 8 waves take 12.7 / 9.6 / 10.7 us; more than one
-// workgroup per compute unit (grids of 344, 512, 688) 11.5-12.6 us.  In-kernel timestamps of this form, median wave, us from
-// the launch's first wave: entered 0.3, first slice asked for 1.3, landed 2.7, K loop done 7.4 (0.69 per slice against some
-// 0.35 of issue for 175 dequantisation instructions and 12 MFMAs), results stored 8.0; the slowest wave 0.9 later.
-// So what is left is the microsecond of set-up (addresses and divisions) and the loop; M = 1 is 0.5 us shorter.
+// (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M <= 16, K % 128 == 0, N, block % 128 == 0, or 64 for
+// _b64) ; M * K < 2^31.
+// grid = one or two workgroups per compute unit, at most ceil(N / 16), block = 256: workgroup g owns tiles / grid consecutive
+// 16-column tiles (the first tiles % grid workgroups one more), three at a time.
+// What bounds it: four waves, one per SIMD, each with eight of the 32 slices at K = 4096, N = 11008, and a wave alone on its SIMD
+// issues one instruction in four cycles, whichever it is.  A slice of three tiles was 255 of them (168 to dequantise, 12 MFMAs,
+// 47 scalar, 11 waits for an operand made just before) and is 228; the last slices of a wave whose number is no multiple of
+// four came one at a time, a trip to memory each, and are now on their way with the others; up to four or eight rows take
+// a quarter or half of the activations' loads.  us, before and now, (M, K, N): (16, 4096, 11008) 9.1 and 8.7, (1, 4096, 11008)
+// 8.2 and 7.1, (16, 4096, 4096) 5.6 and 5.5, (1, 4096, 4096) 4.9 and 4.2, (2, 9600, 3136) 9.2 and 6.2, (13, 1152, 14464) 8.8 and
+// 6.6, (16, 5120, 13824) 16.9 and 13.4; in blocks of 64, against the kernel above: (2, 6656, 960) 9.3 and 4.9, (16, 4096, 11008)
+// 10.6 and 9.2, (13, 1152, 14464) 6.4 and 5.3.  Eight waves (two per SIMD) are no faster: 10.4 us at (16, 4096, 11008).
 constexpr int kStripWaves = 4;
-extern "C" __global__ void __launch_bounds__(64 * kStripWaves) mtrt_gemm_w4a16_strips16(
-    const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[kStripWaves * 4 * 4096];
+template <int G, int SC>
+__device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
+                                       uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block,
+                                       const uint16_t* __restrict__ bias, int8_t* lds) {
   // tiles / grid tiles each, the first tiles % grid workgroups one more (32-bit arithmetic: as 64-bit divisions this was
   // a microsecond of scalar instructions in front of the first load)
-  const uint32_t tiles = uint32_t((N + 15) / 16), grid = gridDim.x, b = blockIdx.x;
+  const uint32_t tiles = (uint32_t(N) + 15) / 16, grid = gridDim.x, b = blockIdx.x;
   const uint32_t per = tiles / grid, rem = tiles - per * grid;
-  const int64_t t0 = int64_t(b * per + (b < rem ? b : rem)), t1 = t0 + per + (b < rem ? 1 : 0);
-  for (int64_t t = t0; t < t1; t += 3) {
-    const int64_t left = t1 - t;
-    if (left >= 3) strips_chunk<kStripWaves, 3>(a, ws, scale, y, M, K, N, block, t, bias, lds);
-    else if (left == 2) strips_chunk<kStripWaves, 2>(a, ws, scale, y, M, K, N, block, t, bias, lds);
-    else strips_chunk<kStripWaves, 1>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+  const uint32_t t0 = b * per + (b < rem ? b : rem), t1 = t0 + per + (b < rem ? 1 : 0);
+  for (uint32_t t = t0; t < t1; t += 3) {
+    const uint32_t left = t1 - t;
+    if (left >= 3) strips_chunk<kStripWaves, 3, G, SC>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else if (left == 2) strips_chunk<kStripWaves, 2, G, SC>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else strips_chunk<kStripWaves, 1, G, SC>(a, ws, scale, y, M, K, N, block, t, bias, lds);
   }
 }
+#define MTRT_W4_STRIPS(NAME, SC)                                                                                          \
+  extern "C" __global__ void __launch_bounds__(64 * kStripWaves) NAME(                                                    \
+      const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,                \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {      \
+    __shared__ __attribute__((aligned(16))) int8_t lds[kStripWaves * 4 * 4096];                                           \
+    if (M <= 4) strips<1, SC>(a, ws, scale, y, M, K, N, block, bias, lds);                                                \
+    else if (M <= 8) strips<2, SC>(a, ws, scale, y, M, K, N, block, bias, lds);                                           \
+    else strips<4, SC>(a, ws, scale, y, M, K, N, block, bias, lds);                                                       \
+  }
+MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16, 1)
+MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16_b64, 2)
 
 // Re-layout for mtrt_gemm_w4a16_strips16: packed [K,N] nibbles -> strip order (above).  One thread per output dword.
 // (w_kn_packed, ws, K, N) ; K % 128 == 0.

@@ -261,18 +261,12 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const v4i* __r
         __asm__ volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(dst.w[j][p]) : "v"(wsrc) : "memory");
       }
   };
-  // four slices issued, the loads of three may fly -> those of the oldest slice have landed
-  auto landed = [&](Slice& sl) {
+  // all loads but those of `in_flight` younger slices have landed
+  auto landed = [&](auto in_flight, Slice& sl) {
 #pragma unroll
     for (int j = 0; j < JT; ++j)
 #pragma unroll
-      for (int p = 0; p < 4; ++p) __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(sl.w[j][p]) : "n"(3 * kLoads) : "memory");
-  };
-  auto landed_all = [&](Slice& sl) {
-#pragma unroll
-    for (int j = 0; j < JT; ++j)
-#pragma unroll
-      for (int p = 0; p < 4; ++p) __asm__ volatile("s_waitcnt vmcnt(0)" : "+v"(sl.w[j][p])::"memory");
+      for (int p = 0; p < 4; ++p) __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(sl.w[j][p]) : "n"(decltype(in_flight)::value * kLoads) : "memory");
   };
 
   v16i acc[JT];
@@ -292,39 +286,36 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const v4i* __r
   };
 
   // Main part: groups of four slices with four register sets, so that nothing is copied (a copy would have
-  // to wait for the load) and the loop has no branch; three slices stay in flight.
-  const int64_t kmain = kb0 + ((kb1 - kb0) & ~int64_t(3));
-  if (kb0 < kmain) {
-    const int64_t clamp = kmain - 1;                   // past the end: the last slice again, into a stage nobody reads
+  // to wait for the load) and the loop has no branch; three slices stay in flight.  The last slices, at most three, are on
+  // their way when it ends.
+  if (kb0 < kb1) {
+    using gemm_core::IntC;
+    const int64_t kmain = kb0 + ((kb1 - kb0) & ~int64_t(3)), clamp = kb1 - 1;   // past the end: the last slice again, into the stage that holds it
     Slice s0, s1, s2, s3;
     fetch(kb0, clamp, s0);
     fetch(kb0 + 1, clamp, s1);
     fetch(kb0 + 2, clamp, s2);
     for (int64_t kb = kb0; kb < kmain; kb += 4) {
       fetch(kb + 3, clamp, s3);
-      landed(s0);
+      landed(IntC<3>{}, s0);
       multiply(kb, s0);
       fetch(kb + 4, clamp, s0);
-      landed(s1);
+      landed(IntC<3>{}, s1);
       multiply(kb + 1, s1);
       fetch(kb + 5, clamp, s1);
-      landed(s2);
+      landed(IntC<3>{}, s2);
       multiply(kb + 2, s2);
       fetch(kb + 6, clamp, s2);
-      landed(s3);
+      landed(IntC<3>{}, s3);
       multiply(kb + 3, s3);
     }
-    // the surplus loads of the last group still target these registers: keep them until they land
-    landed_all(s0);
-    landed_all(s1);
-    landed_all(s2);
-  }
-  for (int64_t kb = kmain; kb < kb1; ++kb) {           // at most three slices, one at a time
-    Slice sl;
-    __builtin_amdgcn_s_waitcnt(0x0070);
-    fetch(kb, kb, sl);
-    landed_all(sl);
-    multiply(kb, sl);
+    // (surplus loads still target these registers: they stay allocated until those land)
+    landed(IntC<2>{}, s0);
+    if (kmain < kb1) multiply(kmain, s0);
+    landed(IntC<1>{}, s1);
+    if (kmain + 1 < kb1) multiply(kmain + 1, s1);
+    landed(IntC<0>{}, s2);
+    if (kmain + 2 < kb1) multiply(kmain + 2, s2);
   }
   __builtin_amdgcn_s_waitcnt(0x0070);                  // surplus loads have landed before the ring is reused
   int (*partial)[16][64] = reinterpret_cast<int (*)[16][64]>(lds);

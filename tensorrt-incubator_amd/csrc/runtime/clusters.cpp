@@ -1312,17 +1312,23 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
   if (!st)
     return MTRT_RUNTIME_ERROR;
   if (w4_fast(a, w_prepacked, K, block)) {
-    const bool strips = K % 128 == 0 && block % 128 == 0;
     const int64_t cus = num_compute_units(st);
     void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias};
-    if (M <= 16 && strips) {
-      // one workgroup per compute unit, each a strip of 16-column tiles over all of K (weights in strip order)
+    // Rows of activations are addressed by 32-bit offsets below.  Blocks of 64 take the strips where each of their four waves has
+    // a slice of 128 k; the kernel behind them, with slices of 64, is as fast below that.
+    const bool strips = M <= 16 && K % 128 == 0 && (block % 128 == 0 || (block == 64 && K >= 512)) && M * K < (int64_t(1) << 31);
+    if (strips) {
+      // 16-column tiles over all of K (weights in strip order).  One workgroup per compute unit; two for more than three
+      // tiles a unit, which a workgroup would take one after the other (K = 4096, M = 16: 768 tiles 9.0 against 10.6 us, 864 tiles
+      // 12.3 against 11.9, 1024 tiles 12.9 against 12.3), and with up to four rows for more than one (M = 1: 320 tiles 5.6 against
+      // 5.2 us, 688 tiles 7.4 against 7.1, 1024 tiles 10.2 against 9.8).
       const void *in_strips = static_cast<const char *>(w_prepacked) + w4_fragment_bytes(K, N);
       void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias};
-      const int64_t tiles = (N + 15) / 16;
-      return launch(st, KernelName("mtrt_gemm_w4a16_strips16"), uint32_t(std::min<int64_t>(tiles, cus)), kBlock, stream, sargs);
+      const int64_t tiles = (N + 15) / 16, most = M <= 4 || tiles > 3 * cus ? 2 * cus : cus;
+      return launch(st, KernelName(block == 64 ? "mtrt_gemm_w4a16_strips16_b64" : "mtrt_gemm_w4a16_strips16"),
+                    uint32_t(std::min<int64_t>(tiles, most)), kBlock, stream, sargs);
     }
-    if (M <= 32) {
+    if (M <= 32 && M * K < (int64_t(1) << 31)) {
       // one workgroup per 32-column tile; between one and two tiles per compute unit, one workgroup per
       // compute unit instead (the kernel then gives workgroup g the tiles g and g + grid, which share the
       // activations; measured: 6 % faster at M = 16, 21 % at M = 32, 3 % slower at M = 5)

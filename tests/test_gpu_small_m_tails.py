@@ -1,0 +1,60 @@
+"""The small-M GEMM kernels at K ranges that leave their waves every number of slices modulo the pipeline's depth, at the row counts
+where they change the form of their activation loads, and at tile counts around one, two and three per workgroup."""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _w4(torch, pkg, M, K, N, block, seed):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    w = torch.randint(-8, 8, (K, N), generator=g, device="cuda")
+    flat = (w & 15).to(torch.uint8).reshape(-1)
+    if flat.numel() % 2:
+        flat = torch.cat([flat, flat.new_zeros(1)])
+    packed = (flat[0::2] | (flat[1::2] << 4)).contiguous()
+    a = torch.randn((M, K), generator=g, device="cuda").half()
+    scale = (torch.rand((K // block, N), generator=g, device="cuda") * 0.015 + 0.005).half()
+    y = pkg.gemm_w4a16(a, scale, K, N, block, w_prepacked=pkg.gemm_w4a16_prepack(packed, K, N))
+    wd = (w.float() * scale.float().repeat_interleave(block, 0)).half().double()     # exact product, one rounding
+    ref, mass = a.double() @ wd, a.double().abs() @ wd.abs()
+    # f32 sums in any order, one rounding to f16
+    tol = 2.0 ** -11 * ref.abs() + (1 + 2.0 ** -11) * (K + 2) * 2.0 ** -24 * mass + 2.0 ** -24
+    bad = int(((y.double() - ref).abs() > tol).sum())
+    assert bad == 0, (M, K, N, block, bad)
+
+
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+def test_w4a16_strips(pkg, M, block):
+    import torch
+    for i, slices in enumerate((2, 4, 5, 6, 7, 8, 11, 13, 18, 28)):
+        K, N = slices * 256, (16, 40, 300, 1000, 4096, 4100, 8209)[i % 7]
+        _w4(torch, pkg, M, K, N, block, 100 * M + i)
+        expect = "mtrt_gemm_w4a16_strips16" + ("_b64" if block == 64 else "")
+        assert pkg.last_kernel() == expect, (K, N)
+    _w4(torch, pkg, M, 1536, 16 * 769, block, M)         # more than three tiles to each of 256 compute units
+
+
+@pytest.mark.parametrize("M", [1, 9, 16, 17, 25, 32])
+def test_w4a16_skinny(pkg, M):
+    import torch
+    for i, slices in enumerate((1, 2, 3, 4, 5, 6, 7, 9, 13, 17, 22, 31)):
+        K, N = slices * 64, (16, 40, 300, 1000, 8224)[i % 5]
+        _w4(torch, pkg, M, K, N, 64, 100 * M + i)
+        if M > 16 or K < 512 or K % 128:
+            assert pkg.last_kernel().startswith("mtrt_gemm_w4a16_skinny"), (K, N)
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+def test_w8a8_small(pkg, M):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    for i, slices in enumerate((1, 2, 3, 4, 5, 6, 7, 9, 12, 13, 15, 18, 23)):
+        K, N = slices * 128, (4128, 5000, 8200)[i % 3]   # more than half as many 32-column tiles as compute units
+        a = torch.randint(-128, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
+        w = torch.randint(-128, 128, (K, N), generator=g, device="cuda", dtype=torch.int8)
+        sa, sw = torch.rand(M, generator=g, device="cuda") * 0.01, torch.rand(N, generator=g, device="cuda") * 0.001
+        y = pkg.gemm_w8a8_fragments(a, pkg.gemm_w8a8_prepack_fragments(w), sa, sw, N)
+        assert pkg.last_kernel() == "mtrt_gemm_w8a8_small16"
+        acc = (a.double() @ w.double()).float()          # exact: below 2^53, and 2^24 here
+        assert torch.equal(y, ((acc * sa[:, None]) * sw[None, :]).half()), (M, K, N)
