@@ -622,6 +622,10 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 // LDS, in wave order, and go out through the epilogue.
 // Traits as for `run`, plus Scalar (the accumulator's element type).  Epilogue: finish(sum, row, col) -> the 16-bit
 // pattern (Y = uint16_t) or the float (Y = float) of y[row, col].  Grid: any (tiles dealt round-robin), block = 64 WAVES.
+// RAGGED: rows of any length from 16 bytes up, at any alignment of their elements, and any M: a workgroup owns 32 rows by 32
+// columns (a column tile's row tiles are neighbours).  A 16-byte piece that would leave its row is read from the row's last
+// sixteen bytes instead, and before it is used, in the last slice only, what it holds of the row is moved to its front and
+// the rest made zero, in both operands.
 namespace rows32 {
 constexpr int kPitch = 144, kStageBytes = 32 * kPitch;
 // MT: activation row tiles of 32 (1: M <= 32, 2: M <= 64, the weight fragments of a k-step serving both)
@@ -630,36 +634,62 @@ template <int WAVES, int MT = 1, bool FRAG = false> constexpr int lds_bytes() { 
 // FRAG: `w` is not the [N,K] array but its fragment-order re-layout (per 32 rows and 128-byte slice four 1 KiB blocks,
 // lane l of block q holding the 16 bytes of k-step q of its row: exactly the second MFMA operand).  The weight
 // fragments then go from memory to registers and into the MFMA without passing LDS, 1 KiB contiguous per instruction.
-template <class Traits, int WAVES, int MT = 1, bool FRAG = false, class Epilogue, typename Y>
+typedef u32x4 u32x4_anywhere __attribute__((aligned(1)));
+
+// The piece of a row that begins `left` bytes before the row's end, read from the row's last sixteen bytes where it would pass it.
+__device__ __forceinline__ u32x4 end_of_row(u32x4 v, int64_t left) {
+  if (left >= 16) return v;
+  if (left <= 0) return (u32x4){0u, 0u, 0u, 0u};
+  uint64_t lo = v[0] | uint64_t(v[1]) << 32, hi = v[2] | uint64_t(v[3]) << 32;
+  const uint32_t drop = 8 * uint32_t(16 - left);       // bits, 8 ... 120
+  if (drop >= 64) {
+    lo = hi >> (drop - 64);
+    hi = 0;
+  } else {
+    lo = lo >> drop | hi << (64 - drop);
+    hi >>= drop;
+  }
+  return (u32x4){uint32_t(lo), uint32_t(lo >> 32), uint32_t(hi), uint32_t(hi >> 32)};
+}
+
+template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool RAGGED = false, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ w, int64_t row_bytes, Epilogue& epi,
                                     Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds) {
+  static_assert(!RAGGED || (MT == 1 && !FRAG), "ragged rows: one row tile, [N,K] weights");
   using Acc = typename Traits::Acc;
   using Scalar = typename Traits::Scalar;
+  using Piece = typename std::conditional<RAGGED, u32x4_anywhere, u32x4>::type;
   constexpr int kWaveBytes = (MT + (FRAG ? 0 : 1)) * kStageBytes;   // fragment-order weights need no stage
   static_assert(kWaveBytes >= MT * 16 * 64 * int(sizeof(Scalar)), "a wave's stages also hold its partial sums");
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int frow = lane & 31, fhalf = lane >> 5;
   const int lrow = lane >> 3, lchunk = (lane & 7) * 16;
-  const int64_t slices = row_bytes / 128;
+  const int64_t slices = RAGGED ? (row_bytes + 127) / 128 : row_bytes / 128;
   const int64_t kb0 = slices * wave / WAVES, kb1 = slices * (wave + 1) / WAVES;
   int8_t* sa = lds + wave * kWaveBytes;
   int8_t* sw = sa + MT * kStageBytes;
-  const int64_t tiles = (N + 31) / 32;
-  for (int64_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+  const int64_t tiles = (N + 31) / 32, tiles_m = RAGGED ? (M + 31) / 32 : 1;
+  for (int64_t item = blockIdx.x; item < tiles * tiles_m; item += gridDim.x) {
+    const int64_t tile = RAGGED ? item / tiles_m : item, m0 = RAGGED ? (item - tile * tiles_m) * 32 : 0;
     const int8_t* ap[4 * MT];
     const int8_t* wp[4];
 #pragma unroll
     for (int i = 0; i < 4 * MT; ++i) {
-      const int64_t m = lrow + 8 * i;
-      ap[i] = a + (m < M ? m : M - 1) * row_bytes + lchunk;
+      const int64_t m = m0 + lrow + 8 * i;
+      ap[i] = a + (m < M ? m : M - 1) * row_bytes + (RAGGED ? 0 : lchunk);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t n = tile * 32 + lrow + 8 * i;
       // fragment order: block i of a slice (the re-layout holds zeros for rows past N); else: row n of the array
-      wp[i] = FRAG ? w + tile * slices * 4096 + i * 1024 + lane * 16 : w + (n < N ? n : N - 1) * row_bytes + lchunk;
+      wp[i] = FRAG ? w + tile * slices * 4096 + i * 1024 + lane * 16 : w + (n < N ? n : N - 1) * row_bytes + (RAGGED ? 0 : lchunk);
     }
     constexpr int64_t kSliceBytes = FRAG ? 4096 : 128;   // from one slice of a lane's weight pieces to the next
+    // bytes from a lane's pointers to its pieces of slice kb
+    const auto piece = [&](int64_t kb) {
+      const int64_t at = kb * 128 + lchunk;
+      return at < row_bytes - 16 ? at : row_bytes - 16;
+    };
     Acc acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = Traits::zero();
@@ -670,14 +700,22 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
       int64_t kb = kb0 + p < kb1 ? kb0 + p : kb1 - 1;
       kb = kb < 0 ? 0 : kb;
 #pragma unroll
-      for (int i = 0; i < 4 * MT; ++i) ra[p][i] = *reinterpret_cast<const u32x4*>(ap[i] + kb * 128);
+      for (int i = 0; i < 4 * MT; ++i) ra[p][i] = *reinterpret_cast<const Piece*>(ap[i] + (RAGGED ? piece(kb) : kb * 128));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const u32x4*>(wp[i] + kb * kSliceBytes);
+      for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const Piece*>(wp[i] + (RAGGED ? piece(kb) : kb * kSliceBytes));
     }
     for (int64_t kb = kb0; kb < kb1; kb += 2) {
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
         if (kb + p < kb1) {
+          if (RAGGED && kb + p == slices - 1) {
+            const int64_t left = row_bytes - (slices - 1) * 128 - lchunk;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              ra[p][i] = end_of_row(ra[p][i], left);
+              rw[p][i] = end_of_row(rw[p][i], left);
+            }
+          }
 #pragma unroll
           for (int i = 0; i < 4 * MT; ++i) *reinterpret_cast<u32x4*>(sa + (lrow + 8 * i) * kPitch + lchunk) = ra[p][i];
           u32x4 held[4];                               // fragment order: this slice's fragments stay in registers
@@ -688,9 +726,9 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
           }
           const int64_t next = kb + p + 2 < kb1 ? kb + p + 2 : kb1 - 1;   // always a load: the waits stay countable
 #pragma unroll
-          for (int i = 0; i < 4 * MT; ++i) ra[p][i] = *reinterpret_cast<const u32x4*>(ap[i] + next * 128);
+          for (int i = 0; i < 4 * MT; ++i) ra[p][i] = *reinterpret_cast<const Piece*>(ap[i] + (RAGGED ? piece(next) : next * 128));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const u32x4*>(wp[i] + next * kSliceBytes);
+          for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const Piece*>(wp[i] + (RAGGED ? piece(next) : next * kSliceBytes));
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             v4i fw;
@@ -720,7 +758,7 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
       Scalar v = reinterpret_cast<const Scalar*>(lds)[e];
 #pragma unroll
       for (int k = 1; k < WAVES; ++k) v = v + reinterpret_cast<const Scalar*>(lds + k * kWaveBytes)[e];
-      const int64_t row = t * 32 + (r >> 2) * 8 + (l >> 5) * 4 + (r & 3);
+      const int64_t row = m0 + t * 32 + (r >> 2) * 8 + (l >> 5) * 4 + (r & 3);
       const int64_t c = tile * 32 + (l & 31);
       if (row < M && c < N) y[row * N + c] = Y(epi.finish(v, row, c));
     }

@@ -394,26 +394,33 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w16_prepack_frag(const ui
   }
 }
 
-// Any K and any alignment on the matrix cores: (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N) ; grid: any
-// (128 x 128 tiles dealt round-robin), block = 256.
-extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_edge_f32(
-    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
-    int64_t K, int64_t N) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::edge::kLdsBytes];
-  dense_cluster::EdgeBiasF32Epilogue epi{bias};
-  gemm_core::edge::run<dense_cluster::F32Traits>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);
-}
-#define MTRT_DENSE_EDGE_KERNEL(XN, XT)                                                                             \
-  extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_edge_##XN(                                     \
+// Any K and any alignment on the matrix cores: (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N, waves) ; grid: any.
+// waves = 0, block = 256: 128 x 128 tiles dealt round-robin, each walked down all of K.  waves = 4 or 8, block = 64 waves, rows of at
+// least 16 bytes: 32 x 32 tiles whose K the waves share (gemm_core::rows32).  The large tile is bound by the one workgroup's walk
+// where there are fewer tiles than compute units, whatever the rows: us, large and small, f32 (1, 5449, 1344) 404 and 33,
+// (9, 1192, 3456) 92 and 11, (300, 2049, 1000) 163 and 31, (900, 1023, 1030) 95 and 37, (2000, 901, 2000) 86 and 118; f16 (1, 5449, 1344)
+// 87 and 15, (64, 2050, 2048) 38 and 9.7, (512, 2049, 2048) 45 and 31, (700, 1023, 8200) 49 and 92.
+#define MTRT_DENSE_EDGE_KERNEL(XN, XT, YT, TRAITS, EDGE, ROWS)                                                     \
+  extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_edge_##XN(                                     \
       const XT::storage* __restrict__ x, const XT::storage* __restrict__ w, const XT::storage* __restrict__ bias,  \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                 \
-    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::edge::kLdsBytes];                                \
-    dense_cluster::EdgeBiasEpilogue<XT> epi{bias};                                                                 \
-    gemm_core::edge::run<dense_cluster::HalfTraits<XT>>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 2, epi, y, \
-                                                        M, N, lds);                                                \
+      YT* __restrict__ y, int64_t M, int64_t K, int64_t N, int32_t waves) {                                        \
+    constexpr int kSmall = gemm_core::rows32::lds_bytes<8>(), kLarge = gemm_core::edge::kLdsBytes;                 \
+    __shared__ __attribute__((aligned(16))) int8_t lds[kSmall > kLarge ? kSmall : kLarge];                         \
+    const int8_t *x8 = reinterpret_cast<const int8_t*>(x), *w8 = reinterpret_cast<const int8_t*>(w);               \
+    const int64_t row_bytes = K * int64_t(sizeof(XT::storage));                                                    \
+    dense_cluster::ROWS rows_epi{bias};                                                                            \
+    if (waves == 8) {                                                                                              \
+      gemm_core::rows32::run<dense_cluster::TRAITS, 8, 1, false, true>(x8, w8, row_bytes, rows_epi, y, M, N, lds); \
+    } else if (waves == 4) {                                                                                       \
+      gemm_core::rows32::run<dense_cluster::TRAITS, 4, 1, false, true>(x8, w8, row_bytes, rows_epi, y, M, N, lds); \
+    } else {                                                                                                       \
+      dense_cluster::EDGE epi{bias};                                                                               \
+      gemm_core::edge::run<dense_cluster::TRAITS>(x8, w8, row_bytes, epi, y, M, N, lds);                           \
+    }                                                                                                              \
   }
-MTRT_DENSE_EDGE_KERNEL(f16, F16)
-MTRT_DENSE_EDGE_KERNEL(bf16, BF16)
+MTRT_DENSE_EDGE_KERNEL(f32, F32, float, F32Traits, EdgeBiasF32Epilogue, RowsBiasF32Epilogue)
+MTRT_DENSE_EDGE_KERNEL(f16, F16, uint16_t, HalfTraits<F16>, EdgeBiasEpilogue<F16>, RowsBiasEpilogue<F16>)
+MTRT_DENSE_EDGE_KERNEL(bf16, BF16, uint16_t, HalfTraits<BF16>, EdgeBiasEpilogue<BF16>, RowsBiasEpilogue<BF16>)
 
 // (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N) ; grid = ceil(M/64) * ceil(N/64), block = 256
 #define MTRT_DENSE_KERNEL(XN, XT)                                                                                  \

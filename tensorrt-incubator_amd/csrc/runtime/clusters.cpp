@@ -42,6 +42,11 @@ constexpr double kRowsFixedUs = 3.0, kRowsBytesPerUs = 3.4e6, kRowsWideBytesPerU
 // The same kernels with four row tiles (65 to 128 rows): one workgroup per compute unit at a time, so rounds of 32-column
 // tiles, each the length of its K loop: 3.7 ns per row byte (int8 M = 128, K = N = 4096 18.4 us, K = N = 8192 30.7 us).
 constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
+// Any-K kernel: rounds of 128 x 128 tiles, each a walk down K in steps of 128 bytes a row, against 32 x 32 tiles, two workgroups of four
+// waves to a compute unit (f32, up to one workgroup a unit: eight waves).  Fitted to 34 products, M 1 ... 2000, K 6 ... 12287, N 7 ... 11000,
+// f32 and f16; the faster form is taken in each of them.
+constexpr double kEdgeFixedUs = 4.0, kEdgeF32StepUs = 2.45, kEdge16StepUs = 1.2;
+constexpr double kEdgeSmallFixedUs = 3.0, kEdgeSmallFewStepUs = 0.2, kEdgeSmallStepUs = 0.5;
 // W4A16 tile choice: a full round of 256 x 256 tiles takes 3.25 times a full round of 128 x 128 tiles (for four times
 // the work), and a last round filled to a fraction f of the units takes 0.56 + 0.44 f^2 of a full one (fewer units
 // share the power budget).  Fitted over M = 48 ... 4096 at (K, N) = (4096, 4096), (4096, 11008), (11008, 4096),
@@ -1237,11 +1242,20 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   }
   void *args[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
   if (K > 0) {
-    // any other K or alignment: 128 x 128 tiles with element-aligned loads and a zero-padded last k-step
-    // (f16 [2048, 4100] x [11008, 4100]: 3761 us on the FMA kernel below)
-    const int64_t edge_tiles = ((M + 127) / 128) * ((N + 127) / 128);
-    return launch(st, KernelName("mtrt_gemm_dense_edge_") + xn, uint32_t(std::min<int64_t>(edge_tiles, int64_t(kMaxGrid) * 1024)),
-                  kBlock, as_hip(stream), args);
+    // any other K or alignment: element-aligned loads and a zero-padded last k-step, in 128 x 128 tiles
+    // (f16 [2048, 4100] x [11008, 4100]: 3761 us on the FMA kernel below) or 32 x 32 ones whose K the waves share
+    const int64_t edge_tiles = ((M + 127) / 128) * ((N + 127) / 128), small_tiles = ((M + 31) / 32) * tiles32, units = num_compute_units(st);
+    const double steps = double((K * eb + 127) / 128);
+    const double edge_us = tuning::kEdgeFixedUs + steps * (dtype == MTRT_F32 ? tuning::kEdgeF32StepUs : tuning::kEdge16StepUs) *
+                                                      double((edge_tiles + units - 1) / units);
+    const double small_us = tuning::kEdgeSmallFixedUs + steps * (small_tiles <= units ? tuning::kEdgeSmallFewStepUs
+                                                                                      : tuning::kEdgeSmallStepUs * std::max(1.0, double(small_tiles) / double(2 * units)));
+    int32_t waves = 0;
+    if (K * eb >= 16 && small_us < edge_us)
+      waves = dtype == MTRT_F32 && small_tiles <= units ? 8 : 4;
+    void *eargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &waves};
+    return launch(st, KernelName("mtrt_gemm_dense_edge_") + xn, uint32_t(std::min<int64_t>(waves ? small_tiles : edge_tiles, int64_t(kMaxGrid) * 1024)),
+                  waves ? uint32_t(64 * waves) : kBlock, as_hip(stream), eargs);
   }
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
   if (tiles > int64_t(kMaxGrid) * 1024)
@@ -1316,7 +1330,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
     void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias};
     // Rows of activations are addressed by 32-bit offsets below.  Blocks of 64 take the strips where each of their four waves has
     // a slice of 128 k; the kernel behind them, with slices of 64, is as fast below that.
-    const bool strips = M <= 16 && K % 128 == 0 && (block % 128 == 0 || (block == 64 && K >= 512)) && M * K < (int64_t(1) << 31);
+    const bool strips = M <= 16 && K % 128 == 0 && (block % 128 == 0 || (block == 64 && K >= 512)) && M * K <= (int64_t(1) << 31);
     if (strips) {
       // 16-column tiles over all of K (weights in strip order).  One workgroup per compute unit; two for more than three
       // tiles a unit, which a workgroup would take one after the other (K = 4096, M = 16: 768 tiles 9.0 against 10.6 us, 864 tiles
@@ -1328,7 +1342,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
       return launch(st, KernelName(block == 64 ? "mtrt_gemm_w4a16_strips16_b64" : "mtrt_gemm_w4a16_strips16"),
                     uint32_t(std::min<int64_t>(tiles, most)), kBlock, stream, sargs);
     }
-    if (M <= 32 && M * K < (int64_t(1) << 31)) {
+    if (M <= 32 && M * K <= (int64_t(1) << 31)) {
       // one workgroup per 32-column tile; between one and two tiles per compute unit, one workgroup per
       // compute unit instead (the kernel then gives workgroup g the tiles g and g + grid, which share the
       // activations; measured: 6 % faster at M = 16, 21 % at M = 32, 3 % slower at M = 5)
