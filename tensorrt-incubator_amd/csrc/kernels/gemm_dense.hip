@@ -258,6 +258,157 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_de
 MTRT_DENSE_MFMA_KERNEL(f16, F16)
 MTRT_DENSE_MFMA_KERNEL(bf16, BF16)
 
+// ---- few rows of f32 -----------------------------------------------------------------------------------
+// A wave takes COLS columns against ROWS rows, a lane four elements of K at a time, all in f32 (multiply-adds on the vector units);
+// KW = 4: the four waves of a workgroup take the same columns and every fourth 256 elements of K.  More rows than ROWS are groups,
+// on workgroups of one XCD that follow each other, so that its L2 has the weights from the first.  Bound by reading the weights up to
+// four rows (M = 1, K = 4096, N = 11008: 26.7 us, 6.8 TB/s), with more by the rows' way through L1, which COLS columns share.  The
+// matrix cores' f32 form works for 32 rows whatever M is and one workgroup walks 32 columns: us on 32 x 32 tiles, and here:
+// (M, K, N) = (1, 4096, 11008) 52.5, 26.7; (1, 5449, 1344) 32.3, 6.8; (3, 2816, 4672) 19.0, 11.5; (8, 4096, 4096) 26.1, 15.8;
+// (5, 12288, 256) 62, 9.8; (16, 1031, 260) 9.1, 4.3; (32, 4097, 4096), four groups, 38.7, 40.5.
+// Any K of at least 4, any alignment of whole elements.
+namespace dense_cluster {
+namespace dot {
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef f32x4 f32x4_words __attribute__((aligned(4)));
+
+// PAST: weights larger than the caches are read past them (M = 1, K = 4096, N = 11008: 28.9 -> 26.7 us; 29 MB in turns of six 6.8 -> 7.7)
+template <bool PAST>
+__device__ __forceinline__ f32x4 load(const f32x4_words* p) {
+  return PAST ? __builtin_nontemporal_load(p) : *p;
+}
+
+template <int ROWS, int COLS, int KW, int UNROLL, bool PAST>
+__device__ __forceinline__ void run(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+                                    float* __restrict__ y, int64_t M, int64_t K, int64_t N, float* lds) {
+  asm volatile("" : "+s"(K));   // what two forms of a kernel have in common is not computed, and held, for both
+  const int lane = int(threadIdx.x & 63), wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6));
+  const uint32_t groups = (uint32_t(M) + ROWS - 1) / ROWS, turn = blockIdx.x >> 3;
+  const int64_t row0 = turn % groups * ROWS, first = (int64_t(turn / groups * 8 + (blockIdx.x & 7)) * (4 / KW) + (KW == 1 ? wave : 0)) * COLS;
+  if (first >= N) return;
+  const float *xr[ROWS], *wr[COLS];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r) xr[r] = x + (row0 + r < M ? row0 + r : M - 1) * K;
+#pragma unroll
+  for (int c = 0; c < COLS; ++c) wr[c] = w + (first + c < N ? first + c : N - 1) * K;
+  float acc[ROWS][COLS];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) acc[r][c] = 0.0f;
+  const int64_t whole = K / 256;
+  const int slot = KW == 1 ? 0 : wave;
+  int64_t b = slot;
+#pragma unroll 1
+  for (; b + (UNROLL - 1) * KW < whole; b += UNROLL * KW) {
+    f32x4 wv[UNROLL][COLS];
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u)
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) wv[u][c] = load<PAST>(reinterpret_cast<const f32x4_words*>(wr[c] + (b + u * KW) * 256 + lane * 4));
+#pragma unroll
+    for (int u = 0; u < UNROLL; ++u) {
+      f32x4 xv[ROWS];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) xv[r] = *reinterpret_cast<const f32x4_words*>(xr[r] + (b + u * KW) * 256 + lane * 4);
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+        for (int c = 0; c < COLS; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[r][c] = __builtin_fmaf(xv[r][e], wv[u][c][e], acc[r][c]);
+    }
+  }
+  // the rest in steps of 256: the last one ends at K, its lanes' vectors moved back to lie within the row, what they then hold twice zero
+#pragma unroll 1
+  for (; b * 256 < K; b += KW) {
+    const int64_t k = b * 256 + lane * 4, at = k + 4 <= K ? k : K - 4;
+    const int skip = int(k - at < 4 ? k - at : 4);
+    f32x4 wv[COLS], xv[ROWS];
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) wv[c] = load<PAST>(reinterpret_cast<const f32x4_words*>(wr[c] + at));
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) xv[r] = *reinterpret_cast<const f32x4_words*>(xr[r] + at);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+#pragma unroll
+      for (int c = 0; c < COLS; ++c) wv[c][e] = e < skip ? 0.0f : wv[c][e];
+#pragma unroll
+      for (int r = 0; r < ROWS; ++r) xv[r][e] = e < skip ? 0.0f : xv[r][e];
+    }
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int c = 0; c < COLS; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[r][c] = __builtin_fmaf(xv[r][e], wv[c][e], acc[r][c]);
+  }
+  // ROWS * COLS sums over the wave: each exchange halves the values a lane holds, then the rest of the lanes' bits are summed
+  constexpr int V = ROWS * COLS;
+  float v[V];
+#pragma unroll
+  for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+    for (int c = 0; c < COLS; ++c) v[r * COLS + c] = acc[r][c];
+  int id = 0;
+#pragma unroll
+  for (int h = V / 2, bit = 1; bit < 64; bit *= 2, h /= 2) {
+    if (h >= 1) {
+      const bool up = lane & bit;
+      id = 2 * id + (up ? 1 : 0);
+#pragma unroll
+      for (int i = 0; i < h; ++i) {
+        const float keep = up ? v[i + h] : v[i], give = up ? v[i] : v[i + h];
+        v[i] = keep + __shfl_xor(give, bit, 64);
+      }
+    } else {
+      v[0] = v[0] + __shfl_xor(v[0], bit, 64);
+    }
+  }
+  // lane < V holds the sum of row id / COLS, column id % COLS
+  if (KW > 1) {
+    if (lane < V) lds[wave * V + lane] = v[0];
+    __syncthreads();
+    if (wave == 0 && lane < V) v[0] = (lds[lane] + lds[V + lane]) + (lds[2 * V + lane] + lds[3 * V + lane]);
+  }
+  const int64_t row = row0 + id / COLS, col = first + id % COLS;
+  if ((KW == 1 || wave == 0) && lane < V && row < M && col < N) y[row * N + col] = bias ? v[0] + bias[col] : v[0];
+}
+
+template <int ROWS, int COLS, int KW, int UNROLL>
+__device__ __forceinline__ void run_any(const float* x, const float* w, const float* bias, float* y, int64_t M, int64_t K, int64_t N, bool past, float* lds) {
+  if (past)
+    run<ROWS, COLS, KW, UNROLL, true>(x, w, bias, y, M, K, N, lds);
+  else
+    run<ROWS, COLS, KW, UNROLL, false>(x, w, bias, y, M, K, N, lds);
+}
+}  // namespace dot
+}  // namespace dense_cluster
+
+// Up to <rows> rows: (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N, form) ; form bit 0: waves share K, bit 1: weights past the
+// caches; grid = 8 * ceil(ceil(N / columns of a workgroup) / 8), block = 256.
+#define MTRT_DENSE_DOT_KERNEL(NAME, ROWS, COLS, UNROLL)                                                            \
+  extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_##NAME##_f32(                                  \
+      const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M, \
+      int64_t K, int64_t N, int32_t form) {                                                                        \
+    __shared__ float lds[4 * ROWS * COLS];                                                                         \
+    if (form & 1)                                                                                                  \
+      dense_cluster::dot::run_any<ROWS, COLS, 4, UNROLL>(x, w, bias, y, M, K, N, form & 2, lds);                   \
+    else                                                                                                           \
+      dense_cluster::dot::run_any<ROWS, COLS, 1, UNROLL>(x, w, bias, y, M, K, N, form & 2, lds);                   \
+  }
+MTRT_DENSE_DOT_KERNEL(rows1, 1, 2, 4)
+MTRT_DENSE_DOT_KERNEL(rows2, 2, 4, 4)
+MTRT_DENSE_DOT_KERNEL(rows4, 4, 4, 4)
+// ... any number in groups of eight: grid * ceil(M / 8); four columns to a wave, and eight (form bit 0 set)
+MTRT_DENSE_DOT_KERNEL(rows8, 8, 4, 2)
+extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_rows8_wide_f32(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
+    int64_t K, int64_t N, int32_t form) {
+  __shared__ float lds[4 * 8 * 8];
+  dense_cluster::dot::run_any<8, 8, 4, 1>(x, w, bias, y, M, K, N, form & 2, lds);
+}
+
 // Up to 32 rows, weights read once as whole rows (gemm_core::rows32): (x [M,K], w [N,K], bias or null, y, M <= 32, K, N) ;
 // rows in whole 128-byte slices, x and w 16-byte aligned; grid: any, block = 512.
 extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows32_f32(

@@ -42,6 +42,11 @@ constexpr double kRowsFixedUs = 3.0, kRowsBytesPerUs = 3.4e6, kRowsWideBytesPerU
 // The same kernels with four row tiles (65 to 128 rows): one workgroup per compute unit at a time, so rounds of 32-column
 // tiles, each the length of its K loop: 3.7 ns per row byte (int8 M = 128, K = N = 4096 18.4 us, K = N = 8192 30.7 us).
 constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
+// f32 products of few rows on the vector units: K from which four waves share it; weights read past the caches above these bytes (us, past
+// and through, M = 1: 180 MB 26.7, 28.9; M = 3, 53 MB 11.5, 12.0; M = 1, 29 MB 7.7, 6.8); the fewest weights (below, the tiles take 3 to 4 us
+// too) and the most columns (a grid); what several groups of rows read through the L2s.
+constexpr int64_t kDotOwnColumnsBelow = 1536, kDotPastBytes = int64_t(48) << 20, kDotMinWeights = 16384, kDotMaxColumns = int64_t(1) << 27;
+constexpr double kDotGroupBytesPerUs = 7.5e6;
 // Any-K kernel: rounds of 128 x 128 tiles, each a walk down K in steps of 128 bytes a row, against 32 x 32 tiles, two workgroups of four
 // waves to a compute unit (f32, up to one workgroup a unit: eight waves).  Fitted to 34 products, M 1 ... 2000, K 6 ... 12287, N 7 ... 11000,
 // f32 and f16; the faster form is taken in each of them.
@@ -1182,6 +1187,24 @@ int32_t mtrt_hip_gemm_w8a8_fragments_ws(mtrt_stream_t stream, const void *a, con
   return w8a8_fragments(as_hip(stream), a, w_frag, a_scale, 1, w_scale, nullptr, y, M, K, N, workspace, workspace_bytes);
 }
 
+namespace {
+// f32 products of few rows on the vector units (against the matrix cores' tiles: beside the kernels).  K below 1536 leaves four waves
+// that share it unequal parts, so each takes columns of its own where that still gives every compute unit a workgroup (us, shared and
+// own: (4, 448, 7680) 5.9, 4.8; (9, 1192, 3456) 9.8, 8.8; (4, 900, 900), 57 workgroups, 3.4, 4.6); more than four rows take eight
+// columns to a wave where that leaves two workgroups to a unit (us, four and eight: (8, 4096, 4096) 17.0, 15.8; (12, 2048, 512) 4.9, 6.1).
+int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const void *x, const void *w_nk, const void *bias, void *y, int64_t M, int64_t K, int64_t N) {
+  const int64_t units = num_compute_units(st), groups = (M + 7) / 8;
+  auto blocks = [&](int64_t columns) { return (N + columns - 1) / columns; };
+  const bool shared = K >= tuning::kDotOwnColumnsBelow || blocks(M == 1 ? 8 : 16) * groups < units;
+  const bool wide = M > 4 && K >= tuning::kDotOwnColumnsBelow && blocks(8) * groups >= 2 * units;
+  const int64_t columns = (M == 1 ? 2 : wide ? 8 : 4) * (shared ? 1 : 4), grid = 8 * ((blocks(columns) + 7) / 8) * groups;
+  int32_t form = (shared ? 1 : 0) | (groups == 1 && K * N * 4 > tuning::kDotPastBytes ? 2 : 0);
+  void *args[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &form};
+  return launch(st, KernelName(M == 1 ? "mtrt_gemm_dense_rows1_f32" : M == 2 ? "mtrt_gemm_dense_rows2_f32" : M <= 4 ? "mtrt_gemm_dense_rows4_f32" :
+                               wide ? "mtrt_gemm_dense_rows8_wide_f32" : "mtrt_gemm_dense_rows8_f32"), uint32_t(grid), kBlock, stream, args);
+}
+} // namespace
+
 int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w_nk, const void *bias, void *y,
                               int32_t dtype, int64_t M, int64_t K, int64_t N) {
   clear_error();
@@ -1204,6 +1227,9 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   DeviceState *st = device_state();
   if (!st)
     return MTRT_RUNTIME_ERROR;
+  const bool few = dtype == MTRT_F32 && K >= 4 && K * N >= tuning::kDotMinWeights && N <= tuning::kDotMaxColumns;
+  if (few && M <= 8)
+    return dense_few_rows_f32(st, as_hip(stream), x, w_nk, bias, y, M, K, N);
   // Decode-sized calls are bound by reading the weights once: up to 32 rows take one workgroup per 32 weight rows, its
   // eight waves splitting K (f16 M = 16, K = 4096, N = 11008: 55 us on the tile loop, 23.3 so, 3.9 TB/s of weights; f32
   // 473 -> 50 us); 33 to 64 rows the form with two activation row tiles per weight fragment; the tile loop (about
@@ -1250,6 +1276,10 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
                                                       double((edge_tiles + units - 1) / units);
     const double small_us = tuning::kEdgeSmallFixedUs + steps * (small_tiles <= units ? tuning::kEdgeSmallFewStepUs
                                                                                       : tuning::kEdgeSmallStepUs * std::max(1.0, double(small_tiles) / double(2 * units)));
+    // up to 32 rows of f32 may be read in groups of eight as well: us, 32 x 32 tiles and so, (9, 1192, 3456) 10.9, 9.4; (16, 1031, 260) 9.1,
+    // 4.4; (16, 600, 8000) 9.1, 9.9; (32, 4097, 4096) 38.7, 40.5
+    if (few && M <= 32 && 3.0 + double((M + 7) / 8) * double(K * N * 4) / tuning::kDotGroupBytesPerUs < std::min(small_us, edge_us))
+      return dense_few_rows_f32(st, as_hip(stream), x, w_nk, bias, y, M, K, N);
     int32_t waves = 0;
     if (K * eb >= 16 && small_us < edge_us)
       waves = dtype == MTRT_F32 && small_tiles <= units ? 8 : 4;

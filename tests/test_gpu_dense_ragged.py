@@ -29,7 +29,8 @@ def test_ragged_rows(pkg, M, N, dname):
         b = torch.randn(N, generator=g, device="cuda").to(td) if i % 2 else None
         out = torch.full((M * N + 128,), 7.0, dtype=td, device="cuda")
         y = pkg.linear_dense(x, w, b, out[64:64 + M * N].view(M, N))
-        assert pkg.last_kernel() == "mtrt_gemm_dense_edge_" + {"float32": "f32", "float16": "f16", "bfloat16": "bf16"}[dname]
+        if dname != "float32" or M > 32 or K * N < 16384:      # few rows of float32: below
+            assert pkg.last_kernel() == "mtrt_gemm_dense_edge_" + {"float32": "f32", "float16": "f16", "bfloat16": "bf16"}[dname]
         xd, wd = x.double(), w.double()
         bd = b.double() if b is not None else torch.zeros(N, dtype=torch.float64, device="cuda")
         ref, mass = xd @ wd.T + bd, xd.abs() @ wd.abs().T + bd.abs()
@@ -40,11 +41,41 @@ def test_ragged_rows(pkg, M, N, dname):
         assert bool((out[:64] == 7).all()) and bool((out[64 + M * N:] == 7).all())
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8, 9, 16, 17, 31, 32])
+def test_few_rows_of_float32(pkg, M):
+    """K around whole steps of 256 and of the four waves that share them, columns around what a wave and a workgroup take, weights
+    read through and past the caches."""
+    import torch
+    kernels = set()
+    for i, (K, N) in enumerate(((4, 4099), (5, 8200), (255, 1001), (256, 300), (257, 70), (513, 4097), (772, 8192), (1023, 16), (1280, 1), (1535, 5000),
+                                (1536, 33), (1539, 4100), (2048, 2047), (4095, 515), (4097, 66), (3071, 4200), (7681, 129))):
+        g = torch.Generator(device="cuda").manual_seed(100 * M + i)
+        x = _inside(torch, torch.randn((M, K), generator=g, device="cuda"), i % 4)
+        w = _inside(torch, torch.randn((N, K), generator=g, device="cuda") * 0.3, (3 * i) % 7)
+        b = torch.randn(N, generator=g, device="cuda") if i % 2 else None
+        out = torch.full((M * N + 128,), 7.0, device="cuda")
+        y = pkg.linear_dense(x, w, b, out[64:64 + M * N].view(M, N))
+        kernels.add(pkg.last_kernel())
+        xd, wd = x.double(), w.double()
+        bd = b.double() if b is not None else torch.zeros(N, dtype=torch.float64, device="cuda")
+        ref, mass = xd @ wd.T + bd, xd.abs() @ wd.abs().T + bd.abs()
+        bad = int(((y.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * mass).logical_not().sum())
+        assert bad == 0, (M, K, N, bad)
+        assert bool((out[:64] == 7).all()) and bool((out[64 + M * N:] == 7).all())
+    rows = 1 if M == 1 else 2 if M == 2 else 4 if M <= 4 else 8
+    assert "mtrt_gemm_dense_rows%d_f32" % rows in kernels
+    assert M not in (5, 8) or "mtrt_gemm_dense_rows8_wide_f32" in kernels
+    if M in (1, 8):                                            # (4100 x 3073: 50 MB)
+        x, w = torch.randn((M, 3073), device="cuda"), torch.randn((4100, 3073), device="cuda") * 0.3
+        ref, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+        assert bool(((pkg.linear_dense(x, w).double() - ref).abs() <= 3075 * 2.0 ** -24 * mass).all())
+
+
 @pytest.mark.parametrize("dname", ["float32", "float16"])
 def test_infinities_stay_in_their_row(pkg, dname):
     import torch
     td = getattr(torch, dname)
-    for M, K, N in ((40, 70, 50), (9, 1031, 300)):
+    for M, K, N in ((40, 70, 50), (9, 1031, 300), (9, 1025, 4100)):
         x, w = torch.ones((M, K), dtype=td, device="cuda"), torch.ones((N, K), dtype=td, device="cuda")
         x[3, K - 1], x[5, 0], w[7, K - 1] = float("inf"), float("nan"), float("-inf")
         y = pkg.linear_dense(x, w).float()
