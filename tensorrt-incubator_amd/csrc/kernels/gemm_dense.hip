@@ -521,6 +521,167 @@ MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
 MTRT_DENSE_FRAG_KERNELS(f16, F16)
 MTRT_DENSE_FRAG_KERNELS(bf16, BF16)
 
+// ---- up to 16 rows on fragment-order weights in ONE launch -----------------------------------------------
+// x goes into LDS whole, quantized and dequantized on its way where the module quantizes its input (the arithmetic of mtrt_act_fake_*,
+// bit for bit), while the first weights are on theirs: at a decode step the pass in front of the GEMM is all launch, and the
+// eight waves of gemm_core::rows32 each read all rows of their slices again, through the L1 that the weights come by.  A workgroup owns
+// 16 columns, half a tile of the fragment order (v_mfma_f32_16x16x32 takes a k-step pair's halves in four groups of lanes); its
+// eight waves share K in slices of 128 bytes, four slices in flight each.  Bound by the weights' way from memory and, with several
+// thousand elements, by their quantization in every workgroup.  bf16, us, rows32 and here (M, K, N): (1, 4096, 4096) 8.1, 7.0; (1, 4096, 11008)
+// 21.7, 16.2; (2, 14336, 512) 15.4, 10.2; (8, 2048, 16384) 15.8, 12.4; (16, 1024, 16384) 9.8, 8.4; (16, 512, 512) 3.5, 3.5; with float8
+// inputs, two launches and here: (1, 3968, 896) 9.3, 4.7; (1, 4096, 4096) 11.1, 7.0; (1, 4096, 11008) 25.0, 16.3; (8, 2048, 16384) 19.0, 14.5.
+// Weights above 48 MB are read past the caches ((1, 4096, 11008) 17.0 -> 16.2; 33 MB in turns of six 8.4 -> 9.8).
+namespace dense_cluster {
+namespace rows16 {
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int kWaves = 8, kMaxRows = 16, kAhead = 4;
+constexpr int kRowPad = 16;                                        // LDS bytes between the rows: their banks differ
+
+template <typename X> __device__ __forceinline__ v4f mfma(v4i a, v4i b, v4f c);
+template <> __device__ __forceinline__ v4f mfma<F16>(v4i a, v4i b, v4f c) {
+  union { v4i i; v8h h; } ua, ub;
+  ua.i = a; ub.i = b;
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(ua.h, ub.h, c, 0, 0, 0);
+}
+template <> __device__ __forceinline__ v4f mfma<BF16>(v4i a, v4i b, v4f c) {
+  union { v4i i; v8b h; } ua, ub;
+  ua.i = a; ub.i = b;
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(ua.h, ub.h, c, 0, 0, 0);
+}
+
+struct Plain {};
+
+template <typename X, typename Q, int kXGroups, bool PAST>
+__device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag,
+                                    const RowsBiasEpilogue<X>& epi, uint16_t* __restrict__ y, int M, int K, int Kp, int64_t N, int8_t* rows,
+                                    float (*partial)[64][4]) {
+  using qdq_cluster::ExactDivisor;
+  using qdq_cluster::FloatGroup;
+  constexpr bool kQuantized = !std::is_same<Q, Plain>::value;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int col = lane & 15, kgroup = lane >> 4;
+  const int slices = Kp / 64, kb0 = slices * wave / kWaves, kb1 = slices * (wave + 1) / kWaves;
+  const int64_t n0 = int64_t(blockIdx.x) * 16;
+
+  // x first: what is asked for first arrives first
+  const int row_groups = Kp / 8, groups = M * row_groups, pitch = 2 * Kp + kRowPad;
+  u32x4 xin[kXGroups];
+#pragma unroll
+  for (int i = 0; i < kXGroups; ++i) {
+    const int g = int(threadIdx.x) + i * 64 * kWaves, row = g / row_groups, k = (g - row * row_groups) * 8;
+    xin[i] = (u32x4){0u, 0u, 0u, 0u};
+    if (g < groups && k + 8 <= K) xin[i] = *reinterpret_cast<const qdq_cluster::u32x4_unaligned*>(x + int64_t(row) * K + k);
+  }
+  const float scale = kQuantized ? x_scale[0] : 1.0f;
+
+  // lane (col, kgroup) of k-step pair p: bytes 64 p + 16 kgroup ... + 15 of its column's slice
+  const int8_t* wp = w_frag + (n0 / 32) * slices * 4096 + (kgroup >> 1) * 1024 + ((kgroup & 1) * 32 + int(n0 & 16) + col) * 16;
+  const int last = kb1 > kb0 ? kb1 - 1 : 0;                        // a slice past the wave's last one is that one again
+  v4i w[kAhead][2];
+  const auto fetch = [&](int kb, v4i (&into)[2]) {
+    const int8_t* from = wp + int64_t(kb < kb1 ? kb : last) * 4096;
+#pragma unroll
+    for (int p = 0; p < 2; ++p) into[p] = PAST ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(from + p * 2048)) : *reinterpret_cast<const v4i*>(from + p * 2048);
+  };
+#pragma unroll
+  for (int s = 0; s < kAhead; ++s) fetch(kb0 + s, w[s]);
+
+  const ExactDivisor dv(scale);
+#pragma unroll
+  for (int i = 0; i < kXGroups; ++i) {
+    const int g = int(threadIdx.x) + i * 64 * kWaves, row = g / row_groups, xk = (g - row * row_groups) * 8;
+    if (g >= groups) continue;
+    const int left = K - xk;                                     // the group that holds a row's end, and the padding behind it
+    if (left > 0 && left < 8) {
+      for (int e = 0; e < left; ++e) {
+        const uint32_t bits = uint32_t(x[int64_t(row) * K + xk + e]) << (16 * (e & 1));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) xin[i][k] |= (e >> 1) == k ? bits : 0u;
+      }
+    }
+    u32x4 t = xin[i];
+    if constexpr (kQuantized) {
+      float v[8];
+      FloatGroup<X>::unpack(xin[i], v);
+      qdq_cluster::quantize_group<Q>(dv, v, 0);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) qdq_cluster::unpack4<Q>(qdq_cluster::pack4<Q>(&v[4 * h], 0), &v[4 * h]);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = v[k] * scale;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t[k] = qdq_cluster::narrow2<X>(v[2 * k], v[2 * k + 1]);
+    }
+    *reinterpret_cast<u32x4*>(rows + row * pitch + 2 * xk) = t;
+  }
+  __syncthreads();
+
+  v4f acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  const int8_t* arow = rows + (col < M ? col : M - 1) * pitch + kgroup * 16;   // as the first operand the lane's row; rows past M repeat the last
+  for (int kb = kb0; kb < kb1; kb += kAhead) {
+#pragma unroll
+    for (int s = 0; s < kAhead; ++s) {
+      v4i held[2] = {w[s][0], w[s][1]};
+      if (kb + kAhead < kb1) fetch(kb + kAhead + s, w[s]);
+      if (kb + s < kb1) {
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+          const v4i a = *reinterpret_cast<const v4i*>(arow + (kb + s) * 128 + p * 64);
+          acc = mfma<X>(a, held[p], acc);
+        }
+      }
+    }
+  }
+  // lane (col, h = lane / 16) holds rows 4 h + r of its column in register r
+#pragma unroll
+  for (int r = 0; r < 4; ++r) partial[wave][lane][r] = acc[r];
+  __syncthreads();
+  if (threadIdx.x < 256) {
+    const int l = threadIdx.x & 63, r = threadIdx.x >> 6;
+    float v = partial[0][l][r];
+#pragma unroll
+    for (int k = 1; k < kWaves; ++k) v = v + partial[k][l][r];
+    const int row = (l >> 4) * 4 + r;
+    const int64_t c = n0 + (l & 15);
+    if (row < M && c < N) y[int64_t(row) * N + c] = uint16_t(epi.finish(v, row, c));
+  }
+}
+
+template <typename X, typename Q, int kXGroups>
+__device__ __forceinline__ void run_any(const uint16_t* x, const float* x_scale, const int8_t* w_frag, const uint16_t* bias, uint16_t* y, int64_t M, int64_t K,
+                                        int64_t Kp, int64_t N, bool past, int8_t* rows, float (*partial)[64][4]) {
+  const RowsBiasEpilogue<X> epi{bias};
+  if (past)
+    run<X, Q, kXGroups, true>(x, x_scale, w_frag, epi, y, int(M), int(K), int(Kp), N, rows, partial);
+  else
+    run<X, Q, kXGroups, false>(x, x_scale, w_frag, epi, y, int(M), int(K), int(Kp), N, rows, partial);
+}
+}  // namespace rows16
+}  // namespace dense_cluster
+
+// (x [M,K], x_scale: one f32 (null without codes), w_frag (K padded to Kp), bias [N] or null, y [M,N], M <= 16, K, Kp, N, past) ; Kp = K rounded
+// up to 64, M * Kp <= 16384 (32768 for _long: twice the registers and LDS for x, one workgroup to a compute unit), w_frag 16-byte
+// aligned, x aligned to its elements; past: weights read past the caches; grid = ceil(N / 16), block = 512.
+#define MTRT_DENSE_ROWS16_KERNEL(NAME, XT, QT, GROUPS)                                                                    \
+  extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##NAME(                                          \
+      const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag, const uint16_t* __restrict__ bias, \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t Kp, int64_t N, int32_t past) {                              \
+    using namespace dense_cluster::rows16;                                                                                \
+    __shared__ __attribute__((aligned(16))) int8_t rows[GROUPS * 64 * kWaves * 16 + kMaxRows * kRowPad];                  \
+    __shared__ __attribute__((aligned(16))) float partial[kWaves][64][4];                                                 \
+    run_any<XT, QT, GROUPS>(x, x_scale, w_frag, bias, y, M, K, Kp, N, past, rows, partial);                               \
+  }
+#define MTRT_DENSE_ROWS16_KERNELS(XN, XT)                               \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16, XT, Plain, 4)                   \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_i8, XT, I8, 4)                   \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_f8, XT, F8, 4)                   \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_i4, XT, I4, 4)                   \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long, XT, Plain, 8)              \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long_i8, XT, I8, 8)              \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long_f8, XT, F8, 8)              \
+  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long_i4, XT, I4, 8)
+MTRT_DENSE_ROWS16_KERNELS(f16, F16)
+MTRT_DENSE_ROWS16_KERNELS(bf16, BF16)
+
 // Re-layout of 16-bit weights [N,K] into fragment order, one 16-byte chunk per thread: (w, w_frag, K, N) ; w_frag holds
 // 32 * ceil(N/32) * 128 * ceil(K/64) bytes, zeros where w has no element.
 extern "C" __global__ void __launch_bounds__(256) mtrt_w16_prepack_frag(const uint16_t* __restrict__ w, u32x4* __restrict__ w_frag,

@@ -42,10 +42,12 @@ constexpr double kRowsFixedUs = 3.0, kRowsBytesPerUs = 3.4e6, kRowsWideBytesPerU
 // The same kernels with four row tiles (65 to 128 rows): one workgroup per compute unit at a time, so rounds of 32-column
 // tiles, each the length of its K loop: 3.7 ns per row byte (int8 M = 128, K = N = 4096 18.4 us, K = N = 8192 30.7 us).
 constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
-// f32 products of few rows on the vector units: K from which four waves share it; weights read past the caches above these bytes (us, past
-// and through, M = 1: 180 MB 26.7, 28.9; M = 3, 53 MB 11.5, 12.0; M = 1, 29 MB 7.7, 6.8); the fewest weights (below, the tiles take 3 to 4 us
+// Products of few rows read weights above these bytes past the caches (us, past and through, f32: M = 1, 180 MB 26.7, 28.9; M = 3, 53 MB
+// 11.5, 12.0; M = 1, 29 MB 7.7, 6.8; bf16: 90 MB 16.2, 17.0; 67 MB 12.4, 13.4; 33 MB 9.8, 8.4).
+constexpr int64_t kWeightsPastBytes = int64_t(48) << 20;
+// f32 products of few rows on the vector units: K from which four waves share it; the fewest weights (below, the tiles take 3 to 4 us
 // too) and the most columns (a grid); what several groups of rows read through the L2s.
-constexpr int64_t kDotOwnColumnsBelow = 1536, kDotPastBytes = int64_t(48) << 20, kDotMinWeights = 16384, kDotMaxColumns = int64_t(1) << 27;
+constexpr int64_t kDotOwnColumnsBelow = 1536, kDotMinWeights = 16384, kDotMaxColumns = int64_t(1) << 27;
 constexpr double kDotGroupBytesPerUs = 7.5e6;
 // Any-K kernel: rounds of 128 x 128 tiles, each a walk down K in steps of 128 bytes a row, against 32 x 32 tiles, two workgroups of four
 // waves to a compute unit (f32, up to one workgroup a unit: eight waves).  Fitted to 34 products, M 1 ... 2000, K 6 ... 12287, N 7 ... 11000,
@@ -1198,7 +1200,7 @@ int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const void *x, c
   const bool shared = K >= tuning::kDotOwnColumnsBelow || blocks(M == 1 ? 8 : 16) * groups < units;
   const bool wide = M > 4 && K >= tuning::kDotOwnColumnsBelow && blocks(8) * groups >= 2 * units;
   const int64_t columns = (M == 1 ? 2 : wide ? 8 : 4) * (shared ? 1 : 4), grid = 8 * ((blocks(columns) + 7) / 8) * groups;
-  int32_t form = (shared ? 1 : 0) | (groups == 1 && K * N * 4 > tuning::kDotPastBytes ? 2 : 0);
+  int32_t form = (shared ? 1 : 0) | (groups == 1 && K * N * 4 > tuning::kWeightsPastBytes ? 2 : 0);
   void *args[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &form};
   return launch(st, KernelName(M == 1 ? "mtrt_gemm_dense_rows1_f32" : M == 2 ? "mtrt_gemm_dense_rows2_f32" : M <= 4 ? "mtrt_gemm_dense_rows4_f32" :
                                wide ? "mtrt_gemm_dense_rows8_wide_f32" : "mtrt_gemm_dense_rows8_f32"), uint32_t(grid), kBlock, stream, args);
@@ -1468,7 +1470,8 @@ int64_t round_up(int64_t v, int64_t step) { return (v + step - 1) / step * step;
 
 // How a plan's call runs: the row length its GEMM sees, whether x goes through the activation pass, and the two parts of the
 // workspace (the pass's result, then the partial tiles).
-// A decode step's W8A8 Linear quantizes its activations inside the GEMM (mtrt_linear_w8a8_decode) up to this many of them.
+// A decode step's Linear takes (and quantizes) its activations inside the GEMM, mtrt_linear_w8a8_decode and mtrt_gemm_dense_frag_*_rows16*,
+// up to this many of them.
 constexpr int64_t kDecodeElements = 16384;
 struct LinearShape {
   bool fragments = false, pass = false, one_launch = false;
@@ -1494,8 +1497,16 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
     // stay on the kernel that takes any K (about 15 us at a gigaflop).
     s.fragments = p.w_frag && eb == 2 && (p.K % 64 == 0 || !p.w || quantized || 2.0 * double(M) * double(p.K) * double(p.N) >= 1e9);
     s.Kp = s.fragments ? round_up(p.K, 64) : p.K;
-    s.pass = quantized || s.Kp != p.K;
-    s.act_bytes = s.pass ? round_up(M * s.Kp * eb, 256) : 0;
+    // Up to 16 rows in one launch.  Its 16-column workgroups each take x: where they are at most one to a compute unit, twice as many
+    // elements (bf16, float8 inputs, us, two launches and one: (8, 4096, 4096) 11.3, 10.1, (2, 14336, 512) 18.5, 12.7; (16, 1536, 8192) 9.4, 11.5);
+    // where they are more than two, half as many to quantize ((16, 1024, 16384) 10.1, 11.4; (8, 1024, 16384) 9.7, 8.5; (16, 1024, 8192) 7.2,
+    // 6.8); and a plain x that needs no pass only saves the 32-column kernel's way to its rows, from 1024 elements a row (us, that and
+    // this, bf16: (16, 512, 8192) 3.6, 4.2; (8, 768, 8192) 3.9, 4.1; (8, 1024, 8192) 4.2, 4.2; (4, 1024, 12000) 6.7, 5.2; (8, 2048, 8192) 5.1, 4.5).
+    const bool passes = quantized || s.Kp != p.K;
+    const int64_t tiles16 = (p.N + 15) / 16, most = tiles16 <= units ? 2 * kDecodeElements : passes && tiles16 > 2 * units ? kDecodeElements / 2 : kDecodeElements;
+    s.one_launch = s.fragments && M <= 16 && M * s.Kp <= most && (passes || tiles16 <= units || s.Kp >= 1024);
+    s.pass = !s.one_launch && passes;
+    s.act_bytes = passes ? round_up(M * s.Kp * eb, 256) : 0;   // asked for, not used, where the GEMM takes x itself
     if (s.fragments) {
       const DensePlan d = dense_frag_plan(M, s.Kp, p.N, units, true);
       s.partial_bytes = !d.rows && d.tile.tile ? d.tile.workspace() : 0;
@@ -1627,11 +1638,23 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   if (p.route == MTRT_LINEAR_W4A16)
     return w4a16(as_hip(stream), x, nullptr, p.w_frag, p.w_scale, p.bias, y, M, p.K, p.N, p.K, workspace, workspace_bytes);
   const LinearShape s = linear_shape(p, M, num_compute_units(st));
-  if (s.fragments && !s.pass && !s.one_launch && !aligned(x, 16))
+  if (p.route == MTRT_LINEAR_DENSE && s.fragments && p.q_dtype < 0 && s.Kp == p.K && !aligned(x, 16))
     return set_error(MTRT_INVALID_ARGUMENT, "x must be 16-byte aligned for these weights");
   const int64_t need = s.act_bytes + s.partial_bytes;
   if (need > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < need))
     return set_error(MTRT_INVALID_ARGUMENT, "workspace of %lld bytes, 16-byte aligned, needed", (long long)need);
+  if (s.one_launch && p.route == MTRT_LINEAR_DENSE) {
+    const float *x_scale = p.x_scale;
+    const void *w_frag = p.w_frag, *bias = p.bias;
+    int64_t K = p.K, Kp = s.Kp, N = p.N;
+    int32_t past = Kp * N * eb > tuning::kWeightsPastBytes;
+    KernelName name("mtrt_gemm_dense_frag_");
+    name + float_name(p.dtype) + (M * Kp <= kDecodeElements ? "_rows16" : "_rows16_long");
+    if (p.q_dtype >= 0)
+      name + "_" + code_name(p.q_dtype);
+    void *args[] = {&x, &x_scale, &w_frag, &bias, &y, &M, &K, &Kp, &N, &past};
+    return launch(st, name, uint32_t((N + 15) / 16), 512, as_hip(stream), args);
+  }
   if (s.one_launch) {
     const float *w_scale = static_cast<const float *>(p.w_scale), *x_scale = p.x_scale;
     const void *w_frag = p.w_frag, *bias = p.bias;
