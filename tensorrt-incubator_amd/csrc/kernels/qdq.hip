@@ -330,7 +330,7 @@ __device__ __forceinline__ float quant_value(float x, float s, int flags) {
   return finish_quotient<Q>(x / s, flags);           // IEEE divide, bit-exact with the host
 }
 
-// Correctly rounded x / s for MANY x and ONE s, in 8 instructions instead of the 13
+// Correctly rounded x / s for MANY x and ONE s, in 8 instructions (to a code: fewer, see quantize_fast1) instead of the 13
 // of the full IEEE divide expansion.  With r = RN(1/s) (one IEEE divide per lane):
 //     q0 = RN(x r);  q1 = RN(q0 + RN(x - q0 s) r);  q2 = RN(q1 + RN(x - q1 s) r)
 // q1 is within a hair of x/s, hence a faithful rounding, and the remainder of a
@@ -369,22 +369,25 @@ struct ExactDivisor {
   // zero is put back after the clamp (a clamp keeps it), so that the clamp's operands are results of arithmetic
   // and need no quieting first.
   // Integer targets: x is clamped to [kLo s, kHi s] instead (either order: s may be negative), which bounds the quotient
-  // to the codes' range, give or take an ulp at its ends, where it rounds to the end's code; a zero needs no sign.  All
-  // on -x and -q, because the clamp is one v_med3, which gives the least operand for a NaN: that of -x is the greatest
-  // of x, as above.  With the rounding in enc this is 8 instructions an element to a code and one to gather it, where
-  // minimum, maximum, rounding, clamp, sign, conversion, mask and shift made it 18: a tensor of 45 M bf16 took 18 us of
-  // the vector units.
+  // to the codes' range, give or take an ulp at its ends, where it rounds to the end's code; a zero needs no sign.  The
+  // clamp is one v_med3 of -x, which gives the least operand for a NaN: that of -x is the greatest of x, as above.
+  // q1 above is enough here.  It differs from the correctly rounded quotient at most where x/s is within a hair of the middle of
+  // two floats, and a code only where one of those two is the middle of two codes (or of the whole numbers, or of the f16 values,
+  // that a float target is rounded to first): a number of at most 12 significant bits.  Of the three x nearest to each such
+  // middle, for all 2^23 mantissas of s, all 2^11 numbers of 12 bits and both neighbours (1.03e11 quotients), none differs.
+  // With the rounding in enc this is 5 instructions an element to a code and one to gather it; with both corrections and
+  // the arithmetic on -q it was 8, and minimum, maximum, rounding, clamp, sign, conversion, mask and shift made it 18: a
+  // tensor of 45 M bf16 took 18 us of the vector units.
   template <typename Q, bool ROUND>
   __device__ __forceinline__ float quantize_fast1(float x) const {
     const float nx = Codes<Q>::kInteger ? __builtin_amdgcn_fmed3f(-x, -Codes<Q>::kLo * s, -Codes<Q>::kHi * s)
                                         : __builtin_amdgcn_fmed3f(-x, bound, -bound);
-    const float n0 = nx * r;
-    float n = __builtin_fmaf(__builtin_fmaf(-n0, s, nx), r, n0);
-    n = __builtin_fmaf(__builtin_fmaf(-n, s, nx), r, n);
-    if (Codes<Q>::kInteger) return -n;
-    if (ROUND) n = __builtin_rintf(n);
-    n = __builtin_amdgcn_fmed3f(n, -Codes<Q>::kHi, -Codes<Q>::kLo);
-    return -__builtin_copysignf(n, n0);
+    const float q0 = nx * -r;
+    float q = __builtin_fmaf(__builtin_fmaf(q0, s, nx), -r, q0);
+    if (Codes<Q>::kInteger) return q;
+    if (ROUND) q = __builtin_rintf(q);
+    q = __builtin_amdgcn_fmed3f(q, Codes<Q>::kLo, Codes<Q>::kHi);
+    return __builtin_copysignf(q, q0);
   }
   template <typename Q, bool ROUND, int G>
   __device__ __forceinline__ void quantize_fast(float (&v)[G]) const {
@@ -423,7 +426,7 @@ constexpr int kColChunkRows = 8;
 // asked for before the reciprocals are formed, and everything about a row but the lane's columns is in scalar registers.
 // bf16 [4096, 11008] to int4 in blocks of 128 rows and back (270 MB), us: 67.7 with 4 rows in flight, chunks of 32 and
 // 18 instructions an element; 55.6 with 8 rows, chunks of 16 and the short arithmetic of ExactDivisor; 53.0 with chunks
-// of 8 rows (of 4: 60.6); 49.4 with the codes left in the caches (see CodeGroup).
+// of 8 rows (of 4: 60.6); 49.9 with the codes left in the caches (see CodeGroup); 48.7 with one correction of the quotient.
 template <typename X, typename Q, int MODE>
 __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                                typename X::storage* __restrict__ y, const float* __restrict__ scale,
