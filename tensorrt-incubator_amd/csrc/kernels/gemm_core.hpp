@@ -218,52 +218,10 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
   }
 }
 
-// The same sub-tiles written as f32, straight from the accumulators: a lane's runs of four consecutive outputs of a
-// row are one 16-byte store each (32-byte pieces of a row per half wave, merged in the write-back cache); no staging.
-// Epilogue: finish4(values of columns col .. col+3, col, N).  For the 2 x 2 waves of `run`.
-template <int JT, class Acc, class Epilogue>
-__device__ __forceinline__ void write_tile_f32(Acc (&acc)[4][JT], Epilogue& epi, float* __restrict__ y, int64_t M, int64_t N,
-                                               int64_t m0, int64_t n0, int wave) {
-  const int lane = threadIdx.x & 63;
-  const int wm = wave >> 1, wn = wave & 1;
-  const int frow = lane & 31, fhalf = lane >> 5;
-  const bool vec_ok = (N % 4 == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int64_t row = m0 + wm * 128 + i * 32 + frow;
-    if (row >= M) continue;
-#pragma unroll
-    for (int j = 0; j < JT; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int64_t col = n0 + wn * (32 * JT) + j * 32 + q * 8 + fhalf * 4;
-        if (col >= N) continue;
-        float v[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * q + e];
-        epi.finish4(v, col, N);
-        if (vec_ok && col + 3 < N) {
-          const f32x4 t = {v[0], v[1], v[2], v[3]};
-          __builtin_nontemporal_store(t, reinterpret_cast<f32x4*>(y + row * N + col));
-        } else if (col + 3 < N) {                      // rows that do not start on 16 bytes
-          *reinterpret_cast<f32x4_words*>(y + row * N + col) = (f32x4){v[0], v[1], v[2], v[3]};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (col + e < N) y[row * N + col + e] = v[e];
-        }
-      }
-  }
-}
 template <int JT, class Acc, class Epilogue>
 __device__ __forceinline__ void finish_tile(Acc (&acc)[4][JT], Epilogue& epi, uint16_t* __restrict__ y, int64_t M, int64_t N,
                                             int64_t m0, int64_t n0, int8_t* lds, int wave) {
   write_tile<JT, 2, 4>(acc, epi, y, M, N, m0, n0, lds, wave, true);
-}
-template <int JT, class Acc, class Epilogue>
-__device__ __forceinline__ void finish_tile(Acc (&acc)[4][JT], Epilogue& epi, float* __restrict__ y, int64_t M, int64_t N,
-                                            int64_t m0, int64_t n0, int8_t*, int wave) {
-  write_tile_f32<JT>(acc, epi, y, M, N, m0, n0, wave);
 }
 
 // Both operands as bytes, K-contiguous per row / per column: a [M, a_row_bytes], b [N, a_row_bytes].
@@ -272,7 +230,7 @@ __device__ __forceinline__ void finish_tile(Acc (&acc)[4][JT], Epilogue& epi, fl
 // Traits: Acc (16-wide accumulator vector), mfma(first, second, acc), zero().
 // Epilogue: setup(lds scratch, m0, M, n0, N), columns<HC>(first column of the lane in the tile), row(row in tile),
 // convert4(acc, q, column tile of the pass, words): outputs 4q .. 4q+3 of the accumulator as two words of two.
-// Y: uint16_t (16-bit outputs through the staged epilogue) or float (direct stores, see write_tile_f32).
+// Y: uint16_t, through the staged epilogue.
 template <class Traits, int JT, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ b, int64_t row_bytes, Epilogue& epi,
                                     Y* __restrict__ y, int64_t M, int64_t N, int64_t slices, int64_t m0,
@@ -622,8 +580,8 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 // LDS, in wave order, and go out through the epilogue.
 // Traits as for `run`, plus Scalar (the accumulator's element type).  Epilogue: finish(sum, row, col) -> the 16-bit
 // pattern (Y = uint16_t) or the float (Y = float) of y[row, col].  Grid: any (tiles dealt round-robin), block = 64 WAVES.
-// RAGGED: rows of any length from 16 bytes up, at any alignment of their elements, and any M: a workgroup owns 32 rows by 32
-// columns (a column tile's row tiles are neighbours).  A 16-byte piece that would leave its row is read from the row's last
+// MANY: any M, a workgroup owns 32 rows by 32 columns (see place for their order).
+// RAGGED (with MANY): rows of any length from 16 bytes up, at any alignment of their elements.  A 16-byte piece that would leave its row is read from the row's last
 // sixteen bytes instead, and before it is used, in the last slice only, what it holds of the row is moved to its front and
 // the rest made zero, in both operands.
 namespace rows32 {
@@ -652,10 +610,24 @@ __device__ __forceinline__ u32x4 end_of_row(u32x4 v, int64_t left) {
   return (u32x4){uint32_t(lo), uint32_t(lo >> 32), uint32_t(hi), uint32_t(hi >> 32)};
 }
 
-template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool RAGGED = false, class Epilogue, typename Y>
+// The tile of work item `item`, 8 * ceil(tiles_m * tiles_n / 8) of them, false where there is none: what goes to one XCD (items with
+// the same remainder by eight) is one stretch of the tiles, and a stretch goes down eight tiles of rows before the next tile of columns, so
+// that what an L2 holds serves both operands (f32, M, K, N: (1024, 3072, 1024) 81 -> 70 us, (300, 3072, 2048) 66 -> 56, (128, 4096, 4096) 52 -> 48.5).
+template <typename I>
+__device__ __forceinline__ bool place(I item, I tiles_m, I tiles_n, int64_t& m, int64_t& n) {
+  const I total = tiles_m * tiles_n, at = (item & 7) * ((total + 7) / 8) + (item >> 3);
+  if (at >= total) return false;
+  const I group = at / (8 * tiles_n), rest = at - group * (8 * tiles_n), tall = tiles_m - 8 * group < 8 ? tiles_m - 8 * group : 8;
+  m = int64_t(8 * group + rest % tall);
+  n = int64_t(rest / tall);
+  return true;
+}
+
+template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool MANY = false, bool RAGGED = false, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ w, int64_t row_bytes, Epilogue& epi,
                                     Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds) {
-  static_assert(!RAGGED || (MT == 1 && !FRAG), "ragged rows: one row tile, [N,K] weights");
+  static_assert(!MANY || MT == 1, "one row tile at a time");
+  static_assert(!RAGGED || (MANY && !FRAG), "ragged rows: [N,K] weights");
   using Acc = typename Traits::Acc;
   using Scalar = typename Traits::Scalar;
   using Piece = typename std::conditional<RAGGED, u32x4_anywhere, u32x4>::type;
@@ -668,9 +640,15 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
   const int64_t kb0 = slices * wave / WAVES, kb1 = slices * (wave + 1) / WAVES;
   int8_t* sa = lds + wave * kWaveBytes;
   int8_t* sw = sa + MT * kStageBytes;
-  const int64_t tiles = (N + 31) / 32, tiles_m = RAGGED ? (M + 31) / 32 : 1;
-  for (int64_t item = blockIdx.x; item < tiles * tiles_m; item += gridDim.x) {
-    const int64_t tile = RAGGED ? item / tiles_m : item, m0 = RAGGED ? (item - tile * tiles_m) * 32 : 0;
+  const int64_t tiles = (N + 31) / 32, tiles_m = MANY ? (M + 31) / 32 : 1;
+  const int64_t items = MANY ? (tiles * tiles_m + 7) / 8 * 8 : tiles;
+  for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+    int64_t tile = item, m0 = 0;
+    if (MANY) {
+      const bool there = items < (int64_t(1) << 28) ? place(uint32_t(item), uint32_t(tiles_m), uint32_t(tiles), m0, tile) : place(item, tiles_m, tiles, m0, tile);
+      if (!there) continue;                            // the whole workgroup
+      m0 *= 32;
+    }
     const int8_t* ap[4 * MT];
     const int8_t* wp[4];
 #pragma unroll

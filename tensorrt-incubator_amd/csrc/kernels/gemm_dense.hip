@@ -118,16 +118,6 @@ struct F32Traits {
     return c;
   }
 };
-struct BiasF32Epilogue {
-  const float* bias;
-  __device__ __forceinline__ void finish4(float (&v)[4], int64_t col, int64_t N) const {
-    if (!bias) return;
-#pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (col + e < N) v[e] = v[e] + bias[col + e];
-  }
-};
-
 template <typename X> __device__ __forceinline__ uint32_t narrow16(float v);
 template <> __device__ __forceinline__ uint32_t narrow16<F16>(float v) { return f32_to_f16_bits(v); }
 template <> __device__ __forceinline__ uint32_t narrow16<BF16>(float v) { return f32_to_bf16_bits(v); }
@@ -183,27 +173,6 @@ __device__ __forceinline__ void dense_mfma_body(const typename X::storage* __res
   }
 }
 
-__device__ __forceinline__ void dense_mfma_f32_body(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
-                                                    float* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t full_panels,
-                                                    int8_t* lds) {
-  const int64_t tiles_m = (M + gemm_core::BM - 1) / gemm_core::BM;
-  const int64_t full_blocks = gemm_core::even_blocks(full_panels * tiles_m);
-  BiasF32Epilogue epi{bias};
-  const int8_t* a8 = reinterpret_cast<const int8_t*>(x);
-  const int8_t* w8 = reinterpret_cast<const int8_t*>(w);
-  int64_t tile_m, panel;
-  if (int64_t(blockIdx.x) < full_blocks) {
-    if (!gemm_core::tile_of_even(blockIdx.x, uint32_t(full_blocks), tiles_m, full_panels, tiles_m, tile_m, panel)) return;
-    gemm_core::run<F32Traits, 4>(a8, w8, K * 4, epi, y, M, N, K * 4 / gemm_core::BKB, tile_m * 256, panel * 256, lds);
-  } else {
-    const int64_t n_full = full_panels * 256;
-    if (!gemm_core::tile_of_even(blockIdx.x - uint32_t(full_blocks), gridDim.x - uint32_t(full_blocks), tiles_m, (N - n_full + 127) / 128,
-                                 tiles_m, tile_m, panel))
-      return;
-    gemm_core::run<F32Traits, 2>(a8, w8, K * 4, epi, y, M, N, K * 4 / gemm_core::BKB, tile_m * 256, n_full + panel * 128, lds);
-  }
-}
-
 // Epilogues of the any-shape tile loop (gemm_core::edge): the same sum + bias, one narrowing.
 template <typename X>
 struct EdgeBiasEpilogue {
@@ -235,15 +204,6 @@ struct RowsBiasF32Epilogue {
 };
 
 }  // namespace dense_cluster
-
-// f32 operands: (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N, full_panels) ; K % 32 == 0, x and w 16-byte aligned
-// and below 4 GiB each; tiles, grid and block as for the 16-bit kernels below.
-extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_dense_mfma_f32(
-    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
-    int64_t K, int64_t N, int64_t full_panels) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::LDS_BYTES];
-  dense_cluster::dense_mfma_f32_body(x, w, bias, y, M, K, N, full_panels, lds);
-}
 
 // (x [M,K], w [N,K], bias [N] or null, y [M,N], M, K, N, full_panels) ; K % 64 == 0, x and w 16-byte aligned and below
 // 4 GiB each; tiles and grid as mtrt_gemm_w8a8_nk (256 x 256 for the first full_panels * 256 columns, 256 x 128 after),
@@ -411,12 +371,19 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_rows8_wide_f32
 
 // Up to 32 rows, weights read once as whole rows (gemm_core::rows32): (x [M,K], w [N,K], bias or null, y, M <= 32, K, N) ;
 // rows in whole 128-byte slices, x and w 16-byte aligned; grid: any, block = 512.
+// f32: tiles != 0; or groups of eight rows on the vector units (dot::run, `form` as there), block = 256.
 extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows32_f32(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
-    int64_t K, int64_t N) {
+    int64_t K, int64_t N, int32_t tiles, int32_t form) {
   __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8>()];
-  dense_cluster::RowsBiasF32Epilogue epi{bias};
-  gemm_core::rows32::run<dense_cluster::F32Traits, 8>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);
+  if (tiles) {
+    dense_cluster::RowsBiasF32Epilogue epi{bias};
+    gemm_core::rows32::run<dense_cluster::F32Traits, 8>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);
+  } else if (form & 1) {
+    dense_cluster::dot::run<8, 4, 4, 2, false>(x, w, bias, y, M, K, N, reinterpret_cast<float*>(lds));
+  } else {
+    dense_cluster::dot::run<8, 4, 1, 2, false>(x, w, bias, y, M, K, N, reinterpret_cast<float*>(lds));
+  }
 }
 #define MTRT_DENSE_ROWS32_KERNEL(XN, XT)                                                                           \
   extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows32_##XN(                                   \
@@ -429,14 +396,23 @@ extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows32_f32(
   }
 MTRT_DENSE_ROWS32_KERNEL(f16, F16)
 MTRT_DENSE_ROWS32_KERNEL(bf16, BF16)
+// f32, more rows (x, w, bias, y, M, K, N): 32 x 32 tiles, K shared by eight waves (any M; rows64 and rows128 differ in name only), or, _tall,
+// the rows against each weight fragment at once; grid: any, block = 512 (rows128_tall: 256).  The matrix cores set the time of a tile
+// column with all its rows (0.18 us to a 128-byte slice of K for every 32 rows), so it is the faster one only where the columns alone
+// fill the chip and K is short: us, so and in tiles, (100, 512, 8192) 17.3 and 18.2, (40, 256, 16384) 12.3 and 12.8, (64, 4096, 4096) 44.9 and 25.6,
+// (109, 3072, 448) 62.7 and 19.2, (128, 4096, 1024) 82.7 and 23.8.
+#define MTRT_DENSE_ROWS_F32_KERNEL(NAME, WAVES, MT, MANY)                                                          \
+  extern "C" __global__ void __launch_bounds__(64 * WAVES) mtrt_gemm_dense_##NAME##_f32(                           \
+      const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M, \
+      int64_t K, int64_t N) {                                                                                      \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<WAVES, MT>()];                 \
+    dense_cluster::RowsBiasF32Epilogue epi{bias};                                                                  \
+    gemm_core::rows32::run<dense_cluster::F32Traits, WAVES, MT, false, MANY>(                                      \
+        reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);         \
+  }
 // ... and up to 64 rows: two activation row tiles against each weight fragment
-extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows64_f32(
-    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
-    int64_t K, int64_t N) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8, 2>()];
-  dense_cluster::RowsBiasF32Epilogue epi{bias};
-  gemm_core::rows32::run<dense_cluster::F32Traits, 8, 2>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);
-}
+MTRT_DENSE_ROWS_F32_KERNEL(rows64, 8, 1, true)
+MTRT_DENSE_ROWS_F32_KERNEL(rows64_tall, 8, 2, false)
 #define MTRT_DENSE_ROWS64_KERNEL(XN, XT)                                                                           \
   extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows64_##XN(                                   \
       const XT::storage* __restrict__ x, const XT::storage* __restrict__ w, const XT::storage* __restrict__ bias,  \
@@ -449,13 +425,8 @@ extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_rows64_f32(
 MTRT_DENSE_ROWS64_KERNEL(f16, F16)
 MTRT_DENSE_ROWS64_KERNEL(bf16, BF16)
 // ... and up to 128 rows: four row tiles, four waves (block = 256)
-extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_rows128_f32(
-    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
-    int64_t K, int64_t N) {
-  __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<4, 4>()];
-  dense_cluster::RowsBiasF32Epilogue epi{bias};
-  gemm_core::rows32::run<dense_cluster::F32Traits, 4, 4>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);
-}
+MTRT_DENSE_ROWS_F32_KERNEL(rows128, 8, 1, true)
+MTRT_DENSE_ROWS_F32_KERNEL(rows128_tall, 4, 4, false)
 #define MTRT_DENSE_ROWS128_KERNEL(XN, XT)                                                                          \
   extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_rows128_##XN(                                  \
       const XT::storage* __restrict__ x, const XT::storage* __restrict__ w, const XT::storage* __restrict__ bias,  \
@@ -467,6 +438,13 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_dense_rows128_f32(
   }
 MTRT_DENSE_ROWS128_KERNEL(f16, F16)
 MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
+
+// ... and where the tiles are more than the compute units: four waves, four workgroups to a unit; grid: any, block = 256.  Bound by the
+// matrix cores (a 32 x 32 x 2 instruction every 64 cycles: 157 TFLOP/s nominal) where the tiles fill the chip, by the walk down K where they
+// do not.  Tiles of 256 x 256 and 256 x 128, which this took before, left most of the chip idle and held 256 registers a lane: us,
+// (M, K, N), those and these: (200, 1024, 1024) 131 and 8.8, (300, 3072, 2048) 366 and 49, (512, 4096, 4096) 482 and 172,
+// (2048, 2048, 2048) 253 and 164, (768, 1024, 11008) 274 and 182, (2048, 512, 8192) 211 and 207, (4096, 1024, 1024) 142 and 89.
+MTRT_DENSE_ROWS_F32_KERNEL(mfma, 4, 1, true)
 
 // ---- weights in fragment order (gemm_frag.hpp) ---------------------------------------------------------
 // What a module's Linear runs on: its weights are re-laid once per parameter set.  Against the loops above, which bring both
@@ -722,9 +700,9 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_w16_prepack_frag(const ui
     const int64_t row_bytes = K * int64_t(sizeof(XT::storage));                                                    \
     dense_cluster::ROWS rows_epi{bias};                                                                            \
     if (waves == 8) {                                                                                              \
-      gemm_core::rows32::run<dense_cluster::TRAITS, 8, 1, false, true>(x8, w8, row_bytes, rows_epi, y, M, N, lds); \
+      gemm_core::rows32::run<dense_cluster::TRAITS, 8, 1, false, true, true>(x8, w8, row_bytes, rows_epi, y, M, N, lds); \
     } else if (waves == 4) {                                                                                       \
-      gemm_core::rows32::run<dense_cluster::TRAITS, 4, 1, false, true>(x8, w8, row_bytes, rows_epi, y, M, N, lds); \
+      gemm_core::rows32::run<dense_cluster::TRAITS, 4, 1, false, true, true>(x8, w8, row_bytes, rows_epi, y, M, N, lds); \
     } else {                                                                                                       \
       dense_cluster::EDGE epi{bias};                                                                               \
       gemm_core::edge::run<dense_cluster::TRAITS>(x8, w8, row_bytes, epi, y, M, N, lds);                           \

@@ -53,6 +53,10 @@ constexpr double kDotGroupBytesPerUs = 7.5e6;
 // waves to a compute unit (f32, up to one workgroup a unit: eight waves).  Fitted to 34 products, M 1 ... 2000, K 6 ... 12287, N 7 ... 11000,
 // f32 and f16; the faster form is taken in each of them.
 constexpr double kEdgeFixedUs = 4.0, kEdgeF32StepUs = 2.45, kEdge16StepUs = 1.2;
+// f32 products of whole slices, by rounds of 32-column tiles with all rows (up to 32, 64 and 128 of them) and by 32 x 32 tiles, two to a compute
+// unit: us to a slice of 128 bytes of K.  Fitted to 27 products, M 16 ... 4096, K 256 ... 12288, N 256 ... 16384.
+constexpr double kF32FixedUs = 3.0, kF32Rows32StepUs = 0.18, kF32Rows64StepUs = 0.36, kF32Rows128StepUs = 0.68;
+constexpr double kF32FewTilesStepUs = 0.2, kF32LaterUs = 2.0, kF32TilesStepUs = 0.4;
 constexpr double kEdgeSmallFixedUs = 3.0, kEdgeSmallFewStepUs = 0.2, kEdgeSmallStepUs = 0.5;
 // W4A16 tile choice: a full round of 256 x 256 tiles takes 3.25 times a full round of 128 x 128 tiles (for four times
 // the work), and a last round filled to a fraction f of the units takes 0.56 + 0.44 f^2 of a full one (fewer units
@@ -1232,20 +1236,42 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   const bool few = dtype == MTRT_F32 && K >= 4 && K * N >= tuning::kDotMinWeights && N <= tuning::kDotMaxColumns;
   if (few && M <= 8)
     return dense_few_rows_f32(st, as_hip(stream), x, w_nk, bias, y, M, K, N);
-  // Decode-sized calls are bound by reading the weights once: up to 32 rows take one workgroup per 32 weight rows, its
-  // eight waves splitting K (f16 M = 16, K = 4096, N = 11008: 55 us on the tile loop, 23.3 so, 3.9 TB/s of weights; f32
-  // 473 -> 50 us); 33 to 64 rows the form with two activation row tiles per weight fragment; the tile loop (about
-  // 8 us + 6 ns per byte of a row, per round) only wins on very large weights.
+  const int64_t tiles32 = (N + 31) / 32, units = num_compute_units(st), small_tiles = ((M + 31) / 32) * tiles32;
   const bool whole_slices = K > 0 && (K * eb) % 128 == 0 && aligned(x, 16) && aligned(w_nk, 16);
+  if (whole_slices && dtype == MTRT_F32) {
+    // In 32 x 32 tiles, or up to 128 rows a column tile's rows together, or up to 32 on the vector units in groups of eight.
+    const double steps = double(K * eb / 128), rounds = double((tiles32 + units - 1) / units);
+    const double rows_us = tuning::kF32FixedUs + rounds * steps * (M <= 32 ? tuning::kF32Rows32StepUs : M <= 64 ? tuning::kF32Rows64StepUs : tuning::kF32Rows128StepUs);
+    const double tiles_us = tuning::kF32FixedUs + (small_tiles <= units ? steps * tuning::kF32FewTilesStepUs
+                                                                        : tuning::kF32LaterUs + steps * tuning::kF32TilesStepUs * std::max(1.0, double(small_tiles) / double(2 * units)));
+    const uint32_t most = uint32_t(kMaxGrid) * 1024;
+    if (M > 32) {
+      // eight waves to a tile while there is a unit for each and (128 rows or more) K gives them slices; four beyond
+      const bool tall = M <= 128 && rows_us <= tiles_us, eight = small_tiles <= units && (M <= 128 || K >= 256);
+      void *rargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
+      return launch(st, KernelName(tall ? (M <= 64 ? "mtrt_gemm_dense_rows64_tall_f32" : "mtrt_gemm_dense_rows128_tall_f32") :
+                                   !eight ? "mtrt_gemm_dense_mfma_f32" : M <= 64 ? "mtrt_gemm_dense_rows64_f32" : "mtrt_gemm_dense_rows128_f32"),
+                    uint32_t(std::min<int64_t>(tall ? tiles32 : 8 * ((small_tiles + 7) / 8), most)), tall ? (M <= 64 ? 512 : 256) : eight ? 512 : 256,
+                    as_hip(stream), rargs);
+    }
+    const int64_t groups = (M + 7) / 8;
+    int32_t as_tiles = !few || rows_us < tuning::kF32FixedUs + double(groups) * double(K * N * 4) / tuning::kDotGroupBytesPerUs;
+    int32_t form = K >= tuning::kDotOwnColumnsBelow || (N + 15) / 16 * groups < units;   // as in dense_few_rows_f32
+    const int64_t columns = form ? 4 : 16;
+    void *fargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &as_tiles, &form};
+    return launch(st, KernelName("mtrt_gemm_dense_rows32_f32"), uint32_t(as_tiles ? std::min<int64_t>(tiles32, most) : 8 * (((N + columns - 1) / columns + 7) / 8) * groups),
+                  as_tiles ? 512 : kBlock, as_hip(stream), fargs);
+  }
+  // 16-bit.  Decode-sized calls are bound by reading the weights once: up to 32 rows take one workgroup per 32 weight rows, its
+  // eight waves splitting K (f16 M = 16, K = 4096, N = 11008: 55 us on the tile loop, 23.3 so, 3.9 TB/s of weights); 33 to 64 rows the form with two activation row tiles per weight fragment; the tile loop (about
+  // 8 us + 6 ns per byte of a row, per round) only wins on very large weights.
   const double tile_us = (tuning::kTileFixedUs + tuning::kTileUsPerRowByte * double(K * eb)) *
                          double(((N + 255) / 256 + num_compute_units(st) - 1) / num_compute_units(st));
   const double small_us = tuning::kRowsFixedUs + double(N) * double(K * eb) / tuning::kRowsWideBytesPerUs;
-  const int64_t tiles32 = (N + 31) / 32;
-  // 65 to 128 rows: four row tiles per weight fragment, rounds of one workgroup per compute unit (3.7 ns per byte of a row);
-  // f32 operands are bound by their matrix instructions there, which the tile loop is as well, at eight times the rows
+  // 65 to 128 rows: four row tiles per weight fragment, rounds of one workgroup per compute unit (3.7 ns per byte of a row)
   const double mid_us = tuning::kRows128FixedUs + tuning::kRows128UsPerRowByte * double(K * eb) *
                                                       double((tiles32 + num_compute_units(st) - 1) / num_compute_units(st));
-  if (whole_slices && (M <= 64 ? small_us < tile_us : M <= 128 && (dtype == MTRT_F32 || mid_us < tile_us))) {
+  if (whole_slices && (M <= 64 ? small_us < tile_us : M <= 128 && mid_us < tile_us)) {
     void *rargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
     return launch(st, KernelName(M <= 32 ? "mtrt_gemm_dense_rows32_" : M <= 64 ? "mtrt_gemm_dense_rows64_" : "mtrt_gemm_dense_rows128_") + xn,
                   uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), M <= 64 ? 512 : 256, as_hip(stream), rargs);
@@ -1253,8 +1279,8 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   if (K > 0 && (K * eb) % 128 == 0 && aligned(x, 16) && aligned(w_nk, 16) && M * K * eb < (int64_t(1) << 32) &&
       N * K * eb < (int64_t(1) << 32)) {
     // operands in whole 128-byte slices of K: the matrix-core tile loop (tiles and rounds as in
-    // mtrt_hip_gemm_w8a8; f16 [2048, 4096] x [11008, 4096]: 3654 us on the FMA kernel below, f32 3835 us)
-    const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256, units = num_compute_units(st);
+    // mtrt_hip_gemm_w8a8; f16 [2048, 4096] x [11008, 4096]: 3654 us on the FMA kernel below)
+    const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256;
     const int64_t tiles256 = panels * tiles_m, rest = tiles256 % units;
     int64_t full_panels = panels;
     if (tiles256 * 2 <= units)
@@ -1272,7 +1298,7 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   if (K > 0) {
     // any other K or alignment: element-aligned loads and a zero-padded last k-step, in 128 x 128 tiles
     // (f16 [2048, 4100] x [11008, 4100]: 3761 us on the FMA kernel below) or 32 x 32 ones whose K the waves share
-    const int64_t edge_tiles = ((M + 127) / 128) * ((N + 127) / 128), small_tiles = ((M + 31) / 32) * tiles32, units = num_compute_units(st);
+    const int64_t edge_tiles = ((M + 127) / 128) * ((N + 127) / 128);
     const double steps = double((K * eb + 127) / 128);
     const double edge_us = tuning::kEdgeFixedUs + steps * (dtype == MTRT_F32 ? tuning::kEdgeF32StepUs : tuning::kEdge16StepUs) *
                                                       double((edge_tiles + units - 1) / units);
@@ -1286,7 +1312,7 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
     if (K * eb >= 16 && small_us < edge_us)
       waves = dtype == MTRT_F32 && small_tiles <= units ? 8 : 4;
     void *eargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &waves};
-    return launch(st, KernelName("mtrt_gemm_dense_edge_") + xn, uint32_t(std::min<int64_t>(waves ? small_tiles : edge_tiles, int64_t(kMaxGrid) * 1024)),
+    return launch(st, KernelName("mtrt_gemm_dense_edge_") + xn, uint32_t(std::min<int64_t>(waves ? 8 * ((small_tiles + 7) / 8) : edge_tiles, int64_t(kMaxGrid) * 1024)),
                   waves ? uint32_t(64 * waves) : kBlock, as_hip(stream), eargs);
   }
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);

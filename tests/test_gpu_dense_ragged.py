@@ -82,3 +82,32 @@ def test_infinities_stay_in_their_row(pkg, dname):
         ref = torch.full((M, N), float(K), dtype=td, device="cuda").float()
         ref[3], ref[:, 7], ref[3, 7], ref[5] = float("inf"), float("-inf"), float("-inf"), float("nan")
         assert torch.equal(torch.nan_to_num(y, nan=-1.0), torch.nan_to_num(ref, nan=-1.0)), (M, K, N)
+
+
+@pytest.mark.parametrize("M", [9, 32, 33, 64, 65, 128, 129, 257])
+def test_whole_slices_of_float32(pkg, M):
+    """K in whole 128-byte slices, fewer and more of them than the waves that share them; columns around tiles; products whose
+    tiles are fewer and more than the compute units, and whose columns alone are (the form that takes all rows at once)."""
+    import torch
+    kernels = set()
+    for i, (K, N) in enumerate(((32, 33), (64, 8193), (224, 31), (256, 1000), (288, 16385), (512, 8200), (1056, 2049), (4128, 65))):
+        g = torch.Generator(device="cuda").manual_seed(100 * M + i)
+        x = torch.randn((M, K), generator=g, device="cuda")
+        w = torch.randn((N, K), generator=g, device="cuda") * 0.3
+        b = torch.randn(N, generator=g, device="cuda") if i % 2 else None
+        out = torch.full((M * N + 128,), 7.0, device="cuda")
+        y = pkg.linear_dense(x, w, b, out[64:64 + M * N].view(M, N))
+        kernels.add(pkg.last_kernel())
+        xd, wd = x.double(), w.double()
+        bd = b.double() if b is not None else torch.zeros(N, dtype=torch.float64, device="cuda")
+        ref, mass = xd @ wd.T + bd, xd.abs() @ wd.abs().T + bd.abs()
+        bad = int(((y.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * mass).logical_not().sum())
+        assert bad == 0, (M, K, N, bad)
+        assert bool((out[:64] == 7).all()) and bool((out[64 + M * N:] == 7).all())
+    if M <= 32:
+        assert kernels == {"mtrt_gemm_dense_rows32_f32"}
+    elif M <= 128:
+        rows = "mtrt_gemm_dense_rows%d" % (64 if M <= 64 else 128)
+        assert {rows + "_f32", rows + "_tall_f32"} <= kernels
+    else:
+        assert kernels == {"mtrt_gemm_dense_rows128_f32", "mtrt_gemm_dense_mfma_f32"}
