@@ -38,6 +38,9 @@ using namespace qdq_cluster;
 using namespace amax_cluster;
 
 constexpr int kDynThreads = 1024;
+// Workgroups up to which each takes the maximum of the whole tensor by itself (64 KB a workgroup at four vectors a lane): us, with the
+// exchange and so, one workgroup (f32 [3, 1000]) 3.1, 2.5, two (bf16 [31, 1344]) 6.0, 5.5, three (bf16 [64, 1344]) 6.1, 6.25, four 5.2, 5.3.
+constexpr uint32_t kReadAll = 2;
 constexpr uint32_t kSlotLine = 33, kSlots = 256, kTagLine = 49;
 
 __device__ __forceinline__ uint32_t block_max(uint32_t m, uint32_t* wave_max) {
@@ -67,8 +70,14 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
 
   unsigned long long* slots = reinterpret_cast<unsigned long long*>(scratch + kAmaxLineWords * kSlotLine);
   uint32_t* tag_word = scratch + kAmaxLineWords * kTagLine;
+  // (results that lie over x, in place, must not be written before the others have read it)
+  const auto apart = [&](const void* p, int64_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p), b = reinterpret_cast<uint64_t>(x);
+    return a + uint64_t(bytes) <= b || b + uint64_t(n) * sizeof(typename X::storage) <= a;
+  };
+  const bool read_all = gridDim.x <= kReadAll && apart(q, n) && (!y || apart(y, n * int64_t(sizeof(typename X::storage))));
   // asked for before the data, needed after it
-  const uint32_t tag = __hip_atomic_load(tag_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+  const uint32_t tag = read_all ? 0u : __hip_atomic_load(tag_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
 
   u32x4 xin[NV];
   uint32_t m = 0;
@@ -82,56 +91,75 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
       m = m > a ? m : a;
     }
   }
-  m = block_max(m, wave_max);
-
-  if (threadIdx.x < kWave) {                         // wave 0: publish, then watch the other slots
-    const uint32_t lane = threadIdx.x;
-    if (lane == 0)
-      __hip_atomic_store(slots + blockIdx.x, ((unsigned long long)tag << 32) | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint32_t total = m, have = 0;
-    for (int spin = 0; spin < spin_limit; ++spin) {
-      uint32_t mx = m;
-      bool ok = true;
+  uint32_t total;
+  if (read_all) {
+    // Few workgroups: each reads the others' parts as well instead of waiting for their maxima.
+    for (uint32_t other = 1; other < gridDim.x; ++other) {
+      const int64_t first = int64_t((blockIdx.x + other) % gridDim.x) * (kDynThreads * NV) + threadIdx.x;
+      u32x4 t[NV];
 #pragma unroll
-      for (uint32_t c = 0; c < kSlots / kWave; ++c) {
-        const uint32_t idx = lane + kWave * c;
-        if (idx < gridDim.x && idx != blockIdx.x) {  // the own slot is known without reading it back
-          const unsigned long long w = __hip_atomic_load(slots + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          ok = ok && uint32_t(w >> 32) == tag;
-          mx = mx > uint32_t(w) ? mx : uint32_t(w);
+      for (int i = 0; i < NV; ++i) {
+        const int64_t v = first + int64_t(i) * kDynThreads;
+        t[i] = *reinterpret_cast<const u32x4*>(x + (v < nvec ? v : nvec - 1) * G);
+      }
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const uint32_t a = A::of(t[i]);
+        m = m > a ? m : a;
+      }
+    }
+    total = block_max(m, wave_max);
+  } else {
+    m = block_max(m, wave_max);
+    if (threadIdx.x < kWave) {                       // wave 0: publish, then watch the other slots
+      const uint32_t lane = threadIdx.x;
+      if (lane == 0)
+        __hip_atomic_store(slots + blockIdx.x, ((unsigned long long)tag << 32) | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      uint32_t total = m, have = 0;
+      for (int spin = 0; spin < spin_limit; ++spin) {
+        uint32_t mx = m;
+        bool ok = true;
+#pragma unroll
+        for (uint32_t c = 0; c < kSlots / kWave; ++c) {
+          const uint32_t idx = lane + kWave * c;
+          if (idx < gridDim.x && idx != blockIdx.x) {  // the own slot is known without reading it back
+            const unsigned long long w = __hip_atomic_load(slots + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = ok && uint32_t(w >> 32) == tag;
+            mx = mx > uint32_t(w) ? mx : uint32_t(w);
+          }
         }
+        if (__ballot(ok) == __ballot(true)) {
+          total = wave_reduce(mx, MaxU32());
+          have = 1;
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
       }
-      if (__ballot(ok) == __ballot(true)) {
-        total = wave_reduce(mx, MaxU32());
-        have = 1;
-        break;
+      if (lane == 0) {
+        bcast[0] = have;
+        bcast[1] = total;
       }
-      __builtin_amdgcn_s_sleep(1);
     }
-    if (lane == 0) {
-      bcast[0] = have;
-      bcast[1] = total;
+    __syncthreads();
+    total = bcast[1];
+    if (bcast[0] == 0u) {
+      // gave up waiting: this workgroup reduces the whole tensor itself (max is exact in any order: same bits)
+      uint32_t mm = 0;
+      for (int64_t v = threadIdx.x; v < nvec; v += kDynThreads) {
+        const uint32_t a = A::of(FG::load(x + v * G));
+        mm = mm > a ? mm : a;
+      }
+      total = block_max(mm, wave_max);
     }
+    // Done with the slots: advance the tag counter for the next launch on this stream.  Every workgroup does it
+    // (a maximum, so it is idempotent) and none waits for an answer: 256 workgroups updating one line within a
+    // microsecond take the memory side up to 3 us to serve, and a lane that waited for its turn would hold its
+    // whole wave back.  The counter cannot move while a workgroup of this launch has yet to read it: nobody gets
+    // here before every slot carries the tag, and a workgroup publishes after it has read the counter.  (Unless
+    // somebody gave up waiting: a workgroup that starts after that reads the advanced counter, finds no slot with
+    // its tag, gives up in turn and computes the maximum itself; right, only slow, like every give-up.)
+    if (threadIdx.x == 0) __hip_atomic_fetch_max(tag_word, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  __syncthreads();
-  uint32_t total = bcast[1];
-  if (bcast[0] == 0u) {
-    // gave up waiting: this workgroup reduces the whole tensor itself (max is exact in any order: same bits)
-    uint32_t mm = 0;
-    for (int64_t v = threadIdx.x; v < nvec; v += kDynThreads) {
-      const uint32_t a = A::of(FG::load(x + v * G));
-      mm = mm > a ? mm : a;
-    }
-    total = block_max(mm, wave_max);
-  }
-  // Done with the slots: advance the tag counter for the next launch on this stream.  Every workgroup does it
-  // (a maximum, so it is idempotent) and none waits for an answer: 256 workgroups updating one line within a
-  // microsecond take the memory side up to 3 us to serve, and a lane that waited for its turn would hold its
-  // whole wave back.  The counter cannot move while a workgroup of this launch has yet to read it: nobody gets
-  // here before every slot carries the tag, and a workgroup publishes after it has read the counter.  (Unless
-  // somebody gave up waiting: a workgroup that starts after that reads the advanced counter, finds no slot with
-  // its tag, gives up in turn and computes the maximum itself; right, only slow, like every give-up.)
-  if (threadIdx.x == 0) __hip_atomic_fetch_max(tag_word, tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
   const float amax = A::finish(total);
   const float scale = amax / qmax;                   // one IEEE divide, as the host does it; identical in every workgroup
