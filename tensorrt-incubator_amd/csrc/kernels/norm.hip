@@ -34,6 +34,7 @@ constexpr int kRowsPerBlock = kNormThreads / kWave;
 template <typename X> struct Vec;     // one 128-bit vector <-> floats
 template <> struct Vec<F32> {
   static constexpr int kElems = 4;
+  static constexpr uint32_t kMinusInf = 0xFF800000u;   // in every element of a word
   static __device__ __forceinline__ void unpack(u32x4 t, float* v) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = bits_to_f32(t[j]);
@@ -47,6 +48,7 @@ template <> struct Vec<F32> {
 };
 template <> struct Vec<BF16> {
   static constexpr int kElems = 8;
+  static constexpr uint32_t kMinusInf = 0xFF80FF80u;
   static __device__ __forceinline__ void unpack(u32x4 t, float* v) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) { v[2 * j] = bits_to_f32(t[j] << 16); v[2 * j + 1] = bits_to_f32(t[j] & 0xFFFF0000u); }
@@ -60,6 +62,7 @@ template <> struct Vec<BF16> {
 };
 template <> struct Vec<F16> {
   static constexpr int kElems = 8;
+  static constexpr uint32_t kMinusInf = 0xFC00FC00u;
   static __device__ __forceinline__ void unpack(u32x4 t, float* v) {
 #pragma unroll
     for (int j = 0; j < 4; ++j) { v[2 * j] = f16_bits_to_f32(t[j] & 0xFFFFu); v[2 * j + 1] = f16_bits_to_f32(t[j] >> 16); }
@@ -259,7 +262,17 @@ __device__ __forceinline__ float group_reduce(float v, Op op, float* lds) {
   return r;                                          // the same value, combined in the same order, in every lane
 }
 
-template <typename X, int NV, int THREADS, bool FULL, bool RAGGED>
+// Whether vector j of any lane of this wave lies in the row (the same for the whole wave): what lies past it for all is not asked for, nor
+// worked on.  A row takes the kernel with the next power of two of vectors, so that may be near half of them.  us, before and after:
+// LayerNorm f16 [2000, 10240] 18.8, 17.2, [2000, 12001] 28.1, 26.5, [8000, 1500] 10.8, 10.1, f32 [4000, 5000] 33.6, 31.5; softmax f16
+// [4000, 9001] 36.2, 31.5, [2000, 20001] 40.6, 35.9, bf16 [1084, 43165] 64.0, 54.6; without it and the fill below, f32 rows of 16388 to
+// 32768 elements off whole vectors took twice the vectors too, for want of registers: [2000, 25001] 102, 76.9, [800, 18001] 41.5, 22.0.  ALL: every vector is worked on.
+template <int THREADS, bool ALL>
+__device__ __forceinline__ bool wave_has(int j, int nvec) {
+  return ALL || (THREADS > kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.x & ~63u)) : 0) + THREADS * j < nvec;
+}
+
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED>
 __device__ __forceinline__ void layernorm_group_row(const typename X::storage* __restrict__ x,
                                                     const typename X::storage* __restrict__ gamma,
                                                     const typename X::storage* __restrict__ beta,
@@ -273,9 +286,10 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
   u32x4 t[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
-    if (RAGGED && nvec == 0) t[j] = (u32x4){0u, 0u, 0u, 0u};   // a row shorter than one vector: only the scalar elements below
-    else t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+    if (!RAGGED || !ALL || nvec > 0)                   // (a row shorter than one vector: only the scalar elements below)
+      t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
   const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
   const int64_t ec = int64_t(nvec) * E + lane;
@@ -284,6 +298,7 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
   float sum = xe;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const bool live = FULL || lane + THREADS * j < nvec;
     float v[E];
     Vec<X>::unpack(t[j], v);
@@ -294,6 +309,7 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
   float sq = extra ? (xe - mu) * (xe - mu) : 0.0f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const bool live = FULL || lane + THREADS * j < nvec;
     float v[E];
     opaque(t[j]);                                    // widen again instead of keeping pass 1's values live
@@ -311,9 +327,10 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
   V* yr = reinterpret_cast<V*>(y + row * d);
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
     const int idc = FULL ? idx : min(idx, nvec - 1);
-    if (RAGGED && nvec == 0) continue;               // no whole vector: nothing to read or store here
+    if (RAGGED && ALL && nvec == 0) continue;          // no whole vector: nothing to read or store here
     float v[E], g[E], b[E], o[E];
     opaque(t[j]);
     Vec<X>::unpack(t[j], v);
@@ -347,14 +364,15 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
   if (!RAGGED && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-    layernorm_group_row<X, NV, THREADS, true, false>(x, gamma, beta, y, row, d, eps, lds);
-  else
-    layernorm_group_row<X, NV, THREADS, false, RAGGED>(x, gamma, beta, y, row, d, eps, lds);
+    layernorm_group_row<X, NV, THREADS, true, true, false>(x, gamma, beta, y, row, d, eps, lds);
+  else   // (ragged f32 rows: nearly full ones, [2000, 15001], 49.4 us with every vector worked on and 51.1 without)
+    layernorm_group_row<X, NV, THREADS, false, RAGGED && Vec<X>::kElems == 4, RAGGED>(x, gamma, beta, y, row, d, eps, lds);
 }
 
 // KEEP: the exponentials stay in registers (f32) between the sum and the output pass; without it they are
-// computed again from the stored row (the 1024-lane form has 128 registers per lane, not enough for both).
-template <typename X, int NV, int THREADS, bool FULL, bool KEEP, bool RAGGED>
+// computed again from the stored row (the 1024-lane form has 128 registers per lane, not enough for both where a lane holds
+// more than 64 elements).
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool KEEP, bool RAGGED>
 __device__ __forceinline__ void softmax_group_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                                   int64_t row, int64_t d, float* lds) {
   constexpr int E = Vec<X>::kElems;
@@ -365,9 +383,21 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   u32x4 t[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
-    if (RAGGED && nvec == 0) t[j] = (u32x4){0u, 0u, 0u, 0u};   // a row shorter than one vector: only the scalar elements below
-    else t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+    if (!RAGGED || !ALL || nvec > 0)                  // (a row shorter than one vector: only the scalar elements below)
+      t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+  }
+  // What lies past the row becomes -infinity where it is loaded: it changes no maximum and its exponential is zero, and the passes
+  // below need not tell it from the row (us, f16 [1084, 50000] 61.5 -> 53.7, f32 [2000, 25001] 102 -> 97; [48000, 1500] 51.1 -> 50.6, bf16 [200, 8191] 7.4 -> 7.0).
+  if (!FULL) {
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+      if (!wave_has<THREADS, ALL>(j, nvec)) break;
+      const bool live = lane + THREADS * j < nvec;
+#pragma unroll
+      for (int k = 0; k < 4; ++k) t[j][k] = live ? t[j][k] : Vec<X>::kMinusInf;
+    }
   }
   const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
   const int64_t ec = int64_t(nvec) * E + lane;
@@ -375,11 +405,11 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   float mx = xe;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const bool live = FULL || lane + THREADS * j < nvec;
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     float v[E];
     Vec<X>::unpack(t[j], v);
 #pragma unroll
-    for (int k = 0; k < E; ++k) mx = fmaxf(mx, live ? v[k] : -INFINITY);
+    for (int k = 0; k < E; ++k) mx = fmaxf(mx, v[k]);
   }
   mx = group_reduce<THREADS>(mx, MaxF32(), lds);
   float e[KEEP ? NV * E : 1];
@@ -387,13 +417,13 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   float s = ee;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    const bool live = FULL || lane + THREADS * j < nvec;
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     float v[E];
     opaque(t[j]);
     Vec<X>::unpack(t[j], v);
 #pragma unroll
     for (int k = 0; k < E; ++k) {
-      const float ev = live ? __expf(v[k] - mx) : 0.0f;
+      const float ev = __expf(v[k] - mx);
       if (KEEP) e[j * E + k] = ev;
       s = s + ev;
     }
@@ -403,6 +433,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   V* yr = reinterpret_cast<V*>(y + row * d);
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
+    if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
     float o[E];
     if (KEEP) {
@@ -424,13 +455,15 @@ template <typename X, int NV, int THREADS, bool RAGGED>
 __device__ __forceinline__ void softmax_group(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                               int64_t rows, int64_t d) {
   __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
-  constexpr bool kKeep = THREADS <= 256;
+  // (the branches cost a wave per row more than they save, f16 [48000, 1500] 50.6 and 53.9 us, and f32 in 256 lanes, [2000, 6001] 18.0 and 18.7)
+  constexpr bool kEnds = THREADS > (Vec<X>::kElems == 4 ? 256 : kWave);
+  constexpr bool kKeep = THREADS <= 256 || NV * Vec<X>::kElems <= 64;
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
   if (!RAGGED && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-    softmax_group_row<X, NV, THREADS, true, kKeep, false>(x, y, row, d, lds);
+    softmax_group_row<X, NV, THREADS, true, true, kKeep, false>(x, y, row, d, lds);
   else
-    softmax_group_row<X, NV, THREADS, false, kKeep, RAGGED>(x, y, row, d, lds);
+    softmax_group_row<X, NV, THREADS, false, !kEnds, kKeep, RAGGED>(x, y, row, d, lds);
 }
 
 // ---- any D, any alignment: one workgroup per row, row re-read from cache -------------

@@ -396,14 +396,10 @@ int32_t pick_nv(int64_t nvec_per_row) {
   return 0;
 }
 
-// Some element-aligned (`_u`) kernels on f32 rows with eight vectors per lane come out of the compiler badly: the
-// LayerNorm ones with 230 registers per lane (one wave per SIMD: f32 [4096, 8190] took 114 us against softmax's 45),
-// the 1024-lane ones of both families with 1.4 KB of scratch memory per lane (whose allocation costs a launch some
-// 10 us).  Their 16-vector forms take under 130 registers and no scratch, so those rows use them (a lane past the
-// end of the row holds nothing).
-int unaligned_nv(int32_t dtype, int nv, int lanes, bool layernorm) {
-  return dtype == MTRT_F32 && nv == 8 && (layernorm || lanes == 1024) ? 16 : nv;
-}
+// The element-aligned (`_u`) LayerNorm kernels on f32 rows with eight vectors per lane come out of the compiler with 230 registers per
+// lane (one wave per SIMD: f32 [4096, 8190] took 114 us against softmax's 45).  Their 16-vector forms take under 130, so those rows use
+// them (a lane past the end of the row holds nothing).
+int unaligned_nv(int32_t dtype, int nv, bool layernorm) { return dtype == MTRT_F32 && nv == 8 && layernorm ? 16 : nv; }
 
 // Rows too long for one wave: a workgroup of 256 or 1024 lanes with 8 or 16 vectors per lane owns the row.
 // Returns false when the row is longer than 1024 * 16 vectors.
@@ -925,11 +921,11 @@ int32_t mtrt_hip_layernorm(mtrt_stream_t stream, const void *x, const void *gamm
   if (!vec_ok && d >= per_vec) {
     int rnv = pick_nv(d / per_vec);
     if (rnv && rows <= kMaxRowsPerWaveKernels) {
-      rnv = unaligned_nv(dtype, rnv, 64, true);
+      rnv = unaligned_nv(dtype, rnv, true);
       return launch(st, KernelName("mtrt_layernorm_") + xn + "_u64v" + rnv, blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
     }
     if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-      return launch(st, KernelName("mtrt_layernorm_") + xn + "_u" + threads + "v" + unaligned_nv(dtype, gnv, threads, true), uint32_t(rows), uint32_t(threads),
+      return launch(st, KernelName("mtrt_layernorm_") + xn + "_u" + threads + "v" + unaligned_nv(dtype, gnv, true), uint32_t(rows), uint32_t(threads),
                     as_hip(stream), args);
   }
   return launch(st, KernelName("mtrt_layernorm_") + xn + "_any",
@@ -978,11 +974,11 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
   if (!vec_ok && d >= per_vec) {
     int rnv = pick_nv(d / per_vec);
     if (rnv && rows <= kMaxRowsPerWaveKernels) {
-      rnv = unaligned_nv(dtype, rnv, 64, false);
+      rnv = unaligned_nv(dtype, rnv, false);
       return launch(st, KernelName("mtrt_softmax_") + xn + "_u64v" + rnv, blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
     }
     if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + unaligned_nv(dtype, gnv, threads, false), uint32_t(rows), uint32_t(threads),
+      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + unaligned_nv(dtype, gnv, false), uint32_t(rows), uint32_t(threads),
                     as_hip(stream), args);
   }
   return launch(st, KernelName("mtrt_softmax_") + xn + "_any",
