@@ -38,9 +38,6 @@ using namespace qdq_cluster;
 using namespace amax_cluster;
 
 constexpr int kDynThreads = 1024;
-// Workgroups up to which each takes the maximum of the whole tensor by itself (64 KB a workgroup at four vectors a lane): us, with the
-// exchange and so, one workgroup (f32 [3, 1000]) 3.1, 2.5, two (bf16 [31, 1344]) 6.0, 5.5, three (bf16 [64, 1344]) 6.1, 6.25, four 5.2, 5.3.
-constexpr uint32_t kReadAll = 2;
 constexpr uint32_t kSlotLine = 33, kSlots = 256, kTagLine = 49;
 
 __device__ __forceinline__ uint32_t block_max(uint32_t m, uint32_t* wave_max) {
@@ -70,14 +67,8 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
 
   unsigned long long* slots = reinterpret_cast<unsigned long long*>(scratch + kAmaxLineWords * kSlotLine);
   uint32_t* tag_word = scratch + kAmaxLineWords * kTagLine;
-  // (results that lie over x, in place, must not be written before the others have read it)
-  const auto apart = [&](const void* p, int64_t bytes) {
-    const uint64_t a = reinterpret_cast<uint64_t>(p), b = reinterpret_cast<uint64_t>(x);
-    return a + uint64_t(bytes) <= b || b + uint64_t(n) * sizeof(typename X::storage) <= a;
-  };
-  const bool read_all = gridDim.x <= kReadAll && apart(q, n) && (!y || apart(y, n * int64_t(sizeof(typename X::storage))));
   // asked for before the data, needed after it
-  const uint32_t tag = read_all ? 0u : __hip_atomic_load(tag_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
+  const uint32_t tag = __hip_atomic_load(tag_word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u;
 
   u32x4 xin[NV];
   uint32_t m = 0;
@@ -92,7 +83,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
     }
   }
   uint32_t total;
-  if (read_all) {
+  if (spin_limit < 0) {
     // Few workgroups: each reads the others' parts as well instead of waiting for their maxima.
     for (uint32_t other = 1; other < gridDim.x; ++other) {
       const int64_t first = int64_t((blockIdx.x + other) % gridDim.x) * (kDynThreads * NV) + threadIdx.x;
@@ -189,7 +180,8 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
 
 // (x, q, y or null, n, qmax, amax_out or null, scale_out or null, scratch, flags, spin_limit)
 //   n % G == 0 (G = 4 for f32, 8 for f16 / bf16), x and y 16-byte aligned, q aligned to G codes,
-//   gridDim.x = ceil(n / G / (1024 * NV)) <= min(number of compute units, 256), block = 1024.
+//   gridDim.x = ceil(n / G / (1024 * NV)) <= min(number of compute units, 256), block = 1024;
+//   spin_limit < 0: every workgroup takes the maximum of the whole tensor by itself (q and y must then not lie over x).
 #define MTRT_DYNQ_KERNEL(XN, XT, QN, QT, NV)                                                                          \
   extern "C" __global__ void __launch_bounds__(1024) mtrt_dynqdq_##XN##_##QN##_v##NV(                                  \
       const XT::storage* x, QT::storage* q, XT::storage* y, int64_t n, float qmax, float* amax_out, float* scale_out,  \
