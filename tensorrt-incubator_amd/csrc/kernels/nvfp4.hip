@@ -19,6 +19,7 @@
 // its codes (1 or 2 KiB) and block scales (128 or 256 B) are parked in the wave's own LDS region
 // and written out as whole cache lines, 16 bytes per lane.
 #include "common.hpp"
+#include "nvfp4_index.hpp"
 
 namespace nvfp4_cluster {
 
@@ -251,7 +252,7 @@ __device__ __forceinline__ void quantize_cols_body(const typename X::storage* __
   constexpr int G = FloatGroup<X>::G;
   constexpr int R = 4;                                 // rows per lane
   __shared__ float inverse_scale[256];
-  const uint32_t groups = uint32_t(d1 / G), units = uint32_t((d0 / 16) * groups);   // below 2^32 for anything that fits in memory
+  const uint32_t groups = uint32_t(d1 / G), units = uint32_t((d0 / 16) * groups);   // 2^32 units are a TiB of x: more than there is
   const uint32_t part = (threadIdx.x >> 4) & 3;
   uint32_t u = blockIdx.x * (kThreads / 4) + (threadIdx.x >> 6) * 16 + (threadIdx.x & 15);
   u = u < units ? u : units - 1;                       // past the end: the last unit once more, which stores the same bytes
@@ -324,18 +325,17 @@ __device__ __forceinline__ void quantize_cols_body(const typename X::storage* __
 }
 
 // (q_packed, scales, tensor_amax, y, d0, d1) ; one lane per output vector
-template <typename Y>
+template <typename Y, bool NARROW>
 __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__ q, const uint8_t* __restrict__ scales,
                                                      const float* __restrict__ tensor_amax,
                                                      typename Y::storage* __restrict__ y, int64_t d0, int64_t d1) {
   constexpr int G = FloatGroup<Y>::G;
-  const int64_t groups = d1 / G, nvec = d0 * groups;   // groups and nvec are below 2^32 for anything that fits in memory
+  const int64_t nvec = d0 * (d1 / G);
   const float s_dec = *tensor_amax / 2688.0f;
   const int64_t stride = int64_t(gridDim.x) * kThreads;
   for (int64_t v = int64_t(blockIdx.x) * kThreads + threadIdx.x; v < nvec; v += stride) {
-    const int64_t r = uint32_t(v) / uint32_t(groups), c0 = (v - r * groups) * G;
     const uint32_t codes = G == 4 ? uint32_t(*reinterpret_cast<const uint16_t*>(q + v * 2)) : *reinterpret_cast<const uint32_t*>(q + v * 4);
-    const uint8_t* sp = scales + (r / 16) * d1 + c0;
+    const uint8_t* sp = scales + scale_of_vector<NARROW, G>(v, d1);
     uint32_t sw[2];
     sw[0] = *reinterpret_cast<const uint32_t*>(sp);
     sw[1] = G == 8 ? *reinterpret_cast<const uint32_t*>(sp + 4) : 0u;
@@ -371,7 +371,8 @@ __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__
     nvfp4_cluster::dequantize_body<XT>(q, scales, tensor_amax, y, nvec);                                                \
   }
 // Blocks along the second-to-last axis: mtrt_nvfp4_qc_<t>(x, q_packed, scales, tensor_amax, d0, d1) with
-// grid = ceil((d0 / 16) * (d1 / G) / 64); mtrt_nvfp4_dqc_<t>(q_packed, scales, tensor_amax, y, d0, d1).
+// grid = ceil((d0 / 16) * (d1 / G) / 64); mtrt_nvfp4_dqc_<t>(q_packed, scales, tensor_amax, y, d0, d1), below 2^32 vectors, and
+// mtrt_nvfp4_dqc_far_<t>, any number of them: grid: any.  (Both divisions in one kernel, whichever way, cost every launch 0.25 us.)
 // d1 % G == 0 (G = 4 for f32, 8 for f16 / bf16), x / y rows 16-byte aligned, scales 4- (G = 4) or 8-byte aligned.
 #define MTRT_NVFP4_COL_KERNELS(XN, XT)                                                                                  \
   extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_qc_##XN(                              \
@@ -380,7 +381,11 @@ __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__
   }                                                                                                                     \
   extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_dqc_##XN(                             \
       const uint8_t* q, const uint8_t* scales, const float* tensor_amax, XT::storage* y, int64_t d0, int64_t d1) {      \
-    nvfp4_cluster::dequantize_cols_body<XT>(q, scales, tensor_amax, y, d0, d1);                                         \
+    nvfp4_cluster::dequantize_cols_body<XT, true>(q, scales, tensor_amax, y, d0, d1);                                   \
+  }                                                                                                                     \
+  extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_dqc_far_##XN(                         \
+      const uint8_t* q, const uint8_t* scales, const float* tensor_amax, XT::storage* y, int64_t d0, int64_t d1) {      \
+    nvfp4_cluster::dequantize_cols_body<XT, false>(q, scales, tensor_amax, y, d0, d1);                                  \
   }
 MTRT_NVFP4_COL_KERNELS(f32, mtrt_dev::F32)
 MTRT_NVFP4_COL_KERNELS(f16, mtrt_dev::F16)

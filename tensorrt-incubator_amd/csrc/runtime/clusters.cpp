@@ -7,6 +7,7 @@
 // (mlir-tensorrt/compiler/lib/Passes/1_Core/KernelToCUDA/KernelToCUDA.cpp:151-186;
 //  mlir-tensorrt/compiler/lib/Passes/2_Host/HostToExecutor/CUDAToExecutor/CUDAToExecutor.cpp:355-413).
 #include "runtime_internal.hpp"
+#include "../kernels/nvfp4_index.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -854,7 +855,7 @@ int32_t nvfp4_dispatch(bool quantize, hipStream_t stream, const void *xy, int32_
     }
     void *args[] = {&q, &scales, &tensor_amax, &xy, &d0, &d1};
     const int64_t blocks = std::min<int64_t>((units + kBlock - 1) / kBlock, int64_t(num_compute_units(st)) * 64);
-    return launch(st, KernelName("mtrt_nvfp4_dqc_") + xn, uint32_t(blocks), kBlock, stream, args);
+    return launch(st, KernelName(nvfp4_cluster::numbers_fit(units) ? "mtrt_nvfp4_dqc_" : "mtrt_nvfp4_dqc_far_") + xn, uint32_t(blocks), kBlock, stream, args);
   }
   int64_t nvec = n / group;
   const int64_t per_block = 4 * 64 * (quantize ? 8 : 2);   // 4 waves x 64 lanes x kTrips or kDqTrips vectors

@@ -177,3 +177,13 @@ def test_the_shapes_that_test_every_tile_take_it(gpu, pkg, family, tiles):
     for shape, tile, split in tiles:
         name, _, s = call(*shape)
         assert (name, s is not None and s[0] > 1) == ("mtrt_gemm_%s_%s" % (family, tile), bool(split)), shape
+
+
+@pytest.mark.parametrize("dtype,vector", [("F32", 4), ("F16", 8), ("BF16", 8)])
+def test_tensors_of_64_gib_are_divided_in_64_bits(gpu, pkg, dtype, vector):
+    for d0, d1 in ((1 << 16, vector << 16), (16, vector << 28), (((1 << 32) // 4099 + 16) // 16 * 16, vector * 4099)):
+        for rows, far in ((d0 - 16, False), (d0, True)):
+            assert (rows * (d1 // vector) >= 1 << 32) == far
+            if rows:
+                assert gpu.lib.mtrt_hip_nvfp4_dequantize(None, 256, 256, 256, 256, getattr(pkg, dtype), rows, d1, 0) == 0
+                assert gpu.launches[-1][0] == ("mtrt_nvfp4_dqc_far_" if far else "mtrt_nvfp4_dqc_") + dtype.lower()

@@ -217,3 +217,24 @@ def test_axes_a_tensor_does_not_have(pkg):
     q, s = pkg.nvfp4_quantize(x, amax, axis=-1)
     q2, s2 = pkg.nvfp4_quantize(x, amax, axis=0)
     assert s.shape == (4,) and torch.equal(q, q2) and torch.equal(s, s2)
+
+
+def test_more_than_2_to_the_32_vectors(pkg):
+    """bf16 of 64 GiB and one block row, blocks along the second-to-last axis: the block rows on both sides of vector 2^32 as they are by
+    themselves."""
+    import torch
+    rows, cols = (1 << 19) + 16, 1 << 16
+    if torch.cuda.mem_get_info()[0] < 100 << 30:
+        pytest.skip("82 GiB of device memory needed")
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q = torch.randint(0, 256, (rows * cols // 2,), generator=g, device="cuda", dtype=torch.uint8)
+    s = torch.randint(0, 0x7F, (rows // 16, cols), generator=g, device="cuda", dtype=torch.uint8)
+    amax = torch.tensor(3.0, device="cuda")
+    y = pkg.nvfp4_dequantize(q, s, amax, torch.bfloat16, (rows, cols), axis=-2)
+    assert pkg.last_kernel() == "mtrt_nvfp4_dqc_far_bf16"
+    for r in (0, rows // 32 * 16, rows - 32, rows - 16):
+        part = pkg.nvfp4_dequantize(q[r * cols // 2:(r + 16) * cols // 2], s[r // 16:r // 16 + 1], amax, torch.bfloat16, (16, cols), axis=-2)
+        assert pkg.last_kernel() == "mtrt_nvfp4_dqc_bf16"
+        assert torch.equal(y[r:r + 16].view(torch.int16), part.view(torch.int16)), r
+    del q, s, y
+    torch.cuda.empty_cache()
