@@ -20,6 +20,9 @@ namespace {
 constexpr int kTile = 16;           // elements per lane per trip in qdq.hip
 constexpr uint32_t kBlock = 256;
 constexpr uint32_t kMaxGrid = 1u << 20;
+// A launch has fewer than 2^32 work items.  kLoopGrid: most workgroups (of up to 512 lanes) of kernels that loop over their tiles.
+constexpr int64_t kLoopGrid = int64_t(1) << 22;
+constexpr bool launchable(int64_t grid, int64_t block) { return grid * block < (int64_t(1) << 32); }
 // The one-wave-per-row kernels (layernorm / softmax `_v*`) map rows to waves from the workgroup index and do
 // not loop, so their grid must cover every row: ceil(rows / 4) workgroups, which blocks_for() caps at
 // kMaxGrid.  Tensors with more rows take the `_any` kernels, which loop over rows.
@@ -47,8 +50,8 @@ constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
 // 11.5, 12.0; M = 1, 29 MB 7.7, 6.8; bf16: 90 MB 16.2, 17.0; 67 MB 12.4, 13.4; 33 MB 9.8, 8.4).
 constexpr int64_t kWeightsPastBytes = int64_t(48) << 20;
 // f32 products of few rows on the vector units: K from which four waves share it; the fewest weights (below, the tiles take 3 to 4 us
-// too) and the most columns (a grid); what several groups of rows read through the L2s.
-constexpr int64_t kDotOwnColumnsBelow = 1536, kDotMinWeights = 16384, kDotMaxColumns = int64_t(1) << 27;
+// too); what several groups of rows read through the L2s.
+constexpr int64_t kDotOwnColumnsBelow = 1536, kDotMinWeights = 16384;
 constexpr double kDotGroupBytesPerUs = 7.5e6;
 // Any-K kernel: rounds of 128 x 128 tiles, each a walk down K in steps of 128 bytes a row, against 32 x 32 tiles, two workgroups of four
 // waves to a compute unit (f32, up to one workgroup a unit: eight waves).  Fitted to 34 products, M 1 ... 2000, K 6 ... 12287, N 7 ... 11000,
@@ -866,8 +869,18 @@ int32_t nvfp4_dispatch(bool quantize, hipStream_t stream, const void *xy, int32_
     void *args[] = {&xy, &q, &scales, &tensor_amax, &nvec};
     return launch(st, KernelName("mtrt_nvfp4_q_") + xn, uint32_t(blocks), kBlock, stream, args);
   }
-  void *args[] = {&q, &scales, &tensor_amax, &xy, &nvec};
-  return launch(st, KernelName("mtrt_nvfp4_dq_") + xn, uint32_t(blocks), kBlock, stream, args);
+  // as many launches as it takes: each of whole workgroups, and a workgroup's vectors are whole blocks of 16
+  const int64_t most = ((int64_t(1) << 32) / kBlock - 1) * per_block;
+  for (int64_t at = 0; at < nvec; at += most) {
+    int64_t some = std::min(most, nvec - at);
+    const void *q_at = static_cast<const char *>(q) + at * group / 2, *s_at = static_cast<const char *>(scales) + at * group / 16,
+               *y_at = static_cast<const char *>(xy) + at * 16;
+    void *args[] = {&q_at, &s_at, &tensor_amax, &y_at, &some};
+    const int32_t status = launch(st, KernelName("mtrt_nvfp4_dq_") + xn, uint32_t((some + per_block - 1) / per_block), kBlock, stream, args);
+    if (status != MTRT_OK)
+      return status;
+  }
+  return MTRT_OK;
 }
 } // namespace
 
@@ -1051,7 +1064,7 @@ int32_t mtrt_hip_gemm_w8a8(mtrt_stream_t stream, const void *a, const void *w_nk
                                                         double((tiles32 + num_compute_units(st) - 1) / num_compute_units(st));
     if (M <= 64 ? small_us < tile_us : M <= 128 && mid_us < tile_us) {
       return launch(st, KernelName(M <= 32 ? "mtrt_gemm_w8a8_nk_rows32" : M <= 64 ? "mtrt_gemm_w8a8_nk_rows64" : "mtrt_gemm_w8a8_nk_rows128"),
-                    uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), M <= 64 ? 512 : 256, as_hip(stream), args);
+                    uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), M <= 64 ? 512 : 256, as_hip(stream), args);
     }
     // 256 x 256 tiles, one workgroup per compute unit at a time, N panels dealt round-robin to the
     // 8 XCDs (gemm_core.hpp), so each set of panels takes 8 * ceil(panels / 8) * tiles_m workgroup
@@ -1161,7 +1174,7 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
   if (plan.kind == W8Plan::kRows) {
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
     return launch(st, KernelName(M <= 32 ? "mtrt_gemm_w8a8_frag_rows32" : "mtrt_gemm_w8a8_frag_rows64"),
-                  uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), 512, stream, args);
+                  uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), 512, stream, args);
   }
   FragPlan &p = plan.tile;
   if (!p.tile)
@@ -1204,16 +1217,26 @@ namespace {
 // that share it unequal parts, so each takes columns of its own where that still gives every compute unit a workgroup (us, shared and
 // own: (4, 448, 7680) 5.9, 4.8; (9, 1192, 3456) 9.8, 8.8; (4, 900, 900), 57 workgroups, 3.4, 4.6); more than four rows take eight
 // columns to a wave where that leaves two workgroups to a unit (us, four and eight: (8, 4096, 4096) 17.0, 15.8; (12, 2048, 512) 4.9, 6.1).
-int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const void *x, const void *w_nk, const void *bias, void *y, int64_t M, int64_t K, int64_t N) {
-  const int64_t units = num_compute_units(st), groups = (M + 7) / 8;
+struct DotShape {
+  bool shared, wide;                                   // waves share K; eight columns to a wave
+  int64_t grid;
+};
+DotShape dot_shape(int64_t M, int64_t K, int64_t N, int64_t units, bool may_be_wide) {
+  const int64_t groups = (M + 7) / 8;
   auto blocks = [&](int64_t columns) { return (N + columns - 1) / columns; };
-  const bool shared = K >= tuning::kDotOwnColumnsBelow || blocks(M == 1 ? 8 : 16) * groups < units;
-  const bool wide = M > 4 && K >= tuning::kDotOwnColumnsBelow && blocks(8) * groups >= 2 * units;
-  const int64_t columns = (M == 1 ? 2 : wide ? 8 : 4) * (shared ? 1 : 4), grid = 8 * ((blocks(columns) + 7) / 8) * groups;
-  int32_t form = (shared ? 1 : 0) | (groups == 1 && K * N * 4 > tuning::kWeightsPastBytes ? 2 : 0);
+  DotShape s;
+  s.shared = K >= tuning::kDotOwnColumnsBelow || blocks(M == 1 ? 8 : 16) * groups < units;
+  s.wide = may_be_wide && M > 4 && K >= tuning::kDotOwnColumnsBelow && blocks(8) * groups >= 2 * units;
+  s.grid = 8 * ((blocks((M == 1 ? 2 : s.wide ? 8 : 4) * (s.shared ? 1 : 4)) + 7) / 8) * groups;
+  return s;
+}
+
+int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const DotShape &shape, const void *x, const void *w_nk, const void *bias, void *y, int64_t M, int64_t K,
+                           int64_t N) {
+  int32_t form = (shape.shared ? 1 : 0) | (M <= 8 && K * N > tuning::kWeightsPastBytes / 4 ? 2 : 0);
   void *args[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &form};
   return launch(st, KernelName(M == 1 ? "mtrt_gemm_dense_rows1_f32" : M == 2 ? "mtrt_gemm_dense_rows2_f32" : M <= 4 ? "mtrt_gemm_dense_rows4_f32" :
-                               wide ? "mtrt_gemm_dense_rows8_wide_f32" : "mtrt_gemm_dense_rows8_f32"), uint32_t(grid), kBlock, stream, args);
+                               shape.wide ? "mtrt_gemm_dense_rows8_wide_f32" : "mtrt_gemm_dense_rows8_f32"), uint32_t(shape.grid), kBlock, stream, args);
 }
 } // namespace
 
@@ -1239,10 +1262,12 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   DeviceState *st = device_state();
   if (!st)
     return MTRT_RUNTIME_ERROR;
-  const bool few = dtype == MTRT_F32 && K >= 4 && K * N >= tuning::kDotMinWeights && N <= tuning::kDotMaxColumns;
+  const int64_t units = num_compute_units(st);
+  const DotShape dot = dot_shape(M, K, N, units, true);
+  const bool few = dtype == MTRT_F32 && M <= 32 && K >= 4 && K * N >= tuning::kDotMinWeights && launchable(dot.grid, kBlock);
   if (few && M <= 8)
-    return dense_few_rows_f32(st, as_hip(stream), x, w_nk, bias, y, M, K, N);
-  const int64_t tiles32 = (N + 31) / 32, units = num_compute_units(st), small_tiles = ((M + 31) / 32) * tiles32;
+    return dense_few_rows_f32(st, as_hip(stream), dot, x, w_nk, bias, y, M, K, N);
+  const int64_t tiles32 = (N + 31) / 32, small_tiles = ((M + 31) / 32) * tiles32;
   const bool whole_slices = K > 0 && (K * eb) % 128 == 0 && aligned(x, 16) && aligned(w_nk, 16);
   if (whole_slices && dtype == MTRT_F32) {
     // In 32 x 32 tiles, or up to 128 rows a column tile's rows together, or up to 32 on the vector units in groups of eight.
@@ -1250,22 +1275,21 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
     const double rows_us = tuning::kF32FixedUs + rounds * steps * (M <= 32 ? tuning::kF32Rows32StepUs : M <= 64 ? tuning::kF32Rows64StepUs : tuning::kF32Rows128StepUs);
     const double tiles_us = tuning::kF32FixedUs + (small_tiles <= units ? steps * tuning::kF32FewTilesStepUs
                                                                         : tuning::kF32LaterUs + steps * tuning::kF32TilesStepUs * std::max(1.0, double(small_tiles) / double(2 * units)));
-    const uint32_t most = uint32_t(kMaxGrid) * 1024;
     if (M > 32) {
       // eight waves to a tile while there is a unit for each and (128 rows or more) K gives them slices; four beyond
       const bool tall = M <= 128 && rows_us <= tiles_us, eight = small_tiles <= units && (M <= 128 || K >= 256);
       void *rargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
       return launch(st, KernelName(tall ? (M <= 64 ? "mtrt_gemm_dense_rows64_tall_f32" : "mtrt_gemm_dense_rows128_tall_f32") :
                                    !eight ? "mtrt_gemm_dense_mfma_f32" : M <= 64 ? "mtrt_gemm_dense_rows64_f32" : "mtrt_gemm_dense_rows128_f32"),
-                    uint32_t(std::min<int64_t>(tall ? tiles32 : 8 * ((small_tiles + 7) / 8), most)), tall ? (M <= 64 ? 512 : 256) : eight ? 512 : 256,
+                    uint32_t(std::min<int64_t>(tall ? tiles32 : 8 * ((small_tiles + 7) / 8), kLoopGrid)), tall ? (M <= 64 ? 512 : 256) : eight ? 512 : 256,
                     as_hip(stream), rargs);
     }
-    const int64_t groups = (M + 7) / 8;
-    int32_t as_tiles = !few || rows_us < tuning::kF32FixedUs + double(groups) * double(K * N * 4) / tuning::kDotGroupBytesPerUs;
-    int32_t form = K >= tuning::kDotOwnColumnsBelow || (N + 15) / 16 * groups < units;   // as in dense_few_rows_f32
-    const int64_t columns = form ? 4 : 16;
+    const DotShape in_groups = dot_shape(M, K, N, units, false);
+    int32_t as_tiles = !few || !launchable(in_groups.grid, kBlock) ||
+                       rows_us < tuning::kF32FixedUs + double((M + 7) / 8) * 4.0 * double(K * N) / tuning::kDotGroupBytesPerUs;
+    int32_t form = in_groups.shared;
     void *fargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &as_tiles, &form};
-    return launch(st, KernelName("mtrt_gemm_dense_rows32_f32"), uint32_t(as_tiles ? std::min<int64_t>(tiles32, most) : 8 * (((N + columns - 1) / columns + 7) / 8) * groups),
+    return launch(st, KernelName("mtrt_gemm_dense_rows32_f32"), uint32_t(as_tiles ? std::min<int64_t>(tiles32, kLoopGrid) : in_groups.grid),
                   as_tiles ? 512 : kBlock, as_hip(stream), fargs);
   }
   // 16-bit.  Decode-sized calls are bound by reading the weights once: up to 32 rows take one workgroup per 32 weight rows, its
@@ -1280,7 +1304,7 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   if (whole_slices && (M <= 64 ? small_us < tile_us : M <= 128 && mid_us < tile_us)) {
     void *rargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
     return launch(st, KernelName(M <= 32 ? "mtrt_gemm_dense_rows32_" : M <= 64 ? "mtrt_gemm_dense_rows64_" : "mtrt_gemm_dense_rows128_") + xn,
-                  uint32_t(std::min<int64_t>(tiles32, int64_t(kMaxGrid) * 1024)), M <= 64 ? 512 : 256, as_hip(stream), rargs);
+                  uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), M <= 64 ? 512 : 256, as_hip(stream), rargs);
   }
   if (K > 0 && (K * eb) % 128 == 0 && aligned(x, 16) && aligned(w_nk, 16) && M * K * eb < (int64_t(1) << 32) &&
       N * K * eb < (int64_t(1) << 32)) {
@@ -1312,13 +1336,13 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
                                                                                       : tuning::kEdgeSmallStepUs * std::max(1.0, double(small_tiles) / double(2 * units)));
     // up to 32 rows of f32 may be read in groups of eight as well: us, 32 x 32 tiles and so, (9, 1192, 3456) 10.9, 9.4; (16, 1031, 260) 9.1,
     // 4.4; (16, 600, 8000) 9.1, 9.9; (32, 4097, 4096) 38.7, 40.5
-    if (few && M <= 32 && 3.0 + double((M + 7) / 8) * double(K * N * 4) / tuning::kDotGroupBytesPerUs < std::min(small_us, edge_us))
-      return dense_few_rows_f32(st, as_hip(stream), x, w_nk, bias, y, M, K, N);
+    if (few && 3.0 + double((M + 7) / 8) * 4.0 * double(K * N) / tuning::kDotGroupBytesPerUs < std::min(small_us, edge_us))
+      return dense_few_rows_f32(st, as_hip(stream), dot, x, w_nk, bias, y, M, K, N);
     int32_t waves = 0;
     if (K * eb >= 16 && small_us < edge_us)
       waves = dtype == MTRT_F32 && small_tiles <= units ? 8 : 4;
     void *eargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &waves};
-    return launch(st, KernelName("mtrt_gemm_dense_edge_") + xn, uint32_t(std::min<int64_t>(waves ? 8 * ((small_tiles + 7) / 8) : edge_tiles, int64_t(kMaxGrid) * 1024)),
+    return launch(st, KernelName("mtrt_gemm_dense_edge_") + xn, uint32_t(std::min<int64_t>(waves ? 8 * ((small_tiles + 7) / 8) : edge_tiles, kLoopGrid)),
                   waves ? uint32_t(64 * waves) : kBlock, as_hip(stream), eargs);
   }
   const int64_t tiles = ((M + 63) / 64) * ((N + 63) / 64);
@@ -1536,7 +1560,7 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
     // this, bf16: (16, 512, 8192) 3.6, 4.2; (8, 768, 8192) 3.9, 4.1; (8, 1024, 8192) 4.2, 4.2; (4, 1024, 12000) 6.7, 5.2; (8, 2048, 8192) 5.1, 4.5).
     const bool passes = quantized || s.Kp != p.K;
     const int64_t tiles16 = (p.N + 15) / 16, most = tiles16 <= units ? 2 * kDecodeElements : passes && tiles16 > 2 * units ? kDecodeElements / 2 : kDecodeElements;
-    s.one_launch = s.fragments && M <= 16 && M * s.Kp <= most && (passes || tiles16 <= units || s.Kp >= 1024);
+    s.one_launch = s.fragments && M <= 16 && M * s.Kp <= most && launchable(tiles16, 512) && (passes || tiles16 <= units || s.Kp >= 1024);
     s.pass = !s.one_launch && passes;
     s.act_bytes = passes ? round_up(M * s.Kp * eb, 256) : 0;   // asked for, not used, where the GEMM takes x itself
     if (s.fragments) {

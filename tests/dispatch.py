@@ -39,7 +39,7 @@ def build(folder):
 class Dispatch:
     """The library with a state of its own (a copy of the file: a loaded library's state is the process's).  `launches`
     collects (kernel, stream, its (splits, per, partial, tickets) or the address of its reduction block or None), `fills` the
-    clears (address, words, stream)."""
+    clears (address, words, stream), `sizes` every launch's (kernel, grid, block)."""
 
     def __init__(self, pkg, path, copy):
         shutil.copy(path, copy)
@@ -54,6 +54,7 @@ class Dispatch:
         self.lib.fake_destroy_stream.argtypes = [_vp]
         self.launches = []
         self.fills = []
+        self.sizes = []
         self._callback = _CALLBACK(self._launched)
         self.lib.fake_set_launch_callback(self._callback)
         assert self.lib.mtrt_hip_init() == 0
@@ -71,6 +72,7 @@ class Dispatch:
 
     def _launched(self, name, grid, block, stream, args):
         name = name.decode()
+        self.sizes.append((name, grid, block))
         if name == "mtrt_fill":
             self.fills.append((ctypes.cast(args[0], ctypes.POINTER(_vp))[0], ctypes.cast(args[1], ctypes.POINTER(_i64))[0], stream))
             return
@@ -78,6 +80,8 @@ class Dispatch:
         split = None
         if name.startswith(("mtrt_amax_", "mtrt_dynqdq_")):
             split = ctypes.cast(args[5 if name.startswith("mtrt_amax_") else 7], ctypes.POINTER(_vp))[0]
+        elif name.startswith("mtrt_nvfp4_dq_"):       # (codes, scales, values, vectors)
+            split = tuple(ctypes.cast(args[i], ctypes.POINTER(_i64))[0] for i in (0, 1, 3, 4))
         elif at is not None:
             s = ctypes.cast(args[at], ctypes.POINTER(Split))[0]
             split = (s.splits, s.per, s.partial, s.tickets)

@@ -187,3 +187,32 @@ def test_tensors_of_64_gib_are_divided_in_64_bits(gpu, pkg, dtype, vector):
             if rows:
                 assert gpu.lib.mtrt_hip_nvfp4_dequantize(None, 256, 256, 256, 256, getattr(pkg, dtype), rows, d1, 0) == 0
                 assert gpu.launches[-1][0] == ("mtrt_nvfp4_dqc_far_" if far else "mtrt_nvfp4_dqc_") + dtype.lower()
+
+
+def test_launches_have_less_than_2_to_the_32_work_items(gpu, pkg):
+    """Operands that fit into the device's 288 GB and need more workgroups of some kernels than a launch can have."""
+    L = gpu.lib
+    for dtype, m, k, n in ((pkg.F32, 1, 1536, (1 << 25) + 40), (pkg.F32, 1, 5, (1 << 27) - 3), (pkg.F32, 8, 1536, (1 << 25) + 1), (pkg.F32, 20, 1600, 1 << 25),
+                           (pkg.F32, 32, 1537, 1 << 24), (pkg.F32, 32, 4, 1 << 29), (pkg.F32, 64, 32, (1 << 28) + 9), (pkg.F32, 120, 32, 1 << 27), (pkg.F32, 1 << 17, 32, 1 << 17),
+                           (pkg.F32, 1 << 24, 32, 1000), (pkg.F16, 1, 9, (1 << 30) + 1), (pkg.BF16, 33, 200, (1 << 29) + 3), (pkg.F16, 4, 64, 1 << 28)):
+        assert L.mtrt_hip_linear_dense(None, 256, 256, 256, 256, dtype, m, k, n) == 0
+    for n in ((1 << 26) + 1, 1 << 27, (1 << 27) + 7):
+        for q_dtype in (-1, pkg.F8E4M3FN):
+            gpu.linear(8, 3, 128, n, pkg.BF16, q_dtype=q_dtype)
+    assert len(gpu.sizes) > 15
+    over = [(name, grid, block) for name, grid, block in gpu.sizes if grid * block >= 1 << 32]
+    assert not over
+
+
+@pytest.mark.parametrize("dtype,vector", [("F32", 4), ("BF16", 8)])
+@pytest.mark.parametrize("vectors", [(1 << 33) - 1024, 1 << 33, (1 << 33) + 4, 3 << 33])
+def test_dequantize_takes_as_many_launches_as_the_tensor_needs(gpu, pkg, dtype, vector, vectors):
+    q, scales, y = 1 << 12, 1 << 44, 1 << 45
+    assert gpu.lib.mtrt_hip_nvfp4_dequantize(None, q, scales, 256, y, getattr(pkg, dtype), vectors // 4, 4 * vector, 1) == 0
+    assert all(grid * block < 1 << 32 and (grid - 1) * 512 < count <= grid * 512
+               for (_, grid, block), (_, _, (_, _, _, count)) in zip(gpu.sizes, gpu.launches))
+    done = 0
+    for _, _, (q_at, s_at, y_at, count) in gpu.launches:
+        assert (q_at, s_at, y_at) == (q + done * vector // 2, scales + done * vector // 16, y + done * 16) and done * vector % 16 == 0
+        done += count
+    assert done == vectors and (len(gpu.launches) == 1) == (vectors < 1 << 33)
