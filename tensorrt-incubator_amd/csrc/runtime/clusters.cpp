@@ -265,6 +265,21 @@ bool element_count(int64_t d0, int64_t d1, int64_t *n) { return !__builtin_mul_o
 // fits in 63 bits.
 constexpr int64_t kMaxMatrixExtent = (int64_t(1) << 31) - 1;
 
+// 256 x 256 tiles, one workgroup to a compute unit at a time; a last round that would fill at most half of the units (or a launch that
+// does) has its panels cut into 256 x 128 halves.  Each kind is dealt evenly to the XCDs.
+struct Panels {
+  int64_t full, full_tiles, half_tiles, grid;
+};
+Panels panels_of(int64_t M, int64_t N, int64_t units) {
+  const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256, tiles = panels * tiles_m, rest = tiles % units;
+  Panels p;
+  p.full = tiles * 2 <= units ? 0 : rest > 0 && rest * 2 <= units ? panels - (rest + tiles_m - 1) / tiles_m : panels;
+  p.full_tiles = p.full * tiles_m;
+  p.half_tiles = std::max<int64_t>(0, (N - p.full * 256 + 127) / 128) * tiles_m;   // (full panels may reach past N)
+  p.grid = 8 * ((p.full_tiles + 7) / 8) + 8 * ((p.half_tiles + 7) / 8);
+  return p;
+}
+
 uint32_t blocks_for(int64_t units, uint32_t per_block) {
   const int64_t b = (units + per_block - 1) / per_block;
   return uint32_t(std::max<int64_t>(1, std::min<int64_t>(b, kMaxGrid)));
@@ -1066,22 +1081,10 @@ int32_t mtrt_hip_gemm_w8a8(mtrt_stream_t stream, const void *a, const void *w_nk
       return launch(st, KernelName(M <= 32 ? "mtrt_gemm_w8a8_nk_rows32" : M <= 64 ? "mtrt_gemm_w8a8_nk_rows64" : "mtrt_gemm_w8a8_nk_rows128"),
                     uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), M <= 64 ? 512 : 256, as_hip(stream), args);
     }
-    // 256 x 256 tiles, one workgroup per compute unit at a time, N panels dealt round-robin to the
-    // 8 XCDs (gemm_core.hpp), so each set of panels takes 8 * ceil(panels / 8) * tiles_m workgroup
-    // ids.  The launch runs in rounds of one tile per unit; when the last round would use at most
-    // half of the units (or the whole launch does), its panels are cut into 128-wide halves.
-    const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256, units = num_compute_units(st);
-    const int64_t tiles = panels * tiles_m, rest = tiles % units;
-    int64_t full_panels = panels;
-    if (tiles * 2 <= units)
-      full_panels = 0;
-    else if (rest > 0 && rest * 2 <= units)
-      full_panels = panels - (rest + tiles_m - 1) / tiles_m;
-    const int64_t half_panels = (N - full_panels * 256 + 127) / 128;
-    const int64_t grid = 8 * ((full_panels * tiles_m + 7) / 8) + 8 * ((half_panels * tiles_m + 7) / 8);   // each kind dealt evenly to the XCDs
-    if (grid <= int64_t(kMaxGrid) * 1024) {
-      void *fast_args[] = {&a, &w_nk, &a_scale, &w_scale, &y, &M, &K, &N, &full_panels};
-      return launch(st, KernelName("mtrt_gemm_w8a8_nk"), uint32_t(grid), kBlock, as_hip(stream), fast_args);
+    Panels panels = panels_of(M, N, num_compute_units(st));
+    if (panels.grid <= int64_t(kMaxGrid) * 1024) {
+      void *fast_args[] = {&a, &w_nk, &a_scale, &w_scale, &y, &M, &K, &N, &panels.full};
+      return launch(st, KernelName("mtrt_gemm_w8a8_nk"), uint32_t(panels.grid), kBlock, as_hip(stream), fast_args);
     }
   }
   if (K > 0) {
@@ -1310,18 +1313,10 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
       N * K * eb < (int64_t(1) << 32)) {
     // operands in whole 128-byte slices of K: the matrix-core tile loop (tiles and rounds as in
     // mtrt_hip_gemm_w8a8; f16 [2048, 4096] x [11008, 4096]: 3654 us on the FMA kernel below)
-    const int64_t panels = (N + 255) / 256, tiles_m = (M + 255) / 256;
-    const int64_t tiles256 = panels * tiles_m, rest = tiles256 % units;
-    int64_t full_panels = panels;
-    if (tiles256 * 2 <= units)
-      full_panels = 0;
-    else if (rest > 0 && rest * 2 <= units)
-      full_panels = panels - (rest + tiles_m - 1) / tiles_m;
-    const int64_t half_panels = (N - full_panels * 256 + 127) / 128;
-    const int64_t grid = 8 * ((full_panels * tiles_m + 7) / 8) + 8 * ((half_panels * tiles_m + 7) / 8);   // each kind dealt evenly to the XCDs
-    if (grid <= int64_t(kMaxGrid) * 1024) {
-      void *margs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &full_panels};
-      return launch(st, KernelName("mtrt_gemm_dense_mfma_") + xn, uint32_t(grid), kBlock, as_hip(stream), margs);
+    Panels panels = panels_of(M, N, units);
+    if (panels.grid <= int64_t(kMaxGrid) * 1024) {
+      void *margs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &panels.full};
+      return launch(st, KernelName("mtrt_gemm_dense_mfma_") + xn, uint32_t(panels.grid), kBlock, as_hip(stream), margs);
     }
   }
   void *args[] = {&x, &w_nk, &bias, &y, &M, &K, &N};

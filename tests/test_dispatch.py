@@ -216,3 +216,13 @@ def test_dequantize_takes_as_many_launches_as_the_tensor_needs(gpu, pkg, dtype, 
         assert (q_at, s_at, y_at) == (q + done * vector // 2, scales + done * vector // 16, y + done * 16) and done * vector % 16 == 0
         done += count
     assert done == vectors and (len(gpu.launches) == 1) == (vectors < 1 << 33)
+
+
+@pytest.mark.parametrize("M,N", [(4096, 2305), (3585, 4097), (9000, 1281), (4096, 2304), (4096, 2306), (2048, 11008), (5000, 65537)])
+def test_large_tiles_cover_the_output(gpu, pkg, M, N):
+    """256 x 256 tiles, also where the last panel holds one column; launches cut into half panels have more workgroups."""
+    tiles = ((M + 255) // 256) * ((N + 255) // 256)
+    assert gpu.lib.mtrt_hip_gemm_w8a8(None, 256, 256, 256, 256, 256, M, 4096, N) == 0
+    assert gpu.lib.mtrt_hip_linear_dense(None, 256, 256, None, 256, pkg.F16, M, 4096, N) == 0
+    assert [name for name, _, _ in gpu.sizes] == ["mtrt_gemm_w8a8_nk", "mtrt_gemm_dense_mfma_f16"]
+    assert all(grid >= tiles for _, grid, _ in gpu.sizes)

@@ -669,3 +669,24 @@ def test_w4a16_tile_choice_and_results_at_mid_m(pkg, orc, shape, kernel):
     ref = np.concatenate([orc.gemm_w4a16(a, wp, s, K, N, B, m0=r, mcount=1) for r in rows])
     orc.set_threads(1)
     _check_w4a16(orc, y[rows].contiguous(), a[rows], w, s, K, N, B, ref)
+
+
+@pytest.mark.parametrize("M,N", [(4096, 2305), (3585, 4097), (4000, 2177), (4096, 2432)])
+def test_columns_just_past_whole_panels(pkg, M, N):
+    """One column into the last panel of 256, or just past half of it, in a launch whose panels stay whole: every tile is there."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(N)
+    K = 128
+    a = torch.randint(-128, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
+    w = torch.randint(-128, 128, (N, K), generator=g, device="cuda", dtype=torch.int8)
+    one = torch.full((max(M, N),), 2.0 ** -10, device="cuda")
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    pkg.gemm_w8a8(a, w, one[:M], one[:N], y)
+    assert pkg.last_kernel() == "mtrt_gemm_w8a8_nk"
+    # sums below 2^24 and scales of powers of two: one rounding to f16
+    assert torch.equal(y, (a.float() @ w.float().t() * 2.0 ** -20).half())
+    x, v = a.half(), w.half() * 2.0 ** -8
+    y.fill_(float("nan"))
+    pkg.linear_dense(x, v, None, y)
+    assert pkg.last_kernel() == "mtrt_gemm_dense_mfma_f16"
+    assert torch.equal(y, (x.float() @ v.float().t()).half())
