@@ -218,10 +218,48 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
   }
 }
 
+// The same sub-tiles written as f32, straight from the accumulators: a lane's runs of four consecutive outputs of a
+// row are one 16-byte store each (32-byte pieces of a row per half wave, merged in the write-back cache); no staging.
+// Epilogue: finish4(values of columns col .. col+3, col, N).  For the 2 x 2 waves of `run`.
+template <int JT, class Acc, class Epilogue>
+__device__ __forceinline__ void write_tile_f32(Acc (&acc)[4][JT], Epilogue& epi, float* __restrict__ y, int64_t M, int64_t N,
+                                               int64_t m0, int64_t n0, int wave) {
+  const int lane = threadIdx.x & 63;
+  const int wm = wave >> 1, wn = wave & 1;
+  const int frow = lane & 31, fhalf = lane >> 5;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t row = m0 + wm * 128 + i * 32 + frow;
+    if (row >= M) continue;
+#pragma unroll
+    for (int j = 0; j < JT; ++j)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int64_t col = n0 + wn * (32 * JT) + j * 32 + q * 8 + fhalf * 4;
+        if (col >= N) continue;
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * q + e];
+        epi.finish4(v, col, N);
+        if (col + 3 < N) {
+          *reinterpret_cast<f32x4_words*>(y + row * N + col) = (f32x4){v[0], v[1], v[2], v[3]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e < N) y[row * N + col + e] = v[e];
+        }
+      }
+  }
+}
 template <int JT, class Acc, class Epilogue>
 __device__ __forceinline__ void finish_tile(Acc (&acc)[4][JT], Epilogue& epi, uint16_t* __restrict__ y, int64_t M, int64_t N,
                                             int64_t m0, int64_t n0, int8_t* lds, int wave) {
   write_tile<JT, 2, 4>(acc, epi, y, M, N, m0, n0, lds, wave, true);
+}
+template <int JT, class Acc, class Epilogue>
+__device__ __forceinline__ void finish_tile(Acc (&acc)[4][JT], Epilogue& epi, float* __restrict__ y, int64_t M, int64_t N,
+                                            int64_t m0, int64_t n0, int8_t*, int wave) {
+  write_tile_f32<JT>(acc, epi, y, M, N, m0, n0, wave);
 }
 
 // Both operands as bytes, K-contiguous per row / per column: a [M, a_row_bytes], b [N, a_row_bytes].
@@ -230,8 +268,9 @@ __device__ __forceinline__ void finish_tile(Acc (&acc)[4][JT], Epilogue& epi, ui
 // Traits: Acc (16-wide accumulator vector), mfma(first, second, acc), zero().
 // Epilogue: setup(lds scratch, m0, M, n0, N), columns<HC>(first column of the lane in the tile), row(row in tile),
 // convert4(acc, q, column tile of the pass, words): outputs 4q .. 4q+3 of the accumulator as two words of two.
-// Y: uint16_t, through the staged epilogue.
-template <class Traits, int JT, class Epilogue, typename Y>
+// Y: uint16_t (16-bit outputs through the staged epilogue) or float (direct stores, see write_tile_f32).
+// CHAINS: K is summed in as many parts of its slices, the parts then in order (f32 sums: the shorter chains of additions have the smaller error).
+template <class Traits, int JT, int CHAINS = 1, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ b, int64_t row_bytes, Epilogue& epi,
                                     Y* __restrict__ y, int64_t M, int64_t N, int64_t slices, int64_t m0,
                                     int64_t n0, int8_t* lds) {
@@ -319,11 +358,43 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
   };
 
   int64_t s = 0;
-  for (; s + 1 < slices; s += 2) {                     // no branch inside: the loop body stays one basic block
-    slice_body(IntC<0>{}, s);
-    slice_body(IntC<1>{}, s + 1);
+  if constexpr (CHAINS > 1) {
+    Acc total[4][JT];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < JT; ++j) total[i][j] = Traits::zero();
+#pragma unroll 1
+    for (int part = 1; part < CHAINS; ++part) {
+#pragma unroll 1
+      for (const int64_t end = slices / 2 * part / CHAINS * 2; s < end; s += 2) {
+        slice_body(IntC<0>{}, s);
+        slice_body(IntC<1>{}, s + 1);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < JT; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = Traits::zero();
+        }
+    }
+    for (; s + 1 < slices; s += 2) {
+      slice_body(IntC<0>{}, s);
+      slice_body(IntC<1>{}, s + 1);
+    }
+    if (s < slices) slice_body(IntC<0>{}, s);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < JT; ++j) acc[i][j] = total[i][j] + acc[i][j];
+  } else {
+    for (; s + 1 < slices; s += 2) {                   // no branch inside: the loop body stays one basic block
+      slice_body(IntC<0>{}, s);
+      slice_body(IntC<1>{}, s + 1);
+    }
+    if (s < slices) slice_body(IntC<0>{}, s);
   }
-  if (s < slices) slice_body(IntC<0>{}, s);
 
   finish_tile<JT>(acc, epi, y, M, N, m0, n0, lds, wave);
 }
@@ -528,7 +599,8 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[2][2], Epilogue& epi, Y* _
   }
 }
 
-template <class Traits, class Epilogue, typename Y>
+// CHAINS: as for gemm_core::run
+template <class Traits, int CHAINS = 1, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ b, int64_t row_bytes, Epilogue& epi,
                                     Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds) {
   using Acc = typename Traits::Acc;
@@ -548,7 +620,7 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
     u32x4 ra[4], rb[4];
     load_chunks(ra, a, m0, M, row_bytes, ccol, steps == 1);
     load_chunks(rb, b, n0, N, row_bytes, ccol, steps == 1);
-    for (int64_t s = 0; s < steps; ++s) {
+    const auto step = [&](int64_t s) {
       __syncthreads();                                 // the previous k-step's (or tile's) LDS reads are done
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
@@ -561,6 +633,36 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
         load_chunks(rb, b, n0, N, row_bytes, (s + 1) * kStep + ccol, s + 2 == steps);
       }
       multiply_stage<Traits>(acc, sa, sb);
+    };
+    int64_t s = 0;
+    if constexpr (CHAINS > 1) {
+      Acc total[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) total[i][j] = Traits::zero();
+#pragma unroll 1
+      for (int part = 1; part < CHAINS; ++part) {
+        const int64_t end = steps * part / CHAINS;
+        if (s == end) continue;
+#pragma unroll 1
+        for (; s < end; ++s) step(s);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            total[i][j] += acc[i][j];
+            acc[i][j] = Traits::zero();
+          }
+      }
+#pragma unroll 1
+      for (; s < steps; ++s) step(s);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = total[i][j] + acc[i][j];
+    } else {
+      for (; s < steps; ++s) step(s);
     }
     write_tile(acc, epi, y, M, N, m0, n0, lds);
   }

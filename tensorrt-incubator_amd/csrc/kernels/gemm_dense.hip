@@ -118,6 +118,16 @@ struct F32Traits {
     return c;
   }
 };
+struct BiasF32Epilogue {
+  const float* bias;
+  __device__ __forceinline__ void finish4(float (&v)[4], int64_t col, int64_t N) const {
+    if (!bias) return;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (col + e < N) v[e] = v[e] + bias[col + e];
+  }
+};
+
 template <typename X> __device__ __forceinline__ uint32_t narrow16(float v);
 template <> __device__ __forceinline__ uint32_t narrow16<F16>(float v) { return f32_to_f16_bits(v); }
 template <> __device__ __forceinline__ uint32_t narrow16<BF16>(float v) { return f32_to_bf16_bits(v); }
@@ -398,9 +408,9 @@ MTRT_DENSE_ROWS32_KERNEL(f16, F16)
 MTRT_DENSE_ROWS32_KERNEL(bf16, BF16)
 // f32, more rows (x, w, bias, y, M, K, N): 32 x 32 tiles, K shared by eight waves (any M; rows64 and rows128 differ in name only), or, _tall,
 // the rows against each weight fragment at once; grid: any, block = 512 (rows128_tall: 256).  The matrix cores set the time of a tile
-// column with all its rows (0.18 us to a 128-byte slice of K for every 32 rows), so it is the faster one only where the columns alone
-// fill the chip and K is short: us, so and in tiles, (100, 512, 8192) 17.3 and 18.2, (40, 256, 16384) 12.3 and 12.8, (64, 4096, 4096) 44.9 and 25.6,
-// (109, 3072, 448) 62.7 and 19.2, (128, 4096, 1024) 82.7 and 23.8.
+// column with all its rows (0.18 us to a 128-byte slice of K for every 32 rows, and 1 to 3 us to a round of tiles): it is level with the tiles at
+// best, where the columns alone fill the chip once or twice and K is short: us, so and in tiles, (100, 512, 8192) 18.1 and 18.1, (40, 256, 16384)
+// 12.7 and 13.0, (64, 512, 32768) 36.7 and 31.7, (64, 4096, 4096) 44.9 and 25.6, (109, 3072, 448) 62.7 and 19.2, (128, 4096, 1024) 82.7 and 23.8.
 #define MTRT_DENSE_ROWS_F32_KERNEL(NAME, WAVES, MT, MANY)                                                          \
   extern "C" __global__ void __launch_bounds__(64 * WAVES) mtrt_gemm_dense_##NAME##_f32(                           \
       const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M, \
@@ -440,11 +450,36 @@ MTRT_DENSE_ROWS128_KERNEL(f16, F16)
 MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
 
 // ... and where the tiles are more than the compute units: four waves, four workgroups to a unit; grid: any, block = 256.  Bound by the
-// matrix cores (a 32 x 32 x 2 instruction every 64 cycles: 157 TFLOP/s nominal) where the tiles fill the chip, by the walk down K where they
-// do not.  Tiles of 256 x 256 and 256 x 128, which this took before, left most of the chip idle and held 256 registers a lane: us,
-// (M, K, N), those and these: (200, 1024, 1024) 131 and 8.8, (300, 3072, 2048) 366 and 49, (512, 4096, 4096) 482 and 172,
-// (2048, 2048, 2048) 253 and 164, (768, 1024, 11008) 274 and 182, (2048, 512, 8192) 211 and 207, (4096, 1024, 1024) 142 and 89.
+// matrix cores (a 32 x 32 x 2 instruction every 64 cycles: 157 TFLOP/s nominal) and, where the tiles fill the chip, by what they read through
+// the L2s, 256 bytes of K for 32 x 32 outputs: no more than 108 TFLOP/s at any size.  Larger tiles read less and leave units idle
+// where they are few.  us, 32 x 32, 128 x 128 and 256 x 128:
+//   (200, 1024, 1024) 10.3, 84, 139      (300, 3072, 2048) 50, 236, 379       (512, 4096, 4096) 176, 311, 500      (768, 1024, 11008) 195, 229, 281
+//   (2048, 512, 8192) 208, 163, 170      (4096, 64, 4096) 78.6, 46.2, 61.3    (120, 64, 65536) 42.4, 25.5, 55.5    (1024, 4096, 4096) 358, 319, 496
+//   (2048, 4096, 4096) 672, 544, 502     (4096, 4096, 4096) 1303, 1075, 1007  (2048, 4096, 11008) 1689, 1614, 1504
+// (256 x 256 tiles, tried before: 254 registers and all accumulators a lane, (2048, 512, 8192) 205, (4096, 4096, 4096) 1001, (2048, 4096, 11008) 1508.)
+// All of them sum K in four parts or more, then the parts: the error against 64 bits is half of one chain's (K = 4096: 4.5e-7 and 9.0e-7 of the result).
 MTRT_DENSE_ROWS_F32_KERNEL(mfma, 4, 1, true)
+
+// ... 128 x 128 tiles: (x, w, bias, y, M, K, N) ; grid: any, block = 256.
+extern "C" __global__ void __launch_bounds__(256, 2) mtrt_gemm_dense_t128x128_f32(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
+    int64_t K, int64_t N) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::edge::kLdsBytes];
+  dense_cluster::EdgeBiasF32Epilogue epi{bias};
+  gemm_core::edge::run<dense_cluster::F32Traits, 4>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds);
+}
+// ... 256 x 128 tiles: (x, w, bias, y, M, K, N) ; x and w below 4 GiB each; grid = 8 * ceil(ceil(M/256) * ceil(N/128) / 8), block = 256.
+extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_dense_t256x128_f32(
+    const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,
+    int64_t K, int64_t N) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::LDS_BYTES];
+  const int64_t tiles_m = (M + 255) / 256;
+  int64_t tile_m, panel;
+  if (!gemm_core::tile_of_even(blockIdx.x, gridDim.x, tiles_m, (N + 127) / 128, tiles_m, tile_m, panel)) return;
+  dense_cluster::BiasF32Epilogue epi{bias};
+  gemm_core::run<dense_cluster::F32Traits, 2, 4>(reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N,
+                                                 K * 4 / gemm_core::BKB, tile_m * 256, panel * 128, lds);
+}
 
 // ---- weights in fragment order (gemm_frag.hpp) ---------------------------------------------------------
 // What a module's Linear runs on: its weights are re-laid once per parameter set.  Against the loops above, which bring both

@@ -57,10 +57,15 @@ constexpr double kDotGroupBytesPerUs = 7.5e6;
 // waves to a compute unit (f32, up to one workgroup a unit: eight waves).  Fitted to 34 products, M 1 ... 2000, K 6 ... 12287, N 7 ... 11000,
 // f32 and f16; the faster form is taken in each of them.
 constexpr double kEdgeFixedUs = 4.0, kEdgeF32StepUs = 2.45, kEdge16StepUs = 1.2;
-// f32 products of whole slices, by rounds of 32-column tiles with all rows (up to 32, 64 and 128 of them) and by 32 x 32 tiles, two to a compute
-// unit: us to a slice of 128 bytes of K.  Fitted to 27 products, M 16 ... 4096, K 256 ... 12288, N 256 ... 16384.
-constexpr double kF32FixedUs = 3.0, kF32Rows32StepUs = 0.18, kF32Rows64StepUs = 0.36, kF32Rows128StepUs = 0.68;
-constexpr double kF32FewTilesStepUs = 0.2, kF32LaterUs = 2.0, kF32TilesStepUs = 0.4;
+// f32 products of whole slices, us to a slice of 128 bytes of K.  By rounds of 32-column tiles with all rows (up to 32, 64 and 128 of them): fitted to 27
+// products, M 16 ... 128, K 256 ... 12288, N 256 ... 16384, of up to two rounds (what a round costs beside its slices is left out).
+constexpr double kF32FixedUs = 3.0, kF32Rows32StepUs = 0.18, kF32Rows64StepUs = 0.36, kF32Rows128StepUs = 0.68, kF32RowsRounds = 2;
+// By 32 x 32 tiles: one or none to a compute unit, and every two to a unit; by 128 x 128 tiles, the rest up to one to a unit and every two to a unit;
+// by rounds of 256 x 128 tiles.  Fitted to 57 products, M 33 ... 65536, K 32 ... 11008, N 96 ... 65536; the form with the least estimate is the
+// fastest in each, or within 2 percent of it.
+constexpr double kF32FewTilesStepUs = 0.2, kF32TilesUs = 1.8, kF32TilesStepUs = 0.32;
+constexpr double kF32T128OneUs = 10.0, kF32T128OneStepUs = 2.36, kF32T128TwoUs = 14.0, kF32T128TwoStepUs = 4.12;
+constexpr double kF32T256RoundUs = 30.0, kF32T256StepUs = 3.68;
 constexpr double kEdgeSmallFixedUs = 3.0, kEdgeSmallFewStepUs = 0.2, kEdgeSmallStepUs = 0.5;
 // W4A16 tile choice: a full round of 256 x 256 tiles takes 3.25 times a full round of 128 x 128 tiles (for four times
 // the work), and a last round filled to a fraction f of the units takes 0.56 + 0.44 f^2 of a full one (fewer units
@@ -1273,15 +1278,25 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   const int64_t tiles32 = (N + 31) / 32, small_tiles = ((M + 31) / 32) * tiles32;
   const bool whole_slices = K > 0 && (K * eb) % 128 == 0 && aligned(x, 16) && aligned(w_nk, 16);
   if (whole_slices && dtype == MTRT_F32) {
-    // In 32 x 32 tiles, or up to 128 rows a column tile's rows together, or up to 32 on the vector units in groups of eight.
+    // In 32 x 32 tiles, or up to 128 rows a column tile's rows together, or up to 32 on the vector units in groups of eight; in larger tiles where
+    // they fill the chip.
     const double steps = double(K * eb / 128), rounds = double((tiles32 + units - 1) / units);
     const double rows_us = tuning::kF32FixedUs + rounds * steps * (M <= 32 ? tuning::kF32Rows32StepUs : M <= 64 ? tuning::kF32Rows64StepUs : tuning::kF32Rows128StepUs);
-    const double tiles_us = tuning::kF32FixedUs + (small_tiles <= units ? steps * tuning::kF32FewTilesStepUs
-                                                                        : tuning::kF32LaterUs + steps * tuning::kF32TilesStepUs * std::max(1.0, double(small_tiles) / double(2 * units)));
     if (M > 32) {
-      // eight waves to a tile while there is a unit for each and (128 rows or more) K gives them slices; four beyond
-      const bool tall = M <= 128 && rows_us <= tiles_us, eight = small_tiles <= units && (M <= 128 || K >= 256);
+      const double tiles_us = tuning::kF32FixedUs + (small_tiles <= units ? steps * tuning::kF32FewTilesStepUs
+                                                                          : (tuning::kF32TilesUs + steps * tuning::kF32TilesStepUs) * std::max(1.0, double(small_tiles) / double(2 * units)));
+      const int64_t tiles128 = ((M + 127) / 128) * ((N + 127) / 128), rest128 = tiles128 % (2 * units), tiles256 = ((M + 255) / 256) * ((N + 127) / 128);
+      const double one_us = tuning::kF32T128OneUs + steps * tuning::kF32T128OneStepUs, two_us = tuning::kF32T128TwoUs + steps * tuning::kF32T128TwoStepUs;
+      const double t128_us = double(tiles128 / (2 * units)) * two_us + (rest128 == 0 ? 0.0 : rest128 <= units ? one_us : two_us);
+      const double t256_us = double((tiles256 + units - 1) / units) * (tuning::kF32T256RoundUs + steps * tuning::kF32T256StepUs);
+      const int64_t grid256 = 8 * ((tiles256 + 7) / 8);
       void *rargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
+      if (t256_us < std::min(t128_us, tiles_us) && M * K < (int64_t(1) << 30) && N * K < (int64_t(1) << 30) && launchable(grid256, kBlock))
+        return launch(st, KernelName("mtrt_gemm_dense_t256x128_f32"), uint32_t(grid256), kBlock, as_hip(stream), rargs);
+      if (t128_us < tiles_us)
+        return launch(st, KernelName("mtrt_gemm_dense_t128x128_f32"), uint32_t(std::min<int64_t>(tiles128, kLoopGrid)), kBlock, as_hip(stream), rargs);
+      // eight waves to a tile while there is a unit for each and (128 rows or more) K gives them slices; four beyond
+      const bool tall = M <= 128 && rounds <= tuning::kF32RowsRounds && rows_us <= tiles_us, eight = small_tiles <= units && (M <= 128 || K >= 256);
       return launch(st, KernelName(tall ? (M <= 64 ? "mtrt_gemm_dense_rows64_tall_f32" : "mtrt_gemm_dense_rows128_tall_f32") :
                                    !eight ? "mtrt_gemm_dense_mfma_f32" : M <= 64 ? "mtrt_gemm_dense_rows64_f32" : "mtrt_gemm_dense_rows128_f32"),
                     uint32_t(std::min<int64_t>(tall ? tiles32 : 8 * ((small_tiles + 7) / 8), kLoopGrid)), tall ? (M <= 64 ? 512 : 256) : eight ? 512 : 256,

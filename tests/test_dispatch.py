@@ -226,3 +226,11 @@ def test_large_tiles_cover_the_output(gpu, pkg, M, N):
     assert gpu.lib.mtrt_hip_linear_dense(None, 256, 256, None, 256, pkg.F16, M, 4096, N) == 0
     assert [name for name, _, _ in gpu.sizes] == ["mtrt_gemm_w8a8_nk", "mtrt_gemm_dense_mfma_f16"]
     assert all(grid >= tiles for _, grid, _ in gpu.sizes)
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(2048, 4096, 11008, "t256x128"), (4096, 4096, 4096, "t256x128"), (2048, 512, 8192, "t128x128"), (128, 256, 65536, "t128x128"),
+                                          (512, 4096, 4096, "mfma"), (300, 3072, 2048, "mfma"), (1 << 19, 4096, 4096, "t128x128"), (1 << 19, 2048, 1024, "t128x128")])
+def test_float32_products_take_the_tiles_that_fill_the_chip(gpu, pkg, M, K, N, kernel):
+    """... of 256 x 128 only while both operands lie below 4 GiB."""
+    assert gpu.lib.mtrt_hip_linear_dense(None, 256, 256, None, 256, pkg.F32, M, K, N) == 0
+    assert gpu.launches[-1][0] == "mtrt_gemm_dense_%s_f32" % kernel

@@ -111,3 +111,29 @@ def test_whole_slices_of_float32(pkg, M):
         assert {rows + "_f32", rows + "_tall_f32"} <= kernels
     else:
         assert kernels == {"mtrt_gemm_dense_rows128_f32", "mtrt_gemm_dense_mfma_f32"}
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [(1024, 32, 4097, "t128x128"), (129, 96, 30001, "t128x128"), (2001, 160, 3968, "t128x128"), (3970, 1056, 1023, "t128x128"),
+                                          (2047, 1664, 3999, "t256x128"), (1793, 2080, 4096, "t256x128"), (3841, 1760, 1921, "t256x128")])
+def test_large_tiles_of_float32(pkg, M, K, N, kernel):
+    """Products of whole slices that fill the chip with larger tiles: the last tiles of rows and of columns hold one of them, all but one, half; fewer slices
+    than parts of their sum, slices that the parts do not divide."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    x = torch.randn((M, K), generator=g, device="cuda")
+    w = torch.randn((N, K), generator=g, device="cuda") * 0.3
+    for bias in (True, False):
+        b = torch.randn(N, generator=g, device="cuda") if bias else None
+        out = torch.full((M * N + 128,), 7.0, device="cuda")
+        y = pkg.linear_dense(x, w, b, out[64:64 + M * N].view(M, N))
+        assert pkg.last_kernel() == "mtrt_gemm_dense_%s_f32" % kernel
+        ref, mass = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+        if bias:
+            ref, mass = ref + b.double(), mass + b.double().abs()
+        bad = int(((y.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * mass).logical_not().sum())
+        assert bad == 0, bad
+        assert bool((out[:64] == 7).all()) and bool((out[64 + M * N:] == 7).all())
+        # the error of all sums together, in 2^-24 of the result: a chain of n random terms errs by 0.29 sqrt(n) (measured, K = 4096: 19), four
+        # chains of n / 4 by half of that; the rounding of a result by 0.3 to 0.6
+        chain = (K + 127) // 128 * 32
+        assert float((y.double() - ref).norm() / ref.norm()) < 2.0 ** -24 * (0.6 + 0.36 * chain ** 0.5)
