@@ -373,8 +373,8 @@ struct ExactDivisor {
   // clamp is one v_med3 of -x, which gives the least operand for a NaN: that of -x is the greatest of x, as above.
   // q1 above is enough here.  It differs from the correctly rounded quotient at most where x/s is within a hair of the middle of
   // two floats, and a code only where one of those two is the middle of two codes (or of the whole numbers, or of the f16 values,
-  // that a float target is rounded to first): a number of at most 12 significant bits.  Of the three x nearest to each such
-  // middle, for all 2^23 mantissas of s, all 2^11 numbers of 12 bits and both neighbours (1.03e11 quotients), none differs.
+  // that a float target is rounded to first): a number of at most 12 significant bits.  Of the three x nearest to s times each such
+  // number and each such middle, for all 2^23 mantissas of s (1.5e11 quotients, tests/test_quotient_to_codes.py), none differs.
   // With the rounding in enc this is 5 instructions an element to a code and one to gather it; with both corrections and
   // the arithmetic on -q it was 8, and minimum, maximum, rounding, clamp, sign, conversion, mask and shift made it 18: a
   // tensor of 45 M bf16 took 18 us of the vector units.
