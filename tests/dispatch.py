@@ -39,7 +39,10 @@ def build(folder):
 class Dispatch:
     """The library with a state of its own (a copy of the file: a loaded library's state is the process's).  `launches`
     collects (kernel, stream, its (splits, per, partial, tickets) or the address of its reduction block or None), `fills` the
-    clears (address, words, stream), `sizes` every launch's (kernel, grid, block)."""
+    clears (address, words, stream), `sizes` every launch's (kernel, grid, block), `forms` the run-time arguments by which some kernels
+    choose what they do."""
+
+    _FORMS = {"mtrt_gemm_dense_rows32_f32": (7, 8), "mtrt_gemm_dense_edge_f32": (7,), "mtrt_gemm_dense_edge_f16": (7,), "mtrt_gemm_dense_edge_bf16": (7,)}
 
     def __init__(self, pkg, path, copy):
         shutil.copy(path, copy)
@@ -55,6 +58,7 @@ class Dispatch:
         self.launches = []
         self.fills = []
         self.sizes = []
+        self.forms = []
         self._callback = _CALLBACK(self._launched)
         self.lib.fake_set_launch_callback(self._callback)
         assert self.lib.mtrt_hip_init() == 0
@@ -73,6 +77,8 @@ class Dispatch:
     def _launched(self, name, grid, block, stream, args):
         name = name.decode()
         self.sizes.append((name, grid, block))
+        if name in self._FORMS:
+            self.forms.append((name,) + tuple(ctypes.cast(args[i], ctypes.POINTER(_i32))[0] for i in self._FORMS[name]))
         if name == "mtrt_fill":
             self.fills.append((ctypes.cast(args[0], ctypes.POINTER(_vp))[0], ctypes.cast(args[1], ctypes.POINTER(_i64))[0], stream))
             return

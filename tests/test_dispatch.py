@@ -4,6 +4,7 @@ whatever reason, runs unsplit, a reduction recorded when there are no more takes
 import pytest
 
 import dispatch
+from test_gpu_dense_ragged import RAGGED, WHOLE, ragged_lengths
 from test_gpu_gemm_split import DENSE_TILES, W4_TILES, W8_TILES
 
 TICKETS = 512 * 4                                                    # bytes a stream keeps
@@ -234,3 +235,40 @@ def test_float32_products_take_the_tiles_that_fill_the_chip(gpu, pkg, M, K, N, k
     """... of 256 x 128 only while both operands lie below 4 GiB."""
     assert gpu.lib.mtrt_hip_linear_dense(None, 256, 256, None, 256, pkg.F32, M, K, N) == 0
     assert gpu.launches[-1][0] == "mtrt_gemm_dense_%s_f32" % kernel
+
+
+@pytest.mark.parametrize("M", [9, 32])
+def test_up_to_32_rows_of_float32_take_every_form(gpu, pkg, M):
+    """One kernel's name: 32-column tiles, or groups of eight rows on the vector units whose waves share K or take columns of their own.
+    The shapes of the GPU test take all three, in launches of the workgroups that each form needs."""
+    seen = set()
+    for K, N in WHOLE:
+        assert gpu.lib.mtrt_hip_linear_dense(None, 256, 256, None, 256, pkg.F32, M, K, N) == 0
+        (name, grid, block), (_, tiles, shared) = gpu.sizes[-1], gpu.forms[-1]
+        assert name == "mtrt_gemm_dense_rows32_f32"
+        if tiles:
+            assert (grid, block) == ((N + 31) // 32, 512)
+        else:
+            blocks, groups = (N + (3 if shared else 15)) // (4 if shared else 16), (M + 7) // 8
+            assert block == 256 and grid % (8 * groups) == 0 and blocks <= grid // groups < blocks + 8
+        seen.add("tiles" if tiles else "shared" if shared else "own")
+    assert seen == {"tiles", "shared", "own"}
+
+
+@pytest.mark.parametrize("dtype,item", [("F32", 4), ("F16", 2), ("BF16", 2)])
+def test_rows_that_are_no_whole_slices_take_every_form(gpu, pkg, dtype, item):
+    """One kernel's name: 128 x 128 tiles, 32 x 32 tiles on four waves and (float32) on eight, those only for rows of 16 bytes and more."""
+    seen = set()
+    for M, N in RAGGED:
+        for K in ragged_lengths(item):
+            assert gpu.lib.mtrt_hip_linear_dense(None, 256 + item, 256 + item, None, 256, getattr(pkg, dtype), M, K, N) == 0
+            name, grid, block = gpu.sizes[-1]
+            if not name.startswith("mtrt_gemm_dense_edge_"):
+                continue
+            waves = gpu.forms[-1][1]
+            side = 32 if waves else 128
+            tiles = ((M + side - 1) // side) * ((N + side - 1) // side)
+            assert block == (64 * waves or 256) and (tiles <= grid < tiles + 8 if waves else grid == tiles)
+            assert K * item >= 16 or not waves
+            seen.add(waves)
+    assert seen == ({0, 4, 8} if dtype == "F32" else {0, 4})

@@ -5,6 +5,14 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 EPS = {"float32": 2.0 ** -24, "float16": 2.0 ** -11, "bfloat16": 2.0 ** -8}
+# (that these take every form of their kernels: test_dispatch.py)
+RAGGED = [(1, 1), (5, 300), (31, 33), (33, 31), (64, 1000), (130, 8209), (300, 1000), (1500, 4100)]
+WHOLE = ((32, 33), (64, 8193), (224, 31), (256, 1000), (288, 16385), (512, 8200), (1056, 2049), (4128, 65))
+
+
+def ragged_lengths(item_bytes):
+    slice_, vec = 128 // item_bytes, 16 // item_bytes
+    return [1, vec - 1, vec, vec + 1, slice_ - 1, slice_ + 1] + [s * slice_ + e for s, e in ((1, vec), (2, -1), (4, 1), (7, vec + 1), (8, 3), (9, -vec), (17, 1))]
 
 
 def _inside(torch, t, lead):
@@ -16,13 +24,11 @@ def _inside(torch, t, lead):
 
 
 @pytest.mark.parametrize("dname", ["float32", "float16", "bfloat16"])
-@pytest.mark.parametrize("M,N", [(1, 1), (5, 300), (31, 33), (33, 31), (64, 1000), (130, 8209), (300, 1000), (1500, 4100)])
+@pytest.mark.parametrize("M,N", RAGGED)
 def test_ragged_rows(pkg, M, N, dname):
     import torch
     td = getattr(torch, dname)
-    slice_, vec = 128 // td.itemsize, 16 // td.itemsize
-    lengths = [1, vec - 1, vec, vec + 1, slice_ - 1, slice_ + 1] + [s * slice_ + e for s, e in ((1, vec), (2, -1), (4, 1), (7, vec + 1), (8, 3), (9, -vec), (17, 1))]
-    for i, K in enumerate(lengths):
+    for i, K in enumerate(ragged_lengths(td.itemsize)):
         g = torch.Generator(device="cuda").manual_seed(1000 * M + i)
         x = _inside(torch, torch.randn((M, K), generator=g, device="cuda").to(td), i % 5)
         w = _inside(torch, (torch.randn((N, K), generator=g, device="cuda") * 0.3).to(td), (3 * i) % 7)
@@ -90,7 +96,7 @@ def test_whole_slices_of_float32(pkg, M):
     tiles are fewer and more than the compute units, and whose columns alone are (the form that takes all rows at once)."""
     import torch
     kernels = set()
-    for i, (K, N) in enumerate(((32, 33), (64, 8193), (224, 31), (256, 1000), (288, 16385), (512, 8200), (1056, 2049), (4128, 65))):
+    for i, (K, N) in enumerate(WHOLE):
         g = torch.Generator(device="cuda").manual_seed(100 * M + i)
         x = torch.randn((M, K), generator=g, device="cuda")
         w = torch.randn((N, K), generator=g, device="cuda") * 0.3
