@@ -1119,14 +1119,18 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
 // _b64) ; M * K < 2^31.
 // grid = one or two workgroups per compute unit, at most ceil(N / 16), block = 256: workgroup g owns tiles / grid consecutive
 // 16-column tiles (the first tiles % grid workgroups one more), three at a time.
-// What bounds it: four waves, one per SIMD, each with eight of the 32 slices at K = 4096, N = 11008, and a wave alone on its SIMD
-// issues one instruction in four cycles, whichever it is.  A slice of three tiles was 255 of them (168 to dequantise, 12 MFMAs,
-// 47 scalar, 11 waits for an operand made just before) and is 228; the last slices of a wave whose number is no multiple of
-// four came one at a time, a trip to memory each, and are now on their way with the others; up to four or eight rows take
-// a quarter or half of the activations' loads.  us, before and now, (M, K, N): (16, 4096, 11008) 9.1 and 8.7, (1, 4096, 11008)
-// 8.2 and 7.1, (16, 4096, 4096) 5.6 and 5.5, (1, 4096, 4096) 4.9 and 4.2, (2, 9600, 3136) 9.2 and 6.2, (13, 1152, 14464) 8.8 and
-// 6.6, (16, 5120, 13824) 16.9 and 13.4; in blocks of 64, against the kernel above: (2, 6656, 960) 9.3 and 4.9, (16, 4096, 11008)
-// 10.6 and 9.2, (13, 1152, 14464) 6.4 and 5.3.  Eight waves (two per SIMD) are no faster: 10.4 us at (16, 4096, 11008).
+// What its time is, from timestamps in a copy of the kernel, (16, 4096, 11008): four waves, one per SIMD, each with eight of the 32
+// slices.  The median wave, us from the launch's first: entered 0.4, three slices asked for 1.7, the first landed 2.3, the eighth done 6.4
+// (0.5 each, of which its 228 instructions, one in four cycles, are 0.38), partial tiles added and stored 7.2; the slowest wave 8.4.  (1, 4096,
+// 11008), two workgroups to a unit: 0.5, 1.1, 1.9, 4.9 (0.4 each), 5.5; 7.1.  So neither issue nor the bytes alone: a third is the way
+// to the first slice, most of it asking for sixteen rows.
+// The last slices of a wave whose number is no multiple of four are on their way with the others, up to four or eight rows take a
+// quarter or half of the activations' loads, and workgroups follow the rows (w4a16 in clusters.cpp).  us, with the last slices one at
+// a time, a trip to memory each, sixteen rows' loads and a workgroup to a unit, and now, (M, K, N): (1, 4096, 11008) 8.3 and 7.5, (1,
+// 4096, 4096) 4.9 and 4.6, (2, 9600, 3136) 9.2 and 6.3, (13, 1152, 14464) 9.0 and 5.3, (16, 5120, 13824) 17.0 and 13.4; where none of
+// that applies, (16, 4096, 11008), 9.0 and 9.0, although a slice of three tiles was 255 instructions.  In blocks of 64, against the
+// kernel above: (2, 6656, 960) 9.4 and 5.0, (16, 4096, 11008) 10.1 and 9.2, (13, 1152, 14464) 6.3 and 5.5.  Eight waves (two per
+// SIMD) are no faster: 10.4 us at (16, 4096, 11008).
 constexpr int kStripWaves = 4;
 template <int G, int SC>
 __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,

@@ -389,7 +389,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
       t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
   // What lies past the row becomes -infinity where it is loaded: it changes no maximum and its exponential is zero, and the passes
-  // below need not tell it from the row (us, f16 [1084, 50000] 61.5 -> 53.7, f32 [2000, 25001] 102 -> 97; [48000, 1500] 51.1 -> 50.6, bf16 [200, 8191] 7.4 -> 7.0).
+  // below need not tell it from the row (us, f16 [1084, 50000] 61.2 -> 53.0, f32 [2000, 25001] 102 -> 97, bf16 [200, 8191] 7.5 -> 7.1; [48000, 1500] as before).
   if (!FULL) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {

@@ -338,8 +338,8 @@ def test_dense_linear_against_float64(tp, pkg, dname):
         lin = tp.Linear(K, N, dtype=d)
         lin.weight, lin.bias = tp.Tensor(w, dtype=d), tp.Tensor(b, dtype=d)
         out = lin(tp.Tensor(x, dtype=d)).torch()
-        # 16-bit weights in fragment order; float32 ones [N, K]: up to 128 rows the kernels that read the weights once, above
-        # the 256 x 256 tile loop.  Rows that are no whole 128-byte slices of K: 128 x 128 tiles with element-aligned loads
+        # 16-bit weights in fragment order; float32 ones [N, K]: whole 128-byte slices of K by the number of rows, other rows with
+        # element-aligned loads
         mfma = K % (32 if dname == "float32" else 64) == 0
         rows = int(np.prod(lead))
         kernel, short = pkg.last_kernel(), {"float32": "f32", "float16": "f16", "bfloat16": "bf16"}[dname]
