@@ -761,7 +761,7 @@ int32_t mtrt_hip_dynamic_quantize_dequantize(mtrt_stream_t stream, const void *x
     // One or two workgroups read all of x instead of waiting for each other, unless results lie over it: us, with the exchange and so, one
     // workgroup (f32 [3, 1000]) 3.2, 2.4, two (bf16 [31, 1344]) 6.9, 6.0, three (bf16 [64, 1344]) 6.1, 6.25, four (f32 [64, 960]) 5.2, 5.3.
     const int64_t bytes = n * float_bytes(x_dtype);
-    const bool alone = grid <= 2 && apart(x, bytes, q, n) && (!y || apart(x, bytes, y, bytes));
+    const bool alone = nv == 4 && grid <= 2 && apart(x, bytes, q, n) && (!y || apart(x, bytes, y, bytes));
     int32_t limit = alone ? -1 : g_wait_limit.load();
     void *args[] = {&x, &q, &y, &n, &qmax, &amax_out, &scale_out, &slot, &flags, &limit};
     return launch(st, KernelName("mtrt_dynqdq_") + xn + "_" + code_name(q_dtype) + "_v" + nv, grid, 1024,

@@ -1,0 +1,26 @@
+"""What the compiled kernels ask of the device, from the code object's own metadata: a one-launch dynamic quantization holds its part of the
+tensor in registers, and private memory beside them means that some of it is written out and read back (16 vectors a lane, f32 of 14 Mi
+elements: 20.9 us with none, 22.9 with 164 bytes)."""
+import os
+import re
+import subprocess
+
+import pytest
+
+
+def metadata(pkg, tmp_path):
+    llvm = "/opt/rocm/llvm/bin/"
+    module = os.path.join(os.path.dirname(pkg.__file__), "lib", "mtrt_kernels.hsaco")
+    try:
+        targets = subprocess.run([llvm + "clang-offload-bundler", "--list", "--type=o", "--input=" + module], capture_output=True, text=True, check=True).stdout
+        target = next(t for t in targets.split() if "gfx950" in t)
+        out = str(tmp_path / "kernels.elf")
+        subprocess.run([llvm + "clang-offload-bundler", "--unbundle", "--type=o", "--targets=" + target, "--input=" + module, "--output=" + out], check=True)
+        return subprocess.run([llvm + "llvm-readelf", "--notes", out], capture_output=True, text=True, check=True).stdout
+    except FileNotFoundError:
+        pytest.skip("no LLVM tools beside the compiler")
+
+
+def test_one_launch_dynamic_quantization_stays_in_registers(pkg, tmp_path):
+    private = dict(re.findall(r"\.name:\s+(mtrt_dynqdq_\S+)\n\s+\.private_segment_fixed_size:\s+(\d+)", metadata(pkg, tmp_path)))
+    assert len(private) == 10 and {name: size for name, size in private.items() if size != "0"} == {}
