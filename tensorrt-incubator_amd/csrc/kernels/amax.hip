@@ -23,6 +23,7 @@
 // (arrival ticket, running max) pair in its first eight bytes, all zero on entry; whoever arrives last at a
 // pair restores its zeros, so back-to-back launches on one stream need no memset.
 #include "common.hpp"
+#include "read_twice.hpp"
 
 using namespace mtrt_dev;
 
@@ -33,17 +34,16 @@ constexpr int kAmaxUnroll = 4;     // 128-bit loads in flight per lane per step
 constexpr uint32_t kAmaxFanIn = 32;     // first-level groups of the cross-workgroup arrival tree
 constexpr uint32_t kAmaxLineWords = 32; // one 128-byte line per (ticket, max) pair
 
-// The pass that quantizes by this maximum reads the tensor again, beginning at its end (last_first_piece in common.hpp), so the
-// last 32 MiB, what the eight L2s hold, are read by ordinary loads, which leaves them there; what lies in front goes past
-// the caches.  amax and the fused pass behind it, bf16 -> f8, us, with contiguous chunks per workgroup and the fused pass
-// forwards; in pieces and from the end with nothing left in the L2s; with 16, 24, 32 and 96 MiB left:
+// The pass that quantizes by this maximum reads the tensor again, forwards, so this one goes from the end to the front (read_twice.hpp)
+// and reads the front 32 MiB by ordinary loads, which leave them in the L2s, and what lies behind past the caches.  amax and the fused
+// pass behind it, bf16 -> f8, us, with contiguous chunks per workgroup, forwards; in pieces with nothing left in the L2s for a second pass
+// from where this one ended; with 16, 24, 32 and 96 MiB left:
 //   33 MB   24.8   25.0   22.8   21.8   20.3   20.7
 //   67 MB   41.5   40.2   38.7   38.4   38.6   37.3
 //   134 MB  73.8   73.9   71.6   70.7   70.8   72.6
 // (amax, NVFP4 and back of 67 MB: 43.5, 41.4, 40.2, 39.1, 38.0, 37.7; f32 -> i8 of 67 MB 41.5, 39.7, 38.9, 36.4, 36.0, 33.0).
 // It turns where both passes together fill the Infinity Cache: 200 MiB 109.4 and (32 left) 108.0, 224 MiB 121.3 and 122.9,
-// 256 MiB 136.6 and 144.9.  Hence kReadTwiceBelow, above which all loads go past the caches and the next pass runs forwards.
-constexpr int64_t kAmaxKept = (int64_t(32) << 20) / 16;   // in vectors
+// 256 MiB 136.6 and 144.9.  Hence kReadTwiceBelow, above which all loads go past the caches.
 
 template <typename X> struct AbsBits;
 template <> struct AbsBits<F32> {  // returns max over the 4 floats, as f32 bit pattern
@@ -106,6 +106,51 @@ __device__ __forceinline__ bool arrive(uint32_t* pair, uint32_t expected, uint32
   return true;
 }
 
+// All whole vectors, this workgroup's turns of TRIPS * kAmaxUnroll a lane.  PAST: all of them past the caches.
+template <typename X, int TRIPS, bool PAST>
+__device__ __forceinline__ void walk(const u32x4* __restrict__ xv, int64_t nvec, uint32_t& m) {
+  using A = AbsBits<X>;
+  constexpr int kStep = kAmaxUnroll * kAmaxThreads;
+  const AmaxTurns<TRIPS * kAmaxUnroll> turns(nvec);
+  const int64_t kept = PAST ? turns.whole : turns.first_kept(kReadTwiceKept / 16);
+  int64_t turn = blockIdx.x;
+  u32x4 t[kAmaxUnroll];
+  const auto fold = [&] {
+#pragma unroll
+    for (int u = 0; u < kAmaxUnroll; ++u) { const uint32_t a = A::of(t[u]); m = m > a ? m : a; }
+  };
+  // (two loops: in the branches of one, the loads would be merged into ordinary ones)
+  for (; turn < kept; turn += gridDim.x) {
+    const u32x4* from = xv + turns.first(turn) + threadIdx.x;
+#pragma unroll 1
+    for (int h = 0; h < TRIPS; ++h, from += kStep) {
+#pragma unroll
+      for (int u = 0; u < kAmaxUnroll; ++u) t[u] = __builtin_nontemporal_load(from + u * kAmaxThreads);
+      fold();
+    }
+  }
+  for (; turn < turns.whole; turn += gridDim.x) {
+    const u32x4* from = xv + turns.first(turn) + threadIdx.x;
+#pragma unroll 1
+    for (int h = 0; h < TRIPS; ++h, from += kStep) {
+#pragma unroll
+      for (int u = 0; u < kAmaxUnroll; ++u) t[u] = from[u * kAmaxThreads];
+      fold();
+    }
+  }
+  for (; turn < turns.turns; turn += gridDim.x) {      // the tensor's end: lanes past it repeat its last vector
+    const int64_t first = turns.first(turn);
+    for (int h = 0; h < TRIPS && first + h * kStep < nvec; ++h) {
+#pragma unroll
+      for (int u = 0; u < kAmaxUnroll; ++u) {
+        const int64_t v = first + h * kStep + u * kAmaxThreads + threadIdx.x;
+        t[u] = xv[v < nvec ? v : nvec - 1];
+      }
+      fold();
+    }
+  }
+}
+
 template <typename X>
 __device__ __forceinline__ void amax_body(const typename X::storage* __restrict__ x, int64_t n, float qmax,
                                           float* __restrict__ amax_out, float* __restrict__ scale_out,
@@ -113,49 +158,18 @@ __device__ __forceinline__ void amax_body(const typename X::storage* __restrict_
   using A = AbsBits<X>;
   // Elements before the first 16-byte boundary ("head") and after the last full
   // vector ("tail") are taken one per lane by workgroup 0; everything between is
-  // streamed as 128-bit vectors, in pieces of 32 KiB that the workgroups take in turn (16 KiB beyond kReadTwiceBelow:
-  // f32 of 256 MiB 41.8 and 41.1 us, 320 MiB 51.5 and 50.4).
+  // streamed as 128-bit vectors, in turns of 32 KiB (16 KiB beyond kReadTwiceBelow: f32 of 256 MiB 41.8 and 41.1 us, 320 MiB
+  // 51.5 and 50.4).
   constexpr int kElemBytes = 16 / A::kPerVec;
-  constexpr int64_t kStep = int64_t(kAmaxThreads) * kAmaxUnroll;
   int64_t head = int64_t((16u - uint32_t(reinterpret_cast<uintptr_t>(x) & 15u)) & 15u) / kElemBytes;
   head = head < n ? head : n;
   const int64_t nvec = (n - head) / A::kPerVec;
   const u32x4* __restrict__ xv = reinterpret_cast<const u32x4*>(x + head);
-  const bool large = nvec * 16 >= kReadTwiceBelow;
-  const int64_t piece = large ? kStep : 2 * kStep, next = int64_t(gridDim.x) * piece;
-  const int64_t past = large ? nvec : nvec - kAmaxKept;   // up to here past the caches
   uint32_t m = 0;
-  int64_t p = int64_t(blockIdx.x) * piece;
-  u32x4 t[kAmaxUnroll];
-  const auto fold = [&] {
-#pragma unroll
-    for (int u = 0; u < kAmaxUnroll; ++u) { const uint32_t a = A::of(t[u]); m = m > a ? m : a; }
-  };
-  // (two loops: in the branches of one, the loads would be merged into ordinary ones)
-  for (; p < past && p + piece <= nvec; p += next) {
-#pragma unroll 1
-    for (int64_t h = 0; h < piece; h += kStep) {
-#pragma unroll
-      for (int u = 0; u < kAmaxUnroll; ++u) t[u] = __builtin_nontemporal_load(xv + p + h + u * kAmaxThreads + threadIdx.x);
-      fold();
-    }
-  }
-  for (; p + piece <= nvec; p += next) {
-#pragma unroll 1
-    for (int64_t h = 0; h < piece; h += kStep) {
-#pragma unroll
-      for (int u = 0; u < kAmaxUnroll; ++u) t[u] = xv[p + h + u * kAmaxThreads + threadIdx.x];
-      fold();
-    }
-  }
-  for (int64_t h = p; h < nvec && h < p + piece; h += kStep) {   // the last piece: lanes past its end repeat its last vector
-#pragma unroll
-    for (int u = 0; u < kAmaxUnroll; ++u) {
-      const int64_t v = h + u * kAmaxThreads + threadIdx.x;
-      t[u] = xv[v < nvec ? v : nvec - 1];
-    }
-    fold();
-  }
+  if (nvec * 16 >= kReadTwiceBelow)
+    walk<X, 1, true>(xv, nvec, m);
+  else
+    walk<X, 2, false>(xv, nvec, m);
   if (blockIdx.x == 0 && threadIdx.x < 2 * A::kPerVec) {
     const int64_t tail0 = head + nvec * A::kPerVec;
     const int64_t e = threadIdx.x < A::kPerVec ? int64_t(threadIdx.x) : tail0 + (threadIdx.x - A::kPerVec);

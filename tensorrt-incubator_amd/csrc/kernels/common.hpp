@@ -87,21 +87,6 @@ __device__ __forceinline__ uint32_t wave_of_block(uint32_t block) {
 __device__ __forceinline__ uint32_t wave_in_launch() { return wave_of_block(blockIdx.x); }
 __device__ __forceinline__ uint32_t waves_in_launch() { return gridDim.x * (block_threads() / kWave); }
 
-// Which of the launch's n pieces workgroup `id` takes in a pass that follows another over the same tensor.  Workgroups are dealt
-// to the eight XCDs in turn, each with an L2 of its own (4 MiB) that keeps what a launch has READ there for the next one
-// (what it has written it does not).  The second pass finds it if it takes the same bytes on the same XCD - PER
-// neighbouring pieces go to one, as many as make up the 32 KiB that a workgroup of the amax pass takes at a time - and
-// begins where the first pass ended: at the tensor's end.  Any n: the last n % (8 PER) pieces stay where they are.
-// x_bytes: tensors above kReadTwiceBelow are read forwards again, see amax.hip.
-constexpr int64_t kReadTwiceBelow = int64_t(192) << 20;
-template <uint32_t PER>
-__device__ __forceinline__ uint32_t last_first_piece(uint32_t id, uint32_t n, int64_t x_bytes) {
-  const uint32_t full = n & ~(8 * PER - 1);
-  if (id >= full || uint32_t(x_bytes >> 20) >= uint32_t(kReadTwiceBelow >> 20)) return id;   // (in 32 bits: scalar comparisons)
-  const uint32_t k = id >> 3;
-  return full - (k / PER + 1) * (8 * PER) + (id & 7) * PER + k % PER;
-}
-
 // f8E4M3FN (OCP) pair conversion in hardware: RNE.  Inputs are pre-clamped to
 // [-448, 448] by every caller, so the saturation rule of the instruction is
 // never exercised.

@@ -123,8 +123,7 @@ __device__ __forceinline__ void quantize_body(const typename X::storage* __restr
   uint8_t* my_codes = lds + wave * (kSpanCodes + kSpanScales);
   uint8_t* my_scales = my_codes + kSpanCodes;
   __shared__ float inverse_scale[256];
-  // from the tensor's end, where the amax pass ended (a workgroup takes 32 KiB)
-  const int64_t span = (int64_t(last_first_piece<1>(blockIdx.x, gridDim.x, nvec * 16)) * (kThreads / 64) + wave) * (kTrips * 64);   // first vector of this wave
+  const int64_t span = (int64_t(blockIdx.x) * (kThreads / 64) + wave) * (kTrips * 64);   // first vector of this wave (a workgroup takes 32 KiB, see read_twice.hpp)
   const float s_enc = 2688.0f / *tensor_amax;
   fill_inverse_scales(inverse_scale, s_enc);
   if (span >= nvec) return;                            // whole wave

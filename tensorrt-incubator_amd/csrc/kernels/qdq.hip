@@ -30,6 +30,7 @@
 // per trip (16 elements), all loads issued before the first use.  The "_any"
 // variants take any shape and alignment, one element per lane.
 #include "common.hpp"
+#include "read_twice.hpp"
 
 using namespace mtrt_dev;
 
@@ -214,10 +215,13 @@ __device__ __forceinline__ void unpack4<F8>(uint32_t w, float* v) {
 //   the launch ends and are written back then.  With the amax in front, bf16 -> f8: 4 Mi 9.2 and 10.0, 9 Mi 13.7 and 14.4, 16 Mi
 //   20.6 and 21.0, 24 Mi 30.8 and 30.8, 48 Mi 56.6 and 54.6, 64 Mi 74.5 and 70.8, 128 Mi 149 and 138; f32 -> i8: 9 Mi and 32 Mi
 //   22.1 and 22.1, 67.0 and 66.6
-//   a quantize with one scale: kept, a dequantize reads them next (both, bf16 -> i4 of 22, 43 and 128 Mi 28.2 and 25.5, 49.4 and 46.6,
-//   131 and 123; f32 -> i8 of 22 and 64 Mi 42.8 and 39.6, 113 and 106; the quantize alone 43 Mi 25.1 and 26.4)
+//   a quantize with one scale (keep_plain): kept above 14 Mi codes, where the dequantize that reads them next gains more than the
+//   quantize loses (both, then the quantize alone, past and kept, bf16 -> i8: 6 Mi 9.1 and 9.1, 5.3 and 5.8; 12 Mi 14.0 and 14.0, 8.9 and 9.0;
+//   16 Mi 17.6 and 17.4, 10.9 and 11.3; 24 Mi 25.1 and 24.3, 15.2 and 15.5; 48 Mi 52.4 and 50.8, 27.0 and 28.5; 128 Mi 131 and 121, 65.4 and 64.9;
+//   f32 -> i8 of 24 and 64 Mi 41.7 and 40.7, 110.8 and 105.6, alone 22.7 and 23.1, 55.7 and 56.8)
 //   ... behind its amax, with no dequantize asked for (kFlagCodesPast): not kept (bf16 -> f8 of 9, 16, 32 and 64 Mi 12.5 and 13.3,
-//   16.6 and 18.5, 29.7 and 31.2, 54.2 and 57.2): dirty lines take the place of the end of x in the L2s
+//   16.6 and 18.5, 29.7 and 31.2, 54.2 and 57.2): dirty lines take the place of what the amax left of x in the L2s
+__device__ __forceinline__ bool keep_plain(int64_t n) { return n > (int64_t(14) << 20); }
 __device__ __forceinline__ bool keep_fused(int64_t n) { return n > (int64_t(24) << 20); }
 template <bool KEEP, typename T> __device__ __forceinline__ void store_codes(T v, T* p) {
   if (KEEP) *p = v;
@@ -527,14 +531,13 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   const int lane = threadIdx.x & (kWave - 1);
   // The fused pass keeps the wave's number per lane: with scalar numbers it was the slower (f16 -> f8 of 14 Mi elements with the amax
   // in front 23.2 -> 24.3 us, bf16 of 128 Mi 155 -> 158), where a quantize and a dequantize of 4 and 128 Mi gained (7.4 -> 7.3, 133 -> 131).
-  // one scale for all may come from an amax pass, which left the end of x in the L2s
-  const uint32_t piece = KIND == kUniform && MODE != 1 ? last_first_piece<8 / sizeof(typename X::storage)>(blockIdx.x, gridDim.x, n * int64_t(sizeof(typename X::storage)))
-                                                    : blockIdx.x;
+  // one scale for all may come from an amax pass, and a dequantize follows the quantize: see read_twice.hpp
+  const uint32_t piece = KIND == kUniform ? piece_of<8 / sizeof(typename X::storage)>(blockIdx.x, gridDim.x, n * int64_t(sizeof(typename X::storage))) : blockIdx.x;
   const int64_t wave = MODE == 2 ? (int64_t(piece) * blockDim.x + threadIdx.x) / kWave : int64_t(wave_of_block(piece));
   const int64_t nwaves = MODE == 2 ? int64_t(gridDim.x) * blockDim.x / kWave : int64_t(waves_in_launch());
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
   const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;
-  const bool keep = MODE == 2 ? keep_fused(n) : KIND != kUniform || !(flags & kFlagCodesPast);
+  const bool keep = MODE == 2 ? keep_fused(n) : KIND != kUniform || (keep_plain(n) && !(flags & kFlagCodesPast));
 
   for (int64_t base = wave * (kWave * J); base < ngroups; base += nwaves * (kWave * J)) {
     // Row scales: the row of the trip's first group by two divisions for the whole wave, the others from there - a lane's
