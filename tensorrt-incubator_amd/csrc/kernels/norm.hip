@@ -263,10 +263,9 @@ __device__ __forceinline__ float group_reduce(float v, Op op, float* lds) {
 }
 
 // Whether vector j of any lane of this wave lies in the row (the same for the whole wave): what lies past it for all is not asked for, nor
-// worked on.  A row takes the kernel with the next power of two of vectors, so that may be near half of them.  us, before and after:
-// LayerNorm f16 [2000, 10240] 18.8, 17.2, [2000, 12001] 28.1, 26.5, [8000, 1500] 10.8, 10.1, f32 [4000, 5000] 33.6, 31.5; softmax f16
-// [4000, 9001] 36.2, 31.5, [2000, 20001] 40.6, 35.9, bf16 [1084, 43165] 64.0, 54.6; without it and the fill below, f32 rows of 16388 to
-// 32768 elements off whole vectors took twice the vectors too, for want of registers: [2000, 25001] 102, 76.9, [800, 18001] 41.5, 22.0.  ALL: every vector is worked on.
+// worked on.  A row takes the kernel with the next power of two of vectors, so that may be near half of them.  ALL: every vector is worked on;
+// which is the faster one stands beside row_form in clusters.cpp.  (Without either and the fill below, f32 softmax rows of 16388 to
+// 32768 elements off whole vectors took twice the vectors too, for want of registers: [2000, 25001] 102 us, [800, 18001] 41.5.)
 template <int THREADS, bool ALL>
 __device__ __forceinline__ bool wave_has(int j, int nvec) {
   return ALL || (THREADS > kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.x & ~63u)) : 0) + THREADS * j < nvec;
@@ -288,8 +287,8 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
   for (int j = 0; j < NV; ++j) {
     if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
-    if (!RAGGED || !ALL || nvec > 0)                   // (a row shorter than one vector: only the scalar elements below)
-      t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+    if (RAGGED && ALL && nvec == 0) t[j] = (u32x4){0u, 0u, 0u, 0u};   // a row shorter than one vector: only the scalar elements below
+    else t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
   const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
   const int64_t ec = int64_t(nvec) * E + lane;
@@ -355,7 +354,7 @@ __device__ __forceinline__ int64_t group_row() {
   return blockIdx.x;
 }
 
-template <typename X, int NV, int THREADS, bool RAGGED>
+template <typename X, int NV, int THREADS, bool RAGGED, bool ENDS>
 __device__ __forceinline__ void layernorm_group(const typename X::storage* __restrict__ x,
                                                 const typename X::storage* __restrict__ gamma,
                                                 const typename X::storage* __restrict__ beta,
@@ -363,10 +362,10 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
   __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  if (!RAGGED && d == int64_t(Vec<X>::kElems) * THREADS * NV)
+  if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
     layernorm_group_row<X, NV, THREADS, true, true, false>(x, gamma, beta, y, row, d, eps, lds);
-  else   // (ragged f32 rows: nearly full ones, [2000, 15001], 49.4 us with every vector worked on and 51.1 without)
-    layernorm_group_row<X, NV, THREADS, false, RAGGED && Vec<X>::kElems == 4, RAGGED>(x, gamma, beta, y, row, d, eps, lds);
+  else
+    layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED>(x, gamma, beta, y, row, d, eps, lds);
 }
 
 // KEEP: the exponentials stay in registers (f32) between the sum and the output pass; without it they are
@@ -451,19 +450,17 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   if (extra) Tile<X>::store1(y + row * d + ec, ee * inv);
 }
 
-template <typename X, int NV, int THREADS, bool RAGGED>
+template <typename X, int NV, int THREADS, bool RAGGED, bool ENDS>
 __device__ __forceinline__ void softmax_group(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                               int64_t rows, int64_t d) {
   __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
-  // (the branches cost a wave per row more than they save, f16 [48000, 1500] 50.6 and 53.9 us, and f32 in 256 lanes, [2000, 6001] 18.0 and 18.7)
-  constexpr bool kEnds = THREADS > (Vec<X>::kElems == 4 ? 256 : kWave);
   constexpr bool kKeep = THREADS <= 256 || NV * Vec<X>::kElems <= 64;
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  if (!RAGGED && d == int64_t(Vec<X>::kElems) * THREADS * NV)
+  if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
     softmax_group_row<X, NV, THREADS, true, true, kKeep, false>(x, y, row, d, lds);
   else
-    softmax_group_row<X, NV, THREADS, false, !kEnds, kKeep, RAGGED>(x, y, row, d, lds);
+    softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED>(x, y, row, d, lds);
 }
 
 // ---- any D, any alignment: one workgroup per row, row re-read from cache -------------
@@ -615,12 +612,17 @@ using namespace norm_cluster;
 // Ragged rows: mtrt_{layernorm,softmax}_<t>_u<THREADS>v<NV>, same arguments; any d >= 1 with d / E <= THREADS * NV,
 //   operands aligned to their element; THREADS <= 64 (NV = 1 below 64): grid = ceil(rows / (256 / THREADS)), block = 256;
 //   else grid = rows, block = THREADS.
-#define MTRT_NORM_GROUP_KERNELS(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK)                                       \
-  extern "C" __global__ void __launch_bounds__(BLOCK) mtrt_layernorm_##XN##_##TAG##THREADS##v##NV(             \
+#define MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK, ENDS, END)                        \
+  extern "C" __global__ void __launch_bounds__(BLOCK) mtrt_layernorm_##XN##_##TAG##THREADS##v##NV##END(        \
       const XT::storage* x, const XT::storage* gamma, const XT::storage* beta, XT::storage* y, int64_t rows,  \
-      int64_t d, float eps) { layernorm_group<XT, NV, THREADS, RAGGED>(x, gamma, beta, y, rows, d, eps); }    \
-  extern "C" __global__ void __launch_bounds__(BLOCK) mtrt_softmax_##XN##_##TAG##THREADS##v##NV(               \
-      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_group<XT, NV, THREADS, RAGGED>(x, y, rows, d); }
+      int64_t d, float eps) { layernorm_group<XT, NV, THREADS, RAGGED, ENDS>(x, gamma, beta, y, rows, d, eps); }
+#define MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK, ENDS, END)                          \
+  extern "C" __global__ void __launch_bounds__(BLOCK) mtrt_softmax_##XN##_##TAG##THREADS##v##NV##END(          \
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_group<XT, NV, THREADS, RAGGED, ENDS>(x, y, rows, d); }
+// (f32 LayerNorm at element alignment: nearly full rows, [2000, 15001], 49.4 us with every vector worked on and 51.1 without)
+#define MTRT_NORM_GROUP_KERNELS(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK)                                       \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK, (THREADS == 1024 && !(RAGGED && Vec<XT>::kElems == 4)), )               \
+  MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK, (THREADS == 1024), )
 #define MTRT_NORM_GROUPS_FOR_TYPE(XN, XT)                                                                      \
   MTRT_NORM_GROUP_KERNELS(XN, XT, 8, 256, g, false, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 256, g, false, 256)      \
   MTRT_NORM_GROUP_KERNELS(XN, XT, 8, 1024, g, false, 1024) MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 1024, g, false, 1024)  \
@@ -638,3 +640,27 @@ MTRT_NORM_FOR_TYPE(bf16, BF16)
 MTRT_NORM_GROUPS_FOR_TYPE(f32, F32)
 MTRT_NORM_GROUPS_FOR_TYPE(f16, F16)
 MTRT_NORM_GROUPS_FOR_TYPE(bf16, BF16)
+
+// Both forms of a kernel where either is the faster one for some rows (row_form in clusters.cpp).  The names above are those that work on every
+// vector, with 1024 lanes those that stop at the row's end; here the other ones: `e`, stop at the row's end (rows that do not fill
+// all vectors, or without a body of its own for those that do), and `a`, every vector.
+#define MTRT_NORM_OTHER_FORMS_16_BIT(XN, XT)                                                                   \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 256, g, false, 256, true, e) MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 16, 256, g, false, 256, true, e)  \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 4, 64, u, true, 256, true, e) MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 64, u, true, 256, true, e)       \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 16, 64, u, true, 256, true, e)                                                                        \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 256, u, true, 256, true, e) MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 16, 256, u, true, 256, true, e)    \
+  MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 8, 256, g, false, 256, true, e) MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 16, 256, g, false, 256, true, e)      \
+  MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 8, 256, u, true, 256, true, e) MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 16, 256, u, true, 256, true, e)
+#define MTRT_NORM_OTHER_FORMS(XN, XT)                                                                          \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 1024, g, false, 1024, false, a)                                       \
+  MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 8, 1024, g, false, 1024, false, a) MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 16, 1024, g, false, 1024, false, a)
+MTRT_LAYERNORM_GROUP_KERNEL(f16, F16, 16, 1024, g, false, 1024, false, a)
+MTRT_LAYERNORM_GROUP_KERNEL(bf16, BF16, 16, 1024, g, false, 1024, false, a)
+MTRT_NORM_OTHER_FORMS_16_BIT(f16, F16)
+MTRT_NORM_OTHER_FORMS_16_BIT(bf16, BF16)
+MTRT_NORM_OTHER_FORMS(f32, F32)
+MTRT_NORM_OTHER_FORMS(f16, F16)
+MTRT_NORM_OTHER_FORMS(bf16, BF16)
+MTRT_LAYERNORM_GROUP_KERNEL(f32, F32, 8, 256, g, false, 256, true, e)
+MTRT_SOFTMAX_GROUP_KERNEL(f32, F32, 8, 1024, u, true, 1024, false, a)
+MTRT_SOFTMAX_GROUP_KERNEL(f32, F32, 16, 1024, u, true, 1024, false, a)

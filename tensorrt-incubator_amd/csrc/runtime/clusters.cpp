@@ -438,6 +438,56 @@ bool pick_group(int64_t nvec_per_row, int *threads, int *nv) {
   return false;
 }
 
+// Two forms of a kernel (norm.hip): one works on every vector, the other stops at a row's end, which asks for less and needs fewer registers, but
+// takes its vectors one after the other.  That one is the faster up to a share of the vectors that a row fills, which depends on the
+// rows to a compute unit: few have nothing to hide the way to memory behind; `window` is where they fit on the chip at once in
+// this form and not in the other.  Lines from 2850 shapes (5 to 6000 rows and 100 MB, shares 0.53 to 1, f32 and bf16), each where the forms
+// are level; us, every vector and to the row's end:
+//   LayerNorm bf16 [1500, 9011] 18.7, 14.7; [4000, 10243] 46.9, 40.8; [3633, 13760] 38.7, 42.8; [500, 27523] 14.7, 15.5; [1500, 31128] 37.8, 44.2;
+//   [500, 47184] 24.3, 17.6; [1500, 36043] 78.5, 56.7; f32 [500, 4504] 5.6, 5.9; [1500, 5120] 13.0, 10.5; [1000, 27524] 48.9, 49.4
+//   softmax bf16 [1500, 10240] 13.7, 9.8; [768, 11792] 7.6, 8.1; [4000, 13763] 48.5, 45.9; [2000, 27520] 39.3, 41.7; [1000, 40963] 51.2, 43.0; f32 [2000,
+//   18023] 63.6, 52.4
+// Kernels that are not listed have one form; fewer than 8 rows, a few us whichever it is, take the one without a letter.
+struct RowForm {
+  bool layernorm, wide, ragged;                        // wide: f32
+  int lanes, nv;
+  double lo, hi;                                       // the window, rows to a compute unit
+  double few, window, many;                            // largest share to stop at the row's end: up to lo, up to hi, beyond
+  double whole = 0;                                    // whole rows too (its body for those has fewer registers): from here on
+};
+constexpr RowForm kRowForms[] = {
+    {true, false, false, 256, 8, 5, 8, 0, 0.75, 0, 5},
+    {true, false, false, 256, 16, 3, 5, 0, 1, 0.63},
+    {true, false, false, 1024, 8, 0, 0, 0, 0, 0.95},
+    {true, false, false, 1024, 16, 0, 0, 0, 0, 0.92},
+    {true, false, true, 64, 4, 0, 0, 0, 0, 0.77},
+    {true, false, true, 64, 8, 0, 0, 0, 0, 0.85},
+    {true, false, true, 64, 16, 0, 0, 0, 0, 0.75},
+    {true, false, true, 256, 8, 2.5, 2.5, 0.72, 0, 0.9},
+    {true, false, true, 256, 16, 2.5, 4, 0.66, 0.95, 0.66},
+    {true, true, false, 256, 8, 4, 4, 0, 0, 0.96},
+    {true, true, false, 1024, 8, 0, 0, 0, 0, 0.7},
+    {false, false, false, 256, 8, 3.5, 6, 0, 0.96, 0},
+    {false, false, false, 256, 16, 2, 4, 0, 0.85, 0},
+    {false, false, false, 1024, 8, 0, 0, 0, 0, 0.85},
+    {false, false, false, 1024, 16, 0, 0, 0, 0, 0.9},
+    {false, false, true, 256, 8, 2.5, 4, 0.66, 1, 0.85},
+    {false, false, true, 256, 16, 1.1, 4, 0.66, 1, 0.85},
+    {false, true, false, 1024, 8, 1, 1, 0.7, 0, 0.95},
+    {false, true, false, 1024, 16, 0, 0, 0, 0, 0.75},
+    {false, true, true, 1024, 8, 1, 1, 0.8, 0, 1},
+    {false, true, true, 1024, 16, 0, 0, 0, 0, 0.8},
+};
+const char *row_form(bool layernorm, int32_t dtype, bool ragged, int lanes, int nv, int64_t rows, int64_t nvec_per_row, int64_t units) {
+  for (const RowForm &r : kRowForms)
+    if (rows >= 8 && r.layernorm == layernorm && r.wide == (dtype == MTRT_F32) && r.ragged == ragged && r.lanes == lanes && r.nv == nv) {
+      const double to_a_unit = double(rows) / double(units), share = double(nvec_per_row) / double(lanes * nv);
+      const bool ends = share <= (to_a_unit <= r.lo ? r.few : to_a_unit <= r.hi ? r.window : r.many) || (share == 1 && r.whole > 0 && to_a_unit > r.whole);
+      return lanes == 1024 ? (ends ? "" : "a") : (ends ? "e" : "");
+    }
+  return "";
+}
+
 } // namespace
 
 extern "C" {
@@ -957,7 +1007,7 @@ int32_t mtrt_hip_layernorm(mtrt_stream_t stream, const void *x, const void *gamm
   }
   int threads, gnv;
   if (vec_ok && !nv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-    return launch(st, KernelName("mtrt_layernorm_") + xn + "_g" + threads + "v" + gnv, uint32_t(rows), uint32_t(threads),
+    return launch(st, KernelName("mtrt_layernorm_") + xn + "_g" + threads + "v" + gnv + row_form(true, dtype, false, threads, gnv, rows, d / per_vec, num_compute_units(st)), uint32_t(rows), uint32_t(threads),
                   as_hip(stream), args);
   // Row lengths that are not whole vectors, or operands that are not 16-byte aligned: the same two schemes with
   // 128-bit accesses at element alignment and the last d % per_vec elements of a row moved one by one.
@@ -965,11 +1015,13 @@ int32_t mtrt_hip_layernorm(mtrt_stream_t stream, const void *x, const void *gamm
     int rnv = pick_nv(d / per_vec);
     if (rnv && rows <= kMaxRowsPerWaveKernels) {
       rnv = unaligned_nv(dtype, rnv, true);
-      return launch(st, KernelName("mtrt_layernorm_") + xn + "_u64v" + rnv, blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
+      return launch(st, KernelName("mtrt_layernorm_") + xn + "_u64v" + rnv + row_form(true, dtype, true, 64, rnv, rows, d / per_vec, num_compute_units(st)), blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
     }
-    if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-      return launch(st, KernelName("mtrt_layernorm_") + xn + "_u" + threads + "v" + unaligned_nv(dtype, gnv, true), uint32_t(rows), uint32_t(threads),
+    if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv)) {
+      gnv = unaligned_nv(dtype, gnv, true);
+      return launch(st, KernelName("mtrt_layernorm_") + xn + "_u" + threads + "v" + gnv + row_form(true, dtype, true, threads, gnv, rows, d / per_vec, num_compute_units(st)), uint32_t(rows), uint32_t(threads),
                     as_hip(stream), args);
+    }
   }
   return launch(st, KernelName("mtrt_layernorm_") + xn + "_any",
                 uint32_t(std::min<int64_t>(rows, int64_t(num_compute_units(st)) * 8)), kBlock, as_hip(stream), args);
@@ -1010,7 +1062,7 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
                   blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
   int threads, gnv;
   if (vec_ok && !nv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-    return launch(st, KernelName("mtrt_softmax_") + xn + "_g" + threads + "v" + gnv, uint32_t(rows), uint32_t(threads),
+    return launch(st, KernelName("mtrt_softmax_") + xn + "_g" + threads + "v" + gnv + row_form(false, dtype, false, threads, gnv, rows, d / per_vec, num_compute_units(st)), uint32_t(rows), uint32_t(threads),
                   as_hip(stream), args);
   // Row lengths that are not whole vectors, or operands that are not 16-byte aligned: the same two schemes with
   // 128-bit accesses at element alignment and the last d % per_vec elements of a row moved one by one.
@@ -1020,9 +1072,11 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
       rnv = unaligned_nv(dtype, rnv, false);
       return launch(st, KernelName("mtrt_softmax_") + xn + "_u64v" + rnv, blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
     }
-    if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + unaligned_nv(dtype, gnv, false), uint32_t(rows), uint32_t(threads),
+    if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv)) {
+      gnv = unaligned_nv(dtype, gnv, false);
+      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + gnv + row_form(false, dtype, true, threads, gnv, rows, d / per_vec, num_compute_units(st)), uint32_t(rows), uint32_t(threads),
                     as_hip(stream), args);
+    }
   }
   return launch(st, KernelName("mtrt_softmax_") + xn + "_any",
                 uint32_t(std::min<int64_t>(rows, int64_t(num_compute_units(st)) * 8)), kBlock, as_hip(stream), args);
@@ -1567,7 +1621,9 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
     // elements (bf16, float8 inputs, us, two launches and one: (8, 4096, 4096) 11.3, 10.1, (2, 14336, 512) 18.5, 12.7; (16, 1536, 8192) 9.4, 11.5);
     // where they are more than two, half as many to quantize ((16, 1024, 16384) 10.1, 11.4; (8, 1024, 16384) 9.7, 8.5; (16, 1024, 8192) 7.2,
     // 6.8); and a plain x that needs no pass only saves the 32-column kernel's way to its rows, from 1024 elements a row (us, that and
-    // this, bf16: (16, 512, 8192) 3.6, 4.2; (8, 768, 8192) 3.9, 4.1; (8, 1024, 8192) 4.2, 4.2; (4, 1024, 12000) 6.7, 5.2; (8, 2048, 8192) 5.1, 4.5).
+    // this, bf16: (16, 512, 8192) 3.6, 4.2; (8, 768, 8192) 3.9, 4.1; (8, 1024, 8192) 4.2, 4.2; (4, 1024, 12000) 6.7, 5.2; (8, 2048, 8192) 5.1, 4.5.
+    // Weights read from memory; where they lie in the Infinity Cache already two launches are the faster between two and three workgroups to
+    // a unit, (1, 1024, 11008) 6.2, 6.9 against 8.8, 7.9.)
     const bool passes = quantized || s.Kp != p.K;
     const int64_t tiles16 = (p.N + 15) / 16, most = tiles16 <= units ? 2 * kDecodeElements : passes && tiles16 > 2 * units ? kDecodeElements / 2 : kDecodeElements;
     s.one_launch = s.fragments && M <= 16 && M * s.Kp <= most && launchable(tiles16, 512) && (passes || tiles16 <= units || s.Kp >= 1024);
