@@ -517,7 +517,7 @@ __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __rest
 //       2 = fused quantize->dequantize (read x, write q and y)
 // Host guarantees: n < 2^35; for row/col scales d1 % G == 0 (a group never
 // straddles rows); operands aligned for their group accesses.
-template <typename X, typename Q, int KIND, int MODE>
+template <typename X, typename Q, int KIND, int MODE, bool SCALAR = MODE != 2>
 __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                            typename X::storage* __restrict__ y, const float* __restrict__ scale,
                                            int64_t n, int64_t d1, int64_t nb, int flags) {
@@ -529,12 +529,12 @@ __device__ __forceinline__ void qdq_groups(const typename X::storage* __restrict
   const int64_t ngroups = n / G;
   const uint32_t groups_per_row = KIND == kUniform ? 1u : uint32_t(d1 / G);
   const int lane = threadIdx.x & (kWave - 1);
-  // The fused pass keeps the wave's number per lane: with scalar numbers it was the slower (f16 -> f8 of 14 Mi elements with the amax
-  // in front 23.2 -> 24.3 us, bf16 of 128 Mi 155 -> 158), where a quantize and a dequantize of 4 and 128 Mi gained (7.4 -> 7.3, 133 -> 131).
+  // SCALAR: the wave's number in a scalar register.  A quantize and a dequantize of 4 and 128 Mi gained (7.4 -> 7.3, 133 -> 131 us); the fused
+  // pass keeps it per lane, but for the sizes that fused_scalar in clusters.cpp names.
   // one scale for all may come from an amax pass, and a dequantize follows the quantize: see read_twice.hpp
   const uint32_t piece = KIND == kUniform ? piece_of<8 / sizeof(typename X::storage)>(blockIdx.x, gridDim.x, n * int64_t(sizeof(typename X::storage))) : blockIdx.x;
-  const int64_t wave = MODE == 2 ? (int64_t(piece) * blockDim.x + threadIdx.x) / kWave : int64_t(wave_of_block(piece));
-  const int64_t nwaves = MODE == 2 ? int64_t(gridDim.x) * blockDim.x / kWave : int64_t(waves_in_launch());
+  const int64_t wave = SCALAR ? int64_t(wave_of_block(piece)) : (int64_t(piece) * blockDim.x + threadIdx.x) / kWave;
+  const int64_t nwaves = SCALAR ? int64_t(waves_in_launch()) : int64_t(gridDim.x) * blockDim.x / kWave;
   const float s_uniform = KIND == kUniform ? scale[0] : 0.0f;
   const uint32_t wrap = KIND == kRow ? uint32_t(nb) : 0u;
   const bool keep = MODE == 2 ? keep_fused(n) : KIND != kUniform || (keep_plain(n) && !(flags & kFlagCodesPast));
@@ -840,6 +840,20 @@ using namespace qdq_cluster;
 MTRT_QDQ_FOR_FLOAT(f32, F32)
 MTRT_QDQ_FOR_FLOAT(f16, F16)
 MTRT_QDQ_FOR_FLOAT(bf16, BF16)
+
+// The fused pass with one scale and the wave's number in a scalar register (fused_scalar in clusters.cpp): mtrt_qdq_uniform_<t>_<code type>s.
+#define MTRT_QDQ_SCALAR_KERNEL(XN, XT, QN, QT)                                                                    \
+  extern "C" __global__ void __launch_bounds__(256) mtrt_qdq_uniform_##XN##_##QN##s(                              \
+      const XT::storage* x, QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb, \
+      int32_t flags) { qdq_groups<XT, QT, kUniform, 2, true>(x, q, y, scale, n, d1, nb, flags); }
+MTRT_QDQ_SCALAR_KERNEL(f32, F32, i8, I8)
+MTRT_QDQ_SCALAR_KERNEL(f32, F32, i4, I4)
+MTRT_QDQ_SCALAR_KERNEL(f16, F16, i8, I8)
+MTRT_QDQ_SCALAR_KERNEL(f16, F16, f8, F8)
+MTRT_QDQ_SCALAR_KERNEL(f16, F16, i4, I4)
+MTRT_QDQ_SCALAR_KERNEL(bf16, BF16, i8, I8)
+MTRT_QDQ_SCALAR_KERNEL(bf16, BF16, f8, F8)
+MTRT_QDQ_SCALAR_KERNEL(bf16, BF16, i4, I4)
 
 // Ragged rows / unaligned operands with row or column scales: mtrt_{q,dq,qdq}_{rowu,colu}_<float type>_<code type>,
 // arguments as the kernels above plus, behind nb, the row pitches in elements of the float operand(s) and of the codes

@@ -6,8 +6,8 @@
 // from the tensor's end to its front, in 32 KiB that a workgroup takes at a time; the passes that quantize by its maximum go
 // forwards, as many neighbouring pieces of theirs on one XCD as make up 32 KiB, and so does the dequantize behind them, which finds their
 // codes in the same way.  us, bf16 -> i8 of 8, 16, 24 and 48 Mi elements, with amax forwards, the quantizing pass from the end and the
-// dequantize forwards piece by piece, and so: amax, then quantize and dequantize in one pass 12.5, 20.0, 30.2, 53.6 and 12.6, 20.0, 30.5, 53.8;
-// a quantize and its dequantize 13.7, 23.8, 27.9, 51.7 and 10.7, 17.3, 24.7, 51.3 (the codes of the one lay in other L2s than the
+// dequantize forwards piece by piece, and so: amax, then quantize and dequantize in one pass 12.6, 20.3, 30.5, 53.8 and 13.0, 20.6, 31.0, 54.0;
+// a quantize and its dequantize 13.8, 23.7, 27.9, 51.7 and 10.7, 17.3, 24.7, 51.3 (the codes of the one lay in other L2s than the
 // other read them through).  Pieces of 8 or 16 KiB to an XCD in all passes: amax of 33 MB from memory 9.0 -> 9.7.
 #pragma once
 #include <stdint.h>

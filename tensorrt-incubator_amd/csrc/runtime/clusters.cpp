@@ -305,6 +305,16 @@ bool bind_split(DeviceState *st, hipStream_t stream, Plan &plan, void *workspace
 
 constexpr int32_t kCodesPast = 1 << 8;  // kFlagCodesPast of the kernels (common.hpp)
 
+// Quantize and dequantize in one pass, one scale: the kernel with the wave's number in a scalar register, for tensors of more than four
+// workgroups to a unit (three, to float8) and up to 9 Mi elements.  us, the number per lane and scalar: bf16 -> i8 of 4, 4.02, 5, 6, 8, 12
+// and 32 Mi 5.2, 5.3; 6.25, 5.5; 7.0, 6.2; 7.6, 7.2; 9.5, 9.3; 12.6, 13.4; 27.6, 29.7; bf16 -> f8 of 3, 3.02, 4, 5 and 8 Mi 4.6, 4.8; 5.4, 4.8;
+// 6.1, 5.4; 7.5, 6.5; 9.6, 9.4; f32 -> i8 of 4, 4.02, 5, 8, 20 and 48 Mi 7.4, 7.6; 8.95, 7.95; 9.95, 9.0; 15.2, 14.4; 32.9, 33.9; 69.7, 72.2;
+// behind an amax the two are level.  f32 -> f8 loses (8 Mi 14.8, 15.9).
+bool fused_scalar(int32_t x_dtype, int32_t q_dtype, int64_t n) {
+  const bool codes = q_dtype == MTRT_I8 || q_dtype == MTRT_I4 || (q_dtype == MTRT_F8E4M3FN && x_dtype != MTRT_F32);
+  return codes && n > (int64_t(q_dtype == MTRT_F8E4M3FN ? 3 : 4) << 20) && n < (int64_t(9) << 20);
+}
+
 // mode: 0 quantize, 1 dequantize, 2 fused.  codes_past: nobody is known to read the codes next (see CodeGroup in qdq.hip)
 int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtype, void *q,
                      int32_t q_dtype, void *y, const float *scale, int32_t kind, int64_t d0,
@@ -378,6 +388,9 @@ int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtyp
   static const char *kRaggedName[] = {"", "rowu", "colu"};
   KernelName name("mtrt_");
   name + kModeName[mode] + "_" + (tiles ? kKindName[kind] : (ragged ? kRaggedName[kind] : "any")) + "_" + xn + "_" + qn;
+
+  if (mode == 2 && tiles && kind == MTRT_SCALE_UNIFORM && fused_scalar(x_dtype, q_dtype, n))
+    name + "s";
 
   int64_t n_arg = n, d1_arg = d1, nb_arg = nb;
   int32_t kind_arg = kind, flags_arg = flags | (codes_past ? kCodesPast : 0);

@@ -1,6 +1,6 @@
-"""Passes over a tensor that another pass has just read: the amax pass takes it in pieces of 32 KiB, and the quantize passes behind
-it go through it from its end.  Sizes around a piece, around the number of workgroups, around the groups of pieces that are
-turned round together, and on both sides of the size beyond which nothing is turned round."""
+"""Passes over a tensor that another pass has just read: the amax pass takes it in pieces of 32 KiB from its end, the passes behind
+it forwards in the same pieces.  Sizes around a piece, around the number of workgroups, around the groups of pieces that are dealt to
+the XCDs together, on both sides of the size beyond which they are dealt singly, and where the kernel of the fused pass changes."""
 import numpy as np
 import pytest
 
@@ -77,3 +77,19 @@ def test_nvfp4_from_the_end_is_the_same_as_in_parts(pkg, shape, dname):
         assert torch.equal(s.reshape(-1), torch.cat([p[1].reshape(-1) for p in parts])), axis
         ys = [pkg.nvfp4_dequantize(p[0], p[1], amax, x.dtype, (16, shape[1]), axis=axis).reshape(-1) for p in parts]
         assert torch.equal(y.reshape(-1), torch.cat(ys)), axis
+
+
+@pytest.mark.parametrize("dname,code", [("float32", "I8"), ("float32", "I4"), ("float32", "F8E4M3FN"), ("float16", "I8"), ("float16", "F8E4M3FN"), ("float16", "I4"),
+                                        ("bfloat16", "I8"), ("bfloat16", "F8E4M3FN"), ("bfloat16", "I4")])
+def test_both_kernels_of_the_fused_pass_are_a_quantize_and_a_dequantize(pkg, dname, code):
+    """From 4 to 9 Mi elements (3, to float8) the fused pass has a kernel of its own but for f32 to float8; whole groups or not."""
+    import torch
+    q_dtype, m = getattr(pkg, code), 1 << 20
+    scale = torch.tensor([0.037], device="cuda")
+    for n, other in ((3 * m, False), (3 * m + 1, code == "F8E4M3FN"), (4 * m, code == "F8E4M3FN"), (4 * m + 1, True), (4 * m + 4096, True), (5 * m - 3, True), (9 * m - 1, True), (9 * m, False)):
+        x = _x(torch, n, dname)
+        q, y = pkg.quantize_dequantize(x, scale, q_dtype)
+        assert pkg.last_kernel().endswith("s") == (other and (dname, code) != ("float32", "F8E4M3FN")), (n, pkg.last_kernel())
+        only = pkg.quantize(x, scale, q_dtype)
+        assert torch.equal(only, q), n
+        assert torch.equal(pkg.dequantize(only, scale, q_dtype, x.dtype, x.shape).view(torch.uint8), y.view(torch.uint8)), n
