@@ -454,10 +454,11 @@ bool pick_group(int64_t nvec_per_row, int *threads, int *nv) {
 // Two forms of a kernel (norm.hip): one works on every vector, the other stops at a row's end, which asks for less and needs fewer registers, but
 // takes its vectors one after the other.  That one is the faster up to a share of the vectors that a row fills, which depends on the
 // rows to a compute unit: few have nothing to hide the way to memory behind; `window` is where they fit on the chip at once in
-// this form and not in the other.  Lines from 2850 shapes (5 to 6000 rows and 100 MB, shares 0.53 to 1, f32 and bf16), each where the forms
+// this form and not in the other.  Lines from 3050 shapes (5 to 6000 rows and 100 MB, shares 0.53 to 1, f32 and bf16), each where the forms
 // are level; us, every vector and to the row's end:
 //   LayerNorm bf16 [1500, 9011] 18.7, 14.7; [4000, 10243] 46.9, 40.8; [3633, 13760] 38.7, 42.8; [500, 27523] 14.7, 15.5; [1500, 31128] 37.8, 44.2;
 //   [500, 47184] 24.3, 17.6; [1500, 36043] 78.5, 56.7; f32 [500, 4504] 5.6, 5.9; [1500, 5120] 13.0, 10.5; [1000, 27524] 48.9, 49.4
+//   from 7 rows to a unit at element alignment [1800, 23595] 48.9, 45.8; [4000, 26179] 104.7, 103.1; [2800, 28179] 79.7, 81.6
 //   softmax bf16 [1500, 10240] 13.7, 9.8; [768, 11792] 7.6, 8.1; [4000, 13763] 48.5, 45.9; [2000, 27520] 39.3, 41.7; [1000, 40963] 51.2, 43.0; f32 [2000,
 //   18023] 63.6, 52.4
 // Kernels that are not listed have one form; fewer than 8 rows, a few us whichever it is, take the one without a letter.
@@ -467,6 +468,7 @@ struct RowForm {
   double lo, hi;                                       // the window, rows to a compute unit
   double few, window, many;                            // largest share to stop at the row's end: up to lo, up to hi, beyond
   double whole = 0;                                    // whole rows too (its body for those has fewer registers): from here on
+  double upto = 1e30;                                  // the entry holds up to here; the kernel's next one beyond
 };
 constexpr RowForm kRowForms[] = {
     {true, false, false, 256, 8, 5, 8, 0, 0.75, 0, 5},
@@ -477,7 +479,8 @@ constexpr RowForm kRowForms[] = {
     {true, false, true, 64, 8, 0, 0, 0, 0, 0.85},
     {true, false, true, 64, 16, 0, 0, 0, 0, 0.75},
     {true, false, true, 256, 8, 2.5, 2.5, 0.72, 0, 0.9},
-    {true, false, true, 256, 16, 2.5, 4, 0.66, 0.95, 0.66},
+    {true, false, true, 256, 16, 2.5, 4, 0.66, 0.95, 0.66, 0, 7},
+    {true, false, true, 256, 16, 0, 0, 0, 0, 0.82},
     {true, true, false, 256, 8, 4, 4, 0, 0, 0.96},
     {true, true, false, 1024, 8, 0, 0, 0, 0, 0.7},
     {false, false, false, 256, 8, 3.5, 6, 0, 0.96, 0},
@@ -492,9 +495,9 @@ constexpr RowForm kRowForms[] = {
     {false, true, true, 1024, 16, 0, 0, 0, 0, 0.8},
 };
 const char *row_form(bool layernorm, int32_t dtype, bool ragged, int lanes, int nv, int64_t rows, int64_t nvec_per_row, int64_t units) {
+  const double to_a_unit = double(rows) / double(units), share = double(nvec_per_row) / double(lanes * nv);
   for (const RowForm &r : kRowForms)
-    if (rows >= 8 && r.layernorm == layernorm && r.wide == (dtype == MTRT_F32) && r.ragged == ragged && r.lanes == lanes && r.nv == nv) {
-      const double to_a_unit = double(rows) / double(units), share = double(nvec_per_row) / double(lanes * nv);
+    if (rows >= 8 && r.layernorm == layernorm && r.wide == (dtype == MTRT_F32) && r.ragged == ragged && r.lanes == lanes && r.nv == nv && to_a_unit <= r.upto) {
       const bool ends = share <= (to_a_unit <= r.lo ? r.few : to_a_unit <= r.hi ? r.window : r.many) || (share == 1 && r.whole > 0 && to_a_unit > r.whole);
       return lanes == 1024 ? (ends ? "" : "a") : (ends ? "e" : "");
     }
