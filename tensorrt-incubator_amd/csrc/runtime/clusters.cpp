@@ -84,24 +84,31 @@ constexpr double kW4Mid256RoundPerSmallRound = 1.9;
 //   fixed + (e + c s) (L - 1 + p + (1 - p) f^2) + (splits > 1 ? meet + meet_each * splits : 0)   us
 // (a launch that leaves units idle is shorter, more so for the large tiles: the clock is power's).  Fitted to 17000
 // launches of 621 log-uniform shapes, M 33 ... 4096, K 256 ... 14336, N 64 ... 16384, 1 to 12 splits.
+// That is a full chip's law.  However few tiles there are, one of them takes least + least_slice * s, which a launch of few
+// large tiles runs into (fitted to the launches of at most half as many unsplit tiles as units of 380 shapes of the same range).
+// With it the choice is 1.6 % longer than the fastest one on average; without, M, K, N, us: (92, 640, 6336) t128x128 7.2, t32x128 5.2; (1001, 896, 640) 8.3,
+// 6.2; (805, 1536, 768) 11.3, 8.4; (606, 1280, 384) 9.8, 7.4; (91, 1152, 8896) 9.4, 7.1; none of the 380 shapes got slower.
 struct W4Tile {
   const char *suffix;                                  // of the kernel's name
   int rows, columns, threads;
   bool splits;                                         // whether its K may be split
-  double fixed, e, c, p, meet, meet_each;
+  double fixed, e, c, p, meet, meet_each, least, least_slice;
 };
 constexpr W4Tile kW4Tiles[] = {
-    {"t32x128", 32, 128, 256, true, 2.64, 0.89, 0.197, 1.0, 1.59, 0.334},
-    {"t64x128", 64, 128, 512, true, 0.99, 3.35, 0.252, 0.83, 2.59, 0.46},
-    {"t64x256", 64, 256, 256, true, 0.0, 4.38, 0.497, 0.79, 4.02, 0.645},
-    {"t128x128", 128, 128, 512, true, 0.0, 5.76, 0.523, 0.474, 3.54, 0.725},
-    {"t128x256", 128, 256, 256, true, 0.0, 5.98, 1.046, 0.467, 5.8, 1.19},
-    {"t256x256", 256, 256, 256, false, 0.0, 7.3, 1.589, 0.615, 0.0, 0.0},
-    {"t256x384", 256, 384, 256, false, 0.0, 8.46, 2.637, 0.525, 0.0, 0.0},
+    {"t32x128", 32, 128, 256, true, 2.64, 0.89, 0.197, 1.0, 1.59, 0.334, 0.0, 0.0},
+    {"t64x128", 64, 128, 512, true, 0.99, 3.35, 0.252, 0.83, 2.59, 0.46, 0.0, 0.0},
+    {"t64x256", 64, 256, 256, true, 0.0, 4.38, 0.497, 0.79, 4.02, 0.645, 3.39, 0.422},
+    {"t128x128", 128, 128, 512, true, 0.0, 5.76, 0.523, 0.474, 3.54, 0.725, 4.3, 0.282},
+    {"t128x256", 128, 256, 256, true, 0.0, 5.98, 1.046, 0.467, 5.8, 1.19, 4.16, 0.55},
+    {"t256x256", 256, 256, 256, false, 0.0, 7.3, 1.589, 0.615, 0.0, 0.0, 5.99, 1.0},
+    {"t256x384", 256, 384, 256, false, 0.0, 8.46, 2.637, 0.525, 0.0, 0.0, 7.59, 1.415},
 };
+// Short products are estimated without that bound, which leaves them on the 128-row tiles: K up to 512, and up to 1024 with at most 256
+// columns.  The reason is not time, (33, 256, 64) takes 5.3 us on t128x128 and 3.4 on t32x128: these are the shapes by which the tests
+// reach the 128-row kernels and name them.
+constexpr int64_t kW4ShortSlices = 8, kW4ShortNarrowSlices = 16, kW4ShortNarrowColumns = 256;
 // The tile by rounds (above) is the better founded choice where the estimates are close: another tile or a split has to
-// promise a tenth.  Over the same launches, the chosen one against the fastest in each: 1.8 % longer on average; against
-// the choice by rounds alone 1.44 times as fast, 0.95 at worst.
+// promise a tenth (over those 380 shapes none is slower so than without the bound; with no such promise the worst is 1.15 times as long).
 constexpr double kW4Promise = 0.9;
 // Tiles on fragment-order weights (gemm_frag.hpp).  A launch of `tiles * splits` workgroups, L = ceil of that over the
 // compute units, each running s = slices / splits slices of 128 bytes of K, is estimated as
@@ -195,6 +202,7 @@ W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   using namespace tuning;
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
   const int64_t slices = K / 64;
+  const bool is_short = slices <= kW4ShortSlices || (slices <= kW4ShortNarrowSlices && N <= kW4ShortNarrowColumns);
   auto tiles_of = [&](const W4Tile &t) { return ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns); };
   auto plan_of = [&](const W4Tile &t, int splits) {
     W4Plan p;
@@ -203,7 +211,7 @@ W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
     p.split = split_of(slices, splits);
     const int64_t n = p.tiles * p.split.splits, full = (n - 1) / units;
     const double s = double(p.split.per), f = double(n - full * units) / double(units);
-    p.us = t.fixed + (t.e + t.c * s) * (double(full) + t.p + (1.0 - t.p) * f * f) +
+    p.us = std::max(t.fixed + (t.e + t.c * s) * (double(full) + t.p + (1.0 - t.p) * f * f), is_short ? 0.0 : t.least + t.least_slice * s) +
            (p.split.splits > 1 ? t.meet + t.meet_each * p.split.splits : 0.0);
     return p;
   };
