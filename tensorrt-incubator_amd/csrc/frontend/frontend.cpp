@@ -3,7 +3,7 @@
 //
 // Why: a call on a small tensor is bound by the host.  One launch costs 2.3 us back to back on this chip, and the same
 // call through ctypes and torch's Python API cost 8 us (package functions) to 12 us (`tp`), of which
-// torch.cuda.current_stream() alone was 2.9 us and each torch.empty() 1.7 us.
+// torch.cuda.current_stream() alone was 2.9 us and each torch.empty() 1.7 us.  From here amax is 4.4 us, the dynamic quantization 5.4.
 //
 // Two sets of functions:
 //   * the package's functions (softmax, quantize, ...): argument for argument what the Python wrappers of the same names
@@ -16,8 +16,11 @@
 // The interpreter lock is released around the calls into the library.
 #include <Python.h>
 
+#include <ATen/EmptyTensor.h>
 #include <ATen/core/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
+#include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -84,21 +87,45 @@ bool float_type(const at::Tensor &t, int32_t *code) {
 
 bool dense_on_gpu(const at::Tensor &t) { return t.is_cuda() && t.is_contiguous(); }
 
-mtrt_stream_t current_stream() { return reinterpret_cast<mtrt_stream_t>(c10::hip::getCurrentHIPStream().stream()); }
+// Where a call works: the current device's current stream, and torch's memory on the device of `x`.  The device is asked for once;
+// on it a tensor is made straight on torch's allocator (one that the program swapped in among them), elsewhere by torch's own
+// function, which changes the device for as long as it allocates.  Per tensor 0.30 us against 0.47, the stream 0.02 against 0.08.
+class Place {
+public:
+  explicit Place(const at::Tensor &x) : device(x.device()), here(x.device().index() == c10::hip::current_device()) {
+    stream = reinterpret_cast<mtrt_stream_t>((here ? c10::hip::getCurrentHIPStream(device.index()) : c10::hip::getCurrentHIPStream()).stream());
+  }
+  at::Tensor empty(at::IntArrayRef shape, at::ScalarType type) const {
+    if (here)
+      return at::Tensor(at::detail::empty_generic(shape, c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get(), c10::DispatchKeySet(c10::DispatchKey::CUDA), type, std::nullopt));
+    return at::Tensor(at::detail::empty_cuda(shape, type, device, std::nullopt));
+  }
+  // Scratch memory of a call: back with torch's allocator when the call returns, which hands it only to work that follows on
+  // the same stream.
+  at::Tensor bytes(int64_t n) const { return empty({n}, at::ScalarType::Byte); }
+  // storage for n codes: int8 for MTRT_I8, else bytes; two to a byte for the packed types
+  at::Tensor codes(int32_t q_dtype, int64_t n) const {
+    const bool packed = q_dtype == MTRT_I4_PACKED || q_dtype == MTRT_F4_PACKED;
+    return empty({packed ? (n + 1) / 2 : n}, q_dtype == MTRT_I8 ? at::ScalarType::Char : at::ScalarType::Byte);
+  }
+  mtrt_stream_t stream;
 
-at::Tensor empty_like_device(at::IntArrayRef shape, at::ScalarType type, const at::Tensor &where) {
-  return at::Tensor(at::detail::empty_cuda(shape, type, where.device(), std::nullopt));
-}
+private:
+  c10::Device device;
+  bool here;
+};
 
-// Scratch memory of a call: back with torch's allocator when the call returns, which hands it only to work that follows on
-// the same stream.
-at::Tensor bytes_on(const at::Tensor &where, int64_t n) { return empty_like_device({n}, at::ScalarType::Byte, where); }
-
-// storage for n codes: int8 for MTRT_I8, else bytes; two to a byte for the packed types
-at::Tensor code_storage(int32_t q_dtype, int64_t n, const at::Tensor &where) {
-  const bool packed = q_dtype == MTRT_I4_PACKED || q_dtype == MTRT_F4_PACKED;
-  return empty_like_device({packed ? (n + 1) / 2 : n}, q_dtype == MTRT_I8 ? at::ScalarType::Char : at::ScalarType::Byte, where);
-}
+// The two f32 numbers of a tensor's amax and scale, side by side in one storage (a second allocation is 0.28 us).
+struct AmaxAndScale {
+  at::Tensor amax, scale;
+  explicit AmaxAndScale(const Place &place) {
+    amax = place.empty({2}, at::ScalarType::Float);
+    scale = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(amax.storage()), c10::DispatchKeySet(c10::DispatchKey::CUDA), amax.dtype());
+    scale.unsafeGetTensorImpl()->set_storage_offset(1);
+    scale.unsafeGetTensorImpl()->set_sizes_contiguous({});
+    amax.unsafeGetTensorImpl()->set_sizes_contiguous({});
+  }
+};
 
 bool check(int32_t status) {
   if (status == MTRT_OK)
@@ -218,8 +245,10 @@ PyObject *f_amax(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return fail("x must be a contiguous tensor on the GPU"), nullptr;
   if (!float_type(*x, &dt) || !number(a[1], &qmax))
     return nullptr;
-  const at::Tensor amax = empty_like_device({}, at::ScalarType::Float, *x), scale = empty_like_device({}, at::ScalarType::Float, *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const AmaxAndScale made(place);
+  const at::Tensor &amax = made.amax, &scale = made.scale;
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_amax(s, x->data_ptr(), dt, x->numel(), qmax, static_cast<float *>(amax.data_ptr()), static_cast<float *>(scale.data_ptr()));
       }))
@@ -242,9 +271,10 @@ PyObject *f_amax_scales(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!float_type(*x, &dt) || !number(a[1], &qmax) || !integer32(a[2], &kind) || !view2d(*x, a[3], a[4], &d0, &d1) || !integer(a[5], &nb))
     return nullptr;
   const int64_t count = kind == MTRT_SCALE_UNIFORM ? 1 : kind == MTRT_SCALE_ROW ? nb : (nb ? d0 / nb * d1 : 0);
-  const at::Tensor amax = empty_like_device({count < 0 ? 0 : count}, at::ScalarType::Float, *x);
-  const at::Tensor scale = empty_like_device({count < 0 ? 0 : count}, at::ScalarType::Float, *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor amax = place.empty({count < 0 ? 0 : count}, at::ScalarType::Float);
+  const at::Tensor scale = place.empty({count < 0 ? 0 : count}, at::ScalarType::Float);
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_amax_scales(s, x->data_ptr(), dt, kind, d0, d1, nb, qmax, static_cast<float *>(amax.data_ptr()),
                                     static_cast<float *>(scale.data_ptr()));
@@ -267,8 +297,9 @@ PyObject *f_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!integer32(a[2], &q_dtype) || !integer32(a[3], &kind) || !view2d(*x, a[4], a[5], &d0, &d1) || !integer(a[6], &nb) ||
       !integer32(a[7], &flags) || !float_type(*x, &dt))
     return nullptr;
-  const at::Tensor q = out ? *out : code_storage(q_dtype, d0 * d1, *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor q = out ? *out : place.codes(q_dtype, d0 * d1);
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_quantize(s, x->data_ptr(), dt, q.data_ptr(), q_dtype, static_cast<const float *>(scale->data_ptr()), kind, d0, d1,
                                  nb, flags);
@@ -301,7 +332,7 @@ bool shape_of(PyObject *o, c10::SmallVector<int64_t, 6> *shape) {
   return true;
 }
 
-bool made_or_given(const at::Tensor *out, PyObject *type, PyObject *shape_arg, const at::Tensor &where, at::Tensor *y) {
+bool made_or_given(const at::Tensor *out, PyObject *type, PyObject *shape_arg, const Place &place, at::Tensor *y) {
   if (out) {
     *y = *out;
     return true;
@@ -313,7 +344,7 @@ bool made_or_given(const at::Tensor *out, PyObject *type, PyObject *shape_arg, c
   c10::SmallVector<int64_t, 6> shape;
   if (!shape_of(shape_arg, &shape))
     return false;
-  *y = empty_like_device(shape, reinterpret_cast<THPDtype *>(type)->scalar_type, where);
+  *y = place.empty(shape, reinterpret_cast<THPDtype *>(type)->scalar_type);
   return true;
 }
 
@@ -328,10 +359,11 @@ PyObject *f_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return nullptr;
   if (!dense_on_gpu(*q) || scale->scalar_type() != at::ScalarType::Float)
     return fail("q must be contiguous and on the GPU, scale float32"), nullptr;
-  if (!made_or_given(out, a[3], a[4], *q, &y) || !integer32(a[2], &q_dtype) || !integer32(a[5], &kind) ||
+  const Place place(*q);
+  if (!made_or_given(out, a[3], a[4], place, &y) || !integer32(a[2], &q_dtype) || !integer32(a[5], &kind) ||
       !view2d(y, a[6], a[7], &d0, &d1) || !integer(a[8], &nb) || !float_type(y, &dt))
     return nullptr;
-  const mtrt_stream_t s = current_stream();
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_dequantize(s, q->data_ptr(), q_dtype, y.data_ptr(), dt, static_cast<const float *>(scale->data_ptr()), kind, d0, d1, nb);
       }))
@@ -354,9 +386,10 @@ PyObject *f_quantize_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!integer32(a[2], &q_dtype) || !integer32(a[3], &kind) || !view2d(*x, a[4], a[5], &d0, &d1) || !integer(a[6], &nb) ||
       !integer32(a[7], &flags) || !float_type(*x, &dt))
     return nullptr;
-  const at::Tensor q = q_out ? *q_out : code_storage(q_dtype, d0 * d1, *x);
-  const at::Tensor y = y_out ? *y_out : empty_like_device(x->sizes(), x->scalar_type(), *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor q = q_out ? *q_out : place.codes(q_dtype, d0 * d1);
+  const at::Tensor y = y_out ? *y_out : place.empty(x->sizes(), x->scalar_type());
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_quantize_dequantize(s, x->data_ptr(), dt, q.data_ptr(), q_dtype, y.data_ptr(),
                                             static_cast<const float *>(scale->data_ptr()), kind, d0, d1, nb, flags);
@@ -379,12 +412,14 @@ PyObject *f_dynamic_quantize_dequantize(PyObject *, PyObject *const *a, Py_ssize
   const int back = PyObject_IsTrue(a[4]);
   if (back < 0 || !integer32(a[1], &q_dtype) || !number(a[2], &qmax) || !integer32(a[3], &flags) || !float_type(*x, &dt))
     return nullptr;
-  const at::Tensor amax = empty_like_device({}, at::ScalarType::Float, *x), scale = empty_like_device({}, at::ScalarType::Float, *x);
-  const at::Tensor q = code_storage(q_dtype, x->numel(), *x);
+  const Place place(*x);
+  const AmaxAndScale made(place);
+  const at::Tensor &amax = made.amax, &scale = made.scale;
+  const at::Tensor q = place.codes(q_dtype, x->numel());
   at::Tensor y;
   if (back)
-    y = empty_like_device(x->sizes(), x->scalar_type(), *x);
-  const mtrt_stream_t s = current_stream();
+    y = place.empty(x->sizes(), x->scalar_type());
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_dynamic_quantize_dequantize(s, x->data_ptr(), dt, q.data_ptr(), q_dtype, back ? y.data_ptr() : nullptr, x->numel(),
                                                     qmax, static_cast<float *>(amax.data_ptr()), static_cast<float *>(scale.data_ptr()), flags);
@@ -413,12 +448,13 @@ PyObject *f_dynamic_quantize_rows(PyObject *, PyObject *const *a, Py_ssize_t n) 
   if (want < 0 || !integer32(a[1], &q_dtype) || !number(a[2], &qmax) || !integer32(a[3], &flags) || !float_type(*x, &dt))
     return nullptr;
   const int64_t d = x->size(-1), rows = d ? x->numel() / d : 0;
-  const at::Tensor scale = empty_like_device({rows}, at::ScalarType::Float, *x);
+  const Place place(*x);
+  const at::Tensor scale = place.empty({rows}, at::ScalarType::Float);
   at::Tensor amax;
   if (want)
-    amax = empty_like_device({rows}, at::ScalarType::Float, *x);
-  const at::Tensor q = code_storage(q_dtype, x->numel(), *x);
-  const mtrt_stream_t s = current_stream();
+    amax = place.empty({rows}, at::ScalarType::Float);
+  const at::Tensor q = place.codes(q_dtype, x->numel());
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_dynamic_quantize_rows(s, x->data_ptr(), dt, q.data_ptr(), q_dtype, rows, d, qmax,
                                               want ? static_cast<float *>(amax.data_ptr()) : nullptr, static_cast<float *>(scale.data_ptr()), flags);
@@ -464,11 +500,12 @@ PyObject *f_nvfp4_quantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
   const int64_t d1 = x->size(-1), d0 = d1 ? x->numel() / d1 : 0;
   c10::SmallVector<int64_t, 6> shape(x->sizes().begin(), x->sizes().end());
   shape[shape.size() - (last ? 1 : 2)] /= 16;
-  const at::Tensor q = empty_like_device({x->numel() / 2}, at::ScalarType::Byte, *x);
-  const at::Tensor scales = empty_like_device(shape, at::ScalarType::Byte, *x);
+  const Place place(*x);
+  const at::Tensor q = place.empty({x->numel() / 2}, at::ScalarType::Byte);
+  const at::Tensor scales = place.empty(shape, at::ScalarType::Byte);
   if (!float_type(*x, &dt))
     return nullptr;
-  const mtrt_stream_t s = current_stream();
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_nvfp4_quantize(s, x->data_ptr(), dt, q.data_ptr(), scales.data_ptr(), static_cast<const float *>(amax->data_ptr()), d0,
                                        d1, last ? 1 : 0);
@@ -490,11 +527,12 @@ PyObject *f_nvfp4_dequantize(PyObject *, PyObject *const *a, Py_ssize_t n) {
       amax->scalar_type() != at::ScalarType::Float)
     return fail("q and scales must be uint8, tensor_amax float32, on the GPU"), nullptr;
   int64_t axis;
-  if (!made_or_given(nullptr, a[3], a[4], *q, &y) || !integer(a[5], &axis) || !float_type(y, &dt))
+  const Place place(*q);
+  if (!made_or_given(nullptr, a[3], a[4], place, &y) || !integer(a[5], &axis) || !float_type(y, &dt))
     return nullptr;
   const bool last = axis == -1 || axis == y.dim() - 1;
   const int64_t d1 = y.size(-1), d0 = d1 ? y.numel() / d1 : 0;
-  const mtrt_stream_t s = current_stream();
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_nvfp4_dequantize(s, q->data_ptr(), scales->data_ptr(), static_cast<const float *>(amax->data_ptr()), y.data_ptr(), dt,
                                          d0, d1, last ? 1 : 0);
@@ -518,8 +556,9 @@ PyObject *f_layernorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!float_type(*x, &dt))
     return nullptr;
   const int64_t d = x->size(-1), rows = d ? x->numel() / d : 0;
-  const at::Tensor y = out ? *out : empty_like_device(x->sizes(), x->scalar_type(), *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor y = out ? *out : place.empty(x->sizes(), x->scalar_type());
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] { return mtrt_hip_layernorm(s, x->data_ptr(), gamma->data_ptr(), beta->data_ptr(), y.data_ptr(), dt, rows, d, eps); }))
     return nullptr;
   return none_or_new(a[4], y);
@@ -538,8 +577,9 @@ PyObject *f_softmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!float_type(*x, &dt))
     return nullptr;
   const int64_t d = x->size(-1), rows = d ? x->numel() / d : 0;
-  const at::Tensor y = out ? *out : empty_like_device(x->sizes(), x->scalar_type(), *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor y = out ? *out : place.empty(x->sizes(), x->scalar_type());
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] { return mtrt_hip_softmax(s, x->data_ptr(), y.data_ptr(), dt, rows, d); }))
     return nullptr;
   return none_or_new(a[1], y);
@@ -555,11 +595,12 @@ PyObject *w8a8(const at::Tensor &x, const at::Tensor &w, const at::Tensor &as, c
   const int64_t M = x.size(0), K = x.size(1);
   if (as.numel() != M || ws.numel() != N || (fragments ? w.numel() != mtrt_hip_gemm_w8a8_fragments_bytes(K, N) : w.size(1) != K))
     return fail("operand extents do not agree"), nullptr;
-  const at::Tensor y = out ? *out : empty_like_device({M, N}, at::ScalarType::Half, x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(x);
+  const at::Tensor y = out ? *out : place.empty({M, N}, at::ScalarType::Half);
+  const mtrt_stream_t s = place.stream;
   const float *asp = static_cast<const float *>(as.data_ptr()), *wsp = static_cast<const float *>(ws.data_ptr());
   const int64_t scratch_bytes = fragments ? mtrt_hip_gemm_w8a8_fragments_workspace(M, K, N) : 0;
-  const at::Tensor scratch = scratch_bytes ? bytes_on(x, scratch_bytes) : at::Tensor();
+  const at::Tensor scratch = scratch_bytes ? place.bytes(scratch_bytes) : at::Tensor();
   if (!launch([&] {
         return fragments ? mtrt_hip_gemm_w8a8_fragments_ws(s, x.data_ptr(), w.data_ptr(), asp, wsp, y.data_ptr(), M, K, N,
                                                            scratch_bytes ? scratch.data_ptr() : nullptr, scratch_bytes)
@@ -605,10 +646,11 @@ PyObject *f_gemm_w4a16(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!dense_on_gpu(*x) || x->scalar_type() != at::ScalarType::Half || x->dim() < 1 || scale->scalar_type() != at::ScalarType::Half)
     return fail("a must be contiguous float16 on the GPU, scale float16"), nullptr;
   const int64_t M = x->size(0);
-  const at::Tensor y = out ? *out : empty_like_device({M, N}, at::ScalarType::Half, *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor y = out ? *out : place.empty({M, N}, at::ScalarType::Half);
+  const mtrt_stream_t s = place.stream;
   const int64_t scratch_bytes = prepacked ? mtrt_hip_gemm_w4a16_workspace(M, K, N, block) : 0;
-  const at::Tensor scratch = scratch_bytes ? bytes_on(*x, scratch_bytes) : at::Tensor();
+  const at::Tensor scratch = scratch_bytes ? place.bytes(scratch_bytes) : at::Tensor();
   if (!launch([&] {
         return mtrt_hip_gemm_w4a16_ws(s, x->data_ptr(), packed ? packed->data_ptr() : nullptr, prepacked ? prepacked->data_ptr() : nullptr,
                                       scale->data_ptr(), y.data_ptr(), M, K, N, block, scratch_bytes ? scratch.data_ptr() : nullptr,
@@ -634,8 +676,9 @@ PyObject *f_linear_dense(PyObject *, PyObject *const *a, Py_ssize_t n) {
     return fail("operand extents or types do not agree"), nullptr;
   if (!float_type(*x, &dt))
     return nullptr;
-  const at::Tensor y = out ? *out : empty_like_device({M, N}, x->scalar_type(), *x);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x);
+  const at::Tensor y = out ? *out : place.empty({M, N}, x->scalar_type());
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_linear_dense(s, x->data_ptr(), w->data_ptr(), bias ? bias->data_ptr() : nullptr, y.data_ptr(), dt, M, K, N);
       }))
@@ -797,9 +840,10 @@ PyObject *f_tp_qdq(PyObject *, PyObject *const *a, Py_ssize_t n) {
       !dense_on_gpu(*in.t) ||
       !scale.read(a[1], QUANTIZE ? in.dtype : target, QUANTIZE ? target : in.dtype, in.t->sizes(), a[3]))
     return not_here();
-  const at::Tensor out = empty_like_device(in.t->sizes(), target->storage, *in.t);
+  const Place place(*in.t);
+  const at::Tensor out = place.empty(in.t->sizes(), target->storage);
   const float *sp = static_cast<const float *>(scale.dev->data_ptr());
-  const mtrt_stream_t s = current_stream();
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return QUANTIZE ? mtrt_hip_quantize(s, in.t->data_ptr(), in.dtype->code, out.data_ptr(), target->code, sp, scale.kind, scale.d0,
                                             scale.d1, scale.nb, 0)
@@ -827,8 +871,9 @@ PyObject *f_tp_layernorm(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!number(a[3], &eps))
     return nullptr;
   const int64_t d = w.t->numel(), rows = d ? x.t->numel() / d : 0;
-  const at::Tensor y = empty_like_device(x.t->sizes(), x.dtype->storage, *x.t);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x.t);
+  const at::Tensor y = place.empty(x.t->sizes(), x.dtype->storage);
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] { return mtrt_hip_layernorm(s, x.t->data_ptr(), w.t->data_ptr(), b.t->data_ptr(), y.data_ptr(), x.dtype->code, rows, d, eps); }))
     return nullptr;
   return produced(y, x.dtype);
@@ -851,8 +896,9 @@ PyObject *f_tp_softmax(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (dim != -1 && dim != x.t->dim() - 1)
     return not_here();
   const int64_t d = x.t->size(-1), rows = d ? x.t->numel() / d : 0;
-  const at::Tensor y = empty_like_device(x.t->sizes(), x.dtype->storage, *x.t);
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x.t);
+  const at::Tensor y = place.empty(x.t->sizes(), x.dtype->storage);
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] { return mtrt_hip_softmax(s, x.t->data_ptr(), y.data_ptr(), x.dtype->code, rows, d); }))
     return nullptr;
   return produced(y, x.dtype);
@@ -995,9 +1041,10 @@ PyObject *f_tp_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
   c10::SmallVector<int64_t, 6> shape(x.t->sizes().begin(), x.t->sizes().end());
   shape.back() = p.N;
   const int64_t M = x.t->numel() / p.K, scratch_bytes = mtrt_hip_linear_workspace(&p, M);
-  const at::Tensor y = empty_like_device(shape, lp->type, *x.t);
-  const at::Tensor scratch = scratch_bytes ? bytes_on(*x.t, scratch_bytes) : at::Tensor();
-  const mtrt_stream_t s = current_stream();
+  const Place place(*x.t);
+  const at::Tensor y = place.empty(shape, lp->type);
+  const at::Tensor scratch = scratch_bytes ? place.bytes(scratch_bytes) : at::Tensor();
+  const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_linear(s, &p, x.t->data_ptr(), y.data_ptr(), M, scratch_bytes ? scratch.data_ptr() : nullptr, scratch_bytes);
       }))

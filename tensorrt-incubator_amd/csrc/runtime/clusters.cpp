@@ -149,6 +149,26 @@ FragSplit split_of(int64_t slices, int splits) {
   return {uint32_t((slices + per - 1) / per), uint32_t(per), nullptr, nullptr};
 }
 
+// A plan follows from the extents alone and costs 0.4 us; a call asks for it two or three times (its workspace, then the launch), so
+// each thread keeps the last one of each kind.
+template <class Plan>
+class LastPlan {
+public:
+  template <class Make>
+  const Plan &of(int64_t M, int64_t N, int64_t K, int64_t units, bool may_split, Make &&make) {
+    const int64_t asked[] = {M, N, K, units, may_split};
+    if (!std::equal(asked, asked + 5, key)) {
+      plan = make();
+      std::copy(asked, asked + 5, key);
+    }
+    return plan;
+  }
+
+private:
+  int64_t key[5] = {-1, -1, -1, -1, -1};               // (extents are not negative)
+  Plan plan;
+};
+
 // The tile and the K split of a GEMM on fragment-order weights (see tuning::kFragTiles).
 struct FragPlan {
   const tuning::FragTile *tile = nullptr;
@@ -158,7 +178,7 @@ struct FragPlan {
   uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(split.splits) + 7) / 8)); }
   int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * tile->rows * tile->columns * 4 : 0; }
 };
-FragPlan frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may_split) {
+FragPlan make_frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may_split) {
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
   FragPlan best;
   for (const tuning::FragTile &t : tuning::kFragTiles) {
@@ -179,6 +199,10 @@ FragPlan frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may
   }
   return best;
 }
+FragPlan frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, bool may_split) {
+  static thread_local LastPlan<FragPlan> last;
+  return last.of(M, N, slices, units, may_split, [&] { return make_frag_plan(M, N, slices, units, may_split); });
+}
 double frag_rows_us(int64_t M, int64_t N, int64_t slices, int64_t units) {
   using namespace tuning;
   const double rounds = double(((N + 31) / 32 + units - 1) / units), s = double(slices);
@@ -198,7 +222,7 @@ struct W4Plan {
   uint32_t grid() const { return uint32_t(8 * ((tiles * int64_t(split.splits) + 7) / 8)); }
   int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * tile->rows * tile->columns * 4 : 0; }
 };
-W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
+W4Plan make_w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   using namespace tuning;
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
   const int64_t slices = K / 64;
@@ -248,6 +272,10 @@ W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
     }
   }
   return best;
+}
+W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
+  static thread_local LastPlan<W4Plan> last;
+  return last.of(M, N, K, units, may_split, [&] { return make_w4_plan(M, K, N, units, may_split); });
 }
 
 const char *float_name(int32_t dt) {

@@ -116,10 +116,13 @@ DeviceState *device_state() {
     set_error(MTRT_RUNTIME_ERROR, "no usable HIP device: %s", hipGetErrorString(e));
     return nullptr;
   }
+  static thread_local DeviceState *last = nullptr;     // states live as long as the process
+  if (last && last->device == device)
+    return last;
   std::lock_guard<std::mutex> lock(g_mu);
   auto it = g_states.find(device);
   if (it != g_states.end())
-    return it->second;
+    return last = it->second;
 
   hipDeviceProp_t prop;
   e = hipGetDeviceProperties(&prop, device);
@@ -164,7 +167,7 @@ DeviceState *device_state() {
     return nullptr;
   }
   g_states[device] = st;
-  return st;
+  return last = st;
 }
 
 hipModule_t builtin_module(DeviceState *st) { return st->module; }

@@ -179,6 +179,17 @@ def test_few_tiles_are_not_estimated_below_what_one_of_them_takes(gpu, shape, ke
     assert gpu.w4a16(8, *shape, 64)[0] == "mtrt_gemm_w4a16_" + kernel
 
 
+def test_a_kept_plan_is_the_calls_own(gpu, pkg):
+    """Calls in an order in which each asks for another plan than the one before it, and in one in which none does, take the same launches."""
+    calls = [lambda s=s, f=f, scratch=scratch: f(8, *s, scratch=scratch) for s in ((200, 12288, 512), (200, 512, 12288), (201, 12288, 512), (64, 8192, 96))
+             for f in (gpu.w8a8, gpu.w4a16) for scratch in (True, False)]
+    calls += [lambda s=s, dt=dt: gpu.linear(8, *s, dt) for s in ((200, 12288, 512), (100, 11520, 320)) for dt in (pkg.F16, pkg.BF16)]
+    in_turn = [c() for _ in range(2) for c in calls]
+    assert in_turn[:len(calls)] == in_turn[len(calls):]
+    assert [c() for c in calls for _ in range(2)][1::2] == in_turn[:len(calls)]
+    assert len({(name, split) for name, _, split in in_turn}) > 8
+
+
 @pytest.mark.parametrize("family,tiles", [("w8a8_frag", W8_TILES), ("w4a16", W4_TILES), ("dense_frag_f16", DENSE_TILES)])
 def test_the_shapes_that_test_every_tile_take_it(gpu, pkg, family, tiles):
     call = {"w8a8_frag": lambda *s: gpu.w8a8(8, *s), "w4a16": lambda *s: gpu.w4a16(8, *s, 64),

@@ -103,3 +103,48 @@ def test_in_place_updates_of_a_scale_are_noticed(tp):
     assert bool((lin(x).torch() == 448).all())
     lin.weight_scale.torch().fill_(2.0 ** -9)                        # 448 * 2^-9 = 0.875
     assert bool((lin(x).torch() == 392).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["amax", "dynamic"])
+def test_amax_and_scale_are_tensors_of_their_own(pkg, call):
+    """They lie in one allocation: each is a dense f32 scalar, in-place work on one leaves the other, either outlives the other, and
+    both serve as the scale of another call; so under inference mode and on a stream that is not the default one."""
+    import torch
+    x = torch.from_numpy(rng(5).standard_normal((7, 96), dtype=np.float32)).cuda()
+
+    def run():
+        if call == "amax":
+            return pkg.amax(x, 127.0)
+        return pkg.dynamic_quantize_dequantize(x, pkg.I8, 127.0)[2:]
+    want = float(x.abs().max())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    for where in (torch.no_grad(), torch.inference_mode(), torch.cuda.stream(side)):
+        with where:
+            amax, scale = run()
+            for t in (amax, scale):
+                assert t.shape == () and t.dtype == torch.float32 and t.is_cuda and t.is_contiguous() and not t.requires_grad
+            codes = pkg.quantize(x, scale.reshape(1), pkg.I8)
+            torch.cuda.synchronize()
+            assert float(amax) == want and float(scale) == float(np.float32(want) / np.float32(127.0))
+            amax.zero_()
+            assert float(scale) == float(np.float32(want) / np.float32(127.0))
+            kept = scale
+            del amax, scale
+            others = [run() for _ in range(64)]
+            assert float(kept) == float(np.float32(want) / np.float32(127.0)) and all(float(a) == want for a, _ in others)
+            assert int(codes.abs().max()) == 127
+
+
+@pytest.mark.gpu
+def test_extents_that_no_tensor_has(pkg):
+    import torch
+    a, s = torch.zeros((2, 64), dtype=torch.float16, device="cuda"), torch.zeros((1, 8), dtype=torch.float16, device="cuda")
+    w = torch.zeros(64 * 8 // 2, dtype=torch.uint8, device="cuda")
+    for n in (-1, 1 << 61):
+        with pytest.raises(RuntimeError):
+            pkg.gemm_w4a16(a, s, 64, n, 64, w_kn_packed=w)
+    q, scales, amax = torch.zeros(128, dtype=torch.uint8, device="cuda"), torch.zeros(16, dtype=torch.uint8, device="cuda"), torch.ones((), device="cuda")
+    with pytest.raises(RuntimeError):
+        pkg.nvfp4_dequantize(q, scales, amax, torch.float16, (-2, 128))
