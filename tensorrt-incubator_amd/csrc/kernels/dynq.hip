@@ -10,8 +10,9 @@
 // tensor fits in the registers of one grid: x is read once (the two-launch form reads it twice) and the time of
 // a second launch is saved, which is most of the cost of a tensor of a few MB.
 //
-// Shape: gridDim.x workgroups of 1024 lanes, one per compute unit at most (and at most 256); each lane keeps NV
-// 128-bit vectors of x in registers.  Every workgroup needs the maximum of all before it can quantize, and the
+// Shape: gridDim.x workgroups of 1024 lanes, one per compute unit at most (and at most 256); each lane keeps nv <= NV
+// 128-bit vectors of x in registers, as many as spread the tensor over the chip (with always 4, or 16, a megabyte was the work of
+// sixteen units and 20 MB that of 80: f32 -> i8 6.7 and 18.4 us, now 5.3 and 13.9; the rule stands beside the launch).  Every workgroup needs the maximum of all before it can quantize, and the
 // exchange is what a launch of a few MB spends most of its time on, so it is built from the cheapest operations
 // the memory system has: every workgroup STORES its maximum, tagged with the launch's number, into a slot of its
 // own (one device-scope store, nobody waits for it) and then reads all slots (64 lanes x 4 slots, one round trip)
@@ -58,14 +59,15 @@ template <typename X, typename Q, int NV, bool ALONE>
 __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                             typename X::storage* __restrict__ y, int64_t n, float qmax,
                                             float* __restrict__ amax_out, float* __restrict__ scale_out,
-                                            uint32_t* __restrict__ scratch, int flags, int spin_limit) {
+                                            uint32_t* __restrict__ scratch, int flags, int spin_limit, int nv) {
   using FG = FloatGroup<X>;
   using A = AbsBits<X>;
   constexpr int G = FG::G;
   __shared__ uint32_t wave_max[kDynThreads / kWave];
   __shared__ uint32_t bcast[2];
   const int64_t nvec = n / G;                        // host: n % G == 0, x / y 16-byte aligned
-  const int64_t base = int64_t(blockIdx.x) * (kDynThreads * NV) + threadIdx.x;
+  const int64_t chunk = int64_t(kDynThreads) * nv, base = blockIdx.x * chunk + threadIdx.x;
+  const int64_t end = (blockIdx.x + 1) * chunk < nvec ? (blockIdx.x + 1) * chunk : nvec;   // nv <= NV: the later vectors are past it
 
   unsigned long long* slots = reinterpret_cast<unsigned long long*>(scratch + kAmaxLineWords * kSlotLine);
   uint32_t* tag_word = scratch + kAmaxLineWords * kTagLine;
@@ -78,7 +80,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
   for (int i = 0; i < NV; ++i) {
     const int64_t v = base + int64_t(i) * kDynThreads;
     xin[i] = (u32x4){0u, 0u, 0u, 0u};
-    if (v < nvec) {
+    if (v < end) {
       xin[i] = FG::load(x + v * G);
       const uint32_t a = A::of(xin[i]);
       m = m > a ? m : a;
@@ -86,8 +88,8 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
   }
   uint32_t total;
   if constexpr (ALONE) {
-    for (uint32_t other = 1; other < gridDim.x; ++other) {
-      const int64_t first = int64_t((blockIdx.x + other) % gridDim.x) * (kDynThreads * NV) + threadIdx.x;
+    // (the own part among them, from the caches)
+    for (int64_t first = threadIdx.x; gridDim.x > 1 && first - threadIdx.x < nvec; first += kDynThreads * NV) {
       u32x4 t[NV];
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
@@ -163,7 +165,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const int64_t v = base + int64_t(i) * kDynThreads;
-    if (v < nvec) {
+    if (v < end) {
       float f[G];
       FG::unpack(xin[i], f);
       quantize_group<Q>(dv, f, flags);
@@ -179,18 +181,18 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
 
 }  // namespace dynq_cluster
 
-// (x, q, y or null, n, qmax, amax_out or null, scale_out or null, scratch, flags, spin_limit)
+// (x, q, y or null, n, qmax, amax_out or null, scale_out or null, scratch, flags, spin_limit, nv)
 //   n % G == 0 (G = 4 for f32, 8 for f16 / bf16), x and y 16-byte aligned, q aligned to G codes,
-//   gridDim.x = ceil(n / G / (1024 * NV)) <= min(number of compute units, 256), block = 1024;
+//   1 <= nv <= NV vectors a lane, gridDim.x = ceil(n / G / (1024 * nv)) <= min(number of compute units, 256), block = 1024;
 //   spin_limit < 0 (NV = 4): every workgroup takes the maximum of the whole tensor by itself (q and y must then not lie over x).
 #define MTRT_DYNQ_KERNEL(XN, XT, QN, QT, NV)                                                                          \
   extern "C" __global__ void __launch_bounds__(1024) mtrt_dynqdq_##XN##_##QN##_v##NV(                                  \
       const XT::storage* x, QT::storage* q, XT::storage* y, int64_t n, float qmax, float* amax_out, float* scale_out,  \
-      uint32_t* scratch, int32_t flags, int32_t spin_limit) {                                                          \
+      uint32_t* scratch, int32_t flags, int32_t spin_limit, int32_t nv) {                                              \
     if (NV == 4 && spin_limit < 0)                                                                                      \
-      dynq_cluster::dynqdq_body<XT, QT, 4, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit);    \
+      dynq_cluster::dynqdq_body<XT, QT, 4, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);    \
     else                                                                                                                \
-      dynq_cluster::dynqdq_body<XT, QT, NV, false>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit); }
+      dynq_cluster::dynqdq_body<XT, QT, NV, false>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv); }
 #define MTRT_DYNQ_KERNELS(XN, XT, QN, QT) MTRT_DYNQ_KERNEL(XN, XT, QN, QT, 4) MTRT_DYNQ_KERNEL(XN, XT, QN, QT, 16)
 MTRT_DYNQ_KERNELS(f32, F32, i8, I8)
 MTRT_DYNQ_KERNELS(f32, F32, f8, F8)

@@ -858,15 +858,21 @@ int32_t mtrt_hip_dynamic_quantize_dequantize(mtrt_stream_t stream, const void *x
     uint32_t *slot = reduction_slot(st, as_hip(stream));
     if (!slot)
       return MTRT_RUNTIME_ERROR;
-    const int nv = nvec <= units * 1024 * 4 ? 4 : 16;
+    // Vectors a lane: as few as leave the exchange a number of workgroups that starts without delay, half to three quarters of the units;
+    // beyond four, as few as hold the tensor.  us, f32 -> i8 (bf16 -> f8), 1, 2, 3 and 4 vectors: 0.5 MB 4.8, 5.1, 5.2, 5.5 (4.8, 5.3, 6.1,
+    // 7.1); 1 MB 5.3, 5.8, 6.4, 6.7 (5.7, 6.4, 7.1, 8.3); 2 MB 6.9, 6.8, 7.2, 7.7 (6.4, 7.0, 7.9, 9.1); 4 MB 9.2, 8.2, 8.2, 8.4 (8.8, 8.2, 8.8,
+    // 9.6); 8 MB -, 10.1, 9.8, 9.7 (-, 10.3, 10.2, 10.7); f32 -> i8 of 20, 32 and 48 MB, 5, 8 and 12 vectors against 16: 13.9, 18.4; 18.4, 21.9;
+    // 25.2, 26.7 (bf16 -> i8 15.3, 22.4; 20.8, 24.1; 28.4, 30.3).
+    const int64_t per = units * 1024;
+    int32_t nv = nvec <= per / 2 ? 1 : nvec <= per * 3 / 2 ? 2 : nvec <= per * 9 / 4 ? 3 : nvec <= per * 4 ? 4 : int32_t((nvec + per - 1) / per);
     const uint32_t grid = uint32_t((nvec + int64_t(1024) * nv - 1) / (int64_t(1024) * nv));
-    // One or two workgroups read all of x instead of waiting for each other, unless results lie over it: us, with the exchange and so, one
-    // workgroup (f32 [3, 1000]) 3.2, 2.4, two (bf16 [31, 1344]) 6.9, 6.0, three (bf16 [64, 1344]) 6.1, 6.25, four (f32 [64, 960]) 5.2, 5.3.
+    // The smallest tensors' workgroups read all of x instead of waiting for each other, unless results lie over it: us, with the exchange and
+    // so, f32 64 KiB 3.6, 3.2; 128 KiB 4.1, 3.7; 256 KiB 4.2, 4.8; 16 bits, twice the instructions a vector, 64 KiB 3.9, 3.7; 128 KiB 4.3, 4.4.
     const int64_t bytes = n * float_bytes(x_dtype);
-    const bool alone = nv == 4 && grid <= 2 && apart(x, bytes, q, n) && (!y || apart(x, bytes, y, bytes));
+    const bool alone = nvec <= (group == 4 ? 8192 : 4096) && apart(x, bytes, q, n) && (!y || apart(x, bytes, y, bytes));
     int32_t limit = alone ? -1 : g_wait_limit.load();
-    void *args[] = {&x, &q, &y, &n, &qmax, &amax_out, &scale_out, &slot, &flags, &limit};
-    return launch(st, KernelName("mtrt_dynqdq_") + xn + "_" + code_name(q_dtype) + "_v" + nv, grid, 1024,
+    void *args[] = {&x, &q, &y, &n, &qmax, &amax_out, &scale_out, &slot, &flags, &limit, &nv};
+    return launch(st, KernelName("mtrt_dynqdq_") + xn + "_" + code_name(q_dtype) + "_v" + (nv <= 4 ? 4 : 16), grid, 1024,
                   as_hip(stream), args);
   }
   // Does not fit in the registers of one grid (or is not vector-aligned): the reduction, then the element-wise pass.
