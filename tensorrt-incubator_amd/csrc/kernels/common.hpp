@@ -131,11 +131,45 @@ __device__ __forceinline__ float f8_to_f32(uint32_t packed) {
 }
 
 // ---- wave / block reductions ------------------------------------------------
+// What lane i holds and what lane i ^ OFF holds, combined; the two operands' order does not matter to `op`.  The exchanges are the
+// vector unit's own (a DPP operand of the combining instruction, or for 16 and 32 the swaps of half rows and half waves), a few
+// cycles each: through LDS (ds_bpermute, what __shfl_xor is) a step of a dependent chain is a trip of about a hundred.
+// REPEATS: lanes eight apart in a row of sixteen hold the same (they have been combined already), so that the lane four on is as good as
+// i ^ 4 and one instruction reaches it.
+template <int OFF, bool REPEATS = false, typename T, typename Op>
+__device__ __forceinline__ T xor_step(T v, Op op) {
+  static_assert(sizeof(T) == 4 && OFF >= 1 && OFF <= 32 && (OFF & (OFF - 1)) == 0, "one 32-bit value per lane");
+  const int i = __builtin_bit_cast(int, v);
+  if constexpr (OFF == 32 || OFF == 16) {
+    const auto two = OFF == 32 ? __builtin_amdgcn_permlane32_swap(i, i, false, false) : __builtin_amdgcn_permlane16_swap(i, i, false, false);
+    return op(__builtin_bit_cast(T, int(two[0])), __builtin_bit_cast(T, int(two[1])));
+  } else {
+    constexpr int kRowShl4 = 0x104, kRowShr4 = 0x114, kRowRor = 0x120, kSwapPairs = 0x4E, kSwapNext = 0xB1;   // quad_perm [2,3,0,1], [1,0,3,2]
+    int other;
+    if constexpr (OFF == 4 && !REPEATS) {              // from the next four lanes into the even fours of a row, from the last four into the odd ones
+      other = __builtin_amdgcn_update_dpp(i, i, kRowShl4, 0xF, 0x5, false);
+      other = __builtin_amdgcn_update_dpp(other, i, kRowShr4, 0xF, 0xA, false);
+    } else {
+      other = __builtin_amdgcn_mov_dpp(i, OFF >= 4 ? kRowRor + OFF : OFF == 2 ? kSwapPairs : kSwapNext, 0xF, 0xF, true);
+    }
+    return op(v, __builtin_bit_cast(T, other));
+  }
+}
+// Every lane gets the value of its group of LANES neighbouring lanes, combined by halves: far lanes first.
+template <int LANES, bool REPEATS = false, typename T, typename Op>
+__device__ __forceinline__ T lanes_reduce(T v, Op op) {
+  if constexpr (LANES > 1) return lanes_reduce<LANES / 2, (LANES >= 16)>(xor_step<LANES / 2, REPEATS>(v, op), op);
+  else return v;
+}
 template <typename T, typename Op>
 __device__ __forceinline__ T wave_reduce(T v, Op op) {
+  return lanes_reduce<kWave>(v, op);
+}
+// The same value through LDS, for kernels that keep the vector unit busy with other waves (see norm.hip).
+template <typename T, typename Op>
+__device__ __forceinline__ T wave_reduce_lds(T v, Op op) {
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1)
-    v = op(v, __shfl_xor(v, off, kWave));
+  for (int off = kWave / 2; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off, kWave));
   return v;
 }
 struct MaxU32 { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return a > b ? a : b; } };

@@ -103,6 +103,13 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
 // Hides a vector's provenance from the optimiser (no instruction is emitted).
 __device__ __forceinline__ void opaque(u32x4& t) { __asm__ volatile("" : "+v"(t)); }
 
+// A row's reduction over its wave.  The exchanges of the vector unit shorten a wave's chain, which is what few rows wait for and most
+// forms gain from; where the waves of aligned short rows fill the chip, LDS takes instructions off the vector unit.  us, LDS and vector unit:
+// LayerNorm f16 [8, 4096] 4.3, 3.9, f32 [22, 1984] 3.9, 3.5, f32 [77101, 204] 26.3, 24.9; softmax f32 [179, 1405] 3.5, 3.1, bf16 [76538, 411] 27.8,
+// 25.8; the other way LayerNorm bf16 [20000, 1024] 15.8, 16.2, [26061, 512] 11.6, 11.9, softmax bf16 [5120, 1024] 5.1, 5.7, f32 [2560, 816] 4.5, 5.1.
+template <bool LDS, typename Op>
+__device__ __forceinline__ float row_reduce(float v, Op op) { return LDS ? wave_reduce_lds(v, op) : wave_reduce(v, op); }
+
 // The row stays in registers in its STORAGE form (NV 128-bit vectors per lane) and is widened
 // again in each of the three passes: for 16-bit types that halves the live registers compared
 // with keeping f32 values (a widening is one shift or mask per element), and the higher
@@ -123,6 +130,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
     t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
 
+  constexpr bool kLds = NV == 2 || NV == 4 || (NV == 1 && E == 8);
   const float fd = float(d);
   float sum = 0.0f;
 #pragma unroll
@@ -133,7 +141,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
 #pragma unroll
     for (int k = 0; k < E; ++k) sum = sum + (live ? v[k] : 0.0f);
   }
-  const float mu = wave_reduce(sum, SumF32()) / fd;
+  const float mu = row_reduce<kLds>(sum, SumF32()) / fd;
   float sq = 0.0f;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -147,7 +155,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
       sq = sq + (live ? dv * dv : 0.0f);
     }
   }
-  const float var = wave_reduce(sq, SumF32()) / fd;
+  const float var = row_reduce<kLds>(sq, SumF32()) / fd;
   const float rstd = 1.0f / sqrtf(var + eps);
 
   const u32x4* gv = reinterpret_cast<const u32x4*>(gamma);
@@ -192,17 +200,18 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
   float v[NV * E];
   load_row<X, NV, FULL>(xr, nvec, lane, -INFINITY, v);
 
+  constexpr bool kLds = NV == 2 || NV == 4;
   float mx = -INFINITY;
 #pragma unroll
   for (int i = 0; i < NV * E; ++i) mx = fmaxf(mx, v[i]);
-  mx = wave_reduce(mx, MaxF32());
+  mx = row_reduce<kLds>(mx, MaxF32());
   float s = 0.0f;
 #pragma unroll
   for (int i = 0; i < NV * E; ++i) {
     v[i] = __expf(v[i] - mx);                        // exp(-inf) = 0 for the fill lanes
     s = s + v[i];
   }
-  s = wave_reduce(s, SumF32());
+  s = row_reduce<kLds>(s, SumF32());
   // e / s as e * (1/s): one correctly rounded reciprocal per row instead of a divide per element; at most one
   // f32 ulp from the quotient.  Together with the hardware exponential (2^(d * log2 e), a few f32 ulps off for
   // |d| ~ 10) that is far below what the order of the row sum already changes: with an exponential good to one
@@ -246,11 +255,7 @@ template <> struct RowVector<true> { typedef u32x4 type __attribute__((aligned(2
 
 template <int THREADS, typename Op>
 __device__ __forceinline__ float group_reduce(float v, Op op, float* lds) {
-  if (THREADS < kWave) {                             // several rows per wave: exchanges stay inside the row's lanes
-#pragma unroll
-    for (int off = THREADS / 2; off > 0; off >>= 1) v = op(v, __shfl_xor(v, off, kWave));
-    return v;
-  }
+  if constexpr (THREADS < kWave) return lanes_reduce<THREADS>(v, op);   // several rows per wave: exchanges stay inside the row's lanes
   v = wave_reduce(v, op);
   if (THREADS == kWave) return v;
   __syncthreads();                                   // lds may still be read from the previous reduction

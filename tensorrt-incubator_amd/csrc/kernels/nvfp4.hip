@@ -142,8 +142,7 @@ __device__ __forceinline__ void quantize_body(const typename X::storage* __restr
     float amax = 0.0f;
 #pragma unroll
     for (int k = 0; k < G; ++k) amax = fmaxf(amax, fabsf(v[k]));
-#pragma unroll
-    for (int off = 1; off < LPB; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
+    amax = lanes_reduce<LPB>(amax, MaxF32());
     const float s_dec_x = divide_by_six(amax);
     uint32_t s8 = f32x2_to_f8_ieee(s_dec_x * s_enc, 0.0f) & 0xFFu;
     s8 = (s8 & 0x7Fu) == 0x7Fu ? 0x7Fu : s8;             // NaN (0 * inf when the tensor amax is 0): 0x7F whatever its sign, as the host class
