@@ -15,11 +15,12 @@
 // Data movement: as in the quantize/dequantize clusters a lane owns one 128-bit vector of the float
 // operand per trip (4 f32 or 8 f16/bf16), so a block of 16 is held by 4 (or 2) neighbouring lanes
 // and its amax is two (one) cross-lane exchanges; every lane of the block then evaluates the
-// block's scalar chain itself.  A wave handles 8 consecutive trips (8 KiB of the float operand);
-// its codes (1 or 2 KiB) and block scales (128 or 256 B) are parked in the wave's own LDS region
+// block's scalar chain itself.  A wave handles 2, 4 or 8 consecutive trips (2 to 8 KiB of the float operand);
+// its codes (8 trips: 1 or 2 KiB) and block scales (128 or 256 B) are parked in the wave's own LDS region
 // and written out as whole cache lines, 16 bytes per lane.
 #include "common.hpp"
 #include "nvfp4_index.hpp"
+#include "read_twice.hpp"
 
 namespace nvfp4_cluster {
 
@@ -32,7 +33,7 @@ typedef float f2 __attribute__((ext_vector_type(2)));
 constexpr int kThreads = 256;
 // vectors per lane.  Codes and scales are a fifth of what a dequantize moves, so it needs little in flight: 2, 4 and 8 vectors take
 // bf16 of 134 MB 25.0, 25.4 and 25.7 us, f32 of 268 MB 42.9, 43.8 and 46.6
-constexpr int kTrips = 8, kDqTrips = 2;
+constexpr int kDqTrips = 2;
 
 // the reference's table on one f16 bit pattern (exact, slow): used for blocks that contain NaN
 __device__ __forceinline__ uint32_t f16_bits_to_f4_exact(uint32_t h) {
@@ -108,35 +109,41 @@ __device__ __forceinline__ void fill_inverse_scales(float* table, float s_enc) {
   __syncthreads();
 }
 
-// (x, q_packed, scales, tensor_amax, nvec) ; nvec 128-bit vectors of x, a multiple of the vectors per block
-template <typename X>
+// (x, q_packed, scales, tensor_amax, nvec) ; nvec 128-bit vectors of x, a multiple of the vectors per block.
+// A wave's time is the trip to memory, the scale table and then its trips one after the other, so few trips keep small tensors short and
+// many amortize the table (the rule and its figures: nvfp4_trips in clusters.cpp).  With few trips x is asked for before the table
+// is filled; with eight other waves cover the wait.  A kernel for each number: the same bodies in one kernel took 0.3 to 0.9 us more (a launch
+// fetches its instructions anew).
+template <typename X, int TRIPS>
 __device__ __forceinline__ void quantize_body(const typename X::storage* __restrict__ x, uint8_t* __restrict__ q,
                                               uint8_t* __restrict__ scales, const float* __restrict__ tensor_amax,
                                               int64_t nvec) {
   constexpr int G = FloatGroup<X>::G;                  // elements per vector: 4 or 8
   constexpr int LPB = 16 / G;                          // lanes per block: 4 or 2
   constexpr int kCodeBytes = G / 2;                    // code bytes per lane and trip
-  constexpr int kSpanCodes = kTrips * 64 * kCodeBytes; // 1 or 2 KiB per wave
-  constexpr int kSpanScales = kTrips * 64 / LPB;       // 128 or 256 B per wave
+  constexpr int kSpanCodes = TRIPS * 64 * kCodeBytes;  // eight trips: 1 or 2 KiB per wave
+  constexpr int kSpanScales = TRIPS * 64 / LPB;        // eight trips: 128 or 256 B per wave
   __shared__ __attribute__((aligned(16))) uint8_t lds[(kThreads / 64) * (kSpanCodes + kSpanScales)];
+  __shared__ float inverse_scale[256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   uint8_t* my_codes = lds + wave * (kSpanCodes + kSpanScales);
   uint8_t* my_scales = my_codes + kSpanCodes;
-  __shared__ float inverse_scale[256];
-  const int64_t span = (int64_t(blockIdx.x) * (kThreads / 64) + wave) * (kTrips * 64);   // first vector of this wave (a workgroup takes 32 KiB, see read_twice.hpp)
+  const uint32_t piece = TRIPS == 8 ? blockIdx.x : piece_of<8 / TRIPS>(blockIdx.x, gridDim.x, nvec * 16);   // behind an amax pass: see read_twice.hpp
+  const int64_t span = (int64_t(piece) * (kThreads / 64) + wave) * (TRIPS * 64);        // first vector of this wave
   const float s_enc = 2688.0f / *tensor_amax;
-  fill_inverse_scales(inverse_scale, s_enc);
-  if (span >= nvec) return;                            // whole wave
-
-  u32x4 t[kTrips];
+  if (TRIPS == 8) fill_inverse_scales(inverse_scale, s_enc);
+  if (TRIPS == 8 && span >= nvec) return;              // whole wave
+  u32x4 t[TRIPS];
 #pragma unroll
-  for (int j = 0; j < kTrips; ++j) {
+  for (int j = 0; j < TRIPS; ++j) {
     int64_t v = span + j * 64 + lane;
     v = v < nvec ? v : nvec - 1;                       // past the end: a valid vector, its results are not stored
     t[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(x) + v);
   }
+  if (TRIPS != 8) fill_inverse_scales(inverse_scale, s_enc);
+  if (TRIPS != 8 && span >= nvec) return;
 #pragma unroll
-  for (int j = 0; j < kTrips; ++j) {
+  for (int j = 0; j < TRIPS; ++j) {
     float v[G];
     FloatGroup<X>::unpack(t[j], v);
     float amax = 0.0f;
@@ -169,13 +176,14 @@ __device__ __forceinline__ void quantize_body(const typename X::storage* __restr
   }
   // this wave's own LDS region only: program order suffices, no barrier
   const int64_t left = nvec - span;                    // vectors of this span that exist (>= 1)
-  const int64_t code_bytes = (left < kTrips * 64 ? left : kTrips * 64) * kCodeBytes;
-  const int64_t scale_bytes = (left < kTrips * 64 ? left : kTrips * 64) / LPB;
+  const int64_t code_bytes = (left < TRIPS * 64 ? left : TRIPS * 64) * kCodeBytes;
+  const int64_t scale_bytes = (left < TRIPS * 64 ? left : TRIPS * 64) / LPB;
   uint8_t* qo = q + span * kCodeBytes;
   uint8_t* so = scales + span / LPB;
 #pragma unroll
-  for (int c = 0; c < kSpanCodes / 1024; ++c) {
+  for (int c = 0; c < (kSpanCodes + 1023) / 1024; ++c) {
     const int o = (c * 64 + lane) * 16;
+    if (kSpanCodes % 1024 != 0 && o >= kSpanCodes) break;
     const u32x4 vv = *reinterpret_cast<const u32x4*>(my_codes + o);
     if (o + 16 <= code_bytes) {
       *reinterpret_cast<u32x4*>(qo + o) = vv;            // q is 16-byte aligned (checked by the host side)
@@ -357,13 +365,17 @@ __device__ __forceinline__ void dequantize_cols_body(const uint8_t* __restrict__
 
 }  // namespace nvfp4_cluster
 
-// mtrt_nvfp4_q_<t>(x, q_packed, scales, tensor_amax, nvec) ; mtrt_nvfp4_dq_<t>(q_packed, scales, tensor_amax, y, nvec)
-// grid = ceil(nvec / (4 waves * 64 * 8 vectors)) and, to dequantize, of 2 vectors; block = 256; x / y and q_packed 16-byte aligned.
-#define MTRT_NVFP4_KERNELS(XN, XT)                                                                                      \
-  extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_q_##XN(                               \
+// mtrt_nvfp4_q_<t>(x, q_packed, scales, tensor_amax, nvec), 8 trips, and with 2 and 4 mtrt_nvfp4_q2_<t>, mtrt_nvfp4_q4_<t> ;
+// mtrt_nvfp4_dq_<t>(q_packed, scales, tensor_amax, y, nvec), 2 trips ; grid = ceil(nvec / (4 waves * 64 * trips)); block = 256; x / y and q_packed 16-byte aligned.
+#define MTRT_NVFP4_QUANTIZE(NAME, XT, TRIPS)                                                                            \
+  extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) NAME(                                           \
       const XT::storage* x, uint8_t* q, uint8_t* scales, const float* tensor_amax, int64_t nvec) {                      \
-    nvfp4_cluster::quantize_body<XT>(x, q, scales, tensor_amax, nvec);                                                  \
-  }                                                                                                                     \
+    nvfp4_cluster::quantize_body<XT, TRIPS>(x, q, scales, tensor_amax, nvec);                                           \
+  }
+#define MTRT_NVFP4_KERNELS(XN, XT)                                                                                      \
+  MTRT_NVFP4_QUANTIZE(mtrt_nvfp4_q2_##XN, XT, 2)                                                                        \
+  MTRT_NVFP4_QUANTIZE(mtrt_nvfp4_q4_##XN, XT, 4)                                                                        \
+  MTRT_NVFP4_QUANTIZE(mtrt_nvfp4_q_##XN, XT, 8)                                                                         \
   extern "C" __global__ void __launch_bounds__(nvfp4_cluster::kThreads) mtrt_nvfp4_dq_##XN(                              \
       const uint8_t* q, const uint8_t* scales, const float* tensor_amax, XT::storage* y, int64_t nvec) {                \
     nvfp4_cluster::dequantize_body<XT>(q, scales, tensor_amax, y, nvec);                                                \

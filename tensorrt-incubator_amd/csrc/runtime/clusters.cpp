@@ -8,6 +8,7 @@
 //  mlir-tensorrt/compiler/lib/Passes/2_Host/HostToExecutor/CUDAToExecutor/CUDAToExecutor.cpp:355-413).
 #include "runtime_internal.hpp"
 #include "../kernels/nvfp4_index.hpp"
+#include "../kernels/read_twice.hpp"
 
 #include <algorithm>
 #include <atomic>
@@ -946,6 +947,18 @@ int32_t mtrt_hip_dynamic_quantize_rows(mtrt_stream_t stream, const void *x, int3
 }
 
 namespace {
+// Vectors that a lane quantizes.  Few where the tensor gives each compute unit little, so that no wave works through a long chain of its own; 8
+// where the launch is long; 2 again where the Infinity Cache keeps nothing of what the amax pass has read.  amax, quantize and dequantize
+// in a row with 2, 4 and 8, us, bf16 (f32): 1 MiB 8.5, 8.8, 9.6 (8.3, 8.6, 9.2); 4 MiB 9.8, 10.1, 10.9 (9.6, 9.9, 10.5); 8 MiB 11.6, 11.8, 12.3
+// (11.0, 11.1, 11.7); 16 MiB 14.9, 14.8, 15.3 (14.1, 13.9, 14.5); 32 MiB 23.3, 22.6, 22.8 (20.9, 20.2, 20.4); 48 MiB 32.1, 31.4, 31.1 (28.8, 27.7,
+// 27.5); 128 MiB 72.4, 71.1, 71.4 (67.2, 67.1, 66.8); 192 MiB 108.5, 107.7, 109.1 (100.1, 101.2, 102.9); 256 MiB 142.4, 141.8, 143.9 (130.6, 133.0, 135.4).
+int64_t nvfp4_trips(int64_t nvec, int64_t units) {
+  const int64_t per = units * kBlock;
+  if (nvec <= 8 * per || (nvec * 16 >= mtrt_dev::kReadTwiceBelow && nvec <= int64_t(1) << 32))   // (a launch has less than 2^32 work items)
+    return 2;
+  return nvec <= 32 * per ? 4 : 8;
+}
+
 int32_t nvfp4_dispatch(bool quantize, hipStream_t stream, const void *xy, int32_t dtype, const void *q, const void *scales,
                        const float *tensor_amax, int64_t d0, int64_t d1, int32_t block_axis) {
   clear_error();
@@ -989,13 +1002,14 @@ int32_t nvfp4_dispatch(bool quantize, hipStream_t stream, const void *xy, int32_
     return launch(st, KernelName(nvfp4_cluster::numbers_fit(units) ? "mtrt_nvfp4_dqc_" : "mtrt_nvfp4_dqc_far_") + xn, uint32_t(blocks), kBlock, stream, args);
   }
   int64_t nvec = n / group;
-  const int64_t per_block = 4 * 64 * (quantize ? 8 : 2);   // 4 waves x 64 lanes x kTrips or kDqTrips vectors
+  const int64_t trips = quantize ? nvfp4_trips(nvec, num_compute_units(st)) : 2;   // (kDqTrips)
+  const int64_t per_block = kBlock * trips;
   const int64_t blocks = (nvec + per_block - 1) / per_block;
   if (blocks > int64_t(kMaxGrid) * 1024)
     return set_error(MTRT_INVALID_ARGUMENT, "tensor of %lld elements is too large", (long long)n);
   if (quantize) {
     void *args[] = {&xy, &q, &scales, &tensor_amax, &nvec};
-    return launch(st, KernelName("mtrt_nvfp4_q_") + xn, uint32_t(blocks), kBlock, stream, args);
+    return launch(st, KernelName(trips == 2 ? "mtrt_nvfp4_q2_" : trips == 4 ? "mtrt_nvfp4_q4_" : "mtrt_nvfp4_q_") + xn, uint32_t(blocks), kBlock, stream, args);
   }
   // as many launches as it takes: each of whole workgroups, and a workgroup's vectors are whole blocks of 16
   const int64_t most = ((int64_t(1) << 32) / kBlock - 1) * per_block;

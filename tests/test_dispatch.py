@@ -238,6 +238,16 @@ def test_dequantize_takes_as_many_launches_as_the_tensor_needs(gpu, pkg, dtype, 
     assert done == vectors and (len(gpu.launches) == 1) == (vectors < 1 << 33)
 
 
+@pytest.mark.parametrize("dtype,vector", [("F32", 4), ("F16", 8), ("BF16", 8)])
+def test_nvfp4_quantizes_few_vectors_a_lane_of_small_and_huge_tensors(gpu, pkg, dtype, vector):
+    per, cached = 256 * 256, (192 << 20) // 16             # a vector for each lane of a workgroup on each unit
+    for nvec, trips in ((4, 2), (8 * per, 2), (8 * per + 4, 4), (32 * per, 4), (32 * per + 4, 8), (cached - 4, 8), (cached, 2), (1 << 32, 2), ((1 << 32) + 4, 8), (1 << 34, 8)):
+        assert gpu.lib.mtrt_hip_nvfp4_quantize(None, 256, getattr(pkg, dtype), 256, 256, 256, nvec // 4, 4 * vector, 1) == 0
+        name, grid, block = gpu.sizes[-1]
+        assert name == "mtrt_nvfp4_q%s_%s" % ("" if trips == 8 else trips, dtype.lower()) and block == 256
+        assert (grid - 1) * 256 * trips < nvec <= grid * 256 * trips and grid * block < 1 << 32
+
+
 @pytest.mark.parametrize("M,N", [(4096, 2305), (3585, 4097), (9000, 1281), (4096, 2304), (4096, 2306), (2048, 11008), (5000, 65537)])
 def test_large_tiles_cover_the_output(gpu, pkg, M, N):
     """256 x 256 tiles, also where the last panel holds one column; launches cut into half panels have more workgroups."""

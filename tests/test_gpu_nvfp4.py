@@ -238,3 +238,24 @@ def test_more_than_2_to_the_32_vectors(pkg):
         assert torch.equal(y[r:r + 16].view(torch.int16), part.view(torch.int16)), r
     del q, s, y
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("dname", ["float32", "float16", "bfloat16"])
+def test_each_number_of_vectors_a_lane(pkg, dname):
+    """Two, four and eight vectors a lane, at the first and last tensors of each on 256 compute units, ends inside a wave's share: as in slices that two
+    vectors a lane quantize, which the oracle checks above."""
+    import torch
+    td = getattr(torch, dname)
+    vector, per, cached = 16 // td.itemsize, 256 * 256, (192 << 20) // 16
+    amax = torch.full((), 5.0, device="cuda")
+    for nvec, trips in ((8 * per - 4, 2), (8 * per + 4, 4), (32 * per, 4), (32 * per + 68, 8), (cached - 4, 8), (cached + 4, 2)):
+        x = torch.randn((nvec // 4, 4 * vector), generator=torch.Generator(device="cuda").manual_seed(nvec), device="cuda").to(td)
+        q, s = pkg.nvfp4_quantize(x, amax)
+        assert pkg.last_kernel() == "mtrt_nvfp4_q%s_%s" % ("" if trips == 8 else trips, {"float32": "f32", "float16": "f16", "bfloat16": "bf16"}[dname])
+        q, s, step = q.view(torch.uint8).flatten(), s.view(torch.uint8).flatten(), 2 * per
+        for at in range(0, nvec, step):
+            count = min(step, nvec - at)
+            part, scales = pkg.nvfp4_quantize(x[at // 4:(at + count) // 4], amax)
+            assert "_q2_" in pkg.last_kernel()
+            assert torch.equal(part.view(torch.uint8).flatten(), q[at * vector // 2:(at + count) * vector // 2]), (nvec, at)
+            assert torch.equal(scales.view(torch.uint8).flatten(), s[at * vector // 16:(at + count) * vector // 16]), (nvec, at)
