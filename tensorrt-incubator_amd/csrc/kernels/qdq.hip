@@ -419,44 +419,42 @@ enum ScaleKind { kUniform = 0, kRow = 1, kCol = 2 };
 
 // Column scales (per-channel on the last axis, blocks of nb rows): in the group loop below every group fetches its
 // own G scales and divides by each once, so the scales cost as many bytes through the vector cache as the tensor
-// and every element an IEEE divide.  Here a wave takes a STRIP of 64 groups of columns and walks kColChunkRows
+// and every element an IEEE divide.  Here a wave takes a STRIP of 64 groups of columns and walks a chunk of U
 // rows of one scale block down it: the lane's G scales are fetched, and their reciprocals formed, once per strip
 // and chunk; every row of the chunk is one contiguous KiB of the float operand per wave, as before.
 // Host guarantees as for qdq_groups<kCol>: d1 % G == 0, n / G < 2^32, operands aligned for group accesses,
 // the scales 16-byte aligned.
-constexpr int kColChunkRows = 8;
 
 // Bound by memory once enough of it is in flight and little else stands in the way: a chunk is what a lane has in flight,
 // asked for before the reciprocals are formed, and everything about a row but the lane's columns is in scalar registers.
 // bf16 [4096, 11008] to int4 in blocks of 128 rows and back (270 MB), us: 67.7 with 4 rows in flight, chunks of 32 and
 // 18 instructions an element; 55.6 with 8 rows, chunks of 16 and the short arithmetic of ExactDivisor; 53.0 with chunks
 // of 8 rows (of 4: 60.6); 49.9 with the codes left in the caches (see CodeGroup); 48.7 with one correction of the quotient.
-template <typename X, typename Q, int MODE>
+// Small tensors and blocks of few rows take four (few_column_rows in clusters.cpp has the rule and its figures), in kernels of their own, as
+// a launch fetches its instructions anew.  Counting in 32 bits takes 0.2 to 0.3 us off every launch.
+template <typename X, typename Q, int MODE, int U>
 __device__ __forceinline__ void qdq_col_strips(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                                typename X::storage* __restrict__ y, const float* __restrict__ scale,
                                                int64_t n, int64_t d1, int64_t nb, int flags) {
   using FG = FloatGroup<X>;
   constexpr int G = FG::G;
-  constexpr int U = kColChunkRows;
   using CG = CodeGroup<Q, G>;
   const uint32_t groups_per_row = uint32_t(d1 / G), strips = (groups_per_row + kWave - 1) / kWave;
-  const int64_t d0 = n / d1, nblocks = d0 / nb;
-  const int64_t chunks = (nb + kColChunkRows - 1) / kColChunkRows;
+  const uint32_t block_rows = uint32_t(nb), blocks = uint32_t(n / G) / groups_per_row / block_rows;     // all below the number of groups
+  const uint32_t chunks = (block_rows - 1) / U + 1;
   const int lane = threadIdx.x & (kWave - 1);
-  const int64_t wave = wave_in_launch(), nwaves = waves_in_launch();
-  const int64_t items = nblocks * chunks * strips;
+  const int64_t items = int64_t(blocks) * chunks * strips, nwaves = waves_in_launch();
   const bool round = !Codes<Q>::kInteger && (flags & kFlagRoundToInt);
   const bool keep = MODE != 2 || keep_fused(n);
 
-  for (int64_t item = wave; item < items; item += nwaves) {
-    const int64_t rest = item / strips;
-    const uint32_t strip = uint32_t(item - rest * strips);
-    const int64_t b = rest / chunks, chunk = rest - b * chunks;
+  for (int64_t item = wave_in_launch(); item < items; item += nwaves) {
+    const uint32_t rest = uint32_t(item) / strips, strip = uint32_t(item) - rest * strips;
+    const uint32_t b = rest / chunks, chunk = rest - b * chunks;
     const uint32_t cg = strip * kWave + lane;
     const bool live = cg < groups_per_row;
     const int64_t c0 = int64_t(live ? cg : groups_per_row - 1) * G;     // idle lanes repeat the last group, store nothing
-    const int64_t r0 = b * nb + chunk * kColChunkRows;
-    const int64_t r1 = r0 + kColChunkRows < (b + 1) * nb ? r0 + kColChunkRows : (b + 1) * nb;
+    const int64_t r0 = int64_t(b) * nb + int64_t(chunk) * U, r_end = (int64_t(b) + 1) * nb;
+    const int64_t r1 = r0 + U < r_end ? r0 + U : r_end;
     u32x4 xin[U];
     uint32_t qin[U][2];
     float sc[G];
@@ -792,16 +790,26 @@ using namespace qdq_cluster;
 // Names: mtrt_{q,dq,qdq}_{uniform,row,col,any}_<float type>_<code type>
 //   q   (x, q, scale, n, d1, nb, flags)        dq  (q, y, scale, n, d1, nb)
 //   qdq (x, q, y, scale, n, d1, nb, flags)     *_any add `kind` after nb
+// Column scales: mtrt_{q,dq,qdq}_col_<float type>_<code type> of four rows to a wave, ..._<code type>r8 of eight.
+#define MTRT_QDQ_COL_KERNELS(XN, XT, QN, QT, END, ROWS)                                                           \
+  extern "C" __global__ void __launch_bounds__(256) mtrt_q_col_##XN##_##QN##END(                                  \
+      const XT::storage* x, QT::storage* q, const float* scale, int64_t n, int64_t d1, int64_t nb, int32_t flags) { \
+    qdq_col_strips<XT, QT, 0, ROWS>(x, q, nullptr, scale, n, d1, nb, flags); }                                    \
+  extern "C" __global__ void __launch_bounds__(256) mtrt_dq_col_##XN##_##QN##END(                                 \
+      const QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb) {              \
+    qdq_col_strips<XT, QT, 1, ROWS>(nullptr, const_cast<QT::storage*>(q), y, scale, n, d1, nb, 0); }              \
+  extern "C" __global__ void __launch_bounds__(256) mtrt_qdq_col_##XN##_##QN##END(                                \
+      const XT::storage* x, QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb, \
+      int32_t flags) { qdq_col_strips<XT, QT, 2, ROWS>(x, q, y, scale, n, d1, nb, flags); }
 #define MTRT_QDQ_KERNELS(XN, XT, QN, QT)                                                                          \
+  MTRT_QDQ_COL_KERNELS(XN, XT, QN, QT, , 4)                                                                       \
+  MTRT_QDQ_COL_KERNELS(XN, XT, QN, QT, r8, 8)                                                                     \
   extern "C" __global__ void __launch_bounds__(256) mtrt_q_uniform_##XN##_##QN(                                   \
       const XT::storage* x, QT::storage* q, const float* scale, int64_t n, int64_t d1, int64_t nb, int32_t flags) { \
     qdq_groups<XT, QT, kUniform, 0>(x, q, nullptr, scale, n, d1, nb, flags); }                                    \
   extern "C" __global__ void __launch_bounds__(256) mtrt_q_row_##XN##_##QN(                                       \
       const XT::storage* x, QT::storage* q, const float* scale, int64_t n, int64_t d1, int64_t nb, int32_t flags) { \
     qdq_groups<XT, QT, kRow, 0>(x, q, nullptr, scale, n, d1, nb, flags); }                                        \
-  extern "C" __global__ void __launch_bounds__(256) mtrt_q_col_##XN##_##QN(                                       \
-      const XT::storage* x, QT::storage* q, const float* scale, int64_t n, int64_t d1, int64_t nb, int32_t flags) { \
-    qdq_col_strips<XT, QT, 0>(x, q, nullptr, scale, n, d1, nb, flags); }                                        \
   extern "C" __global__ void __launch_bounds__(256) mtrt_q_any_##XN##_##QN(                                       \
       const XT::storage* x, QT::storage* q, const float* scale, int64_t n, int64_t d1, int64_t nb, int32_t kind,  \
       int32_t flags) { qdq_any<XT, QT, 0>(x, q, nullptr, scale, n, d1, nb, kind, flags); }                        \
@@ -811,9 +819,6 @@ using namespace qdq_cluster;
   extern "C" __global__ void __launch_bounds__(256) mtrt_dq_row_##XN##_##QN(                                      \
       const QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb) {              \
     qdq_groups<XT, QT, kRow, 1>(nullptr, const_cast<QT::storage*>(q), y, scale, n, d1, nb, 0); }                  \
-  extern "C" __global__ void __launch_bounds__(256) mtrt_dq_col_##XN##_##QN(                                      \
-      const QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb) {              \
-    qdq_col_strips<XT, QT, 1>(nullptr, const_cast<QT::storage*>(q), y, scale, n, d1, nb, 0); }                  \
   extern "C" __global__ void __launch_bounds__(256) mtrt_dq_any_##XN##_##QN(                                      \
       const QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb, int32_t kind) { \
     qdq_any<XT, QT, 1>(nullptr, const_cast<QT::storage*>(q), y, scale, n, d1, nb, kind, 0); }                     \
@@ -823,9 +828,6 @@ using namespace qdq_cluster;
   extern "C" __global__ void __launch_bounds__(256) mtrt_qdq_row_##XN##_##QN(                                     \
       const XT::storage* x, QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb, \
       int32_t flags) { qdq_groups<XT, QT, kRow, 2>(x, q, y, scale, n, d1, nb, flags); }                           \
-  extern "C" __global__ void __launch_bounds__(256) mtrt_qdq_col_##XN##_##QN(                                     \
-      const XT::storage* x, QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb, \
-      int32_t flags) { qdq_col_strips<XT, QT, 2>(x, q, y, scale, n, d1, nb, flags); }                           \
   extern "C" __global__ void __launch_bounds__(256) mtrt_qdq_any_##XN##_##QN(                                     \
       const XT::storage* x, QT::storage* q, XT::storage* y, const float* scale, int64_t n, int64_t d1, int64_t nb, \
       int32_t kind, int32_t flags) { qdq_any<XT, QT, 2>(x, q, y, scale, n, d1, nb, kind, flags); }

@@ -352,6 +352,14 @@ bool fused_scalar(int32_t x_dtype, int32_t q_dtype, int64_t n) {
   return codes && n > (int64_t(q_dtype == MTRT_F8E4M3FN ? 3 : 4) << 20) && n < (int64_t(9) << 20);
 }
 
+// Column scales: four rows of a scale block to a wave instead of eight, for blocks that have no more and tensors of which eight rows would give
+// a compute unit less than six waves.  By the waves that eight rows make, us, four and eight rows: quantize bf16 -> i4, 80 waves 2.9, 3.7;
+// 528 3.7, 4.0; 1024 4.0, 4.2; 1504 5.0, 5.2; 2048 6.2, 5.95; 2519 5.7, 5.4; 4096 11.1, 10.4; 11264 25.1, 25.1; in blocks of four rows, 4096 6.8, 7.9; of
+// one, 32768 23.8, 32.2; f32 -> i8, 2048 4.55, 4.5; 3008 6.0, 5.8; 22016 38.5, 37.3.  To quantize and dequantize in one pass, bf16 -> i4, 1504 6.6, 7.3;
+// 2048 9.3, 8.5.  A dequantize by itself takes four as well at any size (384 2.8, 3.2; 2048 4.2, 4.5; 11264 22.5, 22.6), but behind a quantize it
+// finds the codes in its XCD's L2 only where both take the same rows (four behind eight: bf16 [768, 9152] to i4 and back 12.8, and 10.9).
+bool few_column_rows(int64_t nb, int64_t waves, int64_t units) { return nb <= 4 || waves <= 6 * units; }
+
 // mode: 0 quantize, 1 dequantize, 2 fused.  codes_past: nobody is known to read the codes next (see CodeGroup in qdq.hip)
 int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtype, void *q,
                      int32_t q_dtype, void *y, const float *scale, int32_t kind, int64_t d0,
@@ -423,8 +431,11 @@ int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtyp
   static const char *kModeName[] = {"q", "dq", "qdq"};
   static const char *kKindName[] = {"uniform", "row", "col"};
   static const char *kRaggedName[] = {"", "rowu", "colu"};
+  const bool strips = tiles && kind == MTRT_SCALE_COL;
+  const int64_t row_strips = (d1 / group + 63) / 64;    // of 64 groups
+  const bool few_rows = strips && few_column_rows(nb, d0 / nb * ((nb + 7) / 8) * row_strips, num_compute_units(st));
   KernelName name("mtrt_");
-  name + kModeName[mode] + "_" + (tiles ? kKindName[kind] : (ragged ? kRaggedName[kind] : "any")) + "_" + xn + "_" + qn;
+  name + kModeName[mode] + "_" + (tiles ? kKindName[kind] : (ragged ? kRaggedName[kind] : "any")) + "_" + xn + "_" + qn + (strips && !few_rows ? "r8" : "");
 
   if (mode == 2 && tiles && kind == MTRT_SCALE_UNIFORM && fused_scalar(x_dtype, q_dtype, n))
     name + "s";
@@ -450,9 +461,9 @@ int32_t qdq_dispatch(int mode, hipStream_t stream, const void *x, int32_t x_dtyp
   if (!tiles && !ragged) args[na++] = &kind_arg;
   if (mode != 1) args[na++] = &flags_arg;
 
-  if (tiles && kind == MTRT_SCALE_COL) {
-    // one wave per (scale block, chunk of 8 rows of it, strip of 64 groups of columns): see qdq_col_strips
-    const int64_t items = (d0 / nb) * ((nb + 7) / 8) * ((d1 / group + 63) / 64);
+  if (strips) {
+    // one wave per (scale block, chunk of its rows, strip of 64 groups of columns): see qdq_col_strips
+    const int64_t rows = few_rows ? 4 : 8, items = d0 / nb * ((nb + rows - 1) / rows) * row_strips;
     return launch(st, name, blocks_for(items, kBlock / 64), kBlock, stream, args);
   }
   if (ragged) {

@@ -27,6 +27,18 @@ def test_column_scales(pkg, orc, xname, qname, blocks, nb, d1):
     _check_all(pkg, orc, r.standard_normal((blocks * nb, d1), dtype=np.float32), xname, qname, pkg.SCALE_COL, blocks * nb, d1, nb, s)
 
 
+@pytest.mark.parametrize("xname,qname", [("f32", "i8"), ("bf16", "i4"), ("f16", "f8"), ("f32", "i4p")])
+@pytest.mark.parametrize("blocks,nb,strips,rows", [(2, 6136, 1, 4), (2, 6137, 1, 4), (2, 6145, 1, 8), (1541, 5, 1, 8), (1, 3079, 4, 8), (1539, 4, 1, 4), (1537, 3, 2, 4)])
+def test_rows_of_a_wave_of_column_scales(pkg, orc, xname, qname, blocks, nb, strips, rows):
+    """Four and eight rows to a wave, on both sides of the line between them on 256 compute units, ends inside a chunk, against the oracle."""
+    d0, d1 = blocks * nb, 64 * strips * (4 if xname == "f32" else 8) - 8
+    r = rng(nb + d0)
+    k = _check_all(pkg, orc, r.standard_normal((d0, d1), dtype=np.float32), xname, qname, pkg.SCALE_COL, d0, d1, nb,
+                   r.uniform(0.01, 0.1, (blocks, d1)).astype(np.float32))
+    end = "r8" if rows == 8 else ""
+    assert list(k) == ["mtrt_%s_col_%s_%s%s" % (mode, xname, qname, end) for mode in ("q", "dq", "qdq")]
+
+
 @pytest.mark.parametrize("qname,top", [("i8", 127), ("i4", 7), ("i4p", 7)])
 @pytest.mark.parametrize("kind", ["uniform", "row", "col"])
 @pytest.mark.parametrize("scale", [0.37, -0.37, 1.0, 3e-18, 2.0 ** 60, 2.0 ** -60, 1e-30, 3e38, 1e-40])
