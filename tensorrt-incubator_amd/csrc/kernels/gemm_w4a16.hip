@@ -660,6 +660,230 @@ __device__ __forceinline__ void run_tiles(const int8_t* __restrict__ a, int64_t 
   write_tile<JT, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, true);
 }
 
+// ---- 32- and 64-row tiles, K slices dealt to sets of four waves -------------------------------------------
+// The products of run_tiles on IT x 32 rows and 128 columns by SETS sets of four waves in one workgroup: set i takes the slices i, i + SETS, ... of the
+// workgroup's part, in a ring of LDS stages of its own, and the sets' sums are added through LDS at the end.
+//
+// What bounds it: instructions.  A 32-row slice is 52 vector instructions of dequantisation and 4 MFMAs to a wave, with the loads and the scalar
+// arithmetic about 110 instructions, of which a wave issues one in four to five cycles: one wave to a SIMD takes 0.236 us a slice, 0.057 of them
+// MFMAs.  Two waves issue in each other's gaps, and their slices share a barrier: 0.175 us; four 0.140 (the vector instructions alone are
+// 0.115).  64 rows, eight waves that split each slice before and by whole slices now, 0.220 and 0.193.  So the stages' offsets are constants
+// of the unrolled loop, a load's address moves on by one scalar addition, and the eight weights of a fragment are dequantised in an order in
+// which no instruction waits for the one before it.  us, (M, K, N), run_tiles and two and four sets: (76, 11264, 10560) 45.2, 37.4, 33.5; (85,
+// 3712, 8320) 16.5, 13.9, 13.1; (143, 4352, 4800) 18.9, 15.7, 14.9; short parts want one set: (48, 512, 4096) 4.3, 4.6, 5.5.  64 rows, (257, 2944,
+// 3517) 14.7, 13.4.
+//
+// Eight weights of one dword in the order of dequant4, both halves at once.  The exponents and biases are scalars.
+struct DequantScalars {
+  uint32_t e_lo = 0x64006400u, e_hi = 0x54005400u, b_lo = 0xE408u, b_hi = 0xD480u;   // 1024, 64; -1032, -72
+};
+__device__ __forceinline__ u4 dequant8_interleaved(uint32_t w, uint32_t scale, uint32_t mask, uint32_t mask_hi, const DequantScalars& k) {
+  uint32_t o0, o1, o2, o3, t;
+  __asm__ volatile(
+      "v_lshrrev_b32 %4, 8, %5\n\t"
+      "v_and_or_b32 %0, %5, %7, %9\n\t"
+      "v_and_or_b32 %1, %5, %8, %10\n\t"
+      "v_and_or_b32 %2, %4, %7, %9\n\t"
+      "v_and_or_b32 %3, %4, %8, %10\n\t"
+      "v_pk_add_f16 %0, %0, %11 op_sel_hi:[1,0]\n\t"
+      "v_pk_add_f16 %1, %1, %12 op_sel_hi:[1,0]\n\t"
+      "v_pk_add_f16 %2, %2, %11 op_sel_hi:[1,0]\n\t"
+      "v_pk_add_f16 %3, %3, %12 op_sel_hi:[1,0]\n\t"
+      "v_pk_mul_f16 %0, %6, %0 op_sel_hi:[0,1]\n\t"
+      "v_pk_mul_f16 %1, %6, %1 op_sel_hi:[0,1]\n\t"
+      "v_pk_mul_f16 %2, %6, %2 op_sel_hi:[0,1]\n\t"
+      "v_pk_mul_f16 %3, %6, %3 op_sel_hi:[0,1]"
+      : "=&v"(o0), "=&v"(o1), "=&v"(o2), "=&v"(o3), "=&v"(t)
+      : "v"(w), "v"(scale), "v"(mask), "v"(mask_hi), "s"(k.e_lo), "s"(k.e_hi), "s"(k.b_lo), "s"(k.b_hi));
+  return (u4){o0, o1, o2, o3};
+}
+
+template <int IT, int SETS>
+struct Sets {
+  static constexpr int kStages = 4, kStageBytes = IT * 4096, kRing = kStages * kStageBytes;
+  static constexpr int kOut = 4 * 32 * IT * gemm_core::kOutRow + 2048, kSum = (SETS - 1) * IT * 16384;
+  static constexpr int kMost = SETS * kRing > kSum ? SETS * kRing : kSum;
+  static constexpr int kLds = kMost > kOut ? kMost : kOut;
+};
+
+template <int IT, int SETS, class Epilogue>
+__device__ __forceinline__ void run_sets(const int8_t* __restrict__ a, int64_t row_bytes, const uint32_t* __restrict__ wp,
+                                         const uint16_t* __restrict__ scale, uint32_t slices_per_block, Epilogue& epi, uint16_t* __restrict__ y,
+                                         int64_t M, int64_t N, const gemm_frag::Part& part, int8_t* lds) {
+  using namespace gemm_core;
+  using S = Sets<IT, SETS>;
+  constexpr int NS = S::kStages, DA = NS - 1;          // of a set's slices, the weights of NS and the activations of DA are on their way
+  constexpr int AN = 4;                                // activation fragments read ahead
+  constexpr int TB = 4 - AN / IT;                      // the first k-step that reads a fragment of the next slice
+  constexpr int kSlice = IT + 2;                       // memory instructions of a slice: activations, then nibbles and scales of the one after it
+  static_assert((IT == 1 || IT == 2) && NS % 2 == 0 && (DA - 1) * kSlice + 2 < 64, "fragment sets alternate, wait counter range");
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), slot = wave & 3, set = wave >> 2;
+  const int frow = lane & 31, fhalf = lane >> 5;
+  const int64_t total_slices = row_bytes / 128, ntiles = (N + 31) / 32;
+  const uint32_t nslices = __builtin_amdgcn_readfirstlane(part.nslices), rounds = (nslices + SETS - 1) / SETS, mine = (nslices + SETS - 1 - set) / SETS;
+  // (a set without a slice fetches the part's first ones and multiplies none)
+  const uint32_t slice0 = __builtin_amdgcn_readfirstlane(part.slice0) + (mine ? set : 0);
+
+  v16f acc[IT][1];
+  uint32_t aoff[IT];
+#pragma unroll
+  for (int g = 0; g < IT; ++g) {
+    const int lrow = (slot * IT + g) * 8 + (lane >> 3);
+    const int64_t row = part.m0 + lrow;                // rows past the edge re-read the last row; never stored
+    aoff[g] = uint32_t(row < M ? row : M - 1) * uint32_t(row_bytes) + uint32_t(((lane & 7) ^ ((lrow >> 1) & 7)) << 4);
+  }
+  const int8_t* asrc = a + uint64_t(slice0) * 128;
+  v4i fa[2][AN];
+  u4 fb[2], raw[NS];
+  uint32_t sc[NS];
+  const uint32_t mask = nibble_pair_mask(), mask_hi = mask << 4;
+  const uint32_t wlane = uint32_t(lane) * 16;
+  int64_t tile = int64_t(__builtin_amdgcn_readfirstlane(uint32_t(part.n0 / 32))) + slot;
+  tile = tile < ntiles ? tile : ntiles - 1;            // tiles past N: some valid data, never stored
+  const int8_t* wsrc = reinterpret_cast<const int8_t*>(wp) + (tile * total_slices + slice0) * 1024;
+  const int64_t col = tile * 32 + frow;
+  const uint32_t scol = uint32_t(col < N ? col : N - 1) * 2;
+  int8_t* ring = lds + set * S::kRing;
+  const uint32_t lds_base = uint32_t(uintptr_t((lds_void_t*)ring));
+  uint32_t a_lane[4];
+#pragma unroll
+  for (int p = 0; p < 4; ++p) a_lane[p] = lds_base + uint32_t(lds_off(frow, 2 * p + fhalf));
+  auto read_a = [&](v4i& dst, uint32_t addr, auto at) {  // at: in 4 KiB from the ring's start
+    __asm__ volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(decltype(at)::value * 4096) : "memory");
+  };
+  // Activations and weights each move on to the set's next slice once theirs has been asked for; past its last, that one again.
+  uint32_t aleft = mine ? mine - 1 : 0, wleft = aleft;
+  auto issue_a = [&](auto stage, auto group) {
+    constexpr int ST = decltype(stage)::value, G = decltype(group)::value;
+    __asm__ volatile("" : "+v"(aoff[G]));
+    __builtin_amdgcn_global_load_lds((global_void_t*)(asrc + aoff[G]), (lds_void_t*)(ring + ST * S::kStageBytes + (slot * IT + G) * 1024), 16, 0, 0);
+    if constexpr (G == IT - 1) {
+      const uint32_t go = uint32_t(-int32_t(aleft)) >> 31;   // aleft > 0
+      aleft -= go;
+      asrc += (128u * SETS) & (0u - go);
+    }
+  };
+  const uint32_t scale_row_bytes = uint32_t(N) * 2, block0 = slice0 ? slice0 / slices_per_block : 0;
+  uint32_t frem = slice0 - block0 * slices_per_block;
+  const int8_t* srow = reinterpret_cast<const int8_t*>(scale) + uint64_t(block0) * scale_row_bytes;
+  const uint32_t srem = SETS % slices_per_block;       // SETS slices on: so many slices and whole blocks
+  const uint64_t sbytes = uint64_t(SETS / slices_per_block) * scale_row_bytes;
+  auto issue_w = [&](auto reg) {
+    constexpr int R = decltype(reg)::value;
+    __asm__ volatile("global_load_dwordx4 %0, %1, %2" : "=v"(raw[R]) : "v"(wlane), "s"(wsrc) : "memory");
+    __asm__ volatile("global_load_ushort %0, %1, %2" : "=v"(sc[R]) : "v"(scol), "s"(srow) : "memory");
+    const uint32_t go = uint32_t(-int32_t(wleft)) >> 31, all = 0u - go;
+    wleft -= go;
+    wsrc += (1024u * SETS) & all;
+    frem += srem & all;
+    srow += sbytes & (uint64_t(all) << 32 | all);
+    const uint32_t wrap = 0u - (uint32_t(int32_t(frem - slices_per_block) >> 31) + 1u);   // all ones where frem has reached the block's end
+    frem -= slices_per_block & wrap;
+    srow += scale_row_bytes & wrap;
+  };
+  DequantScalars scalars;
+  __asm__ volatile("" : "+s"(scalars.e_lo), "+s"(scalars.e_hi), "+s"(scalars.b_lo), "+s"(scalars.b_hi));
+  auto dequant = [&](auto reg, auto step, u4& frag) {
+    constexpr int R = decltype(reg)::value;
+    frag = dequant8_interleaved(raw[R][decltype(step)::value], sc[R], mask, mask_hi, scalars);
+  };
+
+  // in front of the loop, as the loop would have issued them
+  issue_w(IntC<0>{});
+  static_for<0, DA>([&](auto v) {
+    static_for<0, IT>([&](auto g) { issue_a(v, g); });
+    issue_w(IntC<decltype(v)::value + 1>{});
+  });
+  __builtin_amdgcn_sched_barrier(0);
+  {                                                    // accumulators cleared by the matrix cores under those loads
+    v4i none = {0, 0, 0, 0};
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+      __asm__ volatile("" : "+v"(none));
+      acc[i][0] = F16Traits::mfma(none, none, F16Traits::zero());
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  // slice 0's: behind them two loads of weights and whole slices
+  __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(raw[0]), "+v"(sc[0]) : "n"(2 + (DA - 1) * kSlice) : "memory");
+  __asm__ volatile("s_barrier" ::: "memory");
+  static_for<0, AN>([&](auto n) {
+    constexpr int X = decltype(n)::value;
+    read_a(fa[0][X], a_lane[X / IT], IntC<X % IT>{});
+  });
+  dequant(IntC<0>{}, IntC<0>{}, fb[0]);
+
+  // k-step T of the slice in stage and weight registers U
+  auto kstep = [&](auto pos, auto step) {
+    constexpr int U = decltype(pos)::value, T = decltype(step)::value, NEXT = (U + 1) % NS;
+    if constexpr (T == TB) {
+      // The next slice's activations have landed: behind them two loads of weights and whole slices.  Past the barrier every wave has used
+      // the fragments of the slice before this one, into whose stage the loads below go.
+      __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(2 + (DA - 2) * kSlice) : "memory");
+      __asm__ volatile("s_barrier" ::: "memory");
+    }
+    // the next slice's weights: behind them whole slices and one load of activations
+    if constexpr (T == 3) __asm__ volatile("s_waitcnt vmcnt(%2)" : "+v"(raw[NEXT]), "+v"(sc[NEXT]) : "n"((DA - 1) * kSlice + 1) : "memory");
+    static_for<0, IT>([&](auto cc) {
+      constexpr int c = decltype(cc)::value, X = (U * 4 + T) * IT + c, SET = (X / AN) % 2, AI = X % AN;
+      constexpr int X2 = T * IT + c + AN, T2 = X2 / IT;  // the fragment read now, AN further on in the stream
+      __asm__ volatile("s_waitcnt lgkmcnt(%1)" : "+v"(fa[SET][AI]) : "n"(AN - 1) : "memory");
+      acc[c][0] = F16Traits::mfma(__builtin_bit_cast(v4i, fb[T % 2]), fa[SET][AI], acc[c][0]);
+      read_a(fa[1 - SET][AI], a_lane[T2 % 4], IntC<(T2 >= 4 ? NEXT : U) * IT + X2 % IT>{});
+      if constexpr (c == 0 && T >= TB && T - TB < IT) issue_a(IntC<(U + DA) % NS>{}, IntC<T - TB>{});
+      if constexpr (c == 0) dequant(IntC<T == 3 ? NEXT : U>{}, IntC<(T + 1) % 4>{}, fb[1 - T % 2]);
+      if constexpr (T == 3 && c == IT - 1) issue_w(pos);
+      __builtin_amdgcn_sched_barrier(0);
+    });
+  };
+  uint32_t s = 0;
+  for (bool more = true; more;) {
+    static_for<0, NS>([&](auto u) {
+      if (!more) return;
+      if (s >= rounds) {
+        more = false;
+        return;
+      }
+      if (s < mine) static_for<0, 4>([&](auto t) { kstep(u, t); });
+      else __asm__ volatile("s_barrier" ::: "memory");   // the last round's slices are other sets'
+      ++s;
+    });
+  }
+  __builtin_amdgcn_s_waitcnt(0x0070);                  // the surplus loads and fragment reads have landed: their
+#pragma unroll                                         // registers stay allocated up to here
+  for (int i = 0; i < AN; ++i) __asm__ volatile("s_waitcnt lgkmcnt(0)" ::"v"(fa[0][i]), "v"(fa[1][i]) : "memory");
+#pragma unroll
+  for (int q = 0; q < NS; ++q) __asm__ volatile("s_waitcnt vmcnt(0)" ::"v"(raw[q]), "v"(sc[q]) : "memory");
+  __syncthreads();
+  f32x4* sum = reinterpret_cast<f32x4*>(lds) + slot * (IT * 256) + lane;
+  if (set) {                                           // the sums to the first set, added in the sets' order
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        sum[(set - 1) * (IT * 1024) + (i * 4 + q) * 64] = (f32x4){acc[i][0][4 * q], acc[i][0][4 * q + 1], acc[i][0][4 * q + 2], acc[i][0][4 * q + 3]};
+  }
+  __syncthreads();
+  if (!set) {
+#pragma unroll
+    for (int k = 0; k < SETS - 1; ++k)
+#pragma unroll
+      for (int i = 0; i < IT; ++i)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const f32x4 o = sum[k * (IT * 1024) + (i * 4 + q) * 64];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) acc[i][0][4 * q + e] = acc[i][0][4 * q + e] + o[e];
+        }
+  }
+  if (part.splits > 1) {
+    __syncthreads();
+    if (!gemm_frag::meet<float, 1>(acc, part, lds, slot, set == 0)) return;
+  }
+  write_tile<1, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, set == 0);
+}
+
 // Common body of the weight-in-register kernels: which tile and which slices, which wave does what.
 template <class S, class Epilogue>
 __device__ __forceinline__ void weight_regs_kernel(const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp,
@@ -742,6 +966,14 @@ extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x384_bi
     EPI<128 * JT> epi{bias};                                                                                            \
     run_tiles<IT, JT, D>(reinterpret_cast<const int8_t*>(a), 2 * K, wp, scale, uint32_t(block / BKH), epi, y, M, N, part, lds); \
   }
+#define MTRT_W4_ROUNDS_KERNEL(TILE, EPI, IT, SETS)                                                                      \
+  extern "C" __global__ void __launch_bounds__(256 * SETS, 4) mtrt_gemm_w4a16_##TILE(MTRT_W4_ARGS) {                    \
+    __shared__ __attribute__((aligned(16))) int8_t lds[Sets<IT, SETS>::kLds];                                           \
+    gemm_frag::Part part;                                                                                               \
+    if (!gemm_frag::part_of<32 * IT, 128>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / BKH, sp, part, 4)) return;         \
+    EPI<128> epi{bias};                                                                                                 \
+    run_sets<IT, SETS>(reinterpret_cast<const int8_t*>(a), 2 * K, wp, scale, uint32_t(block / BKH), epi, y, M, N, part, lds); \
+  }
 #define MTRT_W4_SETS_KERNEL(TILE, EPI, THREADS, WAVES, ...)                                                             \
   extern "C" __global__ void __launch_bounds__(THREADS, WAVES) mtrt_gemm_w4a16_##TILE(MTRT_W4_ARGS) {                   \
     using S = Shape<__VA_ARGS__>;                                                                                       \
@@ -751,7 +983,8 @@ extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x384_bi
   }
 // t128x256: an activation fragment read from LDS serves two MFMAs and the panel is fetched for half as many workgroups as
 // with 128 columns; two slices ahead (a ring of four stages), ahead of eight waves and four slices by 8 % on average.
-// t64x128, t128x128: eight waves in two sets that split each slice, four slices ahead: ahead of four waves (up to 15 %,
+// t32x128x2, t32x128x4, t64x128: run_sets, block = 512 or, x4, 1024.
+// t128x128: eight waves in two sets that split each slice, four slices ahead: ahead of four waves (up to 15 %,
 // M = 200, K = 8832, N = 11520 68 -> 54 us) where the launch is not short.  What a workgroup moves through its CU's L1 is
 // dominated by the activation panel (16 KiB per slice of 128 rows against 4 KiB of weights).
 // t128x64: matrices at most 64 columns wide.
@@ -760,7 +993,9 @@ extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w4a16_t256x384_bi
   MTRT_W4_TILE_KERNEL(t32x128##SUFFIX, EPI, 1, 1, 4, 2)            \
   MTRT_W4_TILE_KERNEL(t64x256##SUFFIX, EPI, 2, 2, 4, 2)            \
   MTRT_W4_TILE_KERNEL(t128x256##SUFFIX, EPI, 4, 2, 2, 1)           \
-  MTRT_W4_SETS_KERNEL(t64x128##SUFFIX, EPI, 512, 2, 1, 4, 1, 2, 4, 8, 2) \
+  MTRT_W4_ROUNDS_KERNEL(t32x128x2##SUFFIX, EPI, 1, 2)              \
+  MTRT_W4_ROUNDS_KERNEL(t32x128x4##SUFFIX, EPI, 1, 4)              \
+  MTRT_W4_ROUNDS_KERNEL(t64x128##SUFFIX, EPI, 2, 2)                \
   MTRT_W4_SETS_KERNEL(t128x128##SUFFIX, EPI, 512, 2, 1, 4, 1, 2, 4, 8)   \
   MTRT_W4_SETS_KERNEL(t128x64##SUFFIX, EPI, 256, 1, 1, 2, 1, 2, 4, 5)
 MTRT_W4_TILE_KERNELS(, PlainEpilogue)

@@ -104,6 +104,17 @@ constexpr W4Tile kW4Tiles[] = {
     {"t256x256", 256, 256, 256, false, 0.0, 7.3, 1.589, 0.615, 0.0, 0.0, 5.99, 1.0},
     {"t256x384", 256, 384, 256, false, 0.0, 8.46, 2.637, 0.525, 0.0, 0.0, 7.59, 1.415},
 };
+// 32-row tiles by two and four sets of four waves (run_sets in gemm_w4a16.hip) take shorter slices and a later start: from 17 slices to a
+// workgroup, and four sets from 24 where each workgroup has a compute unit.  us, one, two and four sets, by slices, unsplit: up to 8 two sets take
+// 1.16 times as long as one, 13 to 16 as long, 21 to 28 0.955, 41 to 80 0.884 (and four 0.81), more 0.853 (0.72).  Fitted like the tiles above to
+// 555 launches of 300 shapes, M 33 ... 2048; a form takes over the tile's own plan, and another tile's where it promises a tenth: over those
+// shapes 2.6 % less time on average, (75, 7680, 10368) 36.9 -> 26.4, (147, 6016, 5888) 28.0 -> 21.3, (62, 3072, 8640) 14.5 -> 11.6.
+constexpr W4Tile kW4Sets[] = {
+    {"t32x128x2", 32, 128, 512, true, 4.175, 0.137, 0.207, 0.593, 1.573, 0.371, 3.056, 0.183},
+    {"t32x128x4", 32, 128, 1024, true, 0.306, 5.059, 0.178, 0.775, 1.789, 0.370, 4.241, 0.139},
+};
+constexpr int64_t kW4TwoSetsFrom = 17, kW4FourSetsFrom = 24, kW4FourSetsSameSplitFrom = 32;
+constexpr double kW4SetsPromise = 0.9;
 // Short products are estimated without that bound, which leaves them on the 128-row tiles: K up to 512, and up to 1024 with at most 256
 // columns.  The reason is not time, (33, 256, 64) takes 5.3 us on t128x128 and 3.4 on t32x128: these are the shapes by which the tests
 // reach the 128-row kernels and name them.
@@ -272,6 +283,25 @@ W4Plan make_w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_spl
         best = p;
     }
   }
+  const W4Tile &one = kW4Tiles[0], &two = kW4Sets[0], &four = kW4Sets[1];
+  if (!best.tile || !fits(tiles_of(one)))
+    return best;
+  W4Plan sets;
+  for (const W4Tile *t : {&two, &four}) {
+    for (int splits : kSplits) {
+      if (splits > 1 && (!may_split || slices < 2 * splits || tiles_of(*t) > int64_t(kTickets) || tiles_of(*t) * splits > 2 * units))
+        break;
+      const W4Plan p = plan_of(*t, splits);
+      if (t == &two ? p.split.per < kW4TwoSetsFrom : p.split.per < kW4FourSetsFrom || p.tiles * p.split.splits > units)
+        continue;
+      if (!sets.tile || p.us < sets.us)
+        sets = p;
+    }
+  }
+  if (sets.tile && sets.us < kW4SetsPromise * best.us)
+    return sets;
+  if (best.tile == &one && best.split.per >= kW4TwoSetsFrom)
+    best.tile = best.split.per >= kW4FourSetsSameSplitFrom && best.tiles * best.split.splits <= units ? &four : &two;
   return best;
 }
 W4Plan w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {

@@ -172,8 +172,8 @@ def test_the_tile_a_shape_takes(gpu, pkg, family, shape, kernel):
 
 
 @pytest.mark.parametrize("shape,kernel", [
-    ((92, 640, 6336), "t32x128"), ((1001, 896, 640), "t32x128"), ((805, 1536, 768), "t32x128"), ((606, 1280, 384), "t32x128"), ((579, 1152, 1550), "t32x128"),
-    ((33, 576, 320), "t32x128"), ((300, 1024, 257), "t32x128"), ((300, 1024, 256), "t128x128"), ((300, 1088, 256), "t32x128"), ((300, 512, 2000), "t128x128")])
+    ((92, 640, 6336), "t32x128"), ((1001, 896, 640), "t32x128"), ((805, 1536, 768), "t32x128x2"), ((606, 1280, 384), "t32x128"), ((579, 1152, 1550), "t32x128x2"),
+    ((33, 576, 320), "t32x128"), ((300, 1024, 257), "t32x128"), ((300, 1024, 256), "t128x128"), ((300, 1088, 256), "t32x128x2"), ((300, 512, 2000), "t128x128")])
 def test_few_tiles_are_not_estimated_below_what_one_of_them_takes(gpu, shape, kernel):
     """On both sides of the lines between short products and others: 512 and 1024 of K, 256 columns."""
     assert gpu.w4a16(8, *shape, 64)[0] == "mtrt_gemm_w4a16_" + kernel

@@ -254,6 +254,28 @@ def test_every_w4a16_tile(pkg, shape, tile, split):
     assert bool(((y.double() - ref).abs() <= tol).all())
 
 
+# Sets of waves that take slices in turn: parts with a whole number of rounds and each rest, the last part of a split another one
+# than the others, ragged rows and columns; blocks of one, two, three and four slices and one block for all.
+@pytest.mark.parametrize("shape,tile,blocks", [
+    ((33, 1152, 130), "t32x128x2", (64, 128, 192, 1152)), ((40, 1088, 130), "t32x128x2", (64,)), ((63, 8768, 130), "t32x128x2", (64,)), ((65, 8256, 130), "t32x128x2", (64, 192)),
+    ((33, 2304, 8641), "t32x128x4", (64, 128, 192, 256, 2304)), ((33, 2368, 8641), "t32x128x4", (64,)), ((33, 2176, 8641), "t32x128x4", (128,)),
+    ((97, 2240, 4100), "t32x128x4", (64, 320)), ((33, 8832, 3000), "t32x128x4", (64, 192)), ((33, 6848, 4100), "t32x128x4", (64,)),
+    ((130, 1152, 8000), "t64x128", (64, 128, 192, 1152)), ((97, 1216, 8641), "t64x128", (64,)), ((33, 2688, 8641), "t64x128", (64, 128)), ((40, 2496, 8641), "t64x128", (192,))])
+def test_w4a16_slices_in_turn(pkg, shape, tile, blocks):
+    import torch
+    M, K, N = shape
+    for block in blocks:
+        a, packed, s, wd = _w4_inputs(M + block, M, K, N, block)
+        a[3, 0], a[4, K - 1] = float("inf"), float("-inf")     # a slice counts once: no infinity of another's, none that cancels
+        y = pkg.gemm_w4a16(a, s, K, N, block, w_prepacked=pkg.gemm_w4a16_prepack(packed, K, N)).double()
+        _is(pkg, "mtrt_gemm_w4a16_" + tile)
+        for row, k, sign in ((3, 0, 1.0), (4, K - 1, -1.0)):
+            assert torch.equal(y[row].nan_to_num(7.0, posinf=1.0, neginf=-1.0), torch.where(wd[k] == 0, torch.full_like(wd[k], 7.0), sign * wd[k].sign()))
+        a[3:5], y[3:5] = 0, 0
+        ref, mass = a.double() @ wd, a.double().abs() @ wd.abs()
+        assert bool(((y - ref).abs() <= 2.0 ** -11 * ref.abs() + (1 + 2.0 ** -11) * (K + 1) * 2.0 ** -24 * mass + 2.0 ** -25).all()), block
+
+
 @pytest.mark.parametrize("dname", ["float16", "bfloat16"])
 @pytest.mark.parametrize("shape,tile,split", DENSE_TILES)
 def test_every_dense_tile(pkg, shape, tile, split, dname):
