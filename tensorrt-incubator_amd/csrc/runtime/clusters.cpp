@@ -1298,17 +1298,20 @@ int32_t mtrt_hip_gemm_w8a8_prepack_fragments(mtrt_stream_t stream, const void *w
 
 namespace {
 // Which kernel a W8A8 call on fragment-order weights takes.  Up to 32 rows: the kernels bound by reading the weights once
-// (17 to 32 rows, and fewer when at most half of the compute units would get a 32-column tile, the wave-private kernel with
+// (17 to 32 rows, and fewer when at most half of the compute units would get a 32-column tile and K is long, the wave-private kernel with
 // eight waves splitting K: M = 32 at (K, N) = (11008, 4096) 18.6 -> 12.9 us, M = 16 there 15.1 -> 11.7; with more tiles and
-// up to 16 rows the four-wave kernel with its hand-counted waits: M = 1 at (4096, 11008) 10.7 against 12.5 us).
+// up to 16 rows the four-wave kernel with its hand-counted waits: M = 1 at (4096, 11008) 10.7 against 12.5 us.  Of few tiles, us, eight and four
+// waves, weights in the L2s (from memory): (1, 1024, 1024) 3.6, 3.6 (3.7, 3.4); (2, 2304, 704) 4.3, 3.5 (4.5, 3.9); (4, 2560, 1600) 4.4, 3.5 (4.7,
+// 4.5); (16, 3072, 2048) 4.6, 3.8 (5.2, 5.5); (12, 4224, 768) 5.2, 4.3 (5.7, 6.1); (5, 11392, 384) 8.2, 6.3 (8.6, 9.4).)
 // 33 to 64 rows: the wave-private kernel or a tile, by estimate.  Above: the tile and K split frag_plan estimates fastest.
+constexpr int64_t kW8LongK = 2688;
 struct W8Plan {
   enum { kSmall16, kRows, kTile } kind;
   FragPlan tile;
 };
 W8Plan w8_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   if (M <= 32)
-    return {M > 16 || 2 * ((N + 31) / 32) <= units ? W8Plan::kRows : W8Plan::kSmall16, {}};
+    return {M > 16 || (K >= kW8LongK && 2 * ((N + 31) / 32) <= units) ? W8Plan::kRows : W8Plan::kSmall16, {}};
   const FragPlan tile = frag_plan(M, N, K / 128, units, may_split);
   if (M <= 64 && frag_rows_us(M, N, K / 128, units) < tile.us)
     return {W8Plan::kRows, {}};
