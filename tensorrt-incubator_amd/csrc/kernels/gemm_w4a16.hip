@@ -1350,8 +1350,10 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
   __syncthreads();                                     // the next chunk of this workgroup reuses the LDS
 }
 
-// (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M <= 16, K % 128 == 0, N, block % 128 == 0, or 64 for
-// _b64) ; M * K < 2^31.
+// (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M, K % 128 == 0, N, block % 128 == 0, or 64 for
+// _b64) ; M * K <= 2^31.  More than 16 rows go in ceil(M / 16) groups, a whole number of which the grid is: each group's workgroups follow one
+// another and the last group may have fewer rows.  A group takes its own activations and all of the weights, which the caches hold by then: what a workgroup
+// moves in is the four waves' 4 KiB of activations and 1 KiB of weights a tile and slice, whatever the rows.
 // grid = one or two workgroups per compute unit, at most ceil(N / 16), block = 256: workgroup g owns tiles / grid consecutive
 // 16-column tiles (the first tiles % grid workgroups one more), three at a time.
 // What its time is, from timestamps in a copy of the kernel, (16, 4096, 11008): four waves, one per SIMD, each with eight of the 32
@@ -1370,10 +1372,10 @@ constexpr int kStripWaves = 4;
 template <int G, int SC>
 __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
                                        uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block,
-                                       const uint16_t* __restrict__ bias, int8_t* lds) {
+                                       const uint16_t* __restrict__ bias, uint32_t b, uint32_t grid, int8_t* lds) {
   // tiles / grid tiles each, the first tiles % grid workgroups one more (32-bit arithmetic: as 64-bit divisions this was
   // a microsecond of scalar instructions in front of the first load)
-  const uint32_t tiles = (uint32_t(N) + 15) / 16, grid = gridDim.x, b = blockIdx.x;
+  const uint32_t tiles = (uint32_t(N) + 15) / 16;
   const uint32_t per = tiles / grid, rem = tiles - per * grid;
   const uint32_t t0 = b * per + (b < rem ? b : rem), t1 = t0 + per + (b < rem ? 1 : 0);
   for (uint32_t t = t0; t < t1; t += 3) {
@@ -1388,9 +1390,18 @@ __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uin
       const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,                \
       uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {      \
     __shared__ __attribute__((aligned(16))) int8_t lds[kStripWaves * 4 * 4096];                                           \
-    if (M <= 4) strips<1, SC>(a, ws, scale, y, M, K, N, block, bias, lds);                                                \
-    else if (M <= 8) strips<2, SC>(a, ws, scale, y, M, K, N, block, bias, lds);                                           \
-    else strips<4, SC>(a, ws, scale, y, M, K, N, block, bias, lds);                                                       \
+    uint32_t b = blockIdx.x, grid = gridDim.x;                                                                            \
+    if (M > 16) {                                                                                                         \
+      grid /= (uint32_t(M) + 15) / 16;                                                                                    \
+      const uint32_t row0 = b / grid * 16;                                                                                \
+      b %= grid;                                                                                                          \
+      a += uint64_t(row0) * K;                                                                                            \
+      y += uint64_t(row0) * N;                                                                                            \
+      M = M - row0 < 16 ? M - row0 : 16;                                                                                  \
+    }                                                                                                                     \
+    if (M <= 4) strips<1, SC>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                       \
+    else if (M <= 8) strips<2, SC>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                  \
+    else strips<4, SC>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                              \
   }
 MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16, 1)
 MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16_b64, 2)

@@ -1573,6 +1573,29 @@ bool w4_fast(const void *a, const void *w_prepacked, int64_t K, int64_t block) {
   return w_prepacked && K > 0 && K % 64 == 0 && block % 64 == 0 && aligned(a, 16) && aligned(w_prepacked, 16);
 }
 
+// Whether the strip kernel (16 rows by 16 columns over all of K, four waves) takes a product.  Up to 16 rows: blocks of 64 where each wave
+// has a slice of 128 k; the kernel behind, with slices of 64, is as fast below that.
+// 17 to 512 rows in groups of 16, where the 32-row kernel and the tiles leave most of the chip idle: by how many of its 16 columns' tiles, side by side,
+// a workgroup has where there is one to a compute unit.  Each slice of 512 k takes 0.34, 0.53 and 0.75 us so, 0.57 in the 32-row kernel,
+// and the walk down K gets long against tiles that share it.  us, (M, K, N), others and strips: one a unit (27, 7040, 384) 10.6, 6.2; (45, 5376, 320)
+// 9.0, 5.8; (146, 5760, 256) 9.8, 6.2; (37, 9216, 1247) 11.8, 8.9; two (22, 13056, 2880) 16.3, 12.9; (190, 1408, 640) 6.9, 4.1; (211, 6784, 384) 11.2, 10.1,
+// (96, 12032, 1088) 13.7, 15.4; three (52, 2432, 2496) 8.1, 6.2; (386, 1920, 448) 8.3, 6.9; (54, 5120, 4032) 12.2, 12.2; (29, 5120, 5056) 10.2, 9.2; four and
+// more (186, 4224, 1664) 11.6, 15.7; (418, 2304, 448) 8.9, 11.1.  Over 80 products of the rule's ranges 1.32 times as fast in the geometric mean.  Blocks of 64 as long as K is 2048: (26, 10240, 832) 12.8, 9.6; (17, 768, 3338) 3.6, 3.8.  Fewer tiles than half of the units
+// share K longer than 6144.  K below 1408: not the time (those would gain as much: (119, 512, 384) 6.6, 2.8, (59, 1152, 302) 6.4, 3.3), these are shapes by which
+// the tests reach the kernels behind and name them.
+bool w4_strips(int64_t M, int64_t K, int64_t N, int64_t block, int64_t units) {
+  if (K % 128 != 0 || (block != 64 && block % 128 != 0) || M > 512 || M * K > (int64_t(1) << 31))
+    return false;
+  if (M <= 16)
+    return block != 64 || K >= 512;
+  const int64_t groups = (M + 15) / 16, tiles = (N + 15) / 16, most = std::max<int64_t>(units / groups, 1), each = (tiles + most - 1) / most;
+  if (K < (block == 64 ? 2048 : 1408) || each > 3)
+    return false;
+  if (M <= 32)
+    return each <= 2;
+  return each == 3 ? K <= 2560 : each == 2 || 2 * groups * tiles < units ? K <= 6144 : K <= 12288;
+}
+
 // bias: f16 [N], added to the rounded product, or null (only with re-laid weights)
 int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const void *w_prepacked, const void *scale, const void *bias, void *y,
               int64_t M, int64_t K, int64_t N, int64_t block, void *workspace, int64_t workspace_bytes) {
@@ -1596,19 +1619,18 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
   if (w4_fast(a, w_prepacked, K, block)) {
     const int64_t cus = num_compute_units(st);
     void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias};
-    // Rows of activations are addressed by 32-bit offsets below.  Blocks of 64 take the strips where each of their four waves has
-    // a slice of 128 k; the kernel behind them, with slices of 64, is as fast below that.
-    const bool strips = M <= 16 && K % 128 == 0 && (block % 128 == 0 || (block == 64 && K >= 512)) && M * K <= (int64_t(1) << 31);
-    if (strips) {
-      // 16-column tiles over all of K (weights in strip order).  One workgroup per compute unit; two for more than three
+    // (rows of activations are addressed by 32-bit offsets below)
+    if (w4_strips(M, K, N, block, cus)) {
+      // 16-column tiles over all of K (weights in strip order).  One workgroup per compute unit; up to 16 rows two for more than three
       // tiles a unit, which a workgroup would take one after the other (K = 4096, M = 16: 768 tiles 9.0 against 10.6 us, 864 tiles
       // 12.3 against 11.9, 1024 tiles 12.9 against 12.3), and with up to four rows for more than one (M = 1: 320 tiles 5.6 against
-      // 5.2 us, 688 tiles 7.4 against 7.1, 1024 tiles 10.2 against 9.8).
+      // 5.2 us, 688 tiles 7.4 against 7.1, 1024 tiles 10.2 against 9.8); more rows' groups share the units ((22, 13056, 2880) 12.9 against 17.0).
       const void *in_strips = static_cast<const char *>(w_prepacked) + w4_fragment_bytes(K, N);
       void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias};
-      const int64_t tiles = (N + 15) / 16, most = M <= 4 || tiles > 3 * cus ? 2 * cus : cus;
+      const int64_t tiles = (N + 15) / 16, groups = (M + 15) / 16;
+      const int64_t most = groups > 1 ? std::max<int64_t>(cus / groups, 1) : M <= 4 || tiles > 3 * cus ? 2 * cus : cus;
       return launch(st, KernelName(block == 64 ? "mtrt_gemm_w4a16_strips16_b64" : "mtrt_gemm_w4a16_strips16"),
-                    uint32_t(std::min<int64_t>(tiles, most)), kBlock, stream, sargs);
+                    uint32_t(std::min<int64_t>(tiles, most) * groups), kBlock, stream, sargs);
     }
     if (M <= 32 && M * K <= (int64_t(1) << 31)) {
       // one workgroup per 32-column tile; between one and two tiles per compute unit, one workgroup per
@@ -1659,6 +1681,8 @@ int64_t mtrt_hip_gemm_w4a16_workspace(int64_t M, int64_t K, int64_t N, int64_t b
     return 0;
   DeviceState *st = device_state();
   if (!st)
+    return 0;
+  if (w4_strips(M, K, N, block, num_compute_units(st)))
     return 0;
   const W4Plan p = w4_plan(M, K, N, num_compute_units(st), true);
   return p.tile ? p.workspace() : 0;

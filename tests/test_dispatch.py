@@ -301,3 +301,23 @@ def test_rows_that_are_no_whole_slices_take_every_form(gpu, pkg, dtype, item):
             assert K * item >= 16 or not waves
             seen.add(waves)
     assert seen == ({0, 4, 8} if dtype == "F32" else {0, 4})
+
+
+def test_strips_of_more_than_16_rows_cover_the_output_and_need_no_workspace(gpu):
+    """Whole groups of 16 rows to a launch, at least one workgroup and at most one to a tile of columns each; on both sides of the rule's lines the
+    workspace asked for is what the launch takes."""
+    seen = set()
+    for M in (17, 32, 33, 100, 497, 512, 513):
+        for K in (1280, 1408, 2048, 2560, 2688, 6144, 6272, 12288, 12416):
+            for N in (1, 16, 17, 250, 500, 1000, 4000, 9000):
+                for block in (64, 128):
+                    name = gpu.w4a16(8, M, K, N, block)[0]
+                    grid, wants = gpu.sizes[-1][1], gpu.lib.mtrt_hip_gemm_w4a16_workspace(M, K, N, block)
+                    strips, groups, tiles = "strips" in name, (M + 15) // 16, (N + 15) // 16
+                    seen.add((strips, M > 32))
+                    if strips:
+                        assert M <= 512 and grid % groups == 0 and 1 <= grid // groups <= tiles and grid <= 256 and -(-tiles // (grid // groups)) <= 3 and wants == 0
+                        assert name.endswith("_b64") == (block == 64) and K >= (2048 if block == 64 else 1408)
+                    elif wants:
+                        assert gpu.launches[-1][2][0] > 1
+    assert seen == {(True, True), (True, False), (False, True), (False, False)}

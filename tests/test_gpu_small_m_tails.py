@@ -75,3 +75,17 @@ def test_w8a8_small_of_few_columns(pkg, M):
             assert pkg.last_kernel() == ("mtrt_gemm_w8a8_frag_rows32" if eight else "mtrt_gemm_w8a8_small16")
         acc = (a.double() @ w.double()).to(torch.int64).float()   # exact sums, one rounding to f32
         assert torch.equal(y, ((acc * sa[:, None]) * sw[None, :]).half()), (M, K, N)
+
+
+@pytest.mark.parametrize("block", [64, 128, 256])
+@pytest.mark.parametrize("M", [17, 20, 21, 24, 25, 32, 33, 63, 64, 65, 100, 256, 497, 512])
+def test_w4a16_strips_in_groups_of_rows(pkg, M, block):
+    """A last group of every form, one, two and three tiles to a workgroup, ragged last tiles, waves with every number of slices modulo four."""
+    import torch
+    units, groups = 256, (M + 15) // 16
+    for i, (K, tiles) in enumerate(((2048, 1), (2048, units // groups), (2560, units // groups + 1), (2304, 2 * (units // groups)), (2560, 3 * (units // groups)))):
+        N = 16 * tiles - (0, 7, 15, 0, 1)[i]
+        if N > 0:
+            _w4(torch, pkg, M, K, N, block, 10 * M + i)
+            if torch.cuda.get_device_properties(0).multi_processor_count == units and (M > 32 or i < 4):
+                assert pkg.last_kernel() == "mtrt_gemm_w4a16_strips16" + ("_b64" if block == 64 else ""), (K, N)
