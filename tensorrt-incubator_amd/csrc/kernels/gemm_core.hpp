@@ -142,9 +142,11 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
   __syncthreads();
   if (!active) return;
   int8_t* out = lds + slot * kOut;
-  const bool vec_ok = (N % 8 == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
+  // Rows of whole cache lines go past the caches; others share lines with their neighbours, whose pieces are to meet in L2 (int8, M = 3043,
+  // K = 768, N = 13616: 71.9 us past the caches, 51 by the general form below; N = 13632 49.3 past them).
+  const bool lines = (N % 64 == 0) && ((reinterpret_cast<uintptr_t>(y) & 15) == 0);
   // all rows of the workgroup's tile lie inside y (the rows of all SLOTS / NWN wave rows)
-  const bool rows_inside = vec_ok && m0 + (SLOTS / NWN) * (32 * IT) <= M;
+  const bool rows_inside = lines && m0 + (SLOTS / NWN) * (32 * IT) <= M;
   // one pass: 128 rows (row group ib) x HCP column tiles starting at column tile jt0 of the wave
   auto pass = [&](auto hcp, int ib, int jt0) {
     constexpr int HCP = decltype(hcp)::value;
@@ -174,7 +176,7 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
     }
     // each wave reads back only what it wrote itself: no workgroup barrier needed
     if (inside) {
-      // every row and column of the tile exists and whole vectors can be stored: no test per store, and the address
+      // every row and column of the tile exists and whole lines can be stored: no test per store, and the address
       // moves on by a constant (the general form below costs about ten branches and a 64-bit multiply per store)
       const int r0 = lane / CHUNKS, ch = lane % CHUNKS;
       uint16_t* dst = y + (m0 + wrow + r0) * N + (n0 + wn * WCOLS + jt0 * 32 + ch * 8);
@@ -187,7 +189,7 @@ __device__ __forceinline__ void write_tile(Acc (&acc)[IT][JT], Epilogue& epi, ui
       }
       return;
     }
-    // The last row or column tile, or rows that do not start on 16 bytes (N % 8 != 0).  Whole chunks go out as 16-byte stores at
+    // The last row or column tile, or rows that do not start on a cache line.  Whole chunks go out as 16-byte stores at
     // element alignment, ordinary ones, so that the pieces of a cache line meet in L2; one element at a time the launch was
     // bound by these stores (int8 M = 2792, K = 2816, N = 6020: 79 us, 42 for N = 6016).
     const int ch = lane % CHUNKS;

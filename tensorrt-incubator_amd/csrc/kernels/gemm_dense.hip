@@ -503,7 +503,7 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_de
   MTRT_DENSE_FRAG_KERNEL(XN, XT, 1, 1, 4, 2, t32x128)                                                                     \
   MTRT_DENSE_FRAG_KERNEL(XN, XT, 2, 1, 4, 2, t64x128)                                                                     \
   MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 1, 2, 2, t128x128)                                                                    \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 2, 2, 1, t128x256)                                                                    \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 2, 2, 2, t128x256)                                                                    \
   MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 3, 2, 1, t128x384)                                                                    \
   MTRT_DENSE_FRAG_KERNEL(XN, XT, 8, 2, 2, 1, t256x256)                                                                    \
   extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_dense_frag_##XN##_t256x384(                              \

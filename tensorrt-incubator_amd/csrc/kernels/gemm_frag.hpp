@@ -307,7 +307,7 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
   __syncthreads();
   // (a tile whose accumulators fill half of the register file is never split: the partial sums would not fit beside them)
   if constexpr (IT * JT < 16) {
-    if (part.splits > 1 && !meet<typename Traits::Scalar, (IT * JT < 2 || IT * JT >= 12 ? 1 : 2)>(acc, part, lds, slot)) return;
+    if (part.splits > 1 && !meet<typename Traits::Scalar, (IT * JT < 2 || IT * JT >= 8 ? 1 : 2)>(acc, part, lds, slot)) return;
   }
   write_tile<JT, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, true);
 }

@@ -123,11 +123,15 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
 // mtrt_gemm_w8a8_frag_t<rows>x<columns> (a [M,K] i8, w_frag, a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, Split,
 // a_step, bias) ; K % 128 == 0, a and w_frag 16-byte aligned, a below 4 GiB; a_step 1, or 0 for a
 // single a_scale; bias f16 [N] or null.
-// grid = 8 * ceil(tiles * splits / 8), block = 256.  Tiles of 32 x 128, 64 x 128 and 128 x 128 (two
-// workgroups per compute unit), 128 x 256, 128 x 384 and 256 x 256 (one; the last never split).  Which tile and how many splits: the host's
+// grid = 8 * ceil(tiles * splits / 8), block = 256.  Tiles of 32 x 128, 64 x 128, 128 x 128 and 128 x 256 (two
+// workgroups per compute unit), 128 x 384 and 256 x 256 (one; the last never split).  Which tile and how many splits: the host's
 // estimate of the launch (frag_plan in clusters.cpp).  Measured, the one 256-row tile loop that these replaced -> now,
 // us: (M, K, N) = (256, 4096, 4096) 21.8 -> 10.4, (398, 11520, 1856) 51.8 -> 19.3, (1024, 2048, 2048) 14.7 -> 8.8,
 // (200, 12288, 512) 52.7 -> 10.6, (999, 4096, 11008) 46.5 -> 44.
+// t128x256: 239 registers, so that one workgroup's first loads and its epilogue (6 us of a tile) lie under the other's loop, where a unit has more
+// than one; what a meeting fetches at a time is one 32 x 32 tile, two would not fit.  One and two to a unit, us: (3043, 768, 13632) 59.6, 42.2;
+// (4011, 256, 12672) 46.5, 37.1; (2048, 4096, 11008) 91.1, 81.7; (999, 4096, 11008) 54.4, 48.3; where a unit has one tile (985, 1152, 4352) 12.0,
+// 11.6; (1296, 4992, 4352) 32.9, 32.1; with K in two parts (2332, 10368, 1024) 38.4, 37.7.
 #define MTRT_W8_FRAG_KERNEL(NAME, IT, JT, D, WG)                                                                          \
   extern "C" __global__ void __launch_bounds__(256, WG) NAME(                                                             \
       const int8_t* __restrict__ a, const int8_t* __restrict__ w_frag, const float* __restrict__ a_scale,                 \
@@ -143,7 +147,7 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t32x128, 1, 1, 4, 2)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t64x128, 2, 1, 4, 2)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x128, 4, 1, 2, 2)
-MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x256, 4, 2, 2, 1)
+MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x256, 4, 2, 2, 2)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t128x384, 4, 3, 2, 1)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t256x256, 8, 2, 2, 1)
 

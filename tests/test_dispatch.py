@@ -321,3 +321,11 @@ def test_strips_of_more_than_16_rows_cover_the_output_and_need_no_workspace(gpu)
                     elif wants:
                         assert gpu.launches[-1][2][0] > 1
     assert seen == {(True, True), (True, False), (False, True), (False, False)}
+
+
+@pytest.mark.parametrize("family,shape,kernel", [
+    ("w8a8", (3043, 768, 13632), "t128x256"), ("w8a8", (2817, 768, 5376), "t128x256"), ("w8a8", (2817, 512, 5376), "t256x256"), ("w8a8", (999, 4096, 11008), "t128x384"),
+    ("dense", (2817, 384, 5391), "t128x256"), ("dense", (2817, 256, 5376), "t256x256"), ("dense", (2981, 1472, 8768), "t256x256")])
+def test_pairs_of_tiles_from_five_slices_on(gpu, pkg, family, shape, kernel):
+    name = gpu.w8a8(8, *shape)[0] if family == "w8a8" else gpu.linear(8, *shape, pkg.F16)[0]
+    assert name == {"w8a8": "mtrt_gemm_w8a8_frag_", "dense": "mtrt_gemm_dense_frag_f16_"}[family] + kernel

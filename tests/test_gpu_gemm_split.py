@@ -294,3 +294,24 @@ def test_every_dense_tile(pkg, shape, tile, split, dname):
     _is(pkg, "mtrt_gemm_dense_frag_%s_%s" % ({"float16": "f16", "bfloat16": "bf16"}[dname], tile))
     ref, mass = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
     assert bool(((y.double() - ref).abs() <= u * ref.abs() + (1 + u) * (K + 2) * 2.0 ** -24 * mass + 2.0 ** -24).all())
+
+
+# More than one 128 x 256 tile to a compute unit, which two workgroups share; rows that are whole cache lines, whole vectors and neither.
+@pytest.mark.parametrize("N", [5376, 5384, 5391])
+def test_pairs_of_tiles_on_a_unit(pkg, N):
+    import importlib
+
+    import torch
+    tp = importlib.import_module(pkg.__name__ + ".tp")
+    M = 2817
+    a, w, a_s, w_s = _inputs(N, M, 768, N)
+    y = pkg.gemm_w8a8_fragments(a, pkg.gemm_w8a8_prepack_fragments(w), a_s, w_s, N)
+    _is(pkg, "mtrt_gemm_w8a8_frag_t128x256")
+    assert torch.equal(y, _expect(a, w, a_s, w_s))
+    x, w, b = (torch.randn(s, device="cuda").half() for s in ((M, 384), (N, 384), (N,)))
+    lin = tp.Linear(384, N, dtype=tp.float16)
+    lin.weight, lin.bias = tp.Tensor(w), tp.Tensor(b)
+    y = lin(tp.Tensor(x)).torch()
+    _is(pkg, "mtrt_gemm_dense_frag_f16_t128x256")
+    ref, mass, u = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs(), 2.0 ** -11
+    assert bool(((y.double() - ref).abs() <= u * ref.abs() + (1 + u) * (384 + 2) * 2.0 ** -24 * mass + 2.0 ** -24).all())
