@@ -103,8 +103,11 @@ __device__ __forceinline__ void load_through(f32x4& dst, const f32x4* src) {
 }
 
 // Adds up the partial tiles of a split tile; true for the workgroup that is to run the epilogue.  Four waves hold the tile;
-// further waves of the workgroup (active = false) only take part in the barriers.
-template <class Scalar, int G, int IT, int JT, class Acc>
+// further waves of the workgroup (active = false) only take part in the barriers.  SUMS: tiles times parts that a trip to memory brings (what the
+// registers beside the accumulators hold), two parts of as many tiles as that is rather than four of half as many: parts past the last are fetched
+// all the same, and most splits are into two or three.  us, four parts and two at a time, W4A16 (136, 4224, 3904) 15.2, 14.7; (282, 3840, 2880) 15.2, 14.7;
+// (106, 10496, 6784) 25.7, 25.2; f16 (1493, 8448, 1152) 36.1, 35.4; more parts the same.
+template <class Scalar, int SUMS, int IT, int JT, class Acc>
 __device__ __forceinline__ bool meet(Acc (&acc)[IT][JT], const Part& part, int8_t* lds, int wave, bool active = true) {
   constexpr int kTiles = IT * JT, kPer = 4 * kTiles;   // 32 x 32 tiles of the wave; 16-byte pieces per lane
   const int lane = threadIdx.x & 63;
@@ -130,8 +133,9 @@ __device__ __forceinline__ bool meet(Acc (&acc)[IT][JT], const Part& part, int8_
   if (*seen != part.splits - 1) return false;
   if (threadIdx.x == 0) __hip_atomic_store(part.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (!active) return true;
-  // A round trip to memory for each group of G tiles, KB splits at a time (what the registers beside the accumulators hold).
-  constexpr int KB = 4;
+  // a round trip to memory for each group of G tiles, KB splits at a time
+  constexpr int KB = SUMS / 2 <= kTiles ? 2 : 4, G = SUMS / KB;
+  static_assert(kTiles % G == 0, "whole groups of tiles");
   const f32x4* all = part.partial + uint64_t(wave) * (kPer * 64) + lane;
 #pragma unroll
   for (int g = 0; g < kTiles; g += G) {
@@ -307,7 +311,7 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
   __syncthreads();
   // (a tile whose accumulators fill half of the register file is never split: the partial sums would not fit beside them)
   if constexpr (IT * JT < 16) {
-    if (part.splits > 1 && !meet<typename Traits::Scalar, (IT * JT < 2 || IT * JT >= 8 ? 1 : 2)>(acc, part, lds, slot)) return;
+    if (part.splits > 1 && !meet<typename Traits::Scalar, (IT * JT < 2 || IT * JT >= 8 ? 4 : 8)>(acc, part, lds, slot)) return;
   }
   write_tile<JT, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, true);
 }

@@ -468,7 +468,7 @@ __device__ __forceinline__ void run_weight_regs(const int8_t* __restrict__ a, in
   if constexpr (IT * JT < 16) {                        // (larger tiles are never split: see gemm_frag::run)
     if (part.splits > 1) {
       __syncthreads();
-      if (!gemm_frag::meet<float, 1>(acc, part, lds, slot, KH == 0)) return;
+      if (!gemm_frag::meet<float, 4>(acc, part, lds, slot, KH == 0)) return;
     }
   }
   write_tile<JT, NWN, S::kSlots>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, KH == 0);
@@ -655,7 +655,7 @@ __device__ __forceinline__ void run_tiles(const int8_t* __restrict__ a, int64_t 
     for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(0)" ::"v"(raw[q][j]), "v"(sc[q][j]) : "memory");
   __syncthreads();
   if constexpr (IT * JT < 16) {
-    if (part.splits > 1 && !gemm_frag::meet<float, (IT * JT < 2 || IT * JT >= 12 ? 1 : 2)>(acc, part, lds, slot)) return;
+    if (part.splits > 1 && !gemm_frag::meet<float, (IT * JT < 2 || IT * JT >= 12 ? 4 : 8)>(acc, part, lds, slot)) return;
   }
   write_tile<JT, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, true);
 }
@@ -879,7 +879,7 @@ __device__ __forceinline__ void run_sets(const int8_t* __restrict__ a, int64_t r
   }
   if (part.splits > 1) {
     __syncthreads();
-    if (!gemm_frag::meet<float, 1>(acc, part, lds, slot, set == 0)) return;
+    if (!gemm_frag::meet<float, 4>(acc, part, lds, slot, set == 0)) return;
   }
   write_tile<1, 4, 4>(acc, epi, y, M, N, part.m0, part.n0, lds, slot, set == 0);
 }
