@@ -1176,7 +1176,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny(
   skinny_tiles<4>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 
-// ---- M <= 16: one strip of columns per compute unit --------------------------------------------------
+// ---- M <= 16, and groups of 16 rows by few columns: one strip of columns per compute unit ----------------
 // At this size a compute unit has its share of the weights to dequantise plus ALL of the activations to take in (16 rows x
 // K).  One workgroup per 32-column tile leaves 344 workgroups on 256 compute units at N = 11008, and the 88 units that
 // hold two set the time.  Here the grid is one or two workgroups per compute unit, each owning a contiguous strip of
