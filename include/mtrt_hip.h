@@ -424,7 +424,7 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_gemm_w8a8_fragments_ws(mtrt_stream_t stream,
  * The matrix-core kernels read the weights from a one-time re-layout (`w_prepacked`, made by the
  * prepack call, mtrt_hip_gemm_w4a16_prepacked_bytes(K, N) bytes, needs K % 64 == 0; it holds the weights in
  * the fragment order of the 32-column kernels and, when K % 128 == 0, once more in the strip order of the
- * M <= 16 kernel, so it is about K * N bytes); they are
+ * kernel of 16-row groups, so it is about K * N bytes); they are
  * used when w_prepacked is given and K % 64 == 0, block % 64 == 0, K % block == 0.  Otherwise a
  * matrix-core kernel that dequantises the original nibbles tile by tile reads w_kn_packed directly
  * (any block that divides K, any K and N; several times slower than the re-laid form).  Either weight

@@ -1583,14 +1583,17 @@ bool w4_fast(const void *a, const void *w_prepacked, int64_t K, int64_t block) {
 
 // Whether the strip kernel (16 rows by 16 columns over all of K, four waves) takes a product.  Up to 16 rows: blocks of 64 where each wave
 // has a slice of 128 k; the kernel behind, with slices of 64, is as fast below that.
-// 17 to 512 rows in groups of 16, where the 32-row kernel and the tiles leave most of the chip idle: by how many of its 16 columns' tiles, side by side,
-// a workgroup has where there is one to a compute unit.  Each slice of 512 k takes 0.34, 0.53 and 0.75 us so, 0.57 in the 32-row kernel,
-// and the walk down K gets long against tiles that share it.  us, (M, K, N), others and strips: one a unit (27, 7040, 384) 10.6, 6.2; (45, 5376, 320)
-// 9.0, 5.8; (146, 5760, 256) 9.8, 6.2; (37, 9216, 1247) 11.8, 8.9; two (22, 13056, 2880) 16.3, 12.9; (190, 1408, 640) 6.9, 4.1; (211, 6784, 384) 11.2, 10.1,
-// (96, 12032, 1088) 13.7, 15.4; three (52, 2432, 2496) 8.1, 6.2; (386, 1920, 448) 8.3, 6.9; (54, 5120, 4032) 12.2, 12.2; (29, 5120, 5056) 10.2, 9.2; four and
-// more (186, 4224, 1664) 11.6, 15.7; (418, 2304, 448) 8.9, 11.1.  Over 80 products of the rule's ranges 1.32 times as fast in the geometric mean.  Blocks of 64 as long as K is 2048: (26, 10240, 832) 12.8, 9.6; (17, 768, 3338) 3.6, 3.8.  Fewer tiles than half of the units
-// share K longer than 6144.  K below 1408: not the time (those would gain as much: (119, 512, 384) 6.6, 2.8, (59, 1152, 302) 6.4, 3.3), these are shapes by which
-// the tests reach the kernels behind and name them.
+// 17 to 512 rows in groups of 16, where the 32-row kernel and the tiles leave most of the chip idle.  The line is the number of 16-column tiles that a
+// workgroup has side by side when there is one to a compute unit (`each`): 512 of K take 0.34, 0.53 and 0.75 us so, 0.57 in the 32-row kernel, and
+// a long walk down K loses against tiles that share it.  us, (M, K, N), the others and this:
+//   one tile (27, 7040, 384) 10.6, 6.2; (45, 5376, 320) 9.0, 5.8; (146, 5760, 256) 9.8, 6.2; (37, 9216, 1247) 11.8, 8.9
+//   two (22, 13056, 2880) 16.3, 12.9; (190, 1408, 640) 6.9, 4.1; (211, 6784, 384) 11.2, 10.1; (96, 12032, 1088) 13.7, 15.4
+//   three (52, 2432, 2496) 8.1, 6.2; (386, 1920, 448) 8.3, 6.9; (54, 5120, 4032) 12.2, 12.2; (29, 5120, 5056) 10.2, 9.2
+//   four and more (186, 4224, 1664) 11.6, 15.7; (418, 2304, 448) 8.9, 11.1
+//   blocks of 64 (26, 10240, 832) 12.8, 9.6; (17, 768, 3338) 3.6, 3.8
+// Over 80 products of these ranges 1.32 times as fast in the geometric mean.  With fewer tiles than half of the units, parts of a K longer than 6144
+// fill the chip.  K below 1408 is not a matter of time (those would gain as much: (119, 512, 384) 6.6, 2.8, (59, 1152, 302) 6.4, 3.3): these are the
+// shapes by which the tests reach the kernels behind and name them.
 bool w4_strips(int64_t M, int64_t K, int64_t N, int64_t block, int64_t units) {
   if (K % 128 != 0 || (block != 64 && block % 128 != 0) || M > 512 || M * K > (int64_t(1) << 31))
     return false;
