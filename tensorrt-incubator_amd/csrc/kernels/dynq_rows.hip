@@ -14,7 +14,10 @@
 // up to 64 * NV vectors per row) or, for longer rows, the four waves of a workgroup share one and meet in LDS;
 // the row maximum is a cross-lane exchange, the quotient the short exact division of qdq.hip (ExactDivisor), so
 // codes and scales are bit-identical to the two launches.  Loads are unconditional (lanes past the end of the row
-// repeat its last vector, which cannot change a maximum) and only the stores are predicated.
+// repeat its last vector, which cannot change a maximum) and only the stores are predicated.  The waves of a unit load, then quantize, all at
+// the same time, so the instructions (about twelve an element) are not hidden: vectors that lie past the row's end for a whole wave are left out
+// of the quantization.  us, with them and without: f16 [2140, 10624] 14.9, 13.9 (f8 16.7, 15.0); [300, 9216] 4.3, 4.0; [8192, 2560] 14.1, 13.1; bf16
+// [1000, 11008] to f8 10.1, 9.1; rows that fill the form's vectors ([2048, 8192], [2000, 14336]) the same.
 #include "common.hpp"
 
 namespace dynq_rows_cluster {
@@ -73,6 +76,8 @@ __device__ __forceinline__ void body(const typename X::storage* __restrict__ x, 
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
     const uint32_t v = first + uint32_t(i) * kLanes;
+    // what a wave has past the row's end is not quantized (the row fills more than half of the vectors, so the first ones need no test)
+    if (NV >= 4 && i >= NV / 2 && uint32_t(WAVES == 1 ? 0 : wave * kWave) + uint32_t(i) * kLanes >= nvec) break;
     float f[G];
     FG::unpack(xin[i], f);
     quantize_group<Q>(dv, f, flags);

@@ -144,3 +144,20 @@ def test_argument_checks(pkg):
     assert call(st, x.data_ptr(), pkg.F32, q.data_ptr(), pkg.F8E4M3FN, 8, 8, 448.0, None, s.data_ptr(), 6) == 1
     assert call(st, x.data_ptr(), pkg.F32, q.data_ptr(), pkg.I8, 0, 8, 127.0, None, s.data_ptr(), 0) == 0
     assert call(st, x.data_ptr(), pkg.F32, q.data_ptr(), pkg.I8, 8, 0, 127.0, None, s.data_ptr(), 0) == 0
+
+
+@pytest.mark.parametrize("qname", ["i8", "f8"])
+@pytest.mark.parametrize("xname", ["f32", "f16", "bf16"])
+def test_rows_that_end_inside_and_between_a_waves_vectors(pkg, orc, xname, qname):
+    """The last vectors of a row in every wave of the forms of four vectors and more, and on both sides of each wave's share."""
+    g = rng(sum(map(ord, qname + xname)))
+    grp = 4 if xname == "f32" else 8
+    k = "mtrt_dynq_rows_%s_%s_" % (xname, qname)
+    orc.set_threads(16)
+    lengths = [(3, 512 + e, "g4v4") for e in (1, 64, 65, 192, 193, 256, 257, 448, 449)] + [(2, 1024 + e, "g4v8") for e in (64, 65, 255, 256, 321, 832, 833, 1023)]
+    lengths += [(5, n, "v4") for n in (129, 192, 193, 255)] if xname == "f32" else []
+    for rows, nvec, kernel in lengths:
+        x = (g.standard_normal((rows, nvec * grp)) * g.uniform(0.1, 30.0, (rows, 1))).astype(np.float32)
+        x[0, -1] = 1000.0
+        _check(pkg, orc, x, xname, qname, k + kernel)
+    orc.set_threads(1)
