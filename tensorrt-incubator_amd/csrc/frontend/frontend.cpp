@@ -115,18 +115,6 @@ private:
   bool here;
 };
 
-// The two f32 numbers of a tensor's amax and scale, side by side in one storage (a second allocation is 0.28 us).
-struct AmaxAndScale {
-  at::Tensor amax, scale;
-  explicit AmaxAndScale(const Place &place) {
-    amax = place.empty({2}, at::ScalarType::Float);
-    scale = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(amax.storage()), c10::DispatchKeySet(c10::DispatchKey::CUDA), amax.dtype());
-    scale.unsafeGetTensorImpl()->set_storage_offset(1);
-    scale.unsafeGetTensorImpl()->set_sizes_contiguous({});
-    amax.unsafeGetTensorImpl()->set_sizes_contiguous({});
-  }
-};
-
 bool check(int32_t status) {
   if (status == MTRT_OK)
     return true;
@@ -246,8 +234,8 @@ PyObject *f_amax(PyObject *, PyObject *const *a, Py_ssize_t n) {
   if (!float_type(*x, &dt) || !number(a[1], &qmax))
     return nullptr;
   const Place place(*x);
-  const AmaxAndScale made(place);
-  const at::Tensor &amax = made.amax, &scale = made.scale;
+  // each its own storage: callers resize, save and free one without the other
+  const at::Tensor amax = place.empty({}, at::ScalarType::Float), scale = place.empty({}, at::ScalarType::Float);
   const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_amax(s, x->data_ptr(), dt, x->numel(), qmax, static_cast<float *>(amax.data_ptr()), static_cast<float *>(scale.data_ptr()));
@@ -413,8 +401,7 @@ PyObject *f_dynamic_quantize_dequantize(PyObject *, PyObject *const *a, Py_ssize
   if (back < 0 || !integer32(a[1], &q_dtype) || !number(a[2], &qmax) || !integer32(a[3], &flags) || !float_type(*x, &dt))
     return nullptr;
   const Place place(*x);
-  const AmaxAndScale made(place);
-  const at::Tensor &amax = made.amax, &scale = made.scale;
+  const at::Tensor amax = place.empty({}, at::ScalarType::Float), scale = place.empty({}, at::ScalarType::Float);
   const at::Tensor q = place.codes(q_dtype, x->numel());
   at::Tensor y;
   if (back)

@@ -108,8 +108,8 @@ def test_in_place_updates_of_a_scale_are_noticed(tp):
 @pytest.mark.gpu
 @pytest.mark.parametrize("call", ["amax", "dynamic"])
 def test_amax_and_scale_are_tensors_of_their_own(pkg, call):
-    """They lie in one allocation: each is a dense f32 scalar, in-place work on one leaves the other, either outlives the other, and
-    both serve as the scale of another call; so under inference mode and on a stream that is not the default one."""
+    """Each is a dense f32 scalar, in-place work on one leaves the other, either outlives the other, and both serve as the scale of
+    another call; so under inference mode and on a stream that is not the default one."""
     import torch
     x = torch.from_numpy(rng(5).standard_normal((7, 96), dtype=np.float32)).cuda()
 
@@ -135,6 +135,27 @@ def test_amax_and_scale_are_tensors_of_their_own(pkg, call):
             others = [run() for _ in range(64)]
             assert float(kept) == float(np.float32(want) / np.float32(127.0)) and all(float(a) == want for a, _ in others)
             assert int(codes.abs().max()) == 127
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("call", ["amax", "dynamic"])
+def test_amax_and_scale_have_storages_of_their_own(pkg, call):
+    """A storage of one number each, where torch's allocator starts one: resized, saved or handed on by address without the other."""
+    import io
+
+    import torch
+    x = torch.from_numpy(rng(6).standard_normal((7, 96), dtype=np.float32)).cuda()
+    amax, scale = pkg.amax(x, 127.0) if call == "amax" else pkg.dynamic_quantize_dequantize(x, pkg.I8, 127.0)[2:]
+    value = float(np.float32(float(x.abs().max())) / np.float32(127.0))
+    for t in (amax, scale):
+        assert t.untyped_storage().nbytes() == 4 and t.storage_offset() == 0 and t.data_ptr() % 256 == 0
+    assert amax.untyped_storage().data_ptr() != scale.untyped_storage().data_ptr()
+    saved = io.BytesIO()
+    torch.save(scale, saved)
+    saved.seek(0)
+    assert torch.load(saved, weights_only=True).untyped_storage().nbytes() == 4
+    amax.untyped_storage().resize_(0)
+    assert float(scale) == value
 
 
 @pytest.mark.gpu
