@@ -107,6 +107,8 @@ __device__ __forceinline__ void opaque(u32x4& t) { __asm__ volatile("" : "+v"(t)
 // forms gain from; where the waves of aligned short rows fill the chip, LDS takes instructions off the vector unit.  us, LDS and vector unit:
 // LayerNorm f16 [8, 4096] 4.3, 3.9, f32 [22, 1984] 3.9, 3.5, f32 [77101, 204] 26.3, 24.9; softmax f32 [179, 1405] 3.5, 3.1, bf16 [76538, 411] 27.8,
 // 25.8; the other way LayerNorm bf16 [20000, 1024] 15.8, 16.2, [26061, 512] 11.6, 11.9, softmax bf16 [5120, 1024] 5.1, 5.7, f32 [2560, 816] 4.5, 5.1.
+// Whole f32 rows of 2048 take 5.0 us where [1280, 2048] lies in the caches from the call before, and 4.7 by LDS; with every call's tensors new it is
+// 5.8 and 5.9, [300, 2048] 3.5 and 3.7, so they stay on the vector unit.
 template <bool LDS, typename Op>
 __device__ __forceinline__ float row_reduce(float v, Op op) { return LDS ? wave_reduce_lds(v, op) : wave_reduce(v, op); }
 
@@ -114,7 +116,9 @@ __device__ __forceinline__ float row_reduce(float v, Op op) { return LDS ? wave_
 // again in each of the three passes: for 16-bit types that halves the live registers compared
 // with keeping f32 values (a widening is one shift or mask per element), and the higher
 // occupancy it buys is worth more to this memory-bound kernel than the extra VALU work.
-template <typename X, int NV, bool FULL>
+// RESIDENT: the form held to 64 registers.  In f32 the exchanges need one more, which lay in private memory: by LDS there (us, f32 [5500,
+// 2048] 17.3, 16.5; [7000, 2048] 21.1, 20.3; [7000, 1100] 13.8, 13.1; [8192, 2048] 24.0, 23.5).
+template <typename X, int NV, bool FULL, bool RESIDENT>
 __device__ __forceinline__ void layernorm_row(const typename X::storage* __restrict__ x,
                                               const typename X::storage* __restrict__ gamma,
                                               const typename X::storage* __restrict__ beta,
@@ -130,7 +134,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
     t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
 
-  constexpr bool kLds = NV == 2 || NV == 4 || (NV == 1 && E == 8);
+  constexpr bool kLds = NV == 2 || NV == 4 || (NV == 1 && E == 8) || (RESIDENT && E == 4);
   const float fd = float(d);
   float sum = 0.0f;
 #pragma unroll
@@ -176,7 +180,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
   }
 }
 
-template <typename X, int NV>
+template <typename X, int NV, bool RESIDENT = false>
 __device__ __forceinline__ void layernorm_rows(const typename X::storage* __restrict__ x,
                                                const typename X::storage* __restrict__ gamma,
                                                const typename X::storage* __restrict__ beta,
@@ -185,9 +189,9 @@ __device__ __forceinline__ void layernorm_rows(const typename X::storage* __rest
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;                           // whole wave leaves together
   if (d == int64_t(Vec<X>::kElems) * kWave * NV)
-    layernorm_row<X, NV, true>(x, gamma, beta, y, row, d, eps);
+    layernorm_row<X, NV, true, RESIDENT>(x, gamma, beta, y, row, d, eps);
   else
-    layernorm_row<X, NV, false>(x, gamma, beta, y, row, d, eps);
+    layernorm_row<X, NV, false, RESIDENT>(x, gamma, beta, y, row, d, eps);
 }
 
 template <typename X, int NV, bool FULL>
@@ -604,7 +608,7 @@ using namespace norm_cluster;
   extern "C" __global__ void __launch_bounds__(kNormThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))        \
   mtrt_layernorm_##XN##_v8r(const XT::storage* x, const XT::storage* gamma, const XT::storage* beta,           \
                             XT::storage* y, int64_t rows, int64_t d, float eps) {                              \
-    layernorm_rows<XT, 8>(x, gamma, beta, y, rows, d, eps);                                                    \
+    layernorm_rows<XT, 8, true>(x, gamma, beta, y, rows, d, eps);                                                    \
   }                                                                                                            \
   extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_layernorm_##XN##_any(                        \
       const XT::storage* x, const XT::storage* gamma, const XT::storage* beta, XT::storage* y, int64_t rows,  \

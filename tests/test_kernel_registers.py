@@ -24,3 +24,12 @@ def metadata(pkg, tmp_path):
 def test_one_launch_dynamic_quantization_stays_in_registers(pkg, tmp_path):
     private = dict(re.findall(r"\.name:\s+(mtrt_dynqdq_\S+)\n\s+\.private_segment_fixed_size:\s+(\d+)", metadata(pkg, tmp_path)))
     assert len(private) == 10 and {name: size for name, size in private.items() if size != "0"} == {}
+
+
+def test_the_resident_layernorm_and_the_tiles_spill_nothing(pkg, tmp_path):
+    """The eight-vector LayerNorm held to 64 registers: none of an f32 row's in private memory (one 8-byte slot: [5500, 2048] 16.5 -> 17.3 us); bf16 has had some
+    (32 bytes) and does not pay.  The GEMM tiles' loops likewise: only the wide W8A8 tile with a bias has a few bytes."""
+    private = dict(re.findall(r"\.name:\s+(mtrt_\S+)\n\s+\.private_segment_fixed_size:\s+(\d+)", metadata(pkg, tmp_path)))
+    names = [n for n in private if re.match(r"mtrt_layernorm_\S+_v8r$|mtrt_gemm_(w4a16|w8a8_frag|dense_frag_\S+)_t\d|mtrt_gemm_w4a16_strips", n)]
+    assert len(names) > 35
+    assert {n: int(private[n]) for n in names if int(private[n]) > {"mtrt_layernorm_bf16_v8r": 32, "mtrt_gemm_w8a8_frag_t256x384_linear": 44}.get(n, 0)} == {}
