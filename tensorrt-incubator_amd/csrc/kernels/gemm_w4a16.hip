@@ -1190,10 +1190,11 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny(
 // whole 256-byte row segments by direct-to-LDS loads, 16-byte chunks XOR-swizzled by the row so that the fragment
 // reads are conflict-free) and never touches another wave's ring: no barriers until the partial tiles are added
 // through LDS at the end.
-// G: groups of four activation rows (M <= 4 G); SC: scale rows per slice of 128 k (2: blocks of 64).
+// G: groups of four activation rows (M <= 4 G); SC: scale rows per slice of 128 k (2: blocks of 64); ONCE: nobody else reads these weights, so that
+// they pass the caches by.
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-template <int WAVES, int JT, int G, int SC>
+template <int WAVES, int JT, int G, int SC, bool ONCE>
 __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws,
                                              const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
                                              int64_t K, int64_t N, int64_t block, uint32_t tile0, const uint16_t* __restrict__ bias, int8_t* lds) {
@@ -1249,7 +1250,10 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
     auto fetch = [&](auto stage, Slice& dst) {
       // opaque register loads, waits placed by hand (see `skinny`); what comes from memory is asked for first
 #pragma unroll
-      for (int j = 0; j < JT; ++j) __asm__ volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
+      for (int j = 0; j < JT; ++j) {
+        if constexpr (ONCE) __asm__ volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
+        else __asm__ volatile("global_load_dwordx4 %0, %1, %2" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
+      }
 #pragma unroll
       for (int j = 0; j < JT; ++j)
 #pragma unroll
@@ -1350,10 +1354,12 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
   __syncthreads();                                     // the next chunk of this workgroup reuses the LDS
 }
 
-// (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M, K % 128 == 0, N, block % 128 == 0, or 64 for
-// _b64) ; M * K <= 2^31.  More than 16 rows go in ceil(M / 16) groups, a whole number of which the grid is: each group's workgroups follow one
-// another and the last group may have fewer rows.  A group takes its own activations and all of the weights, which the caches hold by then: what a workgroup
-// moves in is the four waves' 4 KiB of activations and 1 KiB of weights a tile and slice, whatever the rows.
+// (a [M,K] f16, strip-order weights, scale [K/block, N] f16, y [M,N] f16, M, K, N, block, bias) ; K % 128 == 0, block % 128 == 0, or 64 for
+// _b64, M * K <= 2^31.  More than 16 rows go in ceil(M / 16) groups, a whole number of which the grid is: each group's workgroups follow one
+// another and the last group may have fewer rows.  A group takes its own activations and all of the weights: what a workgroup moves in is the four waves'
+// 4 KiB of activations and 1 KiB of weights a tile and slice, whatever the rows.  The groups run side by side and ask for the same weights at about
+// the same time, so those go through the caches there.  us, past them and through them, (M, K, N): (246, 7680, 103) 8.6, 6.0; (163, 9088, 229) 9.2, 7.2;
+// (54, 11008, 493) 9.7, 7.7; (192, 4864, 696) 10.5, 8.6; over 420 products of 17 to 512 rows 0.7 % longer at worst, 2 % shorter in the geometric mean.
 // grid = one or two workgroups per compute unit, at most ceil(N / 16), block = 256: workgroup g owns tiles / grid consecutive
 // 16-column tiles (the first tiles % grid workgroups one more), three at a time.
 // What its time is, from timestamps in a copy of the kernel, (16, 4096, 11008): four waves, one per SIMD, each with eight of the 32
@@ -1369,7 +1375,7 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
 // kernel above: (2, 6656, 960) 9.4 and 5.0, (16, 4096, 11008) 10.1 and 9.2, (13, 1152, 14464) 6.3 and 5.5.  Eight waves (two per
 // SIMD) are no faster: 10.4 us at (16, 4096, 11008).
 constexpr int kStripWaves = 4;
-template <int G, int SC>
+template <int G, int SC, bool ONCE>
 __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
                                        uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block,
                                        const uint16_t* __restrict__ bias, uint32_t b, uint32_t grid, int8_t* lds) {
@@ -1380,9 +1386,9 @@ __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uin
   const uint32_t t0 = b * per + (b < rem ? b : rem), t1 = t0 + per + (b < rem ? 1 : 0);
   for (uint32_t t = t0; t < t1; t += 3) {
     const uint32_t left = t1 - t;
-    if (left >= 3) strips_chunk<kStripWaves, 3, G, SC>(a, ws, scale, y, M, K, N, block, t, bias, lds);
-    else if (left == 2) strips_chunk<kStripWaves, 2, G, SC>(a, ws, scale, y, M, K, N, block, t, bias, lds);
-    else strips_chunk<kStripWaves, 1, G, SC>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    if (left >= 3) strips_chunk<kStripWaves, 3, G, SC, ONCE>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else if (left == 2) strips_chunk<kStripWaves, 2, G, SC, ONCE>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else strips_chunk<kStripWaves, 1, G, SC, ONCE>(a, ws, scale, y, M, K, N, block, t, bias, lds);
   }
 }
 #define MTRT_W4_STRIPS(NAME, SC)                                                                                          \
@@ -1397,11 +1403,14 @@ __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uin
       b %= grid;                                                                                                          \
       a += uint64_t(row0) * K;                                                                                            \
       y += uint64_t(row0) * N;                                                                                            \
-      M = M - row0 < 16 ? M - row0 : 16;                                                                                  \
+      strips<4, SC, false>(a, ws, scale, y, M - row0 < 16 ? M - row0 : 16, K, N, block, bias, b, grid, lds);              \
+    } else if (M <= 4) {                                                                                                  \
+      strips<1, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                           \
+    } else if (M <= 8) {                                                                                                  \
+      strips<2, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                           \
+    } else {                                                                                                              \
+      strips<4, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                           \
     }                                                                                                                     \
-    if (M <= 4) strips<1, SC>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                       \
-    else if (M <= 8) strips<2, SC>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                  \
-    else strips<4, SC>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                              \
   }
 MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16, 1)
 MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16_b64, 2)
