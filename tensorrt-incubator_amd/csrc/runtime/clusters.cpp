@@ -87,8 +87,11 @@ constexpr double kW4Mid256RoundPerSmallRound = 1.9;
 // launches of 621 log-uniform shapes, M 33 ... 4096, K 256 ... 14336, N 64 ... 16384, 1 to 12 splits.
 // That is a full chip's law.  However few tiles there are, one of them takes least + least_slice * s, which a launch of few
 // large tiles runs into (fitted to the launches of at most half as many unsplit tiles as units of 380 shapes of the same range).
-// With it the choice is 1.6 % longer than the fastest one on average; without, M, K, N, us: (92, 640, 6336) t128x128 7.2, t32x128 5.2; (1001, 896, 640) 8.3,
-// 6.2; (805, 1536, 768) 11.3, 8.4; (606, 1280, 384) 9.8, 7.4; (91, 1152, 8896) 9.4, 7.1; none of the 380 shapes got slower.
+// With it, M, K, N, us: (92, 640, 6336) t128x128 7.2, t32x128 5.2; (805, 1536, 768) 11.3, 8.4; (91, 1152, 8896) 9.4, 7.1; (33, 256, 64) 5.3, 3.4; (300, 1024,
+// 256) 8.1, 5.6; of 575 products of K up to 512, or 1024 by at most 256 columns, none slower and the geometric mean 0.73 of what it is without.
+// t64x128's row was fitted to a kernel that is no more.  On 2779 launches of the present one its estimates are 1.3 % long on average and 9 % off
+// (r.m.s.); a row fitted to those is 7 % off, and the choice with it 1.8 % longer than the fastest one, with this one 1.6 % (985 products, 420 of the
+// ranges above and 565 of short K; 1.32 times at worst, (695, 128, 2098) 4.6 and 6.1).
 struct W4Tile {
   const char *suffix;                                  // of the kernel's name
   int rows, columns, threads;
@@ -115,10 +118,6 @@ constexpr W4Tile kW4Sets[] = {
 };
 constexpr int64_t kW4TwoSetsFrom = 17, kW4FourSetsFrom = 24, kW4FourSetsSameSplitFrom = 32;
 constexpr double kW4SetsPromise = 0.9;
-// Short products are estimated without that bound, which leaves them on the 128-row tiles: K up to 512, and up to 1024 with at most 256
-// columns.  The reason is not time, (33, 256, 64) takes 5.3 us on t128x128 and 3.4 on t32x128: these are the shapes by which the tests
-// reach the 128-row kernels and name them.
-constexpr int64_t kW4ShortSlices = 8, kW4ShortNarrowSlices = 16, kW4ShortNarrowColumns = 256;
 // The tile by rounds (above) is the better founded choice where the estimates are close: another tile or a split has to
 // promise a tenth (over those 380 shapes none is slower so than without the bound; with no such promise the worst is 1.15 times as long).
 constexpr double kW4Promise = 0.9;
@@ -246,7 +245,6 @@ W4Plan make_w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_spl
   using namespace tuning;
   static constexpr int kSplits[] = {1, 2, 3, 4, 6, 8};
   const int64_t slices = K / 64;
-  const bool is_short = slices <= kW4ShortSlices || (slices <= kW4ShortNarrowSlices && N <= kW4ShortNarrowColumns);
   auto tiles_of = [&](const W4Tile &t) { return ((M + t.rows - 1) / t.rows) * ((N + t.columns - 1) / t.columns); };
   auto plan_of = [&](const W4Tile &t, int splits) {
     W4Plan p;
@@ -255,7 +253,7 @@ W4Plan make_w4_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_spl
     p.split = split_of(slices, splits);
     const int64_t n = p.tiles * p.split.splits, full = (n - 1) / units;
     const double s = double(p.split.per), f = double(n - full * units) / double(units);
-    p.us = std::max(t.fixed + (t.e + t.c * s) * (double(full) + t.p + (1.0 - t.p) * f * f), is_short ? 0.0 : t.least + t.least_slice * s) +
+    p.us = std::max(t.fixed + (t.e + t.c * s) * (double(full) + t.p + (1.0 - t.p) * f * f), t.least + t.least_slice * s) +
            (p.split.splits > 1 ? t.meet + t.meet_each * p.split.splits : 0.0);
     return p;
   };

@@ -24,7 +24,7 @@ def gpu(pkg, library, request):
 
 def _calls(gpu, pkg):
     """One call of each family that splits its K."""
-    return [lambda s: gpu.w8a8(s, 200, 12288, 512), lambda s: gpu.w4a16(s, 64, 8192, 96), lambda s: gpu.linear(s, 100, 11520, 320, pkg.F16),
+    return [lambda s: gpu.w8a8(s, 200, 12288, 512), lambda s: gpu.w4a16(s, 64, 8256, 96, 64), lambda s: gpu.linear(s, 100, 11520, 320, pkg.F16),
             lambda s: gpu.linear(s, 100, 11520, 320, pkg.F16, route=0, q_dtype=pkg.I8)]
 
 
@@ -163,7 +163,7 @@ def test_last_kernel_is_the_symbol_that_was_launched(gpu, pkg):
 @pytest.mark.parametrize("family,shape,kernel", [
     ("w8a8", (256, 128, 128), "t32x128"), ("w8a8", (700, 256, 8200), "t128x256"), ("w8a8", (2000, 128, 16416), "t256x384"),
     ("w8a8", (100, 256, 8209), "t64x128"), ("w8a8", (128, 4096, 1030), "t32x128"), ("w8a8", (2048, 4096, 11008), "t256x384"),
-    ("w4a16", (33, 256, 64), "t128x128"), ("w4a16", (128, 512, 64), "t128x64"), ("w4a16", (256, 4096, 11008), "t128x128"),
+    ("w4a16", (512, 256, 384), "t32x128"), ("w4a16", (9000, 128, 64), "t128x64"), ("w4a16", (256, 4096, 11008), "t128x128"),
     ("w4a16", (4096, 4096, 11008), "t256x384"), ("w4a16", (600, 256, 8480), "t128x256"), ("w4a16", (2000, 256, 8000), "t256x256"),
     ("dense", (65, 2048, 33), "t32x128"), ("dense", (700, 1024, 8200), "t128x256"), ("dense", (999, 4096, 11008), "t128x384")])
 def test_the_tile_a_shape_takes(gpu, pkg, family, shape, kernel):
@@ -173,9 +173,10 @@ def test_the_tile_a_shape_takes(gpu, pkg, family, shape, kernel):
 
 @pytest.mark.parametrize("shape,kernel", [
     ((92, 640, 6336), "t32x128"), ((1001, 896, 640), "t32x128"), ((805, 1536, 768), "t32x128x2"), ((606, 1280, 384), "t32x128"), ((579, 1152, 1550), "t32x128x2"),
-    ((33, 576, 320), "t32x128"), ((300, 1024, 257), "t32x128"), ((300, 1024, 256), "t128x128"), ((300, 1088, 256), "t32x128x2"), ((300, 512, 2000), "t128x128")])
+    ((33, 576, 320), "t32x128"), ((300, 960, 257), "t32x128"), ((300, 960, 256), "t32x128"), ((300, 1088, 256), "t32x128x2"), ((300, 512, 2000), "t32x128"),
+    ((33, 64, 64), "t32x128"), ((748, 64, 127), "t32x128"), ((512, 256, 4096), "t128x128")])
 def test_few_tiles_are_not_estimated_below_what_one_of_them_takes(gpu, shape, kernel):
-    """On both sides of the lines between short products and others: 512 and 1024 of K, 256 columns."""
+    """However short K is and however few the columns are."""
     assert gpu.w4a16(8, *shape, 64)[0] == "mtrt_gemm_w4a16_" + kernel
 
 

@@ -18,6 +18,7 @@ typical output, so a kernel that rounded once too often per product would not pa
 import numpy as np
 import pytest
 
+from dispatch import Split
 from helpers import bits16, rng
 
 pytestmark = pytest.mark.gpu
@@ -386,13 +387,17 @@ def _check_w4a16(orc, y, a, w, s, K, N, B, ref_bits, max_share=kMaxShare):
 @pytest.mark.parametrize("shape", [(16, 256, 64), (1, 128, 32), (32, 1024, 96), (7, 512, 40), (33, 256, 64), (128, 512, 64),
                                    (200, 384, 100), (300, 1024, 256), (512, 256, 384), (48, 512, 1000), (64, 256, 96), (50, 384, 8209)])
 def test_w4a16_small_shapes(pkg, orc, shape):
+    """Through the entry point, and more than 32 rows through the 128-row tiles too."""
     M, K, N = shape
     B = 128
     a, w, wp, s = _w4a16_inputs(orc, rng(M + K + N), M, K, N, B)
     y, kernel = _run_w4a16(pkg, a, wp, s, K, N, B)
-    assert kernel == ("mtrt_gemm_w4a16_strips16" if M <= 16 else "mtrt_gemm_w4a16_skinny" if M <= 32 else
-                      "mtrt_gemm_w4a16_t128x64" if M > 64 and N <= 64 else "mtrt_gemm_w4a16_t128x128")
-    _check_w4a16(orc, y, a, w, s, K, N, B, orc.gemm_w4a16(a, wp, s, K, N, B))
+    assert M > 32 or kernel == ("mtrt_gemm_w4a16_strips16" if M <= 16 else "mtrt_gemm_w4a16_skinny")
+    ref = orc.gemm_w4a16(a, wp, s, K, N, B)
+    _check_w4a16(orc, y, a, w, s, K, N, B, ref)
+    if M > 32:
+        tile = "t128x64" if M > 64 and N <= 64 else "t128x128"
+        _check_w4a16(orc, _launch_w4a16(pkg, tile, a, wp, s, K, N, B), a, w, s, K, N, B, ref)
 
 
 def test_w4a16_dequantised_weights_are_bit_exact(pkg, orc):
@@ -411,10 +416,10 @@ def test_w4a16_dequantised_weights_are_bit_exact(pkg, orc):
         assert np.array_equal(bits16(y).reshape(-1, N), wd[rows]), kernel
 
 
-@pytest.mark.parametrize("case", [(2048, 8192, "mtrt_gemm_w4a16_t256x256"), (512, 1024, "mtrt_gemm_w4a16_t128x128"),
+@pytest.mark.parametrize("case", [(2048, 8192, "mtrt_gemm_w4a16_t256x256"), (512, 1024, "mtrt_gemm_w4a16_t32x128"), (1024, 2048, "mtrt_gemm_w4a16_t128x128"),
                                   (2048, 11008, "mtrt_gemm_w4a16_t256x384"), (1536, 4096, "mtrt_gemm_w4a16_t128x256")])
 def test_w4a16_tile_kernels_dequantise_bit_exactly(pkg, orc, case):
-    """Identity activations (M = K) through the 256 x 384, 256 x 256, 128 x 256 and 128 x 128 tile kernels: every output is one product
+    """Identity activations (M = K) through the 256 x 384, 256 x 256, 128 x 256, 128 x 128 and 32 x 128 tile kernels: every output is one product
     1 x wd plus zeros, so y must equal the dequantised weights bit for bit whatever the order of the sums: pins the
     fragment order of the re-laid weights, the nibble decoding, the scale row of every K block and the single f16
     rounding in the kernels that carry the benchmark."""
@@ -433,26 +438,28 @@ def test_w4a16_tile_kernels_dequantise_bit_exactly(pkg, orc, case):
     assert np.array_equal(bits16(y).reshape(K, N), wd)
 
 
-def _launch_wide_w4a16(pkg, a, wp_host, s, K, N, B):
-    """mtrt_gemm_w4a16_t256x384 launched by hand from the built-in module (the entry point takes it only where its
-    rounds come out shorter), with the grid its comment gives."""
+def _launch_w4a16(pkg, tile, a, wp_host, s, K, N, B):
+    """mtrt_gemm_w4a16_t<rows>x<columns> launched by hand from the built-in module, K whole (the entry point takes each where it is estimated
+    to be the fastest), with the grid its comment gives."""
     import ctypes
     import torch
     L = pkg.lib()
     pkg.check(L.mtrt_hip_init())
     M = a.shape[0]
+    rows, columns, threads = {"t256x384": (256, 384, 256), "t256x256": (256, 256, 256), "t128x128": (128, 128, 512), "t128x64": (128, 64, 256)}[tile]
+    assert K % 64 == 0 and B % 64 == 0 and K % B == 0 and a.shape == (M, K) and s.size == K // B * N and 2 * M * K < 1 << 32
     ad = torch.from_numpy(a.view(np.int16)).view(torch.float16).cuda()
     sd = torch.from_numpy(s.view(np.int16)).view(torch.float16).cuda()
     pre = pkg.gemm_w4a16_prepack(torch.from_numpy(wp_host).cuda(), K, N)
     y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
-    name = b"mtrt_gemm_w4a16_t256x384"
+    name = b"mtrt_gemm_w4a16_" + tile.encode()
     fn = L.mtrt_cuda_module_get_function(L.mtrt_hip_builtin_module(), name, len(name))
     assert fn
     vals = [ctypes.c_void_p(ad.data_ptr()), ctypes.c_void_p(pre.data_ptr()), ctypes.c_void_p(sd.data_ptr()), ctypes.c_void_p(y.data_ptr()),
-            ctypes.c_int64(M), ctypes.c_int64(K), ctypes.c_int64(N), ctypes.c_int64(B)]
+            ctypes.c_int64(M), ctypes.c_int64(K), ctypes.c_int64(N), ctypes.c_int64(B), ctypes.c_void_p(None), Split(1, K // 64, None, None)]
     args = (ctypes.c_void_p * len(vals))(*[ctypes.cast(ctypes.pointer(v), ctypes.c_void_p) for v in vals])
-    tiles = ((M + 255) // 256) * ((N + 383) // 384)
-    L.mtrt_cuda_launch_kernel(fn, 8 * ((tiles + 7) // 8), 1, 1, 256, 1, 1, 0, torch.cuda.current_stream().cuda_stream, args)
+    tiles = ((M + rows - 1) // rows) * ((N + columns - 1) // columns)
+    L.mtrt_cuda_launch_kernel(fn, 8 * ((tiles + 7) // 8), 1, 1, threads, 1, 1, 0, torch.cuda.current_stream().cuda_stream, args)
     torch.cuda.synchronize()
     return y
 
@@ -466,7 +473,7 @@ def test_w4a16_wide_tile_kernel(pkg, orc, case):
     M, K, N, B = case
     a, w, wp, s = _w4a16_inputs(orc, rng(M * K + N + 1), M, K, N, B)
     print("case: w4a16 wide tile", case, flush=True)
-    y = _launch_wide_w4a16(pkg, a, wp, s, K, N, B)
+    y = _launch_w4a16(pkg, "t256x384", a, wp, s, K, N, B)
     orc.set_threads(16)
     ref = orc.gemm_w4a16(a, wp, s, K, N, B)
     orc.set_threads(1)
@@ -477,13 +484,8 @@ def test_w4a16_wide_tile_kernel_equals_the_256_x_256_tile_on_random_shapes(pkg, 
     """Both 256-row tile kernels add a row's products in the same order (k ascending, one f32 accumulator per output),
     so their results are the same bits: 16 seeded shapes with ragged M and N, blocks of one to four slices.  (The
     entry point is steered to the 256 x 256 tile by launching it by hand, like the wide one.)"""
-    import ctypes
     import torch
-    L = pkg.lib()
     g = rng(2025)
-    name = b"mtrt_gemm_w4a16_t256x256"
-    fn = L.mtrt_cuda_module_get_function(L.mtrt_hip_builtin_module(), name, len(name))
-    assert fn
     for case in range(16):
         M = int(g.integers(1, 1200))
         B = 64 * int(g.integers(1, 5))
@@ -491,17 +493,8 @@ def test_w4a16_wide_tile_kernel_equals_the_256_x_256_tile_on_random_shapes(pkg, 
         N = int(g.integers(1, 2400))
         a, w, wp, s = _w4a16_inputs(orc, g, M, K, N, B)
         print("case: w4a16 wide vs 256 x 256", (M, K, N, B), flush=True)
-        y_wide = _launch_wide_w4a16(pkg, a, wp, s, K, N, B)
-        ad = torch.from_numpy(a.view(np.int16)).view(torch.float16).cuda()
-        sd = torch.from_numpy(s.view(np.int16)).view(torch.float16).cuda()
-        pre = pkg.gemm_w4a16_prepack(torch.from_numpy(wp).cuda(), K, N)
-        y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
-        vals = [ctypes.c_void_p(ad.data_ptr()), ctypes.c_void_p(pre.data_ptr()), ctypes.c_void_p(sd.data_ptr()), ctypes.c_void_p(y.data_ptr()),
-                ctypes.c_int64(M), ctypes.c_int64(K), ctypes.c_int64(N), ctypes.c_int64(B)]
-        args = (ctypes.c_void_p * len(vals))(*[ctypes.cast(ctypes.pointer(v), ctypes.c_void_p) for v in vals])
-        tiles = ((M + 255) // 256) * ((N + 255) // 256)
-        L.mtrt_cuda_launch_kernel(fn, 8 * ((tiles + 7) // 8), 1, 1, 256, 1, 1, 0, torch.cuda.current_stream().cuda_stream, args)
-        torch.cuda.synchronize()
+        y_wide = _launch_w4a16(pkg, "t256x384", a, wp, s, K, N, B)
+        y = _launch_w4a16(pkg, "t256x256", a, wp, s, K, N, B)
         assert torch.equal(y_wide.view(torch.int16), y.view(torch.int16)), (M, K, N, B)
 
 
@@ -620,11 +613,10 @@ def test_w4a16_strip_kernel(pkg, orc, shape):
 
 def test_w4a16_narrow_mid_tile_kernel(pkg, orc):
     """128 x 64 tiles: matrices at most 64 columns wide (M = 600, N = 40: ragged in M and N), K = 320 (five slices:
-    main loop and tail)."""
+    main loop and tail).  By hand: the entry point takes them for some ten thousand rows."""
     M, K, N, B = 600, 320, 40, 64
     a, w, wp, s = _w4a16_inputs(orc, rng(78), M, K, N, B)
-    y, kernel = _run_w4a16(pkg, a, wp, s, K, N, B)
-    assert kernel == "mtrt_gemm_w4a16_t128x64"
+    y = _launch_w4a16(pkg, "t128x64", a, wp, s, K, N, B)
     rows = sorted(set([0, 1, 127, 128, 255, 256, 511, 512, 598, 599] + list(range(3, M, 41))))
     orc.set_threads(16)
     ref = np.concatenate([orc.gemm_w4a16(a, wp, s, K, N, B, m0=r, mcount=1) for r in rows])

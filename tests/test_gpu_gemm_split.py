@@ -111,15 +111,15 @@ def test_graphs_recorded_on_one_stream_replay_at_once(pkg):
     tp = importlib.import_module(pkg.__name__ + ".tp")
     a8, w8, a_s, w_s = _inputs(5, 200, 12288, 512)
     f8 = pkg.gemm_w8a8_prepack_fragments(w8)
-    a4, packed, s4, _ = _w4_inputs(6, 64, 8192, 96, 128)
-    p4 = pkg.gemm_w4a16_prepack(packed, 8192, 96)
+    a4, packed, s4, _ = _w4_inputs(6, 64, 8256, 96, 64)
+    p4 = pkg.gemm_w4a16_prepack(packed, 8256, 96)
     lin = tp.Linear(11520, 320, dtype=tp.float16)
     lin.weight = tp.Tensor((torch.randn(320, 11520) * 0.05).half())
     x = torch.randn(100, 11520).half().cuda()
 
     def calls(shift):
         return [pkg.gemm_w8a8_fragments(a8.roll(shift, 0), f8, a_s, w_s, 512),
-                pkg.gemm_w4a16(a4.roll(shift, 0), s4, 8192, 96, 128, w_prepacked=p4), lin(tp.Tensor(x.roll(shift, 0))).torch()]
+                pkg.gemm_w4a16(a4.roll(shift, 0), s4, 8256, 96, 64, w_prepacked=p4), lin(tp.Tensor(x.roll(shift, 0))).torch()]
     want = [calls(k) for k in range(3)]
     torch.cuda.synchronize()
     record, streams = torch.cuda.Stream(), [torch.cuda.Stream(), torch.cuda.Stream()]
@@ -188,7 +188,7 @@ def test_w4a16_tiles_and_splits(pkg, case):
 
 def test_some_w4a16_shape_is_split(pkg):
     L = pkg.lib()
-    assert L.mtrt_hip_gemm_w4a16_workspace(64, 8192, 96, 128) > 0
+    assert L.mtrt_hip_gemm_w4a16_workspace(64, 8256, 96, 64) > 0
     assert L.mtrt_hip_gemm_w4a16_workspace(32, 8192, 96, 128) == 0 and L.mtrt_hip_gemm_w4a16_workspace(64, 8192, 96, 96) == 0
 
 
@@ -198,9 +198,9 @@ W8_TILES = [((41, 256, 9), "t32x128", 0), ((41, 3584, 9), "t32x128", 1), ((2115,
             ((2143, 256, 913), "t128x128", 0), ((1187, 8704, 793), "t128x128", 1), ((323, 256, 10933), "t128x256", 0),
             ((1647, 8448, 1253), "t128x256", 1), ((665, 256, 11017), "t128x384", 0), ((2747, 12160, 1423), "t128x384", 1),
             ((1463, 256, 8109), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
-W4_TILES = [((45, 1024, 9), "t32x128", 0), ((41, 1280, 9), "t32x128", 1), ((133, 640, 10297), "t64x128", 0), ((2791, 4736, 9), "t64x128", 1),
-            ((261, 256, 9955), "t64x256", 0), ((1027, 6592, 963), "t64x256", 1), ((65, 64, 9), "t128x64", 0), ((41, 64, 9), "t128x128", 0),
-            ((2727, 5248, 279), "t128x128", 1), ((139, 64, 8901), "t128x256", 0), ((665, 256, 11017), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
+W4_TILES = [((45, 704, 9), "t32x128", 0), ((41, 1344, 9), "t32x128", 1), ((133, 640, 10297), "t64x128", 0), ((2791, 4736, 9), "t64x128", 1),
+            ((261, 256, 9955), "t64x256", 0), ((1027, 6592, 963), "t64x256", 1), ((8389, 64, 13), "t128x64", 0), ((1387, 64, 1287), "t128x128", 0),
+            ((2727, 5248, 279), "t128x128", 1), ((385, 64, 8453), "t128x256", 0), ((665, 256, 11017), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
 DENSE_TILES = [((41, 64, 9), "t32x128", 0), ((53, 1792, 9), "t32x128", 1), ((2115, 256, 387), "t64x128", 0), ((2781, 5568, 9), "t64x128", 1),
                ((2143, 256, 913), "t128x128", 0), ((2727, 5248, 279), "t128x128", 1), ((323, 256, 10933), "t128x256", 0),
                ((2701, 4544, 657), "t128x256", 1), ((665, 256, 11017), "t128x384", 0), ((143, 9024, 11467), "t128x384", 1),
