@@ -87,11 +87,11 @@ constexpr double kW4Mid256RoundPerSmallRound = 1.9;
 // launches of 621 log-uniform shapes, M 33 ... 4096, K 256 ... 14336, N 64 ... 16384, 1 to 12 splits.
 // That is a full chip's law.  However few tiles there are, one of them takes least + least_slice * s, which a launch of few
 // large tiles runs into (fitted to the launches of at most half as many unsplit tiles as units of 380 shapes of the same range).
-// With it, M, K, N, us: (92, 640, 6336) t128x128 7.2, t32x128 5.2; (805, 1536, 768) 11.3, 8.4; (91, 1152, 8896) 9.4, 7.1; (33, 256, 64) 5.3, 3.4; (300, 1024,
-// 256) 8.1, 5.6; of 575 products of K up to 512, or 1024 by at most 256 columns, none slower and the geometric mean 0.73 of what it is without.
+// With it, M, K, N, us: (92, 640, 6336) t128x128 7.2, t32x128 5.2; (805, 1536, 768) 11.3, 8.4; (91, 1152, 8896) 9.4, 7.1; (748, 64, 127) 5.5, 3.3; (304, 704,
+// 238) 8.1, 5.6; of 575 products of K up to 512, or 1024 by at most 256 columns, none slower and the geometric mean 0.73 of what it is without.
 // t64x128's row was fitted to a kernel that is no more.  On 2779 launches of the present one its estimates are 1.3 % long on average and 9 % off
-// (r.m.s.); a row fitted to those is 7 % off, and the choice with it 1.8 % longer than the fastest one, with this one 1.6 % (985 products, 420 of the
-// ranges above and 565 of short K; 1.32 times at worst, (695, 128, 2098) 4.6 and 6.1).
+// (r.m.s.); a row fitted to those is 7 % off, and the choice with it 1.8 % longer than the fastest one, with this one 1.6 % (985 products of 33 to 4096
+// rows, those 575 among them; 1.32 times as long at worst, (695, 128, 2098) 6.1 and 4.6).
 struct W4Tile {
   const char *suffix;                                  // of the kernel's name
   int rows, columns, threads;
@@ -1581,28 +1581,28 @@ bool w4_fast(const void *a, const void *w_prepacked, int64_t K, int64_t block) {
 
 // Whether the strip kernel (16 rows by 16 columns over all of K, four waves) takes a product.  Up to 16 rows: blocks of 64 where each wave
 // has a slice of 128 k; the kernel behind, with slices of 64, is as fast below that.
-// 17 to 512 rows in groups of 16, where the 32-row kernel and the tiles leave most of the chip idle.  The line is the number of 16-column tiles that a
-// workgroup has side by side when there is one to a compute unit (`each`): 512 of K take 0.34, 0.53 and 0.75 us so, 0.57 in the 32-row kernel, and
-// a long walk down K loses against tiles that share it.  us, (M, K, N), the others and this:
-//   one tile (27, 7040, 384) 10.6, 6.2; (45, 5376, 320) 9.0, 5.8; (146, 5760, 256) 9.8, 6.2; (37, 9216, 1247) 11.8, 8.9
-//   two (22, 13056, 2880) 16.3, 12.9; (190, 1408, 640) 6.9, 4.1; (211, 6784, 384) 11.2, 10.1; (96, 12032, 1088) 13.7, 15.4
-//   three (52, 2432, 2496) 8.1, 6.2; (386, 1920, 448) 8.3, 6.9; (54, 5120, 4032) 12.2, 12.2; (29, 5120, 5056) 10.2, 9.2
-//   four and more (186, 4224, 1664) 11.6, 15.7; (418, 2304, 448) 8.9, 11.1
-//   blocks of 64 (26, 10240, 832) 12.8, 9.6; (17, 768, 3338) 3.6, 3.8
-// Over 80 products of these ranges 1.32 times as fast in the geometric mean.  With fewer tiles than half of the units, parts of a K longer than 6144
-// fill the chip.  K below 1408 is not a matter of time (those would gain as much: (119, 512, 384) 6.6, 2.8, (59, 1152, 302) 6.4, 3.3): these are the
-// shapes by which the tests reach the kernels behind and name them.
+// 17 to 512 rows in groups of 16, where the 32-row kernel and the tiles leave most of the chip idle.  The lines are by the number of 16-column tiles that a
+// workgroup has side by side when there is one to a compute unit (`each`), and by K, on which a workgroup walks alone.  How many times as long the
+// others take (geometric means over 569 products, blocks of 64 and of 128 alike):
+//                        K up to 255   511  1023  1407  2559  5000  6144  9000 12288 14336
+//   one, more than 32 rows      1.14  1.35  1.71  2.05  1.92  1.95  1.86  1.67  1.44  1.41
+//   one, up to 32 rows          1.12  1.14  1.19  1.29  1.31  1.48  1.65  1.72  1.79     -
+//   two, more than 32 rows      1.01  1.18  1.39  1.69  1.62  1.71  1.52  1.39  1.13  1.00
+//   two, up to 32 rows          0.98     -  1.03  1.07     -  1.10  1.23     -     -     -
+//   three, more than 32 rows    0.93  1.04  1.17  1.47  1.45  1.35  1.37  1.15  0.97     -
+//   three, up to 32 rows           -  0.91     -     -     -     -  1.04  1.02     -     -
+//   four                        0.77  0.85  1.00  1.21  0.95  1.15  0.84  0.86  0.77     -
+// us, the others and this: (119, 512, 384) 4.6, 3.0; (59, 1152, 302) 6.7, 3.2; (211, 6784, 384) 11.7, 7.9; (64, 8192, 96) 9.8, 6.1; (54, 5120, 4032), four, 12.0,
+// 10.8; (186, 4224, 1664), five, 11.8, 12.8.
 bool w4_strips(int64_t M, int64_t K, int64_t N, int64_t block, int64_t units) {
   if (K % 128 != 0 || (block != 64 && block % 128 != 0) || M > 512 || M * K > (int64_t(1) << 31))
     return false;
   if (M <= 16)
     return block != 64 || K >= 512;
   const int64_t groups = (M + 15) / 16, tiles = (N + 15) / 16, most = std::max<int64_t>(units / groups, 1), each = (tiles + most - 1) / most;
-  if (K < (block == 64 ? 2048 : 1408) || each > 3)
-    return false;
   if (M <= 32)
-    return each <= 2;
-  return each == 3 ? K <= 2560 : each == 2 || 2 * groups * tiles < units ? K <= 6144 : K <= 12288;
+    return each == 1 || (each == 2 && K >= 1024);
+  return each == 1 || (each == 2 && K >= 256 && K <= 12288) || (each == 3 && K >= 512 && K <= 9216);
 }
 
 // bias: f16 [N], added to the rounded product, or null (only with re-laid weights)

@@ -309,16 +309,20 @@ def test_strips_of_more_than_16_rows_cover_the_output_and_need_no_workspace(gpu)
     workspace asked for is what the launch takes."""
     seen = set()
     for M in (17, 32, 33, 100, 497, 512, 513):
-        for K in (1280, 1408, 2048, 2560, 2688, 6144, 6272, 12288, 12416):
+        for K in (128, 256, 384, 512, 896, 1024, 1408, 6272, 9216, 9344, 12288, 12416, 14336):
             for N in (1, 16, 17, 250, 500, 1000, 4000, 9000):
                 for block in (64, 128):
                     name = gpu.w4a16(8, M, K, N, block)[0]
                     grid, wants = gpu.sizes[-1][1], gpu.lib.mtrt_hip_gemm_w4a16_workspace(M, K, N, block)
                     strips, groups, tiles = "strips" in name, (M + 15) // 16, (N + 15) // 16
-                    seen.add((strips, M > 32))
+                    each = -(-tiles // (256 // groups))              # tiles side by side, a workgroup to a unit
+                    wide = M > 32
+                    assert strips == (M <= 512 and (each == 1 or (each == 2 and (256 <= K <= 12288 if wide else K >= 1024)) or
+                                                    (each == 3 and wide and 512 <= K <= 9216))), (M, K, N)
+                    seen.add((strips, wide))
                     if strips:
-                        assert M <= 512 and grid % groups == 0 and 1 <= grid // groups <= tiles and grid <= 256 and -(-tiles // (grid // groups)) <= 3 and wants == 0
-                        assert name.endswith("_b64") == (block == 64) and K >= (2048 if block == 64 else 1408)
+                        assert grid % groups == 0 and 1 <= grid // groups <= tiles and grid <= 256 and -(-tiles // (grid // groups)) == each and wants == 0
+                        assert name.endswith("_b64") == (block == 64)
                     elif wants:
                         assert gpu.launches[-1][2][0] > 1
     assert seen == {(True, True), (True, False), (False, True), (False, False)}

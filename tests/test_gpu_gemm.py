@@ -392,7 +392,7 @@ def test_w4a16_small_shapes(pkg, orc, shape):
     B = 128
     a, w, wp, s = _w4a16_inputs(orc, rng(M + K + N), M, K, N, B)
     y, kernel = _run_w4a16(pkg, a, wp, s, K, N, B)
-    assert M > 32 or kernel == ("mtrt_gemm_w4a16_strips16" if M <= 16 else "mtrt_gemm_w4a16_skinny")
+    assert M > 32 or kernel == "mtrt_gemm_w4a16_strips16"
     ref = orc.gemm_w4a16(a, wp, s, K, N, B)
     _check_w4a16(orc, y, a, w, s, K, N, B, ref)
     if M > 32:
@@ -400,20 +400,25 @@ def test_w4a16_small_shapes(pkg, orc, shape):
         _check_w4a16(orc, _launch_w4a16(pkg, tile, a, wp, s, K, N, B), a, w, s, K, N, B, ref)
 
 
-def test_w4a16_dequantised_weights_are_bit_exact(pkg, orc):
-    """One-hot activations read the dequantised weights back unchanged: pins the prepack order,
+@pytest.mark.parametrize("K,B", [(512, 128), (448, 64)])
+def test_w4a16_dequantised_weights_are_bit_exact(pkg, orc, K, B):
+    """One-hot activations read the dequantised weights back unchanged: pins the prepack orders,
     the nibble decoding, the block index of the scale and the single f16 rounding."""
-    K, N, B = 512, 160, 128
+    N = 160
     g = rng(31)
     w = g.integers(-8, 8, (K, N)).astype(np.int8)
     s = orc.narrow(g.uniform(0.005, 0.02, (K // B, N)).astype(np.float32), orc.F16)
     eye = np.zeros((K, K), np.float32)
     np.fill_diagonal(eye, 1.0)
     wd = (w.astype(np.float16) * np.repeat(s.view(np.float16), B, axis=0)).view(np.uint16)
-    for rows in (slice(0, K), slice(0, 32), slice(100, 116)):        # big-tile, skinny (32 rows), skinny (16 rows)
+    wp = orc.pack_int4(w)
+    for rows in (slice(0, K), slice(0, 32), slice(100, 116)):        # strips in 32 groups, in two, in one; K = 448: 32-row tiles, skinny (32 and 16 rows)
         a = orc.narrow(eye[rows], orc.F16)
-        y, kernel = _run_w4a16(pkg, a, orc.pack_int4(w), s, K, N, B)
+        y, kernel = _run_w4a16(pkg, a, wp, s, K, N, B)
         assert np.array_equal(bits16(y).reshape(-1, N), wd[rows]), kernel
+    for tile in ("t128x128", "t256x256", "t256x384"):
+        y = _launch_w4a16(pkg, tile, orc.narrow(eye, orc.F16), wp, s, K, N, B)
+        assert np.array_equal(bits16(y).reshape(-1, N), wd), tile
 
 
 @pytest.mark.parametrize("case", [(2048, 8192, "mtrt_gemm_w4a16_t256x256"), (512, 1024, "mtrt_gemm_w4a16_t32x128"), (1024, 2048, "mtrt_gemm_w4a16_t128x128"),

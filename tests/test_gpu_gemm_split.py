@@ -257,9 +257,9 @@ def test_every_w4a16_tile(pkg, shape, tile, split):
 # Sets of waves that take slices in turn: parts with a whole number of rounds and each rest, the last part of a split another one
 # than the others, ragged rows and columns; blocks of one, two, three and four slices and one block for all.
 @pytest.mark.parametrize("shape,tile,blocks", [
-    ((33, 1152, 130), "t32x128x2", (64, 128, 192, 1152)), ((40, 1088, 130), "t32x128x2", (64,)), ((63, 8768, 130), "t32x128x2", (64,)), ((65, 8256, 130), "t32x128x2", (64, 192)),
+    ((513, 1152, 130), "t32x128x2", (64, 128, 192, 1152)), ((40, 1088, 130), "t32x128x2", (64,)), ((63, 8768, 130), "t32x128x2", (64,)), ((65, 8256, 130), "t32x128x2", (64, 192)),
     ((33, 2304, 8641), "t32x128x4", (64, 128, 192, 256, 2304)), ((33, 2368, 8641), "t32x128x4", (64,)), ((33, 2176, 8641), "t32x128x4", (128,)),
-    ((97, 2240, 4100), "t32x128x4", (64, 320)), ((33, 8832, 3000), "t32x128x4", (64, 192)), ((33, 6848, 4100), "t32x128x4", (64,)),
+    ((97, 2240, 4100), "t32x128x4", (64, 320)), ((33, 9024, 3000), "t32x128x4", (64, 192)), ((33, 6848, 4100), "t32x128x4", (64,)),
     ((130, 1152, 8000), "t64x128", (64, 128, 192, 1152)), ((97, 1216, 8641), "t64x128", (64,)), ((33, 2688, 8641), "t64x128", (64, 128)), ((40, 2496, 8641), "t64x128", (192,))])
 def test_w4a16_slices_in_turn(pkg, shape, tile, blocks):
     import torch

@@ -39,7 +39,8 @@ def test_w4a16_strips(pkg, M, block):
 def test_w4a16_skinny(pkg, M):
     import torch
     for i, slices in enumerate((1, 2, 3, 4, 5, 6, 7, 9, 13, 17, 22, 31)):
-        K, N = slices * 64, (16, 40, 300, 1000, 8224)[i % 5]
+        # (17 to 32 rows by few columns take the strips where K is a multiple of 128)
+        K, N = slices * 64, (16, 40, 300, 1000, 8224)[i % 5] if M <= 16 or slices % 2 else 8224
         _w4(torch, pkg, M, K, N, 64, 100 * M + i)
         if M > 16 or K < 512 or K % 128:
             assert pkg.last_kernel().startswith("mtrt_gemm_w4a16_skinny"), (K, N)
@@ -89,3 +90,18 @@ def test_w4a16_strips_in_groups_of_rows(pkg, M, block):
             _w4(torch, pkg, M, K, N, block, 10 * M + i)
             if torch.cuda.get_device_properties(0).multi_processor_count == units and (M > 32 or i < 4):
                 assert pkg.last_kernel() == "mtrt_gemm_w4a16_strips16" + ("_b64" if block == 64 else ""), (K, N)
+
+
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("M", [17, 31, 33, 64, 100, 512])
+def test_w4a16_strips_of_few_slices(pkg, M, block):
+    """Fewer slices of 128 k than waves, as many, and one more; one, two and three tiles to a workgroup from where the rule takes them."""
+    import torch
+    groups = (M + 15) // 16
+    for i, (K, each) in enumerate(((128, 1), (256, 1), (384, 1), (512, 1), (640, 1), (1024, 1), (256, 2), (512, 2), (1024, 2), (512, 3), (896, 3))):
+        if M <= 32 and (each == 3 or (each == 2 and K < 1024)):
+            continue
+        N = 16 * ((256 // groups) * (each - 1) + 1) - (0, 9)[i % 2]
+        _w4(torch, pkg, M, K, N, block, 10 * M + i)
+        if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+            assert pkg.last_kernel() == "mtrt_gemm_w4a16_strips16" + ("_b64" if block == 64 else ""), (K, N)
