@@ -142,11 +142,11 @@ constexpr FragTile kFragTiles[] = {
     {"t256x256", 256, 256, false, 11.0, 0.25, 8.63, 0.912, 0.0, 0.0},
     {"t256x384", 256, 384, false, 12.3, 0.764, 9.99, 1.346, 0.0, 0.0},
 };
-// Two 128 x 256 tiles share a unit: L > 1 of them, each with all of K, take `first` + L * (each + slice * s) us, from five slices on (shorter products stay
-// on the wider tiles: by those shapes the tests reach them, (4011, 256, 12672) takes 46.9 us on t256x384 and 37.1 here).  Fitted to 70 products of 200 to
-// 4096 rows beside the others' estimates: (3043, 768, 13632) 49.3 -> 42.2, (2006, 896, 14784) 38.3 -> 32.2.
+// Two 128 x 256 tiles share a unit: L > 1 of them, each with all of K, take `first` + L * (each + slice * s) us.  Fitted to 70 products of 200 to
+// 4096 rows beside the others' estimates: (3043, 768, 13632) 49.3 -> 42.2, (2006, 896, 14784) 38.3 -> 32.2.  So from one slice on: over 330 products
+// of one to eight slices the choice is 2.2 % longer than the fastest one, 3.7 % with the pairs from five slices on only (a line that was there for the tests'
+// shapes); where that changes it, int8 (940, 512, 12416) 14.7 -> 11.3, f16 (3715, 128, 8839) 32.3 -> 25.2; worst (1399, 256, 12352) 15.1 -> 16.2.
 constexpr double kFragPairsUs = 1.24, kFragPairsEachUs = 2.68, kFragPairsSliceUs = 0.515;
-constexpr int64_t kFragPairsFrom = 5;
 // The wave-private kernels up to 32 and 64 rows on the same weights (gemm_core::rows32): L = ceil of their 32-column tiles
 // over the compute units; int8 M = 16, K = N = 4096 5.7 us, (32, 3968, 11328) 13.2; M = 64, K = N = 4096 8.5, (54, 12032, 8682) 32.6.
 constexpr double kFragRows32Us = 2.0, kFragRows32TileUs = 1.2, kFragRows32SliceUs = 0.08, kFragRows32LaterSliceUs = 0.13;
@@ -207,7 +207,7 @@ FragPlan make_frag_plan(int64_t M, int64_t N, int64_t slices, int64_t units, boo
         break;
       const FragSplit split = split_of(slices, splits);
       const double s = double(split.per), rounds = double((tiles * int64_t(split.splits) + units - 1) / units);
-      const bool pairs = splits == 1 && t.rows == 128 && t.columns == 256 && rounds > 1.0 && split.per >= tuning::kFragPairsFrom;
+      const bool pairs = splits == 1 && t.rows == 128 && t.columns == 256 && rounds > 1.0;
       const double full = pairs ? tuning::kFragPairsUs + rounds * (tuning::kFragPairsEachUs + tuning::kFragPairsSliceUs * s)
                                 : rounds * (t.next + t.next_slice * s);
       const double us = std::max(t.first + t.first_slice * s, full) +

@@ -161,7 +161,7 @@ def test_last_kernel_is_the_symbol_that_was_launched(gpu, pkg):
 
 
 @pytest.mark.parametrize("family,shape,kernel", [
-    ("w8a8", (256, 128, 128), "t32x128"), ("w8a8", (700, 256, 8200), "t128x256"), ("w8a8", (2000, 128, 16416), "t256x384"),
+    ("w8a8", (256, 128, 128), "t32x128"), ("w8a8", (700, 256, 8200), "t128x256"), ("w8a8", (2000, 128, 16416), "t128x256"), ("w8a8", (1669, 512, 9249), "t256x384"),
     ("w8a8", (100, 256, 8209), "t64x128"), ("w8a8", (128, 4096, 1030), "t32x128"), ("w8a8", (2048, 4096, 11008), "t256x384"),
     ("w4a16", (512, 256, 384), "t32x128"), ("w4a16", (9000, 128, 64), "t128x64"), ("w4a16", (256, 4096, 11008), "t128x128"),
     ("w4a16", (4096, 4096, 11008), "t256x384"), ("w4a16", (600, 256, 8480), "t128x256"), ("w4a16", (2000, 256, 8000), "t256x256"),
@@ -329,8 +329,8 @@ def test_strips_of_more_than_16_rows_cover_the_output_and_need_no_workspace(gpu)
 
 
 @pytest.mark.parametrize("family,shape,kernel", [
-    ("w8a8", (3043, 768, 13632), "t128x256"), ("w8a8", (2817, 768, 5376), "t128x256"), ("w8a8", (2817, 512, 5376), "t256x256"), ("w8a8", (999, 4096, 11008), "t128x384"),
-    ("dense", (2817, 384, 5391), "t128x256"), ("dense", (2817, 256, 5376), "t256x256"), ("dense", (2981, 1472, 8768), "t256x256")])
-def test_pairs_of_tiles_from_five_slices_on(gpu, pkg, family, shape, kernel):
+    ("w8a8", (3043, 768, 13632), "t128x256"), ("w8a8", (2817, 768, 5376), "t128x256"), ("w8a8", (2817, 512, 5376), "t128x256"), ("w8a8", (2643, 128, 10112), "t128x256"), ("w8a8", (2048, 512, 11008), "t256x384"), ("w8a8", (999, 4096, 11008), "t128x384"),
+    ("dense", (2817, 384, 5391), "t128x256"), ("dense", (2817, 256, 5376), "t128x256"), ("dense", (3636, 64, 5824), "t128x256"), ("dense", (2981, 1472, 8768), "t256x256")])
+def test_pairs_of_tiles_however_short_k_is(gpu, pkg, family, shape, kernel):
     name = gpu.w8a8(8, *shape)[0] if family == "w8a8" else gpu.linear(8, *shape, pkg.F16)[0]
     assert name == {"w8a8": "mtrt_gemm_w8a8_frag_", "dense": "mtrt_gemm_dense_frag_f16_"}[family] + kernel

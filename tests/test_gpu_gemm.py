@@ -313,10 +313,10 @@ def test_w8a8_wide_tile_kernel_equals_the_entry_point_on_random_shapes(pkg):
 
 
 def test_w8a8_wide_tile_is_taken_where_its_rounds_are_shorter(pkg, orc):
-    """At the shape of BASELINE config 4 (344 tiles of 256 x 256 = one and a half rounds on 256 compute units, 232 of
-    256 x 384 = one) the entry point launches the wide kernel; the result is the oracle's either way."""
+    """344 tiles of 256 x 256 = one and a half rounds on 256 compute units, 232 of 256 x 384 = one: the entry point launches the wide
+    kernel; the result is the oracle's either way."""
     import torch
-    M, K, N = 2048, 256, 11008
+    M, K, N = 2048, 512, 11008
     a, w, a_s, w_s = _w8a8_inputs(rng(44), M, K, N)
     y, kernel = _run_w8a8_frag(pkg, a, w, a_s, w_s)
     if torch.cuda.get_device_properties(0).multi_processor_count == 256:
