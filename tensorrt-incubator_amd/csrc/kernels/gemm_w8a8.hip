@@ -129,7 +129,7 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
 // us: (M, K, N) = (256, 4096, 4096) 21.8 -> 10.4, (398, 11520, 1856) 51.8 -> 19.3, (1024, 2048, 2048) 14.7 -> 8.8,
 // (200, 12288, 512) 52.7 -> 10.6, (999, 4096, 11008) 46.5 -> 44.
 // t128x256: 239 registers, so that one workgroup's first loads and its epilogue (6 us of a tile) lie under the other's loop, where a unit has more
-// than one; what a meeting fetches at a time is one 32 x 32 tile, two would not fit.  One and two to a unit, us: (3043, 768, 13632) 59.6, 42.2;
+// than one; a meeting fetches two 32 x 32 tiles of two parts at a time (gemm_frag::meet).  One and two to a unit, us: (3043, 768, 13632) 59.6, 42.2;
 // (4011, 256, 12672) 46.5, 37.1; (2048, 4096, 11008) 91.1, 81.7; (999, 4096, 11008) 54.4, 48.3; where a unit has one tile (985, 1152, 4352) 12.0,
 // 11.6; (1296, 4992, 4352) 32.9, 32.1; with K in two parts (2332, 10368, 1024) 38.4, 37.7.
 #define MTRT_W8_FRAG_KERNEL(NAME, IT, JT, D, WG)                                                                          \

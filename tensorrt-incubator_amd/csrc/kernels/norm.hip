@@ -608,7 +608,7 @@ using namespace norm_cluster;
   extern "C" __global__ void __launch_bounds__(kNormThreads) __attribute__((amdgpu_waves_per_eu(8, 8)))        \
   mtrt_layernorm_##XN##_v8r(const XT::storage* x, const XT::storage* gamma, const XT::storage* beta,           \
                             XT::storage* y, int64_t rows, int64_t d, float eps) {                              \
-    layernorm_rows<XT, 8, true>(x, gamma, beta, y, rows, d, eps);                                                    \
+    layernorm_rows<XT, 8, true>(x, gamma, beta, y, rows, d, eps);                                              \
   }                                                                                                            \
   extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_layernorm_##XN##_any(                        \
       const XT::storage* x, const XT::storage* gamma, const XT::storage* beta, XT::storage* y, int64_t rows,  \
