@@ -193,18 +193,20 @@ def test_some_w4a16_shape_is_split(pkg):
 
 
 # A shape with ragged rows and columns for each tile, with its K whole and shared, as the host's estimate picks them on 256 compute
-# units; `workspace` says whether K is shared.
+# units; `workspace` says whether K is shared.  The tiles wider or higher than 128 x 256 with an odd number of slices too.
 W8_TILES = [((41, 256, 9), "t32x128", 0), ((41, 3584, 9), "t32x128", 1), ((2115, 256, 387), "t64x128", 0), ((2849, 11904, 9), "t64x128", 1),
             ((2143, 256, 913), "t128x128", 0), ((1187, 8704, 793), "t128x128", 1), ((323, 256, 10933), "t128x256", 0),
             ((1647, 8448, 1253), "t128x256", 1), ((2563, 768, 3171), "t128x384", 0), ((2747, 12160, 1423), "t128x384", 1),
-            ((2545, 2304, 4683), "t256x256", 0), ((1669, 512, 9249), "t256x384", 0)]
+            ((2545, 2304, 4683), "t256x256", 0), ((1669, 512, 9249), "t256x384", 0), ((661, 896, 10901), "t128x384", 0),
+            ((2488, 2944, 4629), "t256x256", 0), ((1296, 640, 12203), "t256x384", 0)]
 W4_TILES = [((45, 704, 9), "t32x128", 0), ((41, 1344, 9), "t32x128", 1), ((133, 640, 10297), "t64x128", 0), ((2791, 4736, 9), "t64x128", 1),
             ((261, 256, 9955), "t64x256", 0), ((1027, 6592, 963), "t64x256", 1), ((8389, 64, 13), "t128x64", 0), ((1387, 64, 1287), "t128x128", 0),
             ((2727, 5248, 279), "t128x128", 1), ((385, 64, 8453), "t128x256", 0), ((665, 256, 11017), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
 DENSE_TILES = [((41, 64, 9), "t32x128", 0), ((53, 1792, 9), "t32x128", 1), ((2115, 256, 387), "t64x128", 0), ((2781, 5568, 9), "t64x128", 1),
                ((2143, 256, 913), "t128x128", 0), ((2727, 5248, 279), "t128x128", 1), ((323, 256, 10933), "t128x256", 0),
                ((2701, 4544, 657), "t128x256", 1), ((2399, 384, 3391), "t128x384", 0), ((143, 9024, 11467), "t128x384", 1),
-               ((2473, 1152, 4611), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0)]
+               ((2473, 1152, 4611), "t256x256", 0), ((1497, 256, 10781), "t256x384", 0), ((1055, 576, 7361), "t128x384", 0),
+               ((5433, 1472, 2039), "t256x256", 0), ((2787, 64, 8713), "t256x384", 0), ((1671, 320, 9275), "t256x384", 0)]
 
 
 def _is(pkg, kernel):
