@@ -144,8 +144,8 @@ constexpr FragTile kFragTiles[] = {
 };
 // Two 128 x 256 tiles share a unit: L > 1 of them, each with all of K, take `first` + L * (each + slice * s) us.  Fitted to 70 products of 200 to
 // 4096 rows beside the others' estimates: (3043, 768, 13632) 49.3 -> 42.2, (2006, 896, 14784) 38.3 -> 32.2.  So from one slice on: over 330 products
-// of one to eight slices the choice is 2.2 % longer than the fastest one, 3.7 % with the pairs from five slices on only (a line that was there for the tests'
-// shapes); where that changes it, int8 (940, 512, 12416) 14.7 -> 11.3, f16 (3715, 128, 8839) 32.3 -> 25.2; worst (1399, 256, 12352) 15.1 -> 16.2.
+// of one to eight slices the choice is 2.2 % longer than the fastest one, 3.7 % with the pairs from five slices on only; where that
+// changes it, int8 (940, 512, 12416) 14.7 -> 11.3, f16 (3715, 128, 8839) 32.3 -> 25.2; worst (1399, 256, 12352) 15.1 -> 16.2.
 constexpr double kFragPairsUs = 1.24, kFragPairsEachUs = 2.68, kFragPairsSliceUs = 0.515;
 // The wave-private kernels up to 32 and 64 rows on the same weights (gemm_core::rows32): L = ceil of their 32-column tiles
 // over the compute units; int8 M = 16, K = N = 4096 5.7 us, (32, 3968, 11328) 13.2; M = 64, K = N = 4096 8.5, (54, 12032, 8682) 32.6.
