@@ -217,7 +217,7 @@ struct RowsScaleEpilogue {
 // sums (int32, exact in any order) meet in LDS.  G: groups of 8 activation rows per stage (M <= 8 * G).
 namespace small_m {
 
-template <int G, int WAVES, int JT>
+template <int G, int WAVES, int JT, bool PAST>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const v4i* __restrict__ wfrag, const RowsScaleEpilogue& epi,
                                     uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int8_t* lds) {
   constexpr int kStages = 4, kStageBytes = 8 * G * 128;
@@ -262,7 +262,8 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const v4i* __r
 #pragma unroll
       for (int p = 0; p < 4; ++p) {
         const v4i* wsrc = bp[j] + kb * 256 + p * 64;
-        __asm__ volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(dst.w[j][p]) : "v"(wsrc) : "memory");
+        if constexpr (PAST) __asm__ volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(dst.w[j][p]) : "v"(wsrc) : "memory");
+        else __asm__ volatile("global_load_dwordx4 %0, %1, off" : "=v"(dst.w[j][p]) : "v"(wsrc) : "memory");
       }
   };
   // all loads but those of `in_flight` younger slices have landed
@@ -344,27 +345,30 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const v4i* __r
 // The grid is one workgroup per column tile, or, while that would leave some compute units with two workgroups
 // and the rest with one (tiles between one and two times the compute units), one workgroup per compute unit:
 // workgroup g then also takes tile g + gridDim.x if there is one, and reads the activations once for both.
-template <int G>
+template <int G, bool PAST>
 __device__ __forceinline__ void tiles(const int8_t* __restrict__ a, const v4i* __restrict__ wfrag, const RowsScaleEpilogue& epi,
                                       uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int8_t* lds) {
   const int64_t ntiles = (N + 31) / 32;
   if (int64_t(blockIdx.x) + gridDim.x < ntiles)
-    run<G, 4, 2>(a, wfrag, epi, y, M, K, N, lds);
+    run<G, 4, 2, PAST>(a, wfrag, epi, y, M, K, N, lds);
   else
-    run<G, 4, 1>(a, wfrag, epi, y, M, K, N, lds);
+    run<G, 4, 1, PAST>(a, wfrag, epi, y, M, K, N, lds);
 }
 
 }  // namespace small_m
 
-// (a [M,K] i8, w_frag (fragment order), a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, a_step, bias) ; K % 128 == 0, a
-// and w_frag 16-byte aligned, M * K < 2^32; grid = ceil(N / 32) or the number of compute units (see small_m::tiles), block = 256.
+// (a [M,K] i8, w_frag (fragment order), a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, a_step, bias, past) ; K % 128 == 0, a
+// and w_frag 16-byte aligned, M * K < 2^32; past: the weights are read past the caches (kWeightsPastBytes in clusters.cpp); grid = ceil(N / 32) or
+// the number of compute units (see small_m::tiles), block = 256.
 // M <= 16:
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_small16(
     const int8_t* __restrict__ a, const v4i* __restrict__ w_frag, const float* __restrict__ a_scale,
     const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t a_step,
-    const uint16_t* __restrict__ bias) {
+    const uint16_t* __restrict__ bias, int32_t past) {
   __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 2 * 1024];
-  small_m::tiles<2>(a, w_frag, RowsScaleEpilogue{a_scale, w_scale, a_step, bias}, y, M, K, N, lds);
+  const RowsScaleEpilogue epi{a_scale, w_scale, a_step, bias};
+  if (past) small_m::tiles<2, true>(a, w_frag, epi, y, M, K, N, lds);
+  else small_m::tiles<2, false>(a, w_frag, epi, y, M, K, N, lds);
 }
 // Any K (no alignment needs): one output element per lane, plain loops.  Only K = 0 is left to it (every
 // other shape runs on the matrix cores).

@@ -50,6 +50,12 @@ constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
 // Products of few rows read weights above these bytes past the caches (us, past and through, f32: M = 1, 180 MB 26.7, 28.9; M = 3, 53 MB
 // 11.5, 12.0; M = 1, 29 MB 7.7, 6.8; bf16: 90 MB 16.2, 17.0; 67 MB 12.4, 13.4; 33 MB 9.8, 8.4).
 constexpr int64_t kWeightsPastBytes = int64_t(48) << 20;
+// int8 and int4 weights alike, kernel times in turns of three sets, so with the weights in the Infinity Cache (what lies in HBM takes 0 to 6 % longer
+// through the caches): W4A16 in strips (16, 4096, 2048) 5.1, 4.2; (16, 14336, 4096) 12.3, 9.9; (16, 8192, 16384), 67 MB, 18.6, 15.6, but 2 to 5 % longer
+// from HBM; 17 to 32 rows (32, 7808, 9280) 17.7, 15.9; W8A8 of 9 to 16 rows 8 MB 4 to 26 % shorter, 34 to 45 MB 8 to 21 %, 90 MB 3 % and from HBM
+// 13 % longer.  Up to four rows of W4A16 take in little beside the weights, and the line is lower: (2, 8960, 2304) 5.89, 5.69; (4, 6016, 3200) 4.98,
+// 4.76; (2, 4736, 5184) 5.49, 5.57; (1, 6400, 4864) 6.39, 6.62; (1, 4096, 11008) 6.70, 7.19.
+constexpr int64_t kFewRowsWeightsPastBytes = int64_t(10) << 20;
 // f32 products of few rows on the vector units: K from which four waves share it; the fewest weights (below, the tiles take 3 to 4 us
 // too); what several groups of rows read through the L2s.
 constexpr int64_t kDotOwnColumnsBelow = 1536, kDotMinWeights = 16384;
@@ -1352,7 +1358,8 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     // one workgroup per 32-column tile, its four waves splitting K; between one and two tiles per compute unit one
     // workgroup per unit instead, the first ones taking a second tile (as for the int4 weights)
     const uint32_t grid = uint32_t(M > 8 && tiles32 > units && tiles32 <= 2 * units ? units : tiles32);
-    void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
+    int32_t past = K * N > tuning::kWeightsPastBytes;
+    void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias, &past};
     return launch(st, KernelName("mtrt_gemm_w8a8_small16"), grid, kBlock, stream, args);
   }
   if (plan.kind == W8Plan::kRows) {
@@ -1627,7 +1634,8 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
     return MTRT_RUNTIME_ERROR;
   if (w4_fast(a, w_prepacked, K, block)) {
     const int64_t cus = num_compute_units(st);
-    void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias};
+    int32_t past = K * N / 2 > (M <= 4 ? tuning::kFewRowsWeightsPastBytes : tuning::kWeightsPastBytes);
+    void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias, &past};
     // (rows of activations are addressed by 32-bit offsets below)
     if (w4_strips(M, K, N, block, cus)) {
       // 16-column tiles over all of K (weights in strip order).  One workgroup per compute unit; up to 16 rows two for more than three
@@ -1635,7 +1643,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
       // 12.3 against 11.9, 1024 tiles 12.9 against 12.3), and with up to four rows for more than one (M = 1: 320 tiles 5.6 against
       // 5.2 us, 688 tiles 7.4 against 7.1, 1024 tiles 10.2 against 9.8); more rows' groups share the units ((22, 13056, 2880) 12.9 against 17.0).
       const void *in_strips = static_cast<const char *>(w_prepacked) + w4_fragment_bytes(K, N);
-      void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias};
+      void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias, &past};
       const int64_t tiles = (N + 15) / 16, groups = (M + 15) / 16;
       const int64_t most = groups > 1 ? std::max<int64_t>(cus / groups, 1) : M <= 4 || tiles > 3 * cus ? 2 * cus : cus;
       return launch(st, KernelName(block == 64 ? "mtrt_gemm_w4a16_strips16_b64" : "mtrt_gemm_w4a16_strips16"),

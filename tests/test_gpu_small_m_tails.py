@@ -105,3 +105,25 @@ def test_w4a16_strips_of_few_slices(pkg, M, block):
         _w4(torch, pkg, M, K, N, block, 10 * M + i)
         if torch.cuda.get_device_properties(0).multi_processor_count == 256:
             assert pkg.last_kernel() == "mtrt_gemm_w4a16_strips16" + ("_b64" if block == 64 else ""), (K, N)
+
+
+@pytest.mark.parametrize("M,K,N,block", [(4, 4096, 5120, 128), (4, 4096, 5121, 64), (1, 4096, 5137, 128), (8, 4096, 24577, 128), (16, 4096, 24576, 64),
+                                         (16, 4096, 24609, 128), (25, 4096, 24576, 64), (25, 4096, 24577, 64), (9, 4160, 24577, 64)])
+def test_w4a16_weights_past_the_caches(pkg, M, K, N, block):
+    """The kernels that read the weights once, at the largest weights that go through the caches and above."""
+    import torch
+    _w4(torch, pkg, M, K, N, block, M)
+    assert pkg.last_kernel().startswith("mtrt_gemm_w4a16_strips16" if M <= 16 and K % 128 == 0 else "mtrt_gemm_w4a16_skinny")
+
+
+@pytest.mark.parametrize("M,N", [(1, 12288), (9, 12288), (9, 12289), (16, 12353)])
+def test_w8a8_weights_past_the_caches(pkg, M, N):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    K = 4096
+    a = torch.randint(-128, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
+    w = torch.randint(-128, 128, (K, N), generator=g, device="cuda", dtype=torch.int8)
+    sa, sw = torch.rand(M, generator=g, device="cuda") * 0.01, torch.rand(N, generator=g, device="cuda") * 0.001
+    y = pkg.gemm_w8a8_fragments(a, pkg.gemm_w8a8_prepack_fragments(w), sa, sw, N)
+    acc = (a.double() @ w.double()).to(torch.int64).float()       # exact sums, one rounding to f32
+    assert torch.equal(y, ((acc * sa[:, None]) * sw[None, :]).half())
