@@ -27,6 +27,11 @@
 // of the whole tensor by itself (slow, same bits) and goes on, which frees its compute unit for the workgroups
 // still queued.  No workgroup ever depends on another one making progress.
 //
+// x is read through the caches, of which it takes a quarter at most: what the pass before has left in the Infinity Cache comes at twice the rate
+// at which loads past them bring it, and what lies in memory nearly as before.  us, past and through, tensors of three calls in turn, f32 -> i8 of
+// 4, 8, 17 and 67 MB 7.0, 6.4; 9.1, 8.1; 12.1, 11.3; 31.3, 29.2 (from memory 7.7, 7.1; 9.3, 9.4; 12.2, 12.4; 31.4, 32.1); bf16 -> i8 of 8 and 34 MB 9.4,
+// 8.5; 20.4, 19.1.
+//
 // scratch (the stream's reduction block, zero when the stream first uses it): lines 0..32 belong to the arrival
 // tree of amax.hip and are not touched here; lines 33..48 hold the 256 slots {tag, max bits}, line 49 the tag
 // counter.  Tags repeat after 2^32 launches.
@@ -81,7 +86,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
     const int64_t v = base + int64_t(i) * kDynThreads;
     xin[i] = (u32x4){0u, 0u, 0u, 0u};
     if (v < end) {
-      xin[i] = FG::load(x + v * G);
+      xin[i] = FG::template load<false>(x + v * G);
       const uint32_t a = A::of(xin[i]);
       m = m > a ? m : a;
     }
@@ -140,7 +145,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
       // gave up waiting: this workgroup reduces the whole tensor itself (max is exact in any order: same bits)
       uint32_t mm = 0;
       for (int64_t v = threadIdx.x; v < nvec; v += kDynThreads) {
-        const uint32_t a = A::of(FG::load(x + v * G));
+        const uint32_t a = A::of(FG::template load<false>(x + v * G));
         mm = mm > a ? mm : a;
       }
       total = block_max(mm, wave_max);
