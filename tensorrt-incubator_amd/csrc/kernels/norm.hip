@@ -79,7 +79,7 @@ template <> struct Vec<F16> {
 // the end of the row re-read the row's last vector and are replaced by `fill` afterwards), so the
 // loads are issued back to back with no branches between them; with FULL (the row fills all
 // 64 * NV vectors) the replacement disappears as well.
-template <typename X, int NV, bool FULL>
+template <typename X, int NV, bool FULL, bool PAST>
 __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec, int lane, float fill,
                                          float (&v)[NV * Vec<X>::kElems]) {
   constexpr int E = Vec<X>::kElems;
@@ -87,7 +87,8 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
-    t[j] = __builtin_nontemporal_load(row + (FULL ? idx : min(idx, nvec - 1)));
+    const u32x4* p = row + (FULL ? idx : min(idx, nvec - 1));
+    t[j] = PAST ? __builtin_nontemporal_load(p) : *p;
   }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -99,6 +100,15 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
     }
   }
 }
+
+// Up to which sizes rows are read through the caches: what the pass before has left in the Infinity Cache comes at twice the rate at which loads
+// past them bring it; larger tensors gain nothing, and would push other things out.  us, past and through, tensors of three calls in turn: softmax f32 of
+// 4, 8, 34, 50 and 67 MB 4.2, 3.9; 4.5, 3.9; 11.3, 10.5; 18.1, 15.3; 24.5, 19.9; bf16 12.2, 10.8 and 18.1, 15.6 for 34 and 50 MB; 101 MB 33.6,
+// 33.1; 134 MB 44.1, 46.3; from memory 34 to 67 MB take 2 to 4 % longer.  In between, where x and y together are what the L2s hold, neither is
+// ahead (17 MB: f32 6.3, 6.2, from memory 7.0, 7.2).  LayerNorm f32 of 1 to 8 MB 5.7 to 6.1, 4.9 to 5.2, bf16 of 4 and 8 MB 5.0, 4.5; 5.3, 4.6; 17 MB
+// f32 6.7, 8.3, bf16 6.6, 6.8; 134 MB f32 48.3, 49.2.
+__device__ __forceinline__ bool softmax_past(int64_t bytes) { return bytes > (int64_t(80) << 20) || (bytes > (int64_t(12) << 20) && bytes <= (int64_t(20) << 20)); }
+__device__ __forceinline__ bool layernorm_past(int64_t bytes) { return bytes > (int64_t(8) << 20); }
 
 // Hides a vector's provenance from the optimiser (no instruction is emitted).
 __device__ __forceinline__ void opaque(u32x4& t) { __asm__ volatile("" : "+v"(t)); }
@@ -118,7 +128,7 @@ __device__ __forceinline__ float row_reduce(float v, Op op) { return LDS ? wave_
 // occupancy it buys is worth more to this memory-bound kernel than the extra VALU work.
 // RESIDENT: the form held to 64 registers.  In f32 the exchanges need one more, which lay in private memory: by LDS there (us, f32 [5500,
 // 2048] 17.3, 16.5; [7000, 2048] 21.1, 20.3; [7000, 1100] 13.8, 13.1; [8192, 2048] 24.0, 23.5).
-template <typename X, int NV, bool FULL, bool RESIDENT>
+template <typename X, int NV, bool FULL, bool RESIDENT, bool PAST>
 __device__ __forceinline__ void layernorm_row(const typename X::storage* __restrict__ x,
                                               const typename X::storage* __restrict__ gamma,
                                               const typename X::storage* __restrict__ beta,
@@ -131,7 +141,8 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
-    t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+    const u32x4* p = xr + (FULL ? idx : min(idx, nvec - 1));
+    t[j] = PAST ? __builtin_nontemporal_load(p) : *p;
   }
 
   constexpr bool kLds = NV == 2 || NV == 4 || (NV == 1 && E == 8) || (RESIDENT && E == 4);
@@ -188,13 +199,15 @@ __device__ __forceinline__ void layernorm_rows(const typename X::storage* __rest
   // the wave index as a scalar: the row pointers are then wave-uniform and the accesses need one lane offset, not an address pair each
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;                           // whole wave leaves together
-  if (d == int64_t(Vec<X>::kElems) * kWave * NV)
-    layernorm_row<X, NV, true, RESIDENT>(x, gamma, beta, y, row, d, eps);
-  else
-    layernorm_row<X, NV, false, RESIDENT>(x, gamma, beta, y, row, d, eps);
+  past_or_through(layernorm_past(rows * d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
+    if (d == int64_t(Vec<X>::kElems) * kWave * NV)
+      layernorm_row<X, NV, true, RESIDENT, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps);
+    else
+      layernorm_row<X, NV, false, RESIDENT, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps);
+  });
 }
 
-template <typename X, int NV, bool FULL>
+template <typename X, int NV, bool FULL, bool PAST>
 __device__ __forceinline__ void softmax_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                             int64_t row, int64_t d) {
   constexpr int E = Vec<X>::kElems;
@@ -202,7 +215,7 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
   const int nvec = int(d / E);
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + row * d);
   float v[NV * E];
-  load_row<X, NV, FULL>(xr, nvec, lane, -INFINITY, v);
+  load_row<X, NV, FULL, PAST>(xr, nvec, lane, -INFINITY, v);
 
   constexpr bool kLds = NV == 2 || NV == 4;
   float mx = -INFINITY;
@@ -239,10 +252,12 @@ __device__ __forceinline__ void softmax_rows(const typename X::storage* __restri
   // the wave index as a scalar: the row pointers are then wave-uniform and the accesses need one lane offset, not an address pair each
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;
-  if (d == int64_t(Vec<X>::kElems) * kWave * NV)
-    softmax_row<X, NV, true>(x, y, row, d);
-  else
-    softmax_row<X, NV, false>(x, y, row, d);
+  past_or_through(softmax_past(rows * d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
+    if (d == int64_t(Vec<X>::kElems) * kWave * NV)
+      softmax_row<X, NV, true, decltype(past)::value>(x + zero, y, row, d);
+    else
+      softmax_row<X, NV, false, decltype(past)::value>(x + zero, y, row, d);
+  });
 }
 
 // ---- rows longer than one wave's registers, and rows of any length or alignment: a GROUP of lanes owns one row ----
@@ -280,7 +295,7 @@ __device__ __forceinline__ bool wave_has(int j, int nvec) {
   return ALL || (THREADS > kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.x & ~63u)) : 0) + THREADS * j < nvec;
 }
 
-template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED>
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED, bool PAST>
 __device__ __forceinline__ void layernorm_group_row(const typename X::storage* __restrict__ x,
                                                     const typename X::storage* __restrict__ gamma,
                                                     const typename X::storage* __restrict__ beta,
@@ -297,7 +312,7 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
     if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
     if (RAGGED && ALL && nvec == 0) t[j] = (u32x4){0u, 0u, 0u, 0u};   // a row shorter than one vector: only the scalar elements below
-    else t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+    else t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1))) : xr[FULL ? idx : min(idx, nvec - 1)];
   }
   const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
   const int64_t ec = int64_t(nvec) * E + lane;
@@ -371,16 +386,18 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
   __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-    layernorm_group_row<X, NV, THREADS, true, true, false>(x, gamma, beta, y, row, d, eps, lds);
-  else
-    layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED>(x, gamma, beta, y, row, d, eps, lds);
+  past_or_through(layernorm_past(rows * d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
+    if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
+      layernorm_group_row<X, NV, THREADS, true, true, false, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps, lds);
+    else
+      layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps, lds);
+  });
 }
 
 // KEEP: the exponentials stay in registers (f32) between the sum and the output pass; without it they are
 // computed again from the stored row (the 1024-lane form has 128 registers per lane, not enough for both where a lane holds
 // more than 64 elements).
-template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool KEEP, bool RAGGED>
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool KEEP, bool RAGGED, bool PAST>
 __device__ __forceinline__ void softmax_group_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                                   int64_t row, int64_t d, float* lds) {
   constexpr int E = Vec<X>::kElems;
@@ -394,7 +411,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
     if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
     if (!RAGGED || !ALL || nvec > 0)                  // (a row shorter than one vector: only the scalar elements below)
-      t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
+      t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1))) : xr[FULL ? idx : min(idx, nvec - 1)];
   }
   // What lies past the row becomes -infinity where it is loaded: it changes no maximum and its exponential is zero, and the passes
   // below need not tell it from the row (us, f16 [1084, 50000] 61.2 -> 53.0, f32 [2000, 25001] 102 -> 97, bf16 [200, 8191] 7.5 -> 7.1; [48000, 1500] as before).
@@ -466,10 +483,12 @@ __device__ __forceinline__ void softmax_group(const typename X::storage* __restr
   constexpr bool kKeep = THREADS <= 256 || NV * Vec<X>::kElems <= 64;
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-    softmax_group_row<X, NV, THREADS, true, true, kKeep, false>(x, y, row, d, lds);
-  else
-    softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED>(x, y, row, d, lds);
+  past_or_through(softmax_past(rows * d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
+    if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
+      softmax_group_row<X, NV, THREADS, true, true, kKeep, false, decltype(past)::value>(x + zero, y, row, d, lds);
+    else
+      softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED, decltype(past)::value>(x + zero, y, row, d, lds);
+  });
 }
 
 // ---- any D, any alignment: one workgroup per row, row re-read from cache -------------
