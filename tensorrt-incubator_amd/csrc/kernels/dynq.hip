@@ -60,7 +60,7 @@ __device__ __forceinline__ uint32_t block_max(uint32_t m, uint32_t* wave_max) {
 
 // ALONE: few workgroups, each reads the others' parts as well instead of waiting for their maxima.  (A body of its own: as a branch of
 // the other one it cost launches that wait 4 to 8 percent, codes alone, us: f32 of 2 Mi elements 8.7 -> 9.1, bf16 of 8 Mi 11.2 -> 11.8.)
-template <typename X, typename Q, int NV, bool ALONE>
+template <typename X, typename Q, int NV, bool ALONE, bool PAST>
 __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                             typename X::storage* __restrict__ y, int64_t n, float qmax,
                                             float* __restrict__ amax_out, float* __restrict__ scale_out,
@@ -178,9 +178,26 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
       if (y) {
 #pragma unroll
         for (int k = 0; k < G; ++k) f[k] = f[k] * scale;
-        FG::store(y + v * G, f);
+        FG::template store<PAST>(y + v * G, f);
       }
     }
+  }
+}
+
+// y of more than 36 MiB is left to the caches, whose write-back is then spread over the time that the next launch takes to read; a smaller one is
+// still dirty in the L2s when this launch ends, which waits for it.  us, past and left, x of 34, 42, 50, 59 and 67 MB, from memory as in turns of three:
+// f32 -> i8 17.2, 17.6; 20.2, 19.7; 23.4, 22.1; 26.5, 24.6; 29.5, 28.4; bf16 -> i8 19.1, 18.8; 22.4, 21.1; 26.1, 23.8; 29.6, 26.6; 32.5, 30.1.
+template <typename X, typename Q, int NV>
+__device__ __forceinline__ void dynqdq(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
+                                       typename X::storage* __restrict__ y, int64_t n, float qmax, float* __restrict__ amax_out,
+                                       float* __restrict__ scale_out, uint32_t* __restrict__ scratch, int flags, int spin_limit, int nv) {
+  if constexpr (NV == 4) {                             // (16 MiB at most)
+    if (spin_limit < 0) dynqdq_body<X, Q, NV, true, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);
+    else dynqdq_body<X, Q, NV, false, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);
+  } else {
+    past_or_through(n * int64_t(sizeof(typename X::storage)) <= (int64_t(36) << 20), [&](auto past, int64_t zero) {
+      dynqdq_body<X, Q, NV, false, decltype(past)::value>(x, q, y + zero, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);
+    });
   }
 }
 
@@ -194,10 +211,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
   extern "C" __global__ void __launch_bounds__(1024) mtrt_dynqdq_##XN##_##QN##_v##NV(                                  \
       const XT::storage* x, QT::storage* q, XT::storage* y, int64_t n, float qmax, float* amax_out, float* scale_out,  \
       uint32_t* scratch, int32_t flags, int32_t spin_limit, int32_t nv) {                                              \
-    if (NV == 4 && spin_limit < 0)                                                                                      \
-      dynq_cluster::dynqdq_body<XT, QT, 4, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);    \
-    else                                                                                                                \
-      dynq_cluster::dynqdq_body<XT, QT, NV, false>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv); }
+    dynq_cluster::dynqdq<XT, QT, NV>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv); }
 #define MTRT_DYNQ_KERNELS(XN, XT, QN, QT) MTRT_DYNQ_KERNEL(XN, XT, QN, QT, 4) MTRT_DYNQ_KERNEL(XN, XT, QN, QT, 16)
 MTRT_DYNQ_KERNELS(f32, F32, i8, I8)
 MTRT_DYNQ_KERNELS(f32, F32, f8, F8)

@@ -113,9 +113,9 @@ __device__ __forceinline__ bool layernorm_past(int64_t bytes) { return bytes > (
 // Where rows are read past the caches and what is written fills most of the Infinity Cache, but not more, it is left to the caches: its
 // write-back is then spread over the time that the next launch takes to read.  Smaller results are still dirty in the L2s when the launch ends, which
 // waits for them; larger ones push themselves out.  us, past and left, tensors of three calls in turn, much the same from memory: softmax f32 of
-// 101, 134 and 268 MB 36.2, 34.0; 47.4, 43.0; 93.3, 79.5; bf16 33.6, 32.5; 44.1, 41.6; 86.4, 78.2; f16 [12000, 9001] 84.1, 76.4, but [20000, 9001], 360 MB,
-// 139, 152; 17 to 34 MB 2 to 29 % longer; LayerNorm f32 of 101, 134 and 268 MB 37.9, 37.2; 48.3, 46.7; 93.5, 85.0; bf16 of 101, 134 and 268 MB 35.4, 36.4;
-// 46.4, 45.7; 90.3, 82.5; in the form held to 64 registers, whose waves all write at the end, bf16 of whole rows of 42, 59 and 67 MB 12.5, 13.5; 19.3, 18.7;
+// 101, 134 and 268 MB 36.0, 34.0; 47.4, 42.9; 93.4, 79.6; bf16 33.6, 32.6; 44.1, 41.6; 86.4, 78.2; f16 [12000, 9001] 84.1, 76.4, but [20000, 9001], 360 MB,
+// 139, 152; 17 to 34 MB 2 to 29 % longer; LayerNorm f32 of 101, 134 and 268 MB 37.9, 37.6; 48.2, 46.8; 93.4, 85.1; bf16 of 101, 134 and 268 MB 35.6, 36.7;
+// 46.6, 46.1; 89.9, 82.9; in the form held to 64 registers, whose waves all write at the end, bf16 of whole rows of 42, 59 and 67 MB 12.5, 13.5; 19.3, 18.7;
 // 22.0, 21.1 ([8192, 3500] 23.5, 24.1).
 constexpr int64_t kKeptAtMost = int64_t(272) << 20;
 __device__ __forceinline__ bool softmax_keep(int64_t bytes) { return bytes > (int64_t(80) << 20) && bytes <= kKeptAtMost; }

@@ -125,3 +125,14 @@ def test_bounded_wait_gives_up_cleanly_and_block_restores_itself(pkg, orc):
         assert torch.equal(torch.stack([a, s]).view(torch.int32), torch.stack([a1, s1]).view(torch.int32))
         q2, y2 = pkg.quantize_dequantize(xs, s.reshape(1), pkg.I8)
         assert torch.equal(q1, q2) and torch.equal(y1.view(torch.int32), y2.view(torch.int32))
+
+
+@pytest.mark.parametrize("xname,qname", [("f32", "i8"), ("f32", "f8"), ("bf16", "i8")])
+def test_results_past_the_caches_and_left_to_them(pkg, orc, xname, qname):
+    """The largest tensor whose result is stored past the caches, and one group more."""
+    grp, size = (4, 4) if xname == "f32" else (8, 2)
+    orc.set_threads(16)
+    for n in ((36 << 20) // size, (36 << 20) // size + grp):
+        x = (rng(n % 97).standard_normal(n, dtype=np.float32) * 3)
+        _check(pkg, orc, x, xname, qname, "mtrt_dynqdq_%s_%s_v16" % (xname, qname))
+    orc.set_threads(1)
