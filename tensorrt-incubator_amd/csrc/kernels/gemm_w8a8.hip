@@ -370,6 +370,25 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_small16(
   if (past) small_m::tiles<2, true>(a, w_frag, epi, y, M, K, N, lds);
   else small_m::tiles<2, false>(a, w_frag, epi, y, M, K, N, lds);
 }
+// ... M <= 32, the same arguments; grid = ceil(N / 32) or the number of compute units: which one stands beside the launch.  Against eight waves to
+// a tile that each bring their own rows, as in gemm_core::rows32 (there 64 rows still run so), us, (M, K, N), weights of three calls in turn: (32, 1152, 9216)
+// 7.0, 4.8; (17, 2048, 11008) 9.3, 7.6; (32, 4096, 11008) 13.2, 11.4; (32, 6144, 9216) 16.5, 13.7; (32, 8192, 11008) 24.7, 20.6; (17, 4096, 4096) 6.2, 5.9; from
+// memory 17.0, 13.6; 21.7, 17.6 for the third and fourth; up to 16 rows of few columns (1, 2688, 4096) 4.8, 3.8; (16, 8192, 2048) 7.8, 7.0; (8, 14336, 512) 9.4,
+// 7.3; the other way up to eight slices by no more tiles than units, (32, 640, 4096) 3.4, 3.6.
+extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_frag_rows32(
+    const int8_t* __restrict__ a, const v4i* __restrict__ w_frag, const float* __restrict__ a_scale,
+    const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t a_step,
+    const uint16_t* __restrict__ bias, int32_t past) {
+  __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 4 * 1024];
+  const RowsScaleEpilogue epi{a_scale, w_scale, a_step, bias};
+  if (M <= 16) {
+    if (past) small_m::tiles<2, true>(a, w_frag, epi, y, M, K, N, lds);
+    else small_m::tiles<2, false>(a, w_frag, epi, y, M, K, N, lds);
+  } else {
+    if (past) small_m::tiles<4, true>(a, w_frag, epi, y, M, K, N, lds);
+    else small_m::tiles<4, false>(a, w_frag, epi, y, M, K, N, lds);
+  }
+}
 // Any K (no alignment needs): one output element per lane, plain loops.  Only K = 0 is left to it (every
 // other shape runs on the matrix cores).
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_nk_any(
@@ -410,7 +429,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_nk_rows128(
   gemm_core::rows32::run<I8Traits, 4, 4>(a, w_nk, K, epi, y, M, N, lds);
 }
 
-// Up to 32 and 64 rows on fragment-order weights: the same kernels with the weight fragments straight from
+// Up to 64 rows on fragment-order weights: the same kernel with the weight fragments straight from
 // memory into registers.  (a [M,K] i8, w_frag, a_scale, w_scale, y, M, K, N, a_step, bias) ; K % 128 == 0, a and w_frag
 // 16-byte aligned; a_step and bias as for the tiles; grid: any, block = 512.
 #define MTRT_W8_FRAG_ROWS_KERNEL(NAME, MT)                                                                                \
@@ -422,7 +441,6 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_nk_rows128(
     RowsScaleEpilogue epi{a_scale, w_scale, a_step, bias};                                                                \
     gemm_core::rows32::run<I8Traits, 8, MT, true>(a, w_frag, K, epi, y, M, N, lds);                                       \
   }
-MTRT_W8_FRAG_ROWS_KERNEL(mtrt_gemm_w8a8_frag_rows32, 1)
 MTRT_W8_FRAG_ROWS_KERNEL(mtrt_gemm_w8a8_frag_rows64, 2)
 
 // ---- a decode step's Linear in ONE launch: f16 activations, quantized where they are used ------------------

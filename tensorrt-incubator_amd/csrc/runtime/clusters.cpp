@@ -1309,12 +1309,10 @@ int32_t mtrt_hip_gemm_w8a8_prepack_fragments(mtrt_stream_t stream, const void *w
 }
 
 namespace {
-// Which kernel a W8A8 call on fragment-order weights takes.  Up to 32 rows: the kernels bound by reading the weights once
-// (17 to 32 rows, and fewer when at most half of the compute units would get a 32-column tile and K is long, the wave-private kernel with
-// eight waves splitting K: M = 32 at (K, N) = (11008, 4096) 18.6 -> 12.9 us, M = 16 there 15.1 -> 11.7; with more tiles and
-// up to 16 rows the four-wave kernel with its hand-counted waits: M = 1 at (4096, 11008) 10.7 against 12.5 us.  Of few tiles, us, eight and four
-// waves, weights in the L2s (from memory): (1, 1024, 1024) 3.6, 3.6 (3.7, 3.4); (2, 2304, 704) 4.3, 3.5 (4.5, 3.9); (4, 2560, 1600) 4.4, 3.5 (4.7,
-// 4.5); (16, 3072, 2048) 4.6, 3.8 (5.2, 5.5); (12, 4224, 768) 5.2, 4.3 (5.7, 6.1); (5, 11392, 384) 8.2, 6.3 (8.6, 9.4).)
+// Which kernel a W8A8 call on fragment-order weights takes.  Up to 32 rows: the four-wave kernels that read the weights once, with LDS for 16 or
+// for 32 rows.  (Up to 16 rows that is the same body, which of the two matters only where units hold several workgroups: long K by few columns, where eight
+// waves to a tile once were ahead, keeps the larger one.  Eight waves and four, weights in turns of three sets, us: (1, 2688, 4096) 4.8, 3.8; (16, 8192,
+// 2048) 7.8, 7.0; (8, 14336, 512) 9.4, 7.3; before the weights went through the caches the four took 4.9, 8.9 and 7.3.)
 // 33 to 64 rows: the wave-private kernel or a tile, by estimate.  Above: the tile and K split frag_plan estimates fastest.
 constexpr int64_t kW8LongK = 2688;
 struct W8Plan {
@@ -1354,18 +1352,24 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
   W8Plan plan = w8_plan(M, K, N, units, true);
   if (plan.kind == W8Plan::kTile && !bind_split(st, stream, plan.tile, workspace, workspace_bytes))
     plan = w8_plan(M, K, N, units, false);
-  if (plan.kind == W8Plan::kSmall16) {
-    // one workgroup per 32-column tile, its four waves splitting K; between one and two tiles per compute unit one
-    // workgroup per unit instead, the first ones taking a second tile (as for the int4 weights)
-    const uint32_t grid = uint32_t(M > 8 && tiles32 > units && tiles32 <= 2 * units ? units : tiles32);
-    int32_t past = K * N > tuning::kWeightsPastBytes;
+  if (M <= 32 && tiles32 < (int64_t(1) << 24)) {
+    // One workgroup per 32-column tile, its four waves splitting K; between one and two tiles per compute unit one workgroup per unit
+    // instead, the first ones taking a second tile and the rows once for both: from 9 rows on (as for the int4 weights), and with more than 16
+    // rows where K is long for the tiles that are left over (us, a workgroup to a tile and to a unit: 32 rows, K = 1152 and 288 tiles 4.8, 5.5; 2048 and 288
+    // 8.0, 8.0, from memory 9.8, 9.1; 2048 and 344 8.1, 8.5; 4096 and 288 11.2, 10.6; 4096 and 444 12.5, 13.0; 6144 and 444 19.3, 18.2; 8192
+    // and 512 30.7, 30.4).
+    const bool over = tiles32 > units && tiles32 <= 2 * units;
+    const bool pairs = over && (M > 16 ? K >= 2048 && (tiles32 - units) * 8192 <= K * units : M > 8);
+    const uint32_t grid = uint32_t(pairs ? units : tiles32);
+    // more than 16 rows keep more on its way beside the weights: 58 to 90 MB through the caches and past them 11.8, 14.0; 14.3, 17.6; 21.0, 22.1,
+    // from memory 14.4, 14.3; 18.2, 17.9; 23.5, 22.1; 100 MB 19.9, 19.5
+    int32_t past = K * N > tuning::kWeightsPastBytes * (M > 16 ? 2 : 1);
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias, &past};
-    return launch(st, KernelName("mtrt_gemm_w8a8_small16"), grid, kBlock, stream, args);
+    return launch(st, KernelName(plan.kind == W8Plan::kSmall16 ? "mtrt_gemm_w8a8_small16" : "mtrt_gemm_w8a8_frag_rows32"), grid, kBlock, stream, args);
   }
-  if (plan.kind == W8Plan::kRows) {
+  if (M <= 64 && plan.kind != W8Plan::kTile) {
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
-    return launch(st, KernelName(M <= 32 ? "mtrt_gemm_w8a8_frag_rows32" : "mtrt_gemm_w8a8_frag_rows64"),
-                  uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), 512, stream, args);
+    return launch(st, KernelName("mtrt_gemm_w8a8_frag_rows64"), uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), 512, stream, args);
   }
   FragPlan &p = plan.tile;
   if (!p.tile)

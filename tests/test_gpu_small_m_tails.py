@@ -127,3 +127,21 @@ def test_w8a8_weights_past_the_caches(pkg, M, N):
     y = pkg.gemm_w8a8_fragments(a, pkg.gemm_w8a8_prepack_fragments(w), sa, sw, N)
     acc = (a.double() @ w.double()).to(torch.int64).float()       # exact sums, one rounding to f32
     assert torch.equal(y, ((acc * sa[:, None]) * sw[None, :]).half())
+
+
+@pytest.mark.parametrize("M", [17, 24, 25, 32])
+def test_w8a8_up_to_32_rows(pkg, M):
+    """Waves with no slice and every number of slices modulo four, at tiles below and above a workgroup to a unit, one workgroup to two tiles
+    and to one on both sides of its lines, more than two tiles to a unit, and weights on both sides of the line past the caches."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    shapes = [(128 * s, (40, 4100, 8200, 11008, 16390)[i % 5]) for i, s in enumerate((1, 2, 3, 4, 5, 6, 7, 9, 12, 13, 15, 16, 18, 23))]
+    shapes += [(2048, 10240), (2048, 10273), (4096, 12288), (4096, 12289), (8192, 16384), (8192, 16385), (4096, 24576), (4096, 24577)]
+    for K, N in shapes:
+        a = torch.randint(-128, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
+        w = torch.randint(-128, 128, (K, N), generator=g, device="cuda", dtype=torch.int8)
+        sa, sw = torch.rand(M, generator=g, device="cuda") * 0.01, torch.rand(N, generator=g, device="cuda") * 0.001
+        y = pkg.gemm_w8a8_fragments(a, pkg.gemm_w8a8_prepack_fragments(w), sa, sw, N)
+        assert pkg.last_kernel() == "mtrt_gemm_w8a8_frag_rows32"
+        acc = (a.double() @ w.double()).to(torch.int64).float()   # exact sums, one rounding to f32
+        assert torch.equal(y, ((acc * sa[:, None]) * sw[None, :]).half()), (M, K, N)
