@@ -110,31 +110,10 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
 __device__ __forceinline__ bool softmax_past(int64_t bytes) { return bytes > (int64_t(80) << 20) || (bytes > (int64_t(12) << 20) && bytes <= (int64_t(20) << 20)); }
 __device__ __forceinline__ bool layernorm_past(int64_t bytes) { return bytes > (int64_t(8) << 20); }
 
-// Where rows are read past the caches and what is written fills most of the Infinity Cache, but not more, it is left to the caches: its
-// write-back is then spread over the time that the next launch takes to read.  Smaller results are still dirty in the L2s when the launch ends, which
-// waits for them; larger ones push themselves out.  us, past and left, tensors of three calls in turn, much the same from memory: softmax f32 of
-// 101, 134 and 268 MB 36.0, 34.0; 47.4, 42.9; 93.4, 79.6; bf16 33.6, 32.6; 44.1, 41.6; 86.4, 78.2; f16 [12000, 9001] 84.1, 76.4, but [20000, 9001], 360 MB,
-// 139, 152; 17 to 34 MB 2 to 29 % longer; LayerNorm f32 of 101, 134 and 268 MB 37.9, 37.6; 48.2, 46.8; 93.4, 85.1; bf16 of 101, 134 and 268 MB 35.6, 36.7;
-// 46.6, 46.1; 89.9, 82.9; in the form held to 64 registers, whose waves all write at the end, bf16 of whole rows of 42, 59 and 67 MB 12.5, 13.5; 19.3, 18.7;
-// 22.0, 21.1 ([8192, 3500] 23.5, 24.1).
-constexpr int64_t kKeptAtMost = int64_t(272) << 20;
-__device__ __forceinline__ bool softmax_keep(int64_t bytes) { return bytes > (int64_t(80) << 20) && bytes <= kKeptAtMost; }
-template <int E>
-__device__ __forceinline__ bool layernorm_keep(int64_t bytes) { return bytes > (int64_t(E == 4 ? 88 : 112) << 20) && bytes <= kKeptAtMost; }
-// The three bodies: read through the caches; read past them; and written to them besides.  ALWAYS: the first one is not needed.
-template <bool ALWAYS = false, typename F>
-__device__ __forceinline__ void bodies(bool past, bool keep, F body) {
-  const auto read_past = [&](int64_t x_zero) {
-    past_or_through(!keep, [&](auto write_past, int64_t y_zero) { body(BoolC<true>{}, BoolC<!decltype(write_past)::value>{}, x_zero, y_zero); });
-  };
-  if constexpr (ALWAYS)
-    read_past(0);
-  else
-    past_or_through(past, [&](auto hint, int64_t x_zero) {
-      if constexpr (decltype(hint)::value) read_past(x_zero);
-      else body(BoolC<false>{}, BoolC<false>{}, 0, 0);
-    });
-}
+// What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back:
+// alone softmax bf16 of 134 MB 44.1 -> 46.8 us where each result has memory of its own, 44.3 -> 46.7 from memory, with a copy of 268 MB behind each 133.2 ->
+// 135.7, between the launches that make x and take y 128.7 -> 127.6; LayerNorm bf16 [8178, 4096] 22.6 -> 21.4, 23.0 -> 22.3, 113.6 -> 116.8, 62.0 -> 60.6; of 101 MB
+// 37.0 -> 39.0, 37.6 -> 39.3, 128.0 -> 132.1, 95.3 -> 96.4.)
 
 // Hides a vector's provenance from the optimiser (no instruction is emitted).
 __device__ __forceinline__ void opaque(u32x4& t) { __asm__ volatile("" : "+v"(t)); }
@@ -154,7 +133,7 @@ __device__ __forceinline__ float row_reduce(float v, Op op) { return LDS ? wave_
 // occupancy it buys is worth more to this memory-bound kernel than the extra VALU work.
 // RESIDENT: the form held to 64 registers.  In f32 the exchanges need one more, which lay in private memory: by LDS there (us, f32 [5500,
 // 2048] 17.3, 16.5; [7000, 2048] 21.1, 20.3; [7000, 1100] 13.8, 13.1; [8192, 2048] 24.0, 23.5).
-template <typename X, int NV, bool FULL, bool RESIDENT, bool PAST, bool KEEP_Y>
+template <typename X, int NV, bool FULL, bool RESIDENT, bool PAST>
 __device__ __forceinline__ void layernorm_row(const typename X::storage* __restrict__ x,
                                               const typename X::storage* __restrict__ gamma,
                                               const typename X::storage* __restrict__ beta,
@@ -213,10 +192,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
     Vec<X>::unpack(bv[idc], b);
 #pragma unroll
     for (int k = 0; k < E; ++k) o[k] = (((v[k] - mu) * rstd) * g[k]) + b[k];
-    if (FULL || idx < nvec) {
-      if (KEEP_Y) yr[idx] = Vec<X>::pack(o);
-      else __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
-    }
+    if (FULL || idx < nvec) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
 }
 
@@ -229,18 +205,17 @@ __device__ __forceinline__ void layernorm_rows(const typename X::storage* __rest
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;                           // whole wave leaves together
   const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  const bool full = d == int64_t(Vec<X>::kElems) * kWave * NV;
-  // (rows enough for the form held to 64 registers are always past layernorm_past's line)
-  const bool keep = RESIDENT ? Vec<X>::kElems == 8 && full && bytes > (int64_t(52) << 20) : layernorm_keep<Vec<X>::kElems>(bytes);
-  bodies<RESIDENT>(layernorm_past(bytes), keep, [&](auto past, auto keep, int64_t x_zero, int64_t y_zero) {
-    if (full)
-      layernorm_row<X, NV, true, RESIDENT, decltype(past)::value, decltype(keep)::value>(x + x_zero, gamma, beta, y + y_zero, row, d, eps);
+  const auto body = [&](auto past, int64_t zero) {
+    if (d == int64_t(Vec<X>::kElems) * kWave * NV)
+      layernorm_row<X, NV, true, RESIDENT, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps);
     else
-      layernorm_row<X, NV, false, RESIDENT, decltype(past)::value, decltype(keep)::value>(x + x_zero, gamma, beta, y + y_zero, row, d, eps);
-  });
+      layernorm_row<X, NV, false, RESIDENT, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps);
+  };
+  if constexpr (RESIDENT) body(BoolC<true>{}, 0);    // (rows enough for the form held to 64 registers are always past layernorm_past's line)
+  else past_or_through(layernorm_past(bytes), body);
 }
 
-template <typename X, int NV, bool FULL, bool PAST, bool KEEP_Y>
+template <typename X, int NV, bool FULL, bool PAST>
 __device__ __forceinline__ void softmax_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                             int64_t row, int64_t d) {
   constexpr int E = Vec<X>::kElems;
@@ -275,10 +250,7 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
     float o[E];
 #pragma unroll
     for (int k = 0; k < E; ++k) o[k] = v[j * E + k] * inv;
-    if (FULL || idx < nvec) {
-      if (KEEP_Y) yr[idx] = Vec<X>::pack(o);
-      else __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
-    }
+    if (FULL || idx < nvec) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
 }
 
@@ -289,11 +261,11 @@ __device__ __forceinline__ void softmax_rows(const typename X::storage* __restri
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;
   const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  bodies(softmax_past(bytes), softmax_keep(bytes), [&](auto past, auto keep, int64_t x_zero, int64_t y_zero) {
+  past_or_through(softmax_past(bytes), [&](auto past, int64_t zero) {
     if (d == int64_t(Vec<X>::kElems) * kWave * NV)
-      softmax_row<X, NV, true, decltype(past)::value, decltype(keep)::value>(x + x_zero, y + y_zero, row, d);
+      softmax_row<X, NV, true, decltype(past)::value>(x + zero, y, row, d);
     else
-      softmax_row<X, NV, false, decltype(past)::value, decltype(keep)::value>(x + x_zero, y + y_zero, row, d);
+      softmax_row<X, NV, false, decltype(past)::value>(x + zero, y, row, d);
   });
 }
 
@@ -332,7 +304,7 @@ __device__ __forceinline__ bool wave_has(int j, int nvec) {
   return ALL || (THREADS > kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.x & ~63u)) : 0) + THREADS * j < nvec;
 }
 
-template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED, bool PAST, bool KEEP_Y>
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED, bool PAST>
 __device__ __forceinline__ void layernorm_group_row(const typename X::storage* __restrict__ x,
                                                     const typename X::storage* __restrict__ gamma,
                                                     const typename X::storage* __restrict__ beta,
@@ -398,10 +370,7 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
     Vec<X>::unpack(bv[idc], b);
 #pragma unroll
     for (int k = 0; k < E; ++k) o[k] = (((v[k] - mu) * rstd) * g[k]) + b[k];
-    if (FULL || idx < nvec) {
-      if (KEEP_Y) yr[idx] = Vec<X>::pack(o);
-      else __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
-    }
+    if (FULL || idx < nvec) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
   if (extra)
     Tile<X>::store1(y + row * d + ec, (((xe - mu) * rstd) * Tile<X>::load1(gamma + ec)) + Tile<X>::load1(beta + ec));
@@ -427,18 +396,18 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
   const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  bodies(layernorm_past(bytes), layernorm_keep<Vec<X>::kElems>(bytes), [&](auto past, auto keep, int64_t x_zero, int64_t y_zero) {
+  past_or_through(layernorm_past(bytes), [&](auto past, int64_t zero) {
     if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-      layernorm_group_row<X, NV, THREADS, true, true, false, decltype(past)::value, decltype(keep)::value>(x + x_zero, gamma, beta, y + y_zero, row, d, eps, lds);
+      layernorm_group_row<X, NV, THREADS, true, true, false, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps, lds);
     else
-      layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED, decltype(past)::value, decltype(keep)::value>(x + x_zero, gamma, beta, y + y_zero, row, d, eps, lds);
+      layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps, lds);
   });
 }
 
 // KEEP: the exponentials stay in registers (f32) between the sum and the output pass; without it they are
 // computed again from the stored row (the 1024-lane form has 128 registers per lane, not enough for both where a lane holds
 // more than 64 elements).
-template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool KEEP, bool RAGGED, bool PAST, bool KEEP_Y>
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool KEEP, bool RAGGED, bool PAST>
 __device__ __forceinline__ void softmax_group_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                                   int64_t row, int64_t d, float* lds) {
   constexpr int E = Vec<X>::kElems;
@@ -512,10 +481,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
 #pragma unroll
       for (int k = 0; k < E; ++k) o[k] = __expf(v[k] - mx) * inv;
     }
-    if (FULL || idx < nvec) {
-      if (KEEP_Y) yr[idx] = Vec<X>::pack(o);
-      else __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
-    }
+    if (FULL || idx < nvec) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
   if (extra) Tile<X>::store1(y + row * d + ec, ee * inv);
 }
@@ -528,11 +494,11 @@ __device__ __forceinline__ void softmax_group(const typename X::storage* __restr
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
   const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  bodies(softmax_past(bytes), softmax_keep(bytes), [&](auto past, auto keep, int64_t x_zero, int64_t y_zero) {
+  past_or_through(softmax_past(bytes), [&](auto past, int64_t zero) {
     if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-      softmax_group_row<X, NV, THREADS, true, true, kKeep, false, decltype(past)::value, decltype(keep)::value>(x + x_zero, y + y_zero, row, d, lds);
+      softmax_group_row<X, NV, THREADS, true, true, kKeep, false, decltype(past)::value>(x + zero, y, row, d, lds);
     else
-      softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED, decltype(past)::value, decltype(keep)::value>(x + x_zero, y + y_zero, row, d, lds);
+      softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED, decltype(past)::value>(x + zero, y, row, d, lds);
   });
 }
 

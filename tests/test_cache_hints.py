@@ -1,0 +1,48 @@
+"""Which loads and stores of the compiled kernels go past the caches, from their instructions: results do not depend on it, so that a hint that the
+compiler drops, or a line between two bodies that it folds into one, is seen nowhere else."""
+import collections
+import os
+import re
+import subprocess
+
+import pytest
+
+
+@pytest.fixture(scope="module")
+def code(pkg, tmp_path_factory):
+    """names(pattern) of the module's kernels, and accesses(names): kernel -> Counter of (mnemonic, past the caches)."""
+    llvm, folder = "/opt/rocm/llvm/bin/", tmp_path_factory.mktemp("code")
+    module, out = os.path.join(os.path.dirname(pkg.__file__), "lib", "mtrt_kernels.hsaco"), str(folder / "kernels.elf")
+    if not os.path.exists(llvm + "llvm-objdump"):
+        pytest.skip("no LLVM tools beside the compiler")
+
+    def run(tool, *args):
+        return subprocess.run([llvm + tool] + list(args), capture_output=True, text=True, check=True).stdout
+    target = next(t for t in run("clang-offload-bundler", "--list", "--type=o", "--input=" + module).split() if "gfx950" in t)
+    run("clang-offload-bundler", "--unbundle", "--type=o", "--targets=" + target, "--input=" + module, "--output=" + out)
+    everything = sorted(set(re.findall(r"\bFUNC\s+\S+\s+\S+\s+\S+\s+(mtrt_\S+)", run("llvm-readelf", "-sW", out))))
+
+    def names(pattern):
+        return [n for n in everything if re.fullmatch(pattern, n)]
+
+    def accesses(kernels):
+        found, kernel = {}, None
+        for line in run("llvm-objdump", "-d", "--no-show-raw-insn", "--disassemble-symbols=" + ",".join(kernels), out).splitlines():
+            head = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+            if head:
+                kernel = found.setdefault(head.group(1), collections.Counter())
+            access = re.match(r"\s+(global_(?:load|store)_\w+)\s", line)
+            if access:
+                kernel[access.group(1), re.search(r"\snt\b", line.split("//")[0]) is not None] += 1
+        assert sorted(found) == sorted(kernels)
+        return found
+    return names, accesses
+
+
+def test_rows_held_in_registers_are_written_past_the_caches(code):
+    names, accesses = code
+    kernels = names(r"mtrt_(layernorm|softmax)_\w+_[vgu]\d+(v\d+)?[rea]?")
+    assert len(kernels) > 130
+    folded = {"mtrt_softmax_f32_v1", "mtrt_softmax_bf16_v1"}         # whole rows of up to 64 vectors: the compiler makes one store of two branches
+    for kernel, found in accesses(kernels).items():
+        assert found["global_store_dwordx4", True] > 0 and (found["global_store_dwordx4", False] == 0 or kernel in folded), kernel
