@@ -31,6 +31,10 @@
 // at which loads past them bring it, and what lies in memory nearly as before.  us, past and through, tensors of three calls in turn, f32 -> i8 of
 // 4, 8, 17 and 67 MB 7.0, 6.4; 9.1, 8.1; 12.1, 11.3; 31.3, 29.2 (from memory 7.7, 7.1; 9.3, 9.4; 12.2, 12.4; 31.4, 32.1); bf16 -> i8 of 8 and 34 MB 9.4,
 // 8.5; 20.4, 19.1.
+// What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back.  us, past
+// and left, x of 42, 50, 59 and 67 MB, three results in turn and each with memory of its own, f32 -> i8 20.3, 19.8; 23.5, 27.2; 26.7, 33.0; 29.6, 33.2 and 22.7,
+// 25.2; 25.8, 29.3; 29.9, 33.3; 33.0, 33.9; bf16 -> i8 22.2, 24.4; 26.2, 29.1; 29.6, 34.0; 32.6, 35.9 and 25.1, 26.5; 28.7, 31.2; 33.0, 34.0; 36.3, 36.9.  With a
+// launch that makes x in front and one that reads y behind it is the other way, all three f32 53.6, 52.1; 62.0, 57.2; 71.1, 67.8; 78.6, 76.7.)
 //
 // scratch (the stream's reduction block, zero when the stream first uses it): lines 0..32 belong to the arrival
 // tree of amax.hip and are not touched here; lines 33..48 hold the 256 slots {tag, max bits}, line 49 the tag
@@ -60,7 +64,7 @@ __device__ __forceinline__ uint32_t block_max(uint32_t m, uint32_t* wave_max) {
 
 // ALONE: few workgroups, each reads the others' parts as well instead of waiting for their maxima.  (A body of its own: as a branch of
 // the other one it cost launches that wait 4 to 8 percent, codes alone, us: f32 of 2 Mi elements 8.7 -> 9.1, bf16 of 8 Mi 11.2 -> 11.8.)
-template <typename X, typename Q, int NV, bool ALONE, bool PAST>
+template <typename X, typename Q, int NV, bool ALONE>
 __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
                                             typename X::storage* __restrict__ y, int64_t n, float qmax,
                                             float* __restrict__ amax_out, float* __restrict__ scale_out,
@@ -178,26 +182,9 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
       if (y) {
 #pragma unroll
         for (int k = 0; k < G; ++k) f[k] = f[k] * scale;
-        FG::template store<PAST>(y + v * G, f);
+        FG::store(y + v * G, f);
       }
     }
-  }
-}
-
-// y of more than 36 MiB is left to the caches, whose write-back is then spread over the time that the next launch takes to read; a smaller one is
-// still dirty in the L2s when this launch ends, which waits for it.  us, past and left, x of 34, 42, 50, 59 and 67 MB, from memory as in turns of three:
-// f32 -> i8 17.2, 17.6; 20.2, 19.7; 23.4, 22.1; 26.5, 24.6; 29.5, 28.4; bf16 -> i8 19.1, 18.8; 22.4, 21.1; 26.1, 23.8; 29.6, 26.6; 32.5, 30.1.
-template <typename X, typename Q, int NV>
-__device__ __forceinline__ void dynqdq(const typename X::storage* __restrict__ x, typename Q::storage* __restrict__ q,
-                                       typename X::storage* __restrict__ y, int64_t n, float qmax, float* __restrict__ amax_out,
-                                       float* __restrict__ scale_out, uint32_t* __restrict__ scratch, int flags, int spin_limit, int nv) {
-  if constexpr (NV == 4) {                             // (16 MiB at most)
-    if (spin_limit < 0) dynqdq_body<X, Q, NV, true, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);
-    else dynqdq_body<X, Q, NV, false, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);
-  } else {
-    past_or_through(n * int64_t(sizeof(typename X::storage)) <= (int64_t(36) << 20), [&](auto past, int64_t zero) {
-      dynqdq_body<X, Q, NV, false, decltype(past)::value>(x, q, y + zero, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);
-    });
   }
 }
 
@@ -211,7 +198,10 @@ __device__ __forceinline__ void dynqdq(const typename X::storage* __restrict__ x
   extern "C" __global__ void __launch_bounds__(1024) mtrt_dynqdq_##XN##_##QN##_v##NV(                                  \
       const XT::storage* x, QT::storage* q, XT::storage* y, int64_t n, float qmax, float* amax_out, float* scale_out,  \
       uint32_t* scratch, int32_t flags, int32_t spin_limit, int32_t nv) {                                              \
-    dynq_cluster::dynqdq<XT, QT, NV>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv); }
+    if (NV == 4 && spin_limit < 0)                                                                                      \
+      dynq_cluster::dynqdq_body<XT, QT, 4, true>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv);    \
+    else                                                                                                                \
+      dynq_cluster::dynqdq_body<XT, QT, NV, false>(x, q, y, n, qmax, amax_out, scale_out, scratch, flags, spin_limit, nv); }
 #define MTRT_DYNQ_KERNELS(XN, XT, QN, QT) MTRT_DYNQ_KERNEL(XN, XT, QN, QT, 4) MTRT_DYNQ_KERNEL(XN, XT, QN, QT, 16)
 MTRT_DYNQ_KERNELS(f32, F32, i8, I8)
 MTRT_DYNQ_KERNELS(f32, F32, f8, F8)

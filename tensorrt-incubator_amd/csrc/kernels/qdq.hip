@@ -48,11 +48,9 @@ template <> struct FloatGroup<F32> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] = bits_to_f32(t[k]);
   }
-  template <bool PAST = true>
   static __device__ __forceinline__ void store(float* p, const float (&v)[4]) {
     u32x4 t = {f32_to_bits(v[0]), f32_to_bits(v[1]), f32_to_bits(v[2]), f32_to_bits(v[3])};
-    if (PAST) __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
-    else *reinterpret_cast<u32x4*>(p) = t;
+    __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
   }
 };
 template <> struct FloatGroup<BF16> {
@@ -65,13 +63,11 @@ template <> struct FloatGroup<BF16> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) { v[2 * k] = bits_to_f32(t[k] << 16); v[2 * k + 1] = bits_to_f32(t[k] & 0xFFFF0000u); }
   }
-  template <bool PAST = true>
   static __device__ __forceinline__ void store(uint16_t* p, const float (&v)[8]) {
     u32x4 t;
 #pragma unroll
     for (int k = 0; k < 4; ++k) t[k] = f32x2_to_bf16x2_bits(v[2 * k], v[2 * k + 1]);
-    if (PAST) __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
-    else *reinterpret_cast<u32x4*>(p) = t;
+    __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
   }
 };
 template <> struct FloatGroup<F16> {
@@ -84,13 +80,11 @@ template <> struct FloatGroup<F16> {
 #pragma unroll
     for (int k = 0; k < 4; ++k) { v[2 * k] = f16_bits_to_f32(t[k] & 0xFFFFu); v[2 * k + 1] = f16_bits_to_f32(t[k] >> 16); }
   }
-  template <bool PAST = true>
   static __device__ __forceinline__ void store(uint16_t* p, const float (&v)[8]) {
     u32x4 t;
 #pragma unroll
     for (int k = 0; k < 4; ++k) t[k] = f32x2_to_f16x2_bits(v[2 * k], v[2 * k + 1]);
-    if (PAST) __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
-    else *reinterpret_cast<u32x4*>(p) = t;
+    __builtin_nontemporal_store(t, reinterpret_cast<u32x4*>(p));
   }
 };
 

@@ -46,3 +46,13 @@ def test_rows_held_in_registers_are_written_past_the_caches(code):
     folded = {"mtrt_softmax_f32_v1", "mtrt_softmax_bf16_v1"}         # whole rows of up to 64 vectors: the compiler makes one store of two branches
     for kernel, found in accesses(kernels).items():
         assert found["global_store_dwordx4", True] > 0 and (found["global_store_dwordx4", False] == 0 or kernel in folded), kernel
+
+
+def test_one_launch_dynamic_quantization_writes_past_the_caches(code):
+    """Codes and dequantized values; what the workgroups tell each other is one word or two."""
+    names, accesses = code
+    kernels = names(r"mtrt_dynqdq_\w+")
+    assert len(kernels) == 10
+    for kernel, found in accesses(kernels).items():
+        assert found["global_store_dwordx4", True] > 0 and found["global_store_dwordx4", False] == 0, kernel
+        assert found["global_store_dwordx2" if "f16" in kernel else "global_store_dword", True] > 0, kernel

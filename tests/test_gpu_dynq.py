@@ -128,8 +128,8 @@ def test_bounded_wait_gives_up_cleanly_and_block_restores_itself(pkg, orc):
 
 
 @pytest.mark.parametrize("xname,qname", [("f32", "i8"), ("f32", "f8"), ("bf16", "i8")])
-def test_results_past_the_caches_and_left_to_them(pkg, orc, xname, qname):
-    """The largest tensor whose result is stored past the caches, and one group more."""
+def test_tensors_of_36_mib(pkg, orc, xname, qname):
+    """... and one group more: the last workgroup's part is whole, or a single group."""
     grp, size = (4, 4) if xname == "f32" else (8, 2)
     orc.set_threads(16)
     for n in ((36 << 20) // size, (36 << 20) // size + grp):
