@@ -27,10 +27,10 @@
 // of the whole tensor by itself (slow, same bits) and goes on, which frees its compute unit for the workgroups
 // still queued.  No workgroup ever depends on another one making progress.
 //
-// x is read through the caches, of which it takes a quarter at most: what the pass before has left in the Infinity Cache comes at twice the rate
-// at which loads past them bring it, and what lies in memory nearly as before.  us, past and through, tensors of three calls in turn, f32 -> i8 of
-// 4, 8, 17 and 67 MB 7.0, 6.4; 9.1, 8.1; 12.1, 11.3; 31.3, 29.2 (from memory 7.7, 7.1; 9.3, 9.4; 12.2, 12.4; 31.4, 32.1); bf16 -> i8 of 8 and 34 MB 9.4,
-// 8.5; 20.4, 19.1.
+// x is read past the caches.  (Through them it is the shorter only where an earlier launch of the same tensor has left it there.  us, past and through, three
+// tensors in turn; each from memory; with a launch that makes x in front and one that reads y behind, all three: f32 -> i8 of 4 MB 6.0, 6.0; 7.3, 7.8; 13.0,
+// 13.2; 17 MB 11.9, 11.6; 12.4, 13.0; 27.3, 28.4; 34 MB 18.4, 17.4; 18.9, 19.5; 43.2, 45.4; 67 MB 31.2, 29.6; 31.9, 33.0; 76.4, 78.6; bf16 -> i8 of 8 MB 8.3, 8.0;
+// 9.4, 9.6; 18.3, 18.5; 34 MB 20.4, 19.1; 21.0, 21.3; 45.2, 46.9.)
 // What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back.  us, past
 // and left, x of 42, 50, 59 and 67 MB, three results in turn and each with memory of its own, f32 -> i8 20.3, 19.8; 23.5, 27.2; 26.7, 33.0; 29.6, 33.2 and 22.7,
 // 25.2; 25.8, 29.3; 29.9, 33.3; 33.0, 33.9; bf16 -> i8 22.2, 24.4; 26.2, 29.1; 29.6, 34.0; 32.6, 35.9 and 25.1, 26.5; 28.7, 31.2; 33.0, 34.0; 36.3, 36.9.  With a
@@ -90,7 +90,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
     const int64_t v = base + int64_t(i) * kDynThreads;
     xin[i] = (u32x4){0u, 0u, 0u, 0u};
     if (v < end) {
-      xin[i] = FG::template load<false>(x + v * G);
+      xin[i] = FG::load(x + v * G);
       const uint32_t a = A::of(xin[i]);
       m = m > a ? m : a;
     }
@@ -149,7 +149,7 @@ __device__ __forceinline__ void dynqdq_body(const typename X::storage* __restric
       // gave up waiting: this workgroup reduces the whole tensor itself (max is exact in any order: same bits)
       uint32_t mm = 0;
       for (int64_t v = threadIdx.x; v < nvec; v += kDynThreads) {
-        const uint32_t a = A::of(FG::template load<false>(x + v * G));
+        const uint32_t a = A::of(FG::load(x + v * G));
         mm = mm > a ? mm : a;
       }
       total = block_max(mm, wave_max);

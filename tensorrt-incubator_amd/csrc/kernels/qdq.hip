@@ -40,10 +40,7 @@ namespace qdq_cluster {
 template <typename X> struct FloatGroup;
 template <> struct FloatGroup<F32> {
   static constexpr int G = 4;
-  template <bool PAST = true>                          // past the caches, or through them
-  static __device__ __forceinline__ u32x4 load(const float* p) {
-    return PAST ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)) : *reinterpret_cast<const u32x4*>(p);
-  }
+  static __device__ __forceinline__ u32x4 load(const float* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
   static __device__ __forceinline__ void unpack(u32x4 t, float (&v)[4]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) v[k] = bits_to_f32(t[k]);
@@ -55,10 +52,7 @@ template <> struct FloatGroup<F32> {
 };
 template <> struct FloatGroup<BF16> {
   static constexpr int G = 8;
-  template <bool PAST = true>                          // past the caches, or through them
-  static __device__ __forceinline__ u32x4 load(const uint16_t* p) {
-    return PAST ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)) : *reinterpret_cast<const u32x4*>(p);
-  }
+  static __device__ __forceinline__ u32x4 load(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
   static __device__ __forceinline__ void unpack(u32x4 t, float (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) { v[2 * k] = bits_to_f32(t[k] << 16); v[2 * k + 1] = bits_to_f32(t[k] & 0xFFFF0000u); }
@@ -72,10 +66,7 @@ template <> struct FloatGroup<BF16> {
 };
 template <> struct FloatGroup<F16> {
   static constexpr int G = 8;
-  template <bool PAST = true>                          // past the caches, or through them
-  static __device__ __forceinline__ u32x4 load(const uint16_t* p) {
-    return PAST ? __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)) : *reinterpret_cast<const u32x4*>(p);
-  }
+  static __device__ __forceinline__ u32x4 load(const uint16_t* p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p)); }
   static __device__ __forceinline__ void unpack(u32x4 t, float (&v)[8]) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) { v[2 * k] = f16_bits_to_f32(t[k] & 0xFFFFu); v[2 * k + 1] = f16_bits_to_f32(t[k] >> 16); }

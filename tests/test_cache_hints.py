@@ -48,11 +48,13 @@ def test_rows_held_in_registers_are_written_past_the_caches(code):
         assert found["global_store_dwordx4", True] > 0 and (found["global_store_dwordx4", False] == 0 or kernel in folded), kernel
 
 
-def test_one_launch_dynamic_quantization_writes_past_the_caches(code):
-    """Codes and dequantized values; what the workgroups tell each other is one word or two."""
+def test_one_launch_dynamic_quantization_passes_the_caches_by(code):
+    """The tensor, codes and dequantized values; what the workgroups tell each other is one word or two.  In the four-vector kernels a few workgroups
+    each read the others' parts from the caches as well."""
     names, accesses = code
     kernels = names(r"mtrt_dynqdq_\w+")
     assert len(kernels) == 10
     for kernel, found in accesses(kernels).items():
         assert found["global_store_dwordx4", True] > 0 and found["global_store_dwordx4", False] == 0, kernel
         assert found["global_store_dwordx2" if "f16" in kernel else "global_store_dword", True] > 0, kernel
+        assert found["global_load_dwordx4", True] > 0 and found["global_load_dwordx4", False] == (4 if kernel.endswith("_v4") else 0), kernel
