@@ -101,14 +101,15 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
   }
 }
 
-// Up to which sizes rows are read through the caches: what the pass before has left in the Infinity Cache comes at twice the rate at which loads
+// Up to which sizes softmax reads rows through the caches: what the pass before has left in the Infinity Cache comes at twice the rate at which loads
 // past them bring it; larger tensors gain nothing, and would push other things out.  us, past and through, tensors of three calls in turn: softmax f32 of
 // 4, 8, 34, 50 and 67 MB 4.2, 3.9; 4.5, 3.9; 11.3, 10.5; 18.1, 15.3; 24.5, 19.9; bf16 12.2, 10.8 and 18.1, 15.6 for 34 and 50 MB; 101 MB 33.6,
 // 33.1; 134 MB 44.1, 46.3; from memory 34 to 67 MB take 2 to 4 % longer.  In between, where x and y together are what the L2s hold, neither is
-// ahead (17 MB: f32 6.3, 6.2, from memory 7.0, 7.2).  LayerNorm f32 of 1 to 8 MB 5.7 to 6.1, 4.9 to 5.2, bf16 of 4 and 8 MB 5.0, 4.5; 5.3, 4.6; 17 MB
-// f32 6.7, 8.3, bf16 6.6, 6.8; 134 MB f32 48.3, 49.2.
+// ahead (17 MB: f32 6.3, 6.2, from memory 7.0, 7.2).
+// LayerNorm reads past the caches always.  (us, past and through, three tensors in turn; each from memory; with a launch that makes x in front and one that
+// reads y behind, all three: f32 [256, 4096] 4.8, 4.8; 5.8, 6.2; 11.9, 12.0; [512, 4096] 5.2, 5.2; 6.1, 6.5; 16.7, 17.5; bf16 [512, 4096] 4.4, 4.4; 5.0, 5.4;
+// 11.7, 11.9; [1024, 4096] 4.5, 4.6; 5.6, 6.0; 15.0, 15.4; f16 [2796, 1500] 5.7, 5.5; 6.5, 6.5; 21.3, 21.7; bf16 [250, 14165] 6.6, 6.4; 7.2, 7.5; 16.3, 16.6.)
 __device__ __forceinline__ bool softmax_past(int64_t bytes) { return bytes > (int64_t(80) << 20) || (bytes > (int64_t(12) << 20) && bytes <= (int64_t(20) << 20)); }
-__device__ __forceinline__ bool layernorm_past(int64_t bytes) { return bytes > (int64_t(8) << 20); }
 
 // What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back:
 // alone softmax bf16 of 134 MB 44.1 -> 46.8 us where each result has memory of its own, 44.3 -> 46.7 from memory, with a copy of 268 MB behind each 133.2 ->
@@ -133,7 +134,7 @@ __device__ __forceinline__ float row_reduce(float v, Op op) { return LDS ? wave_
 // occupancy it buys is worth more to this memory-bound kernel than the extra VALU work.
 // RESIDENT: the form held to 64 registers.  In f32 the exchanges need one more, which lay in private memory: by LDS there (us, f32 [5500,
 // 2048] 17.3, 16.5; [7000, 2048] 21.1, 20.3; [7000, 1100] 13.8, 13.1; [8192, 2048] 24.0, 23.5).
-template <typename X, int NV, bool FULL, bool RESIDENT, bool PAST>
+template <typename X, int NV, bool FULL, bool RESIDENT>
 __device__ __forceinline__ void layernorm_row(const typename X::storage* __restrict__ x,
                                               const typename X::storage* __restrict__ gamma,
                                               const typename X::storage* __restrict__ beta,
@@ -146,8 +147,7 @@ __device__ __forceinline__ void layernorm_row(const typename X::storage* __restr
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
-    const u32x4* p = xr + (FULL ? idx : min(idx, nvec - 1));
-    t[j] = PAST ? __builtin_nontemporal_load(p) : *p;
+    t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
 
   constexpr bool kLds = NV == 2 || NV == 4 || (NV == 1 && E == 8) || (RESIDENT && E == 4);
@@ -204,15 +204,10 @@ __device__ __forceinline__ void layernorm_rows(const typename X::storage* __rest
   // the wave index as a scalar: the row pointers are then wave-uniform and the accesses need one lane offset, not an address pair each
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;                           // whole wave leaves together
-  const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  const auto body = [&](auto past, int64_t zero) {
-    if (d == int64_t(Vec<X>::kElems) * kWave * NV)
-      layernorm_row<X, NV, true, RESIDENT, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps);
-    else
-      layernorm_row<X, NV, false, RESIDENT, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps);
-  };
-  if constexpr (RESIDENT) body(BoolC<true>{}, 0);    // (rows enough for the form held to 64 registers are always past layernorm_past's line)
-  else past_or_through(layernorm_past(bytes), body);
+  if (d == int64_t(Vec<X>::kElems) * kWave * NV)
+    layernorm_row<X, NV, true, RESIDENT>(x, gamma, beta, y, row, d, eps);
+  else
+    layernorm_row<X, NV, false, RESIDENT>(x, gamma, beta, y, row, d, eps);
 }
 
 template <typename X, int NV, bool FULL, bool PAST>
@@ -304,7 +299,7 @@ __device__ __forceinline__ bool wave_has(int j, int nvec) {
   return ALL || (THREADS > kWave ? __builtin_amdgcn_readfirstlane(int(threadIdx.x & ~63u)) : 0) + THREADS * j < nvec;
 }
 
-template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED, bool PAST>
+template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool RAGGED>
 __device__ __forceinline__ void layernorm_group_row(const typename X::storage* __restrict__ x,
                                                     const typename X::storage* __restrict__ gamma,
                                                     const typename X::storage* __restrict__ beta,
@@ -321,7 +316,7 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
     if (!wave_has<THREADS, ALL>(j, nvec)) break;
     const int idx = lane + THREADS * j;
     if (RAGGED && ALL && nvec == 0) t[j] = (u32x4){0u, 0u, 0u, 0u};   // a row shorter than one vector: only the scalar elements below
-    else t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1))) : xr[FULL ? idx : min(idx, nvec - 1)];
+    else t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
   const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
   const int64_t ec = int64_t(nvec) * E + lane;
@@ -395,13 +390,10 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
   __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  past_or_through(layernorm_past(bytes), [&](auto past, int64_t zero) {
-    if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-      layernorm_group_row<X, NV, THREADS, true, true, false, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps, lds);
-    else
-      layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED, decltype(past)::value>(x + zero, gamma, beta, y, row, d, eps, lds);
-  });
+  if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
+    layernorm_group_row<X, NV, THREADS, true, true, false>(x, gamma, beta, y, row, d, eps, lds);
+  else
+    layernorm_group_row<X, NV, THREADS, false, !ENDS, RAGGED>(x, gamma, beta, y, row, d, eps, lds);
 }
 
 // KEEP: the exponentials stay in registers (f32) between the sum and the output pass; without it they are

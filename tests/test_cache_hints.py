@@ -58,3 +58,13 @@ def test_one_launch_dynamic_quantization_passes_the_caches_by(code):
         assert found["global_store_dwordx4", True] > 0 and found["global_store_dwordx4", False] == 0, kernel
         assert found["global_store_dwordx2" if "f16" in kernel else "global_store_dword", True] > 0, kernel
         assert found["global_load_dwordx4", True] > 0 and found["global_load_dwordx4", False] == (4 if kernel.endswith("_v4") else 0), kernel
+
+
+def test_layernorm_reads_its_rows_past_the_caches(code):
+    """As many vectors past the caches as it stores; through them only the two parameters' vectors."""
+    names, accesses = code
+    kernels = names(r"mtrt_layernorm_\w+_[vgu]\d+(v\d+)?[rea]?")
+    assert len(kernels) > 60
+    for kernel, found in accesses(kernels).items():
+        past = found["global_load_dwordx4", True]
+        assert past == found["global_store_dwordx4", True] > 0 and found["global_load_dwordx4", False] == 2 * past, kernel
