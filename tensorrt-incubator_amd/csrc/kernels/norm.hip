@@ -23,6 +23,7 @@
 // All arithmetic is f32 with the operation order above; reductions are trees
 // rather than the host's left-to-right sums, which the float tolerance covers.
 #include "common.hpp"
+#include "row_reads.hpp"
 
 using namespace mtrt_dev;
 
@@ -101,16 +102,9 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
   }
 }
 
-// Up to which sizes softmax reads rows through the caches: what the pass before has left in the Infinity Cache comes at twice the rate at which loads
-// past them bring it; larger tensors gain nothing, and would push other things out.  us, past and through, tensors of three calls in turn: softmax f32 of
-// 4, 8, 34, 50 and 67 MB 4.2, 3.9; 4.5, 3.9; 11.3, 10.5; 18.1, 15.3; 24.5, 19.9; bf16 12.2, 10.8 and 18.1, 15.6 for 34 and 50 MB; 101 MB 33.6,
-// 33.1; 134 MB 44.1, 46.3; from memory 34 to 67 MB take 2 to 4 % longer.  In between, where x and y together are what the L2s hold, neither is
-// ahead (17 MB: f32 6.3, 6.2, from memory 7.0, 7.2).
-// LayerNorm reads past the caches always.  (us, past and through, three tensors in turn; each from memory; with a launch that makes x in front and one that
+// LayerNorm reads past the caches always, softmax as in row_reads.hpp.  (LayerNorm, us, past and through, three tensors in turn; each from memory; with a launch that makes x in front and one that
 // reads y behind, all three: f32 [256, 4096] 4.8, 4.8; 5.8, 6.2; 11.9, 12.0; [512, 4096] 5.2, 5.2; 6.1, 6.5; 16.7, 17.5; bf16 [512, 4096] 4.4, 4.4; 5.0, 5.4;
 // 11.7, 11.9; [1024, 4096] 4.5, 4.6; 5.6, 6.0; 15.0, 15.4; f16 [2796, 1500] 5.7, 5.5; 6.5, 6.5; 21.3, 21.7; bf16 [250, 14165] 6.6, 6.4; 7.2, 7.5; 16.3, 16.6.)
-__device__ __forceinline__ bool softmax_past(int64_t bytes) { return bytes > (int64_t(80) << 20) || (bytes > (int64_t(12) << 20) && bytes <= (int64_t(20) << 20)); }
-
 // What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back:
 // alone softmax bf16 of 134 MB 44.1 -> 46.8 us where each result has memory of its own, 44.3 -> 46.7 from memory, with a copy of 268 MB behind each 133.2 ->
 // 135.7, between the launches that make x and take y 128.7 -> 127.6; LayerNorm bf16 [8178, 4096] 22.6 -> 21.4, 23.0 -> 22.3, 113.6 -> 116.8, 62.0 -> 60.6; of 101 MB
@@ -255,13 +249,13 @@ __device__ __forceinline__ void softmax_rows(const typename X::storage* __restri
   // the wave index as a scalar: the row pointers are then wave-uniform and the accesses need one lane offset, not an address pair each
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;
-  const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  past_or_through(softmax_past(bytes), [&](auto past, int64_t zero) {
-    if (d == int64_t(Vec<X>::kElems) * kWave * NV)
-      softmax_row<X, NV, true, decltype(past)::value>(x + zero, y, row, d);
-    else
+  if (d == int64_t(Vec<X>::kElems) * kWave * NV) {   // (whole cache lines)
+    softmax_row<X, NV, true, true>(x, y, row, d);
+  } else {
+    past_or_through(softmax_reads_past(rows, d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
       softmax_row<X, NV, false, decltype(past)::value>(x + zero, y, row, d);
-  });
+    });
+  }
 }
 
 // ---- rows longer than one wave's registers, and rows of any length or alignment: a GROUP of lanes owns one row ----
@@ -485,13 +479,13 @@ __device__ __forceinline__ void softmax_group(const typename X::storage* __restr
   constexpr bool kKeep = THREADS <= 256 || NV * Vec<X>::kElems <= 64;
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  const int64_t bytes = rows * d * int64_t(sizeof(typename X::storage));
-  past_or_through(softmax_past(bytes), [&](auto past, int64_t zero) {
-    if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
-      softmax_group_row<X, NV, THREADS, true, true, kKeep, false, decltype(past)::value>(x + zero, y, row, d, lds);
-    else
+  if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV) {   // (whole cache lines)
+    softmax_group_row<X, NV, THREADS, true, true, kKeep, false, true>(x, y, row, d, lds);
+  } else {
+    past_or_through(softmax_reads_past(rows, d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
       softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED, decltype(past)::value>(x + zero, y, row, d, lds);
-  });
+    });
+  }
 }
 
 // ---- any D, any alignment: one workgroup per row, row re-read from cache -------------

@@ -68,3 +68,14 @@ def test_layernorm_reads_its_rows_past_the_caches(code):
     for kernel, found in accesses(kernels).items():
         past = found["global_load_dwordx4", True]
         assert past == found["global_store_dwordx4", True] > 0 and found["global_load_dwordx4", False] == 2 * past, kernel
+
+
+def test_softmax_reads_its_rows_either_way(code):
+    """Two bodies with as many loads each (row_reads.hpp says which one runs), a third for rows that fill all vectors, past the caches."""
+    names, accesses = code
+    kernels = names(r"mtrt_softmax_\w+_[vgu]\d+(v\d+)?[ea]?")
+    assert len(kernels) > 60
+    for kernel, found in accesses(kernels).items():
+        through, past = found["global_load_dwordx4", False], found["global_load_dwordx4", True]
+        whole = "_u" not in kernel and not ("_g256" in kernel and kernel.endswith("e"))
+        assert through > 0 and past == through * (2 if whole else 1), kernel

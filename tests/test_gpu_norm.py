@@ -306,34 +306,35 @@ def test_softmax_ragged_rows(pkg, orc, name):
         _run_softmax(pkg, orc, name, 5, d, 90 + d % 89, "mtrt_softmax_" + name + suffix, frac=2e-2 if d <= 40000 else 5e-2)
 
 
-@pytest.mark.parametrize("dname", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dname", ["float32", "bfloat16", "float16"])
 @pytest.mark.parametrize("op", ["softmax", "layernorm"])
 def test_rows_read_through_the_caches_and_past_them(pkg, op, dname):
-    """A row's result does not depend on how it was read: tensors of one row more than the largest on either side of each line, in the forms of a wave, of
-    a workgroup and of ragged rows, bit for bit, and the first rows against float64."""
+    """A row's result does not depend on how it was read: tensors of the largest size on one side of each line (row_reads.hpp) and one row more, in the
+    forms of a few lanes, a wave, a workgroup and of ragged rows, bit for bit, and the first and last rows against float64."""
     import torch
     td = getattr(torch, dname)
     gen = torch.Generator(device="cuda").manual_seed(7)
-    lines = [v << 20 for v in ((12, 20, 80) if op == "softmax" else (8,))]
+    # rows that are no whole cache lines: whole 128-bit vectors (1032, 4104, 16392) and not
+    lines, columns = ([20 << 20, 80 << 20], (100, 1032, 4104, 16392, 1001, 9001)) if op == "softmax" else ([8 << 20], (1024, 4096, 16384, 1001))
+    # the exponential's argument (up to 16), the instruction, the sum's additions, the product and the narrowing; tree sums of up to 64 steps in f32, then
+    # six roundings, in units of the largest term
+    eps, tiny = {"float32": (2.0 ** -24, 2.0 ** -126), "bfloat16": (2.0 ** -8, 2.0 ** -126), "float16": (2.0 ** -11, 2.0 ** -24)}[dname]
     for line in lines:
-        for d in (1024, 4096, 16384, 1001):
+        for d in columns:
             rows = line // (d * td.itemsize)
             x = torch.randn((rows + 1, d), generator=gen, device="cuda").to(td)
             gamma, beta = (torch.rand(d, generator=gen, device="cuda") + 0.5).to(td), torch.randn(d, generator=gen, device="cuda").to(td)
             run = (lambda t: pkg.softmax(t)) if op == "softmax" else (lambda t: pkg.layernorm(t, gamma, beta, 1e-5))
             more, kernel = run(x), pkg.last_kernel()
             less = run(x[:rows].contiguous())
-            if pkg.last_kernel() == kernel:            # (the form may change with the number of rows)
-                assert torch.equal(more[:rows], less), (line, d, kernel)
-            xd = x[:8].double()
-            if op == "softmax":
-                ref = torch.softmax(xd, dim=-1)
-                # the exponential's argument (up to 16), the instruction, the sum's additions, the product and the narrowing
-                tol = ref * ({"float32": 2.0 ** -24, "bfloat16": 2.0 ** -8}[dname] + (16 + 16 + 32) * 2.0 ** -24) + 2.0 ** -126
-            else:
-                dev = xd - xd.mean(-1, keepdim=True)
-                ref = dev / torch.sqrt((dev * dev).mean(-1, keepdim=True) + 1e-5) * gamma.double() + beta.double()
-                # tree sums of up to 64 steps in f32, then six roundings, in units of the largest term
-                tol = {"float32": 2.0 ** -24, "bfloat16": 2.0 ** -8}[dname] * ref.abs() + (64 + 6) * 2.0 ** -24 * ((ref - beta.double()).abs() + beta.double().abs() + 1.0)
-            for y in (more, less):
-                assert bool(((y[:8].double() - ref).abs() <= tol).all()), (line, d, kernel)
+            assert pkg.last_kernel() == kernel and torch.equal(more[:rows], less), (line, d, kernel)
+            for part in (slice(0, 8), slice(rows - 7, rows + 1)):
+                xd = x[part].double()
+                if op == "softmax":
+                    ref = torch.softmax(xd, dim=-1)
+                    tol = ref * (eps + (16 + 16 + 32) * 2.0 ** -24) + tiny
+                else:
+                    dev = xd - xd.mean(-1, keepdim=True)
+                    ref = dev / torch.sqrt((dev * dev).mean(-1, keepdim=True) + 1e-5) * gamma.double() + beta.double()
+                    tol = eps * ref.abs() + (64 + 6) * 2.0 ** -24 * ((ref - beta.double()).abs() + beta.double().abs() + 1.0) + tiny
+                assert bool(((more[part].double() - ref).abs() <= tol).all()), (line, d, kernel, part)
