@@ -210,7 +210,7 @@ struct RowsScaleEpilogue {
 // ---- small M (<= 32): one workgroup per 32 columns, four waves split K -----------------------------------
 // A launch of the tile kernel above lasts one tile's whole K loop however few rows it has (M = 16 at K = 4096,
 // N = 11008: 21.7 us) although all it has to do is read the weights once (45 MB).  Here every workgroup owns one
-// tile of 32 columns (or two, see small_m_tiles) over all of K, its four waves a quarter of K each: a wave keeps
+// tile of 32 columns (or two, see `tiles` below) over all of K, its four waves a quarter of K each: a wave keeps
 // a ring of four stages (8 * G rows x 128 k of activations each) of its own in LDS, filled by direct-to-LDS loads
 // three slices ahead as whole 128-byte row segments (a fragment read straight from memory would touch 32 cache
 // lines), and takes the weights from fragment order straight into registers: no barrier until the four partial
@@ -381,13 +381,8 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_frag_rows32(
     const uint16_t* __restrict__ bias, int32_t past) {
   __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 4 * 1024];
   const RowsScaleEpilogue epi{a_scale, w_scale, a_step, bias};
-  if (M <= 16) {
-    if (past) small_m::tiles<2, true>(a, w_frag, epi, y, M, K, N, lds);
-    else small_m::tiles<2, false>(a, w_frag, epi, y, M, K, N, lds);
-  } else {
-    if (past) small_m::tiles<4, true>(a, w_frag, epi, y, M, K, N, lds);
-    else small_m::tiles<4, false>(a, w_frag, epi, y, M, K, N, lds);
-  }
+  if (past) small_m::tiles<4, true>(a, w_frag, epi, y, M, K, N, lds);
+  else small_m::tiles<4, false>(a, w_frag, epi, y, M, K, N, lds);
 }
 // Any K (no alignment needs): one output element per lane, plain loops.  Only K = 0 is left to it (every
 // other shape runs on the matrix cores).

@@ -1310,18 +1310,16 @@ int32_t mtrt_hip_gemm_w8a8_prepack_fragments(mtrt_stream_t stream, const void *w
 
 namespace {
 // Which kernel a W8A8 call on fragment-order weights takes.  Up to 32 rows: the four-wave kernels that read the weights once, with LDS for 16 or
-// for 32 rows.  (Up to 16 rows that is the same body, which of the two matters only where units hold several workgroups: long K by few columns, where eight
-// waves to a tile once were ahead, keeps the larger one.  Eight waves and four, weights in turns of three sets, us: (1, 2688, 4096) 4.8, 3.8; (16, 8192,
-// 2048) 7.8, 7.0; (8, 14336, 512) 9.4, 7.3; before the weights went through the caches the four took 4.9, 8.9 and 7.3.)
+// for 32 rows.  (Eight waves to a tile instead, for long K by few columns, weights in turns of three sets, us, eight and four: (1, 2688, 4096) 4.8, 3.8;
+// (16, 8192, 2048) 7.8, 7.0; (8, 14336, 512) 9.4, 7.3.)
 // 33 to 64 rows: the wave-private kernel or a tile, by estimate.  Above: the tile and K split frag_plan estimates fastest.
-constexpr int64_t kW8LongK = 2688;
 struct W8Plan {
-  enum { kSmall16, kRows, kTile } kind;
+  enum { kRows, kTile } kind;
   FragPlan tile;
 };
 W8Plan w8_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   if (M <= 32)
-    return {M > 16 || (K >= kW8LongK && 2 * ((N + 31) / 32) <= units) ? W8Plan::kRows : W8Plan::kSmall16, {}};
+    return {W8Plan::kRows, {}};
   const FragPlan tile = frag_plan(M, N, K / 128, units, may_split);
   if (M <= 64 && frag_rows_us(M, N, K / 128, units) < tile.us)
     return {W8Plan::kRows, {}};
@@ -1365,9 +1363,9 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     // from memory 14.4, 14.3; 18.2, 17.9; 23.5, 22.1; 100 MB 19.9, 19.5
     int32_t past = K * N > tuning::kWeightsPastBytes * (M > 16 ? 2 : 1);
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias, &past};
-    return launch(st, KernelName(plan.kind == W8Plan::kSmall16 ? "mtrt_gemm_w8a8_small16" : "mtrt_gemm_w8a8_frag_rows32"), grid, kBlock, stream, args);
+    return launch(st, KernelName(M <= 16 ? "mtrt_gemm_w8a8_small16" : "mtrt_gemm_w8a8_frag_rows32"), grid, kBlock, stream, args);
   }
-  if (M <= 64 && plan.kind != W8Plan::kTile) {
+  if (plan.kind == W8Plan::kRows) {
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias};
     return launch(st, KernelName("mtrt_gemm_w8a8_frag_rows64"), uint32_t(std::min<int64_t>(tiles32, kLoopGrid)), 512, stream, args);
   }

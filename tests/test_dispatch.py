@@ -334,3 +334,19 @@ def test_strips_of_more_than_16_rows_cover_the_output_and_need_no_workspace(gpu)
 def test_pairs_of_tiles_however_short_k_is(gpu, pkg, family, shape, kernel):
     name = gpu.w8a8(8, *shape)[0] if family == "w8a8" else gpu.linear(8, *shape, pkg.F16)[0]
     assert name == {"w8a8": "mtrt_gemm_w8a8_frag_", "dense": "mtrt_gemm_dense_frag_f16_"}[family] + kernel
+
+
+def test_w8a8_of_up_to_32_rows(gpu):
+    """One kernel up to 16 rows, however long K and few the columns, another up to 32: a workgroup to a tile of 32 columns, or, between one and two tiles to a
+    unit, a workgroup to a unit from 9 rows on, and above 16 where K is long for the tiles left over."""
+    seen = set()
+    for M in (1, 8, 9, 16, 17, 32):
+        for K in (128, 1920, 2048, 2688, 4096, 8192, 14336):
+            for N in (1, 512, 4096, 8192, 8193, 9216, 10240, 10241, 12289, 16384, 16385):
+                name = gpu.w8a8(None, M, K, N)[0]
+                assert name == ("mtrt_gemm_w8a8_small16" if M <= 16 else "mtrt_gemm_w8a8_frag_rows32")
+                tiles = (N + 31) // 32
+                shared = 256 < tiles <= 512 and (M > 8 if M <= 16 else K >= 2048 and (tiles - 256) * 32 <= K)
+                assert gpu.sizes[-1][1:] == (256 if shared else tiles, 256), (M, K, N)
+                seen.add((M > 16, shared))
+    assert len(seen) == 4

@@ -83,13 +83,9 @@ def test_w8a8_33_to_128_rows_on_row_major_weights(pkg, orc, shape):
     assert np.array_equal(bits16(y).reshape(M, N), orc.gemm_w8a8(a, w, a_s, w_s))
 
 
-# Up to 32 rows on fragment-order weights: the four-wave kernel with hand-counted waits (up to 16 rows) or the
-# wave-private eight-wave kernel; which of the two depends on the number of compute units, the results do not.
-_FRAG_SMALL = {"mtrt_gemm_w8a8_frag_rows32", "mtrt_gemm_w8a8_small16"}
-
-
+# Up to 32 rows on fragment-order weights: the four-wave kernel with hand-counted waits, with LDS for 16 rows or for 32.
 def _frag_small_ok(kernel, M):
-    return kernel in _FRAG_SMALL and (M <= 16 or kernel == "mtrt_gemm_w8a8_frag_rows32")
+    return kernel == ("mtrt_gemm_w8a8_small16" if M <= 16 else "mtrt_gemm_w8a8_frag_rows32")
 
 
 # the tile kernels on fragment-order weights; which one a shape takes is the host's estimate (tests/test_dispatch.py)
@@ -122,7 +118,7 @@ def test_w8a8_weights_in_registers_kernel(pkg, orc, shape):
 @pytest.mark.parametrize("shape", [(1, 128, 32), (16, 4096, 11008), (32, 4096, 11008), (17, 384, 200), (9, 1280, 4099), (13, 640, 8240),
                                    (32, 256, 16384), (25, 512, 16400), (8, 2048, 8209), (16, 128, 40)])
 def test_w8a8_small_m_kernel(pkg, orc, shape):
-    """M <= 32: one workgroup per 32-column tile with four or eight waves splitting K.  K = 128 and 384 leave waves without a
+    """M <= 32: one workgroup per 32-column tile with four waves splitting K.  K = 128 and 384 leave waves without a
     slice, 1280 gives them 2 or 3 (only the one-at-a-time tail), 4096 eight (two groups of four); N = 11008 gives 344
     tiles (one workgroup per compute unit, the first 88 with two tiles), 16384 two each, 16400 and 8209 one tile beyond
     those forms; ragged last tiles; M = 8 stays at one tile per workgroup.  Integer sums: bit-exact."""
