@@ -1004,7 +1004,7 @@ MTRT_W4_TILE_KERNELS(_bias, BiasEpilogue)
 // Small M (<= 32): one workgroup per 32 columns, four waves split K.
 // G: groups of 8 activation rows kept per stage (M <= 8 * G); WAVES: waves that split K;
 // JT: column tiles of the workgroup (blockIdx.x, blockIdx.x + gridDim.x), sharing the activations.
-template <int G, int WAVES, int JT, bool PAST>
+template <int G, int WAVES, int JT>
 __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp,
                                        const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M, int64_t K,
                                        int64_t N, int64_t block, const uint16_t* __restrict__ bias, int8_t* lds) {
@@ -1059,8 +1059,7 @@ __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uin
     for (int j = 0; j < JT; ++j) {
       const u4* wsrc = bp[j] + kb * 64;
       const uint16_t* ssrc = scale + int64_t(uint32_t(kb) / slices_per_block) * N + col[j];
-      if constexpr (PAST) __asm__ volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(dst.w[j]) : "v"(wsrc) : "memory");
-      else __asm__ volatile("global_load_dwordx4 %0, %1, off" : "=v"(dst.w[j]) : "v"(wsrc) : "memory");
+      __asm__ volatile("global_load_dwordx4 %0, %1, off nt" : "=v"(dst.w[j]) : "v"(wsrc) : "memory");
       __asm__ volatile("global_load_ushort %0, %1, off" : "=v"(dst.sc[j]) : "v"(ssrc) : "memory");
     }
   };
@@ -1151,35 +1150,30 @@ __device__ __forceinline__ void skinny(const uint16_t* __restrict__ a, const uin
 // workgroups and the rest with one (tiles between one and two times the compute units), one workgroup
 // per compute unit: workgroup g then also takes tile g + gridDim.x if there is one, and reads the
 // activations once for both.
-template <int G, bool PAST>
+template <int G>
 __device__ __forceinline__ void skinny_tiles(const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp,
                                              const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
                                              int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias, int8_t* lds) {
   const int64_t tiles = (N + 31) / 32;
   if (int64_t(blockIdx.x) + gridDim.x < tiles)
-    skinny<G, 4, 2, PAST>(a, wp, scale, y, M, K, N, block, bias, lds);
+    skinny<G, 4, 2>(a, wp, scale, y, M, K, N, block, bias, lds);
   else
-    skinny<G, 4, 1, PAST>(a, wp, scale, y, M, K, N, block, bias, lds);
+    skinny<G, 4, 1>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 
-// past: the weights are read past the caches (kWeightsPastBytes in clusters.cpp).
 // M <= 16: half the activation rows per stage (8 waves splitting K were no faster than 4).
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny16(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias,
-    int32_t past) {
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
   __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 2 * 1024];
-  if (past) skinny_tiles<2, true>(a, wp, scale, y, M, K, N, block, bias, lds);
-  else skinny_tiles<2, false>(a, wp, scale, y, M, K, N, block, bias, lds);
+  skinny_tiles<2>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 // M <= 32: 4 waves split K.
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny(
     const uint16_t* __restrict__ a, const uint32_t* __restrict__ wp, const uint16_t* __restrict__ scale,
-    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias,
-    int32_t past) {
+    uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {
   __shared__ __attribute__((aligned(16))) int8_t lds[4 * 4 * 4 * 1024];
-  if (past) skinny_tiles<4, true>(a, wp, scale, y, M, K, N, block, bias, lds);
-  else skinny_tiles<4, false>(a, wp, scale, y, M, K, N, block, bias, lds);
+  skinny_tiles<4>(a, wp, scale, y, M, K, N, block, bias, lds);
 }
 
 // ---- M <= 16, and groups of 16 rows by few columns: one strip of columns per compute unit ----------------
@@ -1196,11 +1190,11 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w4a16_skinny(
 // whole 256-byte row segments by direct-to-LDS loads, 16-byte chunks XOR-swizzled by the row so that the fragment
 // reads are conflict-free) and never touches another wave's ring: no barriers until the partial tiles are added
 // through LDS at the end.
-// G: groups of four activation rows (M <= 4 G); SC: scale rows per slice of 128 k (2: blocks of 64); PAST: the weights pass
-// the caches by.
+// G: groups of four activation rows (M <= 4 G); SC: scale rows per slice of 128 k (2: blocks of 64); ONCE: nobody else reads these weights, so that
+// they pass the caches by.
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-template <int WAVES, int JT, int G, int SC, bool PAST>
+template <int WAVES, int JT, int G, int SC, bool ONCE>
 __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws,
                                              const uint16_t* __restrict__ scale, uint16_t* __restrict__ y, int64_t M,
                                              int64_t K, int64_t N, int64_t block, uint32_t tile0, const uint16_t* __restrict__ bias, int8_t* lds) {
@@ -1257,7 +1251,7 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
       // opaque register loads, waits placed by hand (see `skinny`); what comes from memory is asked for first
 #pragma unroll
       for (int j = 0; j < JT; ++j) {
-        if constexpr (PAST) __asm__ volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
+        if constexpr (ONCE) __asm__ volatile("global_load_dwordx4 %0, %1, %2 nt" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
         else __asm__ volatile("global_load_dwordx4 %0, %1, %2" : "=v"(dst.w[j]) : "v"(woff), "s"(wsrc[j]) : "memory");
       }
 #pragma unroll
@@ -1381,7 +1375,7 @@ __device__ __forceinline__ void strips_chunk(const uint16_t* __restrict__ a, con
 // kernel above: (2, 6656, 960) 9.4 and 5.0, (16, 4096, 11008) 10.1 and 9.2, (13, 1152, 14464) 6.3 and 5.5.  Eight waves (two per
 // SIMD) are no faster: 10.4 us at (16, 4096, 11008).
 constexpr int kStripWaves = 4;
-template <int G, int SC, bool PAST>
+template <int G, int SC, bool ONCE>
 __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,
                                        uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block,
                                        const uint16_t* __restrict__ bias, uint32_t b, uint32_t grid, int8_t* lds) {
@@ -1392,16 +1386,15 @@ __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uin
   const uint32_t t0 = b * per + (b < rem ? b : rem), t1 = t0 + per + (b < rem ? 1 : 0);
   for (uint32_t t = t0; t < t1; t += 3) {
     const uint32_t left = t1 - t;
-    if (left >= 3) strips_chunk<kStripWaves, 3, G, SC, PAST>(a, ws, scale, y, M, K, N, block, t, bias, lds);
-    else if (left == 2) strips_chunk<kStripWaves, 2, G, SC, PAST>(a, ws, scale, y, M, K, N, block, t, bias, lds);
-    else strips_chunk<kStripWaves, 1, G, SC, PAST>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    if (left >= 3) strips_chunk<kStripWaves, 3, G, SC, ONCE>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else if (left == 2) strips_chunk<kStripWaves, 2, G, SC, ONCE>(a, ws, scale, y, M, K, N, block, t, bias, lds);
+    else strips_chunk<kStripWaves, 1, G, SC, ONCE>(a, ws, scale, y, M, K, N, block, t, bias, lds);
   }
 }
 #define MTRT_W4_STRIPS(NAME, SC)                                                                                          \
   extern "C" __global__ void __launch_bounds__(64 * kStripWaves) NAME(                                                    \
       const uint16_t* __restrict__ a, const uint32_t* __restrict__ ws, const uint16_t* __restrict__ scale,                \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias,        \
-      int32_t past) {                                                                                                     \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, int64_t block, const uint16_t* __restrict__ bias) {      \
     __shared__ __attribute__((aligned(16))) int8_t lds[kStripWaves * 4 * 4096];                                           \
     uint32_t b = blockIdx.x, grid = gridDim.x;                                                                            \
     if (M > 16) {                                                                                                         \
@@ -1412,14 +1405,11 @@ __device__ __forceinline__ void strips(const uint16_t* __restrict__ a, const uin
       y += uint64_t(row0) * N;                                                                                            \
       strips<4, SC, false>(a, ws, scale, y, M - row0 < 16 ? M - row0 : 16, K, N, block, bias, b, grid, lds);              \
     } else if (M <= 4) {                                                                                                  \
-      if (past) strips<1, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                 \
-      else strips<1, SC, false>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                     \
+      strips<1, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                           \
     } else if (M <= 8) {                                                                                                  \
-      if (past) strips<2, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                 \
-      else strips<2, SC, false>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                     \
+      strips<2, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                           \
     } else {                                                                                                              \
-      if (past) strips<4, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                 \
-      else strips<4, SC, false>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                     \
+      strips<4, SC, true>(a, ws, scale, y, M, K, N, block, bias, b, grid, lds);                                           \
     }                                                                                                                     \
   }
 MTRT_W4_STRIPS(mtrt_gemm_w4a16_strips16, 1)

@@ -214,7 +214,8 @@ struct RowsScaleEpilogue {
 // a ring of four stages (8 * G rows x 128 k of activations each) of its own in LDS, filled by direct-to-LDS loads
 // three slices ahead as whole 128-byte row segments (a fragment read straight from memory would touch 32 cache
 // lines), and takes the weights from fragment order straight into registers: no barrier until the four partial
-// sums (int32, exact in any order) meet in LDS.  G: groups of 8 activation rows per stage (M <= 8 * G).
+// sums (int32, exact in any order) meet in LDS.  G: groups of 8 activation rows per stage (M <= 8 * G); PAST: the weights
+// pass the caches by.
 namespace small_m {
 
 template <int G, int WAVES, int JT, bool PAST>
@@ -358,7 +359,7 @@ __device__ __forceinline__ void tiles(const int8_t* __restrict__ a, const v4i* _
 }  // namespace small_m
 
 // (a [M,K] i8, w_frag (fragment order), a_scale [M] f32, w_scale [N] f32, y [M,N] f16, M, K, N, a_step, bias, past) ; K % 128 == 0, a
-// and w_frag 16-byte aligned, M * K < 2^32; past: the weights are read past the caches (kWeightsPastBytes in clusters.cpp); grid = ceil(N / 32) or
+// and w_frag 16-byte aligned, M * K < 2^32; past: the weights are read past the caches (w8_few_rows_past in clusters.cpp); grid = ceil(N / 32) or
 // the number of compute units (see small_m::tiles), block = 256.
 // M <= 16:
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_small16(
@@ -371,10 +372,9 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_small16(
   else small_m::tiles<2, false>(a, w_frag, epi, y, M, K, N, lds);
 }
 // ... M <= 32, the same arguments; grid = ceil(N / 32) or the number of compute units: which one stands beside the launch.  Against eight waves to
-// a tile that each bring their own rows, as in gemm_core::rows32 (there 64 rows still run so), us, (M, K, N), weights of three calls in turn: (32, 1152, 9216)
-// 7.0, 4.8; (17, 2048, 11008) 9.3, 7.6; (32, 4096, 11008) 13.2, 11.4; (32, 6144, 9216) 16.5, 13.7; (32, 8192, 11008) 24.7, 20.6; (17, 4096, 4096) 6.2, 5.9; from
-// memory 17.0, 13.6; 21.7, 17.6 for the third and fourth; up to 16 rows of few columns (1, 2688, 4096) 4.8, 3.8; (16, 8192, 2048) 7.8, 7.0; (8, 14336, 512) 9.4,
-// 7.3; the other way up to eight slices by no more tiles than units, (32, 640, 4096) 3.4, 3.6.
+// a tile that each bring their own rows, as in gemm_core::rows32 (there 64 rows still run so), us, (M, K, N), weights of three sets in turn: (32, 1152, 9216)
+// 7.0, 5.5; (17, 2048, 11008) 9.3, 7.6; (32, 4096, 11008) 13.2, 11.4; (32, 8192, 11008) 24.7, 22.3; (17, 4096, 4096) 6.2, 5.9; from memory the third 17.0, 13.6;
+// the other way up to eight slices by no more tiles than units, (32, 640, 4096) 3.4, 3.6.
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_frag_rows32(
     const int8_t* __restrict__ a, const v4i* __restrict__ w_frag, const float* __restrict__ a_scale,
     const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t a_step,

@@ -47,15 +47,21 @@ constexpr double kRowsFixedUs = 3.0, kRowsBytesPerUs = 3.4e6, kRowsWideBytesPerU
 // The same kernels with four row tiles (65 to 128 rows): one workgroup per compute unit at a time, so rounds of 32-column
 // tiles, each the length of its K loop: 3.7 ns per row byte (int8 M = 128, K = N = 4096 18.4 us, K = N = 8192 30.7 us).
 constexpr double kRows128FixedUs = 3.0, kRows128UsPerRowByte = 0.0037;
-// Products of few rows read weights above these bytes past the caches (us, past and through, f32: M = 1, 180 MB 26.7, 28.9; M = 3, 53 MB
+// Float products of few rows read weights above these bytes past the caches (us, past and through, f32: M = 1, 180 MB 26.7, 28.9; M = 3, 53 MB
 // 11.5, 12.0; M = 1, 29 MB 7.7, 6.8; bf16: 90 MB 16.2, 17.0; 67 MB 12.4, 13.4; 33 MB 9.8, 8.4).
 constexpr int64_t kWeightsPastBytes = int64_t(48) << 20;
-// int8 and int4 weights alike, kernel times in turns of three sets, so with the weights in the Infinity Cache (what lies in HBM takes 0 to 6 % longer
-// through the caches): W4A16 in strips (16, 4096, 2048) 5.1, 4.2; (16, 14336, 4096) 12.3, 9.9; (16, 8192, 16384), 67 MB, 18.6, 15.6, but 2 to 5 % longer
-// from HBM; 17 to 32 rows (32, 7808, 9280) 17.7, 15.9; W8A8 of 9 to 16 rows 8 MB 4 to 26 % shorter, 34 to 45 MB 8 to 21 %, 90 MB 3 % and from HBM
-// 13 % longer.  Up to four rows of W4A16 take in little beside the weights, and the line is lower: (2, 8960, 2304) 5.89, 5.69; (4, 6016, 3200) 4.98,
-// 4.76; (2, 4736, 5184) 5.49, 5.57; (1, 6400, 4864) 6.39, 6.62; (1, 4096, 11008) 6.70, 7.19.
-constexpr int64_t kFewRowsWeightsPastBytes = int64_t(10) << 20;
+// int8 and int4 weights of few rows are read past the caches: a decode step comes back to a layer's weights when all other layers' have been through, so
+// that they lie in memory, and from there they take longer through the caches.  (us, past and through, weights of three sets in turn, which the Infinity
+// Cache holds, and from memory: W4A16 (1, 4096, 11008) 6.8, 7.4; 7.7, 7.8; (8, 4096, 4096) 3.9, 3.9; 4.8, 5.0; (16, 4096, 11008) 8.6, 8.2; 9.1, 9.3; (32, 8192, 8192)
+// 13.5, 11.5; 13.9, 14.5; W8A8 (1, 4096, 8192) 7.4, 7.5; 7.9, 8.7; (16, 4096, 6144) 6.9, 6.5; 7.5, 7.8; (16, 4096, 11008) 11.8, 10.4; 12.6, 12.8.)
+// But for W8A8, from kThroughFromFewTiles or kThroughFrom to kThroughUpTo, where a workgroup's own rate is the bound, which from the Infinity Cache is 57 to 67
+// GB/s past the caches and 100 through them: with at most half a tile of 32 columns to a unit, and with 17 to 32 rows, which come in beside the weights.  Past the
+// caches these take longer there than eight waves to a tile did, through them they do in neither place.  The eight waves, past and through: (16, 8192, 2048) 7.7,
+// 8.7, 6.8; 10.9, 9.7, 9.9; (8, 11008, 4096) 9.8, 11.6, 9.1; 14.2, 12.0, 12.6; (16, 14336, 4096) 12.2, 16.2, 11.6; 18.4, 16.7, 17.3; (4, 2688, 4096) 4.7, 4.2, 3.9; 6.3,
+// 5.1, 5.3; (24, 4096, 2048) 5.6, 6.7, 5.4; 8.1, 7.2, 7.3; (32, 14336, 1024) 12.2, 15.9, 11.8; 19.4, 18.7, 18.8; (32, 6144, 9216) 16.0, 17.1, 13.8; 21.9, 17.9, 17.8; (32,
+// 8192, 8192) 14.1, 15.6, 14.3; 17.5, 16.3, 17.4.  Smaller (8, 14336, 512) 9.1, 7.2, 7.2; 14.3, 12.4, 12.8; (32, 1152, 9216) 6.7, 5.4, 4.7; 9.0, 6.5, 6.7; larger (32, 12288, 8192)
+// 21.9, 20.5, 21.3; 22.8, 21.2, 21.9.
+constexpr int64_t kThroughFromFewTiles = int64_t(8) << 20, kThroughFrom = int64_t(16) << 20, kThroughUpTo = int64_t(64) << 20;
 // f32 products of few rows on the vector units: K from which four waves share it; the fewest weights (below, the tiles take 3 to 4 us
 // too); what several groups of rows read through the L2s.
 constexpr int64_t kDotOwnColumnsBelow = 1536, kDotMinWeights = 16384;
@@ -1310,8 +1316,7 @@ int32_t mtrt_hip_gemm_w8a8_prepack_fragments(mtrt_stream_t stream, const void *w
 
 namespace {
 // Which kernel a W8A8 call on fragment-order weights takes.  Up to 32 rows: the four-wave kernels that read the weights once, with LDS for 16 or
-// for 32 rows.  (Eight waves to a tile instead, for long K by few columns, weights in turns of three sets, us, eight and four: (1, 2688, 4096) 4.8, 3.8;
-// (16, 8192, 2048) 7.8, 7.0; (8, 14336, 512) 9.4, 7.3.)
+// for 32 rows.
 // 33 to 64 rows: the wave-private kernel or a tile, by estimate.  Above: the tile and K split frag_plan estimates fastest.
 struct W8Plan {
   enum { kRows, kTile } kind;
@@ -1324,6 +1329,12 @@ W8Plan w8_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool may_split) {
   if (M <= 64 && frag_rows_us(M, N, K / 128, units) < tile.us)
     return {W8Plan::kRows, {}};
   return {W8Plan::kTile, tile};
+}
+
+// Whether the weights of up to 32 rows are read past the caches.
+bool w8_few_rows_past(int64_t M, int64_t K, int64_t N, int64_t units) {
+  const bool few_tiles = 2 * ((N + 31) / 32) <= units;
+  return (M <= 16 && !few_tiles) || K * N < (few_tiles ? tuning::kThroughFromFewTiles : tuning::kThroughFrom) || K * N > tuning::kThroughUpTo;
 }
 
 // a_step: 1 for a scale per row, 0 for one scale; bias: f16 [N] or null; workspace: for K-split tiles, may be null.
@@ -1359,9 +1370,7 @@ int32_t w8a8_fragments(hipStream_t stream, const void *a, const void *w_frag, co
     const bool over = tiles32 > units && tiles32 <= 2 * units;
     const bool pairs = over && (M > 16 ? K >= 2048 && (tiles32 - units) * 8192 <= K * units : M > 8);
     const uint32_t grid = uint32_t(pairs ? units : tiles32);
-    // more than 16 rows keep more on its way beside the weights: 58 to 90 MB through the caches and past them 11.8, 14.0; 14.3, 17.6; 21.0, 22.1,
-    // from memory 14.4, 14.3; 18.2, 17.9; 23.5, 22.1; 100 MB 19.9, 19.5
-    int32_t past = K * N > tuning::kWeightsPastBytes * (M > 16 ? 2 : 1);
+    int32_t past = w8_few_rows_past(M, K, N, units);
     void *args[] = {&a, &w_frag, &a_scale, &w_scale, &y, &M, &K, &N, &a_step, &bias, &past};
     return launch(st, KernelName(M <= 16 ? "mtrt_gemm_w8a8_small16" : "mtrt_gemm_w8a8_frag_rows32"), grid, kBlock, stream, args);
   }
@@ -1636,8 +1645,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
     return MTRT_RUNTIME_ERROR;
   if (w4_fast(a, w_prepacked, K, block)) {
     const int64_t cus = num_compute_units(st);
-    int32_t past = K * N / 2 > (M <= 4 ? tuning::kFewRowsWeightsPastBytes : tuning::kWeightsPastBytes);
-    void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias, &past};
+    void *args[] = {&a, &w_prepacked, &scale, &y, &M, &K, &N, &block, &bias};
     // (rows of activations are addressed by 32-bit offsets below)
     if (w4_strips(M, K, N, block, cus)) {
       // 16-column tiles over all of K (weights in strip order).  One workgroup per compute unit; up to 16 rows two for more than three
@@ -1645,7 +1653,7 @@ int32_t w4a16(hipStream_t stream, const void *a, const void *w_kn_packed, const 
       // 12.3 against 11.9, 1024 tiles 12.9 against 12.3), and with up to four rows for more than one (M = 1: 320 tiles 5.6 against
       // 5.2 us, 688 tiles 7.4 against 7.1, 1024 tiles 10.2 against 9.8); more rows' groups share the units ((22, 13056, 2880) 12.9 against 17.0).
       const void *in_strips = static_cast<const char *>(w_prepacked) + w4_fragment_bytes(K, N);
-      void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias, &past};
+      void *sargs[] = {&a, &in_strips, &scale, &y, &M, &K, &N, &block, &bias};
       const int64_t tiles = (N + 15) / 16, groups = (M + 15) / 16;
       const int64_t most = groups > 1 ? std::max<int64_t>(cus / groups, 1) : M <= 4 || tiles > 3 * cus ? 2 * cus : cus;
       return launch(st, KernelName(block == 64 ? "mtrt_gemm_w4a16_strips16_b64" : "mtrt_gemm_w4a16_strips16"),

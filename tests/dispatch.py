@@ -42,7 +42,8 @@ class Dispatch:
     clears (address, words, stream), `sizes` every launch's (kernel, grid, block), `forms` the run-time arguments by which some kernels
     choose what they do."""
 
-    _FORMS = {"mtrt_gemm_dense_rows32_f32": (7, 8), "mtrt_gemm_dense_edge_f32": (7,), "mtrt_gemm_dense_edge_f16": (7,), "mtrt_gemm_dense_edge_bf16": (7,)}
+    _FORMS = {"mtrt_gemm_dense_rows32_f32": (7, 8), "mtrt_gemm_dense_edge_f32": (7,), "mtrt_gemm_dense_edge_f16": (7,), "mtrt_gemm_dense_edge_bf16": (7,),
+              "mtrt_gemm_w8a8_small16": (10,), "mtrt_gemm_w8a8_frag_rows32": (10,), "mtrt_gemm_dense_frag_f16_rows16": (9,), "mtrt_gemm_dense_frag_bf16_rows16_f8": (9,)}
 
     def __init__(self, pkg, path, copy):
         shutil.copy(path, copy)

@@ -79,3 +79,15 @@ def test_softmax_reads_its_rows_either_way(code):
         through, past = found["global_load_dwordx4", False], found["global_load_dwordx4", True]
         whole = "_u" not in kernel and not ("_g256" in kernel and kernel.endswith("e"))
         assert through > 0 and past == through * (2 if whole else 1), kernel
+
+
+def test_few_rows_read_int8_and_int4_weights_past_the_caches(code):
+    """But where several groups of rows read them (the strips' fourth body), and in the second of W8A8's two bodies."""
+    names, accesses = code
+    kernels = names(r"mtrt_gemm_w4a16_(skinny|strips)\w+|mtrt_gemm_w4a16_skinny|mtrt_gemm_w8a8_(small16|frag_rows32)")
+    found = {kernel: (c["global_load_dwordx4", True], c["global_load_dwordx4", False]) for kernel, c in accesses(kernels).items()}
+    assert set(found) == {"mtrt_gemm_w4a16_skinny", "mtrt_gemm_w4a16_skinny16", "mtrt_gemm_w4a16_strips16", "mtrt_gemm_w4a16_strips16_b64", "mtrt_gemm_w8a8_small16",
+                          "mtrt_gemm_w8a8_frag_rows32"}
+    for kernel, (past, through) in found.items():
+        assert past > 0 and past == {"mtrt_gemm_w4a16_strips16": 3 * through, "mtrt_gemm_w4a16_strips16_b64": 3 * through, "mtrt_gemm_w8a8_frag_rows32": through, "mtrt_gemm_w8a8_small16": through}.get(kernel, past)
+        assert (through == 0) == kernel.startswith("mtrt_gemm_w4a16_skinny"), kernel

@@ -350,3 +350,20 @@ def test_w8a8_of_up_to_32_rows(gpu):
                 assert gpu.sizes[-1][1:] == (256 if shared else tiles, 256), (M, K, N)
                 seen.add((M > 16, shared))
     assert len(seen) == 4
+
+
+@pytest.mark.parametrize("M", [1, 16, 17, 25, 32])
+def test_w8a8_of_few_rows_reads_some_weights_through_the_caches(gpu, M):
+    """Up to 64 MiB: with half a tile to a unit at most from 8 MiB on, with more than 16 rows from 16 MiB on."""
+    for K, N, few, more in ((128, 1, 1, 1), (1152, 9216, 1, 1), (4096, 2047, 1, 1), (4096, 2048, 0, 0), (14336, 512, 1, 1), (14336, 640, 0, 0), (4096, 4096, 0, 0),
+                            (4096, 4097, 1, 0), (3968, 4097, 1, 1), (2048, 11008, 1, 0), (16384, 4096, 0, 0), (16512, 4096, 1, 1), (4096, 16384, 1, 0), (4096, 16385, 1, 1)):
+        gpu.w8a8(None, M, K, N)
+        assert gpu.forms[-1] == (("mtrt_gemm_w8a8_small16", few) if M <= 16 else ("mtrt_gemm_w8a8_frag_rows32", more)), (K, N)
+
+
+def test_16_bit_linears_of_few_rows_read_weights_of_more_than_48_mib_past_the_caches(gpu, pkg):
+    for N, past in ((1024, 0), (12288, 0), (12289, 1), (16384, 1)):
+        gpu.linear(None, 2, 2048, N, pkg.F16)
+        assert gpu.forms[-1] == ("mtrt_gemm_dense_frag_f16_rows16", past)
+        gpu.linear(None, 4, 2048, N, pkg.BF16, q_dtype=pkg.F8E4M3FN)
+        assert gpu.forms[-1] == ("mtrt_gemm_dense_frag_bf16_rows16_f8", past)

@@ -63,10 +63,11 @@ def test_w8a8_small(pkg, M):
 
 @pytest.mark.parametrize("M", [1, 8, 9, 16])
 def test_w8a8_small_of_few_columns(pkg, M):
-    """Fewer 32-column tiles than half of the compute units, down to one, and one more than that with a long K."""
+    """32-column tiles for half of the compute units, down to one, and one more; weights on both sides of the lines between loads past the caches and
+    through them."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(M)
-    for K, N in ((128, 1), (256, 32), (640, 33), (1152, 300), (2560, 1281), (2688, 4096), (2688, 4097)):
+    for K, N in ((128, 1), (256, 32), (640, 33), (1152, 300), (2560, 1281), (2688, 4096), (2688, 4097), (4096, 2047), (4096, 2048), (16384, 4096), (16512, 4095)):
         a = torch.randint(-128, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
         w = torch.randint(-128, 128, (K, N), generator=g, device="cuda", dtype=torch.int8)
         sa, sw = torch.rand(M, generator=g, device="cuda") * 0.01, torch.rand(N, generator=g, device="cuda") * 0.001
@@ -107,15 +108,15 @@ def test_w4a16_strips_of_few_slices(pkg, M, block):
 
 @pytest.mark.parametrize("M,K,N,block", [(4, 4096, 5120, 128), (4, 4096, 5121, 64), (1, 4096, 5137, 128), (8, 4096, 24577, 128), (16, 4096, 24576, 64),
                                          (16, 4096, 24609, 128), (25, 4096, 24576, 64), (25, 4096, 24577, 64), (9, 4160, 24577, 64)])
-def test_w4a16_weights_past_the_caches(pkg, M, K, N, block):
-    """The kernels that read the weights once, at the largest weights that go through the caches and above."""
+def test_w4a16_weights_of_10_and_48_mib(pkg, M, K, N, block):
+    """The kernels that read the weights once, on more of them than the tests above, ragged last tiles among them."""
     import torch
     _w4(torch, pkg, M, K, N, block, M)
     assert pkg.last_kernel().startswith("mtrt_gemm_w4a16_strips16" if M <= 16 and K % 128 == 0 else "mtrt_gemm_w4a16_skinny")
 
 
 @pytest.mark.parametrize("M,N", [(1, 12288), (9, 12288), (9, 12289), (16, 12353)])
-def test_w8a8_weights_past_the_caches(pkg, M, N):
+def test_w8a8_weights_of_48_mib(pkg, M, N):
     import torch
     g = torch.Generator(device="cuda").manual_seed(M)
     K = 4096
@@ -130,11 +131,11 @@ def test_w8a8_weights_past_the_caches(pkg, M, N):
 @pytest.mark.parametrize("M", [17, 24, 25, 32])
 def test_w8a8_up_to_32_rows(pkg, M):
     """Waves with no slice and every number of slices modulo four, at tiles below and above a workgroup to a unit, one workgroup to two tiles
-    and to one on both sides of its lines, more than two tiles to a unit, and weights on both sides of the line past the caches."""
+    and to one on both sides of its lines, more than two tiles to a unit, and weights on both sides of the lines between loads past the caches and through them."""
     import torch
     g = torch.Generator(device="cuda").manual_seed(M)
     shapes = [(128 * s, (40, 4100, 8200, 11008, 16390)[i % 5]) for i, s in enumerate((1, 2, 3, 4, 5, 6, 7, 9, 12, 13, 15, 16, 18, 23))]
-    shapes += [(2048, 10240), (2048, 10273), (4096, 12288), (4096, 12289), (8192, 16384), (8192, 16385), (4096, 24576), (4096, 24577)]
+    shapes += [(4096, 2047), (4096, 2048), (3968, 4097), (4096, 4097), (4096, 16384), (4096, 16385), (2048, 10240), (2048, 10273), (4096, 12288), (4096, 12289), (8192, 16384), (8192, 16385), (4096, 24576), (4096, 24577)]
     for K, N in shapes:
         a = torch.randint(-128, 128, (M, K), generator=g, device="cuda", dtype=torch.int8)
         w = torch.randint(-128, 128, (K, N), generator=g, device="cuda", dtype=torch.int8)
