@@ -654,10 +654,14 @@ using namespace norm_cluster;
   MTRT_NORM_GROUP_KERNELS(XN, XT, 1, 8, u, true, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 1, 16, u, true, 256)            \
   MTRT_NORM_GROUP_KERNELS(XN, XT, 1, 32, u, true, 256)                                                                \
   MTRT_NORM_GROUP_KERNELS(XN, XT, 1, 64, u, true, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 2, 64, u, true, 256)           \
-  MTRT_NORM_GROUP_KERNELS(XN, XT, 4, 64, u, true, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 8, 64, u, true, 256)           \
-  MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 64, u, true, 256)                                                               \
-  MTRT_NORM_GROUP_KERNELS(XN, XT, 8, 256, u, true, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 256, u, true, 256)        \
-  MTRT_NORM_GROUP_KERNELS(XN, XT, 8, 1024, u, true, 1024) MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 1024, u, true, 1024)
+  MTRT_NORM_GROUP_KERNELS(XN, XT, 4, 64, u, true, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 64, u, true, 256)          \
+  MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 256, u, true, 256) MTRT_NORM_GROUP_KERNELS(XN, XT, 16, 1024, u, true, 1024)     \
+  MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 8, 64, u, true, 256, false, ) MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 8, 256, u, true, 256, false, )  \
+  MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, 8, 1024, u, true, 1024, true, )
+// (f32 LayerNorm takes the 16-vector forms there: unaligned_nv in clusters.cpp)
+#define MTRT_NORM_GROUPS_OF_8_RAGGED_16_BIT(XN, XT)                                                            \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 64, u, true, 256, false, ) MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 256, u, true, 256, false, )  \
+  MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, 8, 1024, u, true, 1024, true, )
 
 MTRT_NORM_FOR_TYPE(f32, F32)
 MTRT_NORM_FOR_TYPE(f16, F16)
@@ -665,6 +669,8 @@ MTRT_NORM_FOR_TYPE(bf16, BF16)
 MTRT_NORM_GROUPS_FOR_TYPE(f32, F32)
 MTRT_NORM_GROUPS_FOR_TYPE(f16, F16)
 MTRT_NORM_GROUPS_FOR_TYPE(bf16, BF16)
+MTRT_NORM_GROUPS_OF_8_RAGGED_16_BIT(f16, F16)
+MTRT_NORM_GROUPS_OF_8_RAGGED_16_BIT(bf16, BF16)
 
 // Both forms of a kernel where either is the faster one for some rows (row_form in clusters.cpp).  The names above are those that work on every
 // vector, with 1024 lanes those that stop at the row's end; here the other ones: `e`, stop at the row's end (rows that do not fill

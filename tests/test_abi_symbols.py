@@ -91,7 +91,9 @@ def test_embedded_code_object_is_gfx950_and_has_the_kernels(pkg):
         # a workgroup per row (long rows), and the forms for rows that are not whole vectors / short rows
         for v in ("g256v8", "g256v16", "g1024v8", "g1024v16", "u8v1", "u16v1", "u32v1", "u64v1", "u64v2", "u64v4", "u64v8",
                   "u64v16", "u256v8", "u256v16", "u1024v8", "u1024v16"):
-            names += ["mtrt_layernorm_%s_%s" % (x, v), "mtrt_softmax_%s_%s" % (x, v)]
+            names += ["mtrt_softmax_%s_%s" % (x, v)]
+            if not (x == "f32" and v in ("u64v8", "u256v8", "u1024v8")):   # f32 rows take the 16-vector forms: a lane needs fewer registers there
+                names += ["mtrt_layernorm_%s_%s" % (x, v)]
         names += ["mtrt_amax_rows_" + x, "mtrt_amax_cols_" + x, "mtrt_amax_cols_split_" + x, "mtrt_amax_rows_split_" + x, "mtrt_amax_cols_u_" + x, "mtrt_amax_cols_split_u_" + x, "mtrt_amax_finish_" + x,
                   "mtrt_nvfp4_q_" + x, "mtrt_nvfp4_dq_" + x, "mtrt_nvfp4_qc_" + x, "mtrt_nvfp4_dqc_" + x]
         for q in ("i8", "f8", "i4"):

@@ -33,3 +33,10 @@ def test_the_resident_layernorm_and_the_tiles_spill_nothing(pkg, tmp_path):
     names = [n for n in private if re.match(r"mtrt_layernorm_\S+_v8r$|mtrt_gemm_(w4a16|w8a8_frag|dense_frag_\S+)_t\d|mtrt_gemm_w4a16_strips", n)]
     assert len(names) > 35
     assert {n: int(private[n]) for n in names if int(private[n]) > {"mtrt_layernorm_bf16_v8r": 32, "mtrt_gemm_w8a8_frag_t256x384_linear": 44}.get(n, 0)} == {}
+
+
+def test_row_kernels_spill_nothing(pkg, tmp_path):
+    """LayerNorm and softmax hold a row in registers; but for the LayerNorm above."""
+    private = dict(re.findall(r"\.name:\s+(mtrt_(?:layernorm|softmax)_\S+)\n\s+\.private_segment_fixed_size:\s+(\d+)", metadata(pkg, tmp_path)))
+    assert len(private) > 130
+    assert {n for n, size in private.items() if size != "0"} <= {"mtrt_layernorm_bf16_v8r"}
