@@ -196,21 +196,4 @@ template <> struct Tile<F16> {
   static __device__ __forceinline__ void store1(uint16_t* p, float v) { *p = uint16_t(f32_to_f16_bits(v)); }
 };
 
-// Runs `body` with true or false as a constant and an offset of zero, to be added to the pointer that it reads from: two bodies, whose loads
-// go past the caches or through them.  `past` is the same for the whole wave.  (As a branch around the loads alone, tensors read past
-// the caches took 2 to 4 % longer.)  Loads of two branches that differ in nothing but their hint would be made one load without it, so the
-// offset is opaque in one of them, which also ends differently.
-template <bool B> struct BoolC { static constexpr bool value = B; };
-template <typename F>
-__device__ __forceinline__ void past_or_through(bool past, F body) {
-  if (past) {
-    int64_t zero = 0;
-    __asm__ volatile("" : "+s"(zero));
-    body(BoolC<true>{}, zero);
-    __asm__ volatile("");
-  } else {
-    body(BoolC<false>{}, 0);
-  }
-}
-
 }  // namespace mtrt_dev

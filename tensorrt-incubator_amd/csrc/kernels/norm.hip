@@ -23,7 +23,6 @@
 // All arithmetic is f32 with the operation order above; reductions are trees
 // rather than the host's left-to-right sums, which the float tolerance covers.
 #include "common.hpp"
-#include "row_reads.hpp"
 
 using namespace mtrt_dev;
 
@@ -102,7 +101,7 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
   }
 }
 
-// LayerNorm reads past the caches always, softmax as in row_reads.hpp.  (LayerNorm, us, past and through, three tensors in turn; each from memory; with a launch that makes x in front and one that
+// LayerNorm reads past the caches always, softmax but in the kernels whose names end in t (softmax_reads_past in clusters.cpp).  (LayerNorm, us, past and through, three tensors in turn; each from memory; with a launch that makes x in front and one that
 // reads y behind, all three: f32 [256, 4096] 4.8, 4.8; 5.8, 6.2; 11.9, 12.0; [512, 4096] 5.2, 5.2; 6.1, 6.5; 16.7, 17.5; bf16 [512, 4096] 4.4, 4.4; 5.0, 5.4;
 // 11.7, 11.9; [1024, 4096] 4.5, 4.6; 5.6, 6.0; 15.0, 15.4; f16 [2796, 1500] 5.7, 5.5; 6.5, 6.5; 21.3, 21.7; bf16 [250, 14165] 6.6, 6.4; 7.2, 7.5; 16.3, 16.6.)
 // What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back:
@@ -243,19 +242,16 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
   }
 }
 
-template <typename X, int NV>
+template <typename X, int NV, bool PAST>
 __device__ __forceinline__ void softmax_rows(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                              int64_t rows, int64_t d) {
   // the wave index as a scalar: the row pointers are then wave-uniform and the accesses need one lane offset, not an address pair each
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;
-  if (d == int64_t(Vec<X>::kElems) * kWave * NV) {   // (whole cache lines)
+  if (PAST && d == int64_t(Vec<X>::kElems) * kWave * NV)   // (whole cache lines)
     softmax_row<X, NV, true, true>(x, y, row, d);
-  } else {
-    past_or_through(softmax_reads_past(rows, d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
-      softmax_row<X, NV, false, decltype(past)::value>(x + zero, y, row, d);
-    });
-  }
+  else
+    softmax_row<X, NV, false, PAST>(x, y, row, d);
 }
 
 // ---- rows longer than one wave's registers, and rows of any length or alignment: a GROUP of lanes owns one row ----
@@ -472,20 +468,17 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   if (extra) Tile<X>::store1(y + row * d + ec, ee * inv);
 }
 
-template <typename X, int NV, int THREADS, bool RAGGED, bool ENDS>
+template <typename X, int NV, int THREADS, bool RAGGED, bool ENDS, bool PAST>
 __device__ __forceinline__ void softmax_group(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                               int64_t rows, int64_t d) {
   __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
   constexpr bool kKeep = THREADS <= 256 || NV * Vec<X>::kElems <= 64;
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
-  if (!RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV) {   // (whole cache lines)
+  if (PAST && !RAGGED && !(ENDS && THREADS < 1024) && d == int64_t(Vec<X>::kElems) * THREADS * NV)   // (whole cache lines)
     softmax_group_row<X, NV, THREADS, true, true, kKeep, false, true>(x, y, row, d, lds);
-  } else {
-    past_or_through(softmax_reads_past(rows, d * int64_t(sizeof(typename X::storage))), [&](auto past, int64_t zero) {
-      softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED, decltype(past)::value>(x + zero, y, row, d, lds);
-    });
-  }
+  else
+    softmax_group_row<X, NV, THREADS, false, !ENDS, kKeep, RAGGED, PAST>(x, y, row, d, lds);
 }
 
 // ---- any D, any alignment: one workgroup per row, row re-read from cache -------------
@@ -606,6 +599,7 @@ using namespace norm_cluster;
 // [4096, 4096] 11.3 -> 12.7 us and [16384, 4096] 47.4 -> 50.4 us, hence only inside that window).
 // Entry points.  mtrt_layernorm_<t>_v<NV>(x, gamma, beta, y, rows, d, eps)
 //                mtrt_softmax_<t>_v<NV>(x, y, rows, d)         NV = vectors per lane
+// Softmax kernels, here and below, with a t at the end: rows read through the caches, which don't fill all vectors.
 #define MTRT_LN_OCCUPANCY_1
 #define MTRT_LN_OCCUPANCY_2
 #define MTRT_LN_OCCUPANCY_4
@@ -616,7 +610,9 @@ using namespace norm_cluster;
       const XT::storage* x, const XT::storage* gamma, const XT::storage* beta, XT::storage* y, int64_t rows,  \
       int64_t d, float eps) { layernorm_rows<XT, NV>(x, gamma, beta, y, rows, d, eps); }                      \
   extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_softmax_##XN##_v##NV(                        \
-      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV>(x, y, rows, d); }
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, true>(x, y, rows, d); }  \
+  extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_softmax_##XN##_v##NV##t(                     \
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, false>(x, y, rows, d); }
 
 #define MTRT_NORM_FOR_TYPE(XN, XT)                                                                            \
   MTRT_NORM_KERNELS(XN, XT, 1) MTRT_NORM_KERNELS(XN, XT, 2) MTRT_NORM_KERNELS(XN, XT, 4)                       \
@@ -643,7 +639,9 @@ using namespace norm_cluster;
       int64_t d, float eps) { layernorm_group<XT, NV, THREADS, RAGGED, ENDS>(x, gamma, beta, y, rows, d, eps); }
 #define MTRT_SOFTMAX_GROUP_KERNEL(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK, ENDS, END)                          \
   extern "C" __global__ void __launch_bounds__(BLOCK) mtrt_softmax_##XN##_##TAG##THREADS##v##NV##END(          \
-      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_group<XT, NV, THREADS, RAGGED, ENDS>(x, y, rows, d); }
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_group<XT, NV, THREADS, RAGGED, ENDS, true>(x, y, rows, d); }   \
+  extern "C" __global__ void __launch_bounds__(BLOCK) mtrt_softmax_##XN##_##TAG##THREADS##v##NV##END##t(       \
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_group<XT, NV, THREADS, RAGGED, ENDS, false>(x, y, rows, d); }
 // (f32 LayerNorm at element alignment: nearly full rows, [2000, 15001], 49.4 us with every vector worked on and 51.1 without)
 #define MTRT_NORM_GROUP_KERNELS(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK)                                       \
   MTRT_LAYERNORM_GROUP_KERNEL(XN, XT, NV, THREADS, TAG, RAGGED, BLOCK, (THREADS == 1024 && !(RAGGED && Vec<XT>::kElems == 4)), )               \

@@ -600,6 +600,18 @@ const char *row_form(bool layernorm, int32_t dtype, bool ragged, int lanes, int 
   return "";
 }
 
+// Softmax rows that are no whole cache lines, of 20 to 80 MiB together, are read through the caches: the line that two rows share is fetched once, and what an
+// earlier launch has left in the Infinity Cache comes from there.  Whole lines gain from the second alone, and a launch that has just made x, or memory, is the
+// more common place for it to come from.  us, past and through, (rows, columns): three tensors in turn; each from memory; with a launch that makes x in front and
+// one that reads y behind, all three.  No whole lines: f16 (17476, 1500) 19.8, 17.2; 20.7, 20.8; 64.2, 62.2; (8735, 3001) 21.3, 17.8; 22.3, 22.4; 64.7, 61.8; bf16
+// (4368, 9001) 32.9, 26.3; 33.6, 34.1; 88.5, 84.4; f32 (12750, 1028) 19.5, 16.6; 20.3, 20.0; 58.1, 56.7; half lines (6553, 2000) 18.9, 16.4; 19.8, 20.3; 56.5, 57.0.
+// Whole lines: f16 (25600, 1024) 17.7, 16.1; 18.7, 19.5; 54.7, 56.8; (4096, 4096) 11.4, 10.8; 12.8, 13.4; 37.1, 39.3; f32 (12800, 1024) 18.0, 16.5; 19.1, 19.7;
+// 53.6, 56.7; (3268, 6016) 26.7, 23.4; 27.7, 28.8; 79.2, 80.6.  Smaller tensors of either kind: f16 (2097, 1500) 4.6, 4.4; 5.2, 5.3; 18.6, 18.9; f32 (698, 4501) 5.2,
+// 5.6; 5.8, 6.3; 18.7, 19.0; larger ones: f16 (38447, 1500) 41.2, 41.0; 42.1, 42.0; f32 (6406, 4501) 40.5, 41.0; 41.5, 42.1.
+bool softmax_reads_past(int64_t rows, int64_t row_bytes) {
+  return row_bytes % 128 == 0 || rows * row_bytes <= int64_t(20) << 20 || rows * row_bytes > int64_t(80) << 20;
+}
+
 } // namespace
 
 extern "C" {
@@ -1183,17 +1195,18 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
   const int nv = vec_ok ? pick_nv(d / per_vec) : 0;
   int64_t rows_arg = rows, d_arg = d;
   void *args[] = {&x, &y, &rows_arg, &d_arg};
+  const char *through = softmax_reads_past(rows, d * eb) ? "" : "t";
   // Rows of at most 32 vectors: 8, 16 or 32 lanes per row, several rows to a wave (whatever the alignment).
   if (d / per_vec <= 32 && rows <= kMaxRowsPerWaveKernels) {
     const int lanes = d / per_vec <= 8 ? 8 : (d / per_vec <= 16 ? 16 : 32);
-    return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + lanes + "v1", blocks_for(rows, kBlock / lanes), kBlock, as_hip(stream), args);
+    return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + lanes + "v1" + through, blocks_for(rows, kBlock / lanes), kBlock, as_hip(stream), args);
   }
   if (nv && rows <= kMaxRowsPerWaveKernels)
-    return launch(st, KernelName("mtrt_softmax_") + xn + "_v" + nv,
+    return launch(st, KernelName("mtrt_softmax_") + xn + "_v" + nv + through,
                   blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
   int threads, gnv;
   if (vec_ok && !nv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-    return launch(st, KernelName("mtrt_softmax_") + xn + "_g" + threads + "v" + gnv + row_form(false, dtype, false, threads, gnv, rows, d / per_vec, num_compute_units(st)), uint32_t(rows), uint32_t(threads),
+    return launch(st, KernelName("mtrt_softmax_") + xn + "_g" + threads + "v" + gnv + row_form(false, dtype, false, threads, gnv, rows, d / per_vec, num_compute_units(st)) + through, uint32_t(rows), uint32_t(threads),
                   as_hip(stream), args);
   // Row lengths that are not whole vectors, or operands that are not 16-byte aligned: the same two schemes with
   // 128-bit accesses at element alignment and the last d % per_vec elements of a row moved one by one.
@@ -1201,11 +1214,11 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
     int rnv = pick_nv(d / per_vec);
     if (rnv && rows <= kMaxRowsPerWaveKernels) {
       rnv = unaligned_nv(dtype, rnv, false);
-      return launch(st, KernelName("mtrt_softmax_") + xn + "_u64v" + rnv, blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
+      return launch(st, KernelName("mtrt_softmax_") + xn + "_u64v" + rnv + through, blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
     }
     if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv)) {
       gnv = unaligned_nv(dtype, gnv, false);
-      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + gnv + row_form(false, dtype, true, threads, gnv, rows, d / per_vec, num_compute_units(st)), uint32_t(rows), uint32_t(threads),
+      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + gnv + row_form(false, dtype, true, threads, gnv, rows, d / per_vec, num_compute_units(st)) + through, uint32_t(rows), uint32_t(threads),
                     as_hip(stream), args);
     }
   }

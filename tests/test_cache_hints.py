@@ -41,7 +41,7 @@ def code(pkg, tmp_path_factory):
 
 def test_rows_held_in_registers_are_written_past_the_caches(code):
     names, accesses = code
-    kernels = names(r"mtrt_(layernorm|softmax)_\w+_[vgu]\d+(v\d+)?[rea]?")
+    kernels = names(r"mtrt_(layernorm|softmax)_\w+_[vgu]\d+(v\d+)?[rea]?t?")
     assert len(kernels) > 130
     folded = {"mtrt_softmax_f32_v1", "mtrt_softmax_bf16_v1"}         # whole rows of up to 64 vectors: the compiler makes one store of two branches
     for kernel, found in accesses(kernels).items():
@@ -70,15 +70,13 @@ def test_layernorm_reads_its_rows_past_the_caches(code):
         assert past == found["global_store_dwordx4", True] > 0 and found["global_load_dwordx4", False] == 2 * past, kernel
 
 
-def test_softmax_reads_its_rows_either_way(code):
-    """Two bodies with as many loads each (row_reads.hpp says which one runs), a third for rows that fill all vectors, past the caches."""
+def test_softmax_reads_its_rows_as_its_name_says(code):
+    """Through the caches in the kernels that end in t, past them in the others, of which each has one."""
     names, accesses = code
-    kernels = names(r"mtrt_softmax_\w+_[vgu]\d+(v\d+)?[ea]?")
-    assert len(kernels) > 60
+    kernels = names(r"mtrt_softmax_\w+_[vgu]\d+(v\d+)?[ea]?t?")
+    assert len(kernels) > 120 and all(k + "t" in kernels for k in kernels if not k.endswith("t"))
     for kernel, found in accesses(kernels).items():
-        through, past = found["global_load_dwordx4", False], found["global_load_dwordx4", True]
-        whole = "_u" not in kernel and not ("_g256" in kernel and kernel.endswith("e"))
-        assert through > 0 and past == through * (2 if whole else 1), kernel
+        assert found["global_load_dwordx4", not kernel.endswith("t")] > 0 and found["global_load_dwordx4", kernel.endswith("t")] == 0, kernel
 
 
 def test_few_rows_read_int8_and_int4_weights_past_the_caches(code):

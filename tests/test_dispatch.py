@@ -1,6 +1,8 @@
 """What the entry points launch, seen on the CPU (dispatch.py): the words in which workgroups meet (tickets of K-split GEMMs, blocks of
 grid-wide reductions) belong to a stream, or to the one launch where it is recorded into a graph; a GEMM that gets none, for
 whatever reason, runs unsplit, a reduction recorded when there are no more takes its stream's."""
+import re
+
 import pytest
 
 import dispatch
@@ -367,3 +369,17 @@ def test_16_bit_linears_of_few_rows_read_weights_of_more_than_48_mib_past_the_ca
         assert gpu.forms[-1] == ("mtrt_gemm_dense_frag_f16_rows16", past)
         gpu.linear(None, 4, 2048, N, pkg.BF16, q_dtype=pkg.F8E4M3FN)
         assert gpu.forms[-1] == ("mtrt_gemm_dense_frag_bf16_rows16_f8", past)
+
+
+@pytest.mark.parametrize("dtype,item", [("F32", 4), ("F16", 2), ("BF16", 2)])
+def test_softmax_rows_that_share_cache_lines_are_read_through_the_caches_from_20_to_80_mib(gpu, pkg, dtype, item):
+    """... in every form of the kernel, and of rows that are whole lines none, whatever their size."""
+    low, high, seen = 20 << 20, 80 << 20, set()
+    for row_bytes in (20, 64, 100, 192, 400, 1000, 1040, 3000, 3008, 4112, 10004, 12016, 18004, 20016, 49016, 200000, 128, 256, 1920, 2048, 3968, 8192, 24064, 65536, 1 << 17):
+        for rows, inside in ((1, False), (low // row_bytes, False), (low // row_bytes + 1, True), (high // row_bytes, True), (high // row_bytes + 1, False), ((1 << 36) // row_bytes, False)):
+            assert gpu.lib.mtrt_hip_softmax(None, 256, 256, getattr(pkg, dtype), rows, row_bytes // item) == 0
+            name = gpu.launches[-1][0]
+            assert name.endswith("t") == (inside and row_bytes % 128 != 0), (rows, row_bytes, name)
+            seen.add(name)
+    forms = {re.sub("[ea]t$", "t", n.split("_")[3]) for n in seen}
+    assert {f + "t" for f in ("u8v1", "u16v1", "u32v1", "u64v1", "u64v4", "v4", "v16", "g256v8", "g1024v16")} <= forms, forms
