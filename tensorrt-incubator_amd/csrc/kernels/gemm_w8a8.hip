@@ -374,7 +374,7 @@ extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_small16(
 // ... M <= 32, the same arguments; grid = ceil(N / 32) or the number of compute units: which one stands beside the launch.  Against eight waves to
 // a tile that each bring their own rows, as in gemm_core::rows32 (there 64 rows still run so), us, (M, K, N), weights of three sets in turn: (32, 1152, 9216)
 // 7.0, 5.5; (17, 2048, 11008) 9.3, 7.6; (32, 4096, 11008) 13.2, 11.4; (32, 8192, 11008) 24.7, 22.3; (17, 4096, 4096) 6.2, 5.9; from memory the third 17.0, 13.6;
-// the other way up to eight slices by no more tiles than units, (32, 640, 4096) 3.4, 3.6.
+// the other way up to six slices by no more tiles than units, (17, 384, 4096) 2.8, 3.0; (32, 640, 4096) 3.1, 3.5, from memory 3.8, 3.4; 4.2, 4.4.
 extern "C" __global__ void __launch_bounds__(256) mtrt_gemm_w8a8_frag_rows32(
     const int8_t* __restrict__ a, const v4i* __restrict__ w_frag, const float* __restrict__ a_scale,
     const float* __restrict__ w_scale, uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, uint32_t a_step,

@@ -101,9 +101,10 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec
   }
 }
 
-// LayerNorm reads past the caches always, softmax but in the kernels whose names end in t (softmax_reads_past in clusters.cpp).  (LayerNorm, us, past and through, three tensors in turn; each from memory; with a launch that makes x in front and one that
-// reads y behind, all three: f32 [256, 4096] 4.8, 4.8; 5.8, 6.2; 11.9, 12.0; [512, 4096] 5.2, 5.2; 6.1, 6.5; 16.7, 17.5; bf16 [512, 4096] 4.4, 4.4; 5.0, 5.4;
-// 11.7, 11.9; [1024, 4096] 4.5, 4.6; 5.6, 6.0; 15.0, 15.4; f16 [2796, 1500] 5.7, 5.5; 6.5, 6.5; 21.3, 21.7; bf16 [250, 14165] 6.6, 6.4; 7.2, 7.5; 16.3, 16.6.)
+// LayerNorm reads past the caches always, softmax but in the kernels whose names end in t (softmax_reads_past in clusters.cpp).  (LayerNorm, us, past and
+// through, three tensors in turn; each from memory; with a launch that makes x in front and one that reads y behind, all three: f32 [256, 4096] 4.8, 4.8; 5.8, 6.2;
+// 11.9, 12.0; [512, 4096] 5.2, 5.2; 6.1, 6.5; 16.7, 17.5; bf16 [512, 4096] 4.4, 4.4; 5.0, 5.4; 11.7, 11.9; [1024, 4096] 4.5, 4.6; 5.6, 6.0; 15.0, 15.4; f16
+// [2796, 1500] 5.7, 5.5; 6.5, 6.5; 21.3, 21.7; bf16 [250, 14165] 6.6, 6.4; 7.2, 7.5; 16.3, 16.6.)
 // What is written goes past the caches whatever its size.  (Left to them, a large result is shorter by what the launches behind it then write back:
 // alone softmax bf16 of 134 MB 44.1 -> 46.8 us where each result has memory of its own, 44.3 -> 46.7 from memory, with a copy of 268 MB behind each 133.2 ->
 // 135.7, between the launches that make x and take y 128.7 -> 127.6; LayerNorm bf16 [8178, 4096] 22.6 -> 21.4, 23.0 -> 22.3, 113.6 -> 116.8, 62.0 -> 60.6; of 101 MB
