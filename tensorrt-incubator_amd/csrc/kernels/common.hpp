@@ -136,6 +136,8 @@ __device__ __forceinline__ float f8_to_f32(uint32_t packed) {
 // cycles each: through LDS (ds_bpermute, what __shfl_xor is) a step of a dependent chain is a trip of about a hundred.
 // REPEATS: lanes eight apart in a row of sixteen hold the same (they have been combined already), so that the lane four on is as good as
 // i ^ 4 and one instruction reaches it.
+template <int OFF, bool REPEATS = false, typename Op>
+__device__ __forceinline__ double xor_step(double v, Op op);
 template <int OFF, bool REPEATS = false, typename T, typename Op>
 __device__ __forceinline__ T xor_step(T v, Op op) {
   static_assert(sizeof(T) == 4 && OFF >= 1 && OFF <= 32 && (OFF & (OFF - 1)) == 0, "one 32-bit value per lane");
@@ -154,6 +156,21 @@ __device__ __forceinline__ T xor_step(T v, Op op) {
     }
     return op(v, __builtin_bit_cast(T, other));
   }
+}
+// The same for 64-bit values, word by word.
+template <int OFF, bool REPEATS, typename Op>
+__device__ __forceinline__ double xor_step(double v, Op op) {
+  struct Words { uint32_t lo, hi; };
+  struct Pick {                                        // what the exchange hands over: (own, other), or (a, b) in one order in both lanes
+    uint32_t* a;
+    uint32_t* b;
+    __device__ __forceinline__ uint32_t operator()(uint32_t x, uint32_t y) const { *a = x; *b = y; return x; }
+  };
+  const Words w = __builtin_bit_cast(Words, v);
+  Words a, b;
+  (void)xor_step<OFF, REPEATS>(w.lo, Pick{&a.lo, &b.lo});
+  (void)xor_step<OFF, REPEATS>(w.hi, Pick{&a.hi, &b.hi});
+  return op(__builtin_bit_cast(double, a), __builtin_bit_cast(double, b));
 }
 // Every lane gets the value of its group of LANES neighbouring lanes, combined by halves: far lanes first.
 template <int LANES, bool REPEATS = false, typename T, typename Op>
@@ -175,6 +192,7 @@ __device__ __forceinline__ T wave_reduce_lds(T v, Op op) {
 struct MaxU32 { __device__ __forceinline__ uint32_t operator()(uint32_t a, uint32_t b) const { return a > b ? a : b; } };
 struct MaxF32 { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
 struct SumF32 { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
+struct SumF64 { __device__ __forceinline__ double operator()(double a, double b) const { return a + b; } };
 
 // ---- single-element access ------------------------------------------------------
 constexpr int kTile = 16;            // elements a lane carries per trip in the elementwise kernels

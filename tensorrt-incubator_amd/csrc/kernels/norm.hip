@@ -75,26 +75,51 @@ template <> struct Vec<F16> {
   }
 };
 
-// Load the wave's row into registers: NV vectors per lane.  Every lane always loads (vectors past
-// the end of the row re-read the row's last vector and are replaced by `fill` afterwards), so the
+// Where a softmax row that starts off a cache line is cut: an access of the wave covers whole lines but at the row's two ends.  `head` elements in
+// front of the first 16-byte boundary move one per lane, with those behind the last whole vector; `shift` is that vector's place in its
+// line, and so the number of lanes that the first access leaves out (as far as a row that fills its lanes allows).
+// What bounds these rows is memory: an access that starts inside a line leaves a part of it to the next one, which is fetched and written as a part.
+// us, vectors from the row's first element on, on 16-byte boundaries, and on lines, f16 [48000, 1500] 51.9, 51.4, 48.5; [8000, 9001] 58.7, 52.3, 49.5; bf16
+// [1084, 43165] 54.4, 46.9, 44.7; f32 [24000, 1501] 51.4, 51.1, 49.5; whole vectors, f16 [24000, 3000] 49.9, 48.7.  (Staged through LDS, four rows' whole
+// range at once, 48.3 for the first, but 52.9 with 1503 elements and 66 with 4500; LayerNorm bf16 [1500, 9011] 16.0 -> 14.0, but [700, 10243] 8.7 -> 9.4: behind
+// a head its parameters' vectors lie off their boundaries.)
+// A head puts the row's elements into other lanes, so its sum is taken in 64 bits: what the order of the terms changes there is a 2^-28th of the f32
+// result's last place, and equal rows give equal bits wherever they lie.  (48.5 -> 49.3 and 44.7 -> 47.0 for the first and the third; the longer part is the exchange.)
+// A shift alone is undone by one exchange of the lanes' sums.
+struct RowCut { int head, shift; };
+template <bool CUT> struct RowSum { using type = float; using op = SumF32; };
+template <> struct RowSum<true> { using type = double; using op = SumF64; };
+// Of the places that a lane's vectors j = 0, 1, ... have, whether one is the row's, and the nearest that is: only the first can lie in front of it.
+__device__ __forceinline__ bool within(int j, int place, int shift, int end) { return place < end && (j > 0 || place >= shift); }
+__device__ __forceinline__ int held(int j, int place, int shift, int end) { return j > 0 ? min(place, end - 1) : max(shift, min(place, end - 1)); }
+template <typename X, int VECTORS>
+__device__ __forceinline__ RowCut cut_row(const typename X::storage* xr, const typename X::storage* yr, int64_t d) {
+  const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(xr)), to = uint32_t(reinterpret_cast<uintptr_t>(yr));
+  const bool both = ((at ^ to) & 15u) == 0;            // (else no cut puts both on boundaries)
+  const int head = both ? int((0u - at) & 15u) / int(sizeof(typename X::storage)) : 0;
+  return {head, both ? min(int((at + 15u) / 16u) & 7, VECTORS - (int(d) - head) / Vec<X>::kElems) : 0};
+}
+
+// Load the wave's row into registers: NV vectors per lane, those in places [shift, end) the row's (see RowCut).  Every lane always loads (the
+// other places re-read the row's first or last vector and are replaced by `fill` afterwards), so the
 // loads are issued back to back with no branches between them; with FULL (the row fills all
 // 64 * NV vectors) the replacement disappears as well.
 template <typename X, int NV, bool FULL, bool PAST>
-__device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int nvec, int lane, float fill,
+__device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int shift, int end, int lane, float fill,
                                          float (&v)[NV * Vec<X>::kElems]) {
   constexpr int E = Vec<X>::kElems;
   u32x4 t[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
-    const u32x4* p = row + (FULL ? idx : min(idx, nvec - 1));
+    const u32x4* p = row + (FULL ? idx : held(j, idx, shift, end));
     t[j] = PAST ? __builtin_nontemporal_load(p) : *p;
   }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     Vec<X>::unpack(t[j], &v[j * E]);
     if (!FULL) {
-      const bool live = lane + kWave * j < nvec;
+      const bool live = within(j, lane + kWave * j, shift, end);
 #pragma unroll
       for (int k = 0; k < E; ++k) v[j * E + k] = live ? v[j * E + k] : fill;
     }
@@ -211,8 +236,9 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
   const int lane = threadIdx.x & (kWave - 1);
   const int nvec = int(d / E);
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + row * d);
+  const int shift = FULL ? 0 : cut_row<X, kWave * NV>(x + row * d, y + row * d, d).shift, end = nvec + shift;
   float v[NV * E];
-  load_row<X, NV, FULL, PAST>(xr, nvec, lane, -INFINITY, v);
+  load_row<X, NV, FULL, PAST>(xr - shift, shift, end, lane, -INFINITY, v);
 
   constexpr bool kLds = NV == 2 || NV == 4;
   float mx = -INFINITY;
@@ -225,6 +251,7 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
     v[i] = __expf(v[i] - mx);                        // exp(-inf) = 0 for the fill lanes
     s = s + v[i];
   }
+  if (!FULL) s = __shfl(s, (lane + shift) & (kWave - 1));   // each lane's sum to the lane that has it where the row starts on a line
   s = row_reduce<kLds>(s, SumF32());
   // e / s as e * (1/s): one correctly rounded reciprocal per row instead of a divide per element; at most one
   // f32 ulp from the quotient.  Together with the hardware exponential (2^(d * log2 e), a few f32 ulps off for
@@ -232,14 +259,14 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
   // ulp and a remainder-corrected quotient the share of f16 outputs that differ from the host's by one ulp
   // stayed at 0.05 % (4096 x 4096, sigma 2) and the launch took 1 us longer, so the short forms are kept.
   const float inv = 1.0f / s;
-  u32x4* yr = reinterpret_cast<u32x4*>(y + row * d);
+  u32x4* yr = reinterpret_cast<u32x4*>(y + row * d) - shift;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
     float o[E];
 #pragma unroll
     for (int k = 0; k < E; ++k) o[k] = v[j * E + k] * inv;
-    if (FULL || idx < nvec) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
+    if (FULL || within(j, idx, shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
 }
 
@@ -267,15 +294,16 @@ __device__ __forceinline__ void softmax_rows(const typename X::storage* __restri
 template <bool RAGGED> struct RowVector { typedef u32x4 type; };
 template <> struct RowVector<true> { typedef u32x4 type __attribute__((aligned(2))); };
 
-template <int THREADS, typename Op>
-__device__ __forceinline__ float group_reduce(float v, Op op, float* lds) {
+template <int THREADS, typename T, typename Op>
+__device__ __forceinline__ T group_reduce(T v, Op op, void* shared) {
+  T* lds = static_cast<T*>(shared);
   if constexpr (THREADS < kWave) return lanes_reduce<THREADS>(v, op);   // several rows per wave: exchanges stay inside the row's lanes
   v = wave_reduce(v, op);
   if (THREADS == kWave) return v;
   __syncthreads();                                   // lds may still be read from the previous reduction
   if ((threadIdx.x & (kWave - 1)) == 0) lds[threadIdx.x / kWave] = v;
   __syncthreads();
-  float r = lds[0];
+  T r = lds[0];
 #pragma unroll
   for (int w = 1; w < THREADS / kWave; ++w) r = op(r, lds[w]);
   return r;                                          // the same value, combined in the same order, in every lane
@@ -295,12 +323,17 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
                                                     const typename X::storage* __restrict__ gamma,
                                                     const typename X::storage* __restrict__ beta,
                                                     typename X::storage* __restrict__ y, int64_t row, int64_t d, float eps,
-                                                    float* lds) {
+                                                    double* lds) {
   constexpr int E = Vec<X>::kElems;
   using V = typename RowVector<RAGGED>::type;
   const int lane = int(threadIdx.x) & (THREADS - 1);
   const int nvec = int(d / E), tail = RAGGED ? int(d - int64_t(nvec) * E) : 0;
   const V* xr = reinterpret_cast<const V*>(x + row * d);
+  const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
+  const int ec = nvec * E + lane;
+  // asked for with the vectors, by every lane: in a branch, or behind them, it is a second trip to memory
+  typename X::storage xb = 0;
+  if constexpr (RAGGED) xb = (x + row * d)[min(ec, int(d) - 1)];
   u32x4 t[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
@@ -309,9 +342,7 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
     if (RAGGED && ALL && nvec == 0) t[j] = (u32x4){0u, 0u, 0u, 0u};   // a row shorter than one vector: only the scalar elements below
     else t[j] = __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1)));
   }
-  const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
-  const int64_t ec = int64_t(nvec) * E + lane;
-  const float xe = extra ? Tile<X>::load1(x + row * d + ec) : 0.0f;
+  const float xe = extra ? Tile<X>::load1(&xb) : 0.0f;
   const float fd = float(d);
   float sum = xe;
 #pragma unroll
@@ -378,7 +409,7 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
                                                 const typename X::storage* __restrict__ gamma,
                                                 const typename X::storage* __restrict__ beta,
                                                 typename X::storage* __restrict__ y, int64_t rows, int64_t d, float eps) {
-  __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
+  __shared__ double lds[THREADS >= kWave ? THREADS / kWave : 1];
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
   if (!RAGGED && (!ENDS || THREADS == 1024 || NV == 8) && d == int64_t(Vec<X>::kElems) * THREADS * NV)
@@ -392,38 +423,46 @@ __device__ __forceinline__ void layernorm_group(const typename X::storage* __res
 // more than 64 elements).
 template <typename X, int NV, int THREADS, bool FULL, bool ALL, bool KEEP, bool RAGGED, bool PAST>
 __device__ __forceinline__ void softmax_group_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
-                                                  int64_t row, int64_t d, float* lds) {
+                                                  int64_t row, int64_t d, double* lds) {
   constexpr int E = Vec<X>::kElems;
   using V = typename RowVector<RAGGED>::type;
   const int lane = int(threadIdx.x) & (THREADS - 1);
-  const int nvec = int(d / E), tail = RAGGED ? int(d - int64_t(nvec) * E) : 0;
-  const V* xr = reinterpret_cast<const V*>(x + row * d);
+  constexpr bool kCut = RAGGED && THREADS >= kWave && NV > 2;   // (fewer vectors: what the 64-bit sums cost is more, bf16 [96000, 750] 51.3, 54.6)
+  using Sum = typename RowSum<kCut>::type;
+  using Add = typename RowSum<kCut>::op;
+  RowCut cut = {0, 0};
+  if constexpr (kCut) cut = cut_row<X, THREADS * NV>(x + row * d, y + row * d, d);
+  const int nvec = (int(d) - cut.head) / E, tail = RAGGED ? int(d) - nvec * E : 0, end = nvec + cut.shift;
+  const V* xr = reinterpret_cast<const V*>(x + row * d + cut.head) - cut.shift;
+  const bool extra = RAGGED && lane < tail;          // this lane also owns an element outside the vectors
+  const int ec = (lane < cut.head ? 0 : nvec * E) + lane;
+  // asked for with the vectors, by every lane: in a branch, or behind them, it is a second trip to memory
+  typename X::storage xb = 0;
+  if constexpr (RAGGED) xb = (x + row * d)[min(ec, int(d) - 1)];
   u32x4 t[NV];
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    if (!wave_has<THREADS, ALL>(j, nvec)) break;
+    if (!wave_has<THREADS, ALL>(j, end)) break;
     const int idx = lane + THREADS * j;
     if (!RAGGED || !ALL || nvec > 0)                  // (a row shorter than one vector: only the scalar elements below)
-      t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : min(idx, nvec - 1))) : xr[FULL ? idx : min(idx, nvec - 1)];
+      t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : held(j, idx, cut.shift, end))) : xr[FULL ? idx : held(j, idx, cut.shift, end)];
   }
   // What lies past the row becomes -infinity where it is loaded: it changes no maximum and its exponential is zero, and the passes
   // below need not tell it from the row (us, f16 [1084, 50000] 61.2 -> 53.0, f32 [2000, 25001] 102 -> 97, bf16 [200, 8191] 7.5 -> 7.1; [48000, 1500] as before).
   if (!FULL) {
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
-      if (!wave_has<THREADS, ALL>(j, nvec)) break;
-      const bool live = lane + THREADS * j < nvec;
+      if (!wave_has<THREADS, ALL>(j, end)) break;
+      const bool live = within(j, lane + THREADS * j, cut.shift, end);
 #pragma unroll
       for (int k = 0; k < 4; ++k) t[j][k] = live ? t[j][k] : Vec<X>::kMinusInf;
     }
   }
-  const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
-  const int64_t ec = int64_t(nvec) * E + lane;
-  const float xe = extra ? Tile<X>::load1(x + row * d + ec) : -INFINITY;
+  const float xe = extra ? Tile<X>::load1(&xb) : -INFINITY;
   float mx = xe;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    if (!wave_has<THREADS, ALL>(j, nvec)) break;
+    if (!wave_has<THREADS, ALL>(j, end)) break;
     float v[E];
     Vec<X>::unpack(t[j], v);
 #pragma unroll
@@ -432,10 +471,12 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   mx = group_reduce<THREADS>(mx, MaxF32(), lds);
   float e[KEEP ? NV * E : 1];
   const float ee = extra ? __expf(xe - mx) : 0.0f;
-  float s = ee;
+  constexpr int kSums = kCut ? 4 : 1;                  // (a chain of 64-bit additions is long)
+  Sum s[kSums] = {};
+  s[0] = ee;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    if (!wave_has<THREADS, ALL>(j, nvec)) break;
+    if (!wave_has<THREADS, ALL>(j, end)) break;
     float v[E];
     opaque(t[j]);
     Vec<X>::unpack(t[j], v);
@@ -443,15 +484,15 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
     for (int k = 0; k < E; ++k) {
       const float ev = __expf(v[k] - mx);
       if (KEEP) e[j * E + k] = ev;
-      s = s + ev;
+      s[k % kSums] = s[k % kSums] + ev;
     }
   }
-  s = group_reduce<THREADS>(s, SumF32(), lds);
-  const float inv = 1.0f / s;                         // e * (1/s), as in softmax_row
-  V* yr = reinterpret_cast<V*>(y + row * d);
+  if (kCut) s[0] = (s[0] + s[kSums / 2]) + (s[kSums / 4] + s[kSums - 1]);
+  const float inv = 1.0f / float(group_reduce<THREADS>(s[0], Add(), lds));                         // e * (1/s), as in softmax_row
+  V* yr = reinterpret_cast<V*>(y + row * d + cut.head) - cut.shift;
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
-    if (!wave_has<THREADS, ALL>(j, nvec)) break;
+    if (!wave_has<THREADS, ALL>(j, end)) break;
     const int idx = lane + THREADS * j;
     float o[E];
     if (KEEP) {
@@ -464,7 +505,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
 #pragma unroll
       for (int k = 0; k < E; ++k) o[k] = __expf(v[k] - mx) * inv;
     }
-    if (FULL || idx < nvec) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
+    if (FULL || within(j, idx, cut.shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
   if (extra) Tile<X>::store1(y + row * d + ec, ee * inv);
 }
@@ -472,7 +513,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
 template <typename X, int NV, int THREADS, bool RAGGED, bool ENDS, bool PAST>
 __device__ __forceinline__ void softmax_group(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                               int64_t rows, int64_t d) {
-  __shared__ float lds[THREADS >= kWave ? THREADS / kWave : 1];
+  __shared__ double lds[THREADS >= kWave ? THREADS / kWave : 1];
   constexpr bool kKeep = THREADS <= 256 || NV * Vec<X>::kElems <= 64;
   const int64_t row = group_row<THREADS>();
   if (row >= rows) return;                           // groups of a wave or less only (no barrier follows there); grid = rows otherwise
