@@ -466,11 +466,14 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const voi
  *                     w_scale: f16 [1,N] (one block of all of K, K % 64 == 0); w unused
  *   MTRT_LINEAR_DENSE: x' = q_dtype < 0 ? x : dequantize(quantize(x, x_scale, q_dtype), x_scale); y = narrow(x' . w + bias[n]);
  *                     w: [N,K] in dtype, w_frag (F16 and BF16): mtrt_hip_linear_prepack_fragments of w, K rounded up to 64
+ *   MTRT_LINEAR_DENSE_F8W (dtype F16 or BF16): MTRT_LINEAR_DENSE with w = dequantize(codes, w_scale), the weights' f8E4M3FN codes kept as such:
+ *                     w_frag: mtrt_hip_linear_prepack_fragments of the codes [N,K], w_scale: f32 [N], values of `dtype`; w: NULL, or
+ *                     mtrt_hip_linear_prepack_fragments of the dequantized [N,K], which calls of many rows then take
  * w may be NULL when w_frag is given and K is a multiple of 128 (int8) or 64 (16-bit), w_frag when the shape or type has none.
  * The results are those of the single calls (quantize, dequantize, the GEMM entry point, an addition in dtype).
  * `workspace`: mtrt_hip_linear_workspace(plan, M) bytes of device memory, 16-byte aligned, the call's own until its work
  * on `stream` is done; less is MTRT_INVALID_ARGUMENT. */
-enum mtrt_hip_linear_route { MTRT_LINEAR_W8A8 = 0, MTRT_LINEAR_W4A16 = 1, MTRT_LINEAR_DENSE = 2 };
+enum mtrt_hip_linear_route { MTRT_LINEAR_W8A8 = 0, MTRT_LINEAR_W4A16 = 1, MTRT_LINEAR_DENSE = 2, MTRT_LINEAR_DENSE_F8W = 3 };
 typedef struct mtrt_hip_linear_plan {
   int32_t route, dtype, q_dtype, reserved;
   int64_t K, N;
@@ -479,7 +482,7 @@ typedef struct mtrt_hip_linear_plan {
   const void *bias;
 } mtrt_hip_linear_plan;
 /* Bytes of the fragment order of [N,K] weights of int8 (MTRT_I8), f16 or bf16, K rounded up to whole 128-byte slices with
- * zeros; 0 for other types. */
+ * zeros, or of f8E4M3FN codes (those of 16-bit products: K rounded up to 64); 0 for other types. */
 MTRT_CAPI_EXPORTED int64_t mtrt_hip_linear_fragments_bytes(int32_t dtype, int64_t K, int64_t N);
 MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_prepack_fragments(mtrt_stream_t stream, const void *w_nk, int32_t dtype,
                                                              void *w_frag, int64_t K, int64_t N);

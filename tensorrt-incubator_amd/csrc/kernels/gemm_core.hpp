@@ -49,6 +49,7 @@ namespace gemm_core {
 using namespace mtrt_dev;
 
 typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v2i __attribute__((ext_vector_type(2)));
 typedef u32x4 u32x4_halves __attribute__((aligned(2)));
 typedef f32x4 f32x4_words __attribute__((aligned(4)));
 
@@ -671,6 +672,52 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 }
 }  // namespace edge
 
+// How the weights of fragment order lie, per lane and k-step: the matrix instruction's operand itself, ...
+struct Values {
+  using Raw = v4i;
+  struct Scale {};
+  static constexpr bool kCodes = false;
+  static constexpr int kStepBytes = 1024;              // a k-step of 32 columns
+  const int8_t* frag;
+  static __device__ __forceinline__ void dequantize(uint32_t, Scale, int, v4i&) {}
+};
+// ... or, for 16-bit products, eight float8 codes, dequantized in registers with the column's scale: f32(code) * scale rounded once to
+// X, the bits that a dequantize of the weights gives.  (code and scale have 4 and at most 11 bits, so that an f16 product rounds once too.)
+template <typename X> struct F8Codes;
+template <> struct F8Codes<BF16> {
+  using Raw = v2i;
+  using Scale = float;
+  static constexpr bool kCodes = true;
+  static constexpr int kStepBytes = 512;
+  const int8_t* frag;
+  const float* scale;
+  static __device__ __forceinline__ Scale scale_of(const float* scales, int64_t column, int64_t N) { return scales[column < N ? column : N - 1]; }
+  // codes 4 half .. 4 half + 3 of a lane's eight
+  static __device__ __forceinline__ void dequantize(uint32_t codes, Scale scale, int half, v4i& operand) {
+    const auto lo = __builtin_amdgcn_cvt_pk_f32_fp8(int(codes), false), hi = __builtin_amdgcn_cvt_pk_f32_fp8(int(codes), true);
+    operand[2 * half] = int(f32x2_to_bf16x2_bits(lo[0] * scale, lo[1] * scale));
+    operand[2 * half + 1] = int(f32x2_to_bf16x2_bits(hi[0] * scale, hi[1] * scale));
+  }
+};
+template <> struct F8Codes<F16> {
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  using Raw = v2i;
+  using Scale = h2;
+  static constexpr bool kCodes = true;
+  static constexpr int kStepBytes = 512;
+  const int8_t* frag;
+  const float* scale;
+  static __device__ __forceinline__ Scale scale_of(const float* scales, int64_t column, int64_t N) {
+    const _Float16 s = _Float16(scales[column < N ? column : N - 1]);
+    return Scale{s, s};
+  }
+  static __device__ __forceinline__ void dequantize(uint32_t codes, Scale scale, int half, v4i& operand) {
+    const h2 lo = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(codes), 1.0f, false), hi = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(int(codes), 1.0f, true);
+    operand[2 * half] = __builtin_bit_cast(int, lo * scale);
+    operand[2 * half + 1] = __builtin_bit_cast(int, hi * scale);
+  }
+};
+
 // ---- up to 32 rows against K-contiguous weights -----------------------------------------------------------
 // a [M <= 32 MT, row_bytes], w [N, row_bytes], both in whole 128-byte slices and 16-byte aligned.  With so few rows a
 // call is bound by reading the weights once, and a tile of the loops above would spend a whole K loop on padding.
@@ -693,6 +740,7 @@ constexpr int kPitch = 144, kStageBytes = 32 * kPitch;
 // MT: activation row tiles of 32 (1: M <= 32, 2: M <= 64, the weight fragments of a k-step serving both)
 template <int WAVES, int MT = 1, bool FRAG = false> constexpr int lds_bytes() { return WAVES * (MT + (FRAG ? 0 : 1)) * kStageBytes; }
 
+// CODES: the fragments hold float8 codes (F8Codes), dequantized on their way into the MFMA.
 // FRAG: `w` is not the [N,K] array but its fragment-order re-layout (per 32 rows and 128-byte slice four 1 KiB blocks,
 // lane l of block q holding the 16 bytes of k-step q of its row: exactly the second MFMA operand).  The weight
 // fragments then go from memory to registers and into the MFMA without passing LDS, 1 KiB contiguous per instruction.
@@ -727,9 +775,12 @@ __device__ __forceinline__ bool place(I item, I tiles_m, I tiles_n, int64_t& m, 
   return true;
 }
 
-template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool MANY = false, bool RAGGED = false, class Epilogue, typename Y>
+template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool MANY = false, bool RAGGED = false, class W = Values, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ w, int64_t row_bytes, Epilogue& epi,
-                                    Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds) {
+                                    Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds, const float* __restrict__ w_scale = nullptr) {
+  static_assert(!W::kCodes || FRAG, "codes in fragment order");
+  using WPiece = typename std::conditional<W::kCodes, u32x2, u32x4>::type;
+  using WAccess = typename std::conditional<RAGGED, u32x4_anywhere, WPiece>::type;
   static_assert(!MANY || MT == 1, "one row tile at a time");
   static_assert(!RAGGED || (MANY && !FRAG), "ragged rows: [N,K] weights");
   using Acc = typename Traits::Acc;
@@ -764,9 +815,9 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
     for (int i = 0; i < 4; ++i) {
       const int64_t n = tile * 32 + lrow + 8 * i;
       // fragment order: block i of a slice (the re-layout holds zeros for rows past N); else: row n of the array
-      wp[i] = FRAG ? w + tile * slices * 4096 + i * 1024 + lane * 16 : w + (n < N ? n : N - 1) * row_bytes + (RAGGED ? 0 : lchunk);
+      wp[i] = FRAG ? w + tile * slices * (4 * W::kStepBytes) + i * W::kStepBytes + lane * int(sizeof(WPiece)) : w + (n < N ? n : N - 1) * row_bytes + (RAGGED ? 0 : lchunk);
     }
-    constexpr int64_t kSliceBytes = FRAG ? 4096 : 128;   // from one slice of a lane's weight pieces to the next
+    constexpr int64_t kSliceBytes = FRAG ? 4 * W::kStepBytes : 128;   // from one slice of a lane's weight pieces to the next
     // bytes from a lane's pointers to its pieces of slice kb
     const auto piece = [&](int64_t kb) {
       const int64_t at = kb * 128 + lchunk;
@@ -775,7 +826,10 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
     Acc acc[MT];
 #pragma unroll
     for (int t = 0; t < MT; ++t) acc[t] = Traits::zero();
-    u32x4 ra[2][4 * MT], rw[2][4];
+    u32x4 ra[2][4 * MT];
+    WPiece rw[2][4];
+    typename W::Scale scale{};
+    if constexpr (W::kCodes) scale = W::scale_of(w_scale, tile * 32 + frow, N);
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
       // a slice past the wave's last one is the last one again (slice 0 for a wave without slices; slices >= 1)
@@ -784,7 +838,7 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 #pragma unroll
       for (int i = 0; i < 4 * MT; ++i) ra[p][i] = *reinterpret_cast<const Piece*>(ap[i] + (RAGGED ? piece(kb) : kb * 128));
 #pragma unroll
-      for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const Piece*>(wp[i] + (RAGGED ? piece(kb) : kb * kSliceBytes));
+      for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const WAccess*>(wp[i] + (RAGGED ? piece(kb) : kb * kSliceBytes));
     }
     for (int64_t kb = kb0; kb < kb1; kb += 2) {
 #pragma unroll
@@ -795,26 +849,29 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
               ra[p][i] = end_of_row(ra[p][i], left);
-              rw[p][i] = end_of_row(rw[p][i], left);
+              if constexpr (RAGGED) rw[p][i] = end_of_row(rw[p][i], left);
             }
           }
 #pragma unroll
           for (int i = 0; i < 4 * MT; ++i) *reinterpret_cast<u32x4*>(sa + (lrow + 8 * i) * kPitch + lchunk) = ra[p][i];
-          u32x4 held[4];                               // fragment order: this slice's fragments stay in registers
+          WPiece held[4];                              // fragment order: this slice's fragments stay in registers
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            if (FRAG) held[i] = rw[p][i];
+            if constexpr (FRAG) held[i] = rw[p][i];
             else *reinterpret_cast<u32x4*>(sw + (lrow + 8 * i) * kPitch + lchunk) = rw[p][i];
           }
           const int64_t next = kb + p + 2 < kb1 ? kb + p + 2 : kb1 - 1;   // always a load: the waits stay countable
 #pragma unroll
           for (int i = 0; i < 4 * MT; ++i) ra[p][i] = *reinterpret_cast<const Piece*>(ap[i] + (RAGGED ? piece(next) : next * 128));
 #pragma unroll
-          for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const Piece*>(wp[i] + (RAGGED ? piece(next) : next * kSliceBytes));
+          for (int i = 0; i < 4; ++i) rw[p][i] = *reinterpret_cast<const WAccess*>(wp[i] + (RAGGED ? piece(next) : next * kSliceBytes));
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             v4i fw;
-            if (FRAG) {
+            if constexpr (W::kCodes) {
+              W::dequantize(held[q][0], scale, 0, fw);
+              W::dequantize(held[q][1], scale, 1, fw);
+            } else if constexpr (FRAG) {
               fw = v4i{int(held[q][0]), int(held[q][1]), int(held[q][2]), int(held[q][3])};
             } else {
               fw = *reinterpret_cast<const v4i*>(sw + frow * kPitch + q * 32 + fhalf * 16);

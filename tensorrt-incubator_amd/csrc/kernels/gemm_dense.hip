@@ -487,52 +487,61 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_de
 // (256, 4096, 4096) 58 -> 16, (398, 11520, 1856) 165 -> 30, (1024, 2048, 2048) 32 -> 12.5, (200, 12288, 512) 164 -> 12.7.
 // mtrt_gemm_dense_frag_<type>_t<rows>x<columns> (x [M,K], w_frag, bias [N] or null, y [M,N], M, K, N, Split) ;
 // K % 64 == 0, x and w_frag 16-byte aligned, x below 4 GiB; the rest as mtrt_gemm_w8a8_frag_t<rows>x<columns>.
-#define MTRT_DENSE_FRAG_KERNEL(XN, XT, IT, JT, D, WG, TILE)                                                               \
+// mtrt_gemm_dense_frag_<type>_f8_...: float8 codes in their place (mtrt_wf8_prepack_frag), their scales w_scale (f32 [N]) the last argument.  Half the bytes on the way to a
+// unit (a slice of a 128 x 384 tile: 40 instead of 64 KiB) and from memory, for 16 (bf16) or 8 (f16) vector instructions to a fragment of eight
+// weights, which a wave issues beside the IT MFMAs that use it: what bounds it is the weights' way, in tiles of few rows those instructions.  us, values
+// and codes, bf16, weights from memory: (24, 4096, 11008) 0.76 of the time, (128, ..) 0.81, (512, ..) 0.87, (1024, ..) 0.96, (2048, ..) 1.04;
+// f16 0.74, 0.75, 0.81, 0.94, 1.01; from the Infinity Cache (K, N) = (4096, 4096) bf16 1.05, 1.21, 1.31, 1.14, 1.12, and f16 0.95, 1.05, 1.04, 1.04,
+// 1.03.  (By sets of four waves that share K, as W4A16's 32- and 64-row tiles are: no faster, the wave's own instructions are the limit.)
+#define MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, IT, JT, D, WG, TILE)                                            \
   extern "C" __global__ void __launch_bounds__(256, WG) mtrt_gemm_dense_frag_##XN##_##TILE(                               \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, gemm_frag::Split sp) {    \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N, gemm_frag::Split sp MTRT_UNWRAP WPARAM) {    \
     __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<IT, D>(128 * JT)];                            \
     gemm_frag::Part part;                                                                                                 \
     if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / 64, sp, part)) return; \
     dense_cluster::BiasEpilogue<XT, 128 * JT> epi{bias, nullptr, {}};                                                     \
-    gemm_frag::run<dense_cluster::HalfTraits<XT>, IT, JT, D>(x, 2 * K, w_frag, epi, y, M, N, part, lds);                  \
+    gemm_frag::run<dense_cluster::HalfTraits<XT>, IT, JT, D>(x, 2 * K, WT{MTRT_UNWRAP WARGS}, epi, y, M, N, part, lds);               \
   }
 // ... 256 x 384 tiles: (x, w_frag, bias, y, M, K, N) ; grid = 8 * ceil(ceil(M/256) * ceil(N/384) / 8), block = 256.
 // ... up to 32 and 64 rows, a wave for itself (gemm_core::rows32): the same arguments; grid: any, block = 512.
-#define MTRT_DENSE_FRAG_KERNELS(XN, XT)                                                                                   \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 1, 1, 4, 2, t32x128)                                                                     \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 2, 1, 4, 2, t64x128)                                                                     \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 1, 2, 2, t128x128)                                                                    \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 2, 2, 2, t128x256)                                                                    \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 4, 3, 2, 1, t128x384)                                                                    \
-  MTRT_DENSE_FRAG_KERNEL(XN, XT, 8, 2, 2, 1, t256x256)                                                                    \
+#define MTRT_DENSE_FRAG_KERNELS(XN, XT, WT, WPARAM, WARGS, WSCALE)                                                       \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, 1, 1, 4, 2, t32x128)                         \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, 2, 1, 4, 2, t64x128)                         \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, 4, 1, 2, 2, t128x128)                        \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, 4, 2, 2, 2, t128x256)                        \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, 4, 3, 2, 1, t128x384)                        \
+  MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, 8, 2, 2, 1, t256x256)                        \
   extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_dense_frag_##XN##_t256x384(                              \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                        \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N MTRT_UNWRAP WPARAM) {                                     \
     __shared__ __attribute__((aligned(16))) int8_t lds[gemm_frag::lds_bytes<8, 2>(gemm_frag::kWideBN)];                   \
     const int64_t tiles_m = (M + 255) / 256, panels = (N + gemm_frag::kWideBN - 1) / gemm_frag::kWideBN;                  \
     int64_t tile_m, panel;                                                                                                \
     if (!gemm_core::tile_of_even(blockIdx.x, gridDim.x, tiles_m, panels, tiles_m, tile_m, panel)) return;                 \
     dense_cluster::BiasEpilogue<XT, gemm_frag::kWideBN> epi{bias, nullptr, {}};                                           \
-    gemm_frag::run_wide<dense_cluster::HalfTraits<XT>>(x, 2 * K, w_frag, (N + 31) / 32, epi, y, M, N, K / 64, tile_m * 256, \
+    gemm_frag::run_wide<dense_cluster::HalfTraits<XT>>(x, 2 * K, WT{MTRT_UNWRAP WARGS}, (N + 31) / 32, epi, y, M, N, K / 64, tile_m * 256, \
                                                        panel * gemm_frag::kWideBN, lds);                                  \
   }                                                                                                                       \
   extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##XN##_rows32(                                   \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                        \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N MTRT_UNWRAP WPARAM) {                                     \
     __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8, 1, true>()];                       \
     dense_cluster::RowsBiasEpilogue<XT> epi{bias};                                                                        \
-    gemm_core::rows32::run<dense_cluster::HalfTraits<XT>, 8, 1, true>(x, w_frag, 2 * K, epi, y, M, N, lds);               \
+    gemm_core::rows32::run<dense_cluster::HalfTraits<XT>, 8, 1, true, false, false, WT>(x, w_frag, 2 * K, epi, y, M, N, lds, WSCALE); \
   }                                                                                                                       \
   extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##XN##_rows64(                                   \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \
-      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N) {                                                        \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t N MTRT_UNWRAP WPARAM) {                                     \
     __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8, 2, true>()];                       \
     dense_cluster::RowsBiasEpilogue<XT> epi{bias};                                                                        \
-    gemm_core::rows32::run<dense_cluster::HalfTraits<XT>, 8, 2, true>(x, w_frag, 2 * K, epi, y, M, N, lds);               \
+    gemm_core::rows32::run<dense_cluster::HalfTraits<XT>, 8, 2, true, false, false, WT>(x, w_frag, 2 * K, epi, y, M, N, lds, WSCALE); \
   }
-MTRT_DENSE_FRAG_KERNELS(f16, F16)
-MTRT_DENSE_FRAG_KERNELS(bf16, BF16)
+#define MTRT_UNWRAP(...) __VA_ARGS__
+MTRT_DENSE_FRAG_KERNELS(f16, F16, gemm_core::Values, (), (w_frag), nullptr)
+MTRT_DENSE_FRAG_KERNELS(bf16, BF16, gemm_core::Values, (), (w_frag), nullptr)
+MTRT_DENSE_FRAG_KERNELS(f16_f8, F16, gemm_core::F8Codes<F16>, (, const float* __restrict__ w_scale), (w_frag, w_scale), w_scale)
+MTRT_DENSE_FRAG_KERNELS(bf16_f8, BF16, gemm_core::F8Codes<BF16>, (, const float* __restrict__ w_scale), (w_frag, w_scale), w_scale)
 
 // ---- up to 16 rows on fragment-order weights in ONE launch -----------------------------------------------
 // x goes into LDS whole, quantized and dequantized on its way where the module quantizes its input (the arithmetic of mtrt_act_fake_*,
@@ -547,7 +556,7 @@ MTRT_DENSE_FRAG_KERNELS(bf16, BF16)
 namespace dense_cluster {
 namespace rows16 {
 typedef float v4f __attribute__((ext_vector_type(4)));
-constexpr int kWaves = 8, kMaxRows = 16, kAhead = 4;
+constexpr int kWaves = 8, kMaxRows = 16;
 constexpr int kRowPad = 16;                                        // LDS bytes between the rows: their banks differ
 
 template <typename X> __device__ __forceinline__ v4f mfma(v4i a, v4i b, v4f c);
@@ -564,13 +573,15 @@ template <> __device__ __forceinline__ v4f mfma<BF16>(v4i a, v4i b, v4f c) {
 
 struct Plain {};
 
-template <typename X, typename Q, int kXGroups, bool PAST>
-__device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag,
+template <typename X, typename Q, class W, int kXGroups, bool PAST>
+__device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const W& weights,
                                     const RowsBiasEpilogue<X>& epi, uint16_t* __restrict__ y, int M, int K, int Kp, int64_t N, int8_t* rows,
                                     float (*partial)[64][4]) {
   using qdq_cluster::ExactDivisor;
   using qdq_cluster::FloatGroup;
+  using Raw = typename W::Raw;
   constexpr bool kQuantized = !std::is_same<Q, Plain>::value;
+  constexpr int kAhead = W::kCodes ? 8 : 4;                        // slices: the same bytes on their way
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int col = lane & 15, kgroup = lane >> 4;
   const int slices = Kp / 64, kb0 = slices * wave / kWaves, kb1 = slices * (wave + 1) / kWaves;
@@ -587,14 +598,19 @@ __device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float*
   }
   const float scale = kQuantized ? x_scale[0] : 1.0f;
 
-  // lane (col, kgroup) of k-step pair p: bytes 64 p + 16 kgroup ... + 15 of its column's slice
-  const int8_t* wp = w_frag + (n0 / 32) * slices * 4096 + (kgroup >> 1) * 1024 + ((kgroup & 1) * 32 + int(n0 & 16) + col) * 16;
+  // lane (col, kgroup) of k-step pair p: bytes 64 p + 16 kgroup ... + 15 of its column's slice (codes: half as many)
+  const int8_t* wp = weights.frag + (n0 / 32) * slices * (4 * W::kStepBytes) + (kgroup >> 1) * W::kStepBytes + ((kgroup & 1) * 32 + int(n0 & 16) + col) * int(sizeof(Raw));
+  typename W::Scale w_scale{};
+  if constexpr (W::kCodes) w_scale = W::scale_of(weights.scale, n0 + col, N);
   const int last = kb1 > kb0 ? kb1 - 1 : 0;                        // a slice past the wave's last one is that one again
-  v4i w[kAhead][2];
-  const auto fetch = [&](int kb, v4i (&into)[2]) {
-    const int8_t* from = wp + int64_t(kb < kb1 ? kb : last) * 4096;
+  Raw w[kAhead][2];
+  const auto fetch = [&](int kb, Raw (&into)[2]) {
+    const int8_t* from = wp + int64_t(kb < kb1 ? kb : last) * (4 * W::kStepBytes);
 #pragma unroll
-    for (int p = 0; p < 2; ++p) into[p] = PAST ? __builtin_nontemporal_load(reinterpret_cast<const v4i*>(from + p * 2048)) : *reinterpret_cast<const v4i*>(from + p * 2048);
+    for (int p = 0; p < 2; ++p) {
+      const Raw* at = reinterpret_cast<const Raw*>(from + p * (2 * W::kStepBytes));
+      into[p] = PAST ? __builtin_nontemporal_load(at) : *at;
+    }
   };
 #pragma unroll
   for (int s = 0; s < kAhead; ++s) fetch(kb0 + s, w[s]);
@@ -633,7 +649,16 @@ __device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float*
   for (int kb = kb0; kb < kb1; kb += kAhead) {
 #pragma unroll
     for (int s = 0; s < kAhead; ++s) {
-      v4i held[2] = {w[s][0], w[s][1]};
+      v4i held[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        if constexpr (W::kCodes) {
+          W::dequantize(uint32_t(w[s][p][0]), w_scale, 0, held[p]);
+          W::dequantize(uint32_t(w[s][p][1]), w_scale, 1, held[p]);
+        } else {
+          held[p] = w[s][p];
+        }
+      }
       if (kb + kAhead < kb1) fetch(kb + kAhead + s, w[s]);
       if (kb + s < kb1) {
 #pragma unroll
@@ -659,14 +684,14 @@ __device__ __forceinline__ void run(const uint16_t* __restrict__ x, const float*
   }
 }
 
-template <typename X, typename Q, int kXGroups>
-__device__ __forceinline__ void run_any(const uint16_t* x, const float* x_scale, const int8_t* w_frag, const uint16_t* bias, uint16_t* y, int64_t M, int64_t K,
+template <typename X, typename Q, int kXGroups, class W>
+__device__ __forceinline__ void run_any(const uint16_t* x, const float* x_scale, const W& weights, const uint16_t* bias, uint16_t* y, int64_t M, int64_t K,
                                         int64_t Kp, int64_t N, bool past, int8_t* rows, float (*partial)[64][4]) {
   const RowsBiasEpilogue<X> epi{bias};
   if (past)
-    run<X, Q, kXGroups, true>(x, x_scale, w_frag, epi, y, int(M), int(K), int(Kp), N, rows, partial);
+    run<X, Q, W, kXGroups, true>(x, x_scale, weights, epi, y, int(M), int(K), int(Kp), N, rows, partial);
   else
-    run<X, Q, kXGroups, false>(x, x_scale, w_frag, epi, y, int(M), int(K), int(Kp), N, rows, partial);
+    run<X, Q, W, kXGroups, false>(x, x_scale, weights, epi, y, int(M), int(K), int(Kp), N, rows, partial);
 }
 }  // namespace rows16
 }  // namespace dense_cluster
@@ -674,26 +699,58 @@ __device__ __forceinline__ void run_any(const uint16_t* x, const float* x_scale,
 // (x [M,K], x_scale: one f32 (null without codes), w_frag (K padded to Kp), bias [N] or null, y [M,N], M <= 16, K, Kp, N, past) ; Kp = K rounded
 // up to 64, M * Kp <= 16384 (32768 for _long: twice the registers and LDS for x, one workgroup to a compute unit), w_frag 16-byte
 // aligned, x aligned to its elements; past: weights read past the caches; grid = ceil(N / 16), block = 512.
+// Of x that is not quantized or goes through float8 codes (a module of float8 weights), one more argument: w_scale, f32 [N] where w_frag holds float8
+// codes, else null.  Half the bytes: bf16, us, values and codes, (1, 4096, 4096) 7.2, 5.9; (1, 4096, 11008) 16.4, 11.0; (8, 2048, 16384) in f16 17.5, 13.4.
+#define MTRT_DENSE_ROWS16_BODY(GROUPS)                                                                                    \
+  using namespace dense_cluster::rows16;                                                                                  \
+  __shared__ __attribute__((aligned(16))) int8_t rows[GROUPS * 64 * kWaves * 16 + kMaxRows * kRowPad];                    \
+  __shared__ __attribute__((aligned(16))) float partial[kWaves][64][4];
 #define MTRT_DENSE_ROWS16_KERNEL(NAME, XT, QT, GROUPS)                                                                    \
   extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##NAME(                                          \
       const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag, const uint16_t* __restrict__ bias, \
       uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t Kp, int64_t N, int32_t past) {                              \
-    using namespace dense_cluster::rows16;                                                                                \
-    __shared__ __attribute__((aligned(16))) int8_t rows[GROUPS * 64 * kWaves * 16 + kMaxRows * kRowPad];                  \
-    __shared__ __attribute__((aligned(16))) float partial[kWaves][64][4];                                                 \
-    run_any<XT, QT, GROUPS>(x, x_scale, w_frag, bias, y, M, K, Kp, N, past, rows, partial);                               \
+    MTRT_DENSE_ROWS16_BODY(GROUPS)                                                                                        \
+    run_any<XT, QT, GROUPS>(x, x_scale, gemm_core::Values{w_frag}, bias, y, M, K, Kp, N, past, rows, partial);            \
+  }
+#define MTRT_DENSE_ROWS16_CODES_KERNEL(NAME, XT, QT, GROUPS)                                                              \
+  extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_frag_##NAME(                                          \
+      const uint16_t* __restrict__ x, const float* __restrict__ x_scale, const int8_t* __restrict__ w_frag, const uint16_t* __restrict__ bias, \
+      uint16_t* __restrict__ y, int64_t M, int64_t K, int64_t Kp, int64_t N, int32_t past, const float* __restrict__ w_scale) { \
+    MTRT_DENSE_ROWS16_BODY(GROUPS)                                                                                        \
+    if (w_scale)                                                                                                          \
+      run_any<XT, QT, GROUPS>(x, x_scale, gemm_core::F8Codes<XT>{w_frag, w_scale}, bias, y, M, K, Kp, N, past, rows, partial); \
+    else                                                                                                                  \
+      run_any<XT, QT, GROUPS>(x, x_scale, gemm_core::Values{w_frag}, bias, y, M, K, Kp, N, past, rows, partial);          \
   }
 #define MTRT_DENSE_ROWS16_KERNELS(XN, XT)                               \
-  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16, XT, Plain, 4)                   \
+  MTRT_DENSE_ROWS16_CODES_KERNEL(XN##_rows16, XT, Plain, 4)             \
   MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_i8, XT, I8, 4)                   \
-  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_f8, XT, F8, 4)                   \
+  MTRT_DENSE_ROWS16_CODES_KERNEL(XN##_rows16_f8, XT, F8, 4)             \
   MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_i4, XT, I4, 4)                   \
-  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long, XT, Plain, 8)              \
+  MTRT_DENSE_ROWS16_CODES_KERNEL(XN##_rows16_long, XT, Plain, 8)        \
   MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long_i8, XT, I8, 8)              \
-  MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long_f8, XT, F8, 8)              \
+  MTRT_DENSE_ROWS16_CODES_KERNEL(XN##_rows16_long_f8, XT, F8, 8)        \
   MTRT_DENSE_ROWS16_KERNEL(XN##_rows16_long_i4, XT, I4, 8)
 MTRT_DENSE_ROWS16_KERNELS(f16, F16)
 MTRT_DENSE_ROWS16_KERNELS(bf16, BF16)
+
+// Re-layout of float8 codes [N,K] into the fragment order of 16-bit products, the eight codes of a lane and k-step per thread: (w, w_frag,
+// K, N) ; w_frag holds 32 * ceil(N/32) * 64 * ceil(K/64) bytes, zeros where w has no element.
+extern "C" __global__ void __launch_bounds__(256) mtrt_wf8_prepack_frag(const uint8_t* __restrict__ w, u32x2* __restrict__ w_frag,
+                                                                      int64_t K, int64_t N) {
+  const int64_t slices = (K + 63) / 64, ntiles = (N + 31) / 32;
+  const int64_t total = ntiles * slices * 256;
+  for (int64_t id = int64_t(blockIdx.x) * block_threads() + threadIdx.x; id < total; id += int64_t(gridDim.x) * block_threads()) {
+    const int lane = int(id & 63), p = int((id >> 6) & 3);
+    const int64_t slice = (id >> 8) % slices, tile = (id >> 8) / slices;
+    const int64_t n = tile * 32 + (lane & 31), k0 = slice * 64 + 16 * p + 8 * (lane >> 5);
+    u32x2 v = {0u, 0u};
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      if (n < N && k0 + e < K) v[e >> 2] |= uint32_t(w[n * K + k0 + e]) << (8 * (e & 3));
+    w_frag[id] = v;
+  }
+}
 
 // Re-layout of 16-bit weights [N,K] into fragment order, one 16-byte chunk per thread: (w, w_frag, K, N) ; w_frag holds
 // 32 * ceil(N/32) * 128 * ceil(K/64) bytes, zeros where w has no element.

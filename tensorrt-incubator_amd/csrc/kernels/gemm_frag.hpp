@@ -5,7 +5,8 @@
 // Fragment order (mtrt_w8_prepack_frag, mtrt_w16_prepack_frag): for each tile of 32 columns and each slice of 128 bytes
 // of K four 1 KiB blocks, one per k-step p; in a block lane l = 32 h + (n % 32) owns the 16 bytes 128 slice + 32 p + 16 h
 // .. + 15 of column n: the B operand of the 32 x 32 matrix instruction of that k-step, whatever the type (16 int8 or
-// 8 sixteen-bit values), and every load of a wave reads 1 KiB of contiguous memory.
+// 8 sixteen-bit values), and every load of a wave reads 1 KiB of contiguous memory.  Float8 codes of 16-bit products (mtrt_wf8_prepack_frag,
+// gemm_core::F8Codes) lie the same way in half the bytes, eight codes to a lane and k-step.
 //
 // Why one loop for many tiles.  A 256-row tile gives the fewest bytes per MFMA, but a launch lasts one tile's whole K
 // loop: with M in the hundreds, or a short N, such tiles occupied 10 to 60 of the 256 compute units (M = 398, K = 11520,
@@ -39,14 +40,19 @@ __device__ __forceinline__ void static_for(F&& f) {
   }
 }
 
-// 16 bytes per lane of k-step T of a weight slice: scalar base, 32-bit lane offset, the k-step as the instruction's offset
+// 16 bytes (of codes: 8) per lane of k-step T of a weight slice: scalar base, 32-bit lane offset, the k-step as the instruction's offset
+template <int T>
+__device__ __forceinline__ void load_w(v2i& dst, uint32_t lane_off, const int8_t* base) {
+  __asm__ volatile("global_load_dwordx2 %0, %1, %2 offset:%3" : "=v"(dst) : "v"(lane_off), "s"(base), "n"(T * 512) : "memory");
+}
 template <int T>
 __device__ __forceinline__ void load_w(v4i& dst, uint32_t lane_off, const int8_t* base) {
   __asm__ volatile("global_load_dwordx4 %0, %1, %2 offset:%3" : "=v"(dst) : "v"(lane_off), "s"(base), "n"(T * 1024) : "memory");
 }
 
 // The memory instructions of a wave, in issue order: per k-step first its direct-to-LDS loads, then JT weight loads.
-// In k-step T of slice s: the activations of slice s + D, the weights of the k-step 4 D - 1 further on.
+// In k-step T of slice s: the activations of slice s + D, the weights of the k-step 4 D - 1 further on.  Codes are dequantized during the k-step
+// before the one that uses them, so their registers are free, and wanted again, a k-step earlier: 4 D further on, and the counts are the same.
 template <int IT, int JT, int D>
 struct Order {
   static constexpr int kLoads = IT;                    // direct-to-LDS loads per wave and slice (32 IT rows, 4 waves, 8 rows each)
@@ -70,6 +76,12 @@ struct Order {
   // (no weights go with the first loads of all: a slice whose only load comes in k-step 0 has JT fewer behind it)
   static constexpr int activations_in_flight_at_start() {
     return (last_step() == 0 ? 0 : JT) + (3 - last_step()) * JT + (D - 1) * (kLoads + 4 * JT);
+  }
+  // codes: those of the first k-step, issued with the first loads of all, at the end of the prologue
+  static constexpr int first_codes_in_flight() {
+    int n = 0;
+    for (int i = 1; i < 4 * D; ++i) n += JT + dma(i % 4);
+    return n;
   }
 };
 
@@ -178,16 +190,19 @@ __device__ __forceinline__ bool meet(Acc (&acc)[IT][JT], const Part& part, int8_
   return true;
 }
 
-// Traits: Acc (sixteen accumulators), zero(), mfma(weight fragment, activation fragment, acc).
-template <class Traits, int IT, int JT, int D, class Epilogue, typename Y>
-__device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_bytes, const int8_t* __restrict__ wfrag, Epilogue& epi,
+// Traits: Acc (sixteen accumulators), zero(), mfma(weight fragment, activation fragment, acc).  W: gemm_core::Values, or codes, whose fragments are
+// dequantized a k-step ahead, spread over the MFMAs of the k-step before.
+template <class Traits, int IT, int JT, int D, class W, class Epilogue, typename Y>
+__device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_bytes, const W& weights, Epilogue& epi,
                                     Y* __restrict__ y, int64_t M, int64_t N, const Part& part, int8_t* lds) {
   using Acc = typename Traits::Acc;
   using O = Order<IT, JT, D>;
   constexpr int R = O::kRing, NS = stages<IT, D>(), AN = 4, kStageBytes = IT * 32 * 128;
   constexpr int TB = (4 * IT - AN) / IT;               // the first k-step that reads a fragment of the next slice
   static_assert(D % 2 == 0 && O::weights_in_flight(3) < 64 && O::activations_in_flight(TB) < 64 && O::activations_in_flight_at_start() < 64, "wait counter range");
-  const int lane = threadIdx.x & 63;
+  int thread = threadIdx.x;
+  if constexpr (W::kCodes) __asm__ volatile("" : "+v"(thread));   // (the lane is not held through the loop for the epilogue: 256 x 256 tiles have no register left)
+  const int lane = thread & 63;
   const int slot = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int frow = lane & 31, fhalf = lane >> 5;
   const int64_t total_slices = row_bytes / 128, ntiles = (N + 31) / 32;
@@ -198,14 +213,18 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
   DmaLoaderT<IT> al;
   al.init(a + uint64_t(slice0) * 128, M, row_bytes, part.m0);
   v4i fa[2][AN];
-  v4i wr[R][JT];
+  typename W::Raw wr[R][JT];
+  v4i fb[2][JT];                                       // codes: the fragments of this k-step and the next
+  typename W::Scale ws[JT];
   const int8_t* wsrc[JT];                              // the first slice of each column tile (uniform)
-  const uint32_t wlane = uint32_t(lane) * 16;
+  const uint32_t wlane = uint32_t(lane) * uint32_t(sizeof(typename W::Raw));
+  constexpr int kSliceBytes = 4 * W::kStepBytes;
 #pragma unroll
   for (int j = 0; j < JT; ++j) {
     int64_t tile = int64_t(__builtin_amdgcn_readfirstlane(uint32_t(part.n0 / 32))) + slot * JT + j;
     tile = tile < ntiles ? tile : ntiles - 1;          // tiles past N: some valid data, never stored
-    wsrc[j] = wfrag + (tile * total_slices + slice0) * 4096;
+    wsrc[j] = weights.frag + (tile * total_slices + slice0) * kSliceBytes;
+    if constexpr (W::kCodes) ws[j] = W::scale_of(weights.scale, part.n0 + (slot * JT + j) * 32 + frow, N);
   }
   // all ones for a slice of this part, zero past its end: such a load reads one fixed line of the first slice
   auto keep = [&](uint32_t slice) { return uint32_t(int32_t(slice - nslices) >> 31); };
@@ -238,13 +257,16 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
   // (slot of the register ring, k-step inside its slice, slice): column tile j
   auto issue_w = [&](auto slot_c, auto step, uint32_t slice, int j) {
     const uint32_t k = keep(slice);
-    load_w<decltype(step)::value>(wr[decltype(slot_c)::value][j], wlane & k, wsrc[j] + uint64_t(__builtin_amdgcn_readfirstlane(slice & k)) * 4096);
+    load_w<decltype(step)::value>(wr[decltype(slot_c)::value][j], wlane & k, wsrc[j] + uint64_t(__builtin_amdgcn_readfirstlane(slice & k)) * kSliceBytes);
   };
 
   static_for<0, 4 * D>([&](auto v) {                   // the D slices in front of the first, as the loop would have issued them
     constexpr int V = decltype(v)::value, SD = V / 4, T = V % 4;
     issue_dma(IntC<T>{}, SD);
-    if constexpr (V > 0) {
+    if constexpr (W::kCodes) {
+#pragma unroll
+      for (int j = 0; j < JT; ++j) issue_w(IntC<V>{}, IntC<T>{}, SD, j);
+    } else if constexpr (V > 0) {
 #pragma unroll
       for (int j = 0; j < JT; ++j) issue_w(IntC<(V - 1) % R>{}, IntC<(V - 1) % 4>{}, (V - 1) / 4, j);
     }
@@ -267,30 +289,52 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
     constexpr int X = decltype(n)::value;
     read_a(fa[0][X], a_lane[X / IT] + stage_off(0), IntC<X % IT>{});
   });
+  auto dequantize = [&](auto slot_c, int j, int half, v4i& fragment) { W::dequantize(uint32_t(wr[decltype(slot_c)::value][j][half]), ws[j], half, fragment); };
+  if constexpr (W::kCodes) {
+#pragma unroll
+    for (int j = 0; j < JT; ++j) {
+      __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(wr[0][j]) : "n"(O::first_codes_in_flight()) : "memory");
+      dequantize(IntC<0>{}, j, 0, fb[0][j]);
+      dequantize(IntC<0>{}, j, 1, fb[0][j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // k-step T of the slice at position U of the unrolled loop (slice s)
   auto kstep = [&](auto pos, auto step, uint32_t s) {
     constexpr int U = decltype(pos)::value, T = decltype(step)::value, Q = U * 4 + T, SLOT = Q % R;
+    constexpr int WANTED = W::kCodes ? (Q + 1) % R : SLOT;   // codes: the next k-step's, dequantized under this one's MFMAs
     if constexpr (T == TB) {
       // the activations of slice s + 1 have landed for every wave; the stage filled next is not one that is being read
       __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(O::activations_in_flight(TB)) : "memory");
       __asm__ volatile("s_barrier" ::: "memory");
     }
 #pragma unroll
-    for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(wr[SLOT][j]) : "n"(O::weights_in_flight(T)) : "memory");
+    for (int j = 0; j < JT; ++j) __asm__ volatile("s_waitcnt vmcnt(%1)" : "+v"(wr[WANTED][j]) : "n"(O::weights_in_flight(T)) : "memory");
     const uint32_t here = stage_off(s), next = stage_off(s + 1);
     static_for<0, IT>([&](auto cc) {
       constexpr int c = decltype(cc)::value, X = Q * IT + c, SET = (X / AN) % 2, AI = X % AN;
       constexpr int X2 = T * IT + c + AN, T2 = X2 / IT;  // the fragment read now, AN further on in the stream
       __asm__ volatile("s_waitcnt lgkmcnt(%1)" : "+v"(fa[SET][AI]) : "n"(AN - 1) : "memory");
 #pragma unroll
-      for (int j = 0; j < JT; ++j) acc[c][j] = Traits::mfma(wr[SLOT][j], fa[SET][AI], acc[c][j]);
+      for (int j = 0; j < JT; ++j) {
+        if constexpr (W::kCodes) acc[c][j] = Traits::mfma(fb[Q % 2][j], fa[SET][AI], acc[c][j]);
+        else acc[c][j] = Traits::mfma(wr[SLOT][j], fa[SET][AI], acc[c][j]);
+      }
       read_a(fa[1 - SET][AI], a_lane[T2 % 4] + (T2 >= 4 ? next : here), IntC<X2 % IT>{});
       if constexpr (c == 0) issue_dma(step, s + D);
-      // the registers of the k-step before this one, for their next use
+      // the registers of the k-step before this one (codes: of this one), for their next use
 #pragma unroll
       for (int j = 0; j < JT; ++j)
-        if ((1 + j < IT ? 1 + j : IT - 1) == c) issue_w(IntC<(Q + R - 1) % R>{}, IntC<(T + 3) % 4>{}, T == 0 ? s + D - 1 : s + D, j);
+        if ((1 + j < IT ? 1 + j : IT - 1) == c) {
+          if constexpr (W::kCodes) issue_w(IntC<SLOT>{}, step, s + D, j);
+          else issue_w(IntC<(Q + R - 1) % R>{}, IntC<(T + 3) % 4>{}, T == 0 ? s + D - 1 : s + D, j);
+        }
+      if constexpr (W::kCodes) {
+#pragma unroll
+        for (int u = 0; u < 2 * JT; ++u)
+          if ((u * IT) / (2 * JT) == c) dequantize(IntC<WANTED>{}, u >> 1, u & 1, fb[1 - Q % 2][u >> 1]);
+      }
       __builtin_amdgcn_sched_barrier(0);
     });
   };
@@ -335,8 +379,8 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, int64_t row_by
 // int8 at M = 2048, K = 4096, N = 11008 (232 tiles, one round) 77.5 us; 128 x 384 tiles there take 80.5, 256 x 256 ones 89.6.
 constexpr int kWideBN = 384, kStageBytes = 256 * 128;  // columns; one slice of the activation panel
 
-template <class Traits, class Epilogue>
-__device__ __forceinline__ void run_wide(const int8_t* __restrict__ a, int64_t a_row_bytes, const int8_t* __restrict__ wfrag,
+template <class Traits, class W, class Epilogue>
+__device__ __forceinline__ void run_wide(const int8_t* __restrict__ a, int64_t a_row_bytes, const W& weights,
                                          int64_t ntiles, Epilogue& epi, uint16_t* __restrict__ y, int64_t M, int64_t N,
                                          int64_t slices, int64_t m0, int64_t n0, int8_t* lds) {
   constexpr int IT = 8, JT = 3, AN = 4, kG = 8;
@@ -351,17 +395,20 @@ __device__ __forceinline__ void run_wide(const int8_t* __restrict__ a, int64_t a
   DmaLoaderT<kG> al;
   al.init(a, M, a_row_bytes, m0);
   v4i fa[2][AN];
-  v4i wr[4][JT];
+  typename W::Raw wr[4][JT];
+  v4i fb[2][JT];                                       // codes: the fragments of this k-step and the next
+  typename W::Scale ws[JT];
   const int8_t* wsrc[JT];                              // slice 0 of each column tile (uniform)
-  uint32_t wlane = uint32_t(lane) * 16;
+  uint32_t wlane = uint32_t(lane) * uint32_t(sizeof(typename W::Raw));
 #pragma unroll
   for (int j = 0; j < JT; ++j) {
     int64_t tile = n0 / 32 + slot * JT + j;
     tile = tile < ntiles ? tile : ntiles - 1;          // tiles past N: some valid data, never stored
-    wsrc[j] = wfrag + tile * slices * 4096;
+    wsrc[j] = weights.frag + tile * slices * (4 * W::kStepBytes);
+    if constexpr (W::kCodes) ws[j] = W::scale_of(weights.scale, n0 + (slot * JT + j) * 32 + frow, N);
   }
-  auto fetch_w = [&](auto tt, v4i& dst, int j, uint32_t slice) {
-    load_w<decltype(tt)::value>(dst, wlane, wsrc[j] + uint64_t(slice) * 4096);
+  auto fetch_w = [&](auto tt, typename W::Raw& dst, int j, uint32_t slice) {
+    load_w<decltype(tt)::value>(dst, wlane, wsrc[j] + uint64_t(slice) * (4 * W::kStepBytes));
   };
   const uint32_t lds_base = uint32_t(uintptr_t((lds_void_t*)lds));
   uint32_t a_lane[4];
@@ -377,11 +424,11 @@ __device__ __forceinline__ void run_wide(const int8_t* __restrict__ a, int64_t a
   auto stage = [&](uint32_t slice) { return lds + stage_off(slice); };
   auto at_most_last = [&](uint32_t slice) { return slice - ((uint32_t(last - slice) >> 31) * (slice - last)); };  // scalar min
 
-  // slice 0 and its weights for k-steps 0..2 (k-step 3's are asked for in k-step 0, like every slice's), then slice 1
+  // slice 0 and its weights for k-steps 0..2 (k-step 3's are asked for in k-step 0, like every slice's; codes: all four), then slice 1
   const uint32_t one = at_most_last(1);
 #pragma unroll
   for (int g = 0; g < kG; ++g) al.dma_at(al.slice_base(0), stage(0), g);
-  static_for<0, 3>([&](auto t) {
+  static_for<0, W::kCodes ? 4 : 3>([&](auto t) {
     constexpr int T = decltype(t)::value;
 #pragma unroll
     for (int j = 0; j < JT; ++j) fetch_w(t, wr[T][j], j, 0);
@@ -402,33 +449,45 @@ __device__ __forceinline__ void run_wide(const int8_t* __restrict__ a, int64_t a
     __builtin_amdgcn_sched_barrier(0);
   }
 #pragma unroll
-  for (int t = 0; t < 3; ++t) __asm__ volatile("s_waitcnt vmcnt(0)" : "+v"(wr[t][0]), "+v"(wr[t][1]), "+v"(wr[t][2])::"memory");
+  for (int t = 0; t < (W::kCodes ? 4 : 3); ++t) __asm__ volatile("s_waitcnt vmcnt(0)" : "+v"(wr[t][0]), "+v"(wr[t][1]), "+v"(wr[t][2])::"memory");
   drain_and_barrier();
   static_for<0, AN>([&](auto i) { read_a(fa[0][decltype(i)::value], a_lane[0] + stage_off(0), i); });
+  auto dequantize = [&](int t, int j, int half) { W::dequantize(uint32_t(wr[t][j][half]), ws[j], half, fb[t & 1][j]); };
+  if constexpr (W::kCodes) {
+#pragma unroll
+    for (int u = 0; u < 2 * JT; ++u) dequantize(0, u >> 1, u & 1);
+    __builtin_amdgcn_sched_barrier(0);
+  }
 
   // k-step T of slice s0 (the next slice: s1): eight fenced chunks; chunk c multiplies row tile c by the three weight
   // fragments of the k-step.  ca: LDS offset of the stage this k-step reads, ra: of the stage the next k-step reads.
   auto kstep = [&](auto step, uint32_t ca, uint32_t ra, uint32_t s0, uint32_t s1, const int8_t* src, int8_t* nd) {
     constexpr int T = decltype(step)::value;
     const uint32_t raddr = a_lane[(T + 1) & 3] + ra, caddr = a_lane[T] + ca;
-    __asm__ volatile("s_waitcnt vmcnt(%3)" : "+v"(wr[T][0]), "+v"(wr[T][1]), "+v"(wr[T][2]) : "n"(kFly) : "memory");
+    constexpr int WANTED = W::kCodes ? (T + 1) & 3 : T;  // codes: the next k-step's, dequantized under this one's MFMAs
+    __asm__ volatile("s_waitcnt vmcnt(%3)" : "+v"(wr[WANTED][0]), "+v"(wr[WANTED][1]), "+v"(wr[WANTED][2]) : "n"(kFly) : "memory");
     static_for<0, IT>([&](auto cc) {
       constexpr int c = decltype(cc)::value;
       constexpr int ASET = c / AN, AI = c % AN;
       landed_a(fa[ASET][AI]);
 #pragma unroll
       for (int j = 0; j < JT; ++j) {
-        if (j < JA) acc[c][j] = Traits::mfma(wr[T][j], fa[ASET][AI], acc[c][j]);
-        else Traits::mfma_vgpr(wr[T][j], fa[ASET][AI], acc[c][j]);
+        v4i w;
+        if constexpr (W::kCodes) w = fb[T & 1][j];
+        else w = wr[T][j];
+        if (j < JA) acc[c][j] = Traits::mfma(w, fa[ASET][AI], acc[c][j]);
+        else Traits::mfma_vgpr(w, fa[ASET][AI], acc[c][j]);
       }
       if constexpr (c < AN) read_a(fa[1][c], caddr, IntC<c + AN>{});           // row tile c + 4 of this k-step
       else read_a(fa[0][c - AN], raddr, IntC<c - AN>{});                       // row tile c - 4 of the next
       if constexpr (c == 0) al.dma_at(src, nd, 2 * T);
       if constexpr (c == 4) al.dma_at(src, nd, 2 * T + 1);
-      if constexpr (c >= 1 && c <= 3) {                // the registers of the k-step before this one, for their next use
-        if constexpr (T == 0) fetch_w(IntC<3>{}, wr[3][c - 1], c - 1, s0);
+      if constexpr (c >= 1 && c <= 3) {                // the registers of the k-step before this one (codes: of this one), for their next use
+        if constexpr (W::kCodes) fetch_w(step, wr[T][c - 1], c - 1, s1);
+        else if constexpr (T == 0) fetch_w(IntC<3>{}, wr[3][c - 1], c - 1, s0);
         else fetch_w(IntC<T - 1>{}, wr[T - 1][c - 1], c - 1, s1);
       }
+      if constexpr (W::kCodes && c < 2 * JT) dequantize(WANTED, c >> 1, c & 1);
       __builtin_amdgcn_sched_barrier(0);
     });
   };

@@ -142,7 +142,7 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_w8
     gemm_frag::Part part;                                                                                                 \
     if (!gemm_frag::part_of<32 * IT, 128 * JT>(blockIdx.x, gridDim.x, M, N, uint32_t(K) / 128, sp, part)) return; \
     Epilogue epi{a_scale, w_scale, a_step, bias};                                                                         \
-    gemm_frag::run<I8Traits, IT, JT, D>(a, K, w_frag, epi, y, M, N, part, lds);                                           \
+    gemm_frag::run<I8Traits, IT, JT, D>(a, K, gemm_core::Values{w_frag}, epi, y, M, N, part, lds);                                           \
   }
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t32x128, 1, 1, 4, 2)
 MTRT_W8_FRAG_KERNEL(mtrt_gemm_w8a8_frag_t64x128, 2, 1, 4, 2)
@@ -159,7 +159,7 @@ __device__ __forceinline__ void wide_kernel(const int8_t* __restrict__ a, const 
   const int64_t tiles_m = (M + 255) / 256, panels = (N + gemm_frag::kWideBN - 1) / gemm_frag::kWideBN;
   int64_t tile_m, panel;
   if (!gemm_core::tile_of_even(blockIdx.x, gridDim.x, tiles_m, panels, tiles_m, tile_m, panel)) return;
-  gemm_frag::run_wide<I8Traits>(a, K, w_frag, (N + 31) / 32, epi, y, M, N, K / 128, tile_m * 256, panel * gemm_frag::kWideBN, lds);
+  gemm_frag::run_wide<I8Traits>(a, K, gemm_core::Values{w_frag}, (N + 31) / 32, epi, y, M, N, K / 128, tile_m * 256, panel * gemm_frag::kWideBN, lds);
 }
 extern "C" __global__ void __launch_bounds__(256, 1) mtrt_gemm_w8a8_frag_t256x384(
     const int8_t* __restrict__ a, const int8_t* __restrict__ w_frag, const float* __restrict__ a_scale,

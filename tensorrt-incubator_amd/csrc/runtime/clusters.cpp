@@ -1747,23 +1747,24 @@ DensePlan dense_frag_plan(int64_t M, int64_t K, int64_t N, int64_t units, bool m
   p.rows = M <= 64 && (!p.tile.tile || frag_rows_us(M, N, K / 64, units) < p.tile.us);
   return p;
 }
-int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, const void *w_frag, const void *bias, void *y, int32_t dtype,
-                        int64_t M, int64_t K, int64_t N, void *partial, int64_t partial_bytes) {
+// w_scale: of float8 codes (f32 [N]), null where w_frag holds the weights themselves
+int32_t dense_fragments(DeviceState *st, hipStream_t stream, const void *x, const void *w_frag, const float *w_scale, const void *bias, void *y,
+                        int32_t dtype, int64_t M, int64_t K, int64_t N, void *partial, int64_t partial_bytes) {
   DensePlan plan = dense_frag_plan(M, K, N, num_compute_units(st), true);
   if (!plan.rows && !bind_split(st, stream, plan.tile, partial, partial_bytes))
     plan = dense_frag_plan(M, K, N, num_compute_units(st), false);
   const char *xn = float_name(dtype);
   KernelName name("mtrt_gemm_dense_frag_");
-  name + xn + "_" + (plan.rows ? (M <= 32 ? "rows32" : "rows64") : plan.tile.tile ? plan.tile.tile->suffix : "");
-  if (plan.rows || (plan.tile.tile && plan.tile.tile->columns == 384 && plan.tile.tile->rows == 256)) {
-    void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N};
-    return launch(st, name, plan.rows ? uint32_t(std::min<int64_t>((N + 31) / 32, int64_t(kMaxGrid) * 1024)) : plan.tile.grid(),
-                  plan.rows ? 512 : 256, stream, args);
-  }
-  if (!plan.tile.tile)
+  name + xn + (w_scale ? "_f8_" : "_") + (plan.rows ? (M <= 32 ? "rows32" : "rows64") : plan.tile.tile ? plan.tile.tile->suffix : "");
+  if (!plan.rows && !plan.tile.tile)
     return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
-  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &plan.tile.split};
-  return launch(st, name, plan.tile.grid(), 256, stream, args);
+  const uint32_t grid = plan.rows ? uint32_t(std::min<int64_t>((N + 31) / 32, int64_t(kMaxGrid) * 1024)) : plan.tile.grid(), block = plan.rows ? 512 : 256;
+  if (plan.rows || (plan.tile.tile->columns == 384 && plan.tile.tile->rows == 256)) {
+    void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &w_scale};
+    return launch(st, name, grid, block, stream, args);
+  }
+  void *args[] = {&x, &w_frag, &bias, &y, &M, &K, &N, &plan.tile.split, &w_scale};
+  return launch(st, name, grid, block, stream, args);
 }
 
 int64_t round_up(int64_t v, int64_t step) { return (v + step - 1) / step * step; }
@@ -1792,10 +1793,10 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
       const W8Plan w = w8_plan(M, s.Kp, p.N, units, true);
       s.partial_bytes = w.kind == W8Plan::kTile && w.tile.tile ? w.tile.workspace() : 0;
     }
-  } else if (p.route == MTRT_LINEAR_DENSE) {
+  } else if (p.route == MTRT_LINEAR_DENSE || p.route == MTRT_LINEAR_DENSE_F8W) {
     // A K that is no whole number of slices costs an unquantized x a pass of its own (2.3 us and up), so small products
     // stay on the kernel that takes any K (about 15 us at a gigaflop).
-    s.fragments = p.w_frag && eb == 2 && (p.K % 64 == 0 || !p.w || quantized || 2.0 * double(M) * double(p.K) * double(p.N) >= 1e9);
+    s.fragments = p.w_frag && eb == 2 && (p.K % 64 == 0 || !p.w || p.route == MTRT_LINEAR_DENSE_F8W || quantized || 2.0 * double(M) * double(p.K) * double(p.N) >= 1e9);
     s.Kp = s.fragments ? round_up(p.K, 64) : p.K;
     // Up to 16 rows in one launch.  Its 16-column workgroups each take x: where they are at most one to a compute unit, twice as many
     // elements (bf16, float8 inputs, us, two launches and one: (8, 4096, 4096) 11.3, 10.1, (2, 14336, 512) 18.5, 12.7; (16, 1536, 8192) 9.4, 11.5);
@@ -1846,12 +1847,14 @@ int32_t activation_pass(DeviceState *st, hipStream_t stream, bool codes, const v
 const char *linear_fault(const mtrt_hip_linear_plan *p, int64_t M) {
   if (!p)
     return "null plan";
-  if (p->route < MTRT_LINEAR_W8A8 || p->route > MTRT_LINEAR_DENSE || !float_name(p->dtype))
+  if (p->route < MTRT_LINEAR_W8A8 || p->route > MTRT_LINEAR_DENSE_F8W || !float_name(p->dtype))
     return "unknown route or dtype";
   if (M < 0 || p->K <= 0 || p->N <= 0 || M > kMaxMatrixExtent || p->K > kMaxMatrixExtent || p->N > kMaxMatrixExtent)
     return "extents must be positive and below 2^31";
-  if (p->route != MTRT_LINEAR_DENSE && p->dtype != MTRT_F16)
+  if (p->route < MTRT_LINEAR_DENSE && p->dtype != MTRT_F16)
     return "this route computes in f16";
+  if (p->route == MTRT_LINEAR_DENSE_F8W && (float_bytes(p->dtype) != 2 || !p->w_frag || !p->w_scale || (p->q_dtype >= 0 && !p->x_scale)))
+    return "float8 weights need a 16-bit type, their codes, their scales, and a scale where x is quantized";
   if (p->q_dtype >= 0 && p->q_dtype != MTRT_I8 && p->q_dtype != MTRT_F8E4M3FN && p->q_dtype != MTRT_I4)
     return "activations go through i8, f8E4M3FN or i4 codes";
   if (p->route == MTRT_LINEAR_W8A8 && (p->q_dtype != MTRT_I8 || !p->x_scale || !p->w_scale || (!p->w && !p->w_frag)))
@@ -1865,27 +1868,29 @@ const char *linear_fault(const mtrt_hip_linear_plan *p, int64_t M) {
 } // namespace
 
 int64_t mtrt_hip_linear_fragments_bytes(int32_t dtype, int64_t K, int64_t N) {
-  const int eb = dtype == MTRT_I8 ? 1 : dtype == MTRT_F16 || dtype == MTRT_BF16 ? 2 : 0;
+  const int eb = dtype == MTRT_I8 || dtype == MTRT_F8E4M3FN ? 1 : dtype == MTRT_F16 || dtype == MTRT_BF16 ? 2 : 0;
   if (!eb || K <= 0 || N <= 0 || K > kMaxMatrixExtent || N > kMaxMatrixExtent)
     return 0;
-  return ((N + 31) / 32) * 32 * round_up(K * eb, 128);
+  return ((N + 31) / 32) * 32 * round_up(K * eb, dtype == MTRT_F8E4M3FN ? 64 : 128);
 }
 
 int32_t mtrt_hip_linear_prepack_fragments(mtrt_stream_t stream, const void *w_nk, int32_t dtype, void *w_frag, int64_t K, int64_t N) {
   clear_error();
   const int64_t bytes = mtrt_hip_linear_fragments_bytes(dtype, K, N);
   if (bytes == 0)
-    return set_error(MTRT_INVALID_ARGUMENT, "fragment order holds i8, f16 or bf16 weights of positive extents, got dtype %d [%lld, %lld]", dtype,
+    return set_error(MTRT_INVALID_ARGUMENT, "fragment order holds i8, f8E4M3FN, f16 or bf16 weights of positive extents, got dtype %d [%lld, %lld]", dtype,
                      (long long)N, (long long)K);
   if (!w_nk || !w_frag)
     return set_error(MTRT_INVALID_ARGUMENT, "null operand");
-  if (!aligned(w_frag, 16) || (dtype != MTRT_I8 && !aligned(w_nk, 2)))
+  if (!aligned(w_frag, 16) || !aligned(w_nk, float_bytes(dtype) == 2 ? 2 : 1))
     return set_error(MTRT_INVALID_ARGUMENT, "the fragment buffer must be 16-byte aligned, the weights aligned to their elements");
   DeviceState *st = device_state();
   if (!st)
     return MTRT_RUNTIME_ERROR;
   int32_t is_nk = 1;
   void *args8[] = {&w_nk, &w_frag, &K, &N, &is_nk}, *args16[] = {&w_nk, &w_frag, &K, &N};
+  if (dtype == MTRT_F8E4M3FN)
+    return launch(st, KernelName("mtrt_wf8_prepack_frag"), blocks_for(bytes / 8, kBlock), kBlock, as_hip(stream), args16);
   return launch(st, KernelName(dtype == MTRT_I8 ? "mtrt_w8_prepack_frag" : "mtrt_w16_prepack_frag"), blocks_for(bytes / 16, kBlock), kBlock,
                 as_hip(stream), dtype == MTRT_I8 ? args8 : args16);
 }
@@ -1922,7 +1927,8 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   const int eb = float_bytes(p.dtype);
   if (!x || !y)
     return set_error(MTRT_INVALID_ARGUMENT, "null operand");
-  if (!aligned(x, eb) || !aligned(y, eb) || !aligned(p.bias, eb) || !aligned(p.w_frag, 16))
+  if (!aligned(x, eb) || !aligned(y, eb) || !aligned(p.bias, eb) || !aligned(p.w_frag, 16) ||
+      (p.route == MTRT_LINEAR_DENSE_F8W && !aligned(p.w, 16)))
     return set_error(MTRT_INVALID_ARGUMENT, "x, y and bias must be aligned to their elements, w_frag to 16 bytes");
   DeviceState *st = device_state();
   if (!st)
@@ -1940,21 +1946,22 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   if (p.route == MTRT_LINEAR_W4A16)
     return w4a16(as_hip(stream), x, nullptr, p.w_frag, p.w_scale, p.bias, y, M, p.K, p.N, p.K, workspace, workspace_bytes);
   const LinearShape s = linear_shape(p, M, num_compute_units(st));
-  if (p.route == MTRT_LINEAR_DENSE && s.fragments && p.q_dtype < 0 && s.Kp == p.K && !aligned(x, 16))
+  if (p.route >= MTRT_LINEAR_DENSE && s.fragments && p.q_dtype < 0 && s.Kp == p.K && !aligned(x, 16))
     return set_error(MTRT_INVALID_ARGUMENT, "x must be 16-byte aligned for these weights");
   const int64_t need = s.act_bytes + s.partial_bytes;
   if (need > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < need))
     return set_error(MTRT_INVALID_ARGUMENT, "workspace of %lld bytes, 16-byte aligned, needed", (long long)need);
-  if (s.one_launch && p.route == MTRT_LINEAR_DENSE) {
+  const float *codes_scale = p.route == MTRT_LINEAR_DENSE_F8W ? static_cast<const float *>(p.w_scale) : nullptr;
+  if (s.one_launch && p.route >= MTRT_LINEAR_DENSE) {
     const float *x_scale = p.x_scale;
     const void *w_frag = p.w_frag, *bias = p.bias;
     int64_t K = p.K, Kp = s.Kp, N = p.N;
-    int32_t past = Kp * N * eb > tuning::kWeightsPastBytes;
+    int32_t past = Kp * N * (codes_scale ? 1 : eb) > tuning::kWeightsPastBytes;
     KernelName name("mtrt_gemm_dense_frag_");
     name + float_name(p.dtype) + (M * Kp <= kDecodeElements ? "_rows16" : "_rows16_long");
     if (p.q_dtype >= 0)
       name + "_" + code_name(p.q_dtype);
-    void *args[] = {&x, &x_scale, &w_frag, &bias, &y, &M, &K, &Kp, &N, &past};
+    void *args[] = {&x, &x_scale, &w_frag, &bias, &y, &M, &K, &Kp, &N, &past, &codes_scale};
     return launch(st, name, uint32_t((N + 15) / 16), 512, as_hip(stream), args);
   }
   if (s.one_launch) {
@@ -1985,7 +1992,7 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
                   kBlock, as_hip(stream), args);
   }
   if (s.fragments)
-    return dense_fragments(st, as_hip(stream), act, p.w_frag, p.bias, y, p.dtype, M, s.Kp, p.N, partial, s.partial_bytes);
+    return dense_fragments(st, as_hip(stream), act, codes_scale && p.w ? p.w : p.w_frag, p.w ? nullptr : codes_scale, p.bias, y, p.dtype, M, s.Kp, p.N, partial, s.partial_bytes);
   return mtrt_hip_linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N);
 }
 

@@ -443,18 +443,40 @@ class Linear:
                 packed = (kn[0::2] | (kn[1::2] << 4)).contiguous()
                 plan["w_prepacked"] = gemm_w4a16_prepack(packed, K, N)
                 plan["scale_kn"] = _scale_on_device(w_scale).reshape(-1).expand(N).to(torch.float16).reshape(1, N).contiguous()
+            elif self._keeps_codes(w_scale, per_out, has_x_scale, K, N):
+                # the codes themselves, which the kernels dequantize in registers: half the bytes of the dequantized matrix, the same bits
+                codes = q_weight.device_data().contiguous()
+                plan["codes_frag"] = self._fragments(codes, F8E4M3FN)
+                plan["s_w"] = _scale_on_device(w_scale).reshape(-1).expand(N).contiguous()
+                if K * N < self._CODES_ALONE_FROM[self.dtype] and self._room_for(codes, 2):
+                    values = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
+                    plan["values_frag"] = self._fragments(values)
             else:
                 plan["weight"] = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
         self._plan_key, self._plan_owners, self._plan = key, owners, plan
         self._native_plan = self._make_native_plan(plan, has_x_scale, K, N)
         return plan
 
+    # Weights from which on the prepared float8 module is its codes alone.  Where three modules' values stay in the Infinity Cache, a call of more
+    # than 16 rows reads them faster than it dequantizes codes (call times with codes over those with values: K = N = 4096, bf16 1.05 to 1.37 at 24
+    # to 1024 rows, f16 0.95 to 1.11; 3072 x 12800 bf16 1.05 to 1.25, f16 0.73 to 1.00; 5632 x 7616 0.72 to 1.06 and 0.71 to 0.92; from memory 0.70 to
+    # 1.06 and 0.66 to 0.97 at all of these), so smaller modules keep both where the device has room; up to 16 rows codes take 0.57 to 0.87 of the
+    # time, and nothing less than 0.9 where the weights are so few that a call is mostly its launch.
+    _CODES_FROM, _CODES_ALONE_FROM = 8 << 20, {float16: 32 << 20, bfloat16: 40 << 20}
+
+    def _keeps_codes(self, w_scale, per_out, has_x_scale, K, N):
+        """Whether the prepared weights are float8 codes in fragment order: products of 16-bit operands with a scale per tensor or output
+        channel, in every call (a ragged row that is not quantized takes [N, K] where the product is small)."""
+        return (self.quant_dtype == float8 and per_out and self.dtype in (float16, bfloat16) and w_scale.dtype == self.dtype and
+                w_scale.shape in ((), (N,)) and K >= 64 and K * N >= self._CODES_FROM and (K % 64 == 0 or has_x_scale) and
+                not _torch().cuda.is_current_stream_capturing())
+
     @staticmethod
-    def _fragments(w_nk):
-        """[N, K] weights (int8, float16, bfloat16) in the fragment order of the matrix-core kernels."""
+    def _fragments(w_nk, code=None):
+        """[N, K] weights (int8, float16, bfloat16, or codes of the type `code`) in the fragment order of the matrix-core kernels."""
         torch = _torch()
         N, K = w_nk.shape
-        code = {torch.int8: I8, torch.float16: F16, torch.bfloat16: BF16}[w_nk.dtype]
+        code = {torch.int8: I8, torch.float16: F16, torch.bfloat16: BF16}[w_nk.dtype] if code is None else code
         frag = torch.empty(lib().mtrt_hip_linear_fragments_bytes(code, K, N), dtype=torch.int8, device=w_nk.device)
         check(lib().mtrt_hip_linear_prepack_fragments(_stream(), w_nk.data_ptr(), code, frag.data_ptr(), K, N))
         return frag
@@ -476,6 +498,8 @@ class Linear:
             return native.linear_plan(self, 0, q_dtype, K, N, plan.get("w_nk"), plan.get("w_frag"), plan["s_w"], x_scale)
         if plan["route"] == "w4a16":
             return native.linear_plan(self, 1, None, K, N, None, plan["w_prepacked"], plan["scale_kn"], None)
+        if "codes_frag" in plan:
+            return native.linear_plan(self, 3, q_dtype, K, N, plan.get("values_frag"), plan["codes_frag"], plan["s_w"], x_scale)
         w = plan["weight"]
         if w.dtype != _torch_dtype(self.dtype):
             return None
@@ -496,12 +520,12 @@ class Linear:
         return native.linear_plan(self, 2, q_dtype, K, N, w, frag, None, x_scale)
 
     @staticmethod
-    def _room_for(w):
-        """Whether a second copy of the weights `w` leaves a quarter of the device's memory free: 16-bit weights that stay
-        beside their fragments take twice the memory, and a model that fills the device must still run."""
+    def _room_for(w, times=1):
+        """Whether a second copy of the weights `w` (`times` their bytes) leaves a quarter of the device's memory free: 16-bit weights that
+        stay beside their fragments take twice the memory, and a model that fills the device must still run."""
         cuda = _torch().cuda
         free, total = cuda.mem_get_info(w.device)
-        least = total // 4 + w.numel() * w.element_size()
+        least = total // 4 + times * w.numel() * w.element_size()
         # (what torch's allocator holds unused is free as well; asking it costs more than asking the device)
         return free > least or free + cuda.memory_reserved(w.device) - cuda.memory_allocated(w.device) > least
 
