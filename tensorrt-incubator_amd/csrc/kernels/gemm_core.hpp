@@ -775,9 +775,20 @@ __device__ __forceinline__ bool place(I item, I tiles_m, I tiles_n, int64_t& m, 
   return true;
 }
 
-template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool MANY = false, bool RAGGED = false, class W = Values, class Epilogue, typename Y>
+// The K split of tiles over workgroups (clusters.cpp: FragSplit), SPLIT: workgroup (tile, i) walks the slices [i per, (i + 1) per), writes its 32 x 32 sums
+// through to memory (4 KiB) and takes a ticket; the last of a tile's workgroups adds all of them in their order, the same bits whoever it is.
+// Nobody waits.  A tile without it is one unit's walk down K, with the other units idle.
+struct SplitK {
+  uint32_t splits, per;
+  float* partial;                                      // 1024 sums per tile and part, the parts of a tile together
+  uint32_t* tickets;                                   // a zeroed word per tile
+};
+
+template <class Traits, int WAVES, int MT = 1, bool FRAG = false, bool MANY = false, bool RAGGED = false, class W = Values, bool SPLIT = false, class Epilogue, typename Y>
 __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* __restrict__ w, int64_t row_bytes, Epilogue& epi,
-                                    Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds, const float* __restrict__ w_scale = nullptr) {
+                                    Y* __restrict__ y, int64_t M, int64_t N, int8_t* lds, const float* __restrict__ w_scale = nullptr,
+                                    const SplitK* split = nullptr) {
+  static_assert(!SPLIT || (MANY && sizeof(typename Traits::Scalar) == 4), "one 32 x 32 tile at a time, of 32-bit sums");
   static_assert(!W::kCodes || FRAG, "codes in fragment order");
   using WPiece = typename std::conditional<W::kCodes, u32x2, u32x4>::type;
   using WAccess = typename std::conditional<RAGGED, u32x4_anywhere, WPiece>::type;
@@ -792,15 +803,24 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
   const int frow = lane & 31, fhalf = lane >> 5;
   const int lrow = lane >> 3, lchunk = (lane & 7) * 16;
   const int64_t slices = RAGGED ? (row_bytes + 127) / 128 : row_bytes / 128;
-  const int64_t kb0 = slices * wave / WAVES, kb1 = slices * (wave + 1) / WAVES;
+  int64_t kb0 = slices * wave / WAVES, kb1 = slices * (wave + 1) / WAVES;
   int8_t* sa = lds + wave * kWaveBytes;
   int8_t* sw = sa + MT * kStageBytes;
   const int64_t tiles = (N + 31) / 32, tiles_m = MANY ? (M + 31) / 32 : 1;
   const int64_t items = MANY ? (tiles * tiles_m + 7) / 8 * 8 : tiles;
-  for (int64_t item = blockIdx.x; item < items; item += gridDim.x) {
+  const int64_t work = SPLIT ? items * split->splits : items;
+  for (int64_t item = blockIdx.x; item < work; item += gridDim.x) {
     int64_t tile = item, m0 = 0;
+    uint32_t part = 0;
+    if constexpr (SPLIT) {                             // part after part, in each of them as below
+      part = uint32_t(item) / uint32_t(items);
+      tile = item - int64_t(part) * items;
+      const int64_t from = int64_t(part) * split->per, length = part + 1 < split->splits ? split->per : slices - from;
+      kb0 = from + length * wave / WAVES;
+      kb1 = from + length * (wave + 1) / WAVES;
+    }
     if (MANY) {
-      const bool there = items < (int64_t(1) << 28) ? place(uint32_t(item), uint32_t(tiles_m), uint32_t(tiles), m0, tile) : place(item, tiles_m, tiles, m0, tile);
+      const bool there = items < (int64_t(1) << 28) ? place(uint32_t(tile), uint32_t(tiles_m), uint32_t(tiles), m0, tile) : place(tile, tiles_m, tiles, m0, tile);
       if (!there) continue;                            // the whole workgroup
       m0 *= 32;
     }
@@ -892,11 +912,43 @@ __device__ __forceinline__ void run(const int8_t* __restrict__ a, const int8_t* 
 #pragma unroll
       for (int r = 0; r < 16; ++r) mine[(t * 16 + r) * 64 + lane] = acc[t][r];
     __syncthreads();
+    const int64_t id = SPLIT ? tile * tiles_m + m0 / 32 : 0;
+    if constexpr (SPLIT) {
+      float* mine = split->partial + (id * split->splits + part) * 1024;
+      for (int e = threadIdx.x; e < 1024; e += 64 * WAVES) {
+        Scalar v = reinterpret_cast<const Scalar*>(lds)[e];
+#pragma unroll
+        for (int k = 1; k < WAVES; ++k) v = v + reinterpret_cast<const Scalar*>(lds + k * kWaveBytes)[e];
+        __hip_atomic_store(mine + e, __builtin_bit_cast(float, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");   // written through: visible to the whole device
+      __syncthreads();
+      uint32_t* seen = reinterpret_cast<uint32_t*>(lds);
+      if (threadIdx.x == 0) {
+        *seen = __hip_atomic_fetch_add(split->tickets + id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (*seen == split->splits - 1) __hip_atomic_store(split->tickets + id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      __syncthreads();
+      const bool last = *seen == split->splits - 1;
+      __syncthreads();                                 // (read by all before the next tile's slices land there)
+      if (!last) continue;
+    }
     for (int e = threadIdx.x; e < MT * 16 * 64; e += 64 * WAVES) {
       const int t = e >> 10, r = (e >> 6) & 15, l = e & 63;
-      Scalar v = reinterpret_cast<const Scalar*>(lds)[e];
+      Scalar v;
+      if constexpr (SPLIT) {
+        const float* from = split->partial + id * split->splits * 1024 + e;
+        float parts[8];                                // asked for together; what a split of fewer does not have is its first again
 #pragma unroll
-      for (int k = 1; k < WAVES; ++k) v = v + reinterpret_cast<const Scalar*>(lds + k * kWaveBytes)[e];
+        for (int k = 0; k < 8; ++k) parts[k] = __hip_atomic_load(from + (k < int(split->splits) ? k : 0) * 1024, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        v = __builtin_bit_cast(Scalar, parts[0]);
+#pragma unroll
+        for (int k = 1; k < 8; ++k) v = k < int(split->splits) ? v + __builtin_bit_cast(Scalar, parts[k]) : v;
+      } else {
+        v = reinterpret_cast<const Scalar*>(lds)[e];
+#pragma unroll
+        for (int k = 1; k < WAVES; ++k) v = v + reinterpret_cast<const Scalar*>(lds + k * kWaveBytes)[e];
+      }
       const int64_t row = m0 + t * 32 + (r >> 2) * 8 + (l >> 5) * 4 + (r & 3);
       const int64_t c = tile * 32 + (l & 31);
       if (row < M && c < N) y[row * N + c] = Y(epi.finish(v, row, c));

@@ -460,6 +460,25 @@ MTRT_DENSE_ROWS128_KERNEL(bf16, BF16)
 // All of them sum K in four parts or more, then the parts: the error against 64 bits is half of one chain's (K = 4096: 4.5e-7 and 9.0e-7 of the result).
 MTRT_DENSE_ROWS_F32_KERNEL(mfma, 4, 1, true)
 
+// ... 32 x 32 tiles, K shared by eight waves of up to eight workgroups (gemm_core::rows32::SplitK): (x, w, bias, y, M, K, N, SplitK), grid: any, block = 512;
+// _ragged: rows of at least 16 bytes that are no whole slices, any alignment.  Bound by the matrix cores of the units that have a workgroup, and where K is
+// short by 3 us of meeting.  us, whole and in 2, 3, 4, 6 and 8 parts (the units hold 256): (66, 11072, 576), 54 tiles, 60.0; 34.6, 26.8, 22.6, 30.5, 26.9; (96,
+// 12288, 300), 30 tiles, 64.9; 37.5, 27.6, 23.1, 19.0, 17.9; (109, 3072, 448), 56 tiles, 20.7; 15.1, 12.7, 12.1, 16.1, 15.9; (257, 12288, 512), 144, 69.3; 71.6,
+// 52.5, 60.0; (231, 10496, 1318), 336, 108; 89, 81, 89; (200, 2048, 1024), 224, 16.3; 20.6; (70, 608, 942), 90, 7.7; 8.4.  (128 registers instead of 137, so
+// that a unit has two workgroups: 36 bytes of scratch, 2 % slower where it has one and 3 % faster where two.)  The error against 64 bits is 0.3 to 0.7 of the
+// whole walk's.
+#define MTRT_DENSE_SPLIT_F32_KERNEL(NAME, RAGGED)                                                                  \
+  extern "C" __global__ void __launch_bounds__(512) mtrt_gemm_dense_##NAME##_f32(                                  \
+      const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M, \
+      int64_t K, int64_t N, gemm_core::rows32::SplitK split) {                                                     \
+    __shared__ __attribute__((aligned(16))) int8_t lds[gemm_core::rows32::lds_bytes<8>()];                         \
+    dense_cluster::RowsBiasF32Epilogue epi{bias};                                                                  \
+    gemm_core::rows32::run<dense_cluster::F32Traits, 8, 1, false, true, RAGGED, gemm_core::Values, true>(          \
+        reinterpret_cast<const int8_t*>(x), reinterpret_cast<const int8_t*>(w), K * 4, epi, y, M, N, lds, nullptr, &split); \
+  }
+MTRT_DENSE_SPLIT_F32_KERNEL(split, false)
+MTRT_DENSE_SPLIT_F32_KERNEL(split_ragged, true)
+
 // ... 128 x 128 tiles: (x, w, bias, y, M, K, N) ; grid: any, block = 256.
 extern "C" __global__ void __launch_bounds__(256, 2) mtrt_gemm_dense_t128x128_f32(
     const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ y, int64_t M,

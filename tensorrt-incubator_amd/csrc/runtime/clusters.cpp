@@ -77,6 +77,8 @@ constexpr double kF32FixedUs = 3.0, kF32Rows32StepUs = 0.18, kF32Rows64StepUs = 
 // by rounds of 256 x 128 tiles.  Fitted to 57 products, M 33 ... 65536, K 32 ... 11008, N 96 ... 65536; the form with the least estimate is the
 // fastest in each, or within 2 percent of it.
 constexpr double kF32FewTilesStepUs = 0.2, kF32TilesUs = 1.8, kF32TilesStepUs = 0.32;
+// ... K split over workgroups: fixed and meeting, then by rounds of one workgroup to a unit (measured beside the kernels)
+constexpr double kF32SplitUs = 4.0, kF32SplitRoundUs = 3.0, kF32SplitStepUs = 0.18, kF32SplitPromise = 0.95;
 constexpr double kF32T128OneUs = 10.0, kF32T128OneStepUs = 2.36, kF32T128TwoUs = 14.0, kF32T128TwoStepUs = 4.12;
 constexpr double kF32T256RoundUs = 30.0, kF32T256StepUs = 3.68;
 constexpr double kEdgeSmallFixedUs = 3.0, kEdgeSmallFewStepUs = 0.2, kEdgeSmallStepUs = 0.5;
@@ -1455,9 +1457,39 @@ int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const DotShape &
 }
 } // namespace
 
-int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w_nk, const void *bias, void *y,
-                              int32_t dtype, int64_t M, int64_t K, int64_t N) {
-  clear_error();
+namespace {
+// f32 products of more than 32 rows in 32 x 32 tiles whose K workgroups share: the parts with the shortest estimate, where it promises a twentieth
+// against the same tiles unsplit; for tiles that have a ticket each.
+struct F32Split {
+  FragSplit split;
+  int64_t tiles = 0;
+  double us = 0.0;
+  int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * 4096 : 0; }
+};
+F32Split f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
+  F32Split best;
+  best.tiles = ((M + 31) / 32) * ((N + 31) / 32);
+  const int64_t steps = (K * 4 + 127) / 128;
+  if (M <= 32 || best.tiles > int64_t(kTickets) || K < 4)
+    return best;
+  const double alone = tuning::kF32FixedUs + (best.tiles <= units ? double(steps) * tuning::kF32FewTilesStepUs
+                                                                  : (tuning::kF32TilesUs + double(steps) * tuning::kF32TilesStepUs) *
+                                                                        std::max(1.0, double(best.tiles) / double(2 * units)));
+  best.us = tuning::kF32SplitPromise * alone;
+  for (int parts : {2, 3, 4, 6, 8}) {
+    const FragSplit s = split_of(steps, parts);
+    const double rounds = double((best.tiles * int64_t(s.splits) + units - 1) / units);
+    const double us = tuning::kF32SplitUs + rounds * (tuning::kF32SplitRoundUs + tuning::kF32SplitStepUs * double(s.per));
+    if (steps >= 8 * parts && us < best.us) {
+      best.split = s;
+      best.us = us;
+    }
+  }
+  return best;
+}
+
+int32_t linear_dense(mtrt_stream_t stream, const void *x, const void *w_nk, const void *bias, void *y, int32_t dtype, int64_t M, int64_t K, int64_t N,
+                     void *workspace, int64_t workspace_bytes) {
   const char *xn = float_name(dtype);
   if (!xn)
     return set_error(MTRT_INVALID_ARGUMENT, "dense linear dtype %d is not one of f32/f16/bf16", dtype);
@@ -1483,6 +1515,26 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   if (few && M <= 8)
     return dense_few_rows_f32(st, as_hip(stream), dot, x, w_nk, bias, y, M, K, N);
   const int64_t tiles32 = (N + 31) / 32, small_tiles = ((M + 31) / 32) * tiles32;
+  F32Split split;
+  if (dtype == MTRT_F32 && workspace && aligned(workspace, 16)) {
+    split = f32_split(M, K, N, units);
+    if (split.workspace() > workspace_bytes)
+      split = F32Split();
+  }
+  // true: launched (or failed, in *rc) in parts, which take less than `us`
+  const auto in_parts = [&](double us, bool ragged, int32_t *rc) {
+    if (split.split.splits <= 1 || split.us >= us)
+      return false;
+    split.split.partial = workspace;
+    split.split.tickets = split_tickets(st, as_hip(stream), uint32_t(split.tiles));
+    if (!split.split.tickets)
+      return false;
+    void *sargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N, &split.split};
+    *rc = launch(st, KernelName(ragged ? "mtrt_gemm_dense_split_ragged_f32" : "mtrt_gemm_dense_split_f32"),
+                 uint32_t(8 * ((split.tiles + 7) / 8) * int64_t(split.split.splits)), 512, as_hip(stream), sargs);
+    return true;
+  };
+  int32_t rc;
   const bool whole_slices = K > 0 && (K * eb) % 128 == 0 && aligned(x, 16) && aligned(w_nk, 16);
   if (whole_slices && dtype == MTRT_F32) {
     // In 32 x 32 tiles, or up to 128 rows a column tile's rows together, or up to 32 on the vector units in groups of eight; in larger tiles where
@@ -1497,6 +1549,8 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
       const double t128_us = double(tiles128 / (2 * units)) * two_us + (rest128 == 0 ? 0.0 : rest128 <= units ? one_us : two_us);
       const double t256_us = double((tiles256 + units - 1) / units) * (tuning::kF32T256RoundUs + steps * tuning::kF32T256StepUs);
       const int64_t grid256 = 8 * ((tiles256 + 7) / 8);
+      if (in_parts(std::min({t256_us, t128_us, tiles_us, M <= 128 && rounds <= tuning::kF32RowsRounds ? rows_us : tiles_us}), false, &rc))
+        return rc;
       void *rargs[] = {&x, &w_nk, &bias, &y, &M, &K, &N};
       if (t256_us < std::min(t128_us, tiles_us) && M * K < (int64_t(1) << 30) && N * K < (int64_t(1) << 30) && launchable(grid256, kBlock))
         return launch(st, KernelName("mtrt_gemm_dense_t256x128_f32"), uint32_t(grid256), kBlock, as_hip(stream), rargs);
@@ -1555,6 +1609,8 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
     // 4.4; (16, 600, 8000) 9.1, 9.9; (32, 4097, 4096) 38.7, 40.5
     if (few && 3.0 + double((M + 7) / 8) * 4.0 * double(K * N) / tuning::kDotGroupBytesPerUs < std::min(small_us, edge_us))
       return dense_few_rows_f32(st, as_hip(stream), dot, x, w_nk, bias, y, M, K, N);
+    if (in_parts(std::min(small_us, edge_us), true, &rc))
+      return rc;
     int32_t waves = 0;
     if (K * eb >= 16 && small_us < edge_us)
       waves = dtype == MTRT_F32 && small_tiles <= units ? 8 : 4;
@@ -1566,6 +1622,13 @@ int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w
   if (tiles > int64_t(kMaxGrid) * 1024)
     return set_error(MTRT_INVALID_ARGUMENT, "problem [%lld, %lld] needs too many tiles", (long long)M, (long long)N);
   return launch(st, KernelName("mtrt_gemm_dense_") + xn, uint32_t(tiles), kBlock, as_hip(stream), args);
+}
+} // namespace
+
+int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const void *x, const void *w_nk, const void *bias, void *y, int32_t dtype, int64_t M, int64_t K,
+                              int64_t N) {
+  clear_error();
+  return linear_dense(stream, x, w_nk, bias, y, dtype, M, K, N, nullptr, 0);
 }
 
 namespace {
@@ -1813,6 +1876,8 @@ LinearShape linear_shape(const mtrt_hip_linear_plan &p, int64_t M, int64_t units
     if (s.fragments) {
       const DensePlan d = dense_frag_plan(M, s.Kp, p.N, units, true);
       s.partial_bytes = !d.rows && d.tile.tile ? d.tile.workspace() : 0;
+    } else if (eb == 4) {
+      s.partial_bytes = f32_split(M, p.K, p.N, units).workspace();
     }
   }
   return s;
@@ -1993,7 +2058,7 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   }
   if (s.fragments)
     return dense_fragments(st, as_hip(stream), act, codes_scale && p.w ? p.w : p.w_frag, p.w ? nullptr : codes_scale, p.bias, y, p.dtype, M, s.Kp, p.N, partial, s.partial_bytes);
-  return mtrt_hip_linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N);
+  return linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N, partial, s.partial_bytes);
 }
 
 } // extern "C"

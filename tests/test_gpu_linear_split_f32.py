@@ -1,0 +1,50 @@
+"""float32 Linears whose 32 x 32 tiles have their K shared by workgroups: every number of parts, rows and columns at the ends of tiles, rows that are whole slices
+and rows that are not, against float64; the same bits from call to call, with the tickets back at zero, on two streams and in a replayed graph."""
+import importlib
+import math
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+# (M, K, N, parts)
+SHAPES = [(33, 1024, 33, 4), (128, 1056, 512, 4), (300, 1536, 256, 3), (65, 3072, 31, 8), (64, 2048, 1, 8), (109, 3072, 448, 4), (257, 4096, 300, 2), (200, 2048, 180, 6), (33, 8192, 1024, 4), (231, 10496, 1318, 3),
+          (34, 1025, 97, 4), (66, 4099, 64, 8), (150, 5449, 515, 3), (40, 2047, 300, 8)]
+
+
+@pytest.fixture(scope="module")
+def tp(pkg):
+    return importlib.import_module(pkg.__name__ + ".tp")
+
+
+@pytest.mark.parametrize("M,K,N,parts", SHAPES)
+def test_parts_against_float64(tp, pkg, M, K, N, parts):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    w, b = torch.randn((N, K), generator=g, device="cuda") / math.sqrt(K), torch.randn(N, generator=g, device="cuda")
+    lin = tp.Linear(K, N, dtype=tp.float32)
+    lin.load_state_dict({"weight": tp.Tensor(w), "bias": tp.Tensor(b)})
+    x = torch.randn((M, K), generator=g, device="cuda")
+    y = lin(tp.Tensor(x)).torch()
+    assert pkg.last_kernel() == "mtrt_gemm_dense_split%s_f32" % ("_ragged" if K % 32 else ""), (pkg.last_kernel(), parts)
+    ref, mass = x.double() @ w.double().T + b.double(), x.double().abs() @ w.double().abs().T + b.double().abs()
+    # K products and additions, the bias and one more rounding, each within half an ulp of what it rounds
+    assert bool(((y.double() - ref).abs() <= (K + 3) * 2.0 ** -24 * mass).all())
+    for _ in range(3):
+        assert torch.equal(lin(tp.Tensor(x)).torch(), y)
+    streams, out = [torch.cuda.Stream() for _ in range(2)], []
+    torch.cuda.synchronize()
+    for i in range(6):
+        with torch.cuda.stream(streams[i % 2]):
+            out.append(lin(tp.Tensor(x)).torch())
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, y) for o in out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = lin(tp.Tensor(x)).torch()
+    for _ in range(3):
+        captured.fill_(7.0)
+        graph.replay()
+        assert torch.equal(lin(tp.Tensor(x)).torch(), y)
+        torch.cuda.synchronize()
+        assert torch.equal(captured, y)
