@@ -735,3 +735,22 @@ MTRT_NORM_OTHER_FORMS(bf16, BF16)
 MTRT_LAYERNORM_GROUP_KERNEL(f32, F32, 8, 256, g, false, 256, true, e)
 MTRT_SOFTMAX_GROUP_KERNEL(f32, F32, 8, 1024, u, true, 1024, false, a)
 MTRT_SOFTMAX_GROUP_KERNEL(f32, F32, 16, 1024, u, true, 1024, false, a)
+
+// Softmax of 16-bit rows of 32769 to 65536 elements where there are more rows than compute units: the exponentials are computed again in the output pass
+// instead of kept, 62 or 64 registers instead of 84 to 103, so that a unit has two rows and one's arithmetic lies under the other's way to memory; the same bits.
+// What bounds it: memory and the vector units, each idle for a part of a row.  `r`: to the row's end, `ra`: every vector.  us, kept and computed
+// again, bf16 [1084, 43165] 46.8, 41.1; [2000, 34000] 60.4, 52.2; [512, 50000] 24.4, 21.1; [300, 40000] 15.9, 14.6; rows past 0.8 of the vectors [1084, 64000] 59.1,
+// 57.5, every vector 54.1; [300, 64000] 22.2, 21.7, 19.0; up to a row to a unit [230, 40000] 9.6, 10.2; [230, 64000] 14.0, 15.4, 14.5.
+#define MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, TAG, RAGGED, ALL, NAME, PAST)                                     \
+  extern "C" __global__ void __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8, 8))) mtrt_softmax_##XN##_##TAG##1024v8##NAME(  \
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) {                                         \
+    __shared__ double lds[16];                                                                                 \
+    const int64_t row = blockIdx.x;                                                                            \
+    if (row < rows) softmax_group_row<XT, 8, 1024, false, ALL, false, RAGGED, PAST>(x, y, row, d, lds);        \
+  }
+#define MTRT_SOFTMAX_TWO_ROWS_KERNELS(XN, XT)                                                                  \
+  MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, g, false, false, r, true) MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, g, false, false, rt, false)  \
+  MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, g, false, true, ra, true) MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, g, false, true, rat, false)  \
+  MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, u, true, false, r, true) MTRT_SOFTMAX_TWO_ROWS_KERNEL(XN, XT, u, true, false, rt, false)
+MTRT_SOFTMAX_TWO_ROWS_KERNELS(f16, F16)
+MTRT_SOFTMAX_TWO_ROWS_KERNELS(bf16, BF16)

@@ -602,6 +602,13 @@ const char *row_form(bool layernorm, int32_t dtype, bool ragged, int lanes, int 
   return "";
 }
 
+// ... and the softmax kernels of two rows to a unit, where there are rows for them (norm.hip has the figures).
+const char *softmax_form(int32_t dtype, bool ragged, int lanes, int nv, int64_t rows, int64_t nvec_per_row, int64_t units) {
+  if (dtype != MTRT_F32 && lanes == 1024 && nv == 8 && rows > units)
+    return !ragged && 10 * nvec_per_row > 8 * int64_t(lanes * nv) ? "ra" : "r";
+  return row_form(false, dtype, ragged, lanes, nv, rows, nvec_per_row, units);
+}
+
 // Softmax rows that are no whole cache lines, of 20 to 80 MiB together, are read through the caches: the line that two rows share is fetched once, and what an
 // earlier launch has left in the Infinity Cache comes from there.  Whole lines gain from the second alone, and a launch that has just made x, or memory, is the
 // more common place for it to come from.  us, past and through, (rows, columns): three tensors in turn; each from memory; with a launch that makes x in front and
@@ -1208,7 +1215,7 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
                   blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
   int threads, gnv;
   if (vec_ok && !nv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))
-    return launch(st, KernelName("mtrt_softmax_") + xn + "_g" + threads + "v" + gnv + row_form(false, dtype, false, threads, gnv, rows, d / per_vec, num_compute_units(st)) + through, uint32_t(rows), uint32_t(threads),
+    return launch(st, KernelName("mtrt_softmax_") + xn + "_g" + threads + "v" + gnv + softmax_form(dtype, false, threads, gnv, rows, d / per_vec, num_compute_units(st)) + through, uint32_t(rows), uint32_t(threads),
                   as_hip(stream), args);
   // Row lengths that are not whole vectors, or operands that are not 16-byte aligned: the same two schemes with
   // 128-bit accesses at element alignment and the last d % per_vec elements of a row moved one by one.
@@ -1220,7 +1227,7 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
     }
     if (!rnv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv)) {
       gnv = unaligned_nv(dtype, gnv, false);
-      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + gnv + row_form(false, dtype, true, threads, gnv, rows, d / per_vec, num_compute_units(st)) + through, uint32_t(rows), uint32_t(threads),
+      return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + threads + "v" + gnv + softmax_form(dtype, true, threads, gnv, rows, d / per_vec, num_compute_units(st)) + through, uint32_t(rows), uint32_t(threads),
                     as_hip(stream), args);
     }
   }
