@@ -466,7 +466,7 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const voi
  *                     w_scale: f16 [1,N] (one block of all of K, K % 64 == 0); w unused
  *   MTRT_LINEAR_DENSE: x' = q_dtype < 0 ? x : dequantize(quantize(x, x_scale, q_dtype), x_scale); y = narrow(x' . w + bias[n]);
  *                     w: [N,K] in dtype, w_frag (F16 and BF16): mtrt_hip_linear_prepack_fragments of w, K rounded up to 64
- *   MTRT_LINEAR_DENSE_F8W (dtype F16 or BF16): MTRT_LINEAR_DENSE with w = dequantize(codes, w_scale), the weights' f8E4M3FN codes kept as such:
+ *   MTRT_LINEAR_DENSE_F8W (dtype F16 or BF16): MTRT_LINEAR_DENSE, q_dtype < 0 or MTRT_F8E4M3FN, with w = dequantize(codes, w_scale), the weights' f8E4M3FN codes kept as such:
  *                     w_frag: mtrt_hip_linear_prepack_fragments of the codes [N,K], w_scale: f32 [N], values of `dtype`; w: NULL, or
  *                     mtrt_hip_linear_prepack_fragments of the dequantized [N,K], which calls of many rows then take
  * w may be NULL when w_frag is given and K is a multiple of 128 (int8) or 64 (16-bit), w_frag when the shape or type has none.

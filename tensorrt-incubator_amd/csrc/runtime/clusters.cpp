@@ -1927,6 +1927,8 @@ const char *linear_fault(const mtrt_hip_linear_plan *p, int64_t M) {
     return "this route computes in f16";
   if (p->route == MTRT_LINEAR_DENSE_F8W && (float_bytes(p->dtype) != 2 || !p->w_frag || !p->w_scale || (p->q_dtype >= 0 && !p->x_scale)))
     return "float8 weights need a 16-bit type, their codes, their scales, and a scale where x is quantized";
+  if (p->route == MTRT_LINEAR_DENSE_F8W && p->q_dtype >= 0 && p->q_dtype != MTRT_F8E4M3FN)
+    return "float8 weights take an x that goes through f8E4M3FN codes, or a plain one";   // (no other kernel up to 16 rows reads codes)
   if (p->q_dtype >= 0 && p->q_dtype != MTRT_I8 && p->q_dtype != MTRT_F8E4M3FN && p->q_dtype != MTRT_I4)
     return "activations go through i8, f8E4M3FN or i4 codes";
   if (p->route == MTRT_LINEAR_W8A8 && (p->q_dtype != MTRT_I8 || !p->x_scale || !p->w_scale || (!p->w && !p->w_frag)))
