@@ -1466,7 +1466,8 @@ int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const DotShape &
 
 namespace {
 // f32 products of more than 32 rows in 32 x 32 tiles whose K workgroups share: the parts with the shortest estimate, where it promises a twentieth
-// against the same tiles unsplit; for tiles that have a ticket each.
+// against the same tiles unsplit; for tiles that have a ticket each, and at least one to an XCD (products in use have sixteen and more; of fewer the forms stay what
+// they are without a workspace).
 struct F32Split {
   FragSplit split;
   int64_t tiles = 0;
@@ -1477,7 +1478,7 @@ F32Split f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
   F32Split best;
   best.tiles = ((M + 31) / 32) * ((N + 31) / 32);
   const int64_t steps = (K * 4 + 127) / 128;
-  if (M <= 32 || best.tiles > int64_t(kTickets) || K < 4)
+  if (M <= 32 || best.tiles < 8 || best.tiles > int64_t(kTickets) || K < 4)
     return best;
   const double alone = tuning::kF32FixedUs + (best.tiles <= units ? double(steps) * tuning::kF32FewTilesStepUs
                                                                   : (tuning::kF32TilesUs + double(steps) * tuning::kF32TilesStepUs) *

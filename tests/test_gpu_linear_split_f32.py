@@ -8,8 +8,8 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 # (M, K, N, parts)
-SHAPES = [(33, 1024, 33, 4), (128, 1056, 512, 4), (300, 1536, 256, 3), (65, 3072, 31, 8), (64, 2048, 1, 8), (109, 3072, 448, 4), (257, 4096, 300, 2), (200, 2048, 180, 6), (33, 8192, 1024, 4), (231, 10496, 1318, 3),
-          (34, 1025, 97, 4), (66, 4099, 64, 8), (150, 5449, 515, 3), (40, 2047, 300, 8)]
+SHAPES = [(33, 1024, 97, 4), (128, 1056, 512, 4), (300, 1536, 256, 3), (65, 3072, 95, 8), (64, 2048, 97, 8), (109, 3072, 448, 4), (257, 4096, 300, 2), (200, 2048, 180, 6), (33, 8192, 1024, 4), (231, 10496, 1318, 3),
+          (34, 1025, 97, 4), (66, 4099, 65, 8), (150, 5449, 515, 3), (40, 2047, 300, 8)]
 
 
 @pytest.fixture(scope="module")
