@@ -1478,7 +1478,7 @@ F32Split f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
   F32Split best;
   best.tiles = ((M + 31) / 32) * ((N + 31) / 32);
   const int64_t steps = (K * 4 + 127) / 128;
-  if (M <= 32 || best.tiles < 8 || best.tiles > int64_t(kTickets) || K < 4)
+  if (M <= 32 || best.tiles < 8 || best.tiles > int64_t(kTickets) || steps < 16)   // (eight slices to a part at least)
     return best;
   const double alone = tuning::kF32FixedUs + (best.tiles <= units ? double(steps) * tuning::kF32FewTilesStepUs
                                                                   : (tuning::kF32TilesUs + double(steps) * tuning::kF32TilesStepUs) *
