@@ -80,7 +80,7 @@ template <> struct Vec<F16> {
 // line, and so the number of lanes that the first access leaves out (as far as a row that fills its lanes allows).
 // What bounds these rows is memory: an access that starts inside a line leaves a part of it to the next one, which is fetched and written as a part.
 // us, vectors from the row's first element on, on 16-byte boundaries, and on lines, f16 [48000, 1500] 51.9, 51.4, 48.5; [8000, 9001] 58.7, 52.3, 49.5; bf16
-// [1084, 43165] 54.4, 46.9, 44.7; f32 [24000, 1501] 51.4, 51.1, 49.5; whole vectors, f16 [24000, 3000] 49.9, 48.7.  (Staged through LDS, four rows' whole
+// [1084, 43165] 54.4, 46.9, 44.7; whole vectors, f16 [24000, 3000] 49.9, 48.7.  (Staged through LDS, four rows' whole
 // range at once, 48.3 for the first, but 52.9 with 1503 elements and 66 with 4500; LayerNorm bf16 [1500, 9011] 16.0 -> 14.0, but [700, 10243] 8.7 -> 9.4: behind
 // a head its parameters' vectors lie off their boundaries.)
 // A head puts the row's elements into other lanes, so its sum is taken in 64 bits: what the order of the terms changes there is a 2^-28th of the f32
@@ -427,7 +427,9 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   constexpr int E = Vec<X>::kElems;
   using V = typename RowVector<RAGGED>::type;
   const int lane = int(threadIdx.x) & (THREADS - 1);
-  constexpr bool kCut = RAGGED && THREADS >= kWave && NV > 2;   // (fewer vectors: what the 64-bit sums cost is more, bf16 [96000, 750] 51.3, 54.6)
+  // Fewer vectors, or 32-bit elements of which a line has half as many: what the 64-bit sums cost is more (uncut and cut, bf16 [96000, 750] 51.3, 54.6; f32
+  // [20, 20001] 4.5, 5.1; [20, 50001] 8.1, 8.7; [3000, 1001] 4.8, 5.0, for [24000, 1501] 51.4, 48.6; [500, 50001] 43.9, 40.3).
+  constexpr bool kCut = RAGGED && THREADS >= kWave && NV > 2 && sizeof(typename X::storage) == 2;
   using Sum = typename RowSum<kCut>::type;
   using Add = typename RowSum<kCut>::op;
   RowCut cut = {0, 0};
