@@ -472,7 +472,8 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const voi
  * w may be NULL when w_frag is given and K is a multiple of 128 (int8) or 64 (16-bit), w_frag when the shape or type has none.
  * The results are those of the single calls (quantize, dequantize, the GEMM entry point, an addition in dtype).
  * `workspace`: mtrt_hip_linear_workspace(plan, M) bytes of device memory, 16-byte aligned, the call's own until its work
- * on `stream` is done; less is MTRT_INVALID_ARGUMENT. */
+ * on `stream` is done; less is MTRT_INVALID_ARGUMENT, but that an F32 product needs no more than its x where that is quantized
+ * (M K values, rounded up to 256 bytes; otherwise none, or NULL): without room for partial sums its K is not split. */
 enum mtrt_hip_linear_route { MTRT_LINEAR_W8A8 = 0, MTRT_LINEAR_W4A16 = 1, MTRT_LINEAR_DENSE = 2, MTRT_LINEAR_DENSE_F8W = 3 };
 typedef struct mtrt_hip_linear_plan {
   int32_t route, dtype, q_dtype, reserved;

@@ -2023,7 +2023,8 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   const LinearShape s = linear_shape(p, M, num_compute_units(st));
   if (p.route >= MTRT_LINEAR_DENSE && s.fragments && p.q_dtype < 0 && s.Kp == p.K && !aligned(x, 16))
     return set_error(MTRT_INVALID_ARGUMENT, "x must be 16-byte aligned for these weights");
-  const int64_t need = s.act_bytes + s.partial_bytes;
+  // (an f32 product runs unsplit where the workspace has no room for its parts)
+  const int64_t need = s.act_bytes + (eb == 4 ? 0 : s.partial_bytes);
   if (need > 0 && (!workspace || !aligned(workspace, 16) || workspace_bytes < need))
     return set_error(MTRT_INVALID_ARGUMENT, "workspace of %lld bytes, 16-byte aligned, needed", (long long)need);
   const float *codes_scale = p.route == MTRT_LINEAR_DENSE_F8W ? static_cast<const float *>(p.w_scale) : nullptr;
@@ -2068,7 +2069,7 @@ int32_t mtrt_hip_linear(mtrt_stream_t stream, const mtrt_hip_linear_plan *plan, 
   }
   if (s.fragments)
     return dense_fragments(st, as_hip(stream), act, codes_scale && p.w ? p.w : p.w_frag, p.w ? nullptr : codes_scale, p.bias, y, p.dtype, M, s.Kp, p.N, partial, s.partial_bytes);
-  return linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N, partial, s.partial_bytes);
+  return linear_dense(stream, act, p.w, p.bias, y, p.dtype, M, p.K, p.N, partial, workspace_bytes - s.act_bytes);
 }
 
 } // extern "C"

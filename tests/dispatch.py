@@ -71,7 +71,7 @@ class Dispatch:
             return 8
         if name.startswith("mtrt_gemm_w4a16_t") and "_t256" not in name:
             return 9
-        if name.startswith("mtrt_gemm_dense_frag_") and "rows" not in name and "t256x384" not in name:
+        if name.startswith("mtrt_gemm_dense_frag_") and "rows" not in name and "t256x384" not in name or name.startswith("mtrt_gemm_dense_split"):
             return 7
         return None
 
