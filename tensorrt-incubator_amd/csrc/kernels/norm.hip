@@ -89,9 +89,9 @@ template <> struct Vec<F16> {
 struct RowCut { int head, shift; };
 template <bool CUT> struct RowSum { using type = float; using op = SumF32; };
 template <> struct RowSum<true> { using type = double; using op = SumF64; };
-// Of the places that a lane's vectors j = 0, 1, ... have, whether one is the row's, and the nearest that is: only the first can lie in front of it.
-__device__ __forceinline__ bool within(int j, int place, int shift, int end) { return place < end && (j > 0 || place >= shift); }
-__device__ __forceinline__ int held(int j, int place, int shift, int end) { return j > 0 ? min(place, end - 1) : max(shift, min(place, end - 1)); }
+// Of the places that a lane's vectors j = 0, 1, ... have, whether one is the row's, and the nearest that is: only the first can lie in front of a row that is CUT.
+template <bool CUT> __device__ __forceinline__ bool within(int j, int place, int shift, int end) { return place < end && (!CUT || j > 0 || place >= shift); }
+template <bool CUT> __device__ __forceinline__ int held(int j, int place, int shift, int end) { return !CUT || j > 0 ? min(place, end - 1) : max(shift, min(place, end - 1)); }
 template <typename X, int VECTORS>
 __device__ __forceinline__ RowCut cut_row(const typename X::storage* xr, const typename X::storage* yr, int64_t d) {
   const uint32_t at = uint32_t(reinterpret_cast<uintptr_t>(xr)), to = uint32_t(reinterpret_cast<uintptr_t>(yr));
@@ -112,14 +112,14 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int shif
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
-    const u32x4* p = row + (FULL ? idx : held(j, idx, shift, end));
+    const u32x4* p = row + (FULL ? idx : held<true>(j, idx, shift, end));
     t[j] = PAST ? __builtin_nontemporal_load(p) : *p;
   }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     Vec<X>::unpack(t[j], &v[j * E]);
     if (!FULL) {
-      const bool live = within(j, lane + kWave * j, shift, end);
+      const bool live = within<true>(j, lane + kWave * j, shift, end);
 #pragma unroll
       for (int k = 0; k < E; ++k) v[j * E + k] = live ? v[j * E + k] : fill;
     }
@@ -266,7 +266,7 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
     float o[E];
 #pragma unroll
     for (int k = 0; k < E; ++k) o[k] = v[j * E + k] * inv;
-    if (FULL || within(j, idx, shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
+    if (FULL || within<true>(j, idx, shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
 }
 
@@ -434,7 +434,10 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   using Add = typename RowSum<kCut>::op;
   RowCut cut = {0, 0};
   if constexpr (kCut) cut = cut_row<X, THREADS * NV>(x + row * d, y + row * d, d);
-  const int nvec = (int(d) - cut.head) / E, tail = RAGGED ? int(d) - nvec * E : 0, end = nvec + cut.shift;
+  // Uncut rows' vectors are counted from the 64-bit length: of a 32-bit quotient the compiler works each vector's place against the row's end out again in every
+  // pass, where it otherwise keeps the lanes' masks in scalar registers (us, 32 bits and 64, f32 [300, 9001] 6.8, 5.9; [300, 5001] 4.9, 4.6; [300, 60001] 35.5, 33.2;
+  // f16 [300, 18000] 8.05, 7.77).
+  const int nvec = kCut ? (int(d) - cut.head) / E : int(d / E), tail = RAGGED ? int(d) - nvec * E : 0, end = nvec + cut.shift;
   const V* xr = reinterpret_cast<const V*>(x + row * d + cut.head) - cut.shift;
   const bool extra = RAGGED && lane < tail;          // this lane also owns an element outside the vectors
   const int ec = (lane < cut.head ? 0 : nvec * E) + lane;
@@ -447,7 +450,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
     if (!wave_has<THREADS, ALL>(j, end)) break;
     const int idx = lane + THREADS * j;
     if (!RAGGED || !ALL || nvec > 0)                  // (a row shorter than one vector: only the scalar elements below)
-      t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : held(j, idx, cut.shift, end))) : xr[FULL ? idx : held(j, idx, cut.shift, end)];
+      t[j] = PAST ? __builtin_nontemporal_load(xr + (FULL ? idx : held<kCut>(j, idx, cut.shift, end))) : xr[FULL ? idx : held<kCut>(j, idx, cut.shift, end)];
   }
   // What lies past the row becomes -infinity where it is loaded: it changes no maximum and its exponential is zero, and the passes
   // below need not tell it from the row (us, f16 [1084, 50000] 61.2 -> 53.0, f32 [2000, 25001] 102 -> 97, bf16 [200, 8191] 7.5 -> 7.1; [48000, 1500] as before).
@@ -455,7 +458,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
       if (!wave_has<THREADS, ALL>(j, end)) break;
-      const bool live = within(j, lane + THREADS * j, cut.shift, end);
+      const bool live = within<kCut>(j, lane + THREADS * j, cut.shift, end);
 #pragma unroll
       for (int k = 0; k < 4; ++k) t[j][k] = live ? t[j][k] : Vec<X>::kMinusInf;
     }
@@ -507,7 +510,7 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
 #pragma unroll
       for (int k = 0; k < E; ++k) o[k] = __expf(v[k] - mx) * inv;
     }
-    if (FULL || within(j, idx, cut.shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
+    if (FULL || within<kCut>(j, idx, cut.shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
   if (extra) Tile<X>::store1(y + row * d + ec, ee * inv);
 }

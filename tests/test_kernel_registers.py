@@ -40,3 +40,11 @@ def test_row_kernels_spill_nothing(pkg, tmp_path):
     private = dict(re.findall(r"\.name:\s+(mtrt_(?:layernorm|softmax)_\S+)\n\s+\.private_segment_fixed_size:\s+(\d+)", metadata(pkg, tmp_path)))
     assert len(private) > 130
     assert {n for n, size in private.items() if size != "0"} <= {"mtrt_layernorm_bf16_v8r"}
+
+
+def test_softmax_keeps_the_masks_of_a_rows_end(pkg, tmp_path):
+    """A workgroup's softmax that works on every vector asks three times which of them are the row's; the answers stay in scalar registers, two to a
+    vector (worked out in each pass, f32 [300, 9001] takes 6.8 us instead of 5.9)."""
+    scalars = dict(re.findall(r"\.name:\s+(mtrt_softmax_\w+?_[gu](?:256v\d+|1024v\d+a)t?)\n(?:.*\n)*?\s+\.sgpr_count:\s+(\d+)", metadata(pkg, tmp_path)))
+    assert len(scalars) == 40
+    assert {n: int(s) for n, s in scalars.items() if int(s) < 3 * int(re.search(r"v(\d+)a?t?$", n).group(1))} == {}
