@@ -104,7 +104,7 @@ __device__ __forceinline__ RowCut cut_row(const typename X::storage* xr, const t
 // other places re-read the row's first or last vector and are replaced by `fill` afterwards), so the
 // loads are issued back to back with no branches between them; with FULL (the row fills all
 // 64 * NV vectors) the replacement disappears as well.
-template <typename X, int NV, bool FULL, bool PAST>
+template <typename X, int NV, bool FULL, bool PAST, bool CUT>
 __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int shift, int end, int lane, float fill,
                                          float (&v)[NV * Vec<X>::kElems]) {
   constexpr int E = Vec<X>::kElems;
@@ -112,14 +112,14 @@ __device__ __forceinline__ void load_row(const u32x4* __restrict__ row, int shif
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     const int idx = lane + kWave * j;
-    const u32x4* p = row + (FULL ? idx : held<true>(j, idx, shift, end));
+    const u32x4* p = row + (FULL ? idx : held<CUT>(j, idx, shift, end));
     t[j] = PAST ? __builtin_nontemporal_load(p) : *p;
   }
 #pragma unroll
   for (int j = 0; j < NV; ++j) {
     Vec<X>::unpack(t[j], &v[j * E]);
     if (!FULL) {
-      const bool live = within<true>(j, lane + kWave * j, shift, end);
+      const bool live = within<CUT>(j, lane + kWave * j, shift, end);
 #pragma unroll
       for (int k = 0; k < E; ++k) v[j * E + k] = live ? v[j * E + k] : fill;
     }
@@ -229,16 +229,16 @@ __device__ __forceinline__ void layernorm_rows(const typename X::storage* __rest
     layernorm_row<X, NV, false, RESIDENT>(x, gamma, beta, y, row, d, eps);
 }
 
-template <typename X, int NV, bool FULL, bool PAST>
+template <typename X, int NV, bool FULL, bool PAST, bool CUT>
 __device__ __forceinline__ void softmax_row(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                             int64_t row, int64_t d) {
   constexpr int E = Vec<X>::kElems;
   const int lane = threadIdx.x & (kWave - 1);
   const int nvec = int(d / E);
   const u32x4* xr = reinterpret_cast<const u32x4*>(x + row * d);
-  const int shift = FULL ? 0 : cut_row<X, kWave * NV>(x + row * d, y + row * d, d).shift, end = nvec + shift;
+  const int shift = !CUT ? 0 : cut_row<X, kWave * NV>(x + row * d, y + row * d, d).shift, end = nvec + shift;
   float v[NV * E];
-  load_row<X, NV, FULL, PAST>(xr - shift, shift, end, lane, -INFINITY, v);
+  load_row<X, NV, FULL, PAST, CUT>(xr - shift, shift, end, lane, -INFINITY, v);
 
   constexpr bool kLds = NV == 2 || NV == 4;
   float mx = -INFINITY;
@@ -251,7 +251,7 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
     v[i] = __expf(v[i] - mx);                        // exp(-inf) = 0 for the fill lanes
     s = s + v[i];
   }
-  if (!FULL) s = __shfl(s, (lane + shift) & (kWave - 1));   // each lane's sum to the lane that has it where the row starts on a line
+  if (CUT) s = __shfl(s, (lane + shift) & (kWave - 1));   // each lane's sum to the lane that has it where the row starts on a line
   s = row_reduce<kLds>(s, SumF32());
   // e / s as e * (1/s): one correctly rounded reciprocal per row instead of a divide per element; at most one
   // f32 ulp from the quotient.  Together with the hardware exponential (2^(d * log2 e), a few f32 ulps off for
@@ -266,20 +266,20 @@ __device__ __forceinline__ void softmax_row(const typename X::storage* __restric
     float o[E];
 #pragma unroll
     for (int k = 0; k < E; ++k) o[k] = v[j * E + k] * inv;
-    if (FULL || within<true>(j, idx, shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
+    if (FULL || within<CUT>(j, idx, shift, end)) __builtin_nontemporal_store(Vec<X>::pack(o), yr + idx);
   }
 }
 
-template <typename X, int NV, bool PAST>
+template <typename X, int NV, bool PAST, bool CUT>
 __device__ __forceinline__ void softmax_rows(const typename X::storage* __restrict__ x, typename X::storage* __restrict__ y,
                                              int64_t rows, int64_t d) {
   // the wave index as a scalar: the row pointers are then wave-uniform and the accesses need one lane offset, not an address pair each
   const int64_t row = int64_t(blockIdx.x) * kRowsPerBlock + __builtin_amdgcn_readfirstlane(int(threadIdx.x / kWave));
   if (row >= rows) return;
   if (PAST && d == int64_t(Vec<X>::kElems) * kWave * NV)   // (whole cache lines)
-    softmax_row<X, NV, true, true>(x, y, row, d);
+    softmax_row<X, NV, true, true, false>(x, y, row, d);
   else
-    softmax_row<X, NV, false, PAST>(x, y, row, d);
+    softmax_row<X, NV, false, PAST, CUT>(x, y, row, d);
 }
 
 // ---- rows longer than one wave's registers, and rows of any length or alignment: a GROUP of lanes owns one row ----
@@ -646,7 +646,8 @@ using namespace norm_cluster;
 // [4096, 4096] 11.3 -> 12.7 us and [16384, 4096] 47.4 -> 50.4 us, hence only inside that window).
 // Entry points.  mtrt_layernorm_<t>_v<NV>(x, gamma, beta, y, rows, d, eps)
 //                mtrt_softmax_<t>_v<NV>(x, y, rows, d)         NV = vectors per lane
-// Softmax kernels, here and below, with a t at the end: rows read through the caches, which don't fill all vectors.
+// Softmax kernels, here and below, with a t at the end: rows read through the caches, which don't fill all vectors; with a c: rows that are cut, past the caches (those
+// through them are, too).  A body of its own for either kind: both in one kernel are as slow for small tensors as the cut alone, whose code a launch has to fetch.
 #define MTRT_LN_OCCUPANCY_1
 #define MTRT_LN_OCCUPANCY_2
 #define MTRT_LN_OCCUPANCY_4
@@ -657,9 +658,11 @@ using namespace norm_cluster;
       const XT::storage* x, const XT::storage* gamma, const XT::storage* beta, XT::storage* y, int64_t rows,  \
       int64_t d, float eps) { layernorm_rows<XT, NV>(x, gamma, beta, y, rows, d, eps); }                      \
   extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_softmax_##XN##_v##NV(                        \
-      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, true>(x, y, rows, d); }  \
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, true, false>(x, y, rows, d); }  \
   extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_softmax_##XN##_v##NV##t(                     \
-      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, false>(x, y, rows, d); }
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, false, true>(x, y, rows, d); }  \
+  extern "C" __global__ void __launch_bounds__(kNormThreads) mtrt_softmax_##XN##_v##NV##c(                     \
+      const XT::storage* x, XT::storage* y, int64_t rows, int64_t d) { softmax_rows<XT, NV, true, true>(x, y, rows, d); }
 
 #define MTRT_NORM_FOR_TYPE(XN, XT)                                                                            \
   MTRT_NORM_KERNELS(XN, XT, 1) MTRT_NORM_KERNELS(XN, XT, 2) MTRT_NORM_KERNELS(XN, XT, 4)                       \

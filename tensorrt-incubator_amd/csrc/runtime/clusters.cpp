@@ -621,6 +621,13 @@ bool softmax_reads_past(int64_t rows, int64_t row_bytes) {
   return row_bytes % 128 == 0 || rows * row_bytes <= int64_t(20) << 20 || rows * row_bytes > int64_t(80) << 20;
 }
 
+// Softmax rows of whole vectors that start off a cache line are cut there (norm.hip) in tensors of 14 MiB and more.  us, uncut and cut, f16 [2000, 3000] 5.48, 5.59; bf16
+// [200, 5000] 4.26, 4.39; [600, 5000] 5.11, 5.18; f32 [3000, 1000] 4.82, 4.88; from 20 MB f16 [3333, 3000] 8.5, 8.2; bf16 [2000, 5000] 7.9, 7.6; f32 [24000, 1500] 48.7,
+// 47.4.  Whole lines have nothing to cut, and pay for it the same (f16 [3000, 1984] 4.68, 4.81).
+bool softmax_cuts(const void *x, int64_t rows, int64_t row_bytes) {
+  return (row_bytes % 128 != 0 || !aligned(x, 128)) && rows * row_bytes >= int64_t(14) << 20;
+}
+
 } // namespace
 
 extern "C" {
@@ -1211,7 +1218,7 @@ int32_t mtrt_hip_softmax(mtrt_stream_t stream, const void *x, void *y, int32_t d
     return launch(st, KernelName("mtrt_softmax_") + xn + "_u" + lanes + "v1" + through, blocks_for(rows, kBlock / lanes), kBlock, as_hip(stream), args);
   }
   if (nv && rows <= kMaxRowsPerWaveKernels)
-    return launch(st, KernelName("mtrt_softmax_") + xn + "_v" + nv + through,
+    return launch(st, KernelName("mtrt_softmax_") + xn + "_v" + nv + (!*through && softmax_cuts(x, rows, d * eb) ? "c" : through),
                   blocks_for(rows, kBlock / 64), kBlock, as_hip(stream), args);
   int threads, gnv;
   if (vec_ok && !nv && rows <= int64_t(kMaxGrid) * 1024 && pick_group(d / per_vec, &threads, &gnv))

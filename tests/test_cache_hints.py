@@ -79,6 +79,16 @@ def test_softmax_reads_its_rows_as_its_name_says(code):
         assert found["global_load_dwordx4", not kernel.endswith("t")] > 0 and found["global_load_dwordx4", kernel.endswith("t")] == 0, kernel
 
 
+def test_cut_softmax_rows_pass_the_caches_by(code):
+    names, accesses = code
+    kernels = names(r"mtrt_softmax_\w+_v\d+c")
+    assert len(kernels) == 15
+    for kernel, found in accesses(kernels).items():
+        for access in ("load", "store"):                             # (of one vector a lane: the stores of its two bodies folded, as above)
+            past, through = found["global_%s_dwordx4" % access, True], found["global_%s_dwordx4" % access, False]
+            assert past > 0 and (through == 0 or (access == "store" and kernel.endswith("_v1c"))), kernel
+
+
 def test_few_rows_read_int8_and_int4_weights_past_the_caches(code):
     """But where several groups of rows read them (the strips' fourth body), and in the second of W8A8's two bodies."""
     names, accesses = code

@@ -383,3 +383,16 @@ def test_softmax_rows_that_share_cache_lines_are_read_through_the_caches_from_20
             seen.add(name)
     forms = {re.sub("[ea]t$", "t", n.split("_")[3]) for n in seen}
     assert {f + "t" for f in ("u8v1", "u16v1", "u32v1", "u64v1", "u64v4", "v4", "v16", "g256v8", "g1024v16")} <= forms, forms
+
+
+@pytest.mark.parametrize("dtype,item", [("F32", 4), ("F16", 2), ("BF16", 2)])
+def test_whole_vectors_off_the_cache_lines_are_cut_from_14_mib(gpu, pkg, dtype, item):
+    """By the kernels that end in c where they go past the caches; rows that start on lines by none."""
+    for row_bytes, form in ((528, "v1"), (1040, "v2"), (2064, "v4"), (6000, "v8"), (10000, "v16"), (1024, None), (3968, None)):
+        at = -(-(14 << 20) // row_bytes)                             # the least number of rows of 14 MiB
+        for x, rows in [(x, rows) for x in (256, 256 + 16, 256 + 128) for rows in (1, at - 1, at, (20 << 20) // row_bytes, (80 << 20) // row_bytes + 1)]:
+            assert gpu.lib.mtrt_hip_softmax(None, x, 256, getattr(pkg, dtype), rows, row_bytes // item) == 0
+            name = gpu.launches[-1][0]
+            off = row_bytes % 128 != 0 or x % 128 != 0
+            assert name.endswith("c") == (off and rows >= at), (x, row_bytes, rows, name)
+            assert not form or name.split("_")[3] == form + ("c" if rows >= at else ""), name
