@@ -449,8 +449,11 @@ class Linear:
                 plan["codes_frag"] = self._fragments(codes, F8E4M3FN)
                 plan["s_w"] = _scale_on_device(w_scale).reshape(-1).expand(N).contiguous()
                 if K * N < self._CODES_ALONE_FROM[self.dtype] and self._room_for(codes, 2):
-                    values = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
-                    plan["values_frag"] = self._fragments(values)
+                    try:
+                        values = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
+                        plan["values_frag"] = self._fragments(values)
+                    except torch.OutOfMemoryError:     # the codes serve every call
+                        pass
             else:
                 plan["weight"] = dequantize(q_weight, self.weight_scale, self.dtype, self.weight_quant_dim).device_data().contiguous()
         self._plan_key, self._plan_owners, self._plan = key, owners, plan
