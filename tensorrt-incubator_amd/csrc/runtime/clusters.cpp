@@ -1481,7 +1481,7 @@ struct F32Split {
   double us = 0.0;
   int64_t workspace() const { return split.splits > 1 ? tiles * int64_t(split.splits) * 4096 : 0; }
 };
-F32Split f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
+F32Split make_f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
   F32Split best;
   best.tiles = ((M + 31) / 32) * ((N + 31) / 32);
   const int64_t steps = (K * 4 + 127) / 128;
@@ -1501,6 +1501,10 @@ F32Split f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
     }
   }
   return best;
+}
+F32Split f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
+  static thread_local LastPlan<F32Split> last;
+  return last.of(M, N, K, units, true, [&] { return make_f32_split(M, K, N, units); });
 }
 
 int32_t linear_dense(mtrt_stream_t stream, const void *x, const void *w_nk, const void *bias, void *y, int32_t dtype, int64_t M, int64_t K, int64_t N,
