@@ -470,7 +470,11 @@ MTRT_CAPI_EXPORTED int32_t mtrt_hip_linear_dense(mtrt_stream_t stream, const voi
  *                     w_frag: mtrt_hip_linear_prepack_fragments of the codes [N,K], w_scale: f32 [N], values of `dtype`; w: NULL, or
  *                     mtrt_hip_linear_prepack_fragments of the dequantized [N,K], which calls of many rows then take
  * w may be NULL when w_frag is given and K is a multiple of 128 (int8) or 64 (16-bit), w_frag when the shape or type has none.
- * The results are those of the single calls (quantize, dequantize, the GEMM entry point, an addition in dtype).
+ * The results are those of the single calls (quantize, dequantize, the GEMM entry point, an addition in dtype), in integer sums bit for bit, in float
+ * sums up to the order of their terms: in F16 and BF16 w_frag has kernels of its own, and an F32 product of more than 32 rows may have its K
+ * shared by workgroups whose sums are added, which mtrt_hip_linear_dense, without memory for them, does not.  It is not shared either where the
+ * workspace is too small or the workgroups have no words to meet in (hipStreamPerThread, more than 255 streams, recorded launches when their 4 Mi words
+ * are used up).  A call's bits are the same each time it is shared, and each time it is not.
  * `workspace`: mtrt_hip_linear_workspace(plan, M) bytes of device memory, 16-byte aligned, the call's own until its work
  * on `stream` is done; less is MTRT_INVALID_ARGUMENT, but that an F32 product needs no more than its x where that is quantized
  * (M K values, rounded up to 256 bytes; otherwise none, or NULL): without room for partial sums its K is not split. */

@@ -1,9 +1,13 @@
-"""float32 Linears whose 32 x 32 tiles have their K shared by workgroups: every number of parts, rows and columns at the ends of tiles, rows that are whole slices
-and rows that are not, against float64; the same bits from call to call, with the tickets back at zero, on two streams and in a replayed graph."""
+"""float32 Linears whose 32 x 32 tiles have their K shared by workgroups: every number of parts (test_linear_split_f32_plan.py has them on the CPU), rows and columns at
+the ends of tiles, rows that are whole slices and rows that are not, against float64; the same bits from call to call, with the tickets back at zero, on two
+streams and in a replayed graph; and beside the entry point that does not share."""
+import ctypes
 import importlib
 import math
 
 import pytest
+
+from test_gpu_linear_codes import Plan
 
 pytestmark = pytest.mark.gpu
 
@@ -48,3 +52,34 @@ def test_parts_against_float64(tp, pkg, M, K, N, parts):
         assert torch.equal(lin(tp.Tensor(x)).torch(), y)
         torch.cuda.synchronize()
         assert torch.equal(captured, y)
+
+
+@pytest.mark.parametrize("M,K,N,parts", SHAPES)
+def test_beside_the_call_that_does_not_share(tp, pkg, M, K, N, parts):
+    """mtrt_hip_linear without memory for the parts, mtrt_hip_linear_dense and a module whose bias is not contiguous: the same bits, which the shared sum
+    agrees with up to the order of its terms."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    w, b = torch.randn((N, K), generator=g, device="cuda") / math.sqrt(K), torch.randn(N, generator=g, device="cuda")
+    x = torch.randn((M, K), generator=g, device="cuda")
+    L, stream = pkg.lib(), torch.cuda.current_stream().cuda_stream
+    p = Plan(route=2, dtype=pkg.F32, q_dtype=-1, K=K, N=N, w=w.data_ptr(), bias=b.data_ptr())
+    need, out = L.mtrt_hip_linear_workspace(ctypes.byref(p), M), []
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        assert need == (M + 31) // 32 * ((N + 31) // 32) * parts * 4096
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    for memory in (need, need - 1, 0):
+        y = torch.full((M, N), 7.0, device="cuda")
+        pkg.check(L.mtrt_hip_linear(stream, ctypes.byref(p), x.data_ptr(), y.data_ptr(), M, ws.data_ptr() if memory else None, memory))
+        assert ("split" in pkg.last_kernel()) == (memory == need), pkg.last_kernel()
+        out.append(y)
+    shared, dense = out[0], pkg.linear_dense(x, w, b)
+    assert torch.equal(out[1], dense) and torch.equal(out[2], dense)
+    lin = tp.Linear(K, N, dtype=tp.float32)
+    wide = torch.zeros((N, 2), device="cuda")
+    wide[:, 0] = b
+    lin.weight, lin.bias = tp.Tensor(w), tp.Tensor(wide[:, 0])
+    assert torch.equal(lin(tp.Tensor(x)).torch(), dense)
+    # each within (K + 3) half ulps of the sum of the terms' sizes, test_parts_against_float64
+    mass = x.double().abs() @ w.double().abs().T + b.double().abs()
+    assert bool(((shared.double() - dense.double()).abs() <= 2 * (K + 3) * 2.0 ** -24 * mass).all())
