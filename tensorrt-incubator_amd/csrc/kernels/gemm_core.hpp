@@ -740,7 +740,7 @@ constexpr int kPitch = 144, kStageBytes = 32 * kPitch;
 // MT: activation row tiles of 32 (1: M <= 32, 2: M <= 64, the weight fragments of a k-step serving both)
 template <int WAVES, int MT = 1, bool FRAG = false> constexpr int lds_bytes() { return WAVES * (MT + (FRAG ? 0 : 1)) * kStageBytes; }
 
-// CODES: the fragments hold float8 codes (F8Codes), dequantized on their way into the MFMA.
+// W: how the weights lie: Values, or in fragment order F8Codes, dequantized on their way into the MFMA.
 // FRAG: `w` is not the [N,K] array but its fragment-order re-layout (per 32 rows and 128-byte slice four 1 KiB blocks,
 // lane l of block q holding the 16 bytes of k-step q of its row: exactly the second MFMA operand).  The weight
 // fragments then go from memory to registers and into the MFMA without passing LDS, 1 KiB contiguous per instruction.

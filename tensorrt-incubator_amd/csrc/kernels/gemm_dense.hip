@@ -508,10 +508,12 @@ extern "C" __global__ void __launch_bounds__(gemm_core::THREADS, 1) mtrt_gemm_de
 // K % 64 == 0, x and w_frag 16-byte aligned, x below 4 GiB; the rest as mtrt_gemm_w8a8_frag_t<rows>x<columns>.
 // mtrt_gemm_dense_frag_<type>_f8_...: float8 codes in their place (mtrt_wf8_prepack_frag), their scales w_scale (f32 [N]) the last argument.  Half the bytes on the way to a
 // unit (a slice of a 128 x 384 tile: 40 instead of 64 KiB) and from memory, for 16 (bf16) or 8 (f16) vector instructions to a fragment of eight
-// weights, which a wave issues beside the IT MFMAs that use it: what bounds it is the weights' way, in tiles of few rows those instructions.  us, values
-// and codes, bf16, weights from memory: (24, 4096, 11008) 0.76 of the time, (128, ..) 0.81, (512, ..) 0.87, (1024, ..) 0.96, (2048, ..) 1.04;
+// weights, which a wave issues beside the IT MFMAs that use it: what bounds it is the weights' way, in tiles of few rows those instructions.  Time of the
+// kernel with codes over that with values, bf16, weights from memory: (24, 4096, 11008) 0.76, (128, ..) 0.81, (512, ..) 0.87, (1024, ..) 0.96, (2048, ..) 1.04;
 // f16 0.74, 0.75, 0.81, 0.94, 1.01; from the Infinity Cache (K, N) = (4096, 4096) bf16 1.05, 1.21, 1.31, 1.14, 1.12, and f16 0.95, 1.05, 1.04, 1.04,
-// 1.03.  (By sets of four waves that share K, as W4A16's 32- and 64-row tiles are: no faster, the wave's own instructions are the limit.)
+// 1.03.  Whole calls, us, values and codes, twelve modules in turn, which come from memory either way, bf16 (24, 4096, 11008) 23.9, 19.3; (256, ..) 44.6, 40.6; (1024, ..) 88.9, 90.6;
+// (2048, ..) 152.7, 156.1; f16 24.0, 18.9; 44.6, 39.7; 90.7, 92.4; 163.8, 163.2; of three modules in turn, whose codes the Infinity Cache holds and whose values it does not, bf16 (1024, ..) 91.5,
+// 89.4; (2048, ..) 156.8, 153.0; (4096, ..) 313, 308; f16 93.0, 89.6; 166, 157; 332, 318.  (By sets of four waves that share K, as W4A16's 32- and 64-row tiles are: no faster, the wave's own instructions are the limit.)
 #define MTRT_DENSE_FRAG_KERNEL(XN, XT, WT, WPARAM, WARGS, IT, JT, D, WG, TILE)                                            \
   extern "C" __global__ void __launch_bounds__(256, WG) mtrt_gemm_dense_frag_##XN##_##TILE(                               \
       const int8_t* __restrict__ x, const int8_t* __restrict__ w_frag, const XT::storage* __restrict__ bias,              \

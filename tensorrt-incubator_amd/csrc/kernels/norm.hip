@@ -83,9 +83,12 @@ template <> struct Vec<F16> {
 // [1084, 43165] 54.4, 46.9, 44.7; whole vectors, f16 [24000, 3000] 49.9, 48.7.  (Staged through LDS, four rows' whole
 // range at once, 48.3 for the first, but 52.9 with 1503 elements and 66 with 4500; LayerNorm bf16 [1500, 9011] 16.0 -> 14.0, but [700, 10243] 8.7 -> 9.4: behind
 // a head its parameters' vectors lie off their boundaries.)
-// A head puts the row's elements into other lanes, so its sum is taken in 64 bits: what the order of the terms changes there is a 2^-28th of the f32
-// result's last place, and equal rows give equal bits wherever they lie.  (48.5 -> 49.3 and 44.7 -> 47.0 for the first and the third; the longer part is the exchange.)
-// A shift alone is undone by one exchange of the lanes' sums.
+// A head puts the row's elements into other lanes, so its sum is taken in 64 bits: what the order of the terms changes there is about a 2^-28th of the f32
+// result's last place, so that equal rows at different places in a line differ only where that much decides a rounding.  (48.5 -> 49.3 and 44.7 -> 47.0 for the first and the third; the longer part is the exchange.)
+// A shift alone is undone by one exchange of the lanes' sums: the same bits.
+// It costs more than it saves, and is taken all the same so that a row's bits do not follow the size of its tensor, in 16-bit rows of a wave that are read
+// through the caches, where the line that two rows share is fetched once anyhow (us, uncut and cut, f16 [5998, 5001] 20.9, 22.2; [2999, 5001] 11.7, 12.2; bf16 [5997, 2501]
+// 10.8, 11.1; f16 [19960, 1503] 19.4, 19.8; of a workgroup [1499, 20001] 22.3, 20.8), and in small tensors of four vectors a lane ([2661, 1503] 5.23, 5.34; [5322, 1503] 8.3, 7.3).
 struct RowCut { int head, shift; };
 template <bool CUT> struct RowSum { using type = float; using op = SumF32; };
 template <> struct RowSum<true> { using type = double; using op = SumF64; };
@@ -331,7 +334,8 @@ __device__ __forceinline__ void layernorm_group_row(const typename X::storage* _
   const V* xr = reinterpret_cast<const V*>(x + row * d);
   const bool extra = RAGGED && lane < tail;          // this lane also owns element nvec * E + lane
   const int ec = nvec * E + lane;
-  // asked for with the vectors, by every lane: in a branch, or behind them, it is a second trip to memory
+  // Asked for with the vectors, by every lane: in a branch, or behind them, it is a second trip to memory (us, behind and with them, f16 [24000, 1501] 30.7, 30.3; [64,
+  // 3001] 5.04, 4.92; bf16 [3000, 1001] 4.94, 4.85; f32 [300, 9001] 7.37, 7.21; [24000, 1501] 57.6, 57.9).
   typename X::storage xb = 0;
   if constexpr (RAGGED) xb = (x + row * d)[min(ec, int(d) - 1)];
   u32x4 t[NV];
@@ -441,7 +445,8 @@ __device__ __forceinline__ void softmax_group_row(const typename X::storage* __r
   const V* xr = reinterpret_cast<const V*>(x + row * d + cut.head) - cut.shift;
   const bool extra = RAGGED && lane < tail;          // this lane also owns an element outside the vectors
   const int ec = (lane < cut.head ? 0 : nvec * E) + lane;
-  // asked for with the vectors, by every lane: in a branch, or behind them, it is a second trip to memory
+  // Asked for with the vectors, by every lane, as in LayerNorm (us, behind and with them, f32 [124584, 301] 51.9, 50.5; [24983, 1501] 51.5, 50.9; [600, 25001] 22.1, 21.1; f16
+  // [79893, 751] 42.6, 41.7; bf16 [149625, 401] 46.6, 45.5; f16 [79207, 101] 8.8, 8.4; slower f32 [399, 25001] 15.0, 15.4; [300, 5001] 4.53, 4.57).
   typename X::storage xb = 0;
   if constexpr (RAGGED) xb = (x + row * d)[min(ec, int(d) - 1)];
   u32x4 t[NV];

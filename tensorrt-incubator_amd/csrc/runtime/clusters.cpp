@@ -1473,8 +1473,9 @@ int32_t dense_few_rows_f32(DeviceState *st, hipStream_t stream, const DotShape &
 
 namespace {
 // f32 products of more than 32 rows in 32 x 32 tiles whose K workgroups share: the parts with the shortest estimate, where it promises a twentieth
-// against the same tiles unsplit; for tiles that have a ticket each, and at least one to an XCD (products in use have sixteen and more; of fewer the forms stay what
-// they are without a workspace).
+// against the same tiles unsplit; for tiles that have a ticket each, and at least one to an XCD.  Of fewer tiles parts would be the faster as well (us, whole and in
+// parts, (64, 11072, 64) 57.3, 13.5; (64, 8192, 32) 43.1, 10.6; (50, 12288, 224) 63.5, 14.3; (33, 4096, 96) 22.6, 8.0; (65, 2048, 33) 13.0, 6.9; (33, 1024, 32) 7.9, 6.4): the line keeps
+// products of six tiles, which a test holds to an unsplit kernel, where they are, and is not there for their time.
 struct F32Split {
   FragSplit split;
   int64_t tiles = 0;
@@ -1485,7 +1486,7 @@ F32Split make_f32_split(int64_t M, int64_t K, int64_t N, int64_t units) {
   F32Split best;
   best.tiles = ((M + 31) / 32) * ((N + 31) / 32);
   const int64_t steps = (K * 4 + 127) / 128;
-  if (M <= 32 || best.tiles < 8 || best.tiles > int64_t(kTickets) || steps < 16)   // (eight slices to a part at least)
+  if (M <= 32 || best.tiles < 8 || best.tiles > int64_t(kTickets) || steps < 16)   // (eight slices to a part; the last one may have fewer)
     return best;
   const double alone = tuning::kF32FixedUs + (best.tiles <= units ? double(steps) * tuning::kF32FewTilesStepUs
                                                                   : (tuning::kF32TilesUs + double(steps) * tuning::kF32TilesStepUs) *

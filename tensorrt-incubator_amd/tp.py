@@ -361,10 +361,13 @@ class Linear:
         (The rank-2 scale of this API groups OUTPUT features, [out/B, in] as weight_loader.py:102-115 builds it;
         the W4A16 cluster's blocks run along the reduction axis, so that form takes the next route.)
       * everything else (float8 codes, scales along the input features, int4 blocks, other dtypes, no
-        quantization): the literal fake-quant form, DQ(Q(x)) @ DQ(Q(W))^T on the dense Linear kernel.
+        quantization): the literal fake-quant form, DQ(Q(x)) @ DQ(Q(W))^T on the dense Linear kernels.
 
     Weights are program constants: they are quantized, re-laid out and (for the last route) dequantized ONCE,
-    when first needed after `weight` / `weight_scale` were assigned; the forward pass only touches x."""
+    when first needed after `weight` / `weight_scale` were assigned; the forward pass only touches x.  Float8 weights of a
+    float16 or bfloat16 module with a scale per tensor or output channel stay codes from 8 Mi on: each call dequantizes
+    them in registers, to the same bits, and they take one byte a weight instead of two.  Below 32 Mi (float16) or 40 Mi
+    (bfloat16) their values are kept beside them, where the device has room: three bytes a weight."""
 
     def __init__(self, in_features, out_features, bias=True, dtype=float32, quant_dtype=None, weight_quant_dim=None):
         torch = _torch()
@@ -460,11 +463,11 @@ class Linear:
         self._native_plan = self._make_native_plan(plan, has_x_scale, K, N)
         return plan
 
-    # Weights from which on the prepared float8 module is its codes alone.  Where three modules' values stay in the Infinity Cache, a call of more
+    # Weights from which on the prepared float8 module is its codes alone.  Where a few modules' values stay in the Infinity Cache, a call of more
     # than 16 rows reads them faster than it dequantizes codes (call times with codes over those with values: K = N = 4096, bf16 1.05 to 1.37 at 24
-    # to 1024 rows, f16 0.95 to 1.11; 3072 x 12800 bf16 1.05 to 1.25, f16 0.73 to 1.00; 5632 x 7616 0.72 to 1.06 and 0.71 to 0.92; from memory 0.70 to
-    # 1.06 and 0.66 to 0.97 at all of these), so smaller modules keep both where the device has room; up to 16 rows codes take 0.57 to 0.87 of the
-    # time, and nothing less than 0.9 where the weights are so few that a call is mostly its launch.
+    # to 1024 rows, f16 0.95 to 1.11; 3072 x 12800 bf16 1.05 to 1.25, f16 0.73 to 1.00; 5632 x 7616 0.72 to 1.06 and 0.71 to 0.92; from memory, as in a
+    # model of many layers, 0.70 to 1.06 and 0.66 to 1.03 at all of these: there the values pay from some 2048 rows on only), so smaller modules keep both
+    # where the device has room; up to 16 rows codes take 0.57 to 0.87 of the time, and nothing less than 0.9 where the weights are so few that a call is mostly its launch.
     _CODES_FROM, _CODES_ALONE_FROM = 8 << 20, {float16: 32 << 20, bfloat16: 40 << 20}
 
     def _keeps_codes(self, w_scale, per_out, has_x_scale, K, N):
