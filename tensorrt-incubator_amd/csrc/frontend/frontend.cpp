@@ -1027,10 +1027,24 @@ PyObject *f_tp_linear(PyObject *, PyObject *const *a, Py_ssize_t n) {
   p.bias = has_bias ? bias.t->data_ptr() : nullptr;
   c10::SmallVector<int64_t, 6> shape(x.t->sizes().begin(), x.t->sizes().end());
   shape.back() = p.N;
-  const int64_t M = x.t->numel() / p.K, scratch_bytes = mtrt_hip_linear_workspace(&p, M);
+  const int64_t M = x.t->numel() / p.K;
+  int64_t scratch_bytes = mtrt_hip_linear_workspace(&p, M);
   const Place place(*x.t);
   const at::Tensor y = place.empty(shape, lp->type);
-  const at::Tensor scratch = scratch_bytes ? place.bytes(scratch_bytes) : at::Tensor();
+  at::Tensor scratch;
+  if (scratch_bytes) {
+    try {
+      scratch = place.bytes(scratch_bytes);
+    } catch (const c10::OutOfMemoryError &) {
+      // a float32 product without memory for its partial sums runs unsplit; what it cannot do without is that of an x that is quantized
+      const int64_t least = p.dtype != MTRT_F32 ? scratch_bytes : p.q_dtype < 0 ? 0 : (M * p.K * 4 + 255) / 256 * 256;
+      if (least >= scratch_bytes)
+        throw;
+      scratch_bytes = least;
+      if (least)
+        scratch = place.bytes(least);
+    }
+  }
   const mtrt_stream_t s = place.stream;
   if (!launch([&] {
         return mtrt_hip_linear(s, &p, x.t->data_ptr(), y.data_ptr(), M, scratch_bytes ? scratch.data_ptr() : nullptr, scratch_bytes);

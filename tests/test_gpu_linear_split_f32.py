@@ -83,3 +83,37 @@ def test_beside_the_call_that_does_not_share(tp, pkg, M, K, N, parts):
     # each within (K + 3) half ulps of the sum of the terms' sizes, test_parts_against_float64
     mass = x.double().abs() @ w.double().abs().T + b.double().abs()
     assert bool(((shared.double() - dense.double()).abs() <= 2 * (K + 3) * 2.0 ** -24 * mass).all())
+
+
+@pytest.mark.parametrize("M,K,N,quantized", [(257, 12288, 512, False), (33, 4096, 1024, True)])
+def test_a_module_whose_parts_find_no_memory(tp, pkg, M, K, N, quantized):
+    """Where the allocator has room for the result (and an x that is quantized) and none for the partial sums: unsplit, as a call that does not share."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M + K + N)
+    x, wide = tp.Tensor(torch.randn((M, K), generator=g, device="cuda")), torch.zeros((N, 2), device="cuda")
+    wide[:, 0] = torch.randn(N, generator=g, device="cuda")
+    lin = tp.Linear(K, N, dtype=tp.float32, quant_dtype=tp.float8 if quantized else None)
+    lin.weight = tp.Tensor(torch.randn((N, K), generator=g, device="cuda") / math.sqrt(K))
+    if quantized:
+        lin.weight_scale, lin.input_scale = tp.Tensor(torch.tensor(4.0 / math.sqrt(K) / 448)), tp.Tensor(torch.tensor(4.0 / 448))
+    lin.bias = tp.Tensor(wide[:, 0])
+    want = lin(x).torch()                                            # (a strided bias takes the general path, which does not share)
+    assert "split" not in pkg.last_kernel()
+    lin.bias = tp.Tensor(wide[:, 0].contiguous())
+    shared = lin(x).torch()
+    assert "split" in pkg.last_kernel()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    held, mib, total = [], 1 << 20, torch.cuda.get_device_properties(0).total_memory
+    try:
+        # one byte more than a MiB is asked of the device in 20 MiB, anything up to that in 2
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + 8 * mib) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            for _ in range(4096):
+                held.append(torch.empty(mib + 512, dtype=torch.uint8, device="cuda"))
+        y = lin(x).torch()
+        name = pkg.last_kernel()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert "split" not in name and torch.equal(y, want), name
+    assert torch.equal(lin(x).torch(), shared) and "split" in pkg.last_kernel()
